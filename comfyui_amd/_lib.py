@@ -16,6 +16,7 @@ LIB_PATH = os.path.join(_HERE, "libhdmoe.so")
 W_BF16 = 0
 W_E4M3FN = 1
 W_F16 = 2
+W_E4M3FN_UPCAST = 3     # e4m3fn weights, bf16 arithmetic
 SRC_BF16 = 0
 SRC_F32 = 2
 ACT_NONE = 0
@@ -47,6 +48,22 @@ class FfnWeights(ctypes.Structure):
 class LinearWeights(ctypes.Structure):
     """hdmoe_linear_weights"""
     _fields_ = [("weight", c_void_p), ("bias", c_void_p)]
+
+
+class LinearGroup(ctypes.Structure):
+    """hdmoe_linear_group"""
+    _fields_ = [("weight", c_void_p), ("bias", c_void_p), ("scale", c_void_p)]
+
+
+class LinearArgs(ctypes.Structure):
+    """hdmoe_linear_args"""
+    _fields_ = [
+        ("act_dtype", c_int), ("weight_dtype", c_int), ("K", c_int), ("N", c_int), ("act", c_int), ("E", c_int),
+        ("rows", c_int), ("T", c_int), ("rows_static", c_int),
+        ("a", c_void_p), ("perm", c_void_p), ("offsets", c_void_p), ("experts", ctypes.POINTER(LinearGroup)), ("out", c_void_p),
+        ("a_static", c_void_p), ("shared", ctypes.POINTER(LinearGroup)), ("out_static", c_void_p),
+        ("workspace", c_void_p), ("workspace_bytes", c_size_t),
+    ]
 
 
 class LayerArgs(ctypes.Structure):
@@ -109,6 +126,8 @@ SIGNATURES = {
     "hdmoe_grouped_linear_tokens": (c_int, [c_int, c_void_p, c_int, c_void_p, c_void_p, c_int, ctypes.POINTER(LinearWeights),
                                             c_void_p, ctypes.POINTER(LinearWeights), c_void_p, c_int, c_int, c_int,
                                             c_void_p]),
+    "hdmoe_linear_groups_workspace_bytes": (c_size_t, [ctypes.POINTER(LinearArgs)]),
+    "hdmoe_linear_groups": (c_int, [ctypes.POINTER(LinearArgs), c_void_p]),
     "hdmoe_stochastic_round_e4m3fn": (c_int, [c_int, c_void_p, ctypes.c_int64, c_void_p, ctypes.c_uint64, c_void_p,
                                               c_void_p]),
     "hdmoe_ln_modulate_bf16": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, ctypes.c_float, c_void_p,

@@ -28,6 +28,7 @@ HIPCC_FLAGS = [
 
 def build(verbose=True, extra_flags=()):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+    subprocess.check_call([sys.executable, os.path.join(CSRC, "gen_gemm4w.py")])   # -> gemm4w_asm.inc
     objs = []
     procs = []
     for src in SOURCES:

@@ -224,7 +224,7 @@ struct CombinePartialArgs {
   const float* partial;
   long long part_stride;   // floats between two parts
   HdmoeSplitPlan plan;     // the candidate cuts of the down projection; the entry that ran is chosen as its kernel chose
-  int rows_dyn, n_dyn, fp8, has_shared;
+  int rows_dyn, n_dyn, weight_dtype, has_shared;
   const int32_t* offsets;  // segment bounds of the routed rows, n_dyn + 1 entries
   const float* sw[HDMOE_MAX_EXPERTS + 1];   // scale_weight of the down Linear per expert (fp8); the shared expert is entry n_dyn
   const float* sin[HDMOE_MAX_EXPERTS + 1];  // its scale_input or NULL
@@ -241,7 +241,11 @@ __global__ __launch_bounds__(THREADS) void combine_partials_kernel(const Combine
   const bool hg = ex.gate != nullptr;
   const int chunks = (row16 + 63) / 64;   // a wave takes 64 x 8 features of one token at a time
   const int n_out = row16 * 8;
-  auto scale_of = [&](int g) -> float { return pa.fp8 ? (pa.sin[g] ? *pa.sin[g] : 1.0f) * *pa.sw[g] : 1.0f; };
+  auto scale_of = [&](int g) -> float {
+    if (pa.weight_dtype == HDMOE_W_E4M3FN) return (pa.sin[g] ? *pa.sin[g] : 1.0f) * *pa.sw[g];
+    if (pa.weight_dtype == HDMOE_W_E4M3FN_UPCAST && pa.sw[g] != nullptr) return hdmoe_dev_round_bf16(*pa.sw[g]);
+    return 1.0f;
+  };
   auto group_of = [&](int r) {
     int g = 0;
     while (g + 1 < pa.n_dyn && r >= pa.offsets[g + 1]) ++g;
@@ -490,7 +494,7 @@ extern "C" int hdmoe_renorm_top2_bf16(const void* topk_weight_bf16, int T, void*
 // experts[e].scale_w2 / scale_in2 and the shared expert's are the scales of the rows (fp8 weights only).
 int hdmoe_launch_combine_partials(const float* partial, long long part_stride, const HdmoeSplitPlan& plan,
                                   int rows_dyn, int n_dyn,
-                                  const int32_t* offsets, bool fp8, const hdmoe_ffn_weights* experts,
+                                  const int32_t* offsets, int weight_dtype, const hdmoe_ffn_weights* experts,
                                   const hdmoe_ffn_weights* shared, const int32_t* inv_perm, const void* topk_weight_bf16,
                                   const void* gate_bf16, const void* residual_bf16, int tokens_per_batch, int T, int D,
                                   void* out_bf16, hipStream_t s, const char* what) {
@@ -503,7 +507,7 @@ int hdmoe_launch_combine_partials(const float* partial, long long part_stride, c
   pa.plan = plan;
   pa.rows_dyn = rows_dyn;
   pa.n_dyn = n_dyn;
-  pa.fp8 = fp8 ? 1 : 0;
+  pa.weight_dtype = weight_dtype;
   pa.has_shared = shared != nullptr ? 1 : 0;
   pa.offsets = offsets;
   for (int e = 0; e < n_dyn; ++e) { pa.sw[e] = experts[e].scale_w2; pa.sin[e] = experts[e].scale_in2; }

@@ -112,6 +112,9 @@ struct GemmArgs {
   // gather[r] >> alt.shift) instead of what the groups say (the gate kernel of the layer picks the layout of the fp8
   // tokens from the scale values and leaves the flag). flag NULL = off.
   HdmoeAltOperand alt;
+  // gemm4w_kernel only
+  uint8_t* scratch;       // with GELU: G4_SCRATCH bytes per block
+  float* tail;            // room for the parts of tail tiles (G4_TAIL_BYTES), NULL = tiles are not cut
 };
 
 __device__ __forceinline__ int swz(int row) { return ((row >> 1) & 7) ^ ((row & 1) << 2); }
@@ -986,7 +989,8 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_kernel(const GemmArgs a
 struct SplitKReduceArgs {
   const float* partial;     // [nparts][rows_dyn + rows_static][n_out]
   long long part_stride;
-  int nparts, nparts_static, n_out, rows_dyn, rows_static, n_dyn, fp8;  // parts of the dynamic rows, of the static rows
+  int nparts, nparts_static, n_out, rows_dyn, rows_static, n_dyn;  // parts of the dynamic rows, of the static rows
+  int scaled;               // 1: scale_input * scale_weight (fp8), 2: scale_weight rounded to bf16 (one-byte weights, bf16 arithmetic)
   const int32_t* offsets;   // segment bounds of the dynamic rows, n_dyn + 1 entries
   const float* sw[MAX_GROUPS];   // scale_weight per group (fp8); the static group is entry n_dyn
   const float* sin[MAX_GROUPS];  // scale_input per group or NULL
@@ -1006,7 +1010,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const SplitKReduceAr
       while (g + 1 < a.n_dyn && r >= a.offsets[g + 1]) ++g;
     }
     float sc = 1.0f;
-    if (a.fp8) sc = (a.sin[g] ? *a.sin[g] : 1.0f) * *a.sw[g];
+    if (a.scaled == 1) sc = (a.sin[g] ? *a.sin[g] : 1.0f) * *a.sw[g];
+    if (a.scaled == 2 && a.sw[g] != nullptr) sc = hdmoe_dev_round_bf16(*a.sw[g]);
     const float* src = a.partial + (size_t)r * a.n_out + c;
     float4 s = *reinterpret_cast<const float4*>(src);
     const int np = r < a.rows_dyn ? a.nparts : a.nparts_static;
@@ -1043,7 +1048,52 @@ int launch_grouped(const GemmArgs& args, int tile_bound, hipStream_t s, const ch
   return hdmoe_check_launch(what);
 }
 
+#include "gemm4w.h"
 #include "swiglu4w.h"
+
+// rows_mean: rows of a dynamic group when the routing is even (its real size is known on the device only)
+template <bool F16, bool W8, int EPI>
+int launch_gemm4w(GemmArgs& args, int rows_mean, hipStream_t s, const char* what) {
+  constexpr int FEAT = EPI == G4_SWIGLU ? 128 : 256;
+  static bool attr_set[64] = {};
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) device = -1;
+  if (device < 0 || !attr_set[device]) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm4w_kernel<F16, W8, EPI>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, G4_SMEM);
+    if (e != hipSuccess) return hdmoe_fail(HDMOE_E_LAUNCH, "%s: hipFuncSetAttribute: %s", what, hipGetErrorString(e));
+    if (device >= 0) attr_set[device] = true;
+  }
+  // Whether tail tiles may get cut: by the plan of an even routing, and of one whose experts are two standard deviations
+  // (counts are about binomial) below or above it. Without dynamic groups the three are the same and the plan is known here.
+  if (EPI == G4_PARTIAL) args.tail = nullptr;
+  if (args.tail != nullptr) {
+    bool cut = false;
+    for (int k = -1; k <= 1; ++k) {
+      int tiles = 0;
+      double fill = 0;
+      for (int g = 0; g < args.G; ++g) {
+        const GemmGroup& gg = args.g[g];
+        const int nt = gg.n_out / FEAT;
+        int rows = gg.row_end - gg.row_begin;
+        if (gg.row_begin < 0) rows = max(0, rows_mean + k * (int)(2 * sqrt((double)rows_mean)));
+        tiles += (rows + G4_BM - 1) / G4_BM * nt;
+        fill += (double)rows * nt / G4_BM;
+        if (gg.kbytes != args.g[0].kbytes) args.tail = nullptr;   // tiles of two lengths: one cut does not even them out
+      }
+      if (tiles > 0 && tiles <= 24 * HDMOE_NUM_CU)                // one round of more than 24 is not worth a launch
+        cut = cut || g4_plan_tail(tiles, HDMOE_NUM_CU, args.g[0].kbytes / (2 * BK), W8 ? 3 : 2, (float)(fill / tiles)).parts > 1;
+    }
+    if (!cut) args.tail = nullptr;
+  }
+  // one block per CU whatever the number of tiles: a block without any ends at once
+  hipLaunchKernelGGL((gemm4w_kernel<F16, W8, EPI>), dim3(HDMOE_NUM_CU), dim3(G4_THREADS), G4_SMEM, s, args);
+  if constexpr (EPI != G4_PARTIAL) {
+    if (args.tail != nullptr)
+      hipLaunchKernelGGL((gemm4w_tail_kernel<F16, W8, EPI>), dim3(4 * HDMOE_NUM_CU), dim3(256), 0, s, args, HDMOE_NUM_CU);
+  }
+  return hdmoe_check_launch(what);
+}
 
 int launch_swiglu4w(const GemmArgs& args, int tile_bound, hipStream_t s, const char* what) {
   static bool attr_set[64] = {};
@@ -1062,9 +1112,11 @@ int launch_swiglu4w(const GemmArgs& args, int tile_bound, hipStream_t s, const c
   return hdmoe_check_launch(what);
 }
 
+// bytes of an activation
 inline int elem_bytes(int weight_dtype) { return weight_dtype == HDMOE_W_E4M3FN ? 1 : 2; }
 
-int check_dtype(int weight_dtype, const char* what) {
+int check_dtype(int weight_dtype, const char* what, bool upcast_ok = false) {
+  if (upcast_ok && weight_dtype == HDMOE_W_E4M3FN_UPCAST) return HDMOE_OK;
   if (weight_dtype != HDMOE_W_BF16 && weight_dtype != HDMOE_W_E4M3FN)
     return hdmoe_fail(HDMOE_E_SHAPE, "%s: weight_dtype=%d is neither HDMOE_W_BF16 nor HDMOE_W_E4M3FN", what, weight_dtype);
   return HDMOE_OK;
@@ -1102,7 +1154,7 @@ enum GemmForm {
 };
 
 struct GemmShape {
-  bool swiglu, fp8, split;
+  bool swiglu, fp8, split, w8;
   int rows_dyn, n_dyn, rows_static;  // rows_static = 0: no static group
   int N_dyn, N_static;
   bool w4_fits;                      // the 4-wave kernel takes these operands (swiglu4w_fits)
@@ -1110,18 +1162,21 @@ struct GemmShape {
 
 // Expected tiles with evenly loaded experts, static round-robin over the CUs, and a fixed cost per tile of about one
 // 32-token block: rounds x (TT + 1). The taller tile wins when it does not add a round.
-long expected_tile_cost(const GemmShape& sh, int tt) {
+long expected_tiles(const GemmShape& sh, int tt) {
   const int bm = 64 * tt, fpt = sh.swiglu ? BN / 2 : BN;
   long tiles = 0;
   if (sh.n_dyn > 0) tiles += (long)sh.n_dyn * ((sh.rows_dyn / sh.n_dyn + bm - 1) / bm) * (sh.N_dyn / fpt);
   if (sh.rows_static > 0) tiles += (long)((sh.rows_static + bm - 1) / bm) * (sh.N_static / fpt);
-  return ((tiles + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU) * (tt + 1);
+  return tiles;
+}
+long expected_tile_cost(const GemmShape& sh, int tt) {
+  return ((expected_tiles(sh, tt) + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU) * (tt + 1);
 }
 
 // light: the token blocks of a tile that hold no rows are skipped (fp8: the compiler-scheduled K loop instead of the
 // assembly loop, which multiplies padding like rows; 16-bit weights always skip them and take from this only the
 // three-stage ring).
-struct FormChoice { GemmForm form; bool light, ring16, tall; };
+struct FormChoice { GemmForm form; bool light, ring16, tall, one_round5; };
 FormChoice pick_form(const GemmShape& sh) {
   const int f_light = form_of(HDMOE_FORM_LIGHT), f_4w = form_of(HDMOE_FORM_SWIGLU4W);
   const bool few_rows = hdmoe_few_rows(sh.rows_dyn, sh.n_dyn, sh.rows_static);
@@ -1129,9 +1184,11 @@ FormChoice pick_form(const GemmShape& sh) {
   // forcing the 4-wave kernel also keeps the light form's default off
   c.light = sh.fp8 && (f_light != HDMOE_FORM_AUTO ? f_light == HDMOE_FORM_ALWAYS
                                                    : few_rows && !(sh.swiglu && f_4w == HDMOE_FORM_ALWAYS));
-  c.ring16 = !sh.fp8 && few_rows && f_light != HDMOE_FORM_NEVER;
-  // (bf16: the gate/up kernel only; the down projection measured slower on the taller tile)
-  c.tall = (sh.fp8 || sh.swiglu) && !sh.split && !c.light && expected_tile_cost(sh, 5) < expected_tile_cost(sh, 4);
+  c.ring16 = !sh.fp8 && !sh.w8 && few_rows && f_light != HDMOE_FORM_NEVER;
+  // (16-bit weights: where the taller tile fits one round of blocks and the 256-token tile needs a second, e.g. 257 to 320
+  // tokens of a layer with a shared expert: 93 against 96 us in the gate/up contraction)
+  c.one_round5 = !sh.fp8 && !sh.w8 && sh.swiglu && expected_tiles(sh, 5) <= HDMOE_NUM_CU && expected_tiles(sh, 4) > HDMOE_NUM_CU;
+  c.tall = sh.fp8 && !sh.split && !c.light && expected_tile_cost(sh, 5) < expected_tile_cost(sh, 4);
   if (sh.split) { c.form = FORM_SPLIT_K; return c; }
   // Light form, gate/up: with every segment inside one 128-token tile (up to 128 tokens in a top-2 layer of 4 experts)
   // the three-stage ring of the down projection pays here too (whole layer 78 -> 73 us at 16 tokens, 80 -> 75 at 128;
@@ -1174,7 +1231,9 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
                           int K_static, int N_static, hipStream_t s, const char* what,
                           const int32_t* gather_dyn = nullptr, int gather_rows = 0, float* partial = nullptr,
                           int nparts = 1, int gather_shift = 0, bool reduce = true,
-                          const HdmoeSplitPlan* plan = nullptr, const HdmoeAltOperand* alt = nullptr) {
+                          const HdmoeSplitPlan* plan = nullptr, const HdmoeAltOperand* alt = nullptr,
+                          float* tail = nullptr) {
+  const bool w8 = weight_dtype == HDMOE_W_E4M3FN_UPCAST;  // one-byte weights, 16-bit arithmetic
   const int eb = elem_bytes(weight_dtype);
   const bool fp8 = weight_dtype == HDMOE_W_E4M3FN;
   const int feat_per_tile = swiglu ? BN / 2 : BN;
@@ -1182,24 +1241,31 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
   // the plan cuts a tile into (the partial-sum buffer holds that many); no plan = every tile in nparts parts
   const bool split = !swiglu && partial != nullptr && nparts > 1;
   GemmShape shape;
-  shape.swiglu = swiglu; shape.fp8 = fp8; shape.split = split;
+  shape.swiglu = swiglu; shape.fp8 = fp8; shape.split = split; shape.w8 = w8;
   shape.rows_dyn = rows_dyn; shape.n_dyn = n_dyn; shape.rows_static = shared != nullptr ? rows_static : 0;
   shape.N_dyn = N_dyn; shape.N_static = N_static;
   shape.w4_fits = true;  // settled below, once the groups are filled in
   FormChoice choice = pick_form(shape);
   const bool light = choice.light, ring16 = choice.ring16, tall = choice.tall;
-  const int BM = tall ? TileCfg<5>::BM : TileCfg<4>::BM;  // tokens per block tile of the kernel that will run
+  const int BM = tall || choice.one_round5 ? TileCfg<5>::BM : TileCfg<4>::BM;  // tokens per block tile of the kernel that will run
   const int gather_rows_max = (alt != nullptr && alt->rows > gather_rows) ? alt->rows : gather_rows;
   if (gather_dyn != nullptr && (unsigned long long)gather_rows_max * K_dyn * eb >= (1ull << 31))
     return hdmoe_fail(HDMOE_E_SHAPE, "%s: %d gathered rows of %d bytes exceed the 2 GiB offset range", what,
                       gather_rows_max, K_dyn * eb);
+  // few rows and 16-bit weights: the 8-wave kernels, whose forms (ring or not) give the same bytes
+  const bool few_rows = !w8 && hdmoe_few_rows(shape.rows_dyn, shape.n_dyn, shape.rows_static);
+  const bool ring_size = few_rows && shape.rows_static <= TileCfg<2>::BM && (n_dyn <= 0 || rows_dyn <= TileCfg<2>::BM / 2 * n_dyn);
   GemmArgs args;
   memset(&args, 0, sizeof(args));
   if (alt != nullptr && gather_dyn != nullptr) args.alt = *alt;
   args.nparts = 1;
+  args.tail = tail;
   args.offsets = offsets;
   args.n_offsets = n_dyn;
   int G = 0, tile_bound = 0;
+  const long long op_bytes_dyn = (long long)(gather_dyn != nullptr ? gather_rows_max : rows_dyn) * K_dyn * eb;
+  const long long op_bytes = op_bytes_dyn > (long long)rows_static * K_static * eb ? op_bytes_dyn : (long long)rows_static * K_static * eb;
+  const int rows_mean = n_dyn > 0 ? rows_dyn / n_dyn : 0;
   for (int e = 0; e < n_dyn; ++e, ++G) {
     GemmGroup& gg = args.g[G];
     const hdmoe_ffn_weights& w = experts[e];
@@ -1293,10 +1359,14 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
         if (tl > tb_light) tb_light = tl;
       }
     }
+    const bool g4 = !fp8 && !few_rows && gemm4w_fits(args, w8, op_bytes);
+    if (w8 && !g4) return hdmoe_fail(HDMOE_E_SHAPE, "%s: K=%d / %d in %d parts does not fit the kernel for one-byte weights", what, K_dyn, K_static, nparts);
     const int rc = light ? launch_grouped<FP8_PLAIN, 2, true>(args, tb_light, s, what)
+                   : w8 ? launch_gemm4w<false, true, G4_PARTIAL>(args, rows_mean, s, what)
                    : ring16 ? launch_grouped<BF16_PLAIN, 2, true>(args, tb_light, s, what)
                    : fp8 ? launch_grouped<FP8_PLAIN>(args, tile_bound, s, what)
-                         : launch_grouped<BF16_PLAIN>(args, tile_bound, s, what);
+                   : g4 ? launch_gemm4w<false, false, G4_PARTIAL>(args, rows_mean, s, what)
+                        : launch_grouped<BF16_PLAIN>(args, tile_bound, s, what);
     if (rc != HDMOE_OK) return rc;
     if (!reduce) return HDMOE_OK;  // the caller's next kernel adds the parts up (hdmoe_launch_combine_partials)
     SplitKReduceArgs ra;
@@ -1309,7 +1379,7 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
     ra.rows_dyn = n_dyn > 0 ? rows_dyn : 0;
     ra.rows_static = (shared != nullptr && rows_static > 0) ? rows_static : 0;
     ra.n_dyn = n_dyn;
-    ra.fp8 = fp8 ? 1 : 0;
+    ra.scaled = fp8 ? 1 : w8 ? 2 : 0;
     ra.offsets = offsets;
     for (int g = 0; g < G; ++g) {
       const int slot = args.g[g].row_begin < 0 ? args.g[g].dyn : n_dyn;
@@ -1325,9 +1395,24 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
     hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, s, ra);
     return hdmoe_check_launch(what);
   }
+  if (!fp8) {
+    // The 4-wave kernel (gemm4w.h) takes whatever fits it: a K step of a 256 x 256 tile takes 1.36 to 1.45 us there and
+    // 1.7 to 1.8 us in the 8-wave kernel (16384 x 13824 x 2560: 0.81 against 0.96 ms). Left to the 8-wave kernels: the
+    // three-stage ring for gate/up with every segment inside a 128-token tile (16-bit weights), the case one_round5, K that is
+    // not a multiple of 128, and, where tiles cannot be cut (no room for the parts), one Linear on up to 128 rows (2560 x 2560: 37
+    // against 43 us: the 8-wave kernel leaves out the token blocks without rows).
+    const bool g4 = gemm4w_fits(args, w8, op_bytes);
+    if (w8) {
+      if (!g4) return hdmoe_fail(HDMOE_E_SHAPE, "%s: K=%d / %d does not fit the kernel for one-byte weights", what, K_dyn, K_static);
+      return swiglu ? launch_gemm4w<false, true, G4_SWIGLU>(args, rows_mean, s, what)
+                    : launch_gemm4w<false, true, G4_PLAIN>(args, rows_mean, s, what);
+    }
+    if (choice.one_round5) return launch_grouped<BF16_SWIGLU, 5>(args, tile_bound, s, what);
+    if (swiglu && g4 && !ring_size) return launch_gemm4w<false, false, G4_SWIGLU>(args, rows_mean, s, what);
+    if (!swiglu && g4 && (tail != nullptr || rows_mean > 128 || rows_static > 128))
+      return launch_gemm4w<false, false, G4_PLAIN>(args, rows_mean, s, what);
+  }
   if (fp8 && swiglu) {
-    long long op_bytes = (long long)(gather_dyn != nullptr ? gather_rows_max : rows_dyn) * K_dyn;
-    if ((long long)rows_static * K_static > op_bytes) op_bytes = (long long)rows_static * K_static;
     shape.w4_fits = swiglu4w_fits(args, op_bytes);
     choice = pick_form(shape);
   }
@@ -1350,9 +1435,8 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
       return launch_swiglu4w(args, tb, s, what);
     }
     case FORM_TALL5:
-      if (fp8) return swiglu ? launch_grouped<FP8_SWIGLU, 5>(args, tile_bound, s, what)
-                             : launch_grouped<FP8_PLAIN, 5>(args, tile_bound, s, what);
-      return launch_grouped<BF16_SWIGLU, 5>(args, tile_bound, s, what);
+      return swiglu ? launch_grouped<FP8_SWIGLU, 5>(args, tile_bound, s, what)
+                    : launch_grouped<FP8_PLAIN, 5>(args, tile_bound, s, what);
     default:
       break;
   }
@@ -1366,10 +1450,10 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
 // if Hs > 0), by the launcher's own rule and the current form switches: for reports that name the dominant kernel.
 extern "C" const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E, int D, int H, int Hs,
                                                  int has_scale_in2) {
-  if (check_dtype(weight_dtype, "hdmoe_gate_up_kernel_name") != HDMOE_OK || T <= 0 || E < 0 || D <= 0 || H <= 0)
+  if (check_dtype(weight_dtype, "hdmoe_gate_up_kernel_name", true) != HDMOE_OK || T <= 0 || E < 0 || D <= 0 || H <= 0)
     return "";
   GemmShape sh;
-  sh.swiglu = true; sh.fp8 = weight_dtype == HDMOE_W_E4M3FN; sh.split = false;
+  sh.swiglu = true; sh.fp8 = weight_dtype == HDMOE_W_E4M3FN; sh.split = false; sh.w8 = weight_dtype == HDMOE_W_E4M3FN_UPCAST;
   sh.rows_dyn = E > 0 ? T * HDMOE_TOPK : 0; sh.n_dyn = E; sh.rows_static = Hs > 0 ? T : 0;
   sh.N_dyn = H; sh.N_static = Hs;
   const int kb = D * elem_bytes(weight_dtype);
@@ -1379,8 +1463,11 @@ extern "C" const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E,
     case FORM_RING3: return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 2, LIGHT>" : "grouped_gemm_kernel<BF16_SWIGLU, 2, LIGHT>";
     case FORM_LIGHT4: return "grouped_gemm_kernel<FP8_SWIGLU, 4, LIGHT>";
     case FORM_W4: return "swiglu4w_kernel";
-    case FORM_TALL5: return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 5>" : "grouped_gemm_kernel<BF16_SWIGLU, 5>";
-    default: return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 4>" : "grouped_gemm_kernel<BF16_SWIGLU, 4>";
+    case FORM_TALL5: return "grouped_gemm_kernel<FP8_SWIGLU, 5>";
+    default:
+      if (pick_form(sh).one_round5) return "grouped_gemm_kernel<BF16_SWIGLU, 5>";
+      if (!sh.fp8 && kb % (2 * BK) == 0 && kb >= 4 * BK) return "gemm4w_kernel<SWIGLU>";
+      return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 4>" : "grouped_gemm_kernel<BF16_SWIGLU, 4>";
   }
 }
 
@@ -1425,7 +1512,8 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
       t2 += (long)n_dyn * ((seg + bm2 - 1) / bm2) * nt;
     }
     if (rows_static > 0) t2 += (long)((rows_static + bm2 - 1) / bm2) * nt;
-    const int kt2 = ktd > kts ? ktd : kts;
+    int kt2 = ktd > kts ? ktd : kts;
+    if (weight_dtype == HDMOE_W_E4M3FN_UPCAST && ktd > 0 && kts > 0) kt2 = ktd < kts ? ktd : kts;  // no part under three pairs of steps
     long parts = (150 + t2 - 1) / t2;
     if (parts > HDMOE_NUM_CU / t2) parts = HDMOE_NUM_CU / t2;
     if (parts > 6) parts = 6;
@@ -1519,25 +1607,30 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
   return most;
 }
 
-// Linear with bias and optional GELU over expert row segments plus an optional static group (bf16 weights):
+// Linear with bias and optional GELU over expert row segments plus an optional static group:
 // the two stages of a GELU feed-forward (/root/reference/comfy/ldm/hunyuan3dv2_1/hunyuandit.py:28-50, 114-188).
-int hdmoe_launch_linear_groups(const uint8_t* a_dyn, const int32_t* offsets, int rows_dyn, int n_dyn,
-                               const hdmoe_linear_weights* experts, uint8_t* out_dyn, const uint8_t* a_static,
-                               int rows_static, const hdmoe_linear_weights* shared, uint8_t* out_static, int K, int N,
-                               int act, hipStream_t s, const char* what, bool f16 = false,
-                               const int32_t* gather = nullptr, int gather_rows = 0, int gather_shift = 0) {
+// tail, scratch: room of gemm4w_kernel (G4_TAIL_BYTES; G4_SCRATCH per block, GELU only) or NULL.
+template <typename W>
+int hdmoe_launch_linear_groups(const uint8_t* a_dyn, const int32_t* offsets, int rows_dyn, int n_dyn, const W* experts,
+                               uint8_t* out_dyn, const uint8_t* a_static, int rows_static, const W* shared,
+                               uint8_t* out_static, int K, int N, int act, hipStream_t s, const char* what, bool f16,
+                               const int32_t* gather, int gather_rows, int gather_shift, bool w8 = false,
+                               float* tail = nullptr, uint8_t* scratch = nullptr) {
   if (gather != nullptr && (unsigned long long)gather_rows * K * 2 >= (1ull << 31))
     return hdmoe_fail(HDMOE_E_SHAPE, "%s: %d gathered rows of %d bytes exceed the 2 GiB offset range", what, gather_rows,
                       K * 2);
   GemmArgs args;
   memset(&args, 0, sizeof(args));
   args.nparts = 1;
+  args.tail = tail;
+  args.scratch = scratch;
   args.offsets = offsets;
   args.n_offsets = n_dyn;
   int G = 0, tile_bound = 0;
-  auto fill = [&](GemmGroup& gg, const hdmoe_linear_weights& w) {
+  auto fill = [&](GemmGroup& gg, const W& w) {
     gg.b0 = static_cast<const uint8_t*>(w.weight);
     gg.bias = static_cast<const uint16_t*>(w.bias);
+    if constexpr (std::is_same_v<W, hdmoe_linear_group>) gg.sb0 = w.scale;
     gg.act = act;
     gg.n_out = N;
     gg.kbytes = K * 2;
@@ -1554,19 +1647,7 @@ int hdmoe_launch_linear_groups(const uint8_t* a_dyn, const int32_t* offsets, int
     gg.dyn = e;
     if (!gg.b0) return hdmoe_fail(HDMOE_E_NULL, "%s: expert %d has a NULL weight", what, e);
   }
-  // tile height by the rule of the feed-forward GEMMs: the 320-token tile when it saves a round of tiles
-  auto expected_cost = [&](int tt) {
-    const int bm = 64 * tt;
-    long tiles = 0;
-    // a segment taken one standard deviation of an even routing above the mean: at a mean that is a multiple of the
-    // tile height half the segments need one tile more
-    const int seg = n_dyn > 0 ? rows_dyn / n_dyn + (int)sqrtf((float)(rows_dyn / n_dyn)) : 0;
-    if (n_dyn > 0) tiles += (long)n_dyn * ((seg + bm - 1) / bm) * (N / BN);
-    if (shared != nullptr && rows_static > 0) tiles += (long)((rows_static + bm - 1) / bm) * (N / BN);
-    return ((tiles + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU) * (tt + 1);
-  };
-  const bool tall = expected_cost(5) < expected_cost(4);
-  const int BM = tall ? TileCfg<5>::BM : TileCfg<4>::BM;
+  constexpr int BM = TileCfg<4>::BM;
   if (n_dyn > 0) tile_bound += (rows_dyn / BM + n_dyn) * (N / BN);
   if (shared != nullptr && rows_static > 0) {
     GemmGroup& gg = args.g[G];
@@ -1580,8 +1661,21 @@ int hdmoe_launch_linear_groups(const uint8_t* a_dyn, const int32_t* offsets, int
     ++G;
   }
   args.G = G;
-  if (tall) return f16 ? launch_grouped<F16_PLAIN_BIAS, 5>(args, tile_bound, s, what)
-                       : launch_grouped<BF16_PLAIN_BIAS, 5>(args, tile_bound, s, what);
+  // the 4-wave kernel wherever it fits; it needs room of its own for the activation, and room for the parts of tiles where
+  // a few tiles have to be cut (on up to 128 rows the 8-wave kernel is the faster one without: see hdmoe_launch_ffn_gemm)
+  const int rows_mean = n_dyn > 0 ? rows_dyn / n_dyn : 0;
+  const bool g4 = gemm4w_fits(args, w8, gather != nullptr ? (long long)gather_rows * K * 2 : 0);
+  if (w8) {
+    if (!g4 || f16 || act == HDMOE_ACT_GELU)
+      return hdmoe_fail(HDMOE_E_SHAPE, "%s: K=%d act=%d does not fit the kernel for one-byte weights", what, K, act);
+    return launch_gemm4w<false, true, G4_BIAS>(args, rows_mean, s, what);
+  }
+  if (g4 && act == HDMOE_ACT_GELU && scratch != nullptr)
+    return f16 ? launch_gemm4w<true, false, G4_GELU>(args, rows_mean, s, what)
+               : launch_gemm4w<false, false, G4_GELU>(args, rows_mean, s, what);
+  if (g4 && act == HDMOE_ACT_NONE && (tail != nullptr || rows_mean > 128 || rows_static > 128))
+    return f16 ? launch_gemm4w<true, false, G4_BIAS>(args, rows_mean, s, what)
+               : launch_gemm4w<false, false, G4_BIAS>(args, rows_mean, s, what);
   return f16 ? launch_grouped<F16_PLAIN_BIAS>(args, tile_bound, s, what)
              : launch_grouped<BF16_PLAIN_BIAS>(args, tile_bound, s, what);
 }
@@ -1591,6 +1685,12 @@ int hdmoe_launch_linear_bias(int weight_dtype, const uint8_t* a, int rows, int K
                              const float* scale_w, const float* scale_in, const uint16_t* bias, uint8_t* out,
                              hipStream_t s, const char* what) {
   const bool fp8 = weight_dtype == HDMOE_W_E4M3FN;
+  if (!fp8) {
+    const hdmoe_linear_weights lw = {w, bias};
+    return hdmoe_launch_linear_groups(static_cast<const uint8_t*>(nullptr), nullptr, 0, 0, static_cast<const hdmoe_linear_weights*>(nullptr),
+                                      nullptr, a, rows, &lw, out, K, N, HDMOE_ACT_NONE, s, what, weight_dtype == HDMOE_W_F16,
+                                      nullptr, 0, 0);
+  }
   GemmArgs args;
   memset(&args, 0, sizeof(args));
   args.nparts = 1;
@@ -1608,15 +1708,13 @@ int hdmoe_launch_linear_bias(int weight_dtype, const uint8_t* a, int rows, int K
   gg.act = HDMOE_ACT_NONE;
   args.G = 1;
   const int tile_bound = ((rows + TileCfg<4>::BM - 1) / TileCfg<4>::BM) * (N / BN);
-  if (weight_dtype == HDMOE_W_F16) return launch_grouped<F16_PLAIN_BIAS>(args, tile_bound, s, what);
-  return fp8 ? launch_grouped<FP8_PLAIN_BIAS>(args, tile_bound, s, what)
-             : launch_grouped<BF16_PLAIN_BIAS>(args, tile_bound, s, what);
+  return launch_grouped<FP8_PLAIN_BIAS>(args, tile_bound, s, what);
 }
 
 // Size rules shared by the entry points: K bytes per row must be a multiple of the
 // 128-byte K step; total bytes of each operand must fit the 32-bit buffer range.
 int hdmoe_check_gemm_shape(const char* what, int weight_dtype, long rows, int K, int N, int feat_per_tile) {
-  if (int rc = check_dtype(weight_dtype, what)) return rc;
+  if (int rc = check_dtype(weight_dtype, what, true)) return rc;
   const int eb = elem_bytes(weight_dtype);
   if (rows < 0 || K <= 0 || N <= 0 || (K * eb) % BK != 0 || N % feat_per_tile != 0)
     return hdmoe_fail(HDMOE_E_SHAPE, "%s: rows=%ld K=%d N=%d (K*%d must be a multiple of %d, N of %d)", what, rows, K,
@@ -1633,6 +1731,7 @@ extern "C" int hdmoe_grouped_swiglu(int weight_dtype, const void* a, const int32
   HDMOE_REQUIRE_PTR(experts);
   HDMOE_REQUIRE_PTR(h);
   if (E < 1 || E > HDMOE_MAX_EXPERTS) return hdmoe_fail(HDMOE_E_SHAPE, "hdmoe_grouped_swiglu: E=%d", E);
+  if (int rc = check_dtype(weight_dtype, "hdmoe_grouped_swiglu")) return rc;
   if (int rc = hdmoe_check_gemm_shape("hdmoe_grouped_swiglu", weight_dtype, rows_total, D, H, BN / 2)) return rc;
   if (weight_dtype == HDMOE_W_E4M3FN)
     for (int e = 0; e < E; ++e)
@@ -1650,6 +1749,7 @@ extern "C" int hdmoe_grouped_down(int weight_dtype, const void* h, const int32_t
   HDMOE_REQUIRE_PTR(experts);
   HDMOE_REQUIRE_PTR(y_bf16);
   if (E < 1 || E > HDMOE_MAX_EXPERTS) return hdmoe_fail(HDMOE_E_SHAPE, "hdmoe_grouped_down: E=%d", E);
+  if (int rc = check_dtype(weight_dtype, "hdmoe_grouped_down")) return rc;
   if (int rc = hdmoe_check_gemm_shape("hdmoe_grouped_down", weight_dtype, rows_total, H, D, BN)) return rc;
   if (rows_total == 0) return HDMOE_OK;
   return hdmoe_launch_ffn_gemm(false, weight_dtype, static_cast<const uint8_t*>(h), offsets, rows_total, E, experts,
@@ -1663,6 +1763,7 @@ extern "C" int hdmoe_linear(int weight_dtype, const void* a, int rows, int K, in
   HDMOE_REQUIRE_PTR(a);
   HDMOE_REQUIRE_PTR(w);
   HDMOE_REQUIRE_PTR(out_bf16);
+  if (int rc = check_dtype(weight_dtype, "hdmoe_linear")) return rc;
   if (int rc = hdmoe_check_gemm_shape("hdmoe_linear", weight_dtype, rows, K, N, BN)) return rc;
   if (weight_dtype == HDMOE_W_E4M3FN) HDMOE_REQUIRE_PTR(scale_w_dev);
   if (rows == 0) return HDMOE_OK;
@@ -1684,6 +1785,8 @@ extern "C" int hdmoe_linear_bias(int weight_dtype, const void* a, int rows, int 
   HDMOE_REQUIRE_PTR(a);
   HDMOE_REQUIRE_PTR(w);
   HDMOE_REQUIRE_PTR(out_bf16);
+  if (weight_dtype != HDMOE_W_F16)
+    if (int rc = check_dtype(weight_dtype, "hdmoe_linear_bias")) return rc;
   if (int rc = hdmoe_check_gemm_shape("hdmoe_linear_bias", weight_dtype == HDMOE_W_F16 ? HDMOE_W_BF16 : weight_dtype,
                                       rows, K, N, BN))
     return rc;
@@ -1757,3 +1860,60 @@ extern "C" int hdmoe_grouped_linear_tokens(int act_dtype, const void* x, int T, 
   return grouped_linear_entry("hdmoe_grouped_linear_tokens", act_dtype == HDMOE_W_F16, x, offsets, T * HDMOE_TOPK, E,
                               experts, out, x, shared != nullptr ? T : 0, shared, out_shared, K, N, act, stream, perm, T);
 }
+
+// The same Linear for callers that bring working memory (hdmoe_linear_args in hdmoe.h): tiles that would leave most of the
+// chip idle are cut along K, and the GELU hides behind the next tile.
+namespace {
+int linear_groups_check(const hdmoe_linear_args* p) {
+  const char* what = "hdmoe_linear_groups";
+  const bool w8 = p->weight_dtype == HDMOE_W_E4M3FN_UPCAST;
+  if ((p->act_dtype != HDMOE_W_BF16 && p->act_dtype != HDMOE_W_F16) || (w8 ? p->act_dtype != HDMOE_W_BF16 : p->weight_dtype != p->act_dtype))
+    return hdmoe_fail(HDMOE_E_SHAPE, "%s: act_dtype=%d weight_dtype=%d", what, p->act_dtype, p->weight_dtype);
+  if (p->E < 0 || p->E > HDMOE_MAX_EXPERTS || p->rows < 0 || p->rows_static < 0 || p->T < 0)
+    return hdmoe_fail(HDMOE_E_SHAPE, "%s: E=%d rows=%d rows_static=%d T=%d", what, p->E, p->rows, p->rows_static, p->T);
+  if (p->act != HDMOE_ACT_NONE && p->act != HDMOE_ACT_GELU) return hdmoe_fail(HDMOE_E_SHAPE, "%s: act=%d", what, p->act);
+  if (p->perm != nullptr && p->rows != p->T * HDMOE_TOPK)
+    return hdmoe_fail(HDMOE_E_SHAPE, "%s: rows=%d is not %d slots of T=%d tokens", what, p->rows, HDMOE_TOPK, p->T);
+  const long rows_max = p->rows > p->rows_static ? p->rows : p->rows_static;
+  return hdmoe_check_gemm_shape(what, HDMOE_W_BF16, rows_max, p->K, p->N, BN);
+}
+size_t linear_groups_scratch(const hdmoe_linear_args* p) {
+  return p->act == HDMOE_ACT_GELU ? hdmoe_align_up((size_t)HDMOE_NUM_CU * G4_SCRATCH, 256) : 0;
+}
+}  // namespace
+
+extern "C" size_t hdmoe_linear_groups_workspace_bytes(const hdmoe_linear_args* p) {
+  if (p == nullptr || linear_groups_check(p) != HDMOE_OK) return 0;
+  return linear_groups_scratch(p) + G4_TAIL_BYTES;
+}
+
+extern "C" int hdmoe_linear_groups(const hdmoe_linear_args* p, hdmoe_stream_t stream) {
+  HDMOE_REQUIRE_PTR(p);
+  if (int rc = linear_groups_check(p)) return rc;
+  if (p->E > 0 && p->rows > 0) {
+    HDMOE_REQUIRE_PTR(p->a);
+    HDMOE_REQUIRE_PTR(p->offsets);
+    HDMOE_REQUIRE_PTR(p->experts);
+    HDMOE_REQUIRE_PTR(p->out);
+  }
+  if (p->rows_static > 0) {
+    HDMOE_REQUIRE_PTR(p->a_static);
+    HDMOE_REQUIRE_PTR(p->shared);
+    HDMOE_REQUIRE_PTR(p->out_static);
+  }
+  uint8_t* ws = static_cast<uint8_t*>(p->workspace);
+  if (ws != nullptr && (p->workspace_bytes < hdmoe_linear_groups_workspace_bytes(p) || (reinterpret_cast<uintptr_t>(ws) & 255)))
+    return hdmoe_fail(HDMOE_E_WORKSPACE, "hdmoe_linear_groups: workspace %zu bytes, need %zu (256-byte aligned)",
+                      p->workspace_bytes, hdmoe_linear_groups_workspace_bytes(p));
+  if ((p->E == 0 || p->rows == 0) && p->rows_static == 0) return HDMOE_OK;
+  const size_t sb = linear_groups_scratch(p);
+  return hdmoe_launch_linear_groups(static_cast<const uint8_t*>(p->a), p->offsets, p->rows, p->rows > 0 ? p->E : 0, p->experts,
+                                    static_cast<uint8_t*>(p->out), static_cast<const uint8_t*>(p->a_static), p->rows_static,
+                                    p->shared, static_cast<uint8_t*>(p->out_static), p->K, p->N, p->act,
+                                    static_cast<hipStream_t>(stream), "hdmoe_linear_groups", p->act_dtype == HDMOE_W_F16,
+                                    p->perm, p->T, p->perm != nullptr ? 1 : 0, p->weight_dtype == HDMOE_W_E4M3FN_UPCAST,
+                                    ws != nullptr ? reinterpret_cast<float*>(ws + sb) : nullptr, ws != nullptr && sb > 0 ? ws : nullptr);
+}
+
+// Bytes a feed-forward's contractions on 16-bit activations can use for the parts of tail tiles.
+size_t hdmoe_tail_bytes(int weight_dtype) { return weight_dtype == HDMOE_W_E4M3FN ? 0 : G4_TAIL_BYTES; }

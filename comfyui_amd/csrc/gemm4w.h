@@ -1,0 +1,516 @@
+// Grouped GEMM on 16-bit activations with one wave per SIMD: the tile text of gen_gemm4w.py (256 x 256 tile, 4 waves,
+// 512 registers each).
+//
+// Included by gemm.hip inside its unnamed namespace (uses GemmArgs, GemmGroup, swz, make_rsrc, lds_ptr_t). Same
+// contraction, rounding points and LDS tile format as grouped_gemm_kernel's 16-bit modes; weights may also be e4m3fn
+// bytes (W8), converted to bf16 between LDS and the matrix cores.
+//
+// What bounds it: with every CU multiplying N(0,1) values the clock falls to 1.5-1.7 GHz, so the energy per product decides;
+// a K step of a tile takes 1.36-1.5 us then and 0.95 us (the matrix pipe full) with most CUs idle. Against the 8-wave
+// kernel with 32x32x16 MFMAs: half the fragment reads from LDS per product (128 x 128 per wave), the smaller MFMA
+// (less energy), and no barrier that drains the pipe. bf16, M x N x K, 8-wave -> this kernel: 8192 x 8192 x 8192 917 -> 690
+// us, 16384 x 13824 x 2560 964 -> 805 us, 24576 x 2048 x 8192 654 -> 537 us (1.4-1.6 PFLOP/s). What the schedule hangs
+// on: the 16 global->LDS loads of a wave and step are spread over the whole step (every 2 MFMAs: 730 us, every 6: 690 us at
+// 8192^3; 4 waves times 16 lanes' worth of addresses each 16 cycles is all the address unit takes).
+// GELU, 24576 x 8192 x 2048: 846 us in the 8-wave kernel's epilogue, 682 us hidden behind the next tile's K loop (560-585 us
+// without activation; through the outputs themselves instead of a scratch buffer 732 us: the rows are written twice).
+#include "gemm4w_asm.inc"
+
+constexpr int G4_THREADS = 256;
+constexpr int G4_BM = 256;                        // tokens per block tile
+constexpr int G4_STAGE = 32768;
+constexpr int G4_W_TILE = 65536;
+constexpr int G4_TABLE = 131072;                  // LDS: [tok 0 | tok 1 | w 0 | w 1 | work item tables of the 4 waves]
+constexpr int G4_TABLE_ITEMS = 64;                // items a wave's lanes look up at a time
+constexpr int G4_SMEM = G4_TABLE + 4 * G4_TABLE_ITEMS * 16;
+constexpr int G4_SCRATCH = 4 * 28 * 1024;         // GELU: bytes of scratch per block (28 pieces of 16 bytes per lane)
+constexpr int G4_GELU_PAIRS = 16;                 // pairs of K steps a deferred activation needs to hide behind
+
+constexpr int G4_TAIL_MAX_PARTS = 12;
+constexpr size_t G4_TAIL_BYTES = (size_t)HDMOE_NUM_CU * G4_BM * 256 * 4;  // fp32 sums of one tile per block
+
+// What becomes of a tile's sums.
+enum G4Epi { G4_PLAIN, G4_BIAS, G4_GELU, G4_SWIGLU, G4_PARTIAL };
+
+typedef float v32f __attribute__((ext_vector_type(32)));
+typedef int v32i __attribute__((ext_vector_type(32)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+// positions in the context registers v[96:127] (gen_gemm4w.py)
+enum { G4_TOK_ADDR = 0, G4_W_ADDR = 2, G4_TOK_VOFF = 4, G4_W_VOFF = 12, G4_OUT_VOFF = 20, G4_GATHER_VOFF = 22,
+       G4_BIAS_VOFF = 23, G4_DEF_LD = 24, G4_DEF_ST = 25, G4_SCR_VOFF = 26 };
+
+#define G4_A10(b) "a" #b "0", "a" #b "1", "a" #b "2", "a" #b "3", "a" #b "4", "a" #b "5", "a" #b "6", "a" #b "7", "a" #b "8", "a" #b "9"
+#define G4_V10(b) "v" #b "0", "v" #b "1", "v" #b "2", "v" #b "3", "v" #b "4", "v" #b "5", "v" #b "6", "v" #b "7", "v" #b "8", "v" #b "9"
+// what a tile's statement overwrites beside its operands: accumulators, slice 1 fragments, work registers, resources
+#define G4_CLOBBER_V                                                                                                 \
+  "memory", "scc", "v34", "v35", "v36", "v37", "v38", "v39", G4_V10(4), G4_V10(5), G4_V10(6), "v70",    \
+      "v71", "v192", "v193", "v194", "v195", "v196", "v197", "v198", "v199", G4_V10(20), G4_V10(21), G4_V10(22),      \
+      G4_V10(23), G4_V10(24), "v250", "v251", "v252", "v253", "v254", "v255"
+#define G4_CLOBBER                                                                                                   \
+  G4_CLOBBER_V, "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "s72", "s73", "s74", "s75", G4_A10(),         \
+      G4_A10(1), G4_A10(2), G4_A10(3), G4_A10(4), G4_A10(5), G4_A10(6), G4_A10(7), G4_A10(8), G4_A10(9), G4_A10(10),  \
+      G4_A10(11), G4_A10(12), G4_A10(13), G4_A10(14), G4_A10(15), G4_A10(16), G4_A10(17), G4_A10(18), G4_A10(19),     \
+      G4_A10(20), G4_A10(21), G4_A10(22), G4_A10(23), G4_A10(24), "a250", "a251", "a252", "a253", "a254", "a255"
+
+// Segment bounds of the groups: lane g + 1 of off_lane holds the end of dynamic segment g.
+struct G4Segments {
+  const GemmArgs& args;
+  int off_lane;
+  __device__ __forceinline__ G4Segments(const GemmArgs& a, int lane) : args(a), off_lane(0) {
+    if (a.offsets != nullptr && lane <= a.n_offsets) off_lane = a.offsets[lane];
+  }
+  __device__ __forceinline__ void get(const GemmGroup& gg, int& rb, int& re) const {
+    if (gg.row_begin >= 0) { rb = gg.row_begin; re = gg.row_end; }
+    else {
+      const int dyn = __builtin_amdgcn_readfirstlane(gg.dyn);
+      rb = __builtin_amdgcn_readlane(off_lane, dyn);
+      re = __builtin_amdgcn_readlane(off_lane, dyn + 1);
+    }
+  }
+};
+
+// A tile by its index inside a group of mtiles x ntiles: bands of GROUP_M m-tiles, a short remainder joins the last one.
+__device__ __forceinline__ void g4_raster(int L, int mtiles, int ntiles, int& m, int& n) {
+  const int nbands = max(1, (mtiles + GROUP_M / 2) / GROUP_M);
+  const int band = min(L / (GROUP_M * ntiles), nbands - 1);
+  const int first_m = band * GROUP_M;
+  const int gm = band == nbands - 1 ? mtiles - first_m : GROUP_M;
+  const int within = L - band * (GROUP_M * ntiles);
+  m = first_m + within % gm;
+  n = within / gm;
+}
+
+// What is left when every block has had the same number of whole tiles (`rounds`): `tiles` of them, each cut along K into
+// `parts` equal parts for blocks of their own; gemm4w_tail_kernel adds the parts up. parts = 1: not cut.
+struct G4Tail { int rounds, tiles, parts; };
+
+// Costs in units of one pair of K steps (2.0 us with most of the chip idle): a part takes its share of the pairs; leaving the
+// fp32 parts and adding them up costs a second launch (9 us) and their bytes written and read again (256 KiB per part of
+// a full tile, about 6 TB/s). A cut has to pay by a seventh. pairs: K step pairs of a tile; fill: rows / 256 of the
+// average tile.
+__host__ __device__ inline G4Tail g4_plan_tail(int total, int blocks, int pairs, int min_pairs, float fill) {
+  G4Tail t = {total / blocks, total % blocks, 1};
+  if (t.tiles == 0) return t;
+  float best = 0.85f * (float)pairs;
+  for (int p = 2; p <= G4_TAIL_MAX_PARTS && p * t.tiles <= blocks && pairs / p >= min_pairs; ++p) {
+    const float cost = (float)((pairs + p - 1) / p) + 4.5f + 0.04f * fill * (float)(p * t.tiles);
+    if (cost < best) { best = cost; t.parts = p; }
+  }
+  return t;
+}
+
+// The plan of a launch, from the segment sizes on the device; also its number of tiles.
+template <bool W8, int FEAT>
+__device__ __forceinline__ G4Tail g4_tail_of(const GemmArgs& args, const G4Segments& seg, int blocks) {
+  int total = 0;
+  long long rows = 0;
+  for (int g = 0; g < args.G; ++g) {
+    int rb, re;
+    seg.get(args.g[g], rb, re);
+    const int nt = args.g[g].n_out / FEAT;
+    total += ((re - rb + G4_BM - 1) / G4_BM) * nt;
+    rows += (long long)(re - rb) * nt;
+  }
+  if (args.tail == nullptr || total == 0) return {total / blocks, total % blocks, 1};
+  G4Tail t = g4_plan_tail(total, blocks, args.g[0].kbytes / (2 * BK), W8 ? 3 : 2, (float)rows / ((float)total * G4_BM));
+  t.parts = __builtin_amdgcn_readfirstlane(t.parts);   // the same for every lane, which floating point hides
+  return t;
+}
+
+template <bool F16, bool W8, int EPI>
+__global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm4w_kernel(const GemmArgs args) {
+#if defined(__HIP_DEVICE_COMPILE__)   // the host pass drops the stub of a kernel whose register operands it cannot parse
+  constexpr bool SWIGLU = EPI == G4_SWIGLU;
+  constexpr bool HAS_BIAS = EPI == G4_BIAS || EPI == G4_GELU;
+  constexpr int FEAT = SWIGLU ? 128 : 256;
+  constexpr int OUT_BYTES = EPI == G4_PARTIAL ? 4 : 2;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wq = wave & 1, wt = wave >> 1;
+  auto sgpr = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+
+  // ---- work items: as grouped_gemm_kernel's tiles --------------------------------------------------------------
+  // A wave's lanes look its block's next 64 items up at once and leave them in LDS (one by one, the decoding is a serial
+  // chain of integer divisions that the matrix cores would wait for at every tile).
+  const G4Segments segs(args, lane);
+  auto seg = [&](const GemmGroup& gg, int& rb, int& re) { segs.get(gg, rb, re); };
+  int plan_idx = 0;
+  if (EPI == G4_PARTIAL && args.plan.n > 1) {
+    int mt_dyn = 0, mt_static = 0;
+    for (int g = 0; g < args.G; ++g) {
+      int rb, re;
+      seg(args.g[g], rb, re);
+      (args.g[g].row_begin < 0 ? mt_dyn : mt_static) += (re - rb + args.plan.bm - 1) / args.plan.bm;
+    }
+    plan_idx = hdmoe_plan_pick(args.plan, mt_dyn, mt_static, args.g[0].n_out / FEAT);
+  }
+  auto parts_of = [&](const GemmGroup& gg) {
+    return EPI != G4_PARTIAL ? 1 : gg.row_begin < 0 ? args.plan.pd[plan_idx] : args.plan.ps[plan_idx];
+  };
+  // Whole rounds of tiles: each XCD (block ids congruent mod 8) takes a contiguous eighth of the tile list and its blocks
+  // take consecutive tiles, so the CUs of an XCD share operand tiles in their L2. The remainder (tail): the parts of
+  // one K range before those of the next, again consecutive inside an XCD. Groups of different K (`spread`) or cut by the
+  // caller's plan: every XCD takes its eighth of every group, longest tiles first.
+  const int xcd = blockIdx.x % HDMOE_NUM_XCD, slot = blockIdx.x / HDMOE_NUM_XCD;
+  const int nslots = gridDim.x / HDMOE_NUM_XCD;
+  const G4Tail tail = g4_tail_of<W8, FEAT>(args, segs, gridDim.x);
+  v4i* const table = reinterpret_cast<v4i*>(smem + G4_TABLE) + wave * G4_TABLE_ITEMS;
+  auto fill_table = [&](int base) {
+    const int i = base + lane;
+    const bool eighths = EPI == G4_PARTIAL || args.spread != 0;   // every group cut in eighths
+    int rem = slot + i * nslots, tail_part = 0, tail_slot = 0;
+    bool some = true;
+    if (!eighths) {
+      if (i < tail.rounds) {
+        rem = xcd * (tail.rounds * nslots) + slot + i * nslots;
+      } else {
+        const int units = tail.tiles * tail.parts, chunk = (units + HDMOE_NUM_XCD - 1) / HDMOE_NUM_XCD;
+        const int w = xcd * chunk + slot;
+        some = i == tail.rounds && slot < chunk && w < units;
+        const int t = some ? w % tail.tiles : 0;
+        tail_part = some ? w / tail.tiles : 0;
+        rem = tail.rounds * (int)gridDim.x + t;
+        tail_slot = tail.parts > 1 ? 1 + t * tail.parts + tail_part : 0;
+      }
+    }
+    int g_at = -1, mtiles = 1, ntiles = 1, L = 0, rb_at = 0, re_at = 0, parts = 1, kt = 0;
+    for (int k = 0; k < args.G; ++k) {
+      const int g = args.spread < 0 ? args.G - 1 - k : k;
+      const GemmGroup& gg = args.g[g];
+      int rb, re;
+      seg(gg, rb, re);
+      const int mt = (re - rb + G4_BM - 1) / G4_BM, nt = gg.n_out / FEAT, np = parts_of(gg);
+      const long long tiles = (long long)mt * nt * np;
+      const int lo = eighths ? (int)(xcd * tiles / HDMOE_NUM_XCD) : 0;
+      const int hi = eighths ? (int)((xcd + 1) * tiles / HDMOE_NUM_XCD) : (int)tiles;
+      if (some && g_at < 0) {
+        if (rem < hi - lo) { g_at = g; mtiles = mt; ntiles = nt; L = lo + rem; rb_at = rb; re_at = re; parts = np; kt = gg.kbytes / BK; }
+        else rem -= hi - lo;
+      }
+    }
+    v4i e = {-1, 0, 0, 0};
+    if (g_at >= 0) {
+      int part = L / (mtiles * ntiles), m, n;
+      g4_raster(L - part * (mtiles * ntiles), mtiles, ntiles, m, n);
+      const int row0 = rb_at + m * G4_BM;
+      // parts start on a pair of K steps
+      const int of = tail_slot > 0 ? tail.parts : parts, at = tail_slot > 0 ? tail_part : part;
+      const int kt0 = kt / 2 * at / of * 2, kt1 = kt / 2 * (at + 1) / of * 2;
+      e = v4i{g_at | part << 8 | min(re_at - row0, G4_BM) << 16, row0, n | tail_slot << 16, kt0 | (kt1 - kt0) << 16};
+    }
+    table[lane] = e;
+  };
+  // an item as its four packed words (scalar registers are scarce here)
+  struct Item {
+    int x, y, z, w;
+    __device__ __forceinline__ bool some() const { return x >= 0; }
+    __device__ __forceinline__ int g() const { return x & 255; }
+    __device__ __forceinline__ int part() const { return x >> 8 & 255; }
+    __device__ __forceinline__ int rows_here() const { return x >> 16; }
+    __device__ __forceinline__ int row0() const { return y; }
+    __device__ __forceinline__ int n0() const { return (z & 0xffff) * FEAT; }
+    __device__ __forceinline__ int slot() const { return z >> 16; }   // of a part of a tail tile, counted from 1
+    __device__ __forceinline__ int kt0() const { return w & 0xffff; }
+    __device__ __forceinline__ int nkt() const { return w >> 16; }
+  };
+  auto item = [&](int i) -> Item {
+    if (i > 0 && i % G4_TABLE_ITEMS == 0) fill_table(i);
+    const v4i e = table[i % G4_TABLE_ITEMS];
+    return Item{sgpr(e.x), sgpr(e.y), sgpr(e.z), sgpr(e.w)};
+  };
+
+  fill_table(0);
+  Item cur = item(0);
+  if (!cur.some()) return;   // block-uniform: every wave of the block leaves together
+  Item nxt = item(1), nx2 = nxt;
+  if (nxt.some()) nx2 = item(2);
+
+  // ---- addressing ---------------------------------------------------------------------------------------------
+  // A wave-level global->LDS load moves 8 rows of 128 bytes: lane i lands in 16-byte chunk (i & 7) of row (i >> 3) and
+  // fetches logical chunk (i & 7) ^ swz(row). Weight rows are placed so that the two 16-row MFMA tiles of a 32-row group
+  // give a lane 8 consecutive features: row r of tile t holds weight row (r >> 2) * 8 + t * 4 + (r & 3) of the group.
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
+  int ld_row = wave * 8 + (lane >> 3);                 // row within a 32-row slab
+  int ld_chunk = (lane & 7) ^ swz(ld_row);
+  int ld_wrow = ((ld_row & 15) >> 2) * 8 + (ld_row >> 4) * 4 + (ld_row & 3);
+  const int ldsw = sgpr((int)lds0 + wave * 1024);
+  int ldswb = sgpr(ldsw + G4_W_TILE);
+  const int fr_row = lane & 15, fr_grp = lane >> 4, fr_swz = swz(fr_row);
+
+  v32i fa0, fb0, ctx;      // slice 0 fragments of the tile about to start; addresses
+  v16i voff_nxt;           // row offsets of the next tile
+  v8i gi;                  // row indices of the tile after it
+#pragma unroll
+  for (int i = 0; i < 32; ++i) ctx[i] = 0;
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    ctx[G4_TOK_ADDR + ks] = (int)lds0 + (wt * 128 + fr_row) * 128 + ((ks * 4 + fr_grp) ^ fr_swz) * 16;
+    ctx[G4_W_ADDR + ks] = (int)lds0 + G4_W_TILE + (wq * 128 + fr_row) * 128 +
+                          (W8 ? ((ks * 2 + (fr_grp >> 1)) ^ fr_swz) * 16 + (fr_grp & 1) * 8 : ((ks * 4 + fr_grp) ^ fr_swz) * 16);
+  }
+  ctx[G4_BIAS_VOFF] = (wq * 128 + fr_grp * 8) * 2;
+  ctx[G4_DEF_LD] = ctx[G4_SCR_VOFF] = wave * (G4_SCRATCH / 4) + lane * 16;
+  ctx[G4_DEF_ST] = (int)0x80000000u;
+  struct Rsrc { uint64_t lo, hi; };
+  auto rsrc64 = [&](const void* p, uint32_t bytes) -> Rsrc {
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    const uint32_t a0 = sgpr((int)(uint32_t)a), a1 = sgpr((int)((uint32_t)(a >> 32) & 0xffffu)), b = sgpr((int)bytes);
+    return {(uint64_t)a1 << 32 | a0, (uint64_t)0x00020000u << 32 | b};
+  };
+  auto rsrc4 = [&](const void* p, uint32_t bytes) -> v4i {
+    const Rsrc r = rsrc64(p, bytes);
+    return v4i{(int)(uint32_t)r.lo, (int)(uint32_t)(r.lo >> 32), (int)(uint32_t)r.hi, (int)(uint32_t)(r.hi >> 32)};
+  };
+  // the operands of an item's loads: resources of tokens and weights, the lane's row offsets (gi: its row indices where the
+  // group gathers its tokens); rows past the end of the tile get an offset beyond the buffer and read as zeros
+  struct Source { Rsrc a, b0, b1; };
+  auto set_source = [&](const Item& d, const v8i& rows, v16i& voff) -> Source {
+    Source s = {{0, 0}, {0, 0}, {0, 0}};
+    if (!d.some()) return s;   // no further item: the requests still go out, against empty buffers (zeros)
+    const GemmGroup& gg = args.g[d.g()];
+    const int kb = gg.kbytes, wkb = W8 ? kb >> 1 : kb;
+    s.a = gg.gather != nullptr ? rsrc64(gg.a, (uint32_t)gg.a_rows * (uint32_t)kb)
+                               : rsrc64(gg.a + (size_t)d.row0() * kb, (uint32_t)d.rows_here() * (uint32_t)kb);
+    s.b0 = rsrc64(gg.b0 + (size_t)d.n0() * wkb, (uint32_t)FEAT * (uint32_t)wkb);
+    s.b1 = SWIGLU ? rsrc64(gg.b1 + (size_t)d.n0() * wkb, (uint32_t)FEAT * (uint32_t)wkb) : s.b0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int r = j * 32 + ld_row;
+      const int row = gg.gather != nullptr ? rows[j] >> gg.gather_shift : r;
+      voff[j] = r < d.rows_here() ? row * kb + ld_chunk * 16 : (int)0x80000000u;
+      voff[8 + j] = ((SWIGLU ? (j >> 2) * 64 + (j & 1) * 32 : j * 32) + ld_wrow) * wkb + ld_chunk * 16;
+    }
+    return s;
+  };
+  auto load_rows = [&](const Item& d) -> v8i {
+    v8i r = {0, 0, 0, 0, 0, 0, 0, 0};
+    const int32_t* const list = args.g[d.g()].gather;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (list != nullptr && j * 32 + ld_row < d.rows_here()) r[j] = list[d.row0() + j * 32 + ld_row];
+    return r;
+  };
+  auto w_start = [](const Item& d) { return W8 ? d.kt0() * (BK / 2) : d.kt0() * BK; };
+
+  Source src = set_source(cur, load_rows(cur), voff_nxt);
+#pragma unroll
+  for (int j = 0; j < 16; ++j) ctx[G4_TOK_VOFF + j] = voff_nxt[j];
+  // ---- the block's first two K steps (w8: weights of two pairs) as a burst --------------------------------------
+  {
+    const GemmGroup& gg = args.g[cur.g()];
+    const int kb = gg.kbytes, wkb = W8 ? kb >> 1 : kb;
+    const __amdgpu_buffer_rsrc_t pa = gg.gather != nullptr
+        ? make_rsrc(gg.a, (uint32_t)gg.a_rows * (uint32_t)kb)
+        : make_rsrc(gg.a + (size_t)cur.row0() * kb, (uint32_t)cur.rows_here() * (uint32_t)kb);
+    const __amdgpu_buffer_rsrc_t pb0 = make_rsrc(gg.b0 + (size_t)cur.n0() * wkb, (uint32_t)FEAT * (uint32_t)wkb);
+    const __amdgpu_buffer_rsrc_t pb1 = SWIGLU ? make_rsrc(gg.b1 + (size_t)cur.n0() * wkb, (uint32_t)FEAT * (uint32_t)wkb) : pb0;
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      uint8_t* const base = smem + st * G4_STAGE + wave * 1024;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(pa, (lds_ptr_t)(base + j * 4096), 16, ctx[G4_TOK_VOFF + j], (cur.kt0() + st) * BK, 0, 0);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds((j >> 1) & 1 ? pb1 : pb0, (lds_ptr_t)(base + G4_W_TILE + j * 4096), 16,
+                                                 ctx[G4_W_VOFF + j], w_start(cur) + st * BK, 0, 0);
+    }
+  }
+  gi = nxt.some() ? load_rows(nxt) : v8i{0, 0, 0, 0, 0, 0, 0, 0};
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  __syncthreads();
+  if constexpr (W8) asm volatile(HDMOE_G4_FILL_W8 : "={v[128:159]}"(fa0), "={v[160:191]}"(fb0), "+{v[96:127]}"(ctx) : : G4_CLOBBER_V);
+  else asm volatile(HDMOE_G4_FILL : "={v[128:159]}"(fa0), "={v[160:191]}"(fb0), "+{v[96:127]}"(ctx) : : "memory");
+
+  // per-tensor scales come through the scalar cache: a vector load would be waited for together with every global->LDS
+  // request in flight (one in-order counter)
+  typedef const __attribute__((address_space(4))) float* const_float_ptr;
+  auto scale = [&](const float* p) -> int {
+    return sgpr(__float_as_int(p != nullptr ? hdmoe_dev_round_bf16(*(const_float_ptr)(uintptr_t)p) : 1.0f));
+  };
+  // GELU: the tile whose activation is still to be applied (none: an empty buffer)
+  v4i dro = rsrc4(nullptr, 0);
+  int dldo = 0;
+  bool deferred = false;
+  const v4i scr = EPI == G4_GELU ? rsrc4(args.scratch + (size_t)blockIdx.x * G4_SCRATCH, G4_SCRATCH) : rsrc4(nullptr, 0);
+  const int gk = sgpr(__float_as_int(0.84932180f)), gp = sgpr(__float_as_int(0.3f / 0.84932180f));  // gen_gemm4w.py: k, 0.3 / k
+#define G4_DRAIN(TEXT)                                                                                               \
+  asm volatile(TEXT : "+{v[128:159]}"(fa0), "+{v[160:191]}"(fb0), "+{v[96:127]}"(ctx) : [dro] "s"(dro), [dldo] "s"(dldo), [dd] "s"(dd), [scr] "s"(scr), [gk] "s"(gk), [gp] "s"(gp) : G4_CLOBBER_V)
+  // Output offsets of the pieces: the second pair of K steps stores the first two of token block 1, so DEF_ST starts a step in
+  // front of them, at the last two of block 0, and advances by dd = dldo - 128 and 128 in turn.
+  auto drain = [&] {
+    const int dd = sgpr(dldo - 128);
+    if constexpr (EPI == G4_GELU && F16) G4_DRAIN(HDMOE_G4_DRAIN_F16);
+    else if constexpr (EPI == G4_GELU) G4_DRAIN(HDMOE_G4_DRAIN_BF16);
+  };
+
+  for (int i = 0;; ++i) {
+    const GemmGroup& gg = args.g[cur.g()];
+    // keep what depends on them out of registers that would live across the statement below
+    asm volatile("" : "+v"(ld_row), "+v"(ld_chunk), "+v"(ld_wrow));
+    const Source nsrc = set_source(nxt, gi, voff_nxt);
+    Item nx3 = nx2;
+    if (nx2.some()) nx3 = item(i + 3);
+    int n = sgpr(cur.nkt() >> 1), so = sgpr((cur.kt0() + 2) * BK), wso = sgpr(w_start(cur) + 2 * BK);
+    const int nso = sgpr(nxt.kt0() * BK), nwso = sgpr(w_start(nxt));
+    const int ldo = gg.n_out * OUT_BYTES, ldo16 = sgpr(16 * ldo);
+    int slot_u;   // in a scalar register for certain (the compiler drops the builtin where it finds the value uniform)
+    asm volatile("v_readfirstlane_b32 %0, %1" : "=s"(slot_u) : "v"(cur.slot()));
+    const bool part = EPI != G4_PARTIAL && slot_u > 0;   // of a tail tile: raw sums go to the slot's 256 KiB
+    const uint8_t* const out = EPI == G4_PARTIAL
+        ? reinterpret_cast<const uint8_t*>(gg.pout + (size_t)cur.part() * (size_t)args.part_stride + (size_t)cur.row0() * gg.n_out)
+        : gg.out + (size_t)cur.row0() * ldo;
+    const v4i ro = part ? rsrc4(args.tail + (size_t)(slot_u - 1) * (G4_BM * 256), G4_BM * 256 * 4)
+                        : rsrc4(out, (uint32_t)cur.rows_here() * (uint32_t)ldo);
+    ctx[G4_OUT_VOFF] = part ? wave * 65536 + lane * 16
+                            : (wt * 128 + fr_row) * ldo + (cur.n0() + wq * (FEAT / 2) + fr_grp * 8) * OUT_BYTES;
+    const int part_s = slot_u;
+    const int ntt = sgpr((cur.rows_here() - wt * 128 + 15) >> 4);
+    // row indices of nx2 and this tile's biases are loaded inside the statement
+    const int32_t* const list = nx2.some() ? args.g[nx2.g()].gather : nullptr;
+    const v4i gr = rsrc4(list != nullptr ? list + nx2.row0() : nullptr, list != nullptr ? (uint32_t)nx2.rows_here() * 4u : 0u);
+    ctx[G4_GATHER_VOFF] = ld_row * 4;
+    const bool with_bias = HAS_BIAS && gg.bias != nullptr;
+    const v4i br = rsrc4(with_bias ? gg.bias + cur.n0() : nullptr, with_bias ? 512u : 0u);
+    const int sc = W8 ? scale(gg.sb0) : 0, su = W8 && SWIGLU ? scale(gg.sb1) : 0;
+    if (EPI == G4_GELU && deferred && n < G4_GELU_PAIRS) {
+      drain();
+      dro = rsrc4(nullptr, 0);
+      deferred = false;
+    }
+    int dn = sgpr(14), dd = sgpr(dldo - 128);
+#define G4_TILE(TEXT)                                                                                                \
+    asm volatile(TEXT : "+{v[128:159]}"(fa0), "+{v[160:191]}"(fb0), "+{v[96:127]}"(ctx), "={v[72:79]}"(gi),          \
+                        [n] "+s"(n), [so] "+s"(so), [wso] "+s"(wso), [ldswb] "+s"(ldswb), [dn] "+s"(dn), [dd] "+s"(dd) \
+                 : "{v[80:95]}"(voff_nxt), [r0] "s"(src.a.lo), [r1] "s"(src.a.hi), [r2] "s"(src.b0.lo),              \
+                   [r3] "s"(src.b0.hi), [r4] "s"(src.b1.lo), [r5] "s"(src.b1.hi), [nr0] "s"(nsrc.a.lo), [nr1] "s"(nsrc.a.hi),             \
+                   [nr2] "s"(nsrc.b0.lo), [nr3] "s"(nsrc.b0.hi), [nr4] "s"(nsrc.b1.lo), [nr5] "s"(nsrc.b1.hi),       \
+                   [nso] "s"(nso), [nwso] "s"(nwso), [ldsw] "s"(ldsw), [ro] "s"(ro), [ldo16] "s"(ldo16),             \
+                   [gr] "s"(gr), [br] "s"(br), [sc] "s"(sc), [su] "s"(su), [dro] "s"(dro), [dldo] "s"(dldo),         \
+                   [scr] "s"(scr), [gk] "s"(gk), [gp] "s"(gp), [ntt] "s"(ntt), [part] "s"(part_s)                    \
+                 : G4_CLOBBER)
+#define G4_TILE_OR_PART(LOOP, EPILOGUE)                                                                              \
+    G4_TILE(LOOP "s_cmp_lg_u32 %[part], 0\ns_cbranch_scc1 41f\n" EPILOGUE "s_branch 42f\n41:\n" HDMOE_G4_EPI_PART "42:\n")
+    if constexpr (EPI == G4_GELU && F16) { G4_TILE_OR_PART(HDMOE_G4_LOOP_F16_GELU, HDMOE_G4_EPI_F16_GELU); }
+    else if constexpr (EPI == G4_GELU) { G4_TILE_OR_PART(HDMOE_G4_LOOP_BF16_GELU, HDMOE_G4_EPI_BF16_GELU); }
+    else if constexpr (EPI == G4_BIAS && F16) { G4_TILE_OR_PART(HDMOE_G4_LOOP_F16_BIAS, HDMOE_G4_EPI_F16_BIAS); }
+    else if constexpr (EPI == G4_BIAS && W8) { G4_TILE_OR_PART(HDMOE_G4_LOOP_BF16_W8_BIAS, HDMOE_G4_EPI_BF16_W8_BIAS); }
+    else if constexpr (EPI == G4_BIAS) { G4_TILE_OR_PART(HDMOE_G4_LOOP_BF16_BIAS, HDMOE_G4_EPI_BF16_BIAS); }
+    else if constexpr (EPI == G4_SWIGLU && W8) { G4_TILE_OR_PART(HDMOE_G4_LOOP_BF16_W8, HDMOE_G4_EPI_SWIGLU_W8); }
+    else if constexpr (EPI == G4_SWIGLU) { G4_TILE_OR_PART(HDMOE_G4_LOOP_BF16, HDMOE_G4_EPI_SWIGLU); }
+    else if constexpr (EPI == G4_PARTIAL && W8) G4_TILE(HDMOE_G4_LOOP_BF16_W8 HDMOE_G4_EPI_PARTIAL);
+    else if constexpr (EPI == G4_PARTIAL) G4_TILE(HDMOE_G4_LOOP_BF16 HDMOE_G4_EPI_PARTIAL);
+    else if constexpr (W8) { G4_TILE_OR_PART(HDMOE_G4_LOOP_BF16_W8, HDMOE_G4_EPI_BF16_W8); }
+    else { G4_TILE_OR_PART(HDMOE_G4_LOOP_BF16, HDMOE_G4_EPI_BF16); }
+    if (EPI == G4_GELU && !part) {
+      dro = ro;
+      dldo = ldo16;
+      deferred = true;
+      ctx[G4_DEF_LD] = ctx[G4_SCR_VOFF];
+      ctx[G4_DEF_ST] = ctx[G4_OUT_VOFF] + 128;
+    }
+    if (!nxt.some()) break;
+    src = nsrc;
+    cur = nxt;
+    nxt = nx2;
+    nx2 = nx3;
+  }
+  if (deferred) drain();
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // the empty requests of the last pair have come back before the LDS is given up
+#endif
+}
+
+// Adds the parts of the tail tiles up (in order) and finishes them as the epilogues of gen_gemm4w.py do. One thread: one
+// token, 8 consecutive features. Bound by the fp32 sums read (256 KiB per part).
+template <bool F16, bool W8, int EPI>
+__global__ __launch_bounds__(256) void gemm4w_tail_kernel(const GemmArgs args, int blocks) {
+  constexpr bool SWIGLU = EPI == G4_SWIGLU;
+  constexpr int FEAT = SWIGLU ? 128 : 256;
+  using Act = std::conditional_t<F16, HdmoeF16, HdmoeBf16>;
+  const int lane = threadIdx.x & 63;
+  const G4Segments seg(args, lane);
+  const G4Tail tail = g4_tail_of<W8, FEAT>(args, seg, blocks);
+  if (tail.parts <= 1) return;
+  constexpr int PER_TILE = SWIGLU ? 16 : 32;   // blocks' worth of work of a tile
+  for (int item = blockIdx.x; item < tail.tiles * PER_TILE; item += gridDim.x) {
+    const int t = item / PER_TILE;
+    int L = __builtin_amdgcn_readfirstlane(tail.rounds * blocks + t), g = 0, m = 0, n = 0, rb = 0, re = 0;
+    for (; g < args.G; ++g) {
+      seg.get(args.g[g], rb, re);
+      const int mt = (re - rb + G4_BM - 1) / G4_BM, nt = args.g[g].n_out / FEAT;
+      if (L < mt * nt) { g4_raster(L, mt, nt, m, n); break; }
+      L -= mt * nt;
+    }
+    const GemmGroup& gg = args.g[g];
+    const int row0 = rb + m * G4_BM, rows_here = min(re - row0, G4_BM);
+    // the wave's order of gen_gemm4w.py: MFMA tile (tt, ft) of wave w at ((w * 64) + tt * 8 + ft) KiB; ft 2q and 2q + 1 hold
+    // the 8 features
+    const int unit = item % PER_TILE * 4 + (threadIdx.x >> 6);
+    const int q = unit & (SWIGLU ? 1 : 3), tt = (unit >> (SWIGLU ? 1 : 2)) & 7, w = unit >> (SWIGLU ? 4 : 5);
+    const int wq = w & 1, wt = w >> 1;
+    const int row = wt * 128 + tt * 16 + (lane & 15);
+    if (row >= rows_here) continue;
+    const float* src = args.tail + (size_t)t * tail.parts * (G4_BM * 256) + w * 16384 + (tt * 8 + q * 2) * 256 + lane * 4;
+    constexpr int QUADS = SWIGLU ? 4 : 2;
+    float4 s[QUADS];
+#pragma unroll
+    for (int i = 0; i < QUADS; ++i) s[i] = *reinterpret_cast<const float4*>(src + (i & 1) * 256 + (i >> 1) * 1024);
+    for (int p = 1; p < tail.parts; ++p) {
+      src += G4_BM * 256;
+#pragma unroll
+      for (int i = 0; i < QUADS; ++i) {
+        const float4 v = *reinterpret_cast<const float4*>(src + (i & 1) * 256 + (i >> 1) * 1024);
+        s[i].x += v.x; s[i].y += v.y; s[i].z += v.z; s[i].w += v.w;
+      }
+    }
+    float v[8] = {s[0].x, s[0].y, s[0].z, s[0].w, s[1].x, s[1].y, s[1].z, s[1].w};
+    const int feat = n * FEAT + wq * (FEAT / 2) + q * 32 + (lane >> 4) * 8;
+    auto scale = [](const float* p) { return p != nullptr ? hdmoe_dev_round_bf16(*p) : 1.0f; };
+    if constexpr (SWIGLU) {
+      const float u[8] = {s[2].x, s[2].y, s[2].z, s[2].w, s[3].x, s[3].y, s[3].z, s[3].w};
+      const float sg = W8 ? scale(gg.sb0) : 1.0f, su = W8 ? scale(gg.sb1) : 1.0f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float h1 = hdmoe_dev_round_bf16(v[i] * sg), h3 = hdmoe_dev_round_bf16(u[i] * su);
+        v[i] = hdmoe_dev_round_bf16(h1 * __builtin_amdgcn_rcpf(1.0f + __expf(-h1))) * h3;
+      }
+    } else {
+      const float sc = W8 ? scale(gg.sb0) : 1.0f;
+      float b[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+      if (gg.bias != nullptr) {
+        const uint4 bw = *reinterpret_cast<const uint4*>(gg.bias + feat);
+        const uint32_t words[4] = {bw.x, bw.y, bw.z, bw.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { b[2 * i] = Act::lo(words[i]); b[2 * i + 1] = Act::hi(words[i]); }
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        v[i] = W8 ? __builtin_fmaf(v[i], sc, b[i]) : v[i] + b[i];
+        if constexpr (EPI == G4_GELU) {
+          const float h = Act::round(v[i]);
+          v[i] = 0.5f * h * (1.0f + erff(h * 0.70710678118654752440f));
+        }
+      }
+    }
+    uint4 o;
+    o.x = Act::pack(v[0], v[1]); o.y = Act::pack(v[2], v[3]); o.z = Act::pack(v[4], v[5]); o.w = Act::pack(v[6], v[7]);
+    *reinterpret_cast<uint4*>(gg.out + ((size_t)(row0 + row) * gg.n_out + feat) * 2) = o;
+  }
+}
+
+// Whether the launch fits gemm4w_kernel: whole pairs of K steps in every part, at least two of them (w8: three), operands
+// under 2 GiB.
+inline bool gemm4w_fits(const GemmArgs& args, bool w8, long long max_operand_bytes) {
+  if (args.G <= 0) return false;
+  for (int g = 0; g < args.G; ++g) {
+    const int pairs = args.g[g].kbytes / (2 * BK);
+    int parts = 1;
+    if (args.nparts > 1)
+      for (int i = 0; i < args.plan.n; ++i) parts = max(parts, args.g[g].row_begin < 0 ? args.plan.pd[i] : args.plan.ps[i]);
+    if (args.g[g].kbytes % (2 * BK) != 0 || pairs / parts < (w8 ? 3 : 2) || args.g[g].kbytes / BK > 0x7fff) return false;
+  }
+  return max_operand_bytes < (1ll << 31);
+}

@@ -1,0 +1,481 @@
+#!/usr/bin/env python3
+"""Writes gemm4w_asm.inc: the assembly of the 4-wave 16-bit GEMM (gemm4w.h). Run by the build.
+
+    python comfyui_amd/csrc/gen_gemm4w.py [output file]
+
+One wave per SIMD (4 waves, 512 registers each) on a 256-token x 256-weight-row tile, wave tile 128 x 128 of
+v_mfma_f32_16x16x32. A K step is 64 elements (128 bytes per token row) through two LDS stages. The fragments of both
+32-element slices of a step have registers of their own, so a stage has been read for good after about a third of its
+step, and the global->LDS loads of the step after the next go into it from there on: they have about 1.4 steps to
+arrive. Two barriers per step: everyone has read this stage; everyone's loads of the next one have landed. One statement
+holds the K loop and the epilogue of a tile, so that no accumulator crosses compiled code.
+
+Weights of one byte (w8: e4m3fn) are loaded by the pair of K steps (128 bytes per row), read 8 bytes per lane and
+converted to bf16 on the way to the matrix cores (exact), 64 conversions beside the 128 MFMAs of a step.
+
+GELU: an epilogue leaves the rounded sums of a tile in a scratch buffer of the block's own (it stays in the caches); while
+the next tile multiplies, the wave reads them back 16 bytes per lane at a time, applies the activation and stores the
+outputs, one piece per K step behind the MFMAs.
+
+Register map (per wave):
+  a[0:255]    accumulators acc[ft][tt] = a[(8*ft + tt)*4 : +3], ft: 16 weight rows, tt: 16 tokens
+  v[128:159]  token fragments of slice 0, v[160:191] weight fragments of slice 0 (4 registers each, tt / ft ascending)
+  v[192:223]  token fragments of slice 1, v[224:255] weight fragments of slice 1; work registers of the epilogue
+  v[96:127]   addresses (CTX below)
+  v[80:95]    row offsets of the next tile, v[72:79] row indices of the tile after the next
+  v[34:71]    work registers of the K loop
+  s[64:75]    buffer resources of the loads: tokens, weights (rows 0-63 and 64-127 of either half)
+  v[0:33]     left to the compiler
+"""
+import os
+import sys
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+OUT = os.path.join(HERE, "gemm4w_asm.inc")
+
+CTX = 96
+TOK_ADDR = [CTX + 0, CTX + 1]                     # LDS address of the lane's token fragment, per slice
+W_ADDR = [CTX + 2, CTX + 3]                       # same for weights; w8: per slice of the even step (the odd one flips bit 6)
+TOK_VOFF = [CTX + 4 + j for j in range(8)]        # global byte offset of the lane's row of token slab j
+W_VOFF = [CTX + 12 + j for j in range(8)]         # same for weight slab j
+OUT_VOFF = CTX + 20                               # output byte offset of the lane: its token, its 8 features of group 0
+ROW_VOFF = CTX + 21                               # running copy of it
+GATHER_VOFF = CTX + 22                            # byte offset of the lane's entry of slab 0 in the row index list
+BIAS_VOFF = CTX + 23                              # byte offset of the lane's first bias of the tile
+DEF_LD, DEF_ST = CTX + 24, CTX + 25               # GELU: offset in the scratch of the piece read back, in the output of the one stored
+SCR_VOFF = CTX + 26                               # GELU: the lane's offset in the scratch
+NEXT = 80                                         # v[80:95]: TOK_VOFF and W_VOFF of the next tile
+GATHER = 72                                       # v[72:79]
+BIAS = 56                                         # v[56:71]: 8 quads of 16-bit biases
+PIECE = [34, 38]                                  # GELU: pieces read back, by step parity
+RES = 42                                          # GELU: finished piece
+TMP = 46                                          # GELU: v[46:55]
+RAW = 40                                          # w8: v[40:55] weight bytes of a slice, 2 registers per ft
+STAGE = 32768                                     # bytes of one stage of the token tile = of the weight tile
+W_TILE = 65536                                    # LDS: [tok 0 | tok 1 | w 0 | w 1]
+FRAG = {("a", 0): 128, ("b", 0): 160, ("a", 1): 192, ("b", 1): 224}
+MFMA = {"BF16": "v_mfma_f32_16x16x32_bf16", "F16": "v_mfma_f32_16x16x32_f16"}
+PK = {"BF16": "v_cvt_pk_bf16_f32", "F16": "v_cvt_pk_f16_f32"}
+
+# positions (MFMA index within a slice) of the events of a step
+READ1_AT = 0        # slice 0: first read of slice 1
+FREE_AT = 24        # slice 0: the stage has been read; barrier
+LOAD_AT = 25        # first load of the step after the next, and MFMAs between two loads
+LOAD_EVERY = 6
+LAND_AT = 32        # slice 1: the next stage has landed; barrier, then the reads of slice 0 of the next step
+CVT1_AT = 26        # w8, slice 0: first conversion of slice 1
+PIECE_ST_AT, PIECE_LD_AT = 57, 60                 # GELU, slice 0
+
+
+def quad(b):
+    return f"v[{b}:{b + 3}]"
+
+
+def reads(stage, ks, w8, odd):
+    """The 16 fragment reads of a slice, in the order the MFMAs want them."""
+    order = [("b", 0)] + [("a", t) for t in range(8)] + [("b", f) for f in range(1, 8)]
+    if w8:
+        order.sort(key=lambda o: o[0] == "a")     # the weights have to be converted
+    out = []
+    for kind, i in order:
+        if kind == "b" and w8:
+            # 16 rows of 128 bytes per ft; odd steps read the upper 64 bytes of a row (the swizzle is an xor, so the
+            # address of the upper half is the lower one's with bit 6 flipped: a second address register)
+            out.append(f"ds_read_b64 v[{RAW + 2 * i}:{RAW + 2 * i + 1}], v{W_ADDR[ks]} offset:{2048 * i}")
+        else:
+            out.append(f"ds_read_b128 {quad(FRAG[(kind, ks)] + 4 * i)}, v{(TOK_ADDR if kind == 'a' else W_ADDR)[ks]} "
+                       f"offset:{stage * STAGE + 2048 * i}")
+    return out
+
+
+def token_loads(stage):
+    return [(f"s_add_u32 m0, %[ldsw], {stage * STAGE + j * 4096}",
+             f"buffer_load_dwordx4 v{TOK_VOFF[j]}, s[64:67], %[so] offen lds") for j in range(8)]
+
+
+def weight_loads(stage, w8):
+    out = []
+    for j in range(8):
+        rs = "s[68:71]" if (j // 2) % 2 == 0 else "s[72:75]"
+        m0 = f"s_add_u32 m0, %[ldswb], {j * 4096}" if w8 else f"s_add_u32 m0, %[ldsw], {W_TILE + stage * STAGE + j * 4096}"
+        out.append((m0, f"buffer_load_dwordx4 v{W_VOFF[j]}, {rs}, {'%[wso]' if w8 else '%[so]'} offen lds"))
+    return out
+
+
+def mfma_order():
+    o = []
+    for ft in range(8):
+        o += [(ft, tt) for tt in (range(8) if ft % 2 == 0 else range(7, -1, -1))]
+    return o
+
+
+def unpack(dt, dst, src, hi):
+    if dt == "BF16":
+        return f"v_and_b32 v{dst}, 0xffff0000, {src}" if hi else f"v_lshlrev_b32 v{dst}, 16, {src}"
+    return f"v_cvt_f32_f16_sdwa v{dst}, {src} dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_{int(hi)}"
+
+
+# Q(a) = 1 - Phi(a) = exp(-a^2 / 2) * P(t), t = 1 / (1 + 0.3 a): coefficients of t^1 .. t^8, fitted here to
+# erfcx(a / sqrt 2) / 2 on [0, 14] (relative error 1.5e-7, 7e-7 when evaluated in fp32)
+GELU_P = 0.3        # gemm4w.h passes gk and gp = 0.3 / gk
+GELU_C = [0.1196293, 0.12075395, 0.09991351, 0.12856157, -0.05368355, 0.2063534, -0.15720303, 0.03567476]
+
+
+def f32(v):
+    import struct
+    return "0x%08x" % struct.unpack("<I", struct.pack("<f", v))[0]
+
+
+def gelu_words(dt, src, dst, n):
+    """gelu(x) = (x + |x|) / 2 - |x| Q(|x|) of n packed words src.. -> dst.., two values at a time in the work registers
+    TMP..TMP+9: list of (instruction, cycles). No cancellation, so the negative tail keeps its digits; infinities and NaN
+    come out as 0.5 x (1 + erf) has them (the legacy product takes 0 * inf as 0). |x| is carried as a = k |x|,
+    k^2 = log2(e) / 2, so that exp(-x^2 / 2) is one square and one exp2; the factor is folded into the other constants."""
+    k = (0.5 * 1.4426950408889634) ** 0.5
+    c = [v / k for v in GELU_C]
+    o = []
+    for w in range(n):
+        x, a, d, e, p = ((TMP + i, TMP + 5 + i) for i in range(5))
+
+        def both(f, cyc=4):
+            o.extend((f(i), cyc) for i in range(2))
+        both(lambda i: unpack(dt, x[i], f"v{src + w}", i == 1))
+        both(lambda i: f"v_mul_f32 v{a[i]}, |v{x[i]}|, %[gk]")
+        both(lambda i: f"v_fma_f32 v{d[i]}, v{a[i]}, %[gp], 1.0")
+        both(lambda i: f"v_rcp_f32 v{d[i]}, v{d[i]}", 16)
+        both(lambda i: f"v_mul_f32 v{e[i]}, v{a[i]}, v{a[i]}")
+        both(lambda i: f"v_exp_f32 v{e[i]}, -v{e[i]}", 16)
+        both(lambda i: f"v_mul_f32 v{p[i]}, {f32(c[7])}, v{d[i]}")
+        both(lambda i: f"v_add_f32 v{p[i]}, {f32(c[6])}, v{p[i]}")
+        for v in reversed(c[:6]):
+            both(lambda i: f"v_fmaak_f32 v{p[i]}, v{p[i]}, v{d[i]}, {f32(v)}")
+        both(lambda i: f"v_mul_f32 v{p[i]}, v{p[i]}, v{d[i]}")
+        both(lambda i: f"v_mul_f32 v{p[i]}, v{p[i]}, v{e[i]}")
+        both(lambda i: f"v_mul_legacy_f32 v{p[i]}, v{p[i]}, v{a[i]}")
+        both(lambda i: f"v_add_f32 v{x[i]}, v{x[i]}, |v{x[i]}|")
+        both(lambda i: f"v_fma_f32 v{x[i]}, v{x[i]}, 0.5, -v{p[i]}")
+        o.append((f"{PK[dt]} v{dst + w}, v{x[0]}, v{x[1]}", 4))
+    return o
+
+
+class Feeder:
+    """Hands instructions out evenly over a number of places."""
+    def __init__(self, ops, places):
+        self.ops, self.pos, self.spent, self.given = ops, 0, 0, 0.0
+        self.share = sum(c for _, c in ops) / max(1, places)
+
+    def take(self):
+        out = []
+        self.given += self.share
+        while self.pos < len(self.ops) and self.spent < self.given - 1e-9:
+            out.append(self.ops[self.pos][0])
+            self.spent += self.ops[self.pos][1]
+            self.pos += 1
+        return out
+
+    def done(self):
+        return self.pos == len(self.ops)
+
+
+def conversions(ks):
+    """w8: the slice's weight bytes to bf16, in the order of the reads."""
+    o = []
+    for ft in range(8):
+        for h in range(4):
+            o.append((f"v_cvt_scalef32_pk_bf16_fp8 v{FRAG[('b', ks)] + 4 * ft + h}, v{RAW + 2 * ft + h // 2}, 1.0"
+                      + (" op_sel:[1,0,0]" if h % 2 else ""), 4))
+    return o
+
+
+def requests(w8, gelu, stage, first=False):
+    """The vector-memory requests of a step out of `stage` (first: of a tile's first pair) as (position, kind), position =
+    MFMA index over both slices."""
+    n = 8 if w8 and stage == 0 else 16
+    out = [(LOAD_AT + j * LOAD_EVERY, "t" if j < 8 else "w") for j in range(n)]
+    if gelu:
+        out += ([] if first else [(PIECE_ST_AT, "s")]) + [(PIECE_LD_AT, "l")]
+    return sorted(out)
+
+
+def young(w8, gelu, stage, first):
+    """How many vector-memory requests may still be out when the next step's operands must have landed (requests return in
+    order): those issued after the last one that is needed. Needed: the tokens (16-bit weights too) requested a step ago and
+    the piece read back then; one-byte weights were requested two steps ago or earlier."""
+    before = [k for p, k in requests(w8, gelu, stage, first) if p < 64 + LAND_AT]
+    last = [k for _, k in requests(w8, gelu, stage ^ 1)]
+    need = {"t", "l"} | (set() if w8 else {"w"})
+    after = 0
+    for k in reversed(last):
+        if k in need:
+            break
+        after += 1
+    return after + len(before)
+
+
+def step(dt, w8, gelu, stage, first):
+    """One K step out of `stage`. Entry: the reads of its slice 0 are in flight (lgkmcnt; w8: converted). first: of
+    a tile's first pair, whose step 0 starts the accumulators from zero and which has no finished piece to store."""
+    L = []
+    order = mfma_order()
+    # w8: the even step's slice 1 and the odd step's slice 0 read the same weight stage; the next even step's slice 0 reads
+    # the other one (W_ADDR is flipped between the pairs)
+    rd1 = reads(stage, 1, w8, stage)
+    rd0 = reads(stage ^ 1, 0, w8, stage ^ 1)
+    ld = token_loads(stage) + ([] if w8 and stage == 0 else weight_loads(stage, w8))
+    cvt0_at = LAND_AT + 14
+    cvt1, cvt0 = Feeder(conversions(1) if w8 else [], 64 - CVT1_AT), Feeder(conversions(0) if w8 else [], 64 - cvt0_at)
+    # the piece read back a step ago, in two parts around the end of the step (words n_b.. of the one before that first)
+    n_b = 2
+    half_b = Feeder(gelu_words(dt, PIECE[stage ^ 1], RES, n_b) if gelu else [], 64 - LAND_AT)
+    half_a = Feeder(gelu_words(dt, PIECE[stage] + n_b, RES + n_b, 4 - n_b) if gelu else [], PIECE_ST_AT)
+    assert FREE_AT <= LOAD_AT and LOAD_AT + 15 * LOAD_EVERY < 128
+    for q in range(128):
+        ks, i = divmod(q, 64)
+        ft, tt = order[i]
+        if q == 0:
+            L.append("s_waitcnt lgkmcnt(0)")
+        k = q - LOAD_AT
+        now = ld[k // LOAD_EVERY] if k >= 0 and k % LOAD_EVERY == 0 and k // LOAD_EVERY < len(ld) else None
+        if now:
+            L.append(now[0])
+        acc = f"a[{(8 * ft + tt) * 4}:{(8 * ft + tt) * 4 + 3}]"
+        c = "0" if first and stage == 0 and ks == 0 else acc
+        L.append(f"{MFMA[dt]} {acc}, {quad(FRAG[('b', ks)] + 4 * ft)}, {quad(FRAG[('a', ks)] + 4 * tt)}, {c}")
+        if now:
+            L.append(now[1])
+        if ks == 0:
+            if 0 <= i - READ1_AT < 16:
+                L.append(rd1[i - READ1_AT])
+            if i == FREE_AT - 1:
+                L += ["s_waitcnt lgkmcnt(0)", "s_barrier"]
+            if w8 and i >= CVT1_AT:
+                L += cvt1.take()
+            if gelu and i < PIECE_ST_AT:
+                L += half_a.take()
+            if gelu and i == PIECE_ST_AT:
+                assert half_a.done()
+            if gelu and i == PIECE_ST_AT and not first:
+                L.append(f"buffer_store_dwordx4 {quad(RES)}, v{DEF_ST}, %[dro], 0 offen offset:{64 * stage}")
+            if gelu and i == PIECE_LD_AT:
+                L.append(f"buffer_load_dwordx4 {quad(PIECE[stage])}, v{DEF_LD}, %[scr], 0 offen offset:{1024 * stage}")
+        else:
+            if i == LAND_AT - 1:
+                L += [f"s_waitcnt vmcnt({young(w8, gelu, stage, first)})", "s_barrier"]
+                if w8 and stage == 1:   # the next pair's weights
+                    L += [f"v_xor_b32 v{r}, {hex(STAGE)}, v{r}" for r in W_ADDR]
+                if w8:                  # the other 64 bytes of the rows
+                    L += [f"v_xor_b32 v{r}, 64, v{r}" for r in W_ADDR]
+            if 0 <= i - LAND_AT < 16:
+                L.append(rd0[i - LAND_AT])
+            if w8 and i == cvt0_at - 1:   # the weight bytes are there, the tokens may still be under way
+                L.append(f"s_waitcnt lgkmcnt({min(8, cvt0_at - LAND_AT - 8)})")
+            if w8 and i >= cvt0_at:
+                L += cvt0.take()
+            if gelu and i >= LAND_AT:
+                L += half_b.take()
+    assert half_b.done() and cvt0.done() and cvt1.done()
+    L.append("s_add_u32 %[so], %[so], 128")
+    return L
+
+
+def pair(dt, w8, gelu, first):
+    L = []
+    if gelu and not first:
+        # pieces 2p, 2p + 1: the pair of K steps p (0..13) reads them back, pair p + 1 stores them (64 bytes per token each)
+        L += [f"v_add_u32 v{DEF_LD}, 0x800, v{DEF_LD}", f"v_add_u32 v{DEF_ST}, %[dd], v{DEF_ST}", "s_sub_u32 %[dd], %[dldo], %[dd]",
+              "s_sub_u32 %[dn], %[dn], 1", "s_cmp_ge_i32 %[dn], 0", "s_cbranch_scc1 21f", f"v_mov_b32 v{DEF_ST}, 0x80000000", "21:"]
+    L += step(dt, w8, gelu, 0, first) + step(dt, w8, gelu, 1, first)
+    if w8:   # the weight stage of the pair after the next is this pair's
+        L += [f"s_xor_b32 %[ldswb], %[ldswb], {hex(STAGE)}", "s_add_u32 %[wso], %[wso], 128"]
+    return L
+
+
+def k_loop(dt, w8, gelu, bias):
+    """All K steps of a tile in pairs, %[n] of them (at least 2, w8: 3). Before the last pair the loads turn to the first
+    two steps of the next tile; the row indices of the tile after it and this tile's biases are requested there too. w8:
+    the weights of a pair are requested two pairs ahead, so they turn a pair earlier. The wait states at the end cover
+    the distance between the last MFMA and the first read of an accumulator."""
+    L = [f"s_mov_b64 s[{64 + 2 * i}:{65 + 2 * i}], %[r{i}]" for i in range(6)]
+    L += pair(dt, w8, gelu, True) + ["s_sub_u32 %[n], %[n], 1", "11:"]
+    wswitch = [f"s_mov_b64 s[{64 + 2 * i}:{65 + 2 * i}], %[nr{i}]" for i in range(2, 6)]
+    wswitch += [f"v_mov_b32 v{W_VOFF[j]}, v{NEXT + 8 + j}" for j in range(8)]
+    if w8:
+        L += ["s_cmp_eq_u32 %[n], 2", "s_cbranch_scc1 15f", "16:"]
+    L += ["s_cmp_eq_u32 %[n], 1", "s_cbranch_scc1 13f", "14:"]
+    L += pair(dt, w8, gelu, False)
+    L += ["s_sub_u32 %[n], %[n], 1", "s_cmp_lg_u32 %[n], 0", "s_cbranch_scc1 11b", "s_branch 12f"]
+    L += ["13:", "s_mov_b64 s[64:65], %[nr0]", "s_mov_b64 s[66:67], %[nr1]", "s_mov_b32 %[so], %[nso]"]
+    L += [f"v_mov_b32 v{TOK_VOFF[j]}, v{NEXT + j}" for j in range(8)]
+    if not w8:
+        L += wswitch
+    L += [f"buffer_load_dword v{GATHER + j}, v{GATHER_VOFF}, %[gr], 0 offen offset:{128 * j}" for j in range(8)]
+    if bias:
+        L += [f"buffer_load_dwordx2 v[{BIAS + 2 * ft}:{BIAS + 2 * ft + 1}], v{BIAS_VOFF}, %[br], 0 offen "
+              f"offset:{(ft >> 1) * 64 + (ft & 1) * 8}" for ft in range(8)]
+    L += ["s_branch 14b"]
+    if w8:
+        L += ["15:"] + wswitch + ["s_mov_b32 %[wso], %[nwso]", "s_branch 16b"]
+    return L + ["12:", "s_nop 15"]
+
+
+def out_row(tt):
+    return [f"v_add_u32 v{ROW_VOFF}, %[ldo16], v{ROW_VOFF}"] if tt else [f"v_mov_b32 v{ROW_VOFF}, v{OUT_VOFF}"]
+
+
+def epilogue(dt, w8, bias, gelu):
+    """acc (* scale) (+ bias) rounded to 16 bits, 8 consecutive features (16 bytes) per lane and store, 64 bytes per token.
+    v[192:223]: the lane's 32 biases, v[224:255] work. gelu: the first token block is activated at once, the others are
+    left to the next tile's K loop."""
+    L = []
+    if bias:
+        for ft in range(8):
+            for h in range(4):
+                L.append(unpack(dt, 192 + ft * 4 + h, f"v{BIAS + 2 * ft + h // 2}", h % 2))
+    n = 0
+    if gelu:
+        L.append(f"v_mov_b32 v{DEF_LD}, v{SCR_VOFF}")
+    for tt in range(8):
+        L += out_row(tt) if not (gelu and tt) else []
+        for g in range(4):
+            w = 224 + 16 * (n % 2)          # 8 values, then 4 packed words
+            o = w + 8
+            n += 1
+            for p in range(2):
+                for e in range(4):
+                    L.append(f"v_accvgpr_read_b32 v{w + p * 4 + e}, a{(8 * (2 * g + p) + tt) * 4 + e}")
+            for p in range(2):
+                for e in range(4):
+                    v, b = w + p * 4 + e, 192 + (2 * g + p) * 4 + e
+                    if w8 and bias:
+                        L.append(f"v_fma_f32 v{v}, v{v}, %[sc], v{b}")
+                    elif w8:
+                        L.append(f"v_mul_f32 v{v}, %[sc], v{v}")
+                    elif bias:
+                        L.append(f"v_add_f32 v{v}, v{b}, v{v}")
+            for q in range(4):
+                L.append(f"{PK[dt]} v{o + q}, v{w + 2 * q}, v{w + 2 * q + 1}")
+            if gelu and tt == 0:
+                L += [i for i, _ in gelu_words(dt, o, o, 4)]
+            if gelu and tt:
+                L.append(f"buffer_store_dwordx4 {quad(o)}, v{DEF_LD}, %[scr], 0 offen offset:{1024 * g}")
+            else:
+                L.append(f"buffer_store_dwordx4 {quad(o)}, v{ROW_VOFF}, %[ro], 0 offen offset:{64 * g}")
+        if gelu and tt in range(1, 7):
+            L.append(f"v_add_u32 v{DEF_LD}, 0x1000, v{DEF_LD}")
+    return L
+
+
+def swiglu_epilogue(w8):
+    """bf16(bf16(silu(w1 x)) * (w3 x)): the wave's ft 0-3 are w1 rows, ft 4-7 the same features of w3. Two values at a
+    time; registers v[192:255]."""
+    L = []
+    n = 0
+    for tt in range(8):
+        L += out_row(tt)
+        for g in range(2):
+            o = 192 + 4 * (n % 2)
+            n += 1
+            for p in range(4):                   # 2 values each
+                ft, e = 2 * g + p // 2, (p % 2) * 2
+                w = 208 + 16 * (p % 2)
+                ga, gb, ua, ub, ta, tb, pk = w, w + 1, w + 2, w + 3, w + 4, w + 5, w + 6
+                b1, b3 = (8 * ft + tt) * 4 + e, (8 * (ft + 4) + tt) * 4 + e
+                L += [f"v_accvgpr_read_b32 v{ga}, a{b1}", f"v_accvgpr_read_b32 v{gb}, a{b1 + 1}",
+                      f"v_accvgpr_read_b32 v{ua}, a{b3}", f"v_accvgpr_read_b32 v{ub}, a{b3 + 1}"]
+                if w8:
+                    L += [f"v_mul_f32 v{ga}, %[sc], v{ga}", f"v_mul_f32 v{gb}, %[sc], v{gb}",
+                          f"v_mul_f32 v{ua}, %[su], v{ua}", f"v_mul_f32 v{ub}, %[su], v{ub}"]
+                L += [f"v_cvt_pk_bf16_f32 v{ta}, v{ga}, v{gb}", f"v_cvt_pk_bf16_f32 v{tb}, v{ua}, v{ub}",
+                      f"v_lshlrev_b32 v{ga}, 16, v{ta}", f"v_and_b32 v{gb}, 0xffff0000, v{ta}",
+                      f"v_lshlrev_b32 v{ua}, 16, v{tb}", f"v_and_b32 v{ub}, 0xffff0000, v{tb}",
+                      f"v_mul_f32 v{ta}, 0xbfb8aa3b, v{ga}", f"v_mul_f32 v{tb}, 0xbfb8aa3b, v{gb}",
+                      f"v_exp_f32 v{ta}, v{ta}", f"v_exp_f32 v{tb}, v{tb}", "s_nop 0",
+                      f"v_add_f32 v{ta}, 1.0, v{ta}", f"v_add_f32 v{tb}, 1.0, v{tb}",
+                      f"v_rcp_f32 v{ta}, v{ta}", f"v_rcp_f32 v{tb}, v{tb}", "s_nop 0",
+                      f"v_mul_f32 v{ta}, v{ga}, v{ta}", f"v_mul_f32 v{tb}, v{gb}, v{tb}",
+                      f"v_cvt_pk_bf16_f32 v{pk}, v{ta}, v{tb}",
+                      f"v_lshlrev_b32 v{ta}, 16, v{pk}", f"v_and_b32 v{tb}, 0xffff0000, v{pk}",
+                      f"v_mul_f32 v{ta}, v{ta}, v{ua}", f"v_mul_f32 v{tb}, v{tb}, v{ub}",
+                      f"v_cvt_pk_bf16_f32 v{o + p}, v{ta}, v{tb}"]
+            L.append(f"buffer_store_dwordx4 {quad(o)}, v{ROW_VOFF}, %[ro], 0 offen offset:{64 * g}")
+    return L
+
+
+def partial_epilogue():
+    """The raw fp32 sums, straight from the accumulators: 16 bytes (4 features) per lane and store."""
+    L = []
+    for tt in range(8):
+        L += out_row(tt)
+        for ft in range(8):
+            b = (8 * ft + tt) * 4
+            L.append(f"buffer_store_dwordx4 a[{b}:{b + 3}], v{ROW_VOFF}, %[ro], 0 offen offset:{(ft >> 1) * 128 + (ft & 1) * 16}")
+    return L + ["s_nop 7"]
+
+
+def part_epilogue():
+    """The raw fp32 sums of a part of a tile, straight from the accumulators in the wave's own order (1 KiB per MFMA tile,
+    token blocks outermost); token blocks without rows (%[ntt] of the wave's 8 have some) are left out."""
+    L = [f"v_mov_b32 v{ROW_VOFF}, v{OUT_VOFF}"]
+    for tt in range(8):
+        L += [f"s_cmp_le_i32 %[ntt], {tt}", "s_cbranch_scc1 31f"]
+        for ft in range(8):
+            b = (8 * ft + tt) * 4
+            L.append(f"buffer_store_dwordx4 a[{b}:{b + 3}], v{ROW_VOFF}, %[ro], 0 offen offset:{1024 * (ft % 4)}")
+            if ft % 4 == 3:
+                L.append(f"v_add_u32 v{ROW_VOFF}, 0x1000, v{ROW_VOFF}")
+    return L + ["31:", "s_nop 7"]
+
+
+def gelu_drain(dt):
+    """The pieces of the deferred tile with nothing to hide behind: token blocks 1-7, 4 pieces each. v[192:255] free."""
+    L = [f"v_mov_b32 v{ROW_VOFF}, v{DEF_ST}", f"v_mov_b32 v{DEF_LD}, v{SCR_VOFF}"]
+    for tt in range(1, 8):
+        L.append(f"v_add_u32 v{ROW_VOFF}, {'%[dldo]' if tt > 1 else '%[dd]'}, v{ROW_VOFF}")
+        for g in range(4):
+            L.append(f"buffer_load_dwordx4 {quad(192 + 4 * g)}, v{DEF_LD}, %[scr], 0 offen offset:{1024 * g}")
+        L.append("s_waitcnt vmcnt(0)")
+        for g in range(4):
+            L += [i for i, _ in gelu_words(dt, 192 + 4 * g, 208 + 4 * g, 4)]
+            L.append(f"buffer_store_dwordx4 {quad(208 + 4 * g)}, v{ROW_VOFF}, %[dro], 0 offen offset:{64 * g}")
+        L.append(f"v_add_u32 v{DEF_LD}, 0x1000, v{DEF_LD}")
+    return L + ["s_nop 7"]
+
+
+def check_trans(lines):
+    """A transcendental result is read by another instruction at the earliest two instructions later."""
+    import re
+    for a, b in zip(lines, lines[1:]):
+        mm = re.match(r"v_(exp|rcp)_f32 (v\d+),", a)
+        if mm and re.search(rf"[ |\-]{mm.group(2)}\b", b.split(",", 1)[1] if "," in b else ""):
+            raise AssertionError((a, b))
+
+
+def generate():
+    out = ["// Generated by gen_gemm4w.py; do not edit. See that script for the register map and the schedule.", ""]
+    texts = []
+    for dt, w8, gelu, bias in (("BF16", False, False, False), ("BF16", False, False, True), ("F16", False, False, True),
+                               ("BF16", False, True, True), ("F16", False, True, True), ("BF16", True, False, False), ("BF16", True, False, True)):
+        texts.append((f"HDMOE_G4_LOOP_{dt}{'_W8' if w8 else ''}{'_GELU' if gelu else '_BIAS' if bias else ''}", k_loop(dt, w8, gelu, bias)))
+        texts.append((f"HDMOE_G4_EPI_{dt}{'_W8' if w8 else ''}{'_GELU' if gelu else '_BIAS' if bias else ''}", epilogue(dt, w8, bias, gelu)))
+    texts.append(("HDMOE_G4_EPI_SWIGLU", swiglu_epilogue(False)))
+    texts.append(("HDMOE_G4_EPI_SWIGLU_W8", swiglu_epilogue(True)))
+    texts.append(("HDMOE_G4_EPI_PARTIAL", partial_epilogue()))
+    texts.append(("HDMOE_G4_EPI_PART", part_epilogue()))
+    texts.append(("HDMOE_G4_FILL", reads(0, 0, False, 0)))
+    texts.append(("HDMOE_G4_FILL_W8", reads(0, 0, True, 0) + ["s_waitcnt lgkmcnt(0)"] + [i for i, _ in conversions(0)]))
+    for dt in ("BF16", "F16"):
+        texts.append((f"HDMOE_G4_DRAIN_{dt}", gelu_drain(dt)))
+    for name, lines in texts:
+        check_trans(lines)
+        out.append(f"#define {name} \\")
+        out.append(" \\\n".join('  "' + ln + '\\n"' for ln in lines))
+        out.append("")
+    return "\n".join(out)
+
+
+if __name__ == "__main__":
+    path = sys.argv[1] if len(sys.argv) > 1 else OUT
+    text = generate()
+    if not os.path.exists(path) or open(path).read() != text:
+        with open(path, "w") as f:
+            f.write(text)

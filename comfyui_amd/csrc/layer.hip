@@ -10,10 +10,12 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
                           int K_static, int N_static, hipStream_t s, const char* what,
                           const int32_t* gather_dyn = nullptr, int gather_rows = 0, float* partial = nullptr,
                           int nparts = 1, int gather_shift = 0, bool reduce = true,
-                          const HdmoeSplitPlan* plan = nullptr, const HdmoeAltOperand* alt = nullptr);
+                          const HdmoeSplitPlan* plan = nullptr, const HdmoeAltOperand* alt = nullptr,
+                          float* tail = nullptr);
+size_t hdmoe_tail_bytes(int weight_dtype);
 int hdmoe_launch_combine_partials(const float* partial, long long part_stride, const HdmoeSplitPlan& plan,
                                   int rows_dyn, int n_dyn,
-                                  const int32_t* offsets, bool fp8, const hdmoe_ffn_weights* experts,
+                                  const int32_t* offsets, int weight_dtype, const hdmoe_ffn_weights* experts,
                                   const hdmoe_ffn_weights* shared, const int32_t* inv_perm, const void* topk_weight_bf16,
                                   const void* gate_bf16, const void* residual_bf16, int tokens_per_batch, int T, int D,
                                   void* out_bf16, hipStream_t s, const char* what);
@@ -53,7 +55,7 @@ extern "C" int hdmoe_layer_layout_get(int T, int D, int H, int Hs, int E, int we
                                       hdmoe_layer_layout* out) {
   HDMOE_REQUIRE_PTR(out);
   if (T < 0 || D <= 0 || H <= 0 || Hs < 0 || E < 1 || E > HDMOE_MAX_EXPERTS ||
-      (weight_dtype != HDMOE_W_BF16 && weight_dtype != HDMOE_W_E4M3FN))
+      (weight_dtype != HDMOE_W_BF16 && weight_dtype != HDMOE_W_E4M3FN && weight_dtype != HDMOE_W_E4M3FN_UPCAST))
     return hdmoe_fail(HDMOE_E_SHAPE, "hdmoe_layer_layout_get: T=%d D=%d H=%d Hs=%d E=%d dtype=%d", T, D, H, Hs, E,
                       weight_dtype);
   const size_t eb = weight_dtype == HDMOE_W_E4M3FN ? 1 : 2;
@@ -84,7 +86,10 @@ extern "C" int hdmoe_layer_layout_get(int T, int D, int H, int Hs, int E, int we
   out->normed = take((size_t)T * D * 2);
   // fp32 partial sums of a down projection cut along K (small token counts), [parts][2T + T][D]
   const int parts = hdmoe_down_parts((int)n, E, Hs > 0 ? T : 0, D, H, Hs, weight_dtype);
-  out->partials = take(parts > 1 ? (size_t)parts * (n + (Hs > 0 ? (size_t)T : 0)) * D * 4 : 0);
+  // and, before it, the parts of the gate/up contraction's tail tiles (16-bit arithmetic)
+  const size_t down_bytes = parts > 1 ? (size_t)parts * (n + (Hs > 0 ? (size_t)T : 0)) * D * 4 : 0;
+  const size_t tail_bytes = T > 0 ? hdmoe_tail_bytes(weight_dtype) : 0;
+  out->partials = take(down_bytes > tail_bytes ? down_bytes : tail_bytes);
   // one word the gate + cast kernel leaves for the gate/up GEMM: which layout of the fp8 tokens it wrote
   out->flags = take(256);
   out->total = off;
@@ -259,7 +264,9 @@ extern "C" int hdmoe_moe_ffn(const hdmoe_layer_args* p, hdmoe_stream_t stream) {
   if (int rc = hdmoe_launch_ffn_gemm(true, wd, a_dyn, offsets, (int)n, E, p->experts, h_routed,
                                      a_static, Hs > 0 ? T : 0, p->shared, h_shared, D, H, D, Hs, s,
                                      "hdmoe_moe_ffn (gate/up)", perm, per_token ? T : (int)n, nullptr, 1,
-                                     per_token ? 1 : 0, true, nullptr, decide ? &alt : nullptr))
+                                     per_token ? 1 : 0, true, nullptr, decide ? &alt : nullptr,
+                                     // cut tail tiles make a row's summation order depend on the routing as the K cut does
+                                     fp8 || p->fixed_k_cut != 0 ? nullptr : reinterpret_cast<float*>(ws + l.partials)))
     return rc;
   mark();
   // down projections, both in one launch
@@ -273,13 +280,14 @@ extern "C" int hdmoe_moe_ffn(const hdmoe_layer_args* p, hdmoe_stream_t stream) {
   if (int rc = hdmoe_launch_ffn_gemm(false, wd, h_routed, offsets, (int)n, E, p->experts, y_routed, h_shared,
                                      Hs > 0 ? T : 0, p->shared, y_shared, H, D, Hs, D, s, "hdmoe_moe_ffn (down)",
                                      nullptr, 0, parts > 1 ? reinterpret_cast<float*>(ws + l.partials) : nullptr, parts,
-                                     0, /*reduce=*/false, &plan))
+                                     0, /*reduce=*/false, &plan, nullptr,
+                                     fp8 || p->fixed_k_cut != 0 || parts > 1 ? nullptr : reinterpret_cast<float*>(ws + l.partials)))
     return rc;
   mark();
   // cut along K: the combine adds the parts up itself (no launch and no bf16 copy of the rows in between)
   const int rc = parts > 1
       ? hdmoe_launch_combine_partials(reinterpret_cast<const float*>(ws + l.partials),
-                                      (long long)(n + (Hs > 0 ? (size_t)T : 0)) * D, plan, (int)n, E, offsets, fp8,
+                                      (long long)(n + (Hs > 0 ? (size_t)T : 0)) * D, plan, (int)n, E, offsets, wd,
                                       p->experts, Hs > 0 ? p->shared : nullptr, inv_perm, tw,
                                       fused_block ? p->mod_gate : nullptr, fused_block ? p->x : nullptr,
                                       fused_block ? p->tokens_per_batch : 1, T, D, p->out, s, "hdmoe_moe_ffn (combine)")
@@ -293,13 +301,17 @@ extern "C" int hdmoe_moe_ffn(const hdmoe_layer_args* p, hdmoe_stream_t stream) {
 }
 
 extern "C" size_t hdmoe_ffn_workspace_bytes(int rows, int D, int H, int weight_dtype) {
-  if (rows < 0 || D <= 0 || H <= 0 || (weight_dtype != HDMOE_W_BF16 && weight_dtype != HDMOE_W_E4M3FN)) return 0;
+  if (rows < 0 || D <= 0 || H <= 0 || (weight_dtype != HDMOE_W_BF16 && weight_dtype != HDMOE_W_E4M3FN &&
+                                       weight_dtype != HDMOE_W_E4M3FN_UPCAST))
+    return 0;
   const size_t eb = weight_dtype == HDMOE_W_E4M3FN ? 1 : 2;
   // fp8: quantised copy of x, then h; bf16: h only (x itself is the GEMM operand); then the fp32 partial sums of a
   // down projection cut along K (few rows)
   const size_t a = weight_dtype == HDMOE_W_E4M3FN ? hdmoe_align_up((size_t)rows * D * eb, 256) : 0;
   const int parts = hdmoe_down_parts(0, 0, rows, D, 0, H, weight_dtype);
-  const size_t pbytes = parts > 1 ? hdmoe_align_up((size_t)parts * rows * D * 4, 256) : 0;
+  size_t pbytes = parts > 1 ? hdmoe_align_up((size_t)parts * rows * D * 4, 256) : 0;
+  const size_t tail_bytes = rows > 0 ? hdmoe_tail_bytes(weight_dtype) : 0;
+  if (tail_bytes > pbytes) pbytes = tail_bytes;
   return a + hdmoe_align_up((size_t)rows * H * eb, 256) + pbytes;
 }
 
@@ -332,12 +344,14 @@ extern "C" int hdmoe_ffn_swiglu(int weight_dtype, const void* x_bf16, int rows, 
     a = ws;
     h = ws + hdmoe_align_up((size_t)rows * D, 256);
   }
+  float* const room = reinterpret_cast<float*>(h + hdmoe_align_up((size_t)rows * H * (fp8 ? 1 : 2), 256));
+  float* const tail = fp8 ? nullptr : room;
   if (int rc = hdmoe_launch_ffn_gemm(true, weight_dtype, nullptr, nullptr, 0, 0, nullptr, nullptr, a, rows, w, h, 0, 0, D, H,
-                                     s, "hdmoe_ffn_swiglu (gate/up)"))
+                                     s, "hdmoe_ffn_swiglu (gate/up)", nullptr, 0, nullptr, 1, 0, true, nullptr, nullptr, tail))
     return rc;
   const int parts = hdmoe_down_parts(0, 0, rows, D, 0, H, weight_dtype);
-  float* partial = parts > 1 ? reinterpret_cast<float*>(h + hdmoe_align_up((size_t)rows * H * (fp8 ? 1 : 2), 256)) : nullptr;
+  float* partial = parts > 1 ? room : nullptr;
   return hdmoe_launch_ffn_gemm(false, weight_dtype, nullptr, nullptr, 0, 0, nullptr, nullptr, h, rows, w,
                                static_cast<uint8_t*>(out_bf16), 0, 0, H, D, s, "hdmoe_ffn_swiglu (down)", nullptr, 0,
-                               partial, parts);
+                               partial, parts, 0, true, nullptr, nullptr, parts > 1 ? nullptr : tail);
 }

@@ -25,9 +25,6 @@ constexpr int W4_W_TILE = 65536;                  // LDS: [tok 0 | tok 1 | w 0 |
 constexpr int W4_STG = 131072;
 constexpr int W4_SMEM = W4_STG + 4 * 2048;
 
-typedef float v32f __attribute__((ext_vector_type(32)));
-typedef int v32i __attribute__((ext_vector_type(32)));
-
 // positions in the context registers v[32:63] (gen_swiglu4w.py)
 enum { W4_TOK_ADDR = 0, W4_W_ADDR = 4, W4_TOK_VOFF = 8, W4_W_VOFF = 16, W4_STG_WR = 17, W4_STG_RD = 21, W4_OUT_VOFF = 22 };
 

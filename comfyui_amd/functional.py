@@ -7,11 +7,12 @@ import ctypes
 import torch
 
 from . import _lib
-from ._lib import FfnWeights, LayerArgs, LayerLayout, LinearWeights, W_BF16, W_E4M3FN, check, lib, ptr
+from ._lib import FfnWeights, LayerArgs, LayerLayout, W_BF16, W_E4M3FN, check, lib, ptr
 
 FP8 = torch.float8_e4m3fn
 BF16 = torch.bfloat16
 F16 = torch.float16
+FP8_UPCAST = "float8_e4m3fn multiplied in bfloat16"   # a "weight dtype" of moe_ffn / ffn_swiglu: no activation is cast
 ACT_DTYPES = (BF16, F16)   # 16-bit activation formats; fp16 is served by the *_f16 entry points (Hunyuan3D block)
 
 
@@ -41,6 +42,8 @@ def weight_dtype_code(dtype):
         return W_BF16
     if dtype == FP8:
         return W_E4M3FN
+    if dtype == FP8_UPCAST:
+        return _lib.W_E4M3FN_UPCAST
     if dtype == F16:
         return _lib.W_F16      # hdmoe_linear_bias only
     raise TypeError(f"unsupported weight dtype {dtype}: the HIP path takes bfloat16 or float8_e4m3fn weights")
@@ -131,6 +134,46 @@ def permute_bf16(x2d, perm):
     return out
 
 
+def _linear_groups(dt, weight_code, K, N, act, device, experts=(), a=None, perm=None, offsets=None, rows=0, out=None,
+                   shared=None, a_static=None, out_static=None):
+    """hdmoe_linear_groups with its working memory. experts: list of LinearGroup; shared: LinearGroup or None."""
+    args = _lib.LinearArgs()
+    args.act_dtype = W_BF16 if dt == BF16 else _lib.W_F16
+    args.weight_dtype = args.act_dtype if weight_code is None else weight_code
+    args.K, args.N, args.act = K, N, act
+    if len(experts) > 0 and rows > 0:
+        args.E, args.rows = len(experts), rows
+        arr = (_lib.LinearGroup * len(experts))(*experts)
+        args.a, args.offsets, args.experts, args.out = ptr(a), ptr(offsets), arr, ptr(out)
+        if perm is not None:
+            args.perm, args.T = ptr(perm), a.shape[0]
+    if shared is not None and a_static.shape[0] > 0:
+        args.a_static, args.shared, args.out_static = ptr(a_static), ctypes.pointer(shared), ptr(out_static)
+        args.rows_static = a_static.shape[0]
+    if args.rows == 0 and args.rows_static == 0:
+        return
+    ref = ctypes.byref(args)
+    nbytes = lib.hdmoe_linear_groups_workspace_bytes(ref)
+    if nbytes > 0:   # 0: sizes the call below refuses
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        args.workspace, args.workspace_bytes = ws.data_ptr(), nbytes
+    check(lib.hdmoe_linear_groups(ref, torch.cuda.current_stream(device).cuda_stream))
+
+
+def _linear_group(weight, bias, K, N, what, dtype=BF16, scale=None):
+    _need_hip(weight, f"{what} weight", FP8 if scale is not None else dtype)
+    if tuple(weight.shape) != (N, K):
+        raise ValueError(f"{what}: weight shape {tuple(weight.shape)} != ({N}, {K})")
+    g = _lib.LinearGroup()
+    g.weight = ptr(weight)
+    if bias is not None:
+        _need_hip(bias, f"{what} bias", dtype)
+        if tuple(bias.shape) != (N,):
+            raise ValueError(f"{what}: bias shape {tuple(bias.shape)} != ({N},)")
+        g.bias = ptr(bias)
+    return g
+
+
 def linear(a2d, weight, scale_weight=None, scale_input=None, bias=None):
     """a2d [rows,K] (fp8 for fp8 weights, bf16 for bf16 weights, fp16 for fp16 weights) x weight [N,K]^T (+ bias [N])
     -> [rows,N] bf16 (fp16 for fp16 weights); the bias joins the fp32 result before the one rounding."""
@@ -147,9 +190,37 @@ def linear(a2d, weight, scale_weight=None, scale_input=None, bias=None):
         if bias.shape != (N,) or not bias.is_contiguous():
             raise ValueError(f"linear: bias {tuple(bias.shape)} does not match {N} output features")
     out = torch.empty((rows, N), dtype=out_dtype, device=a2d.device)
+    if code != W_E4M3FN:
+        g = _lib.LinearGroup(ptr(weight), ptr(bias), None)
+        _linear_groups(out_dtype, None, K, N, _lib.ACT_NONE, a2d.device, shared=g, a_static=a2d, out_static=out)
+        return out
     check(lib.hdmoe_linear_bias(code, ptr(a2d), rows, K, N, ptr(weight),
                                 _scale_ptr(scale_weight, a2d.device, "scale_weight"),
                                 _scale_ptr(scale_input, a2d.device, "scale_input"), ptr(bias), ptr(out), _stream(a2d)))
+    return out
+
+
+def linear_upcast_fits(K, N):
+    """Whether a Linear of these sizes has a kernel that multiplies its fp8 weight in bf16."""
+    return K % 128 == 0 and K >= 384 and N % 256 == 0
+
+
+def linear_upcast(a2d, weight, scale=None, bias=None):
+    """bf16( (a2d . weight^T) * bf16(scale) + bias ) for bf16 a2d [rows,K] and a float8_e4m3fn weight [N,K]: the Linear
+    without fp8 matrix multiply on the stored bytes (linear_upcast_fits sizes)."""
+    _need_hip(a2d, "linear_upcast activations", BF16)
+    _need_hip(weight, "linear_upcast weight", FP8)
+    rows, K = a2d.shape
+    N = weight.shape[0]
+    if weight.shape[1] != K:
+        raise ValueError(f"linear_upcast: activations [{rows},{K}] do not match weight {tuple(weight.shape)}")
+    if bias is not None:
+        _need_hip(bias, "linear_upcast bias", BF16)
+        if bias.shape != (N,):
+            raise ValueError(f"linear_upcast: bias {tuple(bias.shape)} does not match {N} output features")
+    out = torch.empty((rows, N), dtype=BF16, device=a2d.device)
+    g = _lib.LinearGroup(ptr(weight), ptr(bias), _scale_ptr(scale, a2d.device, "linear_upcast scale"))
+    _linear_groups(BF16, _lib.W_E4M3FN_UPCAST, K, N, _lib.ACT_NONE, a2d.device, shared=g, a_static=a2d, out_static=out)
     return out
 
 
@@ -197,20 +268,6 @@ def combine(y_sorted, inv_perm, topk_weight, shared):
     return out
 
 
-def _linear_weights(weight, bias, K, N, what, dtype=BF16):
-    _need_hip(weight, f"{what} weight", dtype)
-    if tuple(weight.shape) != (N, K):
-        raise ValueError(f"{what}: weight shape {tuple(weight.shape)} != ({N}, {K})")
-    lw = LinearWeights()
-    lw.weight = ptr(weight)
-    if bias is not None:
-        _need_hip(bias, f"{what} bias", dtype)
-        if tuple(bias.shape) != (N,):
-            raise ValueError(f"{what}: bias shape {tuple(bias.shape)} != ({N},)")
-        lw.bias = ptr(bias)
-    return lw
-
-
 def grouped_linear(a_sorted, offsets, experts, a_static=None, shared=None, act="none"):
     """Linear (+ bias, + erf GELU) of every expert over its row segment of `a_sorted` [rows, K] and, optionally, of
     one more (weight, bias) over all rows of `a_static`, in one launch. experts: list of (weight [N,K], bias [N] or
@@ -220,20 +277,14 @@ def grouped_linear(a_sorted, offsets, experts, a_static=None, shared=None, act="
     _need_hip(a_sorted, "grouped_linear a", dt)
     rows, K = a_sorted.shape
     N = experts[0][0].shape[0] if experts else shared[0].shape[0]
-    E = len(experts)
-    arr = (LinearWeights * max(E, 1))(*[_linear_weights(w, b, K, N, f"grouped_linear expert {i}", dt)
-                                        for i, (w, b) in enumerate(experts)])
+    groups = [_linear_group(w, b, K, N, f"grouped_linear expert {i}", dt) for i, (w, b) in enumerate(experts)]
     out = torch.empty((rows, N), dtype=dt, device=a_sorted.device)
-    out_static, sh, rows_static = None, None, 0
+    out_static, sh = None, None
     if shared is not None:
         _need_hip(a_static, "grouped_linear a_static", dt)
-        rows_static = a_static.shape[0]
-        sh = _linear_weights(shared[0], shared[1], K, N, "grouped_linear shared", dt)
-        out_static = torch.empty((rows_static, N), dtype=dt, device=a_sorted.device)
-    fn = lib.hdmoe_grouped_linear if dt == BF16 else lib.hdmoe_grouped_linear_f16
-    check(fn(ptr(a_sorted), ptr(offsets), rows, E, arr, ptr(out), ptr(a_static), rows_static,
-                                   ctypes.byref(sh) if sh is not None else None, ptr(out_static), K, N, code,
-                                   _stream(a_sorted)))
+        sh = _linear_group(shared[0], shared[1], K, N, "grouped_linear shared", dt)
+        out_static = torch.empty((a_static.shape[0], N), dtype=dt, device=a_sorted.device)
+    _linear_groups(dt, None, K, N, code, a_sorted.device, groups, a_sorted, None, offsets, rows, out, sh, a_static, out_static)
     return out, out_static
 
 
@@ -246,17 +297,13 @@ def grouped_linear_tokens(x2d, perm, offsets, experts, shared=None, act="none"):
     _need_hip(x2d, "grouped_linear_tokens x", dt)
     T, K = x2d.shape
     N = experts[0][0].shape[0]
-    E = len(experts)
-    arr = (LinearWeights * E)(*[_linear_weights(w, b, K, N, f"grouped_linear_tokens expert {i}", dt)
-                                for i, (w, b) in enumerate(experts)])
+    groups = [_linear_group(w, b, K, N, f"grouped_linear_tokens expert {i}", dt) for i, (w, b) in enumerate(experts)]
     out = torch.empty((T * _lib.TOPK, N), dtype=dt, device=x2d.device)
     out_shared, sh = None, None
     if shared is not None:
-        sh = _linear_weights(shared[0], shared[1], K, N, "grouped_linear_tokens shared", dt)
+        sh = _linear_group(shared[0], shared[1], K, N, "grouped_linear_tokens shared", dt)
         out_shared = torch.empty((T, N), dtype=dt, device=x2d.device)
-    check(lib.hdmoe_grouped_linear_tokens(_lib.W_BF16 if dt == BF16 else _lib.W_F16, ptr(x2d), T, ptr(perm), ptr(offsets), E,
-                                          arr, ptr(out), ctypes.byref(sh) if sh is not None else None, ptr(out_shared),
-                                          K, N, code, _stream(x2d)))
+    _linear_groups(dt, None, K, N, code, x2d.device, groups, x2d, perm, offsets, T * _lib.TOPK, out, sh, x2d, out_shared)
     return out, out_shared
 
 

@@ -38,7 +38,7 @@
 extern "C" {
 #endif
 
-#define HDMOE_VERSION 114
+#define HDMOE_VERSION 115
 
 #define HDMOE_OK 0
 #define HDMOE_E_NULL (-1)      /* required pointer is NULL */
@@ -54,6 +54,12 @@ extern "C" {
 #define HDMOE_W_E4M3FN 1
 /* fp16 weights with fp16 activations, bias and outputs: hdmoe_linear_bias only (and the *_f16 entry points below) */
 #define HDMOE_W_F16 2
+/* e4m3fn weights multiplied in bf16: the scaled-fp8 Linear without fp8 matrix multiply (comfy/ops.py:405-410) and a
+ * manual-cast Linear that stores fp8 (comfy/ops.py:107-115). The weights become bf16 (exact) on the way to the matrix
+ * cores; bf16(scale_weight) (1 if NULL), which the reference multiplies onto an operand beforehand and rounds there, is
+ * applied to the fp32 sum. Taken by hdmoe_moe_ffn, hdmoe_ffn_swiglu and hdmoe_linear_groups; every contraction length a
+ * multiple of 128 and at least 384. scale_input is not used. */
+#define HDMOE_W_E4M3FN_UPCAST 3
 
 typedef void* hdmoe_stream_t;
 
@@ -271,6 +277,37 @@ int hdmoe_grouped_linear_tokens(int act_dtype, const void* x, int T, const int32
                                 const hdmoe_linear_weights* experts, void* out, const hdmoe_linear_weights* shared,
                                 void* out_shared, int K, int N, int act, hdmoe_stream_t stream);
 
+/* The Linears above with working memory, for callers that have some (all of hdmoe_linear_bias for 16-bit activations,
+ * hdmoe_grouped_linear, hdmoe_grouped_linear_tokens as one description). What it is used for: tiles that would leave most
+ * of the chip idle are cut along K into fp32 parts that a second launch adds up, and the GELU of a tile hides behind the
+ * next one. Without it (workspace NULL) the results are those of the entry points above. */
+typedef struct {
+  const void* weight; /* [N,K] */
+  const void* bias;   /* [N] of act_dtype, or NULL */
+  const float* scale; /* HDMOE_W_E4M3FN_UPCAST: device fp32 scalar or NULL */
+} hdmoe_linear_group;
+typedef struct {
+  int act_dtype;      /* HDMOE_W_BF16 or HDMOE_W_F16: activations, biases, outputs */
+  int weight_dtype;   /* act_dtype, or HDMOE_W_E4M3FN_UPCAST with bf16 activations */
+  int K, N, act;      /* act: HDMOE_ACT_NONE or HDMOE_ACT_GELU (16-bit weights) */
+  int E;              /* experts, 0 = none */
+  int rows;           /* rows of the experts' segments together */
+  int T;              /* rows of a when perm is set (rows == 2 T) */
+  int rows_static;    /* rows of the static group, 0 = none */
+  const void* a;      /* [rows,K] in segment order, or [T,K] read through perm */
+  const int32_t* perm;
+  const int32_t* offsets;
+  const hdmoe_linear_group* experts; /* host array [E] */
+  void* out;          /* [rows,N] */
+  const void* a_static;
+  const hdmoe_linear_group* shared;
+  void* out_static;
+  void* workspace;    /* hdmoe_linear_groups_workspace_bytes(...) bytes, 256-byte aligned, or NULL */
+  size_t workspace_bytes;
+} hdmoe_linear_args;
+size_t hdmoe_linear_groups_workspace_bytes(const hdmoe_linear_args* args);
+int hdmoe_linear_groups(const hdmoe_linear_args* args, hdmoe_stream_t stream);
+
 /* Weight maintenance of a scaled-fp8 Linear (comfy/ops.py:419-426 set_weight, comfy/float.py:14-67):
  * out[i] = stochastic_round_e4m3fn( float16( src[i] / *scale_dev ) ), scale_dev NULL = 1. Each value lands on one of
  * its two e4m3fn neighbours, the upper one with probability equal to its position between them; |v| >= 448
@@ -310,7 +347,7 @@ typedef struct hdmoe_layer_args {
   int H;            /* routed expert hidden width */
   int Hs;           /* shared expert hidden width (0 = no shared expert) */
   int E;            /* routed experts */
-  int weight_dtype; /* HDMOE_W_BF16 or HDMOE_W_E4M3FN */
+  int weight_dtype; /* HDMOE_W_BF16, HDMOE_W_E4M3FN or HDMOE_W_E4M3FN_UPCAST */
   const void* x;            /* [T,D] bf16 device */
   const void* gate_w;       /* [E,D] bf16 device */
   const hdmoe_ffn_weights* experts; /* host array [E] */

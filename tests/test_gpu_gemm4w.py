@@ -1,0 +1,105 @@
+"""The 4-wave 16-bit GEMM (csrc/gemm4w.h) behind the Linears: edges of its 256 x 256 tiles, the cut of tail tiles along K,
+the activation hidden behind the next tile, fp8 weights multiplied in bf16.
+
+Bounds: the kernel adds products in fp32 (K terms, each rounding at most 2^-24 of the running sum of magnitudes) and rounds
+once to the 16-bit format (half a step: 2^-9 of the value in bf16, 2^-12 in fp16)."""
+import pytest
+import torch
+
+from comfyui_amd import synth
+
+pytestmark = pytest.mark.gpu
+BF16, F16, FP8 = torch.bfloat16, torch.float16, torch.float8_e4m3fn
+HALF_STEP = {BF16: 2.0 ** -8, F16: 2.0 ** -11}   # a step's width over the smallest value of a binade, halved, times 2 for slack
+
+
+def reference(a, w, bias, scale=1.0):
+    """float64 result and the bound on the fp32 sum of products."""
+    r = a.double() @ w.double().t()
+    mag = a.double().abs() @ w.double().abs().t()
+    b = 0.0 if bias is None else bias.double()
+    return r * scale + b, mag * abs(scale) * (a.shape[1] * 2.0 ** -24)
+
+
+def within(y, ref, acc, dt):
+    err = (y.double() - ref).abs()
+    lim = acc + HALF_STEP[dt] * ref.abs() + 1e-7
+    assert bool((err <= lim).all()), float((err / lim).max())
+
+
+@pytest.mark.parametrize("rows,N,K", [
+    (1, 256, 256),          # one tile, two pairs of K steps, no middle pair; cut into as few as two
+    (255, 512, 384),        # an odd number of pairs, the last row of a tile missing
+    (257, 256, 2560),       # one row in a second m-tile; cut along K
+    (700, 2560, 2560),      # 30 tiles, cut
+    (2000, 10240, 512),     # more than one whole round of tiles and a tail
+    (66000, 256, 256),      # 258 tiles of two pairs: nothing to cut
+])
+@pytest.mark.parametrize("dt", [BF16, F16])
+def test_linear(dev, rows, N, K, dt):
+    from comfyui_amd import functional as HF
+    g = torch.Generator(device=dev).manual_seed(rows + K)
+    a = torch.randn((rows, K), generator=g, device=dev).to(dt)
+    w = (torch.randn((N, K), generator=g, device=dev) / K ** 0.5).to(dt)
+    b = torch.randn(N, generator=g, device=dev).to(dt)
+    for bias in (None, b):
+        y = HF.linear(a, w, bias=bias)
+        within(y, *reference(a, w, bias), dt)
+        assert torch.equal(y, HF.linear(a, w, bias=bias))
+
+
+@pytest.mark.parametrize("rows,N,K", [(1, 256, 384), (300, 512, 640), (1000, 2560, 2560), (4480, 2560, 2560), (513, 1024, 4096)])
+def test_fp8_weight_in_bf16(dev, rows, N, K):
+    from comfyui_amd import functional as HF
+    g = torch.Generator(device=dev).manual_seed(rows + K)
+    a = torch.randn((rows, K), generator=g, device=dev).to(BF16)
+    w, s = synth.quantize_per_tensor(torch.randn((N, K), generator=g, device=dev) * 0.02)
+    b = torch.randn(N, generator=g, device=dev).to(BF16)
+    within(HF.linear_upcast(a, w, s, b), *reference(a, w, b, float(s.to(BF16))), BF16)
+    within(HF.linear_upcast(a, w), *reference(a, w, None), BF16)
+
+
+@pytest.mark.parametrize("T,E,K,N", [
+    (40, 8, 2048, 256),      # a few rows per expert: every tile cut
+    (1500, 8, 2048, 4096),   # ragged segments, two tiles and a part per block: activation deferred, then drained
+    (700, 5, 512, 1024),     # K too short to hide the activation behind
+    (3000, 4, 2176, 2048),   # 17 pairs: one more than the deferred activation takes
+])
+@pytest.mark.parametrize("dt", [BF16, F16])
+def test_experts_with_gelu(dev, T, E, K, N, dt):
+    from comfyui_amd import functional as HF
+    g = torch.Generator(device=dev).manual_seed(T + N)
+    x = torch.randn((T, K), generator=g, device=dev).to(dt)
+    ws = [((torch.randn((N, K), generator=g, device=dev) / K ** 0.5).to(dt), (torch.randn(N, generator=g, device=dev) * 0.3).to(dt))
+          for _ in range(E + 1)]
+    ws[1] = (ws[1][0], None)
+    idx, _ = HF.gate_top2(x, (torch.randn((E, K), generator=g, device=dev) / K ** 0.5).to(dt))
+    _, offsets, perm, _ = HF.dispatch(idx, E)
+    rows = x[(perm // 2).long()].contiguous()
+    y, ys = HF.grouped_linear_tokens(x, perm, offsets, ws[:E], shared=ws[E], act="gelu")
+    y2, ys2 = HF.grouped_linear(rows, offsets, ws[:E], a_static=x, shared=ws[E], act="gelu")
+    assert torch.equal(y, y2) and torch.equal(ys, ys2)          # gathered or not: the same tiles
+    bounds = offsets.tolist()
+    for out, a, (w, b) in [(y[lo:hi], rows[lo:hi], ws[e]) for e, (lo, hi) in enumerate(zip(bounds, bounds[1:]))] + [(ys, x, ws[E])]:
+        h, acc = reference(a, w, b)
+        # the sum is rounded, then its GELU (slope at most 1.13) is
+        ref = torch.nn.functional.gelu(h)
+        within(out, ref, 1.13 * (acc + HALF_STEP[dt] * h.abs()), dt)
+
+
+def test_gelu_of_special_values(dev):
+    """Infinities, NaN and the far tails come out of the hidden activation as 0.5 h (1 + erf(h / sqrt 2)) has them."""
+    from comfyui_amd import functional as HF
+    K, N = 2048, 256
+    vals = torch.tensor([0.0, -0.0, 1.0, -1.0, 5.0, -5.0, 9.0, -9.0, 60000.0, -60000.0, float("inf"), float("nan")])
+    a = torch.zeros((256 * 260, K), dtype=F16, device=dev)       # 260 tiles: blocks with two, whose first is deferred
+    w = torch.zeros((N, K), dtype=F16, device=dev)
+    b = vals.to(F16).repeat(N // len(vals) + 1)[:N].contiguous().to(dev)
+    _, y = HF.grouped_linear(a[:0], None, [], a_static=a, shared=(w, b), act="gelu")
+    want = torch.nn.functional.gelu(b.double()).to(F16)
+    fin = torch.isfinite(b) & (b.abs() < 8)
+    assert torch.equal(y, y[:1].expand_as(y)) or bool((torch.isnan(y) == torch.isnan(y[:1])).all())
+    assert torch.equal(torch.isnan(y[0]), torch.isnan(b)) and torch.equal(y[0][b == float("inf")], b[b == float("inf")])
+    assert bool(((y[0] - want).abs()[fin] <= HALF_STEP[F16] * want.abs()[fin]).all())
+    big = torch.isfinite(b) & (b.abs() >= 8)
+    assert bool((y[0][big] == torch.where(b[big] > 0, b[big], torch.zeros_like(b[big]))).all())
