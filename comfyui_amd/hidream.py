@@ -38,6 +38,7 @@ def _pack_ffn(ffn, x, wdt, keep):
     cannot be served by the fused kernels (w1/w3 quantising the same input with different scale_input values).
     Tensors that must outlive the call are appended to `keep`."""
     fp8 = wdt == FP8
+    upcast = wdt == HF.FP8_UPCAST
     dev = x.device
     scales = {}
     own = {}   # the Linear's own scale_input (Parameter or tensor, wherever it lives): the stable object to cache on
@@ -45,12 +46,20 @@ def _pack_ffn(ffn, x, wdt, keep):
     for name, l in (("1", ffn.w1), ("2", ffn.w2), ("3", ffn.w3)):
         if _plain(l) and l.weight.device == dev:
             w = l.weight
+        elif upcast:
+            return None   # a weight that is moved or patched per call arrives as bf16: composed per Linear
         else:
             w, _ = amd_ops.cast_bias_weight(l, x, dtype=wdt)   # offloaded weights, weight functions (LowVramPatch)
         w = w.contiguous()
         keep.append(w)
         ws.append(w)
-        if fp8:
+        if upcast:
+            sw = getattr(l, "scale_weight", None)
+            if sw is not None:
+                sw = sw.to(dev)
+                keep.append(sw)
+            scales["scale_w" + name] = sw
+        elif fp8:
             sw = getattr(l, "scale_weight", None)
             sw = amd_ops._one(dev) if sw is None else sw.to(dev)
             si = getattr(l, "scale_input", None)
@@ -76,7 +85,8 @@ def _pack_ffn(ffn, x, wdt, keep):
 
 
 def _fusable_dtype(ffns):
-    """Common storage dtype of all Linears if the fused kernels can run them, else None."""
+    """Common storage dtype of all Linears (FP8_UPCAST: fp8 weights that are multiplied in bf16) if the fused kernels can run
+    them, else None."""
     lins = [l for f in ffns for l in (f.w1, f.w2, f.w3)]
     for l in lins:
         # any Linear that follows the operations contract (this package's or ComfyUI's own classes)
@@ -85,11 +95,24 @@ def _fusable_dtype(ffns):
     wdt = lins[0].weight.dtype
     if wdt not in (BF16, FP8) or any(l.weight.dtype != wdt for l in lins):
         return None
-    if wdt == FP8 and not all(getattr(l, "hdmoe_fp8_matrix_mult", isinstance(l, amd_ops.fp8_ops.Linear)) for l in lins):
-        return None  # scaled fp8 without fp8 matrix multiply: dequantising Linear path
-    if wdt == FP8 and any(isinstance(l, amd_ops.fp8_ops.Linear) and l.training for l in lins):
+    if wdt == BF16:
+        return wdt
+    if all(_upcasts(l) for l in lins):
+        fits = all(HF.linear_upcast_fits(*reversed(l.weight.shape)) for l in lins)
+        return HF.FP8_UPCAST if fits else None
+    if not all(getattr(l, "hdmoe_fp8_matrix_mult", isinstance(l, amd_ops.fp8_ops.Linear)) for l in lins):
+        return None  # mixed, or a foreign class whose forward decides
+    if any(isinstance(l, amd_ops.fp8_ops.Linear) and l.training for l in lins):
         return None  # fp8_ops.Linear computes in the activation dtype while training (comfy/ops.py:368)
     return wdt
+
+
+def _upcasts(l):
+    """Whether this Linear (one of this package's) multiplies its fp8 weight in the activations' dtype."""
+    if not isinstance(l, amd_ops.disable_weight_init.Linear) or isinstance(l, amd_ops.fp8_ops.Linear):
+        return False
+    mm = getattr(l, "hdmoe_fp8_matrix_mult", None)
+    return mm is False or (mm is None and l.comfy_cast_weights)
 
 
 def _lin_tensors(l):

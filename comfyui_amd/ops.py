@@ -177,6 +177,24 @@ def _linear_bf16(input, weight, bias):
     return out.reshape(*shape[:-1], weight.shape[0])
 
 
+def _upcast_ready(lin, input):
+    """Whether the stored fp8 weight of `lin` can be multiplied in bf16 as it stands (no cast copy of it is made)."""
+    return (lin.weight.dtype == FP8 and lin.weight.device == input.device and input.dtype == BF16
+            and len(lin.weight_function) == 0 and HF.linear_upcast_fits(lin.weight.shape[1], lin.weight.shape[0]))
+
+
+def _linear_upcast(lin, input, scale):
+    bias = None
+    if lin.bias is not None:
+        bias = cast_to(lin.bias, input.dtype, input.device, non_blocking=True, copy=len(lin.bias_function) > 0)
+        for f in lin.bias_function:
+            bias = f(bias)
+        bias = bias.contiguous()
+    shape = input.shape
+    out = HF.linear_upcast(input.reshape(-1, shape[-1]).contiguous(), lin.weight.contiguous(), scale, bias)
+    return out.reshape(*shape[:-1], lin.weight.shape[0])
+
+
 class disable_weight_init:
     class Linear(torch.nn.Linear, CastWeightBiasOp):
         def reset_parameters(self):
@@ -187,6 +205,8 @@ class disable_weight_init:
             return super()._load_from_state_dict(*args, **kwargs)
 
         def forward_comfy_cast_weights(self, input):
+            if _upcast_ready(self, input):
+                return _linear_upcast(self, input, None)
             weight, bias = cast_bias_weight(self, input)
             return _linear_bf16(input, weight, bias)
 
@@ -292,6 +312,10 @@ def scaled_fp8_ops(fp8_matrix_mult=False, scale_input=False, override_dtype=None
                 # no fp8 matmul (ops.py:405-410): the weight is cast to the compute dtype and
                 # scale_weight is multiplied onto the smaller of weight and input
                 scale = self.scale_weight.to(input.device)
+                # resident weights of the usual sizes: multiplied as they are stored, bf16(scale_weight) on the fp32 sum
+                # (one rounding where scaling an operand first rounds twice)
+                if _upcast_ready(self, input):
+                    return _linear_upcast(self, input, scale)
                 bias = None
                 if (len(self.weight_function) == 0 and self.bias is None and self.weight.dtype == FP8
                         and self.weight.device == input.device):

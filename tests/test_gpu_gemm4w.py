@@ -103,3 +103,30 @@ def test_gelu_of_special_values(dev):
     assert bool(((y[0] - want).abs()[fin] <= HALF_STEP[F16] * want.abs()[fin]).all())
     big = torch.isfinite(b) & (b.abs() >= 8)
     assert bool((y[0][big] == torch.where(b[big] > 0, b[big], torch.zeros_like(b[big]))).all())
+
+
+@pytest.mark.parametrize("tokens", [1, 70, 300, 900, 2100])
+def test_layer_without_fp8_matrix_multiply(dev, tokens):
+    """The one-call layer on fp8 weights and bf16 arithmetic against the composition of its Linears (their own forward,
+    checked above), and against the oracle."""
+    from comfyui_amd import functional as HF
+    from oracle import hidream_moe_oracle as O
+    from tests.helpers import oracle_params, small_layer
+    dim = 512
+    sd, x = small_layer(seed=tokens, dim=dim, tokens=tokens, weights="fp8")
+    sd = {k: v for k, v in sd.items() if not k.endswith("scale_input")}
+    m = synth.build_module({k: v.to(dev) for k, v in sd.items()}, "fp8", dev, dim=dim, fp8_matrix_mult=False, scale_input=False)
+    xd = x.to(dev)
+    x2 = xd.reshape(-1, dim)
+    assert m._collect(x2) is not None
+    y = m(xd)
+    composed = m._forward_composed(x2, m.gate.weight).view_as(xd)
+    d = O.error_metrics(y.cpu(), composed.cpu())
+    assert d["rel_rms"] <= 1e-3, d      # a bf16 rounding here and there falls the other way
+    idx, w, _, _ = O.gate_fixed_order(x.reshape(-1, dim), sd["gate.weight"])
+    ref = O.moe_forward(x, oracle_params(sd, 4), "upcast", gate_result=(idx, w))
+    d = O.error_metrics(y.cpu(), ref)
+    assert d["rel_rms"] <= 1e-2, d
+    f = m.experts[1]
+    d = O.error_metrics(f(xd).cpu(), f.w2(HF.silu_mul(f.w1(xd), f.w3(xd))).cpu())
+    assert d["rel_rms"] <= 1e-3, d
