@@ -131,6 +131,10 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wq = wave & 1, wt = wave >> 1;
   auto sgpr = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+  // A constant in a register of its own. The compiler otherwise takes constants out of the initial value of a register tuple,
+  // spills the whole tuple and reloads it between the statements below without waiting for the parts that it does not use:
+  // they would arrive while a statement has those registers in use.
+  auto own = [](int v) { asm volatile("" : "+s"(v)); return v; };
 
   // ---- work items: as grouped_gemm_kernel's tiles --------------------------------------------------------------
   // A wave's lanes look its block's next 64 items up at once and leave them in LDS (one by one, the decoding is a serial
@@ -244,7 +248,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   v16i voff_nxt;           // row offsets of the next tile
   v8i gi;                  // row indices of the tile after it
 #pragma unroll
-  for (int i = 0; i < 32; ++i) ctx[i] = 0;
+  for (int i = 0; i < 32; ++i) ctx[i] = own(0);
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
     ctx[G4_TOK_ADDR + ks] = (int)lds0 + (wt * 128 + fr_row) * 128 + ((ks * 4 + fr_grp) ^ fr_swz) * 16;
@@ -253,7 +257,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   }
   ctx[G4_BIAS_VOFF] = (wq * 128 + fr_grp * 8) * 2;
   ctx[G4_DEF_LD] = ctx[G4_SCR_VOFF] = wave * (G4_SCRATCH / 4) + lane * 16;
-  ctx[G4_DEF_ST] = (int)0x80000000u;
+  ctx[G4_DEF_ST] = own((int)0x80000000u);
   struct Rsrc { uint64_t lo, hi; };
   auto rsrc64 = [&](const void* p, uint32_t bytes) -> Rsrc {
     const uint64_t a = reinterpret_cast<uint64_t>(p);
@@ -286,7 +290,9 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     return s;
   };
   auto load_rows = [&](const Item& d) -> v8i {
-    v8i r = {0, 0, 0, 0, 0, 0, 0, 0};
+    v8i r;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) r[j] = own(0);
     const int32_t* const list = args.g[d.g()].gather;
 #pragma unroll
     for (int j = 0; j < 8; ++j)
@@ -333,7 +339,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   };
   // GELU: the tile whose activation is still to be applied (none: an empty buffer)
   v4i dro = rsrc4(nullptr, 0);
-  int dldo = 0;
+  int dldo = own(0);
   bool deferred = false;
   const v4i scr = EPI == G4_GELU ? rsrc4(args.scratch + (size_t)blockIdx.x * G4_SCRATCH, G4_SCRATCH) : rsrc4(nullptr, 0);
   const int gk = sgpr(__float_as_int(0.84932180f)), gp = sgpr(__float_as_int(0.3f / 0.84932180f));  // gen_gemm4w.py: k, 0.3 / k
