@@ -14,6 +14,9 @@
 HDMOE_PHILOX_HD void hdmoe_philox4x32_10(const uint32_t ctr[4], const uint32_t key[2], uint32_t out[4]) {
   uint32_t c0 = ctr[0], c1 = ctr[1], c2 = ctr[2], c3 = ctr[3];
   uint32_t k0 = key[0], k1 = key[1];
+#if defined(__HIPCC__)
+#pragma unroll   // products of a counter word that is zero or the same for the whole wave drop out
+#endif
   for (int r = 0; r < 10; ++r) {
     const uint64_t p0 = (uint64_t)0xD2511F53u * c0;
     const uint64_t p1 = (uint64_t)0xCD9E8D57u * c2;

@@ -41,6 +41,25 @@ def test_bf16_source_bit_exact(dev):
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("src", [torch.float32, BF16])
+@pytest.mark.parametrize("n,offset", [(4095, 0), (4096, 1), (4097, 2), (20481, 0), (20482, 3)])   # a block takes 4096 elements
+def test_any_scale_and_alignment_bit_exact(dev, src, n, offset):
+    """Quotients on and beside the float16 ties, where a division that is off by one bit shows; scales on both sides of the
+    range in which the kernel multiplies by the reciprocal; sources that start anywhere."""
+    from comfyui_amd import functional as HF
+    g = torch.Generator().manual_seed(n)
+    half = torch.exp2(torch.randint(-15, 9, (n,), generator=g).float()) * (1 + torch.randint(0, 2048, (n,), generator=g) / 2048)
+    half = half * torch.where(torch.rand(n, generator=g) < 0.5, -1.0, 1.0)
+    for scale in (0.37, -3.1e-4, 1.9999999, 2.0 ** -40, 2.0 ** -40.5, 1.1 * 2.0 ** 40, 1e-38):
+        s = torch.tensor(scale, dtype=torch.float32)
+        x = (half * s).to(src)
+        x[:8] = torch.tensor([0.0, -0.0, float("inf"), -float("inf"), float("nan"), 1e-40, 3e38, -1e-30])
+        want = O.stochastic_round_e4m3fn(x, s, 2 ** 40 + n).view(torch.uint8)
+        view = torch.cat([torch.zeros(offset, dtype=src), x]).to(dev)[offset:]
+        got = HF.stochastic_round_e4m3fn(view, s.to(dev), 2 ** 40 + n).cpu().view(torch.uint8)
+        assert torch.equal(got, want), (scale, (got != want).nonzero()[:8].flatten().tolist())
+
+
 def test_unbiased_on_a_weight_matrix(dev):
     from comfyui_amd import functional as HF
     g = torch.Generator().manual_seed(1)
