@@ -307,9 +307,10 @@ def grouped_linear_tokens(x2d, perm, offsets, experts, shared=None, act="none"):
     return out, out_shared
 
 
-def stochastic_round_e4m3fn(weight, scale=None, seed=0):
+def stochastic_round_e4m3fn(weight, scale=None, seed=0, out=None):
     """weight (fp32 or bf16, HIP) / scale (fp32 scalar tensor or None) -> float8_e4m3fn by stochastic rounding
-    (comfy/float.py:14-67 behind comfy/ops.py:419-426), one kernel."""
+    (comfy/float.py:14-67 behind comfy/ops.py:419-426), one kernel. `out`: a contiguous float8_e4m3fn tensor of the
+    weight's shape, of other memory than the weight's and starting on 4 bytes, that takes the result."""
     _need_hip(weight, "stochastic_round_e4m3fn weight")
     if weight.dtype == torch.float32:
         code = _lib.SRC_F32
@@ -317,7 +318,13 @@ def stochastic_round_e4m3fn(weight, scale=None, seed=0):
         code = _lib.SRC_BF16
     else:
         raise TypeError(f"stochastic_round_e4m3fn: expected float32 or bfloat16, got {weight.dtype}")
-    out = torch.empty(weight.shape, dtype=FP8, device=weight.device)
+    if out is None:
+        out = torch.empty(weight.shape, dtype=FP8, device=weight.device)
+    else:
+        _need_hip(out, "stochastic_round_e4m3fn out", FP8)
+        if out.shape != weight.shape or out.device != weight.device:
+            raise ValueError(f"stochastic_round_e4m3fn: out {tuple(out.shape)} on {out.device} for a weight "
+                             f"{tuple(weight.shape)} on {weight.device}")
     check(lib.hdmoe_stochastic_round_e4m3fn(code, ptr(weight), weight.numel(),
                                             _scale_ptr(scale, weight.device, "stochastic_round_e4m3fn scale"),
                                             int(seed) & 0xFFFFFFFFFFFFFFFF, ptr(out), _stream(weight)))

@@ -342,7 +342,15 @@ def scaled_fp8_ops(fp8_matrix_mult=False, scale_input=False, override_dtype=None
                         and weight.dtype in (torch.float32, torch.bfloat16)):
                     # division, float16 rounding and stochastic rounding in one kernel
                     from . import functional as HF
-                    weight = HF.stochastic_round_e4m3fn(weight, self.scale_weight.to(weight.device), seed or 0)
+                    scale = self.scale_weight.to(weight.device)
+                    own = self.weight.data
+                    if (inplace_update and not return_weight and own.device == weight.device and own.shape == weight.shape
+                            and own.is_contiguous() and own.data_ptr() % 4 == 0
+                            and own.untyped_storage().data_ptr() != weight.untyped_storage().data_ptr()):
+                        # straight into the weight: a temporary and its copy would read and write every byte once more
+                        HF.stochastic_round_e4m3fn(weight, scale, seed or 0, out=own)
+                        return
+                    weight = HF.stochastic_round_e4m3fn(weight, scale, seed or 0)
                 else:
                     weight = stochastic_rounding(weight / self.scale_weight.to(device=weight.device, dtype=weight.dtype),
                                                  self.weight.dtype, seed=seed)

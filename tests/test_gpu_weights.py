@@ -92,6 +92,27 @@ def test_set_weight_on_the_device_uses_the_kernel(dev):
     assert bool(((back - w).abs() <= w.abs() * 2.0 ** -3 + sw * 2.0 ** -9 + 1e-6).all())
 
 
+@pytest.mark.parametrize("offset", [0, 4, 3])   # of the stored weight in its memory; 3: not aligned for the kernel
+@pytest.mark.parametrize("shared", [False, True])   # the patched weight lives in the same allocation
+def test_set_weight_in_place(dev, offset, shared):
+    from comfyui_amd import ops as amd_ops
+    lin = amd_ops.scaled_fp8_ops(fp8_matrix_mult=True, scale_input=True).Linear(48, 31, bias=False, device=dev, dtype=FP8)
+    w = torch.randn((31, 48), generator=torch.Generator().manual_seed(4))
+    lin.scale_weight.data.fill_(0.01)
+    mem = torch.zeros(2048 + 4 * w.numel(), dtype=torch.uint8, device=dev)
+    lin.weight = torch.nn.Parameter(mem[offset:offset + w.numel()].view(FP8).view(31, 48), requires_grad=False)
+    src = w.to(dev)
+    if shared:
+        src = mem[2048:].view(torch.float32).view(31, 48).copy_(src)
+    at = lin.weight.data_ptr()
+    lin.set_weight(src, seed=9, inplace_update=True)
+    want = O.stochastic_round_e4m3fn(w, torch.tensor(0.01), 9)
+    assert lin.weight.data_ptr() == at and torch.equal(lin.weight.cpu().view(torch.uint8), want.view(torch.uint8))
+    assert not mem[:offset].any() and not mem[offset + w.numel():2048].any()
+    with pytest.raises(RuntimeError):   # a weight of another shape stays refused
+        lin.set_weight(w.to(dev)[:30], seed=9, inplace_update=True)
+
+
 def test_bad_arguments(dev):
     from comfyui_amd import functional as HF
     with pytest.raises(TypeError):
