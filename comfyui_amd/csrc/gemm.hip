@@ -264,7 +264,7 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_kernel(const GemmArgs a
   // requested two ahead. With few rows a K step lasts as long as its loads take to arrive, not as long as its MFMAs.
   constexpr bool RING3 = LIGHT && TT == 2;
   static_assert(!RING3 || !BIAS, "the three-stage ring is built for the feed-forward contractions");
-  static_assert(TT != 3 || (FP8 && !SWIGLU && !LIGHT), "the 192-token tile exists only for the fp8 Linear");
+  static_assert(TT != 3 || (FP8 && !LIGHT), "the 192-token tile exists only with the fp8 assembly loop");
   static_assert(TT != 2 || RING3, "the 128-token tile exists only with the three-stage ring");
   auto a_off = [](int stage) { return RING3 ? stage * STAGE_BYTES : (stage ? A_OFF1 : 0); };
   auto b_off = [](int stage) { return RING3 ? stage * STAGE_BYTES + A_BYTES : (stage ? B_OFF1 : B_OFF0); };
@@ -1187,6 +1187,7 @@ enum GemmForm {
   FORM_LIGHT4,     // 256-token tiles, token blocks without rows skipped
   FORM_W4,         // fp8 gate/up: the 4-wave kernel (256-token tiles)
   FORM_TALL5,      // 320-token tiles
+  FORM_SHORT3,     // 192-token tiles (fp8 gate/up)
   FORM_BASE4       // 256-token tiles
 };
 
@@ -1210,10 +1211,20 @@ long expected_tile_cost(const GemmShape& sh, int tt) {
   return ((expected_tiles(sh, tt) + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU) * (tt + 1);
 }
 
+// The 192-token tile for fp8 gate/up: only without routed groups (a dense feed-forward). Where it saves a round's height there:
+// 768 tokens by 6912 features, whole branch 86.1 -> 77.4 us, 300 tokens 78.1 -> 69.0, 1500 tokens 132.2 -> 127.6. With experts of
+// uneven size the model says the same and is wrong (layer of 768 tokens 183.8 -> 189.8 us, 384 tokens 140.1 -> 141.5). It has to
+// pay by 15 %: the 4-wave kernel hides part of its epilogue, which the model does not know.
+bool short_tile_pays(const GemmShape& sh) {
+  if (!sh.fp8 || !sh.swiglu || sh.split || sh.n_dyn > 0) return false;
+  const long c4 = expected_tile_cost(sh, 4), c5 = expected_tile_cost(sh, 5);
+  return 20 * expected_tile_cost(sh, 3) <= 17 * (c4 < c5 ? c4 : c5);
+}
+
 // light: the token blocks of a tile that hold no rows are skipped (fp8: the compiler-scheduled K loop instead of the
 // assembly loop, which multiplies padding like rows; 16-bit weights always skip them and take from this only the
 // three-stage ring).
-struct FormChoice { GemmForm form; bool light, ring16, tall, one_round5; };
+struct FormChoice { GemmForm form; bool light, ring16, tall, one_round5, short3; };
 FormChoice pick_form(const GemmShape& sh) {
   const int f_light = form_of(HDMOE_FORM_LIGHT), f_4w = form_of(HDMOE_FORM_SWIGLU4W);
   const bool few_rows = hdmoe_few_rows(sh.rows_dyn, sh.n_dyn, sh.rows_static);
@@ -1226,6 +1237,8 @@ FormChoice pick_form(const GemmShape& sh) {
   // tokens of a layer with a shared expert: 93 against 96 us in the gate/up contraction)
   c.one_round5 = !sh.fp8 && !sh.w8 && sh.swiglu && expected_tiles(sh, 5) <= HDMOE_NUM_CU && expected_tiles(sh, 4) > HDMOE_NUM_CU;
   c.tall = sh.fp8 && !sh.split && !c.light && expected_tile_cost(sh, 5) < expected_tile_cost(sh, 4);
+  c.short3 = !c.light && f_4w != HDMOE_FORM_ALWAYS && short_tile_pays(sh);
+  if (c.short3) { c.tall = false; c.form = FORM_SHORT3; return c; }
   if (sh.split) { c.form = FORM_SPLIT_K; return c; }
   // Light form, gate/up: with every segment inside one 128-token tile (up to 128 tokens in a top-2 layer of 4 experts)
   // the three-stage ring of the down projection pays here too (whole layer 78 -> 73 us at 16 tokens, 80 -> 75 at 128;
@@ -1284,7 +1297,7 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
   shape.w4_fits = true;  // settled below, once the groups are filled in
   FormChoice choice = pick_form(shape);
   const bool light = choice.light, ring16 = choice.ring16, tall = choice.tall;
-  const int BM = tall || choice.one_round5 ? TileCfg<5>::BM : TileCfg<4>::BM;  // tokens per block tile of the kernel that will run
+  const int BM = tall || choice.one_round5 ? TileCfg<5>::BM : choice.short3 ? TileCfg<3>::BM : TileCfg<4>::BM;  // tokens per block tile of the kernel that will run
   const int gather_rows_max = (alt != nullptr && alt->rows > gather_rows) ? alt->rows : gather_rows;
   if (gather_dyn != nullptr && (unsigned long long)gather_rows_max * K_dyn * eb >= (1ull << 31))
     return hdmoe_fail(HDMOE_E_SHAPE, "%s: %d gathered rows of %d bytes exceed the 2 GiB offset range", what,
@@ -1471,6 +1484,8 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
       if (shared != nullptr && rows_static > 0) tb += ((rows_static + W4_BM - 1) / W4_BM) * (N_static / W4_FEAT);
       return launch_swiglu4w(args, tb, s, what);
     }
+    case FORM_SHORT3:
+      return launch_grouped<FP8_SWIGLU, 3>(args, tile_bound, s, what);
     case FORM_TALL5:
       return swiglu ? launch_grouped<FP8_SWIGLU, 5>(args, tile_bound, s, what)
                     : launch_grouped<FP8_PLAIN, 5>(args, tile_bound, s, what);
@@ -1500,6 +1515,7 @@ extern "C" const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E,
     case FORM_RING3: return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 2, LIGHT>" : "grouped_gemm_kernel<BF16_SWIGLU, 2, LIGHT>";
     case FORM_LIGHT4: return "grouped_gemm_kernel<FP8_SWIGLU, 4, LIGHT>";
     case FORM_W4: return "swiglu4w_kernel";
+    case FORM_SHORT3: return "grouped_gemm_kernel<FP8_SWIGLU, 3>";
     case FORM_TALL5: return "grouped_gemm_kernel<FP8_SWIGLU, 5>";
     default:
       if (pick_form(sh).one_round5) return "grouped_gemm_kernel<BF16_SWIGLU, 5>";
