@@ -1107,19 +1107,19 @@ int launch_gemm4w(GemmArgs& args, int rows_mean, hipStream_t s, const char* what
   if (args.tail != nullptr) {
     bool cut = false;
     for (int k = -1; k <= 1; ++k) {
-      int tiles = 0;
-      double fill = 0;
+      int tiles = 0, padding = 0;
       for (int g = 0; g < args.G; ++g) {
         const GemmGroup& gg = args.g[g];
         const int nt = gg.n_out / FEAT;
         int rows = gg.row_end - gg.row_begin;
         if (gg.row_begin < 0) rows = max(0, rows_mean + k * (int)(2 * sqrt((double)rows_mean)));
-        tiles += (rows + G4_BM - 1) / G4_BM * nt;
-        fill += (double)rows * nt / G4_BM;
+        const int mt = (rows + G4_BM - 1) / G4_BM;
+        tiles += mt * nt;
+        padding += (mt * G4_BM - rows) * nt;
         if (gg.kbytes != args.g[0].kbytes) args.tail = nullptr;   // tiles of two lengths: one cut does not even them out
       }
       if (tiles > 0 && tiles <= 24 * HDMOE_NUM_CU)                // one round of more than 24 is not worth a launch
-        cut = cut || g4_plan_tail(tiles, HDMOE_NUM_CU, args.g[0].kbytes / (2 * BK), W8 ? 3 : 2, (float)(fill / tiles)).parts > 1;
+        cut = cut || g4_plan_tail(tiles, HDMOE_NUM_CU, args.g[0].kbytes / (2 * BK), W8 ? 3 : 2, padding).parts > 1;
     }
     if (!cut) args.tail = nullptr;
   }
@@ -1970,6 +1970,16 @@ extern "C" int hdmoe_linear_groups(const hdmoe_linear_args* p, hdmoe_stream_t st
                                     static_cast<hipStream_t>(stream), "hdmoe_linear_groups", p->act_dtype == HDMOE_W_F16,
                                     p->perm, p->T, p->perm != nullptr ? 1 : 0, p->weight_dtype == HDMOE_W_E4M3FN_UPCAST,
                                     ws != nullptr ? reinterpret_cast<float*>(ws + sb) : nullptr, ws != nullptr && sb > 0 ? ws : nullptr);
+}
+
+// The plan of gemm4w_kernel's tail tiles for `tiles` tiles of K elements with `padding` rows without a row of a segment between
+// them (0 to 255 per tile): whole rounds, tiles left over, and the parts that each of those is cut into. For tests and reports.
+extern "C" int hdmoe_tail_plan(int weight_dtype, int tiles, int K, int padding, int* rounds, int* left) {
+  if (tiles <= 0 || K <= 0 || K > 0x7fff * BK / 2 || padding < 0 || padding / tiles >= G4_BM) return 0;
+  const G4Tail t = g4_plan_tail(tiles, HDMOE_NUM_CU, K / BK, weight_dtype == HDMOE_W_E4M3FN_UPCAST ? 3 : 2, padding);
+  if (rounds != nullptr) *rounds = t.rounds;
+  if (left != nullptr) *left = t.tiles;
+  return t.parts;
 }
 
 // Bytes a feed-forward's contractions on 16-bit activations can use for the parts of tail tiles.

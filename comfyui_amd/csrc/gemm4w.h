@@ -87,14 +87,17 @@ struct G4Tail { int rounds, tiles, parts; };
 
 // Costs in units of one pair of K steps (2.0 us with most of the chip idle): a part takes its share of the pairs; leaving the
 // fp32 parts and adding them up costs a second launch (9 us) and their bytes written and read again (256 KiB per part of
-// a full tile, about 6 TB/s). A cut has to pay by a seventh. pairs: K step pairs of a tile; fill: rows / 256 of the
-// average tile.
-__host__ __device__ inline G4Tail g4_plan_tail(int total, int blocks, int pairs, int min_pairs, float fill) {
+// a full tile, about 6 TB/s: 0.04 pairs). A cut has to pay by a seventh. pairs: K step pairs of a tile; padding: rows that the
+// tiles have beyond those of their segments, over all tiles.
+// Both kernels of a launch work the plan out for themselves and have to agree, so it is integers throughout: costs in 25600ths
+// of a pair (100ths, times the 256 rows of a tile).
+__host__ __device__ inline G4Tail g4_plan_tail(int total, int blocks, int pairs, int min_pairs, int padding) {
   G4Tail t = {total / blocks, total % blocks, 1};
   if (t.tiles == 0) return t;
-  float best = 0.85f * (float)pairs;
+  const int fill = G4_BM - padding / total;   // rows of the average tile
+  int best = 85 * G4_BM * pairs;
   for (int p = 2; p <= G4_TAIL_MAX_PARTS && p * t.tiles <= blocks && pairs / p >= min_pairs; ++p) {
-    const float cost = (float)((pairs + p - 1) / p) + 4.5f + 0.04f * fill * (float)(p * t.tiles);
+    const int cost = 100 * G4_BM * ((pairs + p - 1) / p) + 450 * G4_BM + 4 * fill * (p * t.tiles);
     if (cost < best) { best = cost; t.parts = p; }
   }
   return t;
@@ -103,19 +106,16 @@ __host__ __device__ inline G4Tail g4_plan_tail(int total, int blocks, int pairs,
 // The plan of a launch, from the segment sizes on the device; also its number of tiles.
 template <bool W8, int FEAT>
 __device__ __forceinline__ G4Tail g4_tail_of(const GemmArgs& args, const G4Segments& seg, int blocks) {
-  int total = 0;
-  long long rows = 0;
+  int total = 0, padding = 0;
   for (int g = 0; g < args.G; ++g) {
     int rb, re;
     seg.get(args.g[g], rb, re);
-    const int nt = args.g[g].n_out / FEAT;
-    total += ((re - rb + G4_BM - 1) / G4_BM) * nt;
-    rows += (long long)(re - rb) * nt;
+    const int nt = args.g[g].n_out / FEAT, mt = (re - rb + G4_BM - 1) / G4_BM;
+    total += mt * nt;
+    padding += (mt * G4_BM - (re - rb)) * nt;
   }
   if (args.tail == nullptr || total == 0) return {total / blocks, total % blocks, 1};
-  G4Tail t = g4_plan_tail(total, blocks, args.g[0].kbytes / (2 * BK), W8 ? 3 : 2, (float)rows / ((float)total * G4_BM));
-  t.parts = __builtin_amdgcn_readfirstlane(t.parts);   // the same for every lane, which floating point hides
-  return t;
+  return g4_plan_tail(total, blocks, args.g[0].kbytes / (2 * BK), W8 ? 3 : 2, padding);
 }
 
 template <bool F16, bool W8, int EPI>

@@ -38,7 +38,7 @@
 extern "C" {
 #endif
 
-#define HDMOE_VERSION 115
+#define HDMOE_VERSION 116
 
 #define HDMOE_OK 0
 #define HDMOE_E_NULL (-1)      /* required pointer is NULL */
@@ -94,6 +94,12 @@ int hdmoe_get_kernel_form(int which);
  * if Hs > 0; has_scale_in2: the w2 Linears carry a scale_input) runs on under the current switches, for reports that
  * name the dominant kernel; "" for sizes the layer does not take. No counterpart in the reference. */
 const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E, int D, int H, int Hs, int has_scale_in2);
+
+/* How a contraction on 16-bit activations is dealt out when its `tiles` (256 rows x 256 features, gate/up 128) do not come out
+ * even over the CUs: whole rounds of tiles, the tiles left over, and (returned) the parts along K that each of those is cut
+ * into, 1 = not cut, 0 = sizes out of range. padding: rows of the tiles beyond the ends of their segments, all tiles
+ * together. For tests and reports. No counterpart in the reference. */
+int hdmoe_tail_plan(int weight_dtype, int tiles, int K, int padding, int* rounds, int* left);
 
 /* ---- stage entry points ------------------------------------------------------ */
 
