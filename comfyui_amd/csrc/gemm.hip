@@ -1313,8 +1313,6 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
   args.offsets = offsets;
   args.n_offsets = n_dyn;
   int G = 0, tile_bound = 0;
-  const long long op_bytes_dyn = (long long)(gather_dyn != nullptr ? gather_rows_max : rows_dyn) * K_dyn * eb;
-  const long long op_bytes = op_bytes_dyn > (long long)rows_static * K_static * eb ? op_bytes_dyn : (long long)rows_static * K_static * eb;
   const int rows_mean = n_dyn > 0 ? rows_dyn / n_dyn : 0;
   for (int e = 0; e < n_dyn; ++e, ++G) {
     GemmGroup& gg = args.g[G];
@@ -1409,7 +1407,7 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
         if (tl > tb_light) tb_light = tl;
       }
     }
-    const bool g4 = !fp8 && !few_rows && gemm4w_fits(args, w8, op_bytes);
+    const bool g4 = !fp8 && !few_rows && gemm4w_fits(args, w8);
     if (w8 && !g4) return hdmoe_fail(HDMOE_E_SHAPE, "%s: K=%d / %d in %d parts does not fit the kernel for one-byte weights", what, K_dyn, K_static, nparts);
     const int rc = light ? launch_grouped<FP8_PLAIN, 2, true>(args, tb_light, s, what)
                    : w8 ? launch_gemm4w<false, true, G4_PARTIAL>(args, rows_mean, s, what)
@@ -1451,7 +1449,7 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
     // three-stage ring for gate/up with every segment inside a 128-token tile (16-bit weights), the case one_round5, K that is
     // not a multiple of 128, and, where tiles cannot be cut (no room for the parts), one Linear on up to 128 rows (2560 x 2560: 37
     // against 43 us: the 8-wave kernel leaves out the token blocks without rows).
-    const bool g4 = gemm4w_fits(args, w8, op_bytes);
+    const bool g4 = gemm4w_fits(args, w8);
     if (w8) {
       if (!g4) return hdmoe_fail(HDMOE_E_SHAPE, "%s: K=%d / %d does not fit the kernel for one-byte weights", what, K_dyn, K_static);
       return swiglu ? launch_gemm4w<false, true, G4_SWIGLU>(args, rows_mean, s, what)
@@ -1463,6 +1461,8 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
       return launch_gemm4w<false, false, G4_PLAIN>(args, rows_mean, s, what);
   }
   if (fp8 && swiglu) {
+    long long op_bytes = (long long)(gather_dyn != nullptr ? gather_rows_max : rows_dyn) * K_dyn;
+    if ((long long)rows_static * K_static > op_bytes) op_bytes = (long long)rows_static * K_static;
     shape.w4_fits = swiglu4w_fits(args, op_bytes);
     choice = pick_form(shape);
   }
@@ -1717,7 +1717,7 @@ int hdmoe_launch_linear_groups(const uint8_t* a_dyn, const int32_t* offsets, int
   // the 4-wave kernel wherever it fits; it needs room of its own for the activation, and room for the parts of tiles where
   // a few tiles have to be cut (on up to 128 rows the 8-wave kernel is the faster one without: see hdmoe_launch_ffn_gemm)
   const int rows_mean = n_dyn > 0 ? rows_dyn / n_dyn : 0;
-  const bool g4 = gemm4w_fits(args, w8, gather != nullptr ? (long long)gather_rows * K * 2 : 0);
+  const bool g4 = gemm4w_fits(args, w8);
   if (w8) {
     if (!g4 || f16 || act == HDMOE_ACT_GELU)
       return hdmoe_fail(HDMOE_E_SHAPE, "%s: K=%d act=%d does not fit the kernel for one-byte weights", what, K, act);

@@ -49,6 +49,12 @@ def weight_dtype_code(dtype):
     raise TypeError(f"unsupported weight dtype {dtype}: the HIP path takes bfloat16 or float8_e4m3fn weights")
 
 
+def moe_ffn_rows_fit(T, D, H, Hs):
+    """Whether hdmoe_moe_ffn takes this many tokens with 16-bit activations (4 GiB per operand, 2 GiB for the tokens that it reads
+    through the permutation)."""
+    return max(3 * T * D, 2 * T * H, T * Hs) * 2 < 2 ** 32 and T * D * 2 < 2 ** 31
+
+
 def gate_top2(x2d, gate_w):
     """MoEGate scoring + top-2 on the device. x2d [T,D] bf16 (or fp16), gate_w [E,D] of the same dtype
     -> topk_idx int32 [T,2], topk_weight [T,2] of that dtype."""

@@ -292,6 +292,19 @@ class MOEFeedForwardSwiGLU(nn.Module):
             self.__dict__["_packed"] = (key, (wdt, packed[:-1], packed[-1], ()), uniform)
         return wdt, packed[:-1], packed[-1], keep
 
+    def _one_call(self, x):
+        """What _collect found and the hidden widths, or None where the stages have to be composed: renormalised gate weights
+        are not part of the one-call path, and fp8 weights multiplied in bf16 are composed from the Linears where the layer
+        has more tokens than one call takes (every expert's own rows may still fit)."""
+        got = None if getattr(self.gate, "norm_topk_prob", False) else self._collect(x)
+        if got is None:
+            return None
+        H = self.experts[0].w1.weight.shape[0]
+        Hs = self.shared_experts.w1.weight.shape[0]
+        if got[0] == HF.FP8_UPCAST and not HF.moe_ffn_rows_fit(x.shape[0], x.shape[1], H, Hs):
+            return None
+        return (*got, H, Hs)
+
     def forward(self, x, stage_events=None):
         """x [B,S,dim] -> [B,S,dim]. `stage_events` (optional, not in the reference signature) is a
         sequence of 7 hipEvent_t handles recorded around the six stages of the one-call path."""
@@ -302,12 +315,9 @@ class MOEFeedForwardSwiGLU(nn.Module):
         orig_shape = x.shape
         x2 = x.reshape(-1, orig_shape[-1]).contiguous()
         gate_w = _gate_weight(self.gate, x2)
-        # renormalised gate weights are not part of the one-call path: the stages are composed
-        got = None if getattr(self.gate, "norm_topk_prob", False) else self._collect(x2)
+        got = self._one_call(x2)
         if got is not None:
-            wdt, experts, shared, keep = got
-            H = self.experts[0].w1.weight.shape[0]
-            Hs = self.shared_experts.w1.weight.shape[0]
+            wdt, experts, shared, keep, H, Hs = got
             y = HF.moe_ffn(x2, gate_w, experts, shared, H, Hs, wdt, stage_events=stage_events,
                            scale_check=amd_ops.scale_check_word(x2.device) if wdt == FP8 else None,
                            fixed_k_cut=self.__dict__.get("batch_invariant", False))
@@ -328,11 +338,9 @@ class MOEFeedForwardSwiGLU(nn.Module):
         x2 = x.reshape(-1, D).contiguous()
         mods = tuple(m.reshape(B, D).contiguous() for m in (shift, scale, gate))
         gate_w = _gate_weight(self.gate, x2)
-        got = None if getattr(self.gate, "norm_topk_prob", False) else self._collect(x2)
+        got = self._one_call(x2)
         if got is not None:
-            wdt, experts, shared, keep = got
-            H = self.experts[0].w1.weight.shape[0]
-            Hs = self.shared_experts.w1.weight.shape[0]
+            wdt, experts, shared, keep, H, Hs = got
             y = HF.moe_ffn(x2, gate_w, experts, shared, H, Hs, wdt, stage_events=stage_events, modulation=mods,
                            scale_check=amd_ops.scale_check_word(x2.device) if wdt == FP8 else None,
                            fixed_k_cut=self.__dict__.get("batch_invariant", False),

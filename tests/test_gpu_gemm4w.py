@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from comfyui_amd import synth
+from oracle import hidream_moe_oracle as O
 
 pytestmark = pytest.mark.gpu
 BF16, F16, FP8 = torch.bfloat16, torch.float16, torch.float8_e4m3fn
@@ -110,7 +111,6 @@ def test_layer_without_fp8_matrix_multiply(dev, tokens):
     """The one-call layer on fp8 weights and bf16 arithmetic against the composition of its Linears (their own forward,
     checked above), and against the oracle."""
     from comfyui_amd import functional as HF
-    from oracle import hidream_moe_oracle as O
     from tests.helpers import oracle_params, small_layer
     dim = 512
     sd, x = small_layer(seed=tokens, dim=dim, tokens=tokens, weights="fp8")
@@ -130,3 +130,41 @@ def test_layer_without_fp8_matrix_multiply(dev, tokens):
     f = m.experts[1]
     d = O.error_metrics(f(xd).cpu(), f.w2(HF.silu_mul(f.w1(xd), f.w3(xd))).cpu())
     assert d["rel_rms"] <= 1e-3, d
+
+
+@pytest.mark.parametrize("tokens", [
+    77_700,    # routed rows of hidden 6912 (their h is the largest operand) just above 2 GiB
+    155_400,   # above 4 GiB: more than one call takes, composed per expert
+])
+def test_layer_without_fp8_matrix_multiply_of_many_tokens(dev, tokens):
+    """fp8 weights multiplied in bf16, up to where an expert's rows fit the Linears. A token's output is that of a small batch
+    but for the order of fp32 sums (the K cut goes by the batch)."""
+    from comfyui_amd import functional as HF
+    dim, hidden_arg = 512, 10240
+    sd = synth.to_state_dict(synth.make_weights(5, dim=dim, hidden_arg=hidden_arg, device=dev)[0], "fp8", scale_input=False)
+    m = synth.build_module(sd, "fp8", dev, dim=dim, hidden_arg=hidden_arg, fp8_matrix_mult=False, scale_input=False)
+    assert m.experts[0].w1.weight.shape[0] == 6912
+    assert HF.moe_ffn_rows_fit(tokens, dim, 6912, 3584) == (tokens < 100_000)
+    x = torch.randn((1, tokens, dim), generator=torch.Generator(device=dev).manual_seed(5), device=dev).to(BF16)
+    with torch.no_grad():
+        y = m(x)
+        for lo in (0, tokens // 2, tokens - 300):
+            d = O.error_metrics(y[:, lo:lo + 300].cpu(), m(x[:, lo:lo + 300].contiguous()).cpu())
+            assert d["rel_rms"] <= 1e-3, (lo, d)     # a bf16 rounding here and there falls the other way
+
+
+def test_dense_feed_forward_without_fp8_matrix_multiply_of_many_rows(dev):
+    """155 400 rows: h of hidden 6912 just above 2 GiB."""
+    from comfyui_amd import functional as HF
+    g = torch.Generator(device=dev).manual_seed(6)
+    ws, scales = [], {}
+    for name, shape in (("1", (6912, 512)), ("2", (512, 6912)), ("3", (6912, 512))):
+        w, s = synth.quantize_per_tensor(torch.randn(shape, generator=g, device=dev) * 0.02)
+        ws.append(w)
+        scales["scale_w" + name] = s
+    fw = HF.make_ffn_weights(*ws, scales)
+    x = torch.randn((155_400, 512), generator=g, device=dev).to(BF16)
+    y = HF.ffn_swiglu(x, fw, 6912, HF.FP8_UPCAST)
+    for lo in (0, 155_100):
+        d = O.error_metrics(y[lo:lo + 300].cpu(), HF.ffn_swiglu(x[lo:lo + 300].contiguous(), fw, 6912, HF.FP8_UPCAST).cpu())
+        assert d["rel_rms"] <= 1e-3, (lo, d)
