@@ -1196,6 +1196,7 @@ struct GemmShape {
   int rows_dyn, n_dyn, rows_static;  // rows_static = 0: no static group
   int N_dyn, N_static;
   bool w4_fits;                      // the 4-wave kernel takes these operands (swiglu4w_fits)
+  bool g4_takes;                     // 16-bit gate/up: K is of the kind that gemm4w_kernel takes
 };
 
 // Expected tiles with evenly loaded experts, static round-robin over the CUs, and a fixed cost per tile of about one
@@ -1236,7 +1237,9 @@ FormChoice pick_form(const GemmShape& sh) {
   // (16-bit weights: where the taller tile fits one round of blocks and the 256-token tile needs a second, e.g. 257 to 320
   // tokens of a layer with a shared expert: 93 against 96 us in the gate/up contraction)
   c.one_round5 = !sh.fp8 && !sh.w8 && sh.swiglu && expected_tiles(sh, 5) <= HDMOE_NUM_CU && expected_tiles(sh, 4) > HDMOE_NUM_CU;
-  c.tall = sh.fp8 && !sh.split && !c.light && expected_tile_cost(sh, 5) < expected_tile_cost(sh, 4);
+  // (16-bit weights: the gate/up contraction that stays with the 8-wave kernel, 2560 rows of 4 experts by 6912 features, K = 2624: 178
+  // against 198 us; the down projection measured slower on the taller tile)
+  c.tall = (sh.fp8 || (sh.swiglu && !sh.g4_takes)) && !sh.split && !c.light && expected_tile_cost(sh, 5) < expected_tile_cost(sh, 4);
   c.short3 = !c.light && f_4w != HDMOE_FORM_ALWAYS && short_tile_pays(sh);
   if (c.short3) { c.tall = false; c.form = FORM_SHORT3; return c; }
   if (sh.split) { c.form = FORM_SPLIT_K; return c; }
@@ -1295,6 +1298,8 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
   shape.rows_dyn = rows_dyn; shape.n_dyn = n_dyn; shape.rows_static = shared != nullptr ? rows_static : 0;
   shape.N_dyn = N_dyn; shape.N_static = N_static;
   shape.w4_fits = true;  // settled below, once the groups are filled in
+  auto g4_takes = [&](int rows, int K) { return rows <= 0 || (K * eb % (2 * BK) == 0 && K * eb >= 4 * BK); };
+  shape.g4_takes = !fp8 && g4_takes(n_dyn > 0 ? rows_dyn : 0, K_dyn) && g4_takes(shape.rows_static, K_static);
   FormChoice choice = pick_form(shape);
   const bool light = choice.light, ring16 = choice.ring16, tall = choice.tall;
   const int BM = tall || choice.one_round5 ? TileCfg<5>::BM : choice.short3 ? TileCfg<3>::BM : TileCfg<4>::BM;  // tokens per block tile of the kernel that will run
@@ -1487,8 +1492,9 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
     case FORM_SHORT3:
       return launch_grouped<FP8_SWIGLU, 3>(args, tile_bound, s, what);
     case FORM_TALL5:
-      return swiglu ? launch_grouped<FP8_SWIGLU, 5>(args, tile_bound, s, what)
-                    : launch_grouped<FP8_PLAIN, 5>(args, tile_bound, s, what);
+      if (fp8) return swiglu ? launch_grouped<FP8_SWIGLU, 5>(args, tile_bound, s, what)
+                             : launch_grouped<FP8_PLAIN, 5>(args, tile_bound, s, what);
+      return launch_grouped<BF16_SWIGLU, 5>(args, tile_bound, s, what);
     default:
       break;
   }
@@ -1509,6 +1515,7 @@ extern "C" const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E,
   sh.rows_dyn = E > 0 ? T * HDMOE_TOPK : 0; sh.n_dyn = E; sh.rows_static = Hs > 0 ? T : 0;
   sh.N_dyn = H; sh.N_static = Hs;
   const int kb = D * elem_bytes(weight_dtype);
+  sh.g4_takes = !sh.fp8 && kb % (2 * BK) == 0 && kb >= 4 * BK;
   sh.w4_fits = sh.fp8 && has_scale_in2 != 0 && kb % (2 * BK) == 0 && kb >= 16 * BK && H % W4_FEAT == 0 &&
                (Hs <= 0 || Hs % W4_FEAT == 0) && (long long)T * kb < (1ll << 31);
   switch (pick_form(sh).form) {
@@ -1516,10 +1523,10 @@ extern "C" const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E,
     case FORM_LIGHT4: return "grouped_gemm_kernel<FP8_SWIGLU, 4, LIGHT>";
     case FORM_W4: return "swiglu4w_kernel";
     case FORM_SHORT3: return "grouped_gemm_kernel<FP8_SWIGLU, 3>";
-    case FORM_TALL5: return "grouped_gemm_kernel<FP8_SWIGLU, 5>";
+    case FORM_TALL5: return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 5>" : "grouped_gemm_kernel<BF16_SWIGLU, 5>";
     default:
       if (pick_form(sh).one_round5) return "grouped_gemm_kernel<BF16_SWIGLU, 5>";
-      if (!sh.fp8 && kb % (2 * BK) == 0 && kb >= 4 * BK) return "gemm4w_kernel<SWIGLU>";
+      if (sh.g4_takes) return "gemm4w_kernel<SWIGLU>";
       return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 4>" : "grouped_gemm_kernel<BF16_SWIGLU, 4>";
   }
 }
@@ -1679,7 +1686,7 @@ int hdmoe_launch_linear_groups(const uint8_t* a_dyn, const int32_t* offsets, int
   args.scratch = scratch;
   args.offsets = offsets;
   args.n_offsets = n_dyn;
-  int G = 0, tile_bound = 0;
+  int G = 0;
   auto fill = [&](GemmGroup& gg, const W& w) {
     gg.b0 = static_cast<const uint8_t*>(w.weight);
     gg.bias = static_cast<const uint16_t*>(w.bias);
@@ -1700,8 +1707,6 @@ int hdmoe_launch_linear_groups(const uint8_t* a_dyn, const int32_t* offsets, int
     gg.dyn = e;
     if (!gg.b0) return hdmoe_fail(HDMOE_E_NULL, "%s: expert %d has a NULL weight", what, e);
   }
-  constexpr int BM = TileCfg<4>::BM;
-  if (n_dyn > 0) tile_bound += (rows_dyn / BM + n_dyn) * (N / BN);
   if (shared != nullptr && rows_static > 0) {
     GemmGroup& gg = args.g[G];
     fill(gg, *shared);
@@ -1710,12 +1715,12 @@ int hdmoe_launch_linear_groups(const uint8_t* a_dyn, const int32_t* offsets, int
     gg.row_begin = 0;
     gg.row_end = rows_static;
     if (!gg.b0) return hdmoe_fail(HDMOE_E_NULL, "%s: static group has a NULL weight", what);
-    tile_bound += ((rows_static + BM - 1) / BM) * (N / BN);
     ++G;
   }
   args.G = G;
-  // the 4-wave kernel wherever it fits; it needs room of its own for the activation, and room for the parts of tiles where
-  // a few tiles have to be cut (on up to 128 rows the 8-wave kernel is the faster one without: see hdmoe_launch_ffn_gemm)
+  // The 4-wave kernel wherever it fits; it needs room of its own for the activation, and room for the parts of tiles where
+  // a few tiles have to be cut. Without that room and with up to 128 rows a group the 8-wave kernel is the faster one (see
+  // hdmoe_launch_ffn_gemm; 8 experts on 600 rows and one more on 300, 2048 x 8192: 104 against 108 us).
   const int rows_mean = n_dyn > 0 ? rows_dyn / n_dyn : 0;
   const bool g4 = gemm4w_fits(args, w8);
   if (w8) {
@@ -1726,9 +1731,28 @@ int hdmoe_launch_linear_groups(const uint8_t* a_dyn, const int32_t* offsets, int
   if (g4 && act == HDMOE_ACT_GELU && scratch != nullptr)
     return f16 ? launch_gemm4w<true, false, G4_GELU>(args, rows_mean, s, what)
                : launch_gemm4w<false, false, G4_GELU>(args, rows_mean, s, what);
-  if (g4 && act == HDMOE_ACT_NONE && (tail != nullptr || rows_mean > 128 || rows_static > 128))
+  const int rows_all = (n_dyn > 0 ? rows_dyn : 0) + (shared != nullptr ? rows_static : 0);
+  if (g4 && act == HDMOE_ACT_NONE && (tail != nullptr || rows_all > 128 * G))
     return f16 ? launch_gemm4w<true, false, G4_BIAS>(args, rows_mean, s, what)
                : launch_gemm4w<false, false, G4_BIAS>(args, rows_mean, s, what);
+  // The 8-wave kernel, by the rule of the feed-forward contractions: the 320-token tile when it saves a round of tiles. A
+  // segment is taken one standard deviation of an even routing above the mean (at a mean that is a multiple of the tile height half the
+  // segments need one tile more). GELU, 8 experts on 5000 rows and one more on 2500, 2048 x 8192: 330 us on 256-token tiles, 272 on 320.
+  auto tiles = [&](int tt) {
+    const int bm = 64 * tt, seg = rows_mean + (int)sqrtf((float)rows_mean);
+    long n = 0;
+    if (n_dyn > 0) n += (long)n_dyn * ((seg + bm - 1) / bm) * (N / BN);
+    if (shared != nullptr && rows_static > 0) n += (long)((rows_static + bm - 1) / bm) * (N / BN);
+    return n;
+  };
+  auto cost = [&](int tt) { return (tiles(tt) + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU * (tt + 1); };
+  const bool tall = cost(5) < cost(4);
+  const int BM = tall ? TileCfg<5>::BM : TileCfg<4>::BM;
+  int tile_bound = 0;
+  if (n_dyn > 0) tile_bound += (rows_dyn / BM + n_dyn) * (N / BN);
+  if (shared != nullptr && rows_static > 0) tile_bound += ((rows_static + BM - 1) / BM) * (N / BN);
+  if (tall) return f16 ? launch_grouped<F16_PLAIN_BIAS, 5>(args, tile_bound, s, what)
+                       : launch_grouped<BF16_PLAIN_BIAS, 5>(args, tile_bound, s, what);
   return f16 ? launch_grouped<F16_PLAIN_BIAS>(args, tile_bound, s, what)
              : launch_grouped<BF16_PLAIN_BIAS>(args, tile_bound, s, what);
 }

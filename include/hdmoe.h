@@ -286,7 +286,8 @@ int hdmoe_grouped_linear_tokens(int act_dtype, const void* x, int T, const int32
 /* The Linears above with working memory, for callers that have some (all of hdmoe_linear_bias for 16-bit activations,
  * hdmoe_grouped_linear, hdmoe_grouped_linear_tokens as one description). What it is used for: tiles that would leave most
  * of the chip idle are cut along K into fp32 parts that a second launch adds up, and the GELU of a tile hides behind the
- * next one. Without it (workspace NULL) the results are those of the entry points above. */
+ * next one. Without it (workspace NULL) the kernels are those of the entry points above; the results differ by the order of
+ * the fp32 sums and the error of the activation's approximation (7e-7 of the value) before the rounding to 16 bits. */
 typedef struct {
   const void* weight; /* [N,K] */
   const void* bias;   /* [N] of act_dtype, or NULL */
