@@ -98,7 +98,7 @@ def _fusable_dtype(ffns):
     if wdt == BF16:
         return wdt
     if all(_upcasts(l) for l in lins):
-        fits = all(HF.linear_upcast_fits(*reversed(l.weight.shape)) for l in lins)
+        fits = all(HF.linear_upcast_fits(*reversed(l.weight.shape)) and _own_forward(l) for l in lins)
         return HF.FP8_UPCAST if fits else None
     if not all(getattr(l, "hdmoe_fp8_matrix_mult", isinstance(l, amd_ops.fp8_ops.Linear)) for l in lins):
         return None  # mixed, or a foreign class whose forward decides
@@ -113,6 +113,25 @@ def _upcasts(l):
         return False
     mm = getattr(l, "hdmoe_fp8_matrix_mult", None)
     return mm is False or (mm is None and l.comfy_cast_weights)
+
+
+def _observed(m):
+    """Whether a call of this module does more than its class: hooks, a forward of its own. Linears that multiply fp8 weights in
+    bf16 were always called one by one, so calibration hooks and wrapped forwards are in use there."""
+    d = m.__dict__
+    return bool(d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d)
+
+
+def _own_forward(l):
+    """Whether calling an _upcasts Linear runs this package's bf16 arithmetic and nothing else: no subclass brings a forward, and the
+    class (not a flag set on the instance, which its forward does not read) is one without fp8 matrix multiply."""
+    cls = type(l)
+    if cls.forward is not amd_ops.disable_weight_init.Linear.forward or _observed(l):
+        return False
+    cast = next(c for c in cls.__mro__ if "forward_comfy_cast_weights" in c.__dict__)
+    if cast is amd_ops.disable_weight_init.Linear:
+        return bool(l.comfy_cast_weights)
+    return cast.__dict__.get("hdmoe_fp8_matrix_mult") is False
 
 
 def _lin_tensors(l):
@@ -143,7 +162,10 @@ def _pack_key(ffns, dev):
             if not w.is_contiguous() or any(t is not None and (t.dtype != torch.float32 or not t.is_contiguous())
                                             for t in (sw, si)):
                 return None
-            key.append((type(l), l.training, w.data_ptr(), w.dtype, b is None, getattr(l, "hdmoe_fp8_matrix_mult", None),
+            mm = getattr(l, "hdmoe_fp8_matrix_mult", None)
+            if not mm and w.dtype == FP8:   # multiplied in bf16, if at all in one call: what _fusable_dtype asks beyond the tensors
+                key.append((_observed(f), _observed(l), l.comfy_cast_weights))
+            key.append((type(l), l.training, w.data_ptr(), w.dtype, b is None, mm,
                         None if sw is None else (sw.data_ptr(), sw._version),
                         None if si is None else (si.data_ptr(), si._version)))
     return tuple(key)
@@ -273,7 +295,7 @@ class MOEFeedForwardSwiGLU(nn.Module):
             return cached[1]
         self.__dict__["_packed"] = None
         wdt = _fusable_dtype(ffns)
-        if wdt is None:
+        if wdt is None or (wdt == HF.FP8_UPCAST and any(_observed(f) for f in ffns)):
             return None
         keep = []
         packed = []
