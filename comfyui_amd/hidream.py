@@ -97,14 +97,13 @@ def _fusable_dtype(ffns):
         return None
     if wdt == BF16:
         return wdt
-    if all(_upcasts(l) for l in lins):
-        fits = all(HF.linear_upcast_fits(*reversed(l.weight.shape)) and _own_forward(l) for l in lins)
-        return HF.FP8_UPCAST if fits else None
-    if not all(getattr(l, "hdmoe_fp8_matrix_mult", isinstance(l, amd_ops.fp8_ops.Linear)) for l in lins):
-        return None  # mixed, or a foreign class whose forward decides
-    if any(isinstance(l, amd_ops.fp8_ops.Linear) and l.training for l in lins):
-        return None  # fp8_ops.Linear computes in the activation dtype while training (comfy/ops.py:368)
-    return wdt
+    if all(getattr(l, "hdmoe_fp8_matrix_mult", isinstance(l, amd_ops.fp8_ops.Linear)) for l in lins):
+        if any(isinstance(l, amd_ops.fp8_ops.Linear) and l.training for l in lins):
+            return None  # fp8_ops.Linear computes in the activation dtype while training (comfy/ops.py:368)
+        return wdt
+    if all(_upcasts(l) and HF.linear_upcast_fits(*reversed(l.weight.shape)) and _own_forward(l) for l in lins):
+        return HF.FP8_UPCAST
+    return None  # mixed, or a foreign class whose forward decides
 
 
 def _upcasts(l):
