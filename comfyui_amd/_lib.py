@@ -59,7 +59,7 @@ class LinearArgs(ctypes.Structure):
     """hdmoe_linear_args"""
     _fields_ = [
         ("act_dtype", c_int), ("weight_dtype", c_int), ("K", c_int), ("N", c_int), ("act", c_int), ("E", c_int),
-        ("rows", c_int), ("T", c_int), ("rows_static", c_int),
+        ("rows", c_int), ("T", c_int), ("rows_static", c_int), ("fixed_k_cut", c_int),
         ("a", c_void_p), ("perm", c_void_p), ("offsets", c_void_p), ("experts", ctypes.POINTER(LinearGroup)), ("out", c_void_p),
         ("a_static", c_void_p), ("shared", ctypes.POINTER(LinearGroup)), ("out_static", c_void_p),
         ("workspace", c_void_p), ("workspace_bytes", c_size_t),

@@ -1993,7 +1993,8 @@ extern "C" int hdmoe_linear_groups(const hdmoe_linear_args* p, hdmoe_stream_t st
                                     p->shared, static_cast<uint8_t*>(p->out_static), p->K, p->N, p->act,
                                     static_cast<hipStream_t>(stream), "hdmoe_linear_groups", p->act_dtype == HDMOE_W_F16,
                                     p->perm, p->T, p->perm != nullptr ? 1 : 0, p->weight_dtype == HDMOE_W_E4M3FN_UPCAST,
-                                    ws != nullptr ? reinterpret_cast<float*>(ws + sb) : nullptr, ws != nullptr && sb > 0 ? ws : nullptr);
+                                    ws != nullptr && p->fixed_k_cut == 0 ? reinterpret_cast<float*>(ws + sb) : nullptr,
+                                    ws != nullptr && sb > 0 ? ws : nullptr);
 }
 
 // The plan of gemm4w_kernel's tail tiles for `tiles` tiles of K elements with `padding` rows without a row of a segment between

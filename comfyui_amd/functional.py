@@ -141,12 +141,12 @@ def permute_bf16(x2d, perm):
 
 
 def _linear_groups(dt, weight_code, K, N, act, device, experts=(), a=None, perm=None, offsets=None, rows=0, out=None,
-                   shared=None, a_static=None, out_static=None):
+                   shared=None, a_static=None, out_static=None, fixed_k_cut=False):
     """hdmoe_linear_groups with its working memory. experts: list of LinearGroup; shared: LinearGroup or None."""
     args = _lib.LinearArgs()
     args.act_dtype = W_BF16 if dt == BF16 else _lib.W_F16
     args.weight_dtype = args.act_dtype if weight_code is None else weight_code
-    args.K, args.N, args.act = K, N, act
+    args.K, args.N, args.act, args.fixed_k_cut = K, N, act, 1 if fixed_k_cut else 0
     if len(experts) > 0 and rows > 0:
         args.E, args.rows = len(experts), rows
         arr = (_lib.LinearGroup * len(experts))(*experts)
@@ -180,9 +180,10 @@ def _linear_group(weight, bias, K, N, what, dtype=BF16, scale=None):
     return g
 
 
-def linear(a2d, weight, scale_weight=None, scale_input=None, bias=None):
+def linear(a2d, weight, scale_weight=None, scale_input=None, bias=None, fixed_k_cut=False):
     """a2d [rows,K] (fp8 for fp8 weights, bf16 for bf16 weights, fp16 for fp16 weights) x weight [N,K]^T (+ bias [N])
-    -> [rows,N] bf16 (fp16 for fp16 weights); the bias joins the fp32 result before the one rounding."""
+    -> [rows,N] bf16 (fp16 for fp16 weights); the bias joins the fp32 result before the one rounding.
+    fixed_k_cut: see grouped_linear (16-bit activations; with fp8 ones a row never depends on the number of rows)."""
     code = weight_dtype_code(weight.dtype)
     _need_hip(a2d, "linear activations", weight.dtype)
     _need_hip(weight, "linear weight")
@@ -198,7 +199,8 @@ def linear(a2d, weight, scale_weight=None, scale_input=None, bias=None):
     out = torch.empty((rows, N), dtype=out_dtype, device=a2d.device)
     if code != W_E4M3FN:
         g = _lib.LinearGroup(ptr(weight), ptr(bias), None)
-        _linear_groups(out_dtype, None, K, N, _lib.ACT_NONE, a2d.device, shared=g, a_static=a2d, out_static=out)
+        _linear_groups(out_dtype, None, K, N, _lib.ACT_NONE, a2d.device, shared=g, a_static=a2d, out_static=out,
+                       fixed_k_cut=fixed_k_cut)
         return out
     check(lib.hdmoe_linear_bias(code, ptr(a2d), rows, K, N, ptr(weight),
                                 _scale_ptr(scale_weight, a2d.device, "scale_weight"),
@@ -211,7 +213,7 @@ def linear_upcast_fits(K, N):
     return K % 128 == 0 and K >= 384 and N % 256 == 0
 
 
-def linear_upcast(a2d, weight, scale=None, bias=None):
+def linear_upcast(a2d, weight, scale=None, bias=None, fixed_k_cut=False):
     """bf16( (a2d . weight^T) * bf16(scale) + bias ) for bf16 a2d [rows,K] and a float8_e4m3fn weight [N,K]: the Linear
     without fp8 matrix multiply on the stored bytes (linear_upcast_fits sizes)."""
     _need_hip(a2d, "linear_upcast activations", BF16)
@@ -226,7 +228,8 @@ def linear_upcast(a2d, weight, scale=None, bias=None):
             raise ValueError(f"linear_upcast: bias {tuple(bias.shape)} does not match {N} output features")
     out = torch.empty((rows, N), dtype=BF16, device=a2d.device)
     g = _lib.LinearGroup(ptr(weight), ptr(bias), _scale_ptr(scale, a2d.device, "linear_upcast scale"))
-    _linear_groups(BF16, _lib.W_E4M3FN_UPCAST, K, N, _lib.ACT_NONE, a2d.device, shared=g, a_static=a2d, out_static=out)
+    _linear_groups(BF16, _lib.W_E4M3FN_UPCAST, K, N, _lib.ACT_NONE, a2d.device, shared=g, a_static=a2d, out_static=out,
+                   fixed_k_cut=fixed_k_cut)
     return out
 
 
@@ -274,10 +277,12 @@ def combine(y_sorted, inv_perm, topk_weight, shared):
     return out
 
 
-def grouped_linear(a_sorted, offsets, experts, a_static=None, shared=None, act="none"):
+def grouped_linear(a_sorted, offsets, experts, a_static=None, shared=None, act="none", fixed_k_cut=False):
     """Linear (+ bias, + erf GELU) of every expert over its row segment of `a_sorted` [rows, K] and, optionally, of
     one more (weight, bias) over all rows of `a_static`, in one launch. experts: list of (weight [N,K], bias [N] or
-    None). Returns (out_sorted [rows, N], out_static [rows_static, N] or None)."""
+    None). Returns (out_sorted [rows, N], out_static [rows_static, N] or None).
+    fixed_k_cut: no tile of the last round is cut along K, which otherwise goes by the segment sizes: a row's bytes then do not
+    depend on the other rows."""
     code = {"none": _lib.ACT_NONE, "gelu": _lib.ACT_GELU}[act]
     dt = _act_dtype(a_sorted, "grouped_linear a")   # bf16, or fp16 throughout
     _need_hip(a_sorted, "grouped_linear a", dt)
@@ -290,11 +295,12 @@ def grouped_linear(a_sorted, offsets, experts, a_static=None, shared=None, act="
         _need_hip(a_static, "grouped_linear a_static", dt)
         sh = _linear_group(shared[0], shared[1], K, N, "grouped_linear shared", dt)
         out_static = torch.empty((a_static.shape[0], N), dtype=dt, device=a_sorted.device)
-    _linear_groups(dt, None, K, N, code, a_sorted.device, groups, a_sorted, None, offsets, rows, out, sh, a_static, out_static)
+    _linear_groups(dt, None, K, N, code, a_sorted.device, groups, a_sorted, None, offsets, rows, out, sh, a_static, out_static,
+                   fixed_k_cut)
     return out, out_static
 
 
-def grouped_linear_tokens(x2d, perm, offsets, experts, shared=None, act="none"):
+def grouped_linear_tokens(x2d, perm, offsets, experts, shared=None, act="none", fixed_k_cut=False):
     """The first Linear (+ bias, + erf GELU) of every expert on the rows of `x2d` [T, K] its segment selects through
     the dispatch permutation (sorted row r = token perm[r] // 2; nothing is copied into expert order), and of
     `shared` (weight, bias) on all T rows, in one launch. Returns (out_sorted [2T, N], out_shared [T, N] or None)."""
@@ -309,7 +315,8 @@ def grouped_linear_tokens(x2d, perm, offsets, experts, shared=None, act="none"):
     if shared is not None:
         sh = _linear_group(shared[0], shared[1], K, N, "grouped_linear_tokens shared", dt)
         out_shared = torch.empty((T, N), dtype=dt, device=x2d.device)
-    _linear_groups(dt, None, K, N, code, x2d.device, groups, x2d, perm, offsets, T * _lib.TOPK, out, sh, x2d, out_shared)
+    _linear_groups(dt, None, K, N, code, x2d.device, groups, x2d, perm, offsets, T * _lib.TOPK, out, sh, x2d, out_shared,
+                   fixed_k_cut)
     return out, out_shared
 
 
@@ -456,8 +463,9 @@ def moe_ffn(x2d, gate_w, experts, shared, H, Hs, weight_dtype, out=None, workspa
     out = x + gate * layer(LayerNorm(x) * (1 + scale) + shift), with T == B * tokens_per_batch.
     uniform_scale_in: accepted and not used (the casting kernel compares the scale_input values on the device and
     casts the tokens once when they agree).
-    fixed_k_cut: the K cut of the down projection (small token counts) is taken from the sizes alone instead of from
-    the segment sizes of the call, so that a row's bytes do not depend on the routing of the other rows.
+    fixed_k_cut: what is cut along K (the down projection at small token counts; with 16-bit activations the tiles of a last
+    round, at any) is taken from the sizes alone instead of from the segment sizes of the call, so that a row's bytes do
+    not depend on the routing of the other rows.
     scale_check: optional pinned int32 tensor of one element that the casting kernel sets to 1 when w1 and w3 of a
     feed-forward turn out to cast the tokens differently (the output is then NaN).
     Returns out [T,D] bf16 (and topk_idx int32, topk_weight bf16 when want_routing)."""

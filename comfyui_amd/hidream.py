@@ -274,8 +274,10 @@ class MOEFeedForwardSwiGLU(nn.Module):
 
     # Not an attribute of the reference class. Set `module.batch_invariant = True` to have every token's output bytes
     # independent of how the other tokens of the batch are routed: between a few hundred and about two thousand tokens
-    # the down projection is cut along K and the cut that runs is otherwise picked from the experts' segment sizes,
-    # which changes the fp32 summation order (the last bit of an output) with the rest of the batch.
+    # the down projection is cut along K, and with 16-bit activations the tiles that either contraction has left over
+    # after whole rounds are, at any number of tokens; the cut that runs is otherwise picked from the experts' segment
+    # sizes, which changes the fp32 summation order (the last bit of an output) with the rest of the batch. Holds for the
+    # one-call path.
 
     # ---- fused path ----------------------------------------------------------------
 

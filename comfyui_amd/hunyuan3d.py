@@ -40,7 +40,8 @@ class _LinearWithBias(amd_ops.disable_weight_init.Linear):
             raise RuntimeError("comfyui_amd.hunyuan3d: expected bfloat16 or float16 HIP tensors and weights of the same "
                                "dtype; there is no CPU path")
         x2 = x.reshape(-1, x.shape[-1]).contiguous()
-        _, y = HF.grouped_linear(x2[:0], None, [], a_static=x2, shared=(self.weight, self.bias), act="none")
+        _, y = HF.grouped_linear(x2[:0], None, [], a_static=x2, shared=(self.weight, self.bias), act="none",
+                                 fixed_k_cut=amd_ops._batch_invariant(self))
         return y.view(*x.shape[:-1], self.weight.shape[0])
 
 
@@ -58,7 +59,8 @@ class GELU(nn.Module):
         _need(x2)
         if not _plain_bf16(self.proj, x2):
             return HF.gelu(self.proj(x2).contiguous()).view(*hidden_states.shape[:-1], self.proj.weight.shape[0])
-        _, y = HF.grouped_linear(x2[:0], None, [], a_static=x2, shared=(self.proj.weight, self.proj.bias), act="gelu")
+        _, y = HF.grouped_linear(x2[:0], None, [], a_static=x2, shared=(self.proj.weight, self.proj.bias), act="gelu",
+                                 fixed_k_cut=amd_ops._batch_invariant(self.proj))
         return y.view(*hidden_states.shape[:-1], self.proj.weight.shape[0])
 
 
@@ -107,8 +109,10 @@ class FeedForward(nn.Module):
             y = self.net[2](self.net[0](x2))     # net[1] is Dropout, the identity at inference
             return y.view(*hidden_states.shape[:-1], y.shape[-1])
         w_in, w_out = self.stage_weights()
-        _, h = HF.grouped_linear(x2[:0], None, [], a_static=x2, shared=w_in, act="gelu")
-        _, y = HF.grouped_linear(h[:0], None, [], a_static=h, shared=w_out, act="none")
+        _, h = HF.grouped_linear(x2[:0], None, [], a_static=x2, shared=w_in, act="gelu",
+                                 fixed_k_cut=amd_ops._batch_invariant(self.net[0].proj))
+        _, y = HF.grouped_linear(h[:0], None, [], a_static=h, shared=w_out, act="none",
+                                 fixed_k_cut=amd_ops._batch_invariant(self.net[2]))
         return y.view(*hidden_states.shape[:-1], y.shape[-1])
 
 
@@ -144,6 +148,11 @@ class MoEBlock(nn.Module):
         self.shared_experts = FeedForward(dim, dropout=dropout, inner_dim=ff_inner_dim, operations=operations,
                                           device=device, dtype=dtype)
 
+    # Not an attribute of the reference class. Set `block.batch_invariant = True` to have every token's output bytes
+    # independent of how the other tokens of the batch are routed: tiles that a grouped launch has left over after whole
+    # rounds are otherwise cut along K, by the experts' segment sizes. Where the experts are called one at a time, the
+    # attribute of the same name on each Linear says so.
+
     def forward(self, hidden_states) -> torch.Tensor:
         if self.training:
             raise NotImplementedError("comfyui_amd.hunyuan3d.MoEBlock is inference only (call .eval())")
@@ -167,7 +176,8 @@ class MoEBlock(nn.Module):
         stage1 = [e.stage_weights()[0] for e in self.experts]
         stage2 = [e.stage_weights()[1] for e in self.experts]
         sh1, sh2 = self.shared_experts.stage_weights()
+        fixed = amd_ops._batch_invariant(self)
         # the experts' first Linear reads the routed rows through the permutation: no copy in expert order
-        h, h_sh = HF.grouped_linear_tokens(x2, perm, offsets, stage1, shared=sh1, act="gelu")
-        y, y_sh = HF.grouped_linear(h, offsets, stage2, a_static=h_sh, shared=sh2, act="none")
+        h, h_sh = HF.grouped_linear_tokens(x2, perm, offsets, stage1, shared=sh1, act="gelu", fixed_k_cut=fixed)
+        y, y_sh = HF.grouped_linear(h, offsets, stage2, a_static=h_sh, shared=sh2, act="none", fixed_k_cut=fixed)
         return HF.combine(y, inv_perm, w, y_sh).view(*orig_shape)

@@ -169,12 +169,18 @@ def scale_value(p, use_cache=None):
     return v
 
 
-def _linear_bf16(input, weight, bias):
+def _linear_bf16(input, weight, bias, lin=None):
     shape = input.shape
     x2 = input.reshape(-1, shape[-1]).contiguous()
     # a bias is added to the fp32 accumulator before the one rounding to bf16, like F.linear's fused epilogue
-    out = HF.linear(x2, weight.contiguous(), bias=None if bias is None else bias.contiguous())
+    out = HF.linear(x2, weight.contiguous(), bias=None if bias is None else bias.contiguous(), fixed_k_cut=_batch_invariant(lin))
     return out.reshape(*shape[:-1], weight.shape[0])
+
+
+def _batch_invariant(module):
+    """`module.batch_invariant = True` on a Linear: its contraction is never cut along K by the number of rows, so that a row's
+    bytes do not depend on which rows come with it. Not an attribute of the reference classes."""
+    return module is not None and module.__dict__.get("batch_invariant", False)
 
 
 def _upcast_ready(lin, input):
@@ -191,7 +197,8 @@ def _linear_upcast(lin, input, scale):
             bias = f(bias)
         bias = bias.contiguous()
     shape = input.shape
-    out = HF.linear_upcast(input.reshape(-1, shape[-1]).contiguous(), lin.weight.contiguous(), scale, bias)
+    out = HF.linear_upcast(input.reshape(-1, shape[-1]).contiguous(), lin.weight.contiguous(), scale, bias,
+                           fixed_k_cut=_batch_invariant(lin))
     return out.reshape(*shape[:-1], lin.weight.shape[0])
 
 
@@ -208,12 +215,12 @@ class disable_weight_init:
             if _upcast_ready(self, input):
                 return _linear_upcast(self, input, None)
             weight, bias = cast_bias_weight(self, input)
-            return _linear_bf16(input, weight, bias)
+            return _linear_bf16(input, weight, bias, self)
 
         def forward(self, *args, **kwargs):
             if self.comfy_cast_weights or len(self.weight_function) > 0 or len(self.bias_function) > 0:
                 return self.forward_comfy_cast_weights(*args, **kwargs)
-            return _linear_bf16(args[0], self.weight, self.bias)
+            return _linear_bf16(args[0], self.weight, self.bias, self)
 
 
 class manual_cast(disable_weight_init):
@@ -275,7 +282,7 @@ class fp8_ops(manual_cast):
                 except Exception as e:
                     logging.info("Exception during fp8 op: {}".format(e))
             weight, bias = cast_bias_weight(self, input)
-            return _linear_bf16(input, weight, bias)
+            return _linear_bf16(input, weight, bias, self)
 
 
 def scaled_fp8_ops(fp8_matrix_mult=False, scale_input=False, override_dtype=None):
@@ -324,10 +331,10 @@ def scaled_fp8_ops(fp8_matrix_mult=False, scale_input=False, override_dtype=None
                     weight, bias = cast_bias_weight(self, input)
                 weight = weight.contiguous()
                 if weight.numel() < input.numel():
-                    return _linear_bf16(input, HF.scale_to_bf16(weight, scale), bias)
+                    return _linear_bf16(input, HF.scale_to_bf16(weight, scale), bias, self)
                 if weight.dtype == FP8:
                     weight = HF.scale_to_bf16(weight, _one(input.device))
-                return _linear_bf16(HF.scale_to_bf16(input.contiguous(), scale), weight, bias)
+                return _linear_bf16(HF.scale_to_bf16(input.contiguous(), scale), weight, bias, self)
 
             def convert_weight(self, weight, inplace=False, **kwargs):
                 s = self.scale_weight.to(device=weight.device, dtype=weight.dtype)

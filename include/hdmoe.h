@@ -301,6 +301,12 @@ typedef struct {
   int rows;           /* rows of the experts' segments together */
   int T;              /* rows of a when perm is set (rows == 2 T) */
   int rows_static;    /* rows of the static group, 0 = none */
+  int fixed_k_cut;    /* nonzero: no tile is cut along K. Which tiles are cut follows from the experts' segment sizes (their fp32
+                       * sums are then added up in another order, and with GELU they are activated through erff instead of the
+                       * polynomial of the other tiles), so the last bit of a row can depend on how the OTHER rows of the call
+                       * are routed. Nonzero makes a row's bytes a function of that row, its weights and the sizes only
+                       * (two Linears with GELU between them, 8 experts and a shared one, 2048 x 8192, on 128 tokens 260 -> 326 us,
+                       * 1000 tokens 313 -> 335 us, from 1500 on no more than 2 %). */
   const void* a;      /* [rows,K] in segment order, or [T,K] read through perm */
   const int32_t* perm;
   const int32_t* offsets;
@@ -392,11 +398,13 @@ typedef struct hdmoe_layer_args {
    * word to 1. A caller that caches its comparison of the values can poll the word and drop the cache. */
   int32_t* scale_check;
   /* With a few hundred to about two thousand tokens the down projection is cut along K, and which of the candidate
-   * cuts runs is chosen on the device from the experts' segment sizes (the cut that fills one round of blocks). The
-   * fp32 summation order of a row then depends on how the OTHER tokens of the batch were routed: the same token can
-   * differ in the last bit of its output between two batches. Nonzero here fixes the cut from the sizes alone (the
-   * cost model's choice), which makes every row's bytes a function of that row, its expert's weights and T only, at
-   * 2 to 10 % of the layer's time at those sizes. */
+   * cuts runs is chosen on the device from the experts' segment sizes (the cut that fills one round of blocks). With
+   * 16-bit activations (HDMOE_W_BF16, HDMOE_W_E4M3FN_UPCAST) the same holds at any T for the tiles that both contractions
+   * have left over after whole rounds over the chip. The fp32 summation order of a row then depends on how the OTHER
+   * tokens of the batch were routed: the same token can differ in the last bit of its output between two batches. Nonzero
+   * here fixes the cut from the sizes alone (the down projection's by the cost model, no tile of a last round), which
+   * makes every row's bytes a function of that row, its expert's weights and T only, at 2 to 10 % of the layer's time
+   * at those sizes (bf16 weights: 400 tokens 189 -> 211 us, 768 tokens 255 -> 280 us, from 1024 on no difference). */
   int fixed_k_cut;
 } hdmoe_layer_args;
 
