@@ -169,18 +169,22 @@ def scale_value(p, use_cache=None):
     return v
 
 
-def _linear_bf16(input, weight, bias, lin=None):
+def _linear_bf16(input, weight, bias, fixed_k_cut=False):
     shape = input.shape
     x2 = input.reshape(-1, shape[-1]).contiguous()
     # a bias is added to the fp32 accumulator before the one rounding to bf16, like F.linear's fused epilogue
-    out = HF.linear(x2, weight.contiguous(), bias=None if bias is None else bias.contiguous(), fixed_k_cut=_batch_invariant(lin))
+    out = HF.linear(x2, weight.contiguous(), bias=None if bias is None else bias.contiguous(), fixed_k_cut=fixed_k_cut)
     return out.reshape(*shape[:-1], weight.shape[0])
 
 
 def _batch_invariant(module):
     """`module.batch_invariant = True` on a Linear: its contraction is never cut along K by the number of rows, so that a row's
     bytes do not depend on which rows come with it. Not an attribute of the reference classes."""
-    return module is not None and module.__dict__.get("batch_invariant", False)
+    return module.__dict__.get("batch_invariant", False)
+
+
+def _fixed_k_cut(lin):
+    return {"fixed_k_cut": True} if _batch_invariant(lin) else {}
 
 
 def _upcast_ready(lin, input):
@@ -215,12 +219,12 @@ class disable_weight_init:
             if _upcast_ready(self, input):
                 return _linear_upcast(self, input, None)
             weight, bias = cast_bias_weight(self, input)
-            return _linear_bf16(input, weight, bias, self)
+            return _linear_bf16(input, weight, bias, **_fixed_k_cut(self))
 
         def forward(self, *args, **kwargs):
             if self.comfy_cast_weights or len(self.weight_function) > 0 or len(self.bias_function) > 0:
                 return self.forward_comfy_cast_weights(*args, **kwargs)
-            return _linear_bf16(args[0], self.weight, self.bias, self)
+            return _linear_bf16(args[0], self.weight, self.bias, **_fixed_k_cut(self))
 
 
 class manual_cast(disable_weight_init):
@@ -282,7 +286,7 @@ class fp8_ops(manual_cast):
                 except Exception as e:
                     logging.info("Exception during fp8 op: {}".format(e))
             weight, bias = cast_bias_weight(self, input)
-            return _linear_bf16(input, weight, bias, self)
+            return _linear_bf16(input, weight, bias, **_fixed_k_cut(self))
 
 
 def scaled_fp8_ops(fp8_matrix_mult=False, scale_input=False, override_dtype=None):
@@ -331,10 +335,10 @@ def scaled_fp8_ops(fp8_matrix_mult=False, scale_input=False, override_dtype=None
                     weight, bias = cast_bias_weight(self, input)
                 weight = weight.contiguous()
                 if weight.numel() < input.numel():
-                    return _linear_bf16(input, HF.scale_to_bf16(weight, scale), bias, self)
+                    return _linear_bf16(input, HF.scale_to_bf16(weight, scale), bias, **_fixed_k_cut(self))
                 if weight.dtype == FP8:
                     weight = HF.scale_to_bf16(weight, _one(input.device))
-                return _linear_bf16(HF.scale_to_bf16(input.contiguous(), scale), weight, bias, self)
+                return _linear_bf16(HF.scale_to_bf16(input.contiguous(), scale), weight, bias, **_fixed_k_cut(self))
 
             def convert_weight(self, weight, inplace=False, **kwargs):
                 s = self.scale_weight.to(device=weight.device, dtype=weight.dtype)
