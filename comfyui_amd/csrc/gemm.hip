@@ -1088,7 +1088,32 @@ int launch_grouped(const GemmArgs& args, int tile_bound, hipStream_t s, const ch
 #include "gemm4w.h"
 #include "swiglu4w.h"
 
-// rows_mean: rows of a dynamic group when the routing is even (its real size is known on the device only)
+// Bytes that the parts of tail tiles take in a launch, 0: none is cut. n_dyn groups with rows_mean rows each when the routing is
+// even (their real sizes are known on the device only), and rows_static of one more; kb: K in bytes of 16-bit activations. Whether
+// tiles may get cut: by the plan of an even routing, and of one whose experts are two standard deviations (counts are about
+// binomial) below or above it. Without dynamic groups the three are the same and the plan is known here.
+size_t g4_tail_room(int n_dyn, int rows_mean, int n_out_dyn, int kb_dyn, int rows_static, int n_out_static, int kb_static,
+                    int feat, bool w8) {
+  if (n_dyn > 0 && rows_static > 0 && kb_dyn != kb_static) return 0;   // tiles of two lengths: one cut does not even them out
+  const int kb = n_dyn > 0 ? kb_dyn : kb_static, min_pairs = w8 ? 3 : 2;
+  if (kb % (2 * BK) != 0 || kb / (2 * BK) < min_pairs) return 0;
+  size_t most = 0;
+  for (int k = n_dyn > 0 ? -1 : 1; k <= 1; ++k) {
+    long tiles = 0, padding = 0;
+    auto add = [&](int groups, int rows, int n_out) {
+      const long mt = (rows + G4_BM - 1) / G4_BM, nt = (long)groups * (n_out / feat);
+      tiles += mt * nt;
+      padding += (mt * G4_BM - rows) * nt;
+    };
+    if (n_dyn > 0) add(n_dyn, max(0, rows_mean + k * (int)(2 * sqrt((double)rows_mean))), n_out_dyn);
+    if (rows_static > 0) add(1, rows_static, n_out_static);
+    if (tiles <= 0 || tiles > 24 * HDMOE_NUM_CU) continue;             // one round of more than 24 is not worth a launch
+    const G4Tail t = g4_plan_tail((int)tiles, HDMOE_NUM_CU, kb / (2 * BK), min_pairs, (int)padding);
+    if (t.parts > 1) most = n_dyn > 0 ? G4_TAIL_BYTES : (size_t)t.parts * t.tiles * G4_BM * 256 * 4;
+  }
+  return most;
+}
+
 template <bool F16, bool W8, int EPI>
 int launch_gemm4w(GemmArgs& args, int rows_mean, hipStream_t s, const char* what) {
   constexpr int FEAT = EPI == G4_SWIGLU ? 128 : 256;
@@ -1101,27 +1126,14 @@ int launch_gemm4w(GemmArgs& args, int rows_mean, hipStream_t s, const char* what
     if (e != hipSuccess) return hdmoe_fail(HDMOE_E_LAUNCH, "%s: hipFuncSetAttribute: %s", what, hipGetErrorString(e));
     if (device >= 0) attr_set[device] = true;
   }
-  // Whether tail tiles may get cut: by the plan of an even routing, and of one whose experts are two standard deviations
-  // (counts are about binomial) below or above it. Without dynamic groups the three are the same and the plan is known here.
   if (EPI == G4_PARTIAL) args.tail = nullptr;
   if (args.tail != nullptr) {
-    bool cut = false;
-    for (int k = -1; k <= 1; ++k) {
-      int tiles = 0, padding = 0;
-      for (int g = 0; g < args.G; ++g) {
-        const GemmGroup& gg = args.g[g];
-        const int nt = gg.n_out / FEAT;
-        int rows = gg.row_end - gg.row_begin;
-        if (gg.row_begin < 0) rows = max(0, rows_mean + k * (int)(2 * sqrt((double)rows_mean)));
-        const int mt = (rows + G4_BM - 1) / G4_BM;
-        tiles += mt * nt;
-        padding += (mt * G4_BM - rows) * nt;
-        if (gg.kbytes != args.g[0].kbytes) args.tail = nullptr;   // tiles of two lengths: one cut does not even them out
-      }
-      if (tiles > 0 && tiles <= 24 * HDMOE_NUM_CU)                // one round of more than 24 is not worth a launch
-        cut = cut || g4_plan_tail(tiles, HDMOE_NUM_CU, args.g[0].kbytes / (2 * BK), W8 ? 3 : 2, padding).parts > 1;
-    }
-    if (!cut) args.tail = nullptr;
+    const GemmGroup& first = args.g[0];
+    const GemmGroup& last = args.g[args.G - 1];
+    const bool has_static = last.row_begin >= 0;   // at most one static group, the last
+    if (g4_tail_room(has_static ? args.G - 1 : args.G, rows_mean, first.n_out, first.kbytes,
+                     has_static ? last.row_end - last.row_begin : 0, last.n_out, last.kbytes, FEAT, W8) == 0)
+      args.tail = nullptr;
   }
   // one block per CU whatever the number of tiles: a block without any ends at once
   hipLaunchKernelGGL((gemm4w_kernel<F16, W8, EPI>), dim3(HDMOE_NUM_CU), dim3(G4_THREADS), G4_SMEM, s, args);
@@ -1259,6 +1271,23 @@ FormChoice pick_form(const GemmShape& sh) {
   c.form = c.tall ? FORM_TALL5 : FORM_BASE4;
   return c;
 }
+
+// Whether gate/up on 16-bit activations runs on the 4-wave kernel: what fits it, but for the three-stage ring (every segment
+// inside a 128-token tile) and the case one_round5 (hdmoe_launch_ffn_gemm).
+bool swiglu_on_g4(const GemmShape& sh) {
+  if (sh.fp8 || !sh.g4_takes) return false;
+  if (sh.w8) return true;
+  if (hdmoe_few_rows(sh.rows_dyn, sh.n_dyn, sh.rows_static) && sh.rows_static <= TileCfg<2>::BM &&
+      (sh.n_dyn <= 0 || sh.rows_dyn <= TileCfg<2>::BM / 2 * sh.n_dyn))
+    return false;
+  return !pick_form(sh).one_round5;
+}
+
+// Whether the 4-wave kernel takes contractions of these lengths (rows = 0: no such group)
+bool g4_takes_k(int rows_dyn, int kb_dyn, int rows_static, int kb_static) {
+  auto ok = [](int rows, int kb) { return rows <= 0 || (kb % (2 * BK) == 0 && kb >= 4 * BK); };
+  return ok(rows_dyn, kb_dyn) && ok(rows_static, kb_static);
+}
 }  // namespace
 
 extern "C" int hdmoe_set_kernel_form(int which, int value) {
@@ -1298,8 +1327,7 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
   shape.rows_dyn = rows_dyn; shape.n_dyn = n_dyn; shape.rows_static = shared != nullptr ? rows_static : 0;
   shape.N_dyn = N_dyn; shape.N_static = N_static;
   shape.w4_fits = true;  // settled below, once the groups are filled in
-  auto g4_takes = [&](int rows, int K) { return rows <= 0 || (K * eb % (2 * BK) == 0 && K * eb >= 4 * BK); };
-  shape.g4_takes = !fp8 && g4_takes(n_dyn > 0 ? rows_dyn : 0, K_dyn) && g4_takes(shape.rows_static, K_static);
+  shape.g4_takes = !fp8 && g4_takes_k(n_dyn > 0 ? rows_dyn : 0, K_dyn * eb, shape.rows_static, K_static * eb);
   FormChoice choice = pick_form(shape);
   const bool light = choice.light, ring16 = choice.ring16, tall = choice.tall;
   const int BM = tall || choice.one_round5 ? TileCfg<5>::BM : choice.short3 ? TileCfg<3>::BM : TileCfg<4>::BM;  // tokens per block tile of the kernel that will run
@@ -1309,7 +1337,6 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
                       gather_rows_max, K_dyn * eb);
   // few rows and 16-bit weights: the 8-wave kernels, whose forms (ring or not) give the same bytes
   const bool few_rows = !w8 && hdmoe_few_rows(shape.rows_dyn, shape.n_dyn, shape.rows_static);
-  const bool ring_size = few_rows && shape.rows_static <= TileCfg<2>::BM && (n_dyn <= 0 || rows_dyn <= TileCfg<2>::BM / 2 * n_dyn);
   GemmArgs args;
   memset(&args, 0, sizeof(args));
   if (alt != nullptr && gather_dyn != nullptr) args.alt = *alt;
@@ -1461,7 +1488,7 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
                     : launch_gemm4w<false, true, G4_PLAIN>(args, rows_mean, s, what);
     }
     if (choice.one_round5) return launch_grouped<BF16_SWIGLU, 5>(args, tile_bound, s, what);
-    if (swiglu && g4 && !ring_size) return launch_gemm4w<false, false, G4_SWIGLU>(args, rows_mean, s, what);
+    if (swiglu && g4 && swiglu_on_g4(shape)) return launch_gemm4w<false, false, G4_SWIGLU>(args, rows_mean, s, what);
     if (!swiglu && g4 && (tail != nullptr || rows_mean > 128 || rows_static > 128))
       return launch_gemm4w<false, false, G4_PLAIN>(args, rows_mean, s, what);
   }
@@ -1732,7 +1759,8 @@ int hdmoe_launch_linear_groups(const uint8_t* a_dyn, const int32_t* offsets, int
     return f16 ? launch_gemm4w<true, false, G4_GELU>(args, rows_mean, s, what)
                : launch_gemm4w<false, false, G4_GELU>(args, rows_mean, s, what);
   const int rows_all = (n_dyn > 0 ? rows_dyn : 0) + (shared != nullptr ? rows_static : 0);
-  if (g4 && act == HDMOE_ACT_NONE && (tail != nullptr || rows_all > 128 * G))
+  const bool room = tail != nullptr && g4_tail_room(n_dyn, rows_mean, N, K * 2, shared != nullptr ? rows_static : 0, N, K * 2, BN, false) > 0;
+  if (g4 && act == HDMOE_ACT_NONE && (room || rows_all > 128 * G))
     return f16 ? launch_gemm4w<true, false, G4_BIAS>(args, rows_mean, s, what)
                : launch_gemm4w<false, false, G4_BIAS>(args, rows_mean, s, what);
   // The 8-wave kernel, by the rule of the feed-forward contractions: the 320-token tile when it saves a round of tiles. A
@@ -1958,14 +1986,22 @@ int linear_groups_check(const hdmoe_linear_args* p) {
   const long rows_max = p->rows > p->rows_static ? p->rows : p->rows_static;
   return hdmoe_check_gemm_shape(what, HDMOE_W_BF16, rows_max, p->K, p->N, BN);
 }
+// what the kernels that run can use: room for the activation, and for the parts of tail tiles
 size_t linear_groups_scratch(const hdmoe_linear_args* p) {
-  return p->act == HDMOE_ACT_GELU ? hdmoe_align_up((size_t)HDMOE_NUM_CU * G4_SCRATCH, 256) : 0;
+  if (p->act != HDMOE_ACT_GELU || !g4_takes_k(1, p->K * 2, 0, 0)) return 0;
+  return hdmoe_align_up((size_t)HDMOE_NUM_CU * G4_SCRATCH, 256);
+}
+size_t linear_groups_tail(const hdmoe_linear_args* p) {
+  if (p->fixed_k_cut != 0) return 0;
+  const int n_dyn = p->rows > 0 ? p->E : 0;
+  return g4_tail_room(n_dyn, n_dyn > 0 ? p->rows / n_dyn : 0, p->N, p->K * 2, p->rows_static, p->N, p->K * 2, BN,
+                      p->weight_dtype == HDMOE_W_E4M3FN_UPCAST);
 }
 }  // namespace
 
 extern "C" size_t hdmoe_linear_groups_workspace_bytes(const hdmoe_linear_args* p) {
   if (p == nullptr || linear_groups_check(p) != HDMOE_OK) return 0;
-  return linear_groups_scratch(p) + G4_TAIL_BYTES;
+  return linear_groups_scratch(p) + linear_groups_tail(p);
 }
 
 extern "C" int hdmoe_linear_groups(const hdmoe_linear_args* p, hdmoe_stream_t stream) {
@@ -1993,7 +2029,7 @@ extern "C" int hdmoe_linear_groups(const hdmoe_linear_args* p, hdmoe_stream_t st
                                     p->shared, static_cast<uint8_t*>(p->out_static), p->K, p->N, p->act,
                                     static_cast<hipStream_t>(stream), "hdmoe_linear_groups", p->act_dtype == HDMOE_W_F16,
                                     p->perm, p->T, p->perm != nullptr ? 1 : 0, p->weight_dtype == HDMOE_W_E4M3FN_UPCAST,
-                                    ws != nullptr && p->fixed_k_cut == 0 ? reinterpret_cast<float*>(ws + sb) : nullptr,
+                                    ws != nullptr && linear_groups_tail(p) > 0 ? reinterpret_cast<float*>(ws + sb) : nullptr,
                                     ws != nullptr && sb > 0 ? ws : nullptr);
 }
 
@@ -2007,5 +2043,18 @@ extern "C" int hdmoe_tail_plan(int weight_dtype, int tiles, int K, int padding, 
   return t.parts;
 }
 
-// Bytes a feed-forward's contractions on 16-bit activations can use for the parts of tail tiles.
-size_t hdmoe_tail_bytes(int weight_dtype) { return weight_dtype == HDMOE_W_E4M3FN ? 0 : G4_TAIL_BYTES; }
+// Bytes a feed-forward's contractions on 16-bit activations can use for the parts of tail tiles: E experts of hidden width H on
+// rows_dyn rows together, one more of width Hs on rows_static. down_uncut: its down projection is not cut along K by itself.
+size_t hdmoe_tail_bytes(int weight_dtype, int rows_dyn, int E, int rows_static, int D, int H, int Hs, bool down_uncut) {
+  if (weight_dtype == HDMOE_W_E4M3FN) return 0;
+  const bool w8 = weight_dtype == HDMOE_W_E4M3FN_UPCAST;
+  const int n_dyn = rows_dyn > 0 ? E : 0, mean = n_dyn > 0 ? rows_dyn / n_dyn : 0;
+  GemmShape sh;
+  sh.swiglu = true; sh.fp8 = false; sh.split = false; sh.w8 = w8; sh.w4_fits = false;
+  sh.rows_dyn = rows_dyn; sh.n_dyn = n_dyn; sh.rows_static = rows_static;
+  sh.N_dyn = H; sh.N_static = Hs;
+  sh.g4_takes = g4_takes_k(rows_dyn, D * 2, rows_static, D * 2);
+  const size_t up = swiglu_on_g4(sh) ? g4_tail_room(n_dyn, mean, H, D * 2, rows_static, Hs, D * 2, BN / 2, w8) : 0;
+  const size_t down = down_uncut ? g4_tail_room(n_dyn, mean, D, H * 2, rows_static, D, Hs * 2, BN, w8) : 0;
+  return up > down ? up : down;
+}

@@ -12,7 +12,7 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
                           int nparts = 1, int gather_shift = 0, bool reduce = true,
                           const HdmoeSplitPlan* plan = nullptr, const HdmoeAltOperand* alt = nullptr,
                           float* tail = nullptr);
-size_t hdmoe_tail_bytes(int weight_dtype);
+size_t hdmoe_tail_bytes(int weight_dtype, int rows_dyn, int E, int rows_static, int D, int H, int Hs, bool down_uncut);
 int hdmoe_launch_combine_partials(const float* partial, long long part_stride, const HdmoeSplitPlan& plan,
                                   int rows_dyn, int n_dyn,
                                   const int32_t* offsets, int weight_dtype, const hdmoe_ffn_weights* experts,
@@ -51,6 +51,18 @@ char* hdmoe_error_buffer() {
 extern "C" int hdmoe_version(void) { return HDMOE_VERSION; }
 extern "C" const char* hdmoe_last_error(void) { return hdmoe_error_buffer(); }
 
+namespace {
+size_t layer_down_bytes(int T, int D, int H, int Hs, int E, int weight_dtype) {
+  const size_t n = (size_t)T * HDMOE_TOPK;
+  const int parts = hdmoe_down_parts((int)n, E, Hs > 0 ? T : 0, D, H, Hs, weight_dtype);
+  return parts > 1 ? (size_t)parts * (n + (Hs > 0 ? (size_t)T : 0)) * D * 4 : 0;
+}
+size_t ffn_down_bytes(int rows, int D, int H, int weight_dtype) {
+  const int parts = hdmoe_down_parts(0, 0, rows, D, 0, H, weight_dtype);
+  return parts > 1 ? hdmoe_align_up((size_t)parts * rows * D * 4, 256) : 0;
+}
+}  // namespace
+
 extern "C" int hdmoe_layer_layout_get(int T, int D, int H, int Hs, int E, int weight_dtype,
                                       hdmoe_layer_layout* out) {
   HDMOE_REQUIRE_PTR(out);
@@ -85,13 +97,14 @@ extern "C" int hdmoe_layer_layout_get(int T, int D, int H, int Hs, int E, int we
   // normalised + modulated tokens of the optional block fusion, [T,D] bf16
   out->normed = take((size_t)T * D * 2);
   // fp32 partial sums of a down projection cut along K (small token counts), [parts][2T + T][D]
-  const int parts = hdmoe_down_parts((int)n, E, Hs > 0 ? T : 0, D, H, Hs, weight_dtype);
-  // and, before it, the parts of the gate/up contraction's tail tiles (16-bit arithmetic)
-  const size_t down_bytes = parts > 1 ? (size_t)parts * (n + (Hs > 0 ? (size_t)T : 0)) * D * 4 : 0;
-  const size_t tail_bytes = T > 0 ? hdmoe_tail_bytes(weight_dtype) : 0;
-  out->partials = take(down_bytes > tail_bytes ? down_bytes : tail_bytes);
+  const size_t down_bytes = layer_down_bytes(T, D, H, Hs, E, weight_dtype);
+  out->partials = take(down_bytes);
   // one word the gate + cast kernel leaves for the gate/up GEMM: which layout of the fp8 tokens it wrote
   out->flags = take(256);
+  // the parts of tail tiles (16-bit arithmetic): in the room of the partial sums, which are written after them, or where that
+  // is too small in room of their own, which a smaller workspace may go without
+  const size_t tail_bytes = T > 0 ? hdmoe_tail_bytes(weight_dtype, (int)n, E, Hs > 0 ? T : 0, D, H, Hs, down_bytes == 0) : 0;
+  if (tail_bytes > down_bytes) take(tail_bytes);
   out->total = off;
   return HDMOE_OK;
 }
@@ -113,9 +126,10 @@ extern "C" int hdmoe_moe_ffn(const hdmoe_layer_args* p, hdmoe_stream_t stream) {
   hdmoe_layer_layout l;
   if (int rc = hdmoe_layer_layout_get(T, D, H, Hs, E, wd, &l)) return rc;
   if (Hs > 0) HDMOE_REQUIRE_PTR(p->shared);
-  if (p->workspace_bytes < l.total || (reinterpret_cast<uintptr_t>(p->workspace) & 255))
+  const size_t need = l.flags + 256;   // the parts of tail tiles may do without theirs
+  if (p->workspace_bytes < need || (reinterpret_cast<uintptr_t>(p->workspace) & 255))
     return hdmoe_fail(HDMOE_E_WORKSPACE, "hdmoe_moe_ffn: workspace %zu bytes, need %zu (256-byte aligned)",
-                      p->workspace_bytes, l.total);
+                      p->workspace_bytes, need);
   const long n = (long)T * HDMOE_TOPK;
   if (int rc = hdmoe_check_gemm_shape("hdmoe_moe_ffn (gate/up)", wd, n + T, D, H, 128)) return rc;
   if (int rc = hdmoe_check_gemm_shape("hdmoe_moe_ffn (down)", wd, n, H, D, 256)) return rc;
@@ -251,6 +265,9 @@ extern "C" int hdmoe_moe_ffn(const hdmoe_layer_args* p, hdmoe_stream_t stream) {
   }
 
   mark();
+  // room for the parts of tail tiles; cut ones make a row's summation order depend on the routing as the K cut does
+  float* const tail = fp8 || p->fixed_k_cut != 0 || p->workspace_bytes < l.total
+                          ? nullptr : reinterpret_cast<float*>(ws + (l.total > need ? need : l.partials));
   // gate/up projections + SiLU*mul, routed experts and shared expert in one launch
   // the routed operand holds one row per token (else one per flat slot); when the gate kernel decided, the
   // one-row-per-token form is described here and the other one as the alternative its flag selects
@@ -265,8 +282,7 @@ extern "C" int hdmoe_moe_ffn(const hdmoe_layer_args* p, hdmoe_stream_t stream) {
                                      a_static, Hs > 0 ? T : 0, p->shared, h_shared, D, H, D, Hs, s,
                                      "hdmoe_moe_ffn (gate/up)", perm, per_token ? T : (int)n, nullptr, 1,
                                      per_token ? 1 : 0, true, nullptr, decide ? &alt : nullptr,
-                                     // cut tail tiles make a row's summation order depend on the routing as the K cut does
-                                     fp8 || p->fixed_k_cut != 0 ? nullptr : reinterpret_cast<float*>(ws + l.partials)))
+                                     tail))
     return rc;
   mark();
   // down projections, both in one launch
@@ -281,7 +297,7 @@ extern "C" int hdmoe_moe_ffn(const hdmoe_layer_args* p, hdmoe_stream_t stream) {
                                      Hs > 0 ? T : 0, p->shared, y_shared, H, D, Hs, D, s, "hdmoe_moe_ffn (down)",
                                      nullptr, 0, parts > 1 ? reinterpret_cast<float*>(ws + l.partials) : nullptr, parts,
                                      0, /*reduce=*/false, &plan, nullptr,
-                                     fp8 || p->fixed_k_cut != 0 || parts > 1 ? nullptr : reinterpret_cast<float*>(ws + l.partials)))
+                                     parts > 1 ? nullptr : tail))
     return rc;
   mark();
   // cut along K: the combine adds the parts up itself (no launch and no bf16 copy of the rows in between)
@@ -308,9 +324,8 @@ extern "C" size_t hdmoe_ffn_workspace_bytes(int rows, int D, int H, int weight_d
   // fp8: quantised copy of x, then h; bf16: h only (x itself is the GEMM operand); then the fp32 partial sums of a
   // down projection cut along K (few rows)
   const size_t a = weight_dtype == HDMOE_W_E4M3FN ? hdmoe_align_up((size_t)rows * D * eb, 256) : 0;
-  const int parts = hdmoe_down_parts(0, 0, rows, D, 0, H, weight_dtype);
-  size_t pbytes = parts > 1 ? hdmoe_align_up((size_t)parts * rows * D * 4, 256) : 0;
-  const size_t tail_bytes = rows > 0 ? hdmoe_tail_bytes(weight_dtype) : 0;
+  size_t pbytes = ffn_down_bytes(rows, D, H, weight_dtype);
+  const size_t tail_bytes = rows > 0 ? hdmoe_tail_bytes(weight_dtype, 0, 0, rows, D, 0, H, pbytes == 0) : 0;
   if (tail_bytes > pbytes) pbytes = tail_bytes;
   return a + hdmoe_align_up((size_t)rows * H * eb, 256) + pbytes;
 }
@@ -324,12 +339,14 @@ extern "C" int hdmoe_ffn_swiglu(int weight_dtype, const void* x_bf16, int rows, 
   HDMOE_REQUIRE_PTR(workspace);
   if (int rc = hdmoe_check_gemm_shape("hdmoe_ffn_swiglu (gate/up)", weight_dtype, rows, D, H, 128)) return rc;
   if (int rc = hdmoe_check_gemm_shape("hdmoe_ffn_swiglu (down)", weight_dtype, rows, H, D, 256)) return rc;
-  const size_t need = hdmoe_ffn_workspace_bytes(rows, D, H, weight_dtype);
+  const bool fp8 = weight_dtype == HDMOE_W_E4M3FN;
+  const size_t h_off = fp8 ? hdmoe_align_up((size_t)rows * D, 256) : 0;
+  const size_t room_off = h_off + hdmoe_align_up((size_t)rows * H * (fp8 ? 1 : 2), 256);
+  const size_t need = room_off + ffn_down_bytes(rows, D, H, weight_dtype);   // the parts of tail tiles may do without
   if (workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 255))
     return hdmoe_fail(HDMOE_E_WORKSPACE, "hdmoe_ffn_swiglu: workspace %zu bytes, need %zu (256-byte aligned)",
                       workspace_bytes, need);
   if (rows == 0) return HDMOE_OK;
-  const bool fp8 = weight_dtype == HDMOE_W_E4M3FN;
   if (fp8)
     if (int rc = hdmoe_check_scale_in13("hdmoe_ffn_swiglu", *w, 0)) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -342,10 +359,10 @@ extern "C" int hdmoe_ffn_swiglu(int weight_dtype, const void* x_bf16, int rows, 
     if (int rc = hdmoe_launch_quant_rows(x_bf16, rows, D, w->scale_in1, w->scale_in3, ws, s, "hdmoe_ffn_swiglu (quantise)"))
       return rc;
     a = ws;
-    h = ws + hdmoe_align_up((size_t)rows * D, 256);
+    h = ws + h_off;
   }
-  float* const room = reinterpret_cast<float*>(h + hdmoe_align_up((size_t)rows * H * (fp8 ? 1 : 2), 256));
-  float* const tail = fp8 ? nullptr : room;
+  float* const room = reinterpret_cast<float*>(ws + room_off);
+  float* const tail = fp8 || workspace_bytes < hdmoe_ffn_workspace_bytes(rows, D, H, weight_dtype) ? nullptr : room;
   if (int rc = hdmoe_launch_ffn_gemm(true, weight_dtype, nullptr, nullptr, 0, 0, nullptr, nullptr, a, rows, w, h, 0, 0, D, H,
                                      s, "hdmoe_ffn_swiglu (gate/up)", nullptr, 0, nullptr, 1, 0, true, nullptr, nullptr, tail))
     return rc;

@@ -160,7 +160,7 @@ def _linear_groups(dt, weight_code, K, N, act, device, experts=(), a=None, perm=
         return
     ref = ctypes.byref(args)
     nbytes = lib.hdmoe_linear_groups_workspace_bytes(ref)
-    if nbytes > 0:   # 0: sizes the call below refuses
+    if nbytes > 0:   # 0: nothing of it would be used, or sizes the call below refuses
         ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
         args.workspace, args.workspace_bytes = ws.data_ptr(), nbytes
     check(lib.hdmoe_linear_groups(ref, torch.cuda.current_stream(device).cuda_stream))

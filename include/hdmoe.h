@@ -315,7 +315,7 @@ typedef struct {
   const void* a_static;
   const hdmoe_linear_group* shared;
   void* out_static;
-  void* workspace;    /* hdmoe_linear_groups_workspace_bytes(...) bytes, 256-byte aligned, or NULL */
+  void* workspace;    /* hdmoe_linear_groups_workspace_bytes(...) bytes (0 to 92 MiB: what these sizes use), 256-byte aligned, or NULL */
   size_t workspace_bytes;
 } hdmoe_linear_args;
 size_t hdmoe_linear_groups_workspace_bytes(const hdmoe_linear_args* args);
@@ -411,7 +411,10 @@ typedef struct hdmoe_layer_args {
 #define HDMOE_NUM_STAGES 6
 #define HDMOE_NUM_STAGE_EVENTS (HDMOE_NUM_STAGES + 1)
 
-/* The workspace size already includes room for the normalised tokens of the block fusion. */
+/* The workspace size already includes room for the normalised tokens of the block fusion and, with 16-bit activations and
+ * sizes whose last round of tiles is cut along K, up to 64 MiB for the parts (at the end, behind hdmoe_layer_layout.flags, unless
+ * the partial sums' room serves). A call with a smaller workspace that holds everything else is taken too: no such tile is
+ * cut then. */
 size_t hdmoe_layer_workspace_bytes(int T, int D, int H, int Hs, int E, int weight_dtype);
 int hdmoe_moe_ffn(const hdmoe_layer_args* args, hdmoe_stream_t stream);
 
@@ -419,7 +422,8 @@ int hdmoe_moe_ffn(const hdmoe_layer_args* args, hdmoe_stream_t stream);
  * feed-forward, or a block built with num_routed_experts == 0): out = w2( silu(w1 x) * w3 x ) with the same
  * per-Linear semantics as above. x [rows,D] bf16 -> out [rows,D] bf16. Three launches (fp8: quantise, gate/up GEMM
  * with the SiLU*mul epilogue, down GEMM; bf16: the two GEMMs). workspace: hdmoe_ffn_workspace_bytes(...) bytes,
- * 256-byte aligned, device. */
+ * 256-byte aligned, device; without the room for the parts of tail tiles that this may include (16-bit activations, behind h
+ * and the parts of a cut down projection) the call is taken too and cuts no such tile. */
 size_t hdmoe_ffn_workspace_bytes(int rows, int D, int H, int weight_dtype);
 int hdmoe_ffn_swiglu(int weight_dtype, const void* x_bf16, int rows, int D, int H,
                      const hdmoe_ffn_weights* w, void* out_bf16, void* workspace,
