@@ -166,8 +166,8 @@ def _linear_groups(dt, weight_code, K, N, act, device, experts=(), a=None, perm=
     check(lib.hdmoe_linear_groups(ref, torch.cuda.current_stream(device).cuda_stream))
 
 
-def _linear_group(weight, bias, K, N, what, dtype=BF16, scale=None):
-    _need_hip(weight, f"{what} weight", FP8 if scale is not None else dtype)
+def _linear_group(weight, bias, K, N, what, dtype=BF16):
+    _need_hip(weight, f"{what} weight", dtype)
     if tuple(weight.shape) != (N, K):
         raise ValueError(f"{what}: weight shape {tuple(weight.shape)} != ({N}, {K})")
     g = _lib.LinearGroup()
