@@ -342,7 +342,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   int dldo = own(0);
   bool deferred = false;
   const v4i scr = EPI == G4_GELU ? rsrc4(args.scratch + (size_t)blockIdx.x * G4_SCRATCH, G4_SCRATCH) : rsrc4(nullptr, 0);
-  const int gk = sgpr(__float_as_int(0.84932180f)), gp = sgpr(__float_as_int(0.3f / 0.84932180f));  // gen_gemm4w.py: k, 0.3 / k
+  const int gk = sgpr(__float_as_int((F16 ? 1.0f : 2.0f) * 0.84932180f)), gp = sgpr(__float_as_int(0.3f / 0.84932180f));  // gen_gemm4w.py: k (2 k), 0.3 / k
 #define G4_DRAIN(TEXT)                                                                                               \
   asm volatile(TEXT : "+{v[128:159]}"(fa0), "+{v[160:191]}"(fb0), "+{v[96:127]}"(ctx) : [dro] "s"(dro), [dldo] "s"(dldo), [dd] "s"(dd), [scr] "s"(scr), [gk] "s"(gk), [gp] "s"(gp) : G4_CLOBBER_V)
   // Output offsets of the pieces: the second pair of K steps stores the first two of token block 1, so DEF_ST starts a step in

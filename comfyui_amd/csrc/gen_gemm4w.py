@@ -130,7 +130,8 @@ def gelu_words(dt, src, dst, n):
     """gelu(x) = (x + |x|) / 2 - |x| Q(|x|) of n packed words src.. -> dst.., two values at a time in the work registers
     TMP..TMP+9: list of (instruction, cycles). No cancellation, so the negative tail keeps its digits; infinities and NaN
     come out as 0.5 x (1 + erf) has them (the legacy product takes 0 * inf as 0). |x| is carried as a = k |x|,
-    k^2 = log2(e) / 2, so that exp(-x^2 / 2) is one square and one exp2; the factor is folded into the other constants."""
+    k^2 = log2(e) / 2, so that exp(-x^2 / 2) is one square and one exp2; the factor is folded into the other constants. bf16:
+    x is halved first, x + |x| would overflow above 1.7e38 (%[gk] is 2 k there)."""
     k = (0.5 * 1.4426950408889634) ** 0.5
     c = [v / k for v in GELU_C]
     o = []
@@ -140,6 +141,8 @@ def gelu_words(dt, src, dst, n):
         def both(f, cyc=4):
             o.extend((f(i), cyc) for i in range(2))
         both(lambda i: unpack(dt, x[i], f"v{src + w}", i == 1))
+        if dt == "BF16":
+            both(lambda i: f"v_mul_f32 v{x[i]}, 0.5, v{x[i]}")
         both(lambda i: f"v_mul_f32 v{a[i]}, |v{x[i]}|, %[gk]")
         both(lambda i: f"v_fma_f32 v{d[i]}, v{a[i]}, %[gp], 1.0")
         both(lambda i: f"v_rcp_f32 v{d[i]}, v{d[i]}", 16)
@@ -153,7 +156,7 @@ def gelu_words(dt, src, dst, n):
         both(lambda i: f"v_mul_f32 v{p[i]}, v{p[i]}, v{e[i]}")
         both(lambda i: f"v_mul_legacy_f32 v{p[i]}, v{p[i]}, v{a[i]}")
         both(lambda i: f"v_add_f32 v{x[i]}, v{x[i]}, |v{x[i]}|")
-        both(lambda i: f"v_fma_f32 v{x[i]}, v{x[i]}, 0.5, -v{p[i]}")
+        both(lambda i: f"v_sub_f32 v{x[i]}, v{x[i]}, v{p[i]}" if dt == "BF16" else f"v_fma_f32 v{x[i]}, v{x[i]}, 0.5, -v{p[i]}")
         o.append((f"{PK[dt]} v{dst + w}, v{x[0]}, v{x[1]}", 4))
     return o
 
