@@ -28,17 +28,26 @@ def within(y, ref, acc, dt):
     assert bool((err <= lim).all()), float((err / lim).max())
 
 
-@pytest.mark.parametrize("rows,N,K", [
-    (1, 256, 256),          # one tile, two pairs of K steps, no middle pair; cut into as few as two
-    (255, 512, 384),        # an odd number of pairs, the last row of a tile missing
-    (257, 256, 2560),       # one row in a second m-tile; cut along K
-    (700, 2560, 2560),      # 30 tiles, cut
-    (2000, 10240, 512),     # more than one whole round of tiles and a tail
-    (66000, 256, 256),      # 258 tiles of two pairs: nothing to cut
+def planned(rows, N, K, code=0):
+    """Parts that the tail tiles of one Linear are cut into."""
+    from comfyui_amd import _lib
+    mt = -(-rows // 256)
+    return _lib.lib.hdmoe_tail_plan(code, mt * (N // 256), K, (mt * 256 - rows) * (N // 256), None, None)
+
+
+@pytest.mark.parametrize("rows,N,K,parts", [
+    (1, 256, 256, 1),          # one tile, two pairs of K steps, no middle pair: too short to be cut
+    (255, 512, 384, 1),        # an odd number of pairs, the last row of a tile missing
+    (257, 256, 2560, 10),      # one row in a second m-tile
+    (700, 2560, 2560, 4),      # 30 tiles
+    (1750, 10240, 2560, 5),    # 280 tiles: one whole round, 24 cut ones
+    (2000, 10240, 512, 1),     # 320 tiles, the second round of 64 not cut
+    (66000, 256, 256, 1),      # 258 tiles of two pairs
 ])
 @pytest.mark.parametrize("dt", [BF16, F16])
-def test_linear(dev, rows, N, K, dt):
+def test_linear(dev, rows, N, K, parts, dt):
     from comfyui_amd import functional as HF
+    assert planned(rows, N, K) == parts
     g = torch.Generator(device=dev).manual_seed(rows + K)
     a = torch.randn((rows, K), generator=g, device=dev).to(dt)
     w = (torch.randn((N, K), generator=g, device=dev) / K ** 0.5).to(dt)
@@ -49,9 +58,15 @@ def test_linear(dev, rows, N, K, dt):
         assert torch.equal(y, HF.linear(a, w, bias=bias))
 
 
-@pytest.mark.parametrize("rows,N,K", [(1, 256, 384), (300, 512, 640), (1000, 2560, 2560), (4480, 2560, 2560), (513, 1024, 4096)])
-def test_fp8_weight_in_bf16(dev, rows, N, K):
+@pytest.mark.parametrize("rows,N,K,parts", [
+    (1, 256, 384, 1), (300, 512, 640, 1),
+    (1000, 2560, 2560, 4),     # 40 tiles
+    (1750, 10240, 2560, 5),    # one whole round, 24 cut tiles
+    (4480, 2560, 2560, 1), (513, 1024, 4096, 8),
+])
+def test_fp8_weight_in_bf16(dev, rows, N, K, parts):
     from comfyui_amd import functional as HF
+    assert planned(rows, N, K, 3) == parts
     g = torch.Generator(device=dev).manual_seed(rows + K)
     a = torch.randn((rows, K), generator=g, device=dev).to(BF16)
     w, s = synth.quantize_per_tensor(torch.randn((N, K), generator=g, device=dev) * 0.02)
@@ -60,9 +75,23 @@ def test_fp8_weight_in_bf16(dev, rows, N, K):
     within(HF.linear_upcast(a, w), *reference(a, w, None), BF16)
 
 
+def test_every_fp8_code_becomes_its_bf16_value(dev):
+    """Each of the 256 codes at every place of a row's first eight (the places that one conversion handles)."""
+    from comfyui_amd import functional as HF
+    codes = torch.arange(256, dtype=torch.uint8, device=dev).view(FP8)
+    a = torch.zeros((8, 384), dtype=BF16, device=dev)
+    a[torch.arange(8), torch.arange(8)] = 1.0
+    for at in range(8):
+        w = torch.zeros((256, 384), device=dev).to(FP8)
+        w.view(torch.uint8)[:, at] = codes.view(torch.uint8)
+        y = HF.linear_upcast(a, w)[at]
+        want = codes.to(BF16)
+        assert torch.equal(torch.isnan(y), torch.isnan(want)) and torch.equal(torch.nan_to_num(y), torch.nan_to_num(want))
+
+
 @pytest.mark.parametrize("T,E,K,N", [
     (40, 8, 2048, 256),      # a few rows per expert: every tile cut
-    (1500, 8, 2048, 4096),   # ragged segments, two tiles and a part per block: activation deferred, then drained
+    (1500, 8, 2048, 4096),   # ragged segments, one or two whole tiles per block: activation deferred, hidden or drained
     (700, 5, 512, 1024),     # K too short to hide the activation behind
     (3000, 4, 2176, 2048),   # 17 pairs: one more than the deferred activation takes
 ])
@@ -141,6 +170,60 @@ def test_layer_without_fp8_matrix_multiply(dev, tokens):
     f = m.experts[1]
     d = O.error_metrics(f(xd).cpu(), f.w2(HF.silu_mul(f.w1(xd), f.w3(xd))).cpu())
     assert d["rel_rms"] <= 1e-3, d
+
+
+def ffn_reference(x, w1, w2, w3, s1, s2, s3):
+    """The feed-forward's dataflow with 64-bit sums: one rounding of every scaled sum, of silu and of the product."""
+    lin = lambda a, w, s: (a.double() @ w.double().t() * float(s.to(BF16))).to(BF16)
+    h = (torch.nn.functional.silu(lin(x, w1, s1).double()).to(BF16).double() * lin(x, w3, s3).double()).to(BF16)
+    return lin(h, w2, s2)
+
+
+def dequant_weights(dev, seed, D, H):
+    """w1, w2, w3 and scales that are far apart (a mixed-up pair is off by a factor)."""
+    g = torch.Generator(device=dev).manual_seed(seed)
+    out = [synth.quantize_per_tensor(torch.randn(s, generator=g, device=dev) * 0.02) for s in ((H, D), (D, H), (H, D))]
+    return [w for w, _ in out], [s * f for (_, s), f in zip(out, (1.0, 0.7, 2.9))]
+
+
+def test_dense_feed_forward_without_fp8_matrix_multiply_with_cut_tiles(dev):
+    """6000 rows at the model's width: 1296 gate/up tiles, the 16 left over cut along K and finished by the kernel that adds up."""
+    from comfyui_amd import _lib
+    from comfyui_amd import functional as HF
+    D, H = synth.DIM, synth.H_ROUTED
+    assert _lib.lib.hdmoe_tail_plan(_lib.W_E4M3FN_UPCAST, 24 * 54, D, 144 * 54, None, None) > 1
+    ws, ss = dequant_weights(dev, 1, D, H)
+    x = torch.randn((6000, D), generator=torch.Generator(device=dev).manual_seed(2), device=dev).to(BF16)
+    y = HF.ffn_swiglu(x, HF.make_ffn_weights(*ws, dict(zip(("scale_w1", "scale_w2", "scale_w3"), ss))), H, HF.FP8_UPCAST)
+    ref = ffn_reference(x, *ws, *ss)
+    for lo in (0, 3000, 5800):          # the last rows lie in the cut tiles
+        d = O.error_metrics(y[lo:lo + 200].cpu(), ref[lo:lo + 200].cpu())
+        assert d["rel_rms"] <= 1e-3 and d["max_over_rms"] <= 0.05, (lo, d)     # a bf16 rounding here and there falls the other way
+
+
+def test_layer_without_fp8_matrix_multiply_with_cut_tiles(dev):
+    """960 tokens at the model's width: two m-tiles per expert and four of the shared one, 544 gate/up tiles, the last 32 (of the shared
+    expert) cut in 4."""
+    from comfyui_amd import _lib
+    from comfyui_amd import functional as HF
+    D, H, Hs, E, T = synth.DIM, synth.H_ROUTED, synth.H_SHARED, 4, 960
+    assert _lib.lib.hdmoe_tail_plan(_lib.W_E4M3FN_UPCAST, 544, D, 0, None, None) == 4
+    g = torch.Generator(device=dev).manual_seed(3)
+    parts = [dequant_weights(dev, 10 + e, D, H if e < E else Hs) for e in range(E + 1)]
+    fw = [HF.make_ffn_weights(*ws, dict(zip(("scale_w1", "scale_w2", "scale_w3"), ss))) for ws, ss in parts]
+    x = torch.randn((T, D), generator=g, device=dev).to(BF16)
+    gate = (torch.randn((E, D), generator=g, device=dev) / D ** 0.5).to(BF16)
+    y, idx, w = HF.moe_ffn(x, gate, fw[:E], fw[E], H, Hs, HF.FP8_UPCAST, want_routing=True)
+    counts = torch.bincount(idx.flatten().long(), minlength=E)
+    assert bool(((counts > 256) & (counts <= 512)).all()), counts
+    terms = torch.zeros((T, 2, D), device=dev, dtype=BF16)
+    for e in range(E):
+        t, slot = (idx == e).nonzero(as_tuple=True)
+        terms[t, slot] = ffn_reference(x[t], *parts[e][0], *parts[e][1])
+    terms = (terms * w.view(T, 2, 1)).to(BF16)
+    ref = (terms[:, 0] + terms[:, 1]) + ffn_reference(x, *parts[E][0], *parts[E][1])
+    d = O.error_metrics(y.cpu(), ref.cpu())
+    assert d["rel_rms"] <= 1e-3 and d["max_over_rms"] <= 0.05, d
 
 
 @pytest.mark.parametrize("tokens", [
