@@ -39,3 +39,27 @@ def test_no_kernel_of_the_4_wave_gemm_spills(tmp_path):
                 assert int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", kernel).group(1)) == 0, name
                 assert int(re.search(r"\.vgpr_spill_count:\s+(\d+)", kernel).group(1)) == 0, name
     assert seen >= 10
+
+
+OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+
+
+@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="needs llvm-objdump")
+def test_no_fragment_of_the_8_wave_kernels_is_spilled(tmp_path):
+    """grouped_gemm_kernel keeps LDS reads in flight in v[200:255] from one statement of its fp8 loop to the next. The 320-token forms
+    spill other registers (28 and 48 accesses); a spilled fragment would be stored before it has arrived."""
+    seen = 0
+    for i, obj in enumerate(code_objects(_lib.LIB_PATH)):
+        f = tmp_path / f"{i}.o"
+        f.write_bytes(obj)
+        text = subprocess.run([OBJDUMP, "-d", str(f)], capture_output=True, text=True, check=True).stdout
+        kernel = ""
+        for line in text.splitlines():
+            head = re.match(r"[0-9a-f]+ <(\S+)>:", line)
+            if head:
+                kernel = head.group(1)
+                seen += "grouped_gemm_kernel" in kernel
+            elif "scratch_" in line and "grouped_gemm_kernel" in kernel:
+                for lo, hi in re.findall(r"\bv\[?(\d+)(?::(\d+))?\]?", line.split("//")[0]):
+                    assert int(hi or lo) < 200, (kernel, line)
+    assert seen >= 10
