@@ -75,6 +75,21 @@ def test_fp8_weight_in_bf16(dev, rows, N, K, parts):
     within(HF.linear_upcast(a, w), *reference(a, w, None), BF16)
 
 
+@pytest.mark.parametrize("rows,N,K", [(16, 2560, 2560), (4480, 2560, 2560), (7000, 2560, 4096)])
+def test_scale_on_the_sum_is_no_further_from_64_bits(dev, rows, N, K):
+    """Against the product with the unrounded scale in 64 bits: scaling the fp32 sum, and scaling the smaller operand first (rounded to
+    bf16) with the sum itself exact."""
+    from comfyui_amd import functional as HF
+    g = torch.Generator(device=dev).manual_seed(rows)
+    a = torch.randn((rows, K), generator=g, device=dev).to(BF16)
+    w, s = synth.quantize_per_tensor(torch.randn((N, K), generator=g, device=dev) * 0.02)
+    true = a.double() @ (w.double() * s.double()).t()
+    sb = s.to(BF16)
+    first = (a.double() @ (w.to(BF16) * sb).double().t()) if N < rows else ((a * sb).double() @ w.double().t())
+    far = lambda y: float((y.double() - true).norm() / true.norm())
+    assert far(HF.linear_upcast(a, w, s)) <= far(first.to(BF16))
+
+
 def test_every_fp8_code_becomes_its_bf16_value(dev):
     """Each of the 256 codes at every place of a row's first eight (the places that one conversion handles)."""
     from comfyui_amd import functional as HF
@@ -262,3 +277,38 @@ def test_dense_feed_forward_without_fp8_matrix_multiply_of_many_rows(dev):
     for lo in (0, 155_100):
         d = O.error_metrics(y[lo:lo + 300].cpu(), HF.ffn_swiglu(x[lo:lo + 300].contiguous(), fw, 6912, HF.FP8_UPCAST).cpu())
         assert d["rel_rms"] <= 1e-3, (lo, d)
+
+
+@pytest.mark.parametrize("dt", [BF16, F16])
+def test_graph_replays_with_cut_tiles_and_hidden_activation(dev, dt):
+    """Experts with GELU (deferred, drained and cut tiles) and a second Linear with cut tiles, captured once and replayed on new inputs
+    in place, with the same calls made eagerly on other data in between."""
+    from comfyui_amd import functional as HF
+    T, E, D, H = 3000, 8, 2048, 4096
+    g = torch.Generator(device=dev).manual_seed(9)
+    rnd = lambda *s: (torch.randn(s, generator=g, device=dev) / s[-1] ** 0.5).to(dt)
+    first, second = [(rnd(H, D), rnd(H)) for _ in range(E + 1)], [(rnd(D, H), rnd(D)) for _ in range(E + 1)]
+    gate = rnd(E, D)
+
+    def block(x):
+        idx, _ = HF.gate_top2(x, gate)
+        _, offsets, perm, _ = HF.dispatch(idx, E)
+        h, hs = HF.grouped_linear_tokens(x, perm, offsets, first[:E], shared=first[E], act="gelu")
+        return HF.grouped_linear(h, offsets, second[:E], a_static=hs, shared=second[E])
+    xs = [torch.randn((T, D), generator=g, device=dev).to(dt) for _ in range(4)]
+    want = [block(x) for x in xs]
+    x = xs[0].clone()
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        block(x)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            out = block(x)
+    torch.cuda.current_stream().wait_stream(s)
+    for i in (1, 2, 3, 0, 2):
+        x.copy_(xs[i])
+        graph.replay()
+        torch.cuda.synchronize()
+        other = block(xs[(i + 1) % 4])
+        assert all(torch.equal(a, b) for a, b in zip(out, want[i])) and all(torch.equal(a, b) for a, b in zip(other, want[(i + 1) % 4]))
