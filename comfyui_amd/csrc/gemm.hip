@@ -1813,7 +1813,9 @@ int hdmoe_launch_linear_bias(int weight_dtype, const uint8_t* a, int rows, int K
   gg.act = HDMOE_ACT_NONE;
   args.G = 1;
   // The 192-token tile where its rounds of tiles cost a tenth less (as expected_tile_cost counts them: rounds x (TT + 1)).
-  // 4480 rows, 2560 x 2560 with the cast in front: 180 tiles of 256 tokens on 256 CUs 39.4 us, 240 tiles of 192 tokens 37.1 us.
+  // With the cast in front, 256- against 192-token tiles, us, rows by K x N: 4480 by 2560 x 2560 37.8, 35.4 (180 and 240 tiles on 256
+  // CUs); 193 by 4096 x 2560 44.5, 39.3 and 1 by 4096 x 2560 40.6, 33.8 (fewer products of padding); 1000 by 2560 x 2560 35.8, 32.0;
+  // 2000 by 2560 x 10240 67.6, 61.6; 9000 by 2048 x 2048 62.1, 55.4; below 30 us the host is the slower one.
   auto tiles = [&](int tt) { return (rows + 64 * tt - 1) / (64 * tt) * (N / BN); };
   auto cost = [&](int tt) { return (long)((tiles(tt) + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU) * (tt + 1); };
   if (10 * cost(3) <= 9 * cost(4)) return launch_grouped<FP8_PLAIN_BIAS, 3>(args, tiles(3), s, what);

@@ -5,12 +5,15 @@
 // contraction, rounding points and LDS tile format as grouped_gemm_kernel's 16-bit modes; weights may also be e4m3fn
 // bytes (W8), converted to bf16 between LDS and the matrix cores.
 //
-// What bounds it: with every CU multiplying N(0,1) values the clock falls to 1.5-1.7 GHz, so the energy per product decides;
-// a K step of a tile takes 1.36-1.5 us then and 0.95 us (the matrix pipe full) with most CUs idle. Against the 8-wave
-// kernel with 32x32x16 MFMAs: half the fragment reads from LDS per product (128 x 128 per wave), the smaller MFMA
-// (less energy), and no barrier that drains the pipe. bf16, M x N x K, 8-wave -> this kernel: 8192 x 8192 x 8192 917 -> 690
-// us, 16384 x 13824 x 2560 964 -> 805 us, 24576 x 2048 x 8192 654 -> 537 us (1.4-1.6 PFLOP/s). What the schedule hangs
-// on: the 16 global->LDS loads of a wave and step are spread over the whole step (every 2 MFMAs: 730 us, every 6: 690 us at
+// What bounds it: the matrix pipe at a clock that falls under it. Counters, MI355X: 24576 x 2048 x 8192 in fp16 has the pipe
+// busy in 84 % of its cycles at 1.55 GHz (620 us); with e4m3fn weights, 8160 + 4080 rows by 2560, gate/up 77 % at 1.82 GHz and
+// down 68 % at 1.88 GHz; with GELU 62 % at 1.59 GHz (the vector instructions of the activation and the stores in between); a
+// last round with idle CUs (1024 tokens in bf16) 58 % at 1.93 GHz. No LDS bank conflicts, the address unit's queue full in 1 to
+// 9 % of the wave cycles. A K step of a tile takes 1.36-1.5 us with every CU multiplying N(0,1) values and 0.95 us (the matrix pipe
+// full) with most CUs idle. Against the 8-wave kernel with 32x32x16 MFMAs: half the fragment reads from LDS per product (128 x
+// 128 per wave), the smaller MFMA (less energy), and no barrier that drains the pipe. bf16, M x N x K, 8-wave -> this kernel:
+// 8192 x 8192 x 8192 917 -> 690 us, 16384 x 13824 x 2560 964 -> 805 us, 24576 x 2048 x 8192 654 -> 537 us (1.4-1.6 PFLOP/s).
+// What the schedule hangs on: the 16 global->LDS loads of a wave and step are spread over the whole step (every 2 MFMAs: 730 us, every 6: 690 us at
 // 8192^3; 4 waves times 16 lanes' worth of addresses each 16 cycles is all the address unit takes).
 // GELU, 24576 x 8192 x 2048: 846 us in the 8-wave kernel's epilogue, 682 us hidden behind the next tile's K loop (560-585 us
 // without activation; through the outputs themselves instead of a scratch buffer 732 us: the rows are written twice).
@@ -87,7 +90,9 @@ struct G4Tail { int rounds, tiles, parts; };
 
 // Costs in units of one pair of K steps (2.0 us with most of the chip idle): a part takes its share of the pairs; leaving the
 // fp32 parts and adding them up costs a second launch (9 us) and their bytes written and read again (256 KiB per part of
-// a full tile, about 6 TB/s: 0.04 pairs). A cut has to pay by a seventh. pairs: K step pairs of a tile; padding: rows that the
+// a full tile, about 6 TB/s: 0.04 pairs). A cut has to pay by a seventh. With and without cuts: Hunyuan3D block of 128 tokens
+// 260 and 326 us, 1000 tokens 313 and 335 us, 8192 tokens 1553 and 1587 us, bf16 layer of 400 tokens 188 and 211 us; the model is
+// too hopeful near the line: bf16 layer of 1024 tokens 300 and 292 us. pairs: K step pairs of a tile; padding: rows that the
 // tiles have beyond those of their segments, over all tiles.
 // Both kernels of a launch work the plan out for themselves and have to agree, so it is integers throughout: costs in 25600ths
 // of a pair (100ths, times the 256 rows of a tile).

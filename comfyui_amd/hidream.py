@@ -11,8 +11,8 @@ gate.weight (+ .scale_weight / .scale_input under scaled-fp8 operations) -- the 
 key maps and checkpoints address.
 
 MOEFeedForwardSwiGLU.forward enqueues the whole layer through ONE library call when all
-Linears share a supported storage dtype (bf16, or float8_e4m3fn with fp8 matrix multiply);
-otherwise it composes the same HIP stages per expert through the Linear modules, which
+Linears share a supported storage dtype (bf16, or float8_e4m3fn with fp8 matrix multiply or multiplied
+in bf16); otherwise it composes the same HIP stages per expert through the Linear modules, which
 needs the per-expert row counts on the host (one sync, as the reference's mask indexing).
 Inputs must be bf16 HIP tensors: there is no CPU path.
 """
@@ -376,8 +376,8 @@ class MOEFeedForwardSwiGLU(nn.Module):
     # ---- composed path -----------------------------------------------------------------
 
     def _forward_composed(self, x2, gate_w, gated_residual=None):
-        """Same stages, one expert at a time through the Linear modules (weight functions,
-        offloaded or mixed-dtype weights, dequantising scaled-fp8 Linears)."""
+        """Same stages, one expert at a time through the Linear modules (mixed-dtype weights; fp8 weights multiplied in
+        bf16 that are offloaded, patched per call, hooked, or of sizes without a kernel)."""
         E = len(self.experts)
         idx, w = HF.gate_top2(x2, gate_w)
         if getattr(self.gate, "norm_topk_prob", False):
