@@ -57,6 +57,8 @@ def _pack_ffn(ffn, x, wdt, keep):
             sw = getattr(l, "scale_weight", None)
             if sw is not None:
                 sw = sw.to(dev)
+                if sw.dtype != torch.float32 or sw.numel() != 1:
+                    return None   # the Linear itself refuses it
                 keep.append(sw)
             scales["scale_w" + name] = sw
         elif fp8:

@@ -78,3 +78,12 @@ def test_hooks_of_a_layer_run(dev):
     hook.remove()
     assert seen[-1] == -1
     assert torch.equal(m(xd), y) and float((z - y).float().norm() / y.float().norm()) <= 1e-3   # other order of fp32 sums
+
+
+def test_a_scale_that_is_no_fp32_scalar_is_not_read_as_one():
+    f = ffn()
+    x = torch.zeros((1, DIM), dtype=torch.bfloat16)
+    assert hidream._pack_ffn(f, x, hidream.HF.FP8_UPCAST, []) is not None
+    for bad in (torch.ones((), dtype=torch.bfloat16), torch.ones(2)):
+        f.w3.scale_weight = torch.nn.Parameter(bad, requires_grad=False)
+        assert hidream._pack_ffn(f, x, hidream.HF.FP8_UPCAST, []) is None
