@@ -514,6 +514,7 @@ __global__ __launch_bounds__(256) void gemm4w_tail_kernel(const GemmArgs args, i
 
 // Whether the launch fits gemm4w_kernel: whole pairs of K steps in every part, at least two of them (w8: three). Operands may
 // have any size: rows are addressed from the start of their tile; gathered ones, which are not, are under 2 GiB for every kernel.
+// Biases are read 8 and 16 bytes at a time.
 inline bool gemm4w_fits(const GemmArgs& args, bool w8) {
   if (args.G <= 0) return false;
   for (int g = 0; g < args.G; ++g) {
@@ -522,6 +523,7 @@ inline bool gemm4w_fits(const GemmArgs& args, bool w8) {
     if (args.nparts > 1)
       for (int i = 0; i < args.plan.n; ++i) parts = max(parts, args.g[g].row_begin < 0 ? args.plan.pd[i] : args.plan.ps[i]);
     if (args.g[g].kbytes % (2 * BK) != 0 || pairs / parts < (w8 ? 3 : 2) || args.g[g].kbytes / BK > 0x7fff) return false;
+    if ((reinterpret_cast<uintptr_t>(args.g[g].bias) & 7) != 0) return false;
   }
   return true;
 }

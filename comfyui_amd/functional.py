@@ -213,6 +213,12 @@ def linear_upcast_fits(K, N):
     return K % 128 == 0 and K >= 384 and N % 256 == 0
 
 
+def linear_upcast_aligned(*tensors):
+    """Whether that kernel may read these as they lie: it loads 16 bytes at a time straight into LDS. (What is not contiguous is
+    copied first, to an aligned place.)"""
+    return all(t.data_ptr() % 16 == 0 or not t.is_contiguous() for t in tensors)
+
+
 def linear_upcast(a2d, weight, scale=None, bias=None, fixed_k_cut=False):
     """bf16( (a2d . weight^T) * bf16(scale) + bias ) for bf16 a2d [rows,K] and a float8_e4m3fn weight [N,K]: the Linear
     without fp8 matrix multiply on the stored bytes (linear_upcast_fits sizes)."""
@@ -226,6 +232,10 @@ def linear_upcast(a2d, weight, scale=None, bias=None, fixed_k_cut=False):
         _need_hip(bias, "linear_upcast bias", BF16)
         if bias.shape != (N,):
             raise ValueError(f"linear_upcast: bias {tuple(bias.shape)} does not match {N} output features")
+    if not linear_upcast_aligned(a2d, weight):
+        raise ValueError("linear_upcast: activations and weight must start on a multiple of 16 bytes")
+    if bias is not None and bias.data_ptr() % 8 != 0:
+        bias = bias.clone()
     out = torch.empty((rows, N), dtype=BF16, device=a2d.device)
     g = _lib.LinearGroup(ptr(weight), ptr(bias), _scale_ptr(scale, a2d.device, "linear_upcast scale"))
     _linear_groups(BF16, _lib.W_E4M3FN_UPCAST, K, N, _lib.ACT_NONE, a2d.device, shared=g, a_static=a2d, out_static=out,

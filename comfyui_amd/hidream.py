@@ -50,6 +50,8 @@ def _pack_ffn(ffn, x, wdt, keep):
             return None   # a weight that is moved or patched per call arrives as bf16: composed per Linear
         else:
             w, _ = amd_ops.cast_bias_weight(l, x, dtype=wdt)   # offloaded weights, weight functions (LowVramPatch)
+        if upcast and not HF.linear_upcast_aligned(w, x):
+            return None
         w = w.contiguous()
         keep.append(w)
         ws.append(w)
@@ -326,7 +328,7 @@ class MOEFeedForwardSwiGLU(nn.Module):
             return None
         H = self.experts[0].w1.weight.shape[0]
         Hs = self.shared_experts.w1.weight.shape[0]
-        if got[0] == HF.FP8_UPCAST and not HF.moe_ffn_rows_fit(x.shape[0], x.shape[1], H, Hs):
+        if got[0] == HF.FP8_UPCAST and not (HF.moe_ffn_rows_fit(x.shape[0], x.shape[1], H, Hs) and HF.linear_upcast_aligned(x)):
             return None
         return (*got, H, Hs)
 

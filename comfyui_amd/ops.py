@@ -190,7 +190,8 @@ def _fixed_k_cut(lin):
 def _upcast_ready(lin, input):
     """Whether the stored fp8 weight of `lin` can be multiplied in bf16 as it stands (no cast copy of it is made)."""
     return (lin.weight.dtype == FP8 and lin.weight.device == input.device and input.dtype == BF16
-            and len(lin.weight_function) == 0 and HF.linear_upcast_fits(lin.weight.shape[1], lin.weight.shape[0]))
+            and len(lin.weight_function) == 0 and HF.linear_upcast_fits(lin.weight.shape[1], lin.weight.shape[0])
+            and HF.linear_upcast_aligned(lin.weight, input))
 
 
 def _linear_upcast(lin, input, scale):

@@ -58,7 +58,7 @@ extern "C" {
  * manual-cast Linear that stores fp8 (comfy/ops.py:107-115). The weights become bf16 (exact) on the way to the matrix
  * cores; bf16(scale_weight) (1 if NULL), which the reference multiplies onto an operand beforehand and rounds there, is
  * applied to the fp32 sum. Taken by hdmoe_moe_ffn, hdmoe_ffn_swiglu and hdmoe_linear_groups; every contraction length a
- * multiple of 128 and at least 384. scale_input is not used. */
+ * multiple of 128 and at least 384, weights and activations 16-byte aligned. scale_input is not used. */
 #define HDMOE_W_E4M3FN_UPCAST 3
 
 typedef void* hdmoe_stream_t;
@@ -290,7 +290,7 @@ int hdmoe_grouped_linear_tokens(int act_dtype, const void* x, int T, const int32
  * the fp32 sums and the error of the activation's approximation (7e-7 of the value) before the rounding to 16 bits. */
 typedef struct {
   const void* weight; /* [N,K] */
-  const void* bias;   /* [N] of act_dtype, or NULL */
+  const void* bias;   /* [N] of act_dtype, or NULL; one-byte weights: 8-byte aligned */
   const float* scale; /* HDMOE_W_E4M3FN_UPCAST: device fp32 scalar or NULL */
 } hdmoe_linear_group;
 typedef struct {

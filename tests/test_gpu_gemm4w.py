@@ -90,6 +90,22 @@ def test_scale_on_the_sum_is_no_further_from_64_bits(dev, rows, N, K):
     assert far(HF.linear_upcast(a, w, s)) <= far(first.to(BF16))
 
 
+@pytest.mark.parametrize("rows", [700, 3000])     # cut tiles (their biases are read by the second kernel), whole ones
+@pytest.mark.parametrize("dt", [BF16, F16])
+def test_bias_that_starts_anywhere(dev, rows, dt):
+    from comfyui_amd import functional as HF
+    g = torch.Generator(device=dev).manual_seed(rows)
+    a = torch.randn((rows, 2560), generator=g, device=dev).to(dt)
+    w = (torch.randn((2560, 2560), generator=g, device=dev) * 0.02).to(dt)
+    store = torch.randn(2560 + 8, generator=g, device=dev).to(dt)
+    for at in (1, 2, 4):
+        b = store[at:at + 2560]
+        within(HF.linear(a, w, bias=b), *reference(a, w, b), dt)
+    if dt == BF16:
+        w8, s = synth.quantize_per_tensor(w.float())
+        assert torch.equal(HF.linear_upcast(a, w8, s, store[1:2561]), HF.linear_upcast(a, w8, s, store[1:2561].clone()))
+
+
 def test_every_fp8_code_becomes_its_bf16_value(dev):
     """Each of the 256 codes at every place of a row's first eight (the places that one conversion handles)."""
     from comfyui_amd import functional as HF

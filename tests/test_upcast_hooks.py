@@ -87,3 +87,19 @@ def test_a_scale_that_is_no_fp32_scalar_is_not_read_as_one():
     for bad in (torch.ones((), dtype=torch.bfloat16), torch.ones(2)):
         f.w3.scale_weight = torch.nn.Parameter(bad, requires_grad=False)
         assert hidream._pack_ffn(f, x, hidream.HF.FP8_UPCAST, []) is None
+
+
+def test_what_does_not_start_on_16_bytes_is_not_loaded_as_it_lies():
+    """The kernel that multiplies stored fp8 weights in bf16 loads 16 bytes at a time into LDS; the conversion in front of the other
+    kernels, which such Linears went through before, writes aligned copies."""
+    f = ffn()
+    x = torch.zeros((2, DIM), dtype=torch.bfloat16)
+    odd = torch.zeros(DIM * DIM * 4 + 16, dtype=torch.uint8)[1:]
+    w = odd[: f.w3.weight.numel()].view(FP8).view(f.w3.weight.shape)
+    off = torch.zeros(2 * DIM + 8, dtype=torch.bfloat16)[1:2 * DIM + 1].view(2, DIM)
+    assert ops._upcast_ready(f.w3, x) and hidream._pack_ffn(f, x, hidream.HF.FP8_UPCAST, []) is not None
+    assert not ops._upcast_ready(f.w3, off) and hidream._pack_ffn(f, off, hidream.HF.FP8_UPCAST, []) is None
+    f.w3.weight = torch.nn.Parameter(w, requires_grad=False)
+    assert not ops._upcast_ready(f.w3, x) and hidream._pack_ffn(f, x, hidream.HF.FP8_UPCAST, []) is None
+    # a copy is made of what is not contiguous
+    assert hidream.HF.linear_upcast_aligned(off[:, ::2])
