@@ -369,7 +369,8 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     const int nso = sgpr(nxt.kt0() * BK), nwso = sgpr(w_start(nxt));
     const int ldo = gg.n_out * OUT_BYTES, ldo16 = sgpr(16 * ldo);
     int slot_u;   // in a scalar register for certain (the compiler drops the builtin where it finds the value uniform)
-    asm volatile("v_readfirstlane_b32 %0, %1" : "=s"(slot_u) : "v"(cur.slot()));
+    // (the wait state between a vector register's write and its readfirstlane, which the compiler does not add inside a statement)
+    asm volatile("s_nop 1\n\tv_readfirstlane_b32 %0, %1" : "=s"(slot_u) : "v"(cur.slot()));
     const bool part = EPI != G4_PARTIAL && slot_u > 0;   // of a tail tile: raw sums go to the slot's 256 KiB
     const uint8_t* const out = EPI == G4_PARTIAL
         ? reinterpret_cast<const uint8_t*>(gg.pout + (size_t)cur.part() * (size_t)args.part_stride + (size_t)cur.row0() * gg.n_out)

@@ -161,6 +161,10 @@ def gelu_words(dt, src, dst, n):
     return o
 
 
+# a resource that the compiler has just read back from a vector register's lanes may not be used by a load before 5 wait states
+DRAIN_WAIT = ["s_nop 4"]
+
+
 class Feeder:
     """Hands instructions out evenly over a number of places."""
     def __init__(self, ops, places):
@@ -318,7 +322,10 @@ def k_loop(dt, w8, gelu, bias):
     L += ["s_branch 14b"]
     if w8:
         L += ["15:"] + wswitch + ["s_mov_b32 %[wso], %[nwso]", "s_branch 16b"]
-    return L + ["12:", "s_nop 15"]
+    L += ["12:", "s_nop 15"]
+    if gelu:   # the last piece read back is there: its registers are the compiler's between two tiles
+        L.append(f"s_waitcnt vmcnt({sum(p > PIECE_LD_AT for p, _ in requests(False, True, 1))})")
+    return L
 
 
 def out_row(tt):
@@ -467,7 +474,7 @@ def generate():
     texts.append(("HDMOE_G4_FILL", reads(0, 0, False, 0)))
     texts.append(("HDMOE_G4_FILL_W8", reads(0, 0, True, 0) + ["s_waitcnt lgkmcnt(0)"] + [i for i, _ in conversions(0)]))
     for dt in ("BF16", "F16"):
-        texts.append((f"HDMOE_G4_DRAIN_{dt}", gelu_drain(dt)))
+        texts.append((f"HDMOE_G4_DRAIN_{dt}", DRAIN_WAIT + gelu_drain(dt)))
     for name, lines in texts:
         check_trans(lines)
         out.append(f"#define {name} \\")
