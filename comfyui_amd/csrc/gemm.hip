@@ -1114,32 +1114,32 @@ size_t g4_tail_room(int n_dyn, int rows_mean, int n_out_dyn, int kb_dyn, int row
   return most;
 }
 
-template <bool F16, bool W8, int EPI>
+template <G4Type TY, int EPI>
 int launch_gemm4w(GemmArgs& args, int rows_mean, hipStream_t s, const char* what) {
   constexpr int FEAT = EPI == G4_SWIGLU ? 128 : 256;
   static bool attr_set[64] = {};
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) device = -1;
   if (device < 0 || !attr_set[device]) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm4w_kernel<F16, W8, EPI>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm4w_kernel<TY, EPI>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, G4_SMEM);
     if (e != hipSuccess) return hdmoe_fail(HDMOE_E_LAUNCH, "%s: hipFuncSetAttribute: %s", what, hipGetErrorString(e));
     if (device >= 0) attr_set[device] = true;
   }
-  if (EPI == G4_PARTIAL) args.tail = nullptr;
+  if (EPI == G4_PARTIAL || TY == G4_F8) args.tail = nullptr;
   if (args.tail != nullptr) {
     const GemmGroup& first = args.g[0];
     const GemmGroup& last = args.g[args.G - 1];
     const bool has_static = last.row_begin >= 0;   // at most one static group, the last
     if (g4_tail_room(has_static ? args.G - 1 : args.G, rows_mean, first.n_out, first.kbytes,
-                     has_static ? last.row_end - last.row_begin : 0, last.n_out, last.kbytes, FEAT, W8) == 0)
+                     has_static ? last.row_end - last.row_begin : 0, last.n_out, last.kbytes, FEAT, TY == G4_W8) == 0)
       args.tail = nullptr;
   }
   // one block per CU whatever the number of tiles: a block without any ends at once
-  hipLaunchKernelGGL((gemm4w_kernel<F16, W8, EPI>), dim3(HDMOE_NUM_CU), dim3(G4_THREADS), G4_SMEM, s, args);
-  if constexpr (EPI != G4_PARTIAL) {
+  hipLaunchKernelGGL((gemm4w_kernel<TY, EPI>), dim3(HDMOE_NUM_CU), dim3(G4_THREADS), G4_SMEM, s, args);
+  if constexpr (EPI != G4_PARTIAL && TY != G4_F8) {
     if (args.tail != nullptr)
-      hipLaunchKernelGGL((gemm4w_tail_kernel<F16, W8, EPI>), dim3(4 * HDMOE_NUM_CU), dim3(256), 0, s, args, HDMOE_NUM_CU);
+      hipLaunchKernelGGL((gemm4w_tail_kernel<TY, EPI>), dim3(4 * HDMOE_NUM_CU), dim3(256), 0, s, args, HDMOE_NUM_CU);
   }
   return hdmoe_check_launch(what);
 }
@@ -1208,7 +1208,7 @@ struct GemmShape {
   int rows_dyn, n_dyn, rows_static;  // rows_static = 0: no static group
   int N_dyn, N_static;
   bool w4_fits;                      // the 4-wave kernel takes these operands (swiglu4w_fits)
-  bool g4_takes;                     // 16-bit gate/up: K is of the kind that gemm4w_kernel takes
+  bool g4_takes;                     // K is of the kind that gemm4w_kernel takes
 };
 
 // Expected tiles with evenly loaded experts, static round-robin over the CUs, and a fixed cost per tile of about one
@@ -1237,7 +1237,8 @@ bool short_tile_pays(const GemmShape& sh) {
 // light: the token blocks of a tile that hold no rows are skipped (fp8: the compiler-scheduled K loop instead of the
 // assembly loop, which multiplies padding like rows; 16-bit weights always skip them and take from this only the
 // three-stage ring).
-struct FormChoice { GemmForm form; bool light, ring16, tall, one_round5, short3; };
+// fp8_g4: an fp8 contraction without activation runs on gemm4w_kernel (cut along K or not).
+struct FormChoice { GemmForm form; bool light, ring16, tall, one_round5, short3, fp8_g4; };
 FormChoice pick_form(const GemmShape& sh) {
   const int f_light = form_of(HDMOE_FORM_LIGHT), f_4w = form_of(HDMOE_FORM_SWIGLU4W);
   const bool few_rows = hdmoe_few_rows(sh.rows_dyn, sh.n_dyn, sh.rows_static);
@@ -1252,6 +1253,13 @@ FormChoice pick_form(const GemmShape& sh) {
   // (16-bit weights: the gate/up contraction that stays with the 8-wave kernel, 2560 rows of 4 experts by 6912 features, K = 2624: 178
   // against 198 us; the down projection measured slower on the taller tile)
   c.tall = (sh.fp8 || (sh.swiglu && !sh.g4_takes)) && !sh.split && !c.light && expected_tile_cost(sh, 5) < expected_tile_cost(sh, 4);
+  // fp8 down projection on the 4-wave kernel, unless the 320-token tile saves more than a quarter of the rounds. Whole layer, 8- against
+  // 4-wave, us: cut along K 260 tokens 110, 103; 600 177, 169; 1024 226, 207; 1536 254, 240; 2000 304, 284; whole tiles 4000
+  // 537, 503; 5000 649, 624 (320-token tiles would take 0.8 of the rounds); 8000 969, 917; 2300 (0.6 of the rounds) 341, 349. The forced forms
+  // are kernels of one family with the same bytes; this one sums 128 products at a time instead of 64 (an output of 1e7 differs).
+  c.fp8_g4 = sh.fp8 && !sh.swiglu && sh.g4_takes && !c.light && f_light == HDMOE_FORM_AUTO && f_4w == HDMOE_FORM_AUTO &&
+             !(c.tall && 4 * expected_tile_cost(sh, 5) < 3 * expected_tile_cost(sh, 4));
+  if (c.fp8_g4) c.tall = false;
   c.short3 = !c.light && f_4w != HDMOE_FORM_ALWAYS && short_tile_pays(sh);
   if (c.short3) { c.tall = false; c.form = FORM_SHORT3; return c; }
   if (sh.split) { c.form = FORM_SPLIT_K; return c; }
@@ -1327,7 +1335,7 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
   shape.rows_dyn = rows_dyn; shape.n_dyn = n_dyn; shape.rows_static = shared != nullptr ? rows_static : 0;
   shape.N_dyn = N_dyn; shape.N_static = N_static;
   shape.w4_fits = true;  // settled below, once the groups are filled in
-  shape.g4_takes = !fp8 && g4_takes_k(n_dyn > 0 ? rows_dyn : 0, K_dyn * eb, shape.rows_static, K_static * eb);
+  shape.g4_takes = g4_takes_k(n_dyn > 0 ? rows_dyn : 0, K_dyn * eb, shape.rows_static, K_static * eb);
   FormChoice choice = pick_form(shape);
   const bool light = choice.light, ring16 = choice.ring16, tall = choice.tall;
   const int BM = tall || choice.one_round5 ? TileCfg<5>::BM : choice.short3 ? TileCfg<3>::BM : TileCfg<4>::BM;  // tokens per block tile of the kernel that will run
@@ -1442,10 +1450,11 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
     const bool g4 = !fp8 && !few_rows && gemm4w_fits(args, w8);
     if (w8 && !g4) return hdmoe_fail(HDMOE_E_SHAPE, "%s: K=%d / %d in %d parts does not fit the kernel for one-byte weights", what, K_dyn, K_static, nparts);
     const int rc = light ? launch_grouped<FP8_PLAIN, 2, true>(args, tb_light, s, what)
-                   : w8 ? launch_gemm4w<false, true, G4_PARTIAL>(args, rows_mean, s, what)
+                   : w8 ? launch_gemm4w<G4_W8, G4_PARTIAL>(args, rows_mean, s, what)
                    : ring16 ? launch_grouped<BF16_PLAIN, 2, true>(args, tb_light, s, what)
+                   : fp8 && choice.fp8_g4 && gemm4w_fits(args, false) ? launch_gemm4w<G4_F8, G4_PARTIAL>(args, rows_mean, s, what)
                    : fp8 ? launch_grouped<FP8_PLAIN>(args, tile_bound, s, what)
-                   : g4 ? launch_gemm4w<false, false, G4_PARTIAL>(args, rows_mean, s, what)
+                   : g4 ? launch_gemm4w<G4_BF16, G4_PARTIAL>(args, rows_mean, s, what)
                         : launch_grouped<BF16_PLAIN>(args, tile_bound, s, what);
     if (rc != HDMOE_OK) return rc;
     if (!reduce) return HDMOE_OK;  // the caller's next kernel adds the parts up (hdmoe_launch_combine_partials)
@@ -1484,14 +1493,15 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
     const bool g4 = gemm4w_fits(args, w8);
     if (w8) {
       if (!g4) return hdmoe_fail(HDMOE_E_SHAPE, "%s: K=%d / %d does not fit the kernel for one-byte weights", what, K_dyn, K_static);
-      return swiglu ? launch_gemm4w<false, true, G4_SWIGLU>(args, rows_mean, s, what)
-                    : launch_gemm4w<false, true, G4_PLAIN>(args, rows_mean, s, what);
+      return swiglu ? launch_gemm4w<G4_W8, G4_SWIGLU>(args, rows_mean, s, what)
+                    : launch_gemm4w<G4_W8, G4_PLAIN>(args, rows_mean, s, what);
     }
     if (choice.one_round5) return launch_grouped<BF16_SWIGLU, 5>(args, tile_bound, s, what);
-    if (swiglu && g4 && swiglu_on_g4(shape)) return launch_gemm4w<false, false, G4_SWIGLU>(args, rows_mean, s, what);
+    if (swiglu && g4 && swiglu_on_g4(shape)) return launch_gemm4w<G4_BF16, G4_SWIGLU>(args, rows_mean, s, what);
     if (!swiglu && g4 && (tail != nullptr || rows_mean > 128 || rows_static > 128))
-      return launch_gemm4w<false, false, G4_PLAIN>(args, rows_mean, s, what);
+      return launch_gemm4w<G4_BF16, G4_PLAIN>(args, rows_mean, s, what);
   }
+  if (choice.fp8_g4 && gemm4w_fits(args, false)) return launch_gemm4w<G4_F8, G4_PLAIN>(args, rows_mean, s, what);
   if (fp8 && swiglu) {
     long long op_bytes = (long long)(gather_dyn != nullptr ? gather_rows_max : rows_dyn) * K_dyn;
     if ((long long)rows_static * K_static > op_bytes) op_bytes = (long long)rows_static * K_static;
@@ -1542,7 +1552,7 @@ extern "C" const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E,
   sh.rows_dyn = E > 0 ? T * HDMOE_TOPK : 0; sh.n_dyn = E; sh.rows_static = Hs > 0 ? T : 0;
   sh.N_dyn = H; sh.N_static = Hs;
   const int kb = D * elem_bytes(weight_dtype);
-  sh.g4_takes = !sh.fp8 && kb % (2 * BK) == 0 && kb >= 4 * BK;
+  sh.g4_takes = kb % (2 * BK) == 0 && kb >= 4 * BK;
   sh.w4_fits = sh.fp8 && has_scale_in2 != 0 && kb % (2 * BK) == 0 && kb >= 16 * BK && H % W4_FEAT == 0 &&
                (Hs <= 0 || Hs % W4_FEAT == 0) && (long long)T * kb < (1ll << 31);
   switch (pick_form(sh).form) {
@@ -1553,7 +1563,7 @@ extern "C" const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E,
     case FORM_TALL5: return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 5>" : "grouped_gemm_kernel<BF16_SWIGLU, 5>";
     default:
       if (pick_form(sh).one_round5) return "grouped_gemm_kernel<BF16_SWIGLU, 5>";
-      if (sh.g4_takes) return "gemm4w_kernel<SWIGLU>";
+      if (!sh.fp8 && sh.g4_takes) return "gemm4w_kernel<SWIGLU>";
       return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 4>" : "grouped_gemm_kernel<BF16_SWIGLU, 4>";
   }
 }
@@ -1753,16 +1763,16 @@ int hdmoe_launch_linear_groups(const uint8_t* a_dyn, const int32_t* offsets, int
   if (w8) {
     if (!g4 || f16 || act == HDMOE_ACT_GELU)
       return hdmoe_fail(HDMOE_E_SHAPE, "%s: K=%d act=%d does not fit the kernel for one-byte weights", what, K, act);
-    return launch_gemm4w<false, true, G4_BIAS>(args, rows_mean, s, what);
+    return launch_gemm4w<G4_W8, G4_BIAS>(args, rows_mean, s, what);
   }
   if (g4 && act == HDMOE_ACT_GELU && scratch != nullptr)
-    return f16 ? launch_gemm4w<true, false, G4_GELU>(args, rows_mean, s, what)
-               : launch_gemm4w<false, false, G4_GELU>(args, rows_mean, s, what);
+    return f16 ? launch_gemm4w<G4_F16, G4_GELU>(args, rows_mean, s, what)
+               : launch_gemm4w<G4_BF16, G4_GELU>(args, rows_mean, s, what);
   const int rows_all = (n_dyn > 0 ? rows_dyn : 0) + (shared != nullptr ? rows_static : 0);
   const bool room = tail != nullptr && g4_tail_room(n_dyn, rows_mean, N, K * 2, shared != nullptr ? rows_static : 0, N, K * 2, BN, false) > 0;
   if (g4 && act == HDMOE_ACT_NONE && (room || rows_all > 128 * G))
-    return f16 ? launch_gemm4w<true, false, G4_BIAS>(args, rows_mean, s, what)
-               : launch_gemm4w<false, false, G4_BIAS>(args, rows_mean, s, what);
+    return f16 ? launch_gemm4w<G4_F16, G4_BIAS>(args, rows_mean, s, what)
+               : launch_gemm4w<G4_BF16, G4_BIAS>(args, rows_mean, s, what);
   // The 8-wave kernel, by the rule of the feed-forward contractions: the 320-token tile when it saves a round of tiles. A
   // segment is taken one standard deviation of an even routing above the mean (at a mean that is a multiple of the tile height half the
   // segments need one tile more). GELU, 8 experts on 5000 rows and one more on 2500, 2048 x 8192: 330 us on 256-token tiles, 272 on 320.
@@ -1819,6 +1829,9 @@ int hdmoe_launch_linear_bias(int weight_dtype, const uint8_t* a, int rows, int K
   auto tiles = [&](int tt) { return (rows + 64 * tt - 1) / (64 * tt) * (N / BN); };
   auto cost = [&](int tt) { return (long)((tiles(tt) + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU) * (tt + 1); };
   if (10 * cost(3) <= 9 * cost(4)) return launch_grouped<FP8_PLAIN_BIAS, 3>(args, tiles(3), s, what);
+  // Else the 4-wave kernel. Without the cast, 8- against 4-wave on 256-token tiles: 8192 by 2560 x 10240 169.8, 157.7; 3000 67.8, 65.7;
+  // 1300 36.2, 35.3; 5000 by 6912 x 2560 72.6, 68.5; 5000 by 2560 x 2560 33.8, 33.8.
+  if (gemm4w_fits(args, false)) return launch_gemm4w<G4_F8, G4_BIAS>(args, rows, s, what);
   return launch_grouped<FP8_PLAIN_BIAS>(args, tiles(4), s, what);
 }
 

@@ -1,8 +1,7 @@
-// Grouped GEMM on 16-bit activations with one wave per SIMD: the tile text of gen_gemm4w.py (256 x 256 tile, 4 waves,
-// 512 registers each).
+// Grouped GEMM with one wave per SIMD: the tile text of gen_gemm4w.py (256 x 256 tile, 4 waves, 512 registers each).
 //
 // Included by gemm.hip inside its unnamed namespace (uses GemmArgs, GemmGroup, swz, make_rsrc, lds_ptr_t). Same
-// contraction, rounding points and LDS tile format as grouped_gemm_kernel's 16-bit modes; weights may also be e4m3fn
+// contraction, rounding points and LDS tile format as grouped_gemm_kernel; with bf16 activations weights may also be e4m3fn
 // bytes (W8), converted to bf16 between LDS and the matrix cores.
 //
 // What bounds it: the matrix pipe at a clock that falls under it. Counters, MI355X: 24576 x 2048 x 8192 in fp16 has the pipe
@@ -17,6 +16,10 @@
 // 8192^3; 4 waves times 16 lanes' worth of addresses each 16 cycles is all the address unit takes).
 // GELU, 24576 x 8192 x 2048: 846 us in the 8-wave kernel's epilogue, 682 us hidden behind the next tile's K loop (560-585 us
 // without activation; through the outputs themselves instead of a scratch buffer 732 us: the rows are written twice).
+// fp8 (F8: e4m3fn activations and weights, no activation function): the same bytes and matrix cycles per K step as 16 bits, on
+// v_mfma_f32_16x16x128_f8f6f4, whose fragments of a whole step (128 registers) are refilled quadrant by quadrant. M x N x K, 8-wave
+// kernel with its assembly loop -> this one: 16384 x 13824 x 2560 511 -> 430 us (2.7 PFLOP/s), 16384 x 2560 x 6912 226 -> 213 us, 8192^3
+// 374 -> 338 us, 16384^3 3076 -> 2637 us (3.3 PFLOP/s). One K step of one tile takes 0.88 us with few rows, a launch 8 us beside its steps.
 #include "gemm4w_asm.inc"
 
 constexpr int G4_THREADS = 256;
@@ -32,6 +35,8 @@ constexpr int G4_GELU_PAIRS = 16;                 // pairs of K steps a deferred
 constexpr int G4_TAIL_MAX_PARTS = 12;
 constexpr size_t G4_TAIL_BYTES = (size_t)HDMOE_NUM_CU * G4_BM * 256 * 4;  // fp32 sums of one tile per block
 
+// Activations and weights: 16-bit alike, bf16 with e4m3fn weights that are converted, e4m3fn alike.
+enum G4Type { G4_BF16, G4_F16, G4_W8, G4_F8 };
 // What becomes of a tile's sums.
 enum G4Epi { G4_PLAIN, G4_BIAS, G4_GELU, G4_SWIGLU, G4_PARTIAL };
 
@@ -109,7 +114,7 @@ __host__ __device__ inline G4Tail g4_plan_tail(int total, int blocks, int pairs,
 }
 
 // The plan of a launch, from the segment sizes on the device; also its number of tiles.
-template <bool W8, int FEAT>
+template <G4Type TY, int FEAT>
 __device__ __forceinline__ G4Tail g4_tail_of(const GemmArgs& args, const G4Segments& seg, int blocks) {
   int total = 0, padding = 0;
   for (int g = 0; g < args.G; ++g) {
@@ -120,15 +125,17 @@ __device__ __forceinline__ G4Tail g4_tail_of(const GemmArgs& args, const G4Segme
     padding += (mt * G4_BM - (re - rb)) * nt;
   }
   if (args.tail == nullptr || total == 0) return {total / blocks, total % blocks, 1};
-  return g4_plan_tail(total, blocks, args.g[0].kbytes / (2 * BK), W8 ? 3 : 2, padding);
+  return g4_plan_tail(total, blocks, args.g[0].kbytes / (2 * BK), TY == G4_W8 ? 3 : 2, padding);
 }
 
-template <bool F16, bool W8, int EPI>
+template <G4Type TY, int EPI>
 __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm4w_kernel(const GemmArgs args) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass drops the stub of a kernel whose register operands it cannot parse
+  constexpr bool F16 = TY == G4_F16, W8 = TY == G4_W8, F8 = TY == G4_F8;
   constexpr bool SWIGLU = EPI == G4_SWIGLU;
   constexpr bool HAS_BIAS = EPI == G4_BIAS || EPI == G4_GELU;
   constexpr int FEAT = SWIGLU ? 128 : 256;
+  static_assert(!F8 || (EPI != G4_SWIGLU && EPI != G4_GELU), "fp8: plain contractions");
   constexpr int OUT_BYTES = EPI == G4_PARTIAL ? 4 : 2;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int tid = threadIdx.x;
@@ -165,7 +172,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   // caller's plan: every XCD takes its eighth of every group, longest tiles first.
   const int xcd = blockIdx.x % HDMOE_NUM_XCD, slot = blockIdx.x / HDMOE_NUM_XCD;
   const int nslots = gridDim.x / HDMOE_NUM_XCD;
-  const G4Tail tail = g4_tail_of<W8, FEAT>(args, segs, gridDim.x);
+  const G4Tail tail = g4_tail_of<TY, FEAT>(args, segs, gridDim.x);
   v4i* const table = reinterpret_cast<v4i*>(smem + G4_TABLE) + wave * G4_TABLE_ITEMS;
   auto fill_table = [&](int base) {
     const int i = base + lane;
@@ -285,10 +292,12 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
                                : rsrc64(gg.a + (size_t)d.row0() * kb, (uint32_t)d.rows_here() * (uint32_t)kb);
     s.b0 = rsrc64(gg.b0 + (size_t)d.n0() * wkb, (uint32_t)FEAT * (uint32_t)wkb);
     s.b1 = SWIGLU ? rsrc64(gg.b1 + (size_t)d.n0() * wkb, (uint32_t)FEAT * (uint32_t)wkb) : s.b0;
+    const bool by_list = gg.gather != nullptr;
+    const int shift = by_list ? gg.gather_shift : 0;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int r = j * 32 + ld_row;
-      const int row = gg.gather != nullptr ? rows[j] >> gg.gather_shift : r;
+      const int row = by_list ? rows[j] >> shift : r;
       voff[j] = r < d.rows_here() ? row * kb + ld_chunk * 16 : (int)0x80000000u;
       voff[8 + j] = ((SWIGLU ? (j >> 2) * 64 + (j & 1) * 32 : j * 32) + ld_wrow) * wkb + ld_chunk * 16;
     }
@@ -334,6 +343,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   __syncthreads();
   if constexpr (W8) asm volatile(HDMOE_G4_FILL_W8 : "={v[128:159]}"(fa0), "={v[160:191]}"(fb0), "+{v[96:127]}"(ctx) : : G4_CLOBBER_V);
+  else if constexpr (F8) asm volatile(HDMOE_G4_FILL_F8 : "={v[128:159]}"(fa0), "={v[160:191]}"(fb0), "+{v[96:127]}"(ctx) : : "memory");
   else asm volatile(HDMOE_G4_FILL : "={v[128:159]}"(fa0), "={v[160:191]}"(fb0), "+{v[96:127]}"(ctx) : : "memory");
 
   // per-tensor scales come through the scalar cache: a vector load would be waited for together with every global->LDS
@@ -341,6 +351,9 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   typedef const __attribute__((address_space(4))) float* const_float_ptr;
   auto scale = [&](const float* p) -> int {
     return sgpr(__float_as_int(p != nullptr ? hdmoe_dev_round_bf16(*(const_float_ptr)(uintptr_t)p) : 1.0f));
+  };
+  auto scale8 = [&](const float* s_in, const float* s_w) -> int {   // fp8: scale_input * scale_weight
+    return sgpr(__float_as_int((s_in != nullptr ? *(const_float_ptr)(uintptr_t)s_in : 1.0f) * *(const_float_ptr)(uintptr_t)s_w));
   };
   // GELU: the tile whose activation is still to be applied (none: an empty buffer)
   v4i dro = rsrc4(nullptr, 0);
@@ -387,7 +400,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     ctx[G4_GATHER_VOFF] = ld_row * 4;
     const bool with_bias = HAS_BIAS && gg.bias != nullptr;
     const v4i br = rsrc4(with_bias ? gg.bias + cur.n0() : nullptr, with_bias ? 512u : 0u);
-    const int sc = W8 ? scale(gg.sb0) : 0, su = W8 && SWIGLU ? scale(gg.sb1) : 0;
+    const int sc = W8 ? scale(gg.sb0) : F8 && EPI != G4_PARTIAL ? scale8(gg.s_in, gg.sb0) : 0, su = W8 && SWIGLU ? scale(gg.sb1) : 0;
     if (EPI == G4_GELU && deferred && n < G4_GELU_PAIRS) {
       drain();
       dro = rsrc4(nullptr, 0);
@@ -406,7 +419,10 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
                  : G4_CLOBBER)
 #define G4_TILE_OR_PART(LOOP, EPILOGUE)                                                                              \
     G4_TILE(LOOP "s_cmp_lg_u32 %[part], 0\ns_cbranch_scc1 41f\n" EPILOGUE "s_branch 42f\n41:\n" HDMOE_G4_EPI_PART "42:\n")
-    if constexpr (EPI == G4_GELU && F16) { G4_TILE_OR_PART(HDMOE_G4_LOOP_F16_GELU, HDMOE_G4_EPI_F16_GELU); }
+    if constexpr (F8 && EPI == G4_BIAS) { G4_TILE_OR_PART(HDMOE_G4_LOOP_F8_BIAS, HDMOE_G4_EPI_F8_BIAS); }
+    else if constexpr (F8 && EPI == G4_PARTIAL) G4_TILE(HDMOE_G4_LOOP_F8 HDMOE_G4_EPI_PARTIAL);
+    else if constexpr (F8) { G4_TILE_OR_PART(HDMOE_G4_LOOP_F8, HDMOE_G4_EPI_F8); }
+    else if constexpr (EPI == G4_GELU && F16) { G4_TILE_OR_PART(HDMOE_G4_LOOP_F16_GELU, HDMOE_G4_EPI_F16_GELU); }
     else if constexpr (EPI == G4_GELU) { G4_TILE_OR_PART(HDMOE_G4_LOOP_BF16_GELU, HDMOE_G4_EPI_BF16_GELU); }
     else if constexpr (EPI == G4_BIAS && F16) { G4_TILE_OR_PART(HDMOE_G4_LOOP_F16_BIAS, HDMOE_G4_EPI_F16_BIAS); }
     else if constexpr (EPI == G4_BIAS && W8) { G4_TILE_OR_PART(HDMOE_G4_LOOP_BF16_W8_BIAS, HDMOE_G4_EPI_BF16_W8_BIAS); }
@@ -437,14 +453,15 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
 
 // Adds the parts of the tail tiles up (in order) and finishes them as the epilogues of gen_gemm4w.py do. One thread: one
 // token, 8 consecutive features. Bound by the fp32 sums read (256 KiB per part).
-template <bool F16, bool W8, int EPI>
+template <G4Type TY, int EPI>
 __global__ __launch_bounds__(256) void gemm4w_tail_kernel(const GemmArgs args, int blocks) {
+  constexpr bool F16 = TY == G4_F16, W8 = TY == G4_W8;
   constexpr bool SWIGLU = EPI == G4_SWIGLU;
   constexpr int FEAT = SWIGLU ? 128 : 256;
   using Act = std::conditional_t<F16, HdmoeF16, HdmoeBf16>;
   const int lane = threadIdx.x & 63;
   const G4Segments seg(args, lane);
-  const G4Tail tail = g4_tail_of<W8, FEAT>(args, seg, blocks);
+  const G4Tail tail = g4_tail_of<TY, FEAT>(args, seg, blocks);
   if (tail.parts <= 1) return;
   constexpr int PER_TILE = SWIGLU ? 16 : 32;   // blocks' worth of work of a tile
   for (int item = blockIdx.x; item < tail.tiles * PER_TILE; item += gridDim.x) {

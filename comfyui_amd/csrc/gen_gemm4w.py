@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Writes gemm4w_asm.inc: the assembly of the 4-wave 16-bit GEMM (gemm4w.h). Run by the build.
+"""Writes gemm4w_asm.inc: the assembly of the 4-wave GEMM (gemm4w.h). Run by the build.
 
     python comfyui_amd/csrc/gen_gemm4w.py [output file]
 
@@ -13,6 +13,8 @@ holds the K loop and the epilogue of a tile, so that no accumulator crosses comp
 Weights of one byte (w8: e4m3fn) are loaded by the pair of K steps (128 bytes per row), read 8 bytes per lane and
 converted to bf16 on the way to the matrix cores (exact), 64 conversions beside the 128 MFMAs of a step.
 
+fp8 (F8: e4m3fn activations and weights): a K step of 128 elements is one v_mfma_f32_16x16x128_f8f6f4 deep. See step8.
+
 GELU: an epilogue leaves the rounded sums of a tile in a scratch buffer of the block's own (it stays in the caches); while
 the next tile multiplies, the wave reads them back 16 bytes per lane at a time, applies the activation and stores the
 outputs, one piece per K step behind the MFMAs.
@@ -21,6 +23,7 @@ Register map (per wave):
   a[0:255]    accumulators acc[ft][tt] = a[(8*ft + tt)*4 : +3], ft: 16 weight rows, tt: 16 tokens
   v[128:159]  token fragments of slice 0, v[160:191] weight fragments of slice 0 (4 registers each, tt / ft ascending)
   v[192:223]  token fragments of slice 1, v[224:255] weight fragments of slice 1; work registers of the epilogue
+              (F8: tt / ft 0-3 in v[128:159] / v[160:191], 4-7 in v[192:223] / v[224:255], 8 registers each)
   v[96:127]   addresses (CTX below)
   v[80:95]    row offsets of the next tile, v[72:79] row indices of the tile after the next
   v[34:71]    work registers of the K loop
@@ -55,7 +58,7 @@ STAGE = 32768                                     # bytes of one stage of the to
 W_TILE = 65536                                    # LDS: [tok 0 | tok 1 | w 0 | w 1]
 FRAG = {("a", 0): 128, ("b", 0): 160, ("a", 1): 192, ("b", 1): 224}
 MFMA = {"BF16": "v_mfma_f32_16x16x32_bf16", "F16": "v_mfma_f32_16x16x32_f16"}
-PK = {"BF16": "v_cvt_pk_bf16_f32", "F16": "v_cvt_pk_f16_f32"}
+PK = {"BF16": "v_cvt_pk_bf16_f32", "F16": "v_cvt_pk_f16_f32", "F8": "v_cvt_pk_bf16_f32"}   # F8: the outputs are bf16
 
 # positions (MFMA index within a slice) of the events of a step
 READ1_AT = 0        # slice 0: first read of slice 1
@@ -65,6 +68,13 @@ LOAD_EVERY = 6
 LAND_AT = 32        # slice 1: the next stage has landed; barrier, then the reads of slice 0 of the next step
 CVT1_AT = 26        # w8, slice 0: first conversion of slice 1
 PIECE_ST_AT, PIECE_LD_AT = 57, 60                 # GELU, slice 0
+
+
+# the same for the fp8 step (64 MFMAs)
+FREE8_AT = 16
+LOAD8_AT = 18
+LOAD8_EVERY = 3
+LAND8_AT = 44
 
 
 def quad(b):
@@ -110,7 +120,7 @@ def mfma_order():
 
 
 def unpack(dt, dst, src, hi):
-    if dt == "BF16":
+    if dt in ("BF16", "F8"):
         return f"v_and_b32 v{dst}, 0xffff0000, {src}" if hi else f"v_lshlrev_b32 v{dst}, 16, {src}"
     return f"v_cvt_f32_f16_sdwa v{dst}, {src} dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_{int(hi)}"
 
@@ -285,7 +295,80 @@ def step(dt, w8, gelu, stage, first):
     return L
 
 
+def frag8(kind, i):
+    """fp8: the 8 registers of a fragment (32 bytes per lane: its 16-byte chunks g and 4 + g, g = lane / 16)."""
+    return FRAG[(kind, i // 4)] + 8 * (i % 4)
+
+
+def reads8(stage, frags):
+    out = []
+    for kind, i in frags:
+        for h in range(2):
+            out.append(f"ds_read_b128 {quad(frag8(kind, i) + 4 * h)}, v{(TOK_ADDR if kind == 'a' else W_ADDR)[h]} "
+                       f"offset:{stage * STAGE + 2048 * i}")
+    return out
+
+
+def burst8(stage):
+    """The reads that a step out of `stage` starts from, and those it issues itself for its second half."""
+    t0, t1 = (range(4), range(4, 8)) if stage == 0 else (range(4, 8), range(4))
+    t0, t1 = [("a", t) for t in t0], [("a", t) for t in t1]
+    w0, w1 = [("b", f) for f in range(4)], [("b", f) for f in range(4, 8)]
+    return reads8(stage, [w0[0], t0[0]] + w0[1:] + t0[1:]), reads8(stage, [t1[0], w1[0], t1[1], t1[2], t1[3]] + w1[1:])
+
+
+def mfma_order8(stage):
+    """Four quadrants of 4 x 4 MFMA tiles: (w0, t0), (w0, t1), (w1, t1), (w1, t0), t0 and t1 by step parity; token blocks outermost."""
+    t0, t1 = (range(4), range(4, 8)) if stage == 0 else (range(4, 8), range(4))
+    o = []
+    for fts, tts in ((range(4), t0), (range(4), t1), (range(4, 8), t1), (range(4, 8), t0)):
+        for k, tt in enumerate(tts):
+            o += [(ft, tt) for ft in (fts if k % 2 == 0 else reversed(fts))]
+    return o
+
+
+def young8(stage):
+    """As young(): the requests that may still be out when the next step's operands are there, those of this step."""
+    return sum(LOAD8_AT + j * LOAD8_EVERY < LAND8_AT for j in range(16))
+
+
+def step8(stage, first):
+    """One fp8 K step out of `stage`: 128 bytes are one MFMA deep, so a step has no second slice to read ahead; its 64 MFMAs go in
+    quadrants instead, and the fragments of quadrants that are done are refilled from the next stage. Entry: the reads of
+    the first quadrant are in flight (burst8)."""
+    L = []
+    order = mfma_order8(stage)
+    own, nxt = burst8(stage)[1], burst8(stage ^ 1)[0]
+    ld = token_loads(stage) + weight_loads(stage, False)
+    events = {LOAD8_AT + j * LOAD8_EVERY: ld[j] for j in range(16)}
+    assert FREE8_AT <= LOAD8_AT and max(events) < 64
+    for q in range(64):
+        ft, tt = order[q]
+        if q == 0:
+            L.append("s_waitcnt lgkmcnt(0)")
+        now = events.get(q)
+        if now:
+            L.append(now[0])
+        acc = f"a[{(8 * ft + tt) * 4}:{(8 * ft + tt) * 4 + 3}]"
+        b, a = frag8("b", ft), frag8("a", tt)
+        L.append(f"v_mfma_f32_16x16x128_f8f6f4 {acc}, v[{b}:{b + 7}], v[{a}:{a + 7}], {'0' if first and stage == 0 else acc}")
+        if now:
+            L.append(now[1])
+        if q < 8:
+            L += own[2 * q:2 * q + 2]
+        if q == FREE8_AT - 1:
+            L += ["s_waitcnt lgkmcnt(0)", "s_barrier"]
+        if q == LAND8_AT - 1:
+            L += [f"s_waitcnt vmcnt({young8(stage)})", "s_barrier"]
+        if 0 <= q - LAND8_AT < 8:   # they overwrite fragments of the quadrants behind; those of the third are freed four MFMAs apart
+            L += nxt[2 * (q - LAND8_AT):2 * (q - LAND8_AT) + 2]
+    L.append("s_add_u32 %[so], %[so], 128")
+    return L
+
+
 def pair(dt, w8, gelu, first):
+    if dt == "F8":
+        return step8(0, first) + step8(1, first)
     L = []
     if gelu and not first:
         # pieces 2p, 2p + 1: the pair of K steps p (0..13) reads them back, pair p + 1 stores them (64 bytes per token each)
@@ -356,9 +439,11 @@ def epilogue(dt, w8, bias, gelu):
             for p in range(2):
                 for e in range(4):
                     v, b = w + p * 4 + e, 192 + (2 * g + p) * 4 + e
-                    if w8 and bias:
+                    if dt == "F8" and bias:   # the product is rounded before the bias is added, as the 8-wave kernel has it
+                        L += [f"v_mul_f32 v{v}, %[sc], v{v}", f"v_add_f32 v{v}, v{b}, v{v}"]
+                    elif w8 and bias:
                         L.append(f"v_fma_f32 v{v}, v{v}, %[sc], v{b}")
-                    elif w8:
+                    elif w8 or dt == "F8":
                         L.append(f"v_mul_f32 v{v}, %[sc], v{v}")
                     elif bias:
                         L.append(f"v_add_f32 v{v}, v{b}, v{v}")
@@ -475,6 +560,10 @@ def generate():
     texts.append(("HDMOE_G4_FILL_W8", reads(0, 0, True, 0) + ["s_waitcnt lgkmcnt(0)"] + [i for i, _ in conversions(0)]))
     for dt in ("BF16", "F16"):
         texts.append((f"HDMOE_G4_DRAIN_{dt}", DRAIN_WAIT + gelu_drain(dt)))
+    for bias in (False, True):
+        texts.append((f"HDMOE_G4_LOOP_F8{'_BIAS' if bias else ''}", k_loop("F8", False, False, bias)))
+        texts.append((f"HDMOE_G4_EPI_F8{'_BIAS' if bias else ''}", epilogue("F8", False, bias, False)))
+    texts.append(("HDMOE_G4_FILL_F8", burst8(0)[0]))
     for name, lines in texts:
         check_trans(lines)
         out.append(f"#define {name} \\")
