@@ -28,7 +28,8 @@ HIPCC_FLAGS = [
 
 def build(verbose=True, extra_flags=()):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-    subprocess.check_call([sys.executable, os.path.join(CSRC, "gen_gemm4w.py")])   # -> gemm4w_asm.inc
+    for script in ("gen_gemm4w.py", "gen_swiglu224.py"):   # -> *_asm.inc
+        subprocess.check_call([sys.executable, os.path.join(CSRC, script)])
     objs = []
     procs = []
     for src in SOURCES:

@@ -1087,6 +1087,7 @@ int launch_grouped(const GemmArgs& args, int tile_bound, hipStream_t s, const ch
 
 #include "gemm4w.h"
 #include "swiglu4w.h"
+#include "swiglu224.h"
 
 // Bytes that the parts of tail tiles take in a launch, 0: none is cut. n_dyn groups with rows_mean rows each when the routing is
 // even (their real sizes are known on the device only), and rows_static of one more; kb: K in bytes of 16-bit activations. Whether
@@ -1161,6 +1162,21 @@ int launch_swiglu4w(const GemmArgs& args, int tile_bound, hipStream_t s, const c
   return hdmoe_check_launch(what);
 }
 
+int launch_swiglu224(const GemmArgs& args, hipStream_t s, const char* what) {
+  static bool attr_set[64] = {};
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) device = -1;
+  if (device < 0 || !attr_set[device]) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&swiglu224_kernel),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, S224_SMEM);
+    if (e != hipSuccess) return hdmoe_fail(HDMOE_E_LAUNCH, "%s: hipFuncSetAttribute: %s", what, hipGetErrorString(e));
+    if (device >= 0) attr_set[device] = true;
+  }
+  // one block per CU whatever the number of tiles: a block without any ends at once
+  hipLaunchKernelGGL(swiglu224_kernel, dim3(HDMOE_NUM_CU), dim3(G4_THREADS), S224_SMEM, s, args);
+  return hdmoe_check_launch(what);
+}
+
 // bytes of an activation
 inline int elem_bytes(int weight_dtype) { return weight_dtype == HDMOE_W_E4M3FN ? 1 : 2; }
 
@@ -1200,6 +1216,7 @@ enum GemmForm {
   FORM_W4,         // fp8 gate/up: the 4-wave kernel (256-token tiles)
   FORM_TALL5,      // 320-token tiles
   FORM_SHORT3,     // 192-token tiles (fp8 gate/up)
+  FORM_S224,       // fp8 gate/up: the 4-wave kernel on 224-token tiles (swiglu224.h)
   FORM_BASE4       // 256-token tiles
 };
 
@@ -1208,18 +1225,20 @@ struct GemmShape {
   int rows_dyn, n_dyn, rows_static;  // rows_static = 0: no static group
   int N_dyn, N_static;
   bool w4_fits;                      // the 4-wave kernel takes these operands (swiglu4w_fits)
+  bool s224_fits;                    // the one on 224-token tiles does (swiglu224_fits)
   bool g4_takes;                     // K is of the kind that gemm4w_kernel takes
 };
 
 // Expected tiles with evenly loaded experts, static round-robin over the CUs, and a fixed cost per tile of about one
 // 32-token block: rounds x (TT + 1). The taller tile wins when it does not add a round.
-long expected_tiles(const GemmShape& sh, int tt) {
-  const int bm = 64 * tt, fpt = sh.swiglu ? BN / 2 : BN;
+long expected_tiles_of(const GemmShape& sh, int bm) {
+  const int fpt = sh.swiglu ? BN / 2 : BN;
   long tiles = 0;
   if (sh.n_dyn > 0) tiles += (long)sh.n_dyn * ((sh.rows_dyn / sh.n_dyn + bm - 1) / bm) * (sh.N_dyn / fpt);
   if (sh.rows_static > 0) tiles += (long)((sh.rows_static + bm - 1) / bm) * (sh.N_static / fpt);
   return tiles;
 }
+long expected_tiles(const GemmShape& sh, int tt) { return expected_tiles_of(sh, 64 * tt); }
 long expected_tile_cost(const GemmShape& sh, int tt) {
   return ((expected_tiles(sh, tt) + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU) * (tt + 1);
 }
@@ -1232,6 +1251,15 @@ bool short_tile_pays(const GemmShape& sh) {
   if (!sh.fp8 || !sh.swiglu || sh.split || sh.n_dyn > 0) return false;
   const long c4 = expected_tile_cost(sh, 4), c5 = expected_tile_cost(sh, 5);
   return 20 * expected_tile_cost(sh, 3) <= 17 * (c4 < c5 ? c4 : c5);
+}
+
+// The 224-token tile for fp8 gate/up: a round of it takes 3.85 units of expected_tile_cost (8192 tokens: 28.8 us, the 320-token
+// tile of 6 units 45), and half a unit goes for the last tile's activation, which nothing hides. Whole pass without and with it, us: layer of 260
+// tokens 105, 114; 350 129, 121; 512 145, 146; 600 167, 151; 1024 209, 208; 1300 229, 202; 1536 236, 226; 2300 338, 316; 4000 502, 449; 8000
+// 920, 823; 12000 1355, 1190; dense branch of 768 rows 78.5, 80.6; 1024 92, 105; 1500 115.2, 115.6; 1800 135, 123; 2048 138, 145.
+bool s224_pays(const GemmShape& sh, long other) {
+  const long rounds = (expected_tiles_of(sh, S224_BM) + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU;
+  return 77 * rounds + 10 <= 21 * other;
 }
 
 // light: the token blocks of a tile that hold no rows are skipped (fp8: the compiler-scheduled K loop instead of the
@@ -1261,6 +1289,12 @@ FormChoice pick_form(const GemmShape& sh) {
              !(c.tall && 4 * expected_tile_cost(sh, 5) < 3 * expected_tile_cost(sh, 4));
   if (c.fp8_g4) c.tall = false;
   c.short3 = !c.light && f_4w != HDMOE_FORM_ALWAYS && short_tile_pays(sh);
+  if (f_light == HDMOE_FORM_AUTO && f_4w == HDMOE_FORM_AUTO && !c.light &&
+      sh.fp8 && sh.swiglu && sh.s224_fits && s224_pays(sh, expected_tile_cost(sh, c.short3 ? 3 : c.tall ? 5 : 4))) {
+    c.tall = c.short3 = false;
+    c.form = FORM_S224;
+    return c;
+  }
   if (c.short3) { c.tall = false; c.form = FORM_SHORT3; return c; }
   if (sh.split) { c.form = FORM_SPLIT_K; return c; }
   // Light form, gate/up: with every segment inside one 128-token tile (up to 128 tokens in a top-2 layer of 4 experts)
@@ -1272,8 +1306,8 @@ FormChoice pick_form(const GemmShape& sh) {
     return c;
   }
   if (c.light) { c.form = FORM_LIGHT4; return c; }
-  // The 4-wave form of the gate/up kernel (swiglu4w.h) has the 256-token tile; it takes the launch whenever the
-  // 8-wave kernel would not use its 320-token tile (2-3 % faster there: part of its epilogue hides in the K loop).
+  // The 4-wave form of the gate/up kernel on 256-token tiles (swiglu4w.h) takes the launch where neither the 224-token nor the
+  // 320-token tile does (2-3 % faster there than the 8-wave kernel: part of its epilogue hides in the K loop).
   const bool want4w = f_4w != HDMOE_FORM_AUTO ? f_4w == HDMOE_FORM_ALWAYS : !c.tall;
   if (sh.fp8 && sh.swiglu && want4w && sh.w4_fits) { c.form = FORM_W4; return c; }
   c.form = c.tall ? FORM_TALL5 : FORM_BASE4;
@@ -1335,6 +1369,9 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
   shape.rows_dyn = rows_dyn; shape.n_dyn = n_dyn; shape.rows_static = shared != nullptr ? rows_static : 0;
   shape.N_dyn = N_dyn; shape.N_static = N_static;
   shape.w4_fits = true;  // settled below, once the groups are filled in
+  const int K_any = n_dyn > 0 ? K_dyn : K_static;
+  shape.s224_fits = fp8 && swiglu && K_any % (2 * BK) == 0 && K_any >= 16 * BK && (shape.rows_static == 0 || (K_static == K_any && shared->scale_in2 != nullptr));
+  for (int e = 0; e < n_dyn; ++e) shape.s224_fits = shape.s224_fits && experts[e].scale_in2 != nullptr;
   shape.g4_takes = g4_takes_k(n_dyn > 0 ? rows_dyn : 0, K_dyn * eb, shape.rows_static, K_static * eb);
   FormChoice choice = pick_form(shape);
   const bool light = choice.light, ring16 = choice.ring16, tall = choice.tall;
@@ -1506,7 +1543,9 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
     long long op_bytes = (long long)(gather_dyn != nullptr ? gather_rows_max : rows_dyn) * K_dyn;
     if ((long long)rows_static * K_static > op_bytes) op_bytes = (long long)rows_static * K_static;
     shape.w4_fits = swiglu4w_fits(args, op_bytes);
+    shape.s224_fits = shape.s224_fits && swiglu224_fits(args);
     choice = pick_form(shape);
+    if (choice.form == FORM_S224) return launch_swiglu224(args, s, what);
   }
   switch (choice.form) {
     case FORM_RING3: {
@@ -1553,12 +1592,14 @@ extern "C" const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E,
   sh.N_dyn = H; sh.N_static = Hs;
   const int kb = D * elem_bytes(weight_dtype);
   sh.g4_takes = kb % (2 * BK) == 0 && kb >= 4 * BK;
+  sh.s224_fits = sh.fp8 && has_scale_in2 != 0 && kb % (2 * BK) == 0 && kb >= 16 * BK && H % S224_FEAT == 0 && (Hs <= 0 || Hs % S224_FEAT == 0);
   sh.w4_fits = sh.fp8 && has_scale_in2 != 0 && kb % (2 * BK) == 0 && kb >= 16 * BK && H % W4_FEAT == 0 &&
                (Hs <= 0 || Hs % W4_FEAT == 0) && (long long)T * kb < (1ll << 31);
   switch (pick_form(sh).form) {
     case FORM_RING3: return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 2, LIGHT>" : "grouped_gemm_kernel<BF16_SWIGLU, 2, LIGHT>";
     case FORM_LIGHT4: return "grouped_gemm_kernel<FP8_SWIGLU, 4, LIGHT>";
     case FORM_W4: return "swiglu4w_kernel";
+    case FORM_S224: return "swiglu224_kernel";
     case FORM_SHORT3: return "grouped_gemm_kernel<FP8_SWIGLU, 3>";
     case FORM_TALL5: return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 5>" : "grouped_gemm_kernel<BF16_SWIGLU, 5>";
     default:
@@ -2065,7 +2106,7 @@ size_t hdmoe_tail_bytes(int weight_dtype, int rows_dyn, int E, int rows_static, 
   const bool w8 = weight_dtype == HDMOE_W_E4M3FN_UPCAST;
   const int n_dyn = rows_dyn > 0 ? E : 0, mean = n_dyn > 0 ? rows_dyn / n_dyn : 0;
   GemmShape sh;
-  sh.swiglu = true; sh.fp8 = false; sh.split = false; sh.w8 = w8; sh.w4_fits = false;
+  sh.swiglu = true; sh.fp8 = false; sh.split = false; sh.w8 = w8; sh.w4_fits = sh.s224_fits = false;
   sh.rows_dyn = rows_dyn; sh.n_dyn = n_dyn; sh.rows_static = rows_static;
   sh.N_dyn = H; sh.N_static = Hs;
   sh.g4_takes = g4_takes_k(rows_dyn, D * 2, rows_static, D * 2);

@@ -69,13 +69,13 @@ const char* hdmoe_last_error(void);
 /* Kernel-form switches. No counterpart in the reference: both choose between kernels of this library whose results are
  * the same bit for bit, for tests that compare the forms and for measurements. Process-wide; a call in flight on
  * another thread sees the old or the new value. A HIP graph keeps the kernels that were captured. Where both are AUTO,
- * the fp8 down projection may run on a kernel outside of that family, with sums of 128 products where these have 64: about
+ * the fp8 contractions may run on kernels outside of that family, with sums of 128 products where these have 64: about
  * one output in 10^7 then differs from the forced forms' by a rounding.
  *   HDMOE_FORM_SWIGLU4W: the fp8 gate/up contraction has an 8-wave kernel (256- or 320-token tiles) and a 4-wave one
  *     (one wave per SIMD, 256-token tiles, a tile's SiLU*mul epilogue issued between the MFMAs of the next tile; needs
- *     K a multiple of 256 and at least 2048, and scale_in2). AUTO: the 4-wave kernel runs where the 320-token tile
- *     would not be used (up to about 5000 tokens for HiDream's sizes; it is 2-3 % faster there and 1-2 % slower
- *     above). NEVER / ALWAYS (whenever the shapes allow).
+ *     K a multiple of 256 and at least 2048, and scale_in2). AUTO: the 4-wave kernel runs where neither the kernel on
+ *     224-token tiles (most sizes above 256 tokens) nor the 320-token tile would be used. NEVER / ALWAYS (whenever the
+ *     shapes allow).
  *   HDMOE_FORM_LIGHT: the 8-wave kernels (gate/up and down) have a form whose K loop skips the 32-token blocks of a
  *     tile that hold no rows. AUTO: it runs when every segment is one tile and the experts' tiles are half empty on
  *     average (rows per expert <= 128 and shared rows <= 256: up to 256 tokens for HiDream's sizes; 3-12 % faster

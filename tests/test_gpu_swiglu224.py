@@ -1,0 +1,105 @@
+"""The fp8 gate/up kernel on 224-token tiles (csrc/swiglu224.h) against the 8-wave kernel (csrc/gemm.hip, forced by
+hdmoe_set_kernel_form), the same contraction and rounding points. Its matrix instruction adds 128 products where the other's adds
+64, so an fp32 sum may differ in its last bit and, where that falls on a rounding to bf16 and then on one to e4m3fn, a byte by one code."""
+import pytest
+import torch
+
+from comfyui_amd import _lib, functional as HF, synth
+from tests.helpers import saved_forms, set_form, small_layer
+
+pytestmark = pytest.mark.gpu
+FP8 = torch.float8_e4m3fn
+
+
+@pytest.fixture
+def forms():
+    yield from saved_forms()
+
+
+def codes(h):
+    """e4m3fn bytes as integers in the order of their values."""
+    b = h.view(torch.uint8).to(torch.int16)
+    return torch.where(b >= 128, -(b - 128), b)
+
+
+def assert_alike(base, new):
+    d = (codes(base) - codes(new)).abs()
+    assert int(d.max()) <= 1 and float((d > 0).float().mean()) < 1e-5, (int(d.max()), float((d > 0).float().mean()))
+
+
+@pytest.mark.parametrize("sizes,D,H,s_next", [
+    ((224,), 2048, 128, 1.0),                # one full tile, the fewest K steps the kernel takes (8 pairs: 7 written out, 1 in the loop)
+    ((226,), 2304, 256, 0.5),                # two rows in the last tile; a scale for the consuming Linear that is not 1
+    ((447, 449), 2560, 384, 0.37),           # one row less than two tiles, one more
+    ((1, 0, 700, 2299), 2560, 1024, 1.0),    # empty and nearly empty segments
+    ((1500, 1500), 6912, 256, 0.25),         # 27 pairs of K steps
+    ((8192,), 2048, 57600, 2.0),             # 65 tiles for some blocks: the tables of work are filled a second time
+])
+def test_grouped_swiglu(dev, forms, sizes, D, H, s_next):
+    g = torch.Generator(device=dev).manual_seed(sum(sizes) + H)
+    E, rows = len(sizes), sum(sizes)
+    a = torch.randn((rows, D), generator=g, device=dev).to(FP8)
+    offsets = torch.tensor([0] + list(torch.tensor(sizes).cumsum(0)), dtype=torch.int32, device=dev)
+    ws = [[(torch.randn((H, D), generator=g, device=dev) * 40).to(FP8) for _ in range(2)] for _ in range(E)]
+    scales = torch.tensor([[0.0006 + 0.0001 * e, 0.0008] for e in range(E)], device=dev)
+    s_in, s_nx = torch.tensor(1.0, device=dev), torch.tensor(s_next, device=dev)
+    arr = (_lib.FfnWeights * E)()
+    for e in range(E):
+        arr[e].w1, arr[e].w3 = ws[e][0].data_ptr(), ws[e][1].data_ptr()
+        arr[e].scale_w1, arr[e].scale_w3 = scales[e, 0:].data_ptr(), scales[e, 1:].data_ptr()
+        arr[e].scale_in1 = arr[e].scale_in3 = s_in.data_ptr()
+        arr[e].scale_in2 = s_nx.data_ptr()
+    out = []
+    for form in ("0", None):
+        set_form("HDMOE_SWIGLU4W", form)
+        h = torch.full((rows + 1, H), 0x55, dtype=torch.uint8, device=dev)
+        _lib.check(_lib.lib.hdmoe_grouped_swiglu(_lib.W_E4M3FN, a.data_ptr(), offsets.data_ptr(), rows, E, D, H, arr, h.data_ptr(), None))
+        torch.cuda.synchronize()
+        assert bool((h[rows] == 0x55).all())
+        out.append(h[:rows])
+    assert not bool((out[1] == 0x55).all())
+    assert_alike(*out)
+
+
+@pytest.mark.parametrize("same_scale", [True, False])
+def test_layer(dev, forms, same_scale):
+    """Rows gathered through the dispatch permutation, shared expert in the same launch; with a scale_input per expert the gate kernel
+    writes a row per slot and the kernel reads the alternative operand."""
+    dim = 2048
+    sd, x = small_layer(seed=93, dim=dim, tokens=1300, weights="fp8", scale_in=0.5)
+    m = synth.build_module({k: v.to(dev) for k, v in sd.items()}, "fp8", dev, dim=dim)
+    if not same_scale:
+        for i, f in enumerate(m.experts):
+            for lin in (f.w1, f.w3):
+                lin.scale_input.data.fill_(0.3 + 0.1 * i)
+    widths = m.experts[0].w1.weight.shape[0], m.shared_experts.w1.weight.shape[0]
+    assert _lib.lib.hdmoe_gate_up_kernel_name(_lib.W_E4M3FN, 1300, 4, dim, *widths, 1) == b"swiglu224_kernel"
+    y = m(x.to(dev))
+    set_form("HDMOE_LIGHT", "0")     # any forced form keeps to the 8-wave kernels
+    base = m(x.to(dev))
+    err = (y.double() - base.double()).norm() / base.double().norm()
+    assert bool(torch.isfinite(y.float()).all()) and float(err) < 1e-4, float(err)
+
+
+def test_graph_replays(dev, forms):
+    dim = 2048
+    sd, x = small_layer(seed=17, dim=dim, tokens=1300, weights="fp8")
+    m = synth.build_module({k: v.to(dev) for k, v in sd.items()}, "fp8", dev, dim=dim)
+    xs = [x.to(dev), (x * 0.5).to(dev), x.flip(1).contiguous().to(dev)]
+    eager = [m(v).clone() for v in xs]
+    static_x = xs[0].clone()
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        m(static_x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        static_y = m(static_x)
+    for _ in range(2):
+        for v, want in zip(xs, eager):
+            static_x.copy_(v)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(static_y, want)
+            assert torch.equal(m(v), want)
