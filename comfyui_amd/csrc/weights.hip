@@ -7,8 +7,6 @@
 // in [0,1)), magnitudes of 448 and more saturate to +-448, zero stays zero. The uniform numbers are not torch's:
 // element i takes word (i & 3) of Philox4x32-10(counter = i >> 2, key = seed), 24 bits of it, so the result depends
 // only on (value, seed, i).
-#include <hip/hip_fp16.h>
-
 #include "common.h"
 #include "numfmt.h"
 #include "philox.h"
@@ -19,22 +17,55 @@ constexpr int THREADS = 256;
 constexpr int GROUPS = 4;                       // groups of 4 elements per thread, THREADS apart
 constexpr long CHUNK = (long)THREADS * GROUPS;  // groups per block
 
-// What bounds the kernel: vector instructions (18 32 x 32 -> 64 bit products and 50 other operations for the random words of 4
-// elements, about 25 per element beside them): 24 us where the bytes take 14 us at 6.4 TB/s. Hence no branches per element, a division
-// by the one divisor that multiplies by its reciprocal, and all loads of a thread (16 or 8 bytes each) in flight at once.
-// 6912 x 2560 fp32 on MI355X, whole set_weight: 37.9 us with the general division, branches, element loads and a copy of the
-// result into the weight; 24.4 us.
+// What bounds the kernel: vector instructions (18 32 x 32 -> 64 bit products, which are the larger half of the time, and 18 other
+// operations for the random words of 4 elements, about 22 per element beside them; the bytes take 14 us at 6.4 TB/s). Hence no branches per element, one product
+// where the division's last bits cannot matter, the rounding on float16 bits, two values to a register where the instruction set
+// has it, and all loads of a thread (16 or 8 bytes each) in flight at once. 6912 x 2560 fp32 on MI355X, whole set_weight: 24.4 us with a
+// corrected division and fp32 arithmetic for every element, 19.8 us so; bf16 30.0 -> 21.7.
 
-// |value| already rounded to float16 (as fp32), one 32-bit random word -> e4m3fn code without sign
-__device__ __forceinline__ uint32_t sr_code(float a, uint32_t rnd) {
-  const float u = (float)(rnd >> 8) * 0x1p-24f;
-  const int e = max((int)(__float_as_uint(a) >> 23), 120);  // biased exponent; 120: everything below the smallest normal, 2^-6
-  // normal binade 2^(e-127) * (1 + k/8): position in eighths, counted from the binade's start; below: steps of 2^-9
-  const float scaled = a * __uint_as_float((uint32_t)(257 - max(e, 121)) << 23);
-  const float pos = e > 120 ? scaled - 8.0f : scaled;                  // exact
-  uint32_t code = ((uint32_t)(e - 120) << 3) + (uint32_t)(pos + u);     // 0..8, 8 carries into the next binade
-  code = a < 448.0f ? code : 0x7eu;                                    // 448 and beyond (inf too) saturate
-  return a != a ? 0x7fu : code;
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+// two values rounded to float16 (to nearest even)
+__device__ __forceinline__ uint32_t half_pair(float a, float b) {
+  const f32x2 v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2));
+}
+__device__ __forceinline__ u16x2 pk(uint32_t v) { return __builtin_bit_cast(u16x2, v); }
+
+// Four values in float16 (packed pairs), four random words -> four e4m3fn bytes.
+// Normal binades: a float16's exponent and mantissa are the code's with 7 more bits, so the sum of mantissa and u (in 128ths of a step)
+// carries into the code by itself. Below 2^-6: steps of 2^-9 from zero. The sum is rounded to fp32 once.
+__device__ __forceinline__ uint32_t sr_bytes(const uint32_t (&w)[2], const uint32_t (&rnd)[4]) {
+  u16x2 code[2], odd = {0, 0};
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const uint32_t mag = w[p] & 0x7fff7fffu, mant = w[p] & 0x03ff03ffu;
+    odd = __builtin_elementwise_max(odd, pk(mag) - pk(0x00010001u));      // zeros and NaN: 0x7c00 and above
+    uint32_t sum[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float a = (float)__builtin_bit_cast(f16x2, mag)[h];
+      const float m = (float)(h ? mant >> 16 : mant & 0xffffu);
+      const float t = a < 0x1p-6f ? a * 65536.0f : m;
+      sum[h] = (uint32_t)__builtin_fmaf((float)(rnd[2 * p + h] >> 8), 0x1p-17f, t);   // up to 1152
+    }
+    const u16x2 expo = __builtin_elementwise_max(pk(w[p] & 0x7c007c00u), pk(0x20002000u)) - pk(0x20002000u);
+    code[p] = __builtin_elementwise_min((expo + pk(sum[0] | sum[1] << 16)) >> 7, pk(0x007e007eu));   // 448 and beyond (inf too) saturate
+  }
+  uint32_t codes = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, code[1]), __builtin_bit_cast(uint32_t, code[0]), 0x06040200u);
+  uint32_t signs = __builtin_amdgcn_perm(w[1], w[0], 0x07050301u) & 0x80808080u;
+  if (__any(max(odd.x, odd.y) >= 0x7c00)) {   // somewhere in the wave
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t mag = (j & 1 ? w[j >> 1] >> 16 : w[j >> 1]) & 0x7fffu;
+      if (mag > 0x7c00u) codes |= 0x7fu << (8 * j);
+      // a zero becomes +0 (the reference multiplies by sign(0) = 0); a value rounded down to zero keeps its sign
+      if (mag == 0) signs &= ~(0x80u << (8 * j));
+    }
+  }
+  return codes | signs;
 }
 
 // Division of many values by one divisor, with the bits of a correctly rounded division wherever the float16 or bf16 rounding
@@ -42,6 +73,8 @@ __device__ __forceinline__ uint32_t sr_code(float a, uint32_t rnd) {
 // last place, RN(q + RN(x - q s) y) is RN(x / s); the first product may be off by more, so the step is taken twice).
 // Needs the remainders exact: |s| in [2^-40, 2^40]; a quotient below 2^-50 may lose digits and is 0 in float16 either way;
 // one of 2^20 or more is kept as the plain product (it saturates, and infinities and NaN pass unharmed).
+// The plain product and the correctly rounded quotient are both within 0.75 * 2^-22 of the product: where the ends of an interval of twice that
+// round to the same number, so do they (rounding is monotonic). That settles all but one in 1300 values.
 template <bool ANY_DIVISOR>
 struct Divider {
   float s, y;
@@ -91,18 +124,34 @@ __device__ __forceinline__ void round_groups(const Raw4<SRC> (&raw)[GROUPS], lon
     const uint32_t ctr[4] = {(uint32_t)g, ctr1, 0u, 0u};
     uint32_t r[4];
     hdmoe_philox4x32_10(ctr, key, r);
-    uint32_t packed = 0;
+    float x[4];
+    uint32_t w[2];
+    bool settled = !ANY_DIVISOR;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      float q;
-      if constexpr (BF16) q = hdmoe_round_bf16(div(hdmoe_bf16_to_f32(raw[i].v[j])));
-      else q = div(raw[i].v[j]);
-      const float x = __half2float(__float2half_rn(q));
-      // an exact zero stays +0 (the reference multiplies by sign(0) = 0); a value rounded down to zero keeps its sign
-      const uint32_t code = sr_code(__builtin_fabsf(x), r[j]);
-      const uint32_t sign = x != 0.0f ? (__float_as_uint(x) >> 24) & 0x80u : 0u;
-      packed |= (code | sign) << (8 * j);
+      if constexpr (BF16) x[j] = hdmoe_bf16_to_f32(raw[i].v[j]);
+      else x[j] = raw[i].v[j];
     }
+    // two values in the format the quotient is rounded to first: bf16 for bf16 weights
+    auto pair = [](float a, float b) { return BF16 ? hdmoe_dev_pack_bf16(a, b) : half_pair(a, b); };
+    if constexpr (!ANY_DIVISOR) {
+      constexpr float LOW = 1.0f - 0x1.8p-22f, HIGH = 1.0f + 0x1.8p-22f;
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const float a = x[2 * p] * div.y, b = x[2 * p + 1] * div.y;
+        w[p] = pair(a * LOW, b * LOW);
+        settled = settled && w[p] == pair(a * HIGH, b * HIGH);
+      }
+    }
+    if (!__all(settled)) {
+#pragma unroll
+      for (int p = 0; p < 2; ++p) w[p] = pair(div(x[2 * p]), div(x[2 * p + 1]));
+    }
+    if constexpr (BF16) {
+#pragma unroll
+      for (int p = 0; p < 2; ++p) w[p] = half_pair(__uint_as_float(w[p] << 16), __uint_as_float(w[p] & 0xffff0000u));
+    }
+    const uint32_t packed = sr_bytes(w, r);
     if (g * 4 + 3 < n) {
       *reinterpret_cast<uint32_t*>(out + g * 4) = packed;
     } else {

@@ -119,3 +119,14 @@ def test_bad_arguments(dev):
         HF.stochastic_round_e4m3fn(torch.zeros(8, dtype=torch.float16, device=dev))
     with pytest.raises(RuntimeError):
         HF.stochastic_round_e4m3fn(torch.zeros(8))
+
+
+@pytest.mark.parametrize("scale", [0.37, 3.0, -0.0078125, 1.0, 5e-3, 700.0])
+def test_every_bf16_value(dev, scale):
+    """All 65536 bf16 inputs: quotients on and beside the bf16 ties, zeros and NaN alone in a wave of other values."""
+    from comfyui_amd import functional as HF
+    x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(BF16)[torch.randperm(65536, generator=torch.Generator().manual_seed(2))]
+    s = torch.tensor(scale)
+    want = O.stochastic_round_e4m3fn(x, s, 5).view(torch.uint8)
+    got = HF.stochastic_round_e4m3fn(x.to(dev), s.to(dev), 5).cpu().view(torch.uint8)
+    assert torch.equal(got, want), (got != want).nonzero()[:8].flatten().tolist()
