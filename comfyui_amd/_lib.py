@@ -141,6 +141,9 @@ SIGNATURES = {
     "hdmoe_layer_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "hdmoe_moe_ffn": (c_int, [ctypes.POINTER(LayerArgs), c_void_p]),
     "hdmoe_ffn_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
+    "hdmoe_ffn_branch_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
+    "hdmoe_ffn_branch": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, ctypes.c_float, c_int, c_int, c_int,
+                                 ctypes.POINTER(FfnWeights), c_void_p, c_void_p, c_size_t, c_void_p]),
     "hdmoe_ffn_swiglu": (c_int, [c_int, c_void_p, c_int, c_int, c_int, ctypes.POINTER(FfnWeights), c_void_p, c_void_p,
                                  c_size_t, c_void_p]),
     "hdmoe_layer_layout_get": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, ctypes.POINTER(LayerLayout)]),

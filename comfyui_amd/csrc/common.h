@@ -76,6 +76,13 @@ struct HdmoeAltOperand {
   int shift;     // row = gather[r] >> shift
 };
 
+// What follows the down projection of a dense feed-forward branch: out = bf16(bf16(gate[row / rows_per_batch] * y) + residual)
+struct HdmoeGatedResidual {
+  const uint16_t* gate;      // bf16 [batches, N]
+  const uint16_t* residual;  // bf16 [rows, N]
+  int rows_per_batch;
+};
+
 constexpr int HDMOE_NUM_CU = 256;   // MI355X
 constexpr int HDMOE_NUM_XCD = 8;
 

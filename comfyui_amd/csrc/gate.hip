@@ -777,10 +777,21 @@ int dispatch_gate(const void* x_bf16, const void* gate_w_bf16, int T, int D, int
 // as the gate kernel; mean and variance are two passes over the registers with the same fixed fp32 order
 // (per-lane ascending elements, then the xor butterfly), so the CPU checker can restate it bit for bit.
 // The root is __builtin_sqrtf, which hipcc rounds correctly; __fsqrt_rn is the approximate native root here.
-template <int NCHUNK>  // NCHUNK * 512 == D: row held in registers; 0: any D % 8 == 0, row re-read from cache
+// CAST: the rows are cast to e4m3fn for the Linears behind (scale_in, and scale_in_also of the second Linear that reads the cast, as in
+// quant_rows_kernel: NaN rows where the two factors differ) and never written as bf16. 768 rows of 2560 in two launches 11.3 us, in one 6.3.
+template <int NCHUNK, bool CAST = false>  // NCHUNK * 512 == D: row held in registers; 0: any D % 8 == 0, row re-read from cache
 __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void ln_modulate_kernel(
     const uint4* __restrict__ x, const uint4* __restrict__ scale, const uint4* __restrict__ shift, int T, int D,
-    int tokens_per_batch, float eps, uint4* __restrict__ out) {
+    int tokens_per_batch, float eps, void* __restrict__ out_rows, const float* scale_in, const float* scale_in_also) {
+  float inv = 1.0f;
+  if constexpr (CAST) {
+    inv = hdmoe_q_uniform(hdmoe_q_inv_scale(scale_in));
+    if (scale_in_also != scale_in && hdmoe_q_uniform(hdmoe_q_inv_scale(scale_in_also)) != inv) inv = __builtin_nanf("");
+  }
+  auto put = [&](size_t unit, const uint4& v) {
+    if constexpr (CAST) static_cast<uint2*>(out_rows)[unit] = hdmoe_q_8(v, inv);
+    else static_cast<uint4*>(out_rows)[unit] = v;
+  };
   const int lane = threadIdx.x & 63;
   const int wave = blockIdx.x * WAVES_PER_BLOCK + (threadIdx.x >> 6);
   const int nwaves = gridDim.x * WAVES_PER_BLOCK;
@@ -797,8 +808,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void ln_modulate_kernel(
       ln_stats<NCHUNK>(v, fD, eps, mean, rstd);
 #pragma unroll
       for (int c = 0; c < NCHUNK; ++c)
-        out[(size_t)t * row16 + c * 64 + lane] =
-            modulate8(v[c], scale[brow + c * 64 + lane], shift[brow + c * 64 + lane], mean, rstd);
+        put((size_t)t * row16 + c * 64 + lane, modulate8(v[c], scale[brow + c * 64 + lane], shift[brow + c * 64 + lane], mean, rstd));
     } else {
       float s = 0.0f;
       for (int u = lane; u < row16; u += 64) {
@@ -817,7 +827,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void ln_modulate_kernel(
       }
       const float rstd = __fdiv_rn(1.0f, __builtin_sqrtf(__fdiv_rn(wave_sum(s2), fD) + eps));
       for (int u = lane; u < row16; u += 64)
-        out[(size_t)t * row16 + u] = modulate8(xr[u], scale[brow + u], shift[brow + u], mean, rstd);
+        put((size_t)t * row16 + u, modulate8(xr[u], scale[brow + u], shift[brow + u], mean, rstd));
     }
   }
 }
@@ -916,25 +926,35 @@ int hdmoe_launch_gate_quant(const void* x_bf16, const void* gate_w_bf16, int T, 
   return dispatch_gate(x_bf16, gate_w_bf16, T, D, E, topk_idx, topk_weight_bf16, &q, block_hist, s, what);
 }
 
+// Rows in bf16 (out_bf16), or cast for the fp8 Linears with scale_in (out_fp8).
+int hdmoe_launch_ln_modulate(const void* x_bf16, const void* scale_bf16, const void* shift_bf16, int T, int D, int tokens_per_batch,
+                             float eps, void* out_bf16, void* out_fp8, const float* scale_in, const float* scale_in_also, hipStream_t s,
+                             const char* what) {
+  if (T < 0 || D <= 0 || D % 8 != 0 || tokens_per_batch <= 0 || !(eps >= 0.0f))
+    return hdmoe_fail(HDMOE_E_SHAPE, "%s: T=%d D=%d tokens_per_batch=%d eps=%g", what, T, D, tokens_per_batch, (double)eps);
+  if (T == 0) return HDMOE_OK;
+  int blocks = (T + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
+  if (blocks > HDMOE_NUM_CU * 16) blocks = HDMOE_NUM_CU * 16;
+  const dim3 grid(blocks), block(WAVES_PER_BLOCK * 64);
+  const uint4* xp = static_cast<const uint4*>(x_bf16);
+  const uint4* sc = static_cast<const uint4*>(scale_bf16);
+  const uint4* sh = static_cast<const uint4*>(shift_bf16);
+  if (out_fp8 != nullptr) {
+    if (D == 2560) hipLaunchKernelGGL((ln_modulate_kernel<5, true>), grid, block, 0, s, xp, sc, sh, T, D, tokens_per_batch, eps, out_fp8, scale_in, scale_in_also);
+    else hipLaunchKernelGGL((ln_modulate_kernel<0, true>), grid, block, 0, s, xp, sc, sh, T, D, tokens_per_batch, eps, out_fp8, scale_in, scale_in_also);
+  } else {
+    if (D == 2560) hipLaunchKernelGGL(ln_modulate_kernel<5>, grid, block, 0, s, xp, sc, sh, T, D, tokens_per_batch, eps, out_bf16, nullptr, nullptr);
+    else hipLaunchKernelGGL(ln_modulate_kernel<0>, grid, block, 0, s, xp, sc, sh, T, D, tokens_per_batch, eps, out_bf16, nullptr, nullptr);
+  }
+  return hdmoe_check_launch(what);
+}
+
 extern "C" int hdmoe_ln_modulate_bf16(const void* x_bf16, const void* scale_bf16, const void* shift_bf16, int T, int D,
                                       int tokens_per_batch, float eps, void* out_bf16, hdmoe_stream_t stream) {
   HDMOE_REQUIRE_PTR(x_bf16);
   HDMOE_REQUIRE_PTR(scale_bf16);
   HDMOE_REQUIRE_PTR(shift_bf16);
   HDMOE_REQUIRE_PTR(out_bf16);
-  if (T < 0 || D <= 0 || D % 8 != 0 || tokens_per_batch <= 0 || !(eps >= 0.0f))
-    return hdmoe_fail(HDMOE_E_SHAPE, "hdmoe_ln_modulate_bf16: T=%d D=%d tokens_per_batch=%d eps=%g", T, D,
-                      tokens_per_batch, (double)eps);
-  if (T == 0) return HDMOE_OK;
-  int blocks = (T + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-  if (blocks > HDMOE_NUM_CU * 16) blocks = HDMOE_NUM_CU * 16;
-  const dim3 grid(blocks), block(WAVES_PER_BLOCK * 64);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const uint4* xp = static_cast<const uint4*>(x_bf16);
-  const uint4* sc = static_cast<const uint4*>(scale_bf16);
-  const uint4* sh = static_cast<const uint4*>(shift_bf16);
-  uint4* op = static_cast<uint4*>(out_bf16);
-  if (D == 2560) hipLaunchKernelGGL(ln_modulate_kernel<5>, grid, block, 0, s, xp, sc, sh, T, D, tokens_per_batch, eps, op);
-  else hipLaunchKernelGGL(ln_modulate_kernel<0>, grid, block, 0, s, xp, sc, sh, T, D, tokens_per_batch, eps, op);
-  return hdmoe_check_launch("hdmoe_ln_modulate_bf16");
+  return hdmoe_launch_ln_modulate(x_bf16, scale_bf16, shift_bf16, T, D, tokens_per_batch, eps, out_bf16, nullptr, nullptr, nullptr,
+                                  static_cast<hipStream_t>(stream), "hdmoe_ln_modulate_bf16");
 }

@@ -11,7 +11,10 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
                           const int32_t* gather_dyn = nullptr, int gather_rows = 0, float* partial = nullptr,
                           int nparts = 1, int gather_shift = 0, bool reduce = true,
                           const HdmoeSplitPlan* plan = nullptr, const HdmoeAltOperand* alt = nullptr,
-                          float* tail = nullptr);
+                          float* tail = nullptr, const HdmoeGatedResidual* end = nullptr);
+int hdmoe_launch_ln_modulate(const void* x_bf16, const void* scale_bf16, const void* shift_bf16, int T, int D, int tokens_per_batch,
+                             float eps, void* out_bf16, void* out_fp8, const float* scale_in, const float* scale_in_also, hipStream_t s,
+                             const char* what);
 size_t hdmoe_tail_bytes(int weight_dtype, int rows_dyn, int E, int rows_static, int D, int H, int Hs, bool down_uncut);
 int hdmoe_launch_combine_partials(const float* partial, long long part_stride, const HdmoeSplitPlan& plan,
                                   int rows_dyn, int n_dyn,
@@ -330,6 +333,67 @@ extern "C" size_t hdmoe_ffn_workspace_bytes(int rows, int D, int H, int weight_d
   return a + hdmoe_align_up((size_t)rows * H * eb, 256) + pbytes;
 }
 
+extern "C" size_t hdmoe_ffn_branch_workspace_bytes(int rows, int D, int H, int weight_dtype) {
+  // beside the feed-forward's: the normalised rows (16-bit activations) or the down projection's rows (not cut along K)
+  const size_t ffn = hdmoe_ffn_workspace_bytes(rows, D, H, weight_dtype);
+  return ffn == 0 ? 0 : ffn + hdmoe_align_up((size_t)rows * D * 2, 256);
+}
+
+namespace {
+// mod: LayerNorm and modulation in front, gate and residual (x itself) behind; NULL = the feed-forward alone. rows_bf16: room for
+// [rows, D] bf16 in that case.
+struct BranchMod { const void *scale, *shift, *gate; int rows_per_batch; float eps; };
+int run_ffn(const char* what, int weight_dtype, const void* x_bf16, int rows, int D, int H, const hdmoe_ffn_weights* w, void* out_bf16,
+            void* workspace, size_t workspace_bytes, const BranchMod* mod, uint8_t* rows_bf16, hipStream_t s) {
+  if (int rc = hdmoe_check_gemm_shape(what, weight_dtype, rows, D, H, 128)) return rc;
+  if (int rc = hdmoe_check_gemm_shape(what, weight_dtype, rows, H, D, 256)) return rc;
+  const bool fp8 = weight_dtype == HDMOE_W_E4M3FN;
+  const size_t h_off = fp8 ? hdmoe_align_up((size_t)rows * D, 256) : 0;
+  const size_t room_off = h_off + hdmoe_align_up((size_t)rows * H * (fp8 ? 1 : 2), 256);
+  const size_t need = room_off + ffn_down_bytes(rows, D, H, weight_dtype);   // the parts of tail tiles may do without
+  if (workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 255))
+    return hdmoe_fail(HDMOE_E_WORKSPACE, "%s: workspace %zu bytes, need %zu (256-byte aligned)", what, workspace_bytes, need);
+  if (rows == 0) return HDMOE_OK;
+  if (fp8)
+    if (int rc = hdmoe_check_scale_in13(what, *w, 0)) return rc;
+  uint8_t* ws = static_cast<uint8_t*>(workspace);
+  const uint8_t* a = static_cast<const uint8_t*>(x_bf16);
+  uint8_t* h = ws;
+  if (fp8) {
+    if (D % 8 != 0) return hdmoe_fail(HDMOE_E_SHAPE, "%s: D=%d must be a multiple of 8", what, D);
+    // one cast for w1 and w3, made with w1's factor and checked against w3's on the device
+    if (int rc = mod != nullptr ? hdmoe_launch_ln_modulate(x_bf16, mod->scale, mod->shift, rows, D, mod->rows_per_batch, mod->eps, nullptr, ws,
+                                                           w->scale_in1, w->scale_in3, s, what)
+                                : hdmoe_launch_quant_rows(x_bf16, rows, D, w->scale_in1, w->scale_in3, ws, s, what))
+      return rc;
+    a = ws;
+    h = ws + h_off;
+  } else if (mod != nullptr) {
+    if (int rc = hdmoe_launch_ln_modulate(x_bf16, mod->scale, mod->shift, rows, D, mod->rows_per_batch, mod->eps, rows_bf16, nullptr, nullptr,
+                                          nullptr, s, what))
+      return rc;
+    a = rows_bf16;
+  }
+  float* const room = reinterpret_cast<float*>(ws + room_off);
+  float* const tail = fp8 || workspace_bytes < hdmoe_ffn_workspace_bytes(rows, D, H, weight_dtype) ? nullptr : room;
+  if (int rc = hdmoe_launch_ffn_gemm(true, weight_dtype, nullptr, nullptr, 0, 0, nullptr, nullptr, a, rows, w, h, 0, 0, D, H,
+                                     s, what, nullptr, 0, nullptr, 1, 0, true, nullptr, nullptr, tail))
+    return rc;
+  const int parts = hdmoe_down_parts(0, 0, rows, D, 0, H, weight_dtype);
+  float* partial = parts > 1 ? room : nullptr;
+  HdmoeGatedResidual end = {nullptr, nullptr, 1};
+  if (mod != nullptr) end = {static_cast<const uint16_t*>(mod->gate), static_cast<const uint16_t*>(x_bf16), mod->rows_per_batch};
+  const bool end_here = mod != nullptr && parts > 1;   // the kernel that adds the parts up does the rest
+  uint8_t* const y = mod != nullptr && !end_here ? rows_bf16 : static_cast<uint8_t*>(out_bf16);   // (the normalised rows are used up)
+  if (int rc = hdmoe_launch_ffn_gemm(false, weight_dtype, nullptr, nullptr, 0, 0, nullptr, nullptr, h, rows, w, y, 0, 0, H, D, s, what,
+                                     nullptr, 0, partial, parts, 0, true, nullptr, nullptr, parts > 1 ? nullptr : tail,
+                                     end_here ? &end : nullptr))
+    return rc;
+  return mod == nullptr || end_here ? HDMOE_OK
+                                    : hdmoe_gated_residual_bf16(y, mod->gate, x_bf16, mod->rows_per_batch, rows, D, out_bf16, s);
+}
+}  // namespace
+
 extern "C" int hdmoe_ffn_swiglu(int weight_dtype, const void* x_bf16, int rows, int D, int H,
                                 const hdmoe_ffn_weights* w, void* out_bf16, void* workspace, size_t workspace_bytes,
                                 hdmoe_stream_t stream) {
@@ -337,38 +401,29 @@ extern "C" int hdmoe_ffn_swiglu(int weight_dtype, const void* x_bf16, int rows, 
   HDMOE_REQUIRE_PTR(w);
   HDMOE_REQUIRE_PTR(out_bf16);
   HDMOE_REQUIRE_PTR(workspace);
-  if (int rc = hdmoe_check_gemm_shape("hdmoe_ffn_swiglu (gate/up)", weight_dtype, rows, D, H, 128)) return rc;
-  if (int rc = hdmoe_check_gemm_shape("hdmoe_ffn_swiglu (down)", weight_dtype, rows, H, D, 256)) return rc;
-  const bool fp8 = weight_dtype == HDMOE_W_E4M3FN;
-  const size_t h_off = fp8 ? hdmoe_align_up((size_t)rows * D, 256) : 0;
-  const size_t room_off = h_off + hdmoe_align_up((size_t)rows * H * (fp8 ? 1 : 2), 256);
-  const size_t need = room_off + ffn_down_bytes(rows, D, H, weight_dtype);   // the parts of tail tiles may do without
-  if (workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 255))
-    return hdmoe_fail(HDMOE_E_WORKSPACE, "hdmoe_ffn_swiglu: workspace %zu bytes, need %zu (256-byte aligned)",
-                      workspace_bytes, need);
-  if (rows == 0) return HDMOE_OK;
-  if (fp8)
-    if (int rc = hdmoe_check_scale_in13("hdmoe_ffn_swiglu", *w, 0)) return rc;
-  hipStream_t s = static_cast<hipStream_t>(stream);
+  return run_ffn("hdmoe_ffn_swiglu", weight_dtype, x_bf16, rows, D, H, w, out_bf16, workspace, workspace_bytes, nullptr, nullptr,
+                 static_cast<hipStream_t>(stream));
+}
+
+extern "C" int hdmoe_ffn_branch(int weight_dtype, const void* x_bf16, const void* scale_bf16, const void* shift_bf16,
+                                const void* gate_bf16, int tokens_per_batch, float ln_eps, int rows, int D, int H,
+                                const hdmoe_ffn_weights* w, void* out_bf16, void* workspace, size_t workspace_bytes,
+                                hdmoe_stream_t stream) {
+  HDMOE_REQUIRE_PTR(x_bf16);
+  HDMOE_REQUIRE_PTR(scale_bf16);
+  HDMOE_REQUIRE_PTR(shift_bf16);
+  HDMOE_REQUIRE_PTR(gate_bf16);
+  HDMOE_REQUIRE_PTR(w);
+  HDMOE_REQUIRE_PTR(out_bf16);
+  HDMOE_REQUIRE_PTR(workspace);
+  if (rows < 0 || tokens_per_batch <= 0 || rows % tokens_per_batch != 0 || !(ln_eps >= 0.0f))
+    return hdmoe_fail(HDMOE_E_SHAPE, "hdmoe_ffn_branch: rows=%d tokens_per_batch=%d ln_eps=%g", rows, tokens_per_batch, (double)ln_eps);
+  // the bf16 rows come first, so that what the feed-forward sees is its own workspace, whole or without the parts of tail tiles
+  const size_t own = hdmoe_align_up((size_t)rows * (D > 0 ? D : 0) * 2, 256);
+  if (workspace_bytes < own || (reinterpret_cast<uintptr_t>(workspace) & 255))
+    return hdmoe_fail(HDMOE_E_WORKSPACE, "hdmoe_ffn_branch: workspace %zu bytes, need more than %zu (256-byte aligned)", workspace_bytes, own);
+  const BranchMod mod = {scale_bf16, shift_bf16, gate_bf16, tokens_per_batch, ln_eps};
   uint8_t* ws = static_cast<uint8_t*>(workspace);
-  const uint8_t* a = static_cast<const uint8_t*>(x_bf16);
-  uint8_t* h = ws;
-  if (fp8) {
-    if (D % 8 != 0) return hdmoe_fail(HDMOE_E_SHAPE, "hdmoe_ffn_swiglu: D=%d must be a multiple of 8", D);
-    // one cast for w1 and w3, made with w1's factor and checked against w3's on the device
-    if (int rc = hdmoe_launch_quant_rows(x_bf16, rows, D, w->scale_in1, w->scale_in3, ws, s, "hdmoe_ffn_swiglu (quantise)"))
-      return rc;
-    a = ws;
-    h = ws + h_off;
-  }
-  float* const room = reinterpret_cast<float*>(ws + room_off);
-  float* const tail = fp8 || workspace_bytes < hdmoe_ffn_workspace_bytes(rows, D, H, weight_dtype) ? nullptr : room;
-  if (int rc = hdmoe_launch_ffn_gemm(true, weight_dtype, nullptr, nullptr, 0, 0, nullptr, nullptr, a, rows, w, h, 0, 0, D, H,
-                                     s, "hdmoe_ffn_swiglu (gate/up)", nullptr, 0, nullptr, 1, 0, true, nullptr, nullptr, tail))
-    return rc;
-  const int parts = hdmoe_down_parts(0, 0, rows, D, 0, H, weight_dtype);
-  float* partial = parts > 1 ? room : nullptr;
-  return hdmoe_launch_ffn_gemm(false, weight_dtype, nullptr, nullptr, 0, 0, nullptr, nullptr, h, rows, w,
-                               static_cast<uint8_t*>(out_bf16), 0, 0, H, D, s, "hdmoe_ffn_swiglu (down)", nullptr, 0,
-                               partial, parts, 0, true, nullptr, nullptr, parts > 1 ? nullptr : tail);
+  return run_ffn("hdmoe_ffn_branch", weight_dtype, x_bf16, rows, D, H, w, out_bf16, ws + own, workspace_bytes - own, &mod, ws,
+                 static_cast<hipStream_t>(stream));
 }

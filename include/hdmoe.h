@@ -431,6 +431,16 @@ int hdmoe_ffn_swiglu(int weight_dtype, const void* x_bf16, int rows, int D, int 
                      const hdmoe_ffn_weights* w, void* out_bf16, void* workspace,
                      size_t workspace_bytes, hdmoe_stream_t stream);
 
+/* The same with the branch of a block around it (model.py:518-523): out = x + gate * FFN(LayerNorm(x, ln_eps) * (1 + scale) + shift),
+ * scale / shift / gate [rows / tokens_per_batch, D] bf16, D a multiple of 8; the bytes of hdmoe_ln_modulate_bf16, hdmoe_ffn_swiglu and
+ * hdmoe_gated_residual_bf16 one after the other. fp8: the normalised rows are cast where they are made; a down projection that is
+ * cut along K is added up, scaled, gated and added to x in one kernel. out may not overlap x. */
+size_t hdmoe_ffn_branch_workspace_bytes(int rows, int D, int H, int weight_dtype);
+int hdmoe_ffn_branch(int weight_dtype, const void* x_bf16, const void* scale_bf16, const void* shift_bf16,
+                     const void* gate_bf16, int tokens_per_batch, float ln_eps, int rows, int D, int H,
+                     const hdmoe_ffn_weights* w, void* out_bf16, void* workspace, size_t workspace_bytes,
+                     hdmoe_stream_t stream);
+
 /* Where the pieces of the workspace live, for tests that inspect intermediates. */
 typedef struct hdmoe_layer_layout {
   size_t topk_idx, topk_weight, counts, offsets, perm, inv_perm, dispatch_ws;
