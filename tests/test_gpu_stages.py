@@ -99,6 +99,14 @@ def test_quant_fp8_scaled(dev, scale):
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("rows,D", [(1, 8), (3, 1368), (1, 4096), (1, 4104), (511, 8), (513, 8), (5000, 2560)])   # a block takes 512 units of 8
+def test_quant_fp8_sizes(dev, rows, D):
+    x = torch.randn((rows, D), generator=torch.Generator().manual_seed(rows)).to(BF16)
+    s = torch.tensor(0.13, dtype=torch.float32)
+    got = _hf().quant_fp8(x.to(dev), s.to(dev)).cpu().view(torch.uint8)
+    assert torch.equal(got, (x * (1.0 / s).to(BF16)).to(FP8).view(torch.uint8))
+
+
 def test_quant_fp8_clamp_rule(dev):
     x = torch.tensor([[1000.0, -1000.0, 448.0, 460.0, -470.0, 0.3, 1e-4, -0.0]], dtype=torch.float32).repeat(1, 64).to(BF16)
     want = torch.clamp(x, min=-448, max=448).to(FP8).view(torch.uint8)
