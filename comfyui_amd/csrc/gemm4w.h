@@ -1,4 +1,5 @@
-// Grouped GEMM with one wave per SIMD: the tile text of gen_gemm4w.py (256 x 256 tile, 4 waves, 512 registers each).
+// Grouped GEMM with one wave per SIMD: the tile text of gen_gemm4w.py (tile of 256 weight rows by 256 tokens, or 128 to 224 in steps of
+// 32 where fewer fill the rounds better; 4 waves, 512 registers each).
 //
 // Included by gemm.hip inside its unnamed namespace (uses GemmArgs, GemmGroup, swz, make_rsrc, lds_ptr_t). Same
 // contraction, rounding points and LDS tile format as grouped_gemm_kernel; with bf16 activations weights may also be e4m3fn
@@ -28,7 +29,9 @@ constexpr int G4_STAGE = 32768;
 constexpr int G4_W_TILE = 65536;
 constexpr int G4_TABLE = 131072;                  // LDS: [tok 0 | tok 1 | w 0 | w 1 | work item tables of the 4 waves]
 constexpr int G4_TABLE_ITEMS = 64;                // items a wave's lanes look up at a time
-constexpr int G4_SMEM = G4_TABLE + 4 * G4_TABLE_ITEMS * 16;
+constexpr int G4_HEIGHTS = G4_TABLE + 4 * G4_TABLE_ITEMS * 16;   // 16 bytes per group
+constexpr int G4_SMEM = G4_HEIGHTS + MAX_GROUPS * 16;
+constexpr int G4_MIN_BLOCKS = 4;                  // least height of a tile of 16-bit activations, in token blocks of 32 rows
 constexpr int G4_SCRATCH = 4 * 28 * 1024;         // GELU: bytes of scratch per block (28 pieces of 16 bytes per lane)
 constexpr int G4_GELU_PAIRS = 16;                 // pairs of K steps a deferred activation needs to hide behind
 
@@ -128,6 +131,57 @@ __device__ __forceinline__ G4Tail g4_tail_of(const GemmArgs& args, const G4Segme
   return g4_plan_tail(total, blocks, args.g[0].kbytes / (2 * BK), TY == G4_W8 ? 3 : 2, padding);
 }
 
+// Tiles of fewer rows, where the tiles left over are not cut. A segment of U blocks of 32 rows takes ceil(U / cap) m-tiles for a
+// cap of 4 to 8 blocks, all as high as its blocks need (the last one may be lower). The groups follow each other from the highest
+// tiles to the lowest and go round by round over the grid, so that a round takes what its first tile does.
+// Costs as in g4_plan_tail, a pair of K steps of 8 blocks being 100 (a step costs a little beside its MFMAs: 13 us less for a round of
+// 5 blocks of K = 2048, where 17 would be in proportion), and 150 for a tile's start and end. Lower tiles have to pay by a
+// twelfth: the model takes a round with idle CUs for as long as a full one, but it has the higher clock. Whole tiles -> this: Linears in bf16,
+// 700 x 2560 x 10240 48.8 -> 38.8 us (240 tiles of 4 blocks for 120), 1700 x 2560 x 2560 48.1 -> 38.1, 3300 x 2560 x 2560 49.2 -> 43.0; with
+// e4m3fn weights 50.0 -> 37.4, 49.0 -> 36.8, 50.1 -> 42.3; Hunyuan3D block of 1250 tokens 367 -> 330, 1500 358 -> 348 (375 rows per expert:
+// 3 rounds of 8 or of 6 to 7 blocks). Not for SWIGLU, whose two halves of the weights every further m-tile reads again: 1300 tokens
+// in bf16 361 -> 367 us, 1024 tokens 294 -> 298. More than 24 rounds: one is not worth the search.
+struct G4Heights { int mt, height; };
+__device__ __forceinline__ G4Heights g4_heights(int rows, int cap) {
+  const int units = (rows + 31) >> 5, mt = (units + cap - 1) / cap;
+  return {mt, max((units + mt - 1) / max(mt, 1), G4_MIN_BLOCKS)};
+}
+
+// What the caps come to, one per lane 0 .. 4 (4 blocks to 8): the cheapest one if it is worth leaving whole tiles for, else 0.
+template <G4Type TY, int FEAT>
+__device__ __forceinline__ int g4_cap(const GemmArgs& args, const G4Segments& seg, const G4Tail& tail, int blocks, int lane) {
+  constexpr int PAIR[5] = {58, 70, 80, 90, 100}, TILE = 150;
+  const int whole = tail.rounds + (tail.tiles > 0 ? 1 : 0);
+  if (TY == G4_F8 || tail.parts > 1 || whole == 0 || whole > 24) return 0;
+  const int cap = G4_MIN_BLOCKS + min(lane, 4);
+  int n[5] = {0, 0, 0, 0, 0};                  // tiles of each height
+  for (int g = 0; g < args.G; ++g) {
+    int rb, re;
+    seg.get(args.g[g], rb, re);
+    if (re <= rb) continue;
+    const G4Heights t = g4_heights(re - rb, cap);
+    const int tiles = t.mt * (args.g[g].n_out / FEAT);
+#pragma unroll
+    for (int h = 0; h < 5; ++h) n[h] += t.height == h + G4_MIN_BLOCKS ? tiles : 0;
+  }
+  const int pairs = args.g[0].kbytes / (2 * BK);
+  int cost = 0, at = 0;
+#pragma unroll
+  for (int h = 4; h >= 0; --h) {
+    const int to = at + n[h];
+    cost += ((to + blocks - 1) / blocks - (at + blocks - 1) / blocks) * (pairs * PAIR[h] + TILE);
+    at = to;
+  }
+  const int old = whole * (100 * pairs + TILE);
+  int best = 0, limit = old - old / 12;
+#pragma unroll
+  for (int c = 4; c >= 0; --c) {
+    const int v = __builtin_amdgcn_readlane(cost, c);
+    if (v < limit) { limit = v; best = c + G4_MIN_BLOCKS; }
+  }
+  return best;
+}
+
 template <G4Type TY, int EPI>
 __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm4w_kernel(const GemmArgs args) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass drops the stub of a kernel whose register operands it cannot parse
@@ -173,9 +227,44 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   const int xcd = blockIdx.x % HDMOE_NUM_XCD, slot = blockIdx.x / HDMOE_NUM_XCD;
   const int nslots = gridDim.x / HDMOE_NUM_XCD;
   const G4Tail tail = g4_tail_of<TY, FEAT>(args, segs, gridDim.x);
+  const int cap = EPI == G4_PARTIAL || SWIGLU || args.spread != 0 ? 0 : sgpr(g4_cap<TY, FEAT>(args, segs, tail, gridDim.x, lane));
+  // cap > 0: lane g looks up where group g comes in the order of heights: [first tile, tiles, height, m-tiles]
+  v4i* const heights = reinterpret_cast<v4i*>(smem + G4_HEIGHTS);
+  if (cap > 0) {
+    v4i e = {0, 0, 0, 0};
+    for (int g = 0; g < args.G; ++g) {
+      int rb, re;
+      seg(args.g[g], rb, re);
+      if (re > rb && lane == g) {
+        const G4Heights t = g4_heights(re - rb, cap);
+        e = v4i{0, t.mt * (args.g[g].n_out / FEAT), t.height, t.mt};
+      }
+    }
+    for (int k = 0; k < args.G; ++k) {
+      const int h = __builtin_amdgcn_readlane(e.z, k), tiles = __builtin_amdgcn_readlane(e.y, k);
+      if (h > e.z || (h == e.z && k < lane)) e.x += tiles;
+    }
+    if (lane < args.G) heights[lane] = e;   // every wave the same
+  }
   v4i* const table = reinterpret_cast<v4i*>(smem + G4_TABLE) + wave * G4_TABLE_ITEMS;
   auto fill_table = [&](int base) {
     const int i = base + lane;
+    if (cap > 0) {
+      const int L = i * (int)gridDim.x + xcd * nslots + slot;
+      v4i e = {-1, 0, 0, 0};
+      for (int g = 0; g < args.G; ++g) {
+        const v4i t = heights[g];
+        const int first = sgpr(t.x), tiles = sgpr(t.y), rows = sgpr(t.z) * 32, mtiles = sgpr(t.w);
+        int rb, re, m, n;
+        seg(args.g[g], rb, re);
+        if (L < first || L >= first + tiles) continue;
+        g4_raster(L - first, mtiles, args.g[g].n_out / FEAT, m, n);
+        const int row0 = rb + m * rows;
+        e = v4i{g | min(re - row0, rows) << 16, row0, n, args.g[g].kbytes / BK << 16};
+      }
+      table[lane] = e;
+      return;
+    }
     const bool eighths = EPI == G4_PARTIAL || args.spread != 0;   // every group cut in eighths
     int rem = slot + i * nslots, tail_part = 0, tail_slot = 0;
     bool some = true;
@@ -263,7 +352,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   for (int i = 0; i < 32; ++i) ctx[i] = own(0);
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
-    ctx[G4_TOK_ADDR + ks] = (int)lds0 + (wt * 128 + fr_row) * 128 + ((ks * 4 + fr_grp) ^ fr_swz) * 16;
+    ctx[G4_TOK_ADDR + ks] = (int)lds0 + (wt * 16 + fr_row) * 128 + ((ks * 4 + fr_grp) ^ fr_swz) * 16;
     ctx[G4_W_ADDR + ks] = (int)lds0 + G4_W_TILE + (wq * 128 + fr_row) * 128 +
                           (W8 ? ((ks * 2 + (fr_grp >> 1)) ^ fr_swz) * 16 + (fr_grp & 1) * 8 : ((ks * 4 + fr_grp) ^ fr_swz) * 16);
   }
@@ -357,12 +446,12 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   };
   // GELU: the tile whose activation is still to be applied (none: an empty buffer)
   v4i dro = rsrc4(nullptr, 0);
-  int dldo = own(0);
+  int dldo = own(0), dnt = own(0);
   bool deferred = false;
   const v4i scr = EPI == G4_GELU ? rsrc4(args.scratch + (size_t)blockIdx.x * G4_SCRATCH, G4_SCRATCH) : rsrc4(nullptr, 0);
   const int gk = sgpr(__float_as_int((F16 ? 1.0f : 2.0f) * 0.84932180f)), gp = sgpr(__float_as_int(0.3f / 0.84932180f));  // gen_gemm4w.py: k (2 k), 0.3 / k
 #define G4_DRAIN(TEXT)                                                                                               \
-  asm volatile(TEXT : "+{v[128:159]}"(fa0), "+{v[160:191]}"(fb0), "+{v[96:127]}"(ctx) : [dro] "s"(dro), [dldo] "s"(dldo), [dd] "s"(dd), [scr] "s"(scr), [gk] "s"(gk), [gp] "s"(gp) : G4_CLOBBER_V)
+  asm volatile(TEXT : "+{v[128:159]}"(fa0), "+{v[160:191]}"(fb0), "+{v[96:127]}"(ctx) : [dro] "s"(dro), [dldo] "s"(dldo), [dnt] "s"(dnt), [dd] "s"(dd), [scr] "s"(scr), [gk] "s"(gk), [gp] "s"(gp) : G4_CLOBBER_V)
   // Output offsets of the pieces: the second pair of K steps stores the first two of token block 1, so DEF_ST starts a step in
   // front of them, at the last two of block 0, and advances by dd = dldo - 128 and 128 in turn.
   auto drain = [&] {
@@ -380,7 +469,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     if (nx2.some()) nx3 = item(i + 3);
     int n = sgpr(cur.nkt() >> 1), so = sgpr((cur.kt0() + 2) * BK), wso = sgpr(w_start(cur) + 2 * BK);
     const int nso = sgpr(nxt.kt0() * BK), nwso = sgpr(w_start(nxt));
-    const int ldo = gg.n_out * OUT_BYTES, ldo16 = sgpr(16 * ldo);
+    const int ldo = gg.n_out * OUT_BYTES, ldo32 = sgpr(32 * ldo);
     int slot_u;   // in a scalar register for certain (the compiler drops the builtin where it finds the value uniform)
     // (the wait state between a vector register's write and its readfirstlane, which the compiler does not add inside a statement)
     asm volatile("s_nop 1\n\tv_readfirstlane_b32 %0, %1" : "=s"(slot_u) : "v"(cur.slot()));
@@ -391,9 +480,9 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     const v4i ro = part ? rsrc4(args.tail + (size_t)(slot_u - 1) * (G4_BM * 256), G4_BM * 256 * 4)
                         : rsrc4(out, (uint32_t)cur.rows_here() * (uint32_t)ldo);
     ctx[G4_OUT_VOFF] = part ? wave * 65536 + lane * 16
-                            : (wt * 128 + fr_row) * ldo + (cur.n0() + wq * (FEAT / 2) + fr_grp * 8) * OUT_BYTES;
-    const int part_s = slot_u;
-    const int ntt = sgpr((cur.rows_here() - wt * 128 + 15) >> 4);
+                            : (wt * 16 + fr_row) * ldo + (cur.n0() + wq * (FEAT / 2) + fr_grp * 8) * OUT_BYTES;
+    const int part_s = part ? sgpr((cur.rows_here() + 31) >> 5) : 0;   // token blocks of a part
+    const int nt = sgpr(cap > 0 ? max((cur.rows_here() + 31) >> 5, G4_MIN_BLOCKS) : G4_BM / 32);   // token blocks
     // row indices of nx2 and this tile's biases are loaded inside the statement
     const int32_t* const list = nx2.some() ? args.g[nx2.g()].gather : nullptr;
     const v4i gr = rsrc4(list != nullptr ? list + nx2.row0() : nullptr, list != nullptr ? (uint32_t)nx2.rows_here() * 4u : 0u);
@@ -406,36 +495,35 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
       dro = rsrc4(nullptr, 0);
       deferred = false;
     }
-    int dn = sgpr(14), dd = sgpr(dldo - 128);
+    int dn = sgpr(2 * dnt - 2), dd = sgpr(dldo - 128);
 #define G4_TILE(TEXT)                                                                                                \
     asm volatile(TEXT : "+{v[128:159]}"(fa0), "+{v[160:191]}"(fb0), "+{v[96:127]}"(ctx), "={v[72:79]}"(gi),          \
                         [n] "+s"(n), [so] "+s"(so), [wso] "+s"(wso), [ldswb] "+s"(ldswb), [dn] "+s"(dn), [dd] "+s"(dd) \
                  : "{v[80:95]}"(voff_nxt), [r0] "s"(src.a.lo), [r1] "s"(src.a.hi), [r2] "s"(src.b0.lo),              \
                    [r3] "s"(src.b0.hi), [r4] "s"(src.b1.lo), [r5] "s"(src.b1.hi), [nr0] "s"(nsrc.a.lo), [nr1] "s"(nsrc.a.hi),             \
                    [nr2] "s"(nsrc.b0.lo), [nr3] "s"(nsrc.b0.hi), [nr4] "s"(nsrc.b1.lo), [nr5] "s"(nsrc.b1.hi),       \
-                   [nso] "s"(nso), [nwso] "s"(nwso), [ldsw] "s"(ldsw), [ro] "s"(ro), [ldo16] "s"(ldo16),             \
+                   [nso] "s"(nso), [nwso] "s"(nwso), [ldsw] "s"(ldsw), [ro] "s"(ro), [ldo32] "s"(ldo32),             \
                    [gr] "s"(gr), [br] "s"(br), [sc] "s"(sc), [su] "s"(su), [dro] "s"(dro), [dldo] "s"(dldo),         \
-                   [scr] "s"(scr), [gk] "s"(gk), [gp] "s"(gp), [ntt] "s"(ntt), [part] "s"(part_s)                    \
+                   [scr] "s"(scr), [gk] "s"(gk), [gp] "s"(gp), [nt] "s"(nt), [part] "s"(part_s)                    \
                  : G4_CLOBBER)
-#define G4_TILE_OR_PART(LOOP, EPILOGUE)                                                                              \
-    G4_TILE(LOOP "s_cmp_lg_u32 %[part], 0\ns_cbranch_scc1 41f\n" EPILOGUE "s_branch 42f\n41:\n" HDMOE_G4_EPI_PART "42:\n")
-    if constexpr (F8 && EPI == G4_BIAS) { G4_TILE_OR_PART(HDMOE_G4_LOOP_F8_BIAS, HDMOE_G4_EPI_F8_BIAS); }
-    else if constexpr (F8 && EPI == G4_PARTIAL) G4_TILE(HDMOE_G4_LOOP_F8 HDMOE_G4_EPI_PARTIAL);
-    else if constexpr (F8) { G4_TILE_OR_PART(HDMOE_G4_LOOP_F8, HDMOE_G4_EPI_F8); }
-    else if constexpr (EPI == G4_GELU && F16) { G4_TILE_OR_PART(HDMOE_G4_LOOP_F16_GELU, HDMOE_G4_EPI_F16_GELU); }
-    else if constexpr (EPI == G4_GELU) { G4_TILE_OR_PART(HDMOE_G4_LOOP_BF16_GELU, HDMOE_G4_EPI_BF16_GELU); }
-    else if constexpr (EPI == G4_BIAS && F16) { G4_TILE_OR_PART(HDMOE_G4_LOOP_F16_BIAS, HDMOE_G4_EPI_F16_BIAS); }
-    else if constexpr (EPI == G4_BIAS && W8) { G4_TILE_OR_PART(HDMOE_G4_LOOP_BF16_W8_BIAS, HDMOE_G4_EPI_BF16_W8_BIAS); }
-    else if constexpr (EPI == G4_BIAS) { G4_TILE_OR_PART(HDMOE_G4_LOOP_BF16_BIAS, HDMOE_G4_EPI_BF16_BIAS); }
-    else if constexpr (EPI == G4_SWIGLU && W8) { G4_TILE_OR_PART(HDMOE_G4_LOOP_BF16_W8, HDMOE_G4_EPI_SWIGLU_W8); }
-    else if constexpr (EPI == G4_SWIGLU) { G4_TILE_OR_PART(HDMOE_G4_LOOP_BF16, HDMOE_G4_EPI_SWIGLU); }
-    else if constexpr (EPI == G4_PARTIAL && W8) G4_TILE(HDMOE_G4_LOOP_BF16_W8 HDMOE_G4_EPI_PARTIAL);
-    else if constexpr (EPI == G4_PARTIAL) G4_TILE(HDMOE_G4_LOOP_BF16 HDMOE_G4_EPI_PARTIAL);
-    else if constexpr (W8) { G4_TILE_OR_PART(HDMOE_G4_LOOP_BF16_W8, HDMOE_G4_EPI_BF16_W8); }
-    else { G4_TILE_OR_PART(HDMOE_G4_LOOP_BF16, HDMOE_G4_EPI_BF16); }
+    if constexpr (F8 && EPI == G4_BIAS) G4_TILE(HDMOE_G4_TILE_F8_BIAS);
+    else if constexpr (F8 && EPI == G4_PARTIAL) G4_TILE(HDMOE_G4_TILE_F8_PARTIAL);
+    else if constexpr (F8) G4_TILE(HDMOE_G4_TILE_F8);
+    else if constexpr (EPI == G4_GELU && F16) G4_TILE(HDMOE_G4_TILE_F16_GELU);
+    else if constexpr (EPI == G4_GELU) G4_TILE(HDMOE_G4_TILE_BF16_GELU);
+    else if constexpr (EPI == G4_BIAS && F16) G4_TILE(HDMOE_G4_TILE_F16_BIAS);
+    else if constexpr (EPI == G4_BIAS && W8) G4_TILE(HDMOE_G4_TILE_BF16_W8_BIAS);
+    else if constexpr (EPI == G4_BIAS) G4_TILE(HDMOE_G4_TILE_BF16_BIAS);
+    else if constexpr (EPI == G4_SWIGLU && W8) G4_TILE(HDMOE_G4_TILE_BF16_W8_SWIGLU);
+    else if constexpr (EPI == G4_SWIGLU) G4_TILE(HDMOE_G4_TILE_BF16_SWIGLU);
+    else if constexpr (EPI == G4_PARTIAL && W8) G4_TILE(HDMOE_G4_TILE_BF16_W8_PARTIAL);
+    else if constexpr (EPI == G4_PARTIAL) G4_TILE(HDMOE_G4_TILE_BF16_PARTIAL);
+    else if constexpr (W8) G4_TILE(HDMOE_G4_TILE_BF16_W8);
+    else G4_TILE(HDMOE_G4_TILE_BF16);
     if (EPI == G4_GELU && !part) {
       dro = ro;
-      dldo = ldo16;
+      dldo = ldo32;
+      dnt = nt;
       deferred = true;
       ctx[G4_DEF_LD] = ctx[G4_SCR_VOFF];
       ctx[G4_DEF_ST] = ctx[G4_OUT_VOFF] + 128;
@@ -480,7 +568,7 @@ __global__ __launch_bounds__(256) void gemm4w_tail_kernel(const GemmArgs args, i
     const int unit = item % PER_TILE * 4 + (threadIdx.x >> 6);
     const int q = unit & (SWIGLU ? 1 : 3), tt = (unit >> (SWIGLU ? 1 : 2)) & 7, w = unit >> (SWIGLU ? 4 : 5);
     const int wq = w & 1, wt = w >> 1;
-    const int row = wt * 128 + tt * 16 + (lane & 15);
+    const int row = tt * 32 + wt * 16 + (lane & 15);
     if (row >= rows_here) continue;
     const float* src = args.tail + (size_t)t * tail.parts * (G4_BM * 256) + w * 16384 + (tt * 8 + q * 2) * 256 + lane * 4;
     constexpr int QUADS = SWIGLU ? 4 : 2;

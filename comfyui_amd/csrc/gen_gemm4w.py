@@ -4,7 +4,9 @@
     python comfyui_amd/csrc/gen_gemm4w.py [output file]
 
 One wave per SIMD (4 waves, 512 registers each) on a 256-token x 256-weight-row tile, wave tile 128 x 128 of
-v_mfma_f32_16x16x32. A K step is 64 elements (128 bytes per token row) through two LDS stages. The fragments of both
+v_mfma_f32_16x16x32. Token block tt of wave pair wt is rows 32 tt + 16 wt of the tile, so a tile with fewer tokens is one with fewer
+token blocks: with 16-bit activations there is a text for each of HEIGHTS, and a tile runs the one of its size. A pair of K steps
+that ends a tile of fewer blocks still fetches all of the next tile, whatever its height. A K step is 64 elements (128 bytes per token row) through two LDS stages. The fragments of both
 32-element slices of a step have registers of their own, so a stage has been read for good after about a third of its
 step, and the global->LDS loads of the step after the next go into it from there on: they have about 1.4 steps to
 arrive. Two barriers per step: everyone has read this stage; everyone's loads of the next one have landed. One statement
@@ -60,14 +62,21 @@ FRAG = {("a", 0): 128, ("b", 0): 160, ("a", 1): 192, ("b", 1): 224}
 MFMA = {"BF16": "v_mfma_f32_16x16x32_bf16", "F16": "v_mfma_f32_16x16x32_f16"}
 PK = {"BF16": "v_cvt_pk_bf16_f32", "F16": "v_cvt_pk_f16_f32", "F8": "v_cvt_pk_bf16_f32"}   # F8: the outputs are bf16
 
-# positions (MFMA index within a slice) of the events of a step
-READ1_AT = 0        # slice 0: first read of slice 1
-FREE_AT = 24        # slice 0: the stage has been read; barrier
-LOAD_AT = 25        # first load of the step after the next, and MFMAs between two loads
-LOAD_EVERY = 6
-LAND_AT = 32        # slice 1: the next stage has landed; barrier, then the reads of slice 0 of the next step
-CVT1_AT = 26        # w8, slice 0: first conversion of slice 1
-PIECE_ST_AT, PIECE_LD_AT = 57, 60                 # GELU, slice 0
+HEIGHTS = (8, 7, 6, 5, 4)                         # token blocks of a wave: 32 tokens of the tile each
+
+
+class At:
+    """Positions (MFMA index within a slice of `m`) of the events of a step of `nt` token blocks. last: of the pair that ends a
+    tile, which fetches 8 token blocks whatever nt is."""
+    def __init__(self, nt, last=False):
+        self.nt, self.m = nt, 8 * nt
+        self.loads = 8 if last else nt          # token loads of a step
+        self.free = 16 + nt                     # slice 0: the stage has been read (8 + nt reads, one per MFMA); barrier
+        self.load = self.free + 1               # first load of the step after the next, and MFMAs between two loads
+        self.every = (2 * self.m - self.load - 8) // (self.loads + 7)
+        self.land = self.m - 16 - 2 * nt        # slice 1: the next stage has landed; barrier, then the reads of slice 0 of the next step
+        self.cvt1 = self.free + 2               # w8, slice 0: first conversion of slice 1
+        self.st, self.ld = self.m - 7, self.m - 4   # GELU, slice 0: piece stored, piece read back
 
 
 # the same for the fp8 step (64 MFMAs)
@@ -81,9 +90,9 @@ def quad(b):
     return f"v[{b}:{b + 3}]"
 
 
-def reads(stage, ks, w8, odd):
-    """The 16 fragment reads of a slice, in the order the MFMAs want them."""
-    order = [("b", 0)] + [("a", t) for t in range(8)] + [("b", f) for f in range(1, 8)]
+def reads(stage, ks, w8, odd, nt=8):
+    """The 8 + nt fragment reads of a slice, in the order the MFMAs want them."""
+    order = [("b", 0)] + [("a", t) for t in range(nt)] + [("b", f) for f in range(1, 8)]
     if w8:
         order.sort(key=lambda o: o[0] == "a")     # the weights have to be converted
     out = []
@@ -94,13 +103,13 @@ def reads(stage, ks, w8, odd):
             out.append(f"ds_read_b64 v[{RAW + 2 * i}:{RAW + 2 * i + 1}], v{W_ADDR[ks]} offset:{2048 * i}")
         else:
             out.append(f"ds_read_b128 {quad(FRAG[(kind, ks)] + 4 * i)}, v{(TOK_ADDR if kind == 'a' else W_ADDR)[ks]} "
-                       f"offset:{stage * STAGE + 2048 * i}")
+                       f"offset:{stage * STAGE + (4096 if kind == 'a' else 2048) * i}")
     return out
 
 
-def token_loads(stage):
+def token_loads(stage, nt=8):
     return [(f"s_add_u32 m0, %[ldsw], {stage * STAGE + j * 4096}",
-             f"buffer_load_dwordx4 v{TOK_VOFF[j]}, s[64:67], %[so] offen lds") for j in range(8)]
+             f"buffer_load_dwordx4 v{TOK_VOFF[j]}, s[64:67], %[so] offen lds") for j in range(nt)]
 
 
 def weight_loads(stage, w8):
@@ -112,10 +121,10 @@ def weight_loads(stage, w8):
     return out
 
 
-def mfma_order():
+def mfma_order(nt):
     o = []
     for ft in range(8):
-        o += [(ft, tt) for tt in (range(8) if ft % 2 == 0 else range(7, -1, -1))]
+        o += [(ft, tt) for tt in (range(nt) if ft % 2 == 0 else range(nt - 1, -1, -1))]
     return o
 
 
@@ -204,55 +213,60 @@ def conversions(ks):
     return o
 
 
-def requests(w8, gelu, stage, first=False):
+def requests(w8, gelu, stage, at, first=False):
     """The vector-memory requests of a step out of `stage` (first: of a tile's first pair) as (position, kind), position =
     MFMA index over both slices."""
-    n = 8 if w8 and stage == 0 else 16
-    out = [(LOAD_AT + j * LOAD_EVERY, "t" if j < 8 else "w") for j in range(n)]
+    n = at.loads + (0 if w8 and stage == 0 else 8)
+    out = [(at.load + j * at.every, "t" if j < at.loads else "w") for j in range(n)]
     if gelu:
-        out += ([] if first else [(PIECE_ST_AT, "s")]) + [(PIECE_LD_AT, "l")]
+        out += ([] if first else [(at.st, "s")]) + [(at.ld, "l")]
     return sorted(out)
 
 
-def young(w8, gelu, stage, first):
+def young(w8, gelu, stage, at, first):
     """How many vector-memory requests may still be out when the next step's operands must have landed (requests return in
     order): those issued after the last one that is needed. Needed: the tokens (16-bit weights too) requested a step ago and
-    the piece read back then; one-byte weights were requested two steps ago or earlier."""
-    before = [k for p, k in requests(w8, gelu, stage, first) if p < 64 + LAND_AT]
-    last = [k for _, k in requests(w8, gelu, stage ^ 1)]
+    the piece read back then; one-byte weights were requested two steps ago or earlier. The step before may be one of another
+    height: what it issues behind the last needed request is the same for all."""
+    before = [k for p, k in requests(w8, gelu, stage, at, first) if p < at.m + at.land]
     need = {"t", "l"} | (set() if w8 else {"w"})
-    after = 0
-    for k in reversed(last):
-        if k in need:
-            break
-        after += 1
-    return after + len(before)
+    behind = set()
+    for other in [At(nt, end) for nt in HEIGHTS for end in (False, True)]:
+        after = 0
+        for _, k in reversed(requests(w8, gelu, stage ^ 1, other)):
+            if k in need:
+                break
+            after += 1
+        behind.add(after)
+    assert len(behind) == 1
+    return behind.pop() + len(before)
 
 
-def step(dt, w8, gelu, stage, first):
+def step(dt, w8, gelu, stage, first, at):
     """One K step out of `stage`. Entry: the reads of its slice 0 are in flight (lgkmcnt; w8: converted). first: of
     a tile's first pair, whose step 0 starts the accumulators from zero and which has no finished piece to store."""
     L = []
-    order = mfma_order()
+    order = mfma_order(at.nt)
     # w8: the even step's slice 1 and the odd step's slice 0 read the same weight stage; the next even step's slice 0 reads
     # the other one (W_ADDR is flipped between the pairs)
-    rd1 = reads(stage, 1, w8, stage)
-    rd0 = reads(stage ^ 1, 0, w8, stage ^ 1)
-    ld = token_loads(stage) + ([] if w8 and stage == 0 else weight_loads(stage, w8))
-    cvt0_at = LAND_AT + 14
-    cvt1, cvt0 = Feeder(conversions(1) if w8 else [], 64 - CVT1_AT), Feeder(conversions(0) if w8 else [], 64 - cvt0_at)
+    rd1 = reads(stage, 1, w8, stage, at.nt)
+    rd0 = reads(stage ^ 1, 0, w8, stage ^ 1, at.loads if stage == 1 else at.nt)
+    ld = token_loads(stage, at.loads) + ([] if w8 and stage == 0 else weight_loads(stage, w8))
+    # w8: first conversion of the next step's slice 0, when a few of the reads behind the 8 of the weights have been issued
+    cvt0_at = at.land + 14 - (8 - at.nt) // 2
+    cvt1, cvt0 = Feeder(conversions(1) if w8 else [], at.m - at.cvt1), Feeder(conversions(0) if w8 else [], at.m - cvt0_at)
     # the piece read back a step ago, in two parts around the end of the step (words n_b.. of the one before that first)
     n_b = 2
-    half_b = Feeder(gelu_words(dt, PIECE[stage ^ 1], RES, n_b) if gelu else [], 64 - LAND_AT)
-    half_a = Feeder(gelu_words(dt, PIECE[stage] + n_b, RES + n_b, 4 - n_b) if gelu else [], PIECE_ST_AT)
-    assert FREE_AT <= LOAD_AT and LOAD_AT + 15 * LOAD_EVERY < 128
-    for q in range(128):
-        ks, i = divmod(q, 64)
+    half_b = Feeder(gelu_words(dt, PIECE[stage ^ 1], RES, n_b) if gelu else [], at.m - at.land)
+    half_a = Feeder(gelu_words(dt, PIECE[stage] + n_b, RES + n_b, 4 - n_b) if gelu else [], at.st)
+    assert len(rd1) <= at.free <= at.load and at.load + (at.loads + 7) * at.every < 2 * at.m and at.land + len(rd0) <= at.m
+    for q in range(2 * at.m):
+        ks, i = divmod(q, at.m)
         ft, tt = order[i]
         if q == 0:
             L.append("s_waitcnt lgkmcnt(0)")
-        k = q - LOAD_AT
-        now = ld[k // LOAD_EVERY] if k >= 0 and k % LOAD_EVERY == 0 and k // LOAD_EVERY < len(ld) else None
+        k = q - at.load
+        now = ld[k // at.every] if k >= 0 and k % at.every == 0 and k // at.every < len(ld) else None
         if now:
             L.append(now[0])
         acc = f"a[{(8 * ft + tt) * 4}:{(8 * ft + tt) * 4 + 3}]"
@@ -261,34 +275,36 @@ def step(dt, w8, gelu, stage, first):
         if now:
             L.append(now[1])
         if ks == 0:
-            if 0 <= i - READ1_AT < 16:
-                L.append(rd1[i - READ1_AT])
-            if i == FREE_AT - 1:
+            if i < len(rd1):
+                L.append(rd1[i])
+            if i == at.free - 1:
                 L += ["s_waitcnt lgkmcnt(0)", "s_barrier"]
-            if w8 and i >= CVT1_AT:
+            if w8 and i >= at.cvt1:
                 L += cvt1.take()
-            if gelu and i < PIECE_ST_AT:
+            if gelu and i < at.st:
                 L += half_a.take()
-            if gelu and i == PIECE_ST_AT:
+            if gelu and i == at.st:
                 assert half_a.done()
-            if gelu and i == PIECE_ST_AT and not first:
+            if gelu and i == at.st and not first:
                 L.append(f"buffer_store_dwordx4 {quad(RES)}, v{DEF_ST}, %[dro], 0 offen offset:{64 * stage}")
-            if gelu and i == PIECE_LD_AT:
+            if gelu and i == at.ld:
                 L.append(f"buffer_load_dwordx4 {quad(PIECE[stage])}, v{DEF_LD}, %[scr], 0 offen offset:{1024 * stage}")
         else:
-            if i == LAND_AT - 1:
-                L += [f"s_waitcnt vmcnt({young(w8, gelu, stage, first)})", "s_barrier"]
+            if i == at.land - 1:
+                L += [f"s_waitcnt vmcnt({young(w8, gelu, stage, at, first)})", "s_barrier"]
                 if w8 and stage == 1:   # the next pair's weights
                     L += [f"v_xor_b32 v{r}, {hex(STAGE)}, v{r}" for r in W_ADDR]
                 if w8:                  # the other 64 bytes of the rows
                     L += [f"v_xor_b32 v{r}, 64, v{r}" for r in W_ADDR]
-            if 0 <= i - LAND_AT < 16:
-                L.append(rd0[i - LAND_AT])
+            if 0 <= i - at.land < len(rd0):
+                L.append(rd0[i - at.land])
             if w8 and i == cvt0_at - 1:   # the weight bytes are there, the tokens may still be under way
-                L.append(f"s_waitcnt lgkmcnt({min(8, cvt0_at - LAND_AT - 8)})")
+                issued = min(len(rd0), cvt0_at - at.land)
+                assert issued > 8
+                L.append(f"s_waitcnt lgkmcnt({issued - 8})")
             if w8 and i >= cvt0_at:
                 L += cvt0.take()
-            if gelu and i >= LAND_AT:
+            if gelu and i >= at.land:
                 L += half_b.take()
     assert half_b.done() and cvt0.done() and cvt1.done()
     L.append("s_add_u32 %[so], %[so], 128")
@@ -305,7 +321,7 @@ def reads8(stage, frags):
     for kind, i in frags:
         for h in range(2):
             out.append(f"ds_read_b128 {quad(frag8(kind, i) + 4 * h)}, v{(TOK_ADDR if kind == 'a' else W_ADDR)[h]} "
-                       f"offset:{stage * STAGE + 2048 * i}")
+                       f"offset:{stage * STAGE + (4096 if kind == 'a' else 2048) * i}")
     return out
 
 
@@ -366,7 +382,7 @@ def step8(stage, first):
     return L
 
 
-def pair(dt, w8, gelu, first):
+def pair(dt, w8, gelu, first, at):
     if dt == "F8":
         return step8(0, first) + step8(1, first)
     L = []
@@ -374,26 +390,29 @@ def pair(dt, w8, gelu, first):
         # pieces 2p, 2p + 1: the pair of K steps p (0..13) reads them back, pair p + 1 stores them (64 bytes per token each)
         L += [f"v_add_u32 v{DEF_LD}, 0x800, v{DEF_LD}", f"v_add_u32 v{DEF_ST}, %[dd], v{DEF_ST}", "s_sub_u32 %[dd], %[dldo], %[dd]",
               "s_sub_u32 %[dn], %[dn], 1", "s_cmp_ge_i32 %[dn], 0", "s_cbranch_scc1 21f", f"v_mov_b32 v{DEF_ST}, 0x80000000", "21:"]
-    L += step(dt, w8, gelu, 0, first) + step(dt, w8, gelu, 1, first)
+    L += step(dt, w8, gelu, 0, first, at) + step(dt, w8, gelu, 1, first, at)
     if w8:   # the weight stage of the pair after the next is this pair's
         L += [f"s_xor_b32 %[ldswb], %[ldswb], {hex(STAGE)}", "s_add_u32 %[wso], %[wso], 128"]
     return L
 
 
-def k_loop(dt, w8, gelu, bias):
+def k_loop(dt, w8, gelu, bias, nt=8):
     """All K steps of a tile in pairs, %[n] of them (at least 2, w8: 3). Before the last pair the loads turn to the first
     two steps of the next tile; the row indices of the tile after it and this tile's biases are requested there too. w8:
     the weights of a pair are requested two pairs ahead, so they turn a pair earlier. The wait states at the end cover
     the distance between the last MFMA and the first read of an accumulator."""
+    at, end = At(nt), At(nt, True)
     L = [f"s_mov_b64 s[{64 + 2 * i}:{65 + 2 * i}], %[r{i}]" for i in range(6)]
-    L += pair(dt, w8, gelu, True) + ["s_sub_u32 %[n], %[n], 1", "11:"]
+    L += pair(dt, w8, gelu, True, at) + ["s_sub_u32 %[n], %[n], 1", "11:"]
     wswitch = [f"s_mov_b64 s[{64 + 2 * i}:{65 + 2 * i}], %[nr{i}]" for i in range(2, 6)]
     wswitch += [f"v_mov_b32 v{W_VOFF[j]}, v{NEXT + 8 + j}" for j in range(8)]
     if w8:
         L += ["s_cmp_eq_u32 %[n], 2", "s_cbranch_scc1 15f", "16:"]
     L += ["s_cmp_eq_u32 %[n], 1", "s_cbranch_scc1 13f", "14:"]
-    L += pair(dt, w8, gelu, False)
+    L += pair(dt, w8, gelu, False, at)
     L += ["s_sub_u32 %[n], %[n], 1", "s_cmp_lg_u32 %[n], 0", "s_cbranch_scc1 11b", "s_branch 12f"]
+    if w8:
+        L += ["15:"] + wswitch + ["s_mov_b32 %[wso], %[nwso]", "s_branch 16b"]
     L += ["13:", "s_mov_b64 s[64:65], %[nr0]", "s_mov_b64 s[66:67], %[nr1]", "s_mov_b32 %[so], %[nso]"]
     L += [f"v_mov_b32 v{TOK_VOFF[j]}, v{NEXT + j}" for j in range(8)]
     if not w8:
@@ -402,20 +421,18 @@ def k_loop(dt, w8, gelu, bias):
     if bias:
         L += [f"buffer_load_dwordx2 v[{BIAS + 2 * ft}:{BIAS + 2 * ft + 1}], v{BIAS_VOFF}, %[br], 0 offen "
               f"offset:{(ft >> 1) * 64 + (ft & 1) * 8}" for ft in range(8)]
-    L += ["s_branch 14b"]
-    if w8:
-        L += ["15:"] + wswitch + ["s_mov_b32 %[wso], %[nwso]", "s_branch 16b"]
+    L += ["s_branch 14b"] if nt == 8 else pair(dt, w8, gelu, False, end)
     L += ["12:", "s_nop 15"]
     if gelu:   # the last piece read back is there: its registers are the compiler's between two tiles
-        L.append(f"s_waitcnt vmcnt({sum(p > PIECE_LD_AT for p, _ in requests(False, True, 1))})")
+        L.append(f"s_waitcnt vmcnt({sum(p > end.ld for p, _ in requests(False, True, 1, end))})")
     return L
 
 
 def out_row(tt):
-    return [f"v_add_u32 v{ROW_VOFF}, %[ldo16], v{ROW_VOFF}"] if tt else [f"v_mov_b32 v{ROW_VOFF}, v{OUT_VOFF}"]
+    return [f"v_add_u32 v{ROW_VOFF}, %[ldo32], v{ROW_VOFF}"] if tt else [f"v_mov_b32 v{ROW_VOFF}, v{OUT_VOFF}"]
 
 
-def epilogue(dt, w8, bias, gelu):
+def epilogue(dt, w8, bias, gelu, nt=8):
     """acc (* scale) (+ bias) rounded to 16 bits, 8 consecutive features (16 bytes) per lane and store, 64 bytes per token.
     v[192:223]: the lane's 32 biases, v[224:255] work. gelu: the first token block is activated at once, the others are
     left to the next tile's K loop."""
@@ -427,7 +444,7 @@ def epilogue(dt, w8, bias, gelu):
     n = 0
     if gelu:
         L.append(f"v_mov_b32 v{DEF_LD}, v{SCR_VOFF}")
-    for tt in range(8):
+    for tt in range(nt):
         L += out_row(tt) if not (gelu and tt) else []
         for g in range(4):
             w = 224 + 16 * (n % 2)          # 8 values, then 4 packed words
@@ -455,7 +472,7 @@ def epilogue(dt, w8, bias, gelu):
                 L.append(f"buffer_store_dwordx4 {quad(o)}, v{DEF_LD}, %[scr], 0 offen offset:{1024 * g}")
             else:
                 L.append(f"buffer_store_dwordx4 {quad(o)}, v{ROW_VOFF}, %[ro], 0 offen offset:{64 * g}")
-        if gelu and tt in range(1, 7):
+        if gelu and tt in range(1, nt - 1):
             L.append(f"v_add_u32 v{DEF_LD}, 0x1000, v{DEF_LD}")
     return L
 
@@ -509,10 +526,10 @@ def partial_epilogue():
 
 def part_epilogue():
     """The raw fp32 sums of a part of a tile, straight from the accumulators in the wave's own order (1 KiB per MFMA tile,
-    token blocks outermost); token blocks without rows (%[ntt] of the wave's 8 have some) are left out."""
+    token blocks outermost); token blocks without rows (%[part] of the 8 have some) are left out."""
     L = [f"v_mov_b32 v{ROW_VOFF}, v{OUT_VOFF}"]
     for tt in range(8):
-        L += [f"s_cmp_le_i32 %[ntt], {tt}", "s_cbranch_scc1 31f"]
+        L += [f"s_cmp_le_i32 %[part], {tt}", "s_cbranch_scc1 31f"]
         for ft in range(8):
             b = (8 * ft + tt) * 4
             L.append(f"buffer_store_dwordx4 a[{b}:{b + 3}], v{ROW_VOFF}, %[ro], 0 offen offset:{1024 * (ft % 4)}")
@@ -522,18 +539,39 @@ def part_epilogue():
 
 
 def gelu_drain(dt):
-    """The pieces of the deferred tile with nothing to hide behind: token blocks 1-7, 4 pieces each. v[192:255] free."""
+    """The pieces of the deferred tile with nothing to hide behind: token blocks 1 .. %[dnt] - 1, 4 pieces each, those of a block read
+    back while the one before is worked on. v[192:255] free."""
     L = [f"v_mov_b32 v{ROW_VOFF}, v{DEF_ST}", f"v_mov_b32 v{DEF_LD}, v{SCR_VOFF}"]
+
+    def back(tt):
+        return [f"buffer_load_dwordx4 {quad(192 + 16 * (tt % 2) + 4 * g)}, v{DEF_LD}, %[scr], 0 offen offset:{1024 * g}" for g in range(4)]
+    L += back(1)
     for tt in range(1, 8):
-        L.append(f"v_add_u32 v{ROW_VOFF}, {'%[dldo]' if tt > 1 else '%[dd]'}, v{ROW_VOFF}")
+        if tt < 7:
+            L += [f"s_cmp_le_i32 %[dnt], {tt + 1}", "s_cbranch_scc1 51f", f"v_add_u32 v{DEF_LD}, 0x1000, v{DEF_LD}"] + back(tt + 1)
+            L += [f"s_waitcnt vmcnt({4 if tt == 1 else 8})", "s_branch 52f", "51:"]   # younger: the stores of the block before, these loads
+        L += ["s_waitcnt vmcnt(0)", "52:", f"v_add_u32 v{ROW_VOFF}, {'%[dldo]' if tt > 1 else '%[dd]'}, v{ROW_VOFF}"]
         for g in range(4):
-            L.append(f"buffer_load_dwordx4 {quad(192 + 4 * g)}, v{DEF_LD}, %[scr], 0 offen offset:{1024 * g}")
-        L.append("s_waitcnt vmcnt(0)")
-        for g in range(4):
-            L += [i for i, _ in gelu_words(dt, 192 + 4 * g, 208 + 4 * g, 4)]
-            L.append(f"buffer_store_dwordx4 {quad(208 + 4 * g)}, v{ROW_VOFF}, %[dro], 0 offen offset:{64 * g}")
-        L.append(f"v_add_u32 v{DEF_LD}, 0x1000, v{DEF_LD}")
-    return L + ["s_nop 7"]
+            L += [i for i, _ in gelu_words(dt, 192 + 16 * (tt % 2) + 4 * g, 224 + 4 * g, 4)]
+            L.append(f"buffer_store_dwordx4 {quad(224 + 4 * g)}, v{ROW_VOFF}, %[dro], 0 offen offset:{64 * g}")
+        if tt < 7:
+            L += [f"s_cmp_le_i32 %[dnt], {tt + 1}", "s_cbranch_scc1 53f"]
+    return L + ["53:", "s_nop 7"]
+
+
+def tile(dt, w8, gelu, bias, epi, heights=HEIGHTS):
+    """A tile of any height: the text of its number of token blocks, %[nt]. Raw sums where it is a part of a tile, which has 8 (%[part])."""
+    texts = []
+    for nt in heights:
+        L = [f"{100 + nt}:"] + k_loop(dt, w8, gelu, bias, nt)
+        L += ["s_cmp_lg_u32 %[part], 0", "s_cbranch_scc1 41f"] if nt == 8 else []
+        L += epi(nt)
+        L += ["s_branch 199f", "41:"] + part_epilogue() if nt == 8 else []
+        texts += L + ["s_branch 199f"]
+    jumps = []
+    for nt in heights[1:]:
+        jumps += [f"s_cmp_eq_u32 %[nt], {nt}", f"s_cbranch_scc1 {100 + nt}f"]
+    return jumps + texts[:-1] + ["199:"]
 
 
 def check_trans(lines):
@@ -550,19 +588,18 @@ def generate():
     texts = []
     for dt, w8, gelu, bias in (("BF16", False, False, False), ("BF16", False, False, True), ("F16", False, False, True),
                                ("BF16", False, True, True), ("F16", False, True, True), ("BF16", True, False, False), ("BF16", True, False, True)):
-        texts.append((f"HDMOE_G4_LOOP_{dt}{'_W8' if w8 else ''}{'_GELU' if gelu else '_BIAS' if bias else ''}", k_loop(dt, w8, gelu, bias)))
-        texts.append((f"HDMOE_G4_EPI_{dt}{'_W8' if w8 else ''}{'_GELU' if gelu else '_BIAS' if bias else ''}", epilogue(dt, w8, bias, gelu)))
-    texts.append(("HDMOE_G4_EPI_SWIGLU", swiglu_epilogue(False)))
-    texts.append(("HDMOE_G4_EPI_SWIGLU_W8", swiglu_epilogue(True)))
-    texts.append(("HDMOE_G4_EPI_PARTIAL", partial_epilogue()))
-    texts.append(("HDMOE_G4_EPI_PART", part_epilogue()))
+        name = f"HDMOE_G4_TILE_{dt}{'_W8' if w8 else ''}{'_GELU' if gelu else '_BIAS' if bias else ''}"
+        texts.append((name, tile(dt, w8, gelu, bias, lambda nt: epilogue(dt, w8, bias, gelu, nt))))
+    for w8 in (False, True):
+        texts.append((f"HDMOE_G4_TILE_BF16{'_W8' if w8 else ''}_SWIGLU", tile("BF16", w8, False, False, lambda nt: swiglu_epilogue(w8), HEIGHTS[:1])))
+        texts.append((f"HDMOE_G4_TILE_BF16{'_W8' if w8 else ''}_PARTIAL", k_loop("BF16", w8, False, False) + partial_epilogue()))
     texts.append(("HDMOE_G4_FILL", reads(0, 0, False, 0)))
     texts.append(("HDMOE_G4_FILL_W8", reads(0, 0, True, 0) + ["s_waitcnt lgkmcnt(0)"] + [i for i, _ in conversions(0)]))
     for dt in ("BF16", "F16"):
         texts.append((f"HDMOE_G4_DRAIN_{dt}", DRAIN_WAIT + gelu_drain(dt)))
     for bias in (False, True):
-        texts.append((f"HDMOE_G4_LOOP_F8{'_BIAS' if bias else ''}", k_loop("F8", False, False, bias)))
-        texts.append((f"HDMOE_G4_EPI_F8{'_BIAS' if bias else ''}", epilogue("F8", False, bias, False)))
+        texts.append((f"HDMOE_G4_TILE_F8{'_BIAS' if bias else ''}", k_loop("F8", False, False, bias) + epilogue("F8", False, bias, False)))
+    texts.append(("HDMOE_G4_TILE_F8_PARTIAL", k_loop("F8", False, False, False) + partial_epilogue()))
     texts.append(("HDMOE_G4_FILL_F8", burst8(0)[0]))
     for name, lines in texts:
         check_trans(lines)
