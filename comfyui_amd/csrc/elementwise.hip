@@ -7,6 +7,8 @@
 #include "numfmt.h"
 #include "quant.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int THREADS = 256;
@@ -226,6 +228,9 @@ __global__ __launch_bounds__(THREADS) void combine_kernel(const uint4* __restric
 // splitk_reduce_kernel (gemm.hip) does for a row, bf16((sum over the parts in ascending order) * scale of the row's
 // Linear), then what combine_kernel does with the three rows of a token. Same operations in the same order as the two
 // kernels it replaces, so the same bytes; one launch and one bf16 round trip of the rows less.
+// Few tokens: bound by the chain of loads that wait for each other. So the row's segment is found in the lanes of one load of the
+// bounds, and the parts of all three rows come two at a time (one row and part after the other: 64 tokens 7.25 us, 256 7.6; this 6.2 and 7.0;
+// four at a time 6.0 and 7.3). Many tokens: by the sums read, 1024 tokens in bf16 12.9 us before and after (four at a time: 15.5, half the waves).
 struct CombinePartialArgs {
   const float* partial;
   long long part_stride;   // floats between two parts
@@ -241,7 +246,7 @@ __global__ __launch_bounds__(THREADS) void combine_partials_kernel(const Combine
                                                                    const uint32_t* __restrict__ w, int T, int row16,
                                                                    CombineExtra ex, uint4* __restrict__ out) {
   const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * WAVES + (threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * WAVES + (threadIdx.x >> 6));
   const int nwaves = gridDim.x * WAVES;
   const bool hs = pa.has_shared != 0;
   const bool hg = ex.gate != nullptr;
@@ -252,30 +257,12 @@ __global__ __launch_bounds__(THREADS) void combine_partials_kernel(const Combine
     if (pa.weight_dtype == HDMOE_W_E4M3FN_UPCAST && pa.sw[g] != nullptr) return hdmoe_dev_round_bf16(*pa.sw[g]);
     return 1.0f;
   };
-  auto group_of = [&](int r) {
-    int g = 0;
-    while (g + 1 < pa.n_dyn && r >= pa.offsets[g + 1]) ++g;
-    return g;
-  };
-  // the 8 features of row r at column c, as splitk_reduce_kernel leaves them (values of the 16-bit format)
-  auto row_vals = [&](int r, int c, float sc, int nparts, float (&v)[8]) {
-    const float* src = pa.partial + (size_t)r * n_out + c;
-    float4 s0 = *reinterpret_cast<const float4*>(src), s1 = *reinterpret_cast<const float4*>(src + 4);
-    for (int p = 1; p < nparts; ++p) {
-      const float* q = src + (size_t)p * (size_t)pa.part_stride;
-      const float4 t0 = *reinterpret_cast<const float4*>(q), t1 = *reinterpret_cast<const float4*>(q + 4);
-      s0.x += t0.x; s0.y += t0.y; s0.z += t0.z; s0.w += t0.w;
-      s1.x += t1.x; s1.y += t1.y; s1.z += t1.z; s1.w += t1.w;
-    }
-    v[0] = A::round(s0.x * sc); v[1] = A::round(s0.y * sc); v[2] = A::round(s0.z * sc); v[3] = A::round(s0.w * sc);
-    v[4] = A::round(s1.x * sc); v[5] = A::round(s1.y * sc); v[6] = A::round(s1.z * sc); v[7] = A::round(s1.w * sc);
-  };
-  const float sc_sh = hs ? scale_of(pa.n_dyn) : 1.0f;
+  // the bounds as one vector load (at most 17 entries), then lane reads
+  const int off_lane = lane <= pa.n_dyn ? pa.offsets[lane] : 0;
+  auto group_of = [&](int r) { return (int)__popcll(__ballot(lane > 0 && lane < pa.n_dyn && r >= off_lane)); };
   // which cut the down projection ran with (the same function of the segment bounds as in its kernel)
   int nparts = pa.plan.pd[0], nparts_static = pa.plan.ps[0];
   if (pa.plan.n > 1) {
-    // the bounds as one vector load (at most 17 entries), then lane reads
-    const int off_lane = lane <= pa.n_dyn ? pa.offsets[lane] : 0;
     int mt_dyn = 0;
     for (int e = 0; e < pa.n_dyn; ++e)
       mt_dyn += (__builtin_amdgcn_readlane(off_lane, e + 1) - __builtin_amdgcn_readlane(off_lane, e) + pa.plan.bm - 1) / pa.plan.bm;
@@ -286,15 +273,48 @@ __global__ __launch_bounds__(THREADS) void combine_partials_kernel(const Combine
   }
   for (int unit = wave; unit < T * chunks; unit += nwaves) {
     const int t = unit / chunks;
-    const int u = (unit - t * chunks) * 64 + lane;
-    if (u >= row16) continue;
+    const int u0 = (unit - t * chunks) * 64, u = min(u0 + lane, row16 - 1);
     const int2 r = inv_perm[t];
     const uint32_t wp = w[t];
     const float w0 = A::lo(wp), w1 = A::hi(wp);
-    float y0[8], y1[8], sh[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    row_vals(r.x, u * 8, scale_of(group_of(r.x)), nparts, y0);
-    row_vals(r.y, u * 8, scale_of(group_of(r.y)), nparts, y1);
-    if (hs) row_vals(pa.rows_dyn + t, u * 8, sc_sh, nparts_static, sh);
+    const float sc[3] = {scale_of(group_of(r.x)), scale_of(group_of(r.y)), hs ? scale_of(pa.n_dyn) : 1.0f};
+    const float* const src[3] = {pa.partial + (size_t)r.x * n_out + u * 8, pa.partial + (size_t)r.y * n_out + u * 8,
+                                 pa.partial + (size_t)(pa.rows_dyn + t) * n_out + u * 8};
+    const int parts[3] = {nparts, nparts, hs ? nparts_static : 0};
+    // the 8 features of the three rows, as splitk_reduce_kernel leaves them (values of the 16-bit format)
+    float v[3][8];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[i][k] = -0.0f;   // the first part as it is, a negative zero too
+    auto add = [&](auto n, int p) {   // parts p .. p + n - 1 of the rows that have them
+      constexpr int N = decltype(n)::value;
+      float4 in[N][3][2];
+#pragma unroll
+      for (int k = 0; k < N; ++k)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          if (p + k >= parts[i]) continue;
+          const float4* const q = reinterpret_cast<const float4*>(src[i] + (size_t)(p + k) * (size_t)pa.part_stride);
+          in[k][i][0] = q[0];
+          in[k][i][1] = q[1];
+        }
+#pragma unroll
+      for (int k = 0; k < N; ++k)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          if (p + k >= parts[i]) continue;
+          const float4 a = in[k][i][0], b = in[k][i][1];
+          v[i][0] += a.x; v[i][1] += a.y; v[i][2] += a.z; v[i][3] += a.w;
+          v[i][4] += b.x; v[i][5] += b.y; v[i][6] += b.z; v[i][7] += b.w;
+        }
+    };
+    for (int p = 0; p < max(nparts, parts[2]); p += 2) add(std::integral_constant<int, 2>{}, p);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[i][k] = i < 2 || hs ? A::round(v[i][k] * sc[i]) : 0.0f;
+    const float (&y0)[8] = v[0], (&y1)[8] = v[1], (&sh)[8] = v[2];
     uint4 g = make_uint4(0, 0, 0, 0), res = g;
     if (hg) {
       g = ex.gate[(long)(t / ex.tokens_per_batch) * row16 + u];
@@ -309,7 +329,7 @@ __global__ __launch_bounds__(THREADS) void combine_partials_kernel(const Combine
     o.y = two(2, g.y, res.y);
     o.z = two(4, g.z, res.z);
     o.w = two(6, g.w, res.w);
-    out[(long)t * row16 + u] = o;
+    if (u0 + lane < row16) out[(long)t * row16 + u] = o;
   }
 }
 
