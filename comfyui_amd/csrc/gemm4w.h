@@ -22,6 +22,7 @@
 // kernel with its assembly loop -> this one: 16384 x 13824 x 2560 511 -> 430 us (2.7 PFLOP/s), 16384 x 2560 x 6912 226 -> 213 us, 8192^3
 // 374 -> 338 us, 16384^3 3076 -> 2637 us (3.3 PFLOP/s). One K step of one tile takes 0.88 us with few rows, a launch 8 us beside its steps.
 #include "gemm4w_asm.inc"
+#include "tail_units.h"
 
 constexpr int G4_THREADS = 256;
 constexpr int G4_BM = 256;                        // tokens per block tile
@@ -479,7 +480,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
         : gg.out + (size_t)cur.row0() * ldo;
     const v4i ro = part ? rsrc4(args.tail + (size_t)(slot_u - 1) * (G4_BM * 256), G4_BM * 256 * 4)
                         : rsrc4(out, (uint32_t)cur.rows_here() * (uint32_t)ldo);
-    ctx[G4_OUT_VOFF] = part ? wave * 65536 + lane * 16
+    ctx[G4_OUT_VOFF] = part ? wave * 8192 + lane * 16
                             : (wt * 16 + fr_row) * ldo + (cur.n0() + wq * (FEAT / 2) + fr_grp * 8) * OUT_BYTES;
     const int part_s = part ? sgpr((cur.rows_here() + 31) >> 5) : 0;   // token blocks of a part
     const int nt = sgpr(cap > 0 ? max((cur.rows_here() + 31) >> 5, G4_MIN_BLOCKS) : G4_BM / 32);   // token blocks
@@ -563,14 +564,13 @@ __global__ __launch_bounds__(256) void gemm4w_tail_kernel(const GemmArgs args, i
     }
     const GemmGroup& gg = args.g[g];
     const int row0 = rb + m * G4_BM, rows_here = min(re - row0, G4_BM);
-    // the wave's order of gen_gemm4w.py: MFMA tile (tt, ft) of wave w at ((w * 64) + tt * 8 + ft) KiB; ft 2q and 2q + 1 hold
-    // the 8 features
-    const int unit = item % PER_TILE * 4 + (threadIdx.x >> 6);
-    const int q = unit & (SWIGLU ? 1 : 3), tt = (unit >> (SWIGLU ? 1 : 2)) & 7, w = unit >> (SWIGLU ? 4 : 5);
+    // the order of gen_gemm4w.py: MFMA tile (tt, ft) of wave w at (tt * 32 + w * 8 + ft) KiB; ft 2q and 2q + 1 hold the 8 features.
+    const G4TailUnit mine = g4_tail_unit(SWIGLU, item % PER_TILE, threadIdx.x >> 6, t);
+    const int q = mine.q, tt = mine.tt, w = mine.w;
     const int wq = w & 1, wt = w >> 1;
     const int row = tt * 32 + wt * 16 + (lane & 15);
     if (row >= rows_here) continue;
-    const float* src = args.tail + (size_t)t * tail.parts * (G4_BM * 256) + w * 16384 + (tt * 8 + q * 2) * 256 + lane * 4;
+    const float* src = args.tail + (size_t)t * tail.parts * (G4_BM * 256) + (tt * 32 + w * 8 + q * 2) * 256 + lane * 4;
     constexpr int QUADS = SWIGLU ? 4 : 2;
     float4 s[QUADS];
 #pragma unroll

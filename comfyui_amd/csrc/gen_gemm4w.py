@@ -525,8 +525,8 @@ def partial_epilogue():
 
 
 def part_epilogue():
-    """The raw fp32 sums of a part of a tile, straight from the accumulators in the wave's own order (1 KiB per MFMA tile,
-    token blocks outermost); token blocks without rows (%[part] of the 8 have some) are left out."""
+    """The raw fp32 sums of a part of a tile, straight from the accumulators: 1 KiB per MFMA tile, 8 KiB per wave, token blocks
+    outermost over all waves; token blocks without rows (%[part] of the 8 have some) are left out."""
     L = [f"v_mov_b32 v{ROW_VOFF}, v{OUT_VOFF}"]
     for tt in range(8):
         L += [f"s_cmp_le_i32 %[part], {tt}", "s_cbranch_scc1 31f"]
@@ -534,7 +534,7 @@ def part_epilogue():
             b = (8 * ft + tt) * 4
             L.append(f"buffer_store_dwordx4 a[{b}:{b + 3}], v{ROW_VOFF}, %[ro], 0 offen offset:{1024 * (ft % 4)}")
             if ft % 4 == 3:
-                L.append(f"v_add_u32 v{ROW_VOFF}, 0x1000, v{ROW_VOFF}")
+                L.append(f"v_add_u32 v{ROW_VOFF}, {0x1000 if ft == 3 else 0x7000:#x}, v{ROW_VOFF}")
     return L + ["31:", "s_nop 7"]
 
 

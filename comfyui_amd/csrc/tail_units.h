@@ -1,0 +1,24 @@
+// How gemm4w_tail_kernel deals out the work of adding up a tail tile's parts (gemm4w.h), also for the host.
+//
+// A unit is what one wave does: the 16 rows that wave w of the GEMM has of token block tt (32 tt + 16 (w >> 1) on) by 32 of its 128
+// features (gate/up: 32 of its 64 outputs). A block takes four units that follow each other; its XCD is its index mod 8. With few
+// rows only the first token blocks of each tile have any, so a unit's place in its tile turns with the tile: else those
+// blocks fall to a few XCDs. Token block in the low bits of the block's index -> so, Linear of 128 rows in bf16, us: by
+// 2560 x 10240 (40 tiles) 10.5 -> 7.7; by 2048 x 2048 (8 tiles) 6.0 -> 6.0, but the GEMM in front, which writes the parts, 18.8 -> 15.4 (the
+// lines that it overwrites are then held by all XCDs' caches).
+#pragma once
+
+#if defined(__HIPCC__)
+#define HDMOE_TAIL_HD __host__ __device__ __forceinline__
+#else
+#define HDMOE_TAIL_HD static inline
+#endif
+
+struct G4TailUnit { int q, w, tt; };
+
+// 128 units per tile, gate/up 64. item: the block's index within the tile.
+HDMOE_TAIL_HD G4TailUnit g4_tail_unit(bool swiglu, int item, int wave, int tile) {
+  const int unit = item * 4 + wave, bits = swiglu ? 1 : 2;
+  const int at = ((unit >> bits) + (swiglu ? 10 : 5) * tile) & 31;   // by 5 blocks (a block holds two places of gate/up)
+  return {unit & ((1 << bits) - 1), at & 3, at >> 2};
+}

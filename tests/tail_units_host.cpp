@@ -1,0 +1,6 @@
+// Host-side export of comfyui_amd/csrc/tail_units.h for the CPU tests.
+#include "../comfyui_amd/csrc/tail_units.h"
+extern "C" void t_tail_unit(int swiglu, int item, int wave, int tile, int* out) {
+  const G4TailUnit u = g4_tail_unit(swiglu != 0, item, wave, tile);
+  out[0] = u.q; out[1] = u.w; out[2] = u.tt;
+}

@@ -1,0 +1,41 @@
+"""The order in which gemm4w_tail_kernel adds up the parts of tail tiles (csrc/tail_units.h): every unit of a tile once, and the ones
+that have rows spread over the XCDs (a block's index mod 8) whatever the number of rows."""
+import ctypes
+import subprocess
+
+import pytest
+
+
+@pytest.fixture(scope="module")
+def unit(tmp_path_factory):
+    so = tmp_path_factory.mktemp("units") / "libtail_units.so"
+    subprocess.check_call(["g++", "-O2", "-shared", "-fPIC", "-o", str(so), "tests/tail_units_host.cpp"])
+    lib = ctypes.CDLL(str(so))
+
+    def call(swiglu, item, wave, tile):
+        out = (ctypes.c_int * 3)()
+        lib.t_tail_unit(int(swiglu), item, wave, tile, out)
+        return tuple(out)
+    return call
+
+
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_every_unit_once(unit, swiglu):
+    items, quarters = (16, 2) if swiglu else (32, 4)
+    want = {(q, w, tt) for q in range(quarters) for w in range(4) for tt in range(8)}
+    for tile in (0, 1, 7, 31, 250):
+        got = [unit(swiglu, i, v, tile) for i in range(items) for v in range(4)]
+        assert len(got) == len(want) and set(got) == want
+
+
+@pytest.mark.parametrize("swiglu", [False, True])
+@pytest.mark.parametrize("tiles", [8, 10, 40])
+def test_units_with_rows_are_spread_over_the_xcds(unit, swiglu, tiles):
+    items = 16 if swiglu else 32
+    units = [(t, i, v, *unit(swiglu, i, v, t)) for t in range(tiles) for i in range(items) for v in range(4)]
+    for rows in (1, 16, 17, 33, 64, 100, 128, 129, 200, 256):
+        load = [0] * 8
+        for t, i, _, _, w, tt in units:
+            load[(t * items + i) % 8] += tt * 32 + (w >> 1) * 16 < rows
+        # 16 rows of a tile are 8 units (4 for gate/up): with 8 tiles on 8 XCDs some unevenness is left
+        assert min(load) > 0 and max(load) <= 2 * sum(load) / 8, (rows, load)
