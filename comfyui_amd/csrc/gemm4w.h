@@ -482,7 +482,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
                         : rsrc4(out, (uint32_t)cur.rows_here() * (uint32_t)ldo);
     ctx[G4_OUT_VOFF] = part ? wave * 8192 + lane * 16
                             : (wt * 16 + fr_row) * ldo + (cur.n0() + wq * (FEAT / 2) + fr_grp * 8) * OUT_BYTES;
-    const int part_s = part ? sgpr((cur.rows_here() + 31) >> 5) : 0;   // token blocks of a part
+    const int part_s = part ? sgpr(g4_part_blocks(cur.rows_here(), wave)) + 1 : 0;
     const int nt = sgpr(cap > 0 ? max((cur.rows_here() + 31) >> 5, G4_MIN_BLOCKS) : G4_BM / 32);   // token blocks
     // row indices of nx2 and this tile's biases are loaded inside the statement
     const int32_t* const list = nx2.some() ? args.g[nx2.g()].gather : nullptr;

@@ -526,10 +526,10 @@ def partial_epilogue():
 
 def part_epilogue():
     """The raw fp32 sums of a part of a tile, straight from the accumulators: 1 KiB per MFMA tile, 8 KiB per wave, token blocks
-    outermost over all waves; token blocks without rows (%[part] of the 8 have some) are left out."""
+    outermost over all waves; token blocks without rows (%[part] - 1 of the wave's 8 have some) are left out."""
     L = [f"v_mov_b32 v{ROW_VOFF}, v{OUT_VOFF}"]
     for tt in range(8):
-        L += [f"s_cmp_le_i32 %[part], {tt}", "s_cbranch_scc1 31f"]
+        L += [f"s_cmp_le_i32 %[part], {tt + 1}", "s_cbranch_scc1 31f"]
         for ft in range(8):
             b = (8 * ft + tt) * 4
             L.append(f"buffer_store_dwordx4 a[{b}:{b + 3}], v{ROW_VOFF}, %[ro], 0 offen offset:{1024 * (ft % 4)}")

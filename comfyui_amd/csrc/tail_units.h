@@ -22,3 +22,7 @@ HDMOE_TAIL_HD G4TailUnit g4_tail_unit(bool swiglu, int item, int wave, int tile)
   const int at = ((unit >> bits) + (swiglu ? 10 : 5) * tile) & 31;   // by 5 blocks (a block holds two places of gate/up)
   return {unit & ((1 << bits) - 1), at & 3, at >> 2};
 }
+
+// Token blocks of which wave w of the GEMM has rows, in a tile of `rows`: those are what it leaves of a part. A Linear of up to 16 rows by
+// 2560 x 10240 in bf16, whole blocks of 32 rows -> so: 17.3 -> 16.6 us (240 parts of 16 KiB instead of 32).
+HDMOE_TAIL_HD int g4_part_blocks(int rows, int w) { return (rows - (w >> 1) * 16 + 31) >> 5; }

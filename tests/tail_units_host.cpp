@@ -4,3 +4,4 @@ extern "C" void t_tail_unit(int swiglu, int item, int wave, int tile, int* out) 
   const G4TailUnit u = g4_tail_unit(swiglu != 0, item, wave, tile);
   out[0] = u.q; out[1] = u.w; out[2] = u.tt;
 }
+extern "C" int t_part_blocks(int rows, int w) { return g4_part_blocks(rows, w); }

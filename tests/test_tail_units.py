@@ -7,14 +7,17 @@ import pytest
 
 
 @pytest.fixture(scope="module")
-def unit(tmp_path_factory):
+def units(tmp_path_factory):
     so = tmp_path_factory.mktemp("units") / "libtail_units.so"
     subprocess.check_call(["g++", "-O2", "-shared", "-fPIC", "-o", str(so), "tests/tail_units_host.cpp"])
-    lib = ctypes.CDLL(str(so))
+    return ctypes.CDLL(str(so))
 
+
+@pytest.fixture(scope="module")
+def unit(units):
     def call(swiglu, item, wave, tile):
         out = (ctypes.c_int * 3)()
-        lib.t_tail_unit(int(swiglu), item, wave, tile, out)
+        units.t_tail_unit(int(swiglu), item, wave, tile, out)
         return tuple(out)
     return call
 
@@ -39,3 +42,9 @@ def test_units_with_rows_are_spread_over_the_xcds(unit, swiglu, tiles):
             load[(t * items + i) % 8] += tt * 32 + (w >> 1) * 16 < rows
         # 16 rows of a tile are 8 units (4 for gate/up): with 8 tiles on 8 XCDs some unevenness is left
         assert min(load) > 0 and max(load) <= 2 * sum(load) / 8, (rows, load)
+
+
+def test_blocks_of_a_part_are_the_ones_with_rows(units):
+    for rows in range(1, 257):
+        for w in range(4):
+            assert units.t_part_blocks(rows, w) == sum(tt * 32 + (w >> 1) * 16 < rows for tt in range(8))
