@@ -96,6 +96,7 @@ SIGNATURES = {
     "hdmoe_get_kernel_form": (c_int, [c_int]),
     "hdmoe_gate_up_kernel_name": (ctypes.c_char_p, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     "hdmoe_tail_plan": (c_int, [c_int, c_int, c_int, c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_int)]),
+    "hdmoe_linear_tile_rows": (c_int, [c_int, c_int, c_int, c_int]),
     "hdmoe_gate_top2": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "hdmoe_gate_top2_f16": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "hdmoe_renorm_top2_bf16": (c_int, [c_void_p, c_int, c_void_p, c_void_p]),

@@ -116,6 +116,7 @@ struct GemmArgs {
   // gemm4w_kernel only
   uint8_t* scratch;       // with GELU: G4_SCRATCH bytes per block
   float* tail;            // room for the parts of tail tiles (G4_TAIL_BYTES), NULL = tiles are not cut
+  int cap;                // height of the tiles in blocks of 32 rows at most, 0 = whole tiles, -1 = by the segments' sizes
 };
 
 __device__ __forceinline__ int swz(int row) { return ((row >> 1) & 7) ^ ((row & 1) << 2); }
@@ -1155,6 +1156,7 @@ int launch_gemm4w(GemmArgs& args, int rows_mean, hipStream_t s, const char* what
                      has_static ? last.row_end - last.row_begin : 0, last.n_out, last.kbytes, FEAT, TY == G4_W8) == 0)
       args.tail = nullptr;
   }
+  args.cap = TY == G4_F8 ? 0 : g4_host_cap(args, FEAT, TY == G4_W8 ? 3 : 2, HDMOE_NUM_CU);
   // one block per CU whatever the number of tiles: a block without any ends at once
   hipLaunchKernelGGL((gemm4w_kernel<TY, EPI>), dim3(HDMOE_NUM_CU), dim3(G4_THREADS), G4_SMEM, s, args);
   if constexpr (EPI != G4_PARTIAL && TY != G4_F8) {
@@ -2118,6 +2120,26 @@ extern "C" int hdmoe_tail_plan(int weight_dtype, int tiles, int K, int padding, 
   if (rounds != nullptr) *rounds = t.rounds;
   if (left != nullptr) *left = t.tiles;
   return t.parts;
+}
+
+// Height of the tiles of a Linear on 16-bit activations that is given the working memory it asks for: 256, or fewer rows where no
+// tile is cut and lower ones fill the rounds better (g4_best_cap). For tests and reports.
+extern "C" int hdmoe_linear_tile_rows(int weight_dtype, int rows, int K, int N) {
+  const bool w8 = weight_dtype == HDMOE_W_E4M3FN_UPCAST;
+  if ((!w8 && weight_dtype != HDMOE_W_BF16 && weight_dtype != HDMOE_W_F16) || rows <= 0 || K <= 0 || N <= 0 || N % BN != 0 ||
+      K > 0x7fff * BK / 2 || K % BK != 0 || K / BK < (w8 ? 3 : 2))
+    return 0;
+  GemmArgs args;
+  memset(&args, 0, sizeof(args));
+  args.G = 1;
+  args.g[0].row_end = rows;
+  args.g[0].n_out = N;
+  args.g[0].kbytes = K * 2;
+  float room = 0.0f;
+  if (g4_tail_room(0, 0, 0, 0, rows, N, K * 2, BN, w8) > 0) args.tail = &room;
+  else if (rows <= 128 && !w8) return 0;   // the 8-wave kernel's
+  const int cap = g4_host_cap(args, BN, w8 ? 3 : 2, HDMOE_NUM_CU);
+  return 32 * (cap > 0 ? g4_heights(rows, cap).height : G4_BM / 32);
 }
 
 // Bytes a feed-forward's contractions on 16-bit activations can use for the parts of tail tiles: E experts of hidden width H on

@@ -142,26 +142,23 @@ __device__ __forceinline__ G4Tail g4_tail_of(const GemmArgs& args, const G4Segme
 // e4m3fn weights 50.0 -> 37.4, 49.0 -> 36.8, 50.1 -> 42.3; Hunyuan3D block of 1250 tokens 367 -> 330, 1500 358 -> 348 (375 rows per expert:
 // 3 rounds of 8 or of 6 to 7 blocks). Not for SWIGLU, whose two halves of the weights every further m-tile reads again: 1300 tokens
 // in bf16 361 -> 367 us, 1024 tokens 294 -> 298. More than 24 rounds: one is not worth the search.
+constexpr int G4_TILE_COST = 150, G4_CAP_ROUNDS = 24;
 struct G4Heights { int mt, height; };
-__device__ __forceinline__ G4Heights g4_heights(int rows, int cap) {
+__host__ __device__ __forceinline__ G4Heights g4_heights(int rows, int cap) {
   const int units = (rows + 31) >> 5, mt = (units + cap - 1) / cap;
   return {mt, max((units + mt - 1) / max(mt, 1), G4_MIN_BLOCKS)};
 }
 
-// What the caps come to, one per lane 0 .. 4 (4 blocks to 8): the cheapest one if it is worth leaving whole tiles for, else 0.
-template <G4Type TY, int FEAT>
-__device__ __forceinline__ int g4_cap(const GemmArgs& args, const G4Segments& seg, const G4Tail& tail, int blocks, int lane) {
-  constexpr int PAIR[5] = {58, 70, 80, 90, 100}, TILE = 150;
-  const int whole = tail.rounds + (tail.tiles > 0 ? 1 : 0);
-  if (TY == G4_F8 || tail.parts > 1 || whole == 0 || whole > 24) return 0;
-  const int cap = G4_MIN_BLOCKS + min(lane, 4);
+// What a cap comes to; rows(g): the rows of group g.
+template <class Rows>
+__host__ __device__ __forceinline__ int g4_cap_cost(const GemmArgs& args, int feat, const Rows& rows, int blocks, int cap) {
+  constexpr int PAIR[5] = {58, 70, 80, 90, 100};
   int n[5] = {0, 0, 0, 0, 0};                  // tiles of each height
   for (int g = 0; g < args.G; ++g) {
-    int rb, re;
-    seg.get(args.g[g], rb, re);
-    if (re <= rb) continue;
-    const G4Heights t = g4_heights(re - rb, cap);
-    const int tiles = t.mt * (args.g[g].n_out / FEAT);
+    const int have = rows(g);
+    if (have <= 0) continue;
+    const G4Heights t = g4_heights(have, cap);
+    const int tiles = t.mt * (args.g[g].n_out / feat);
 #pragma unroll
     for (int h = 0; h < 5; ++h) n[h] += t.height == h + G4_MIN_BLOCKS ? tiles : 0;
   }
@@ -170,17 +167,61 @@ __device__ __forceinline__ int g4_cap(const GemmArgs& args, const G4Segments& se
 #pragma unroll
   for (int h = 4; h >= 0; --h) {
     const int to = at + n[h];
-    cost += ((to + blocks - 1) / blocks - (at + blocks - 1) / blocks) * (pairs * PAIR[h] + TILE);
+    cost += ((to + blocks - 1) / blocks - (at + blocks - 1) / blocks) * (pairs * PAIR[h] + G4_TILE_COST);
     at = to;
   }
-  const int old = whole * (100 * pairs + TILE);
+  return cost;
+}
+
+// Rounds of whole tiles that lower ones may replace, 0 = none.
+__host__ __device__ __forceinline__ int g4_cap_rounds(const G4Tail& tail) {
+  const int whole = tail.rounds + (tail.tiles > 0 ? 1 : 0);
+  return tail.parts > 1 || whole > G4_CAP_ROUNDS ? 0 : whole;
+}
+
+// The cheapest cap if it is worth leaving `whole` rounds of whole tiles for, else 0. cost: of a cap.
+template <class Cost>
+__host__ __device__ __forceinline__ int g4_best_cap(int whole, int pairs, const Cost& cost) {
+  const int old = whole * (100 * pairs + G4_TILE_COST);
   int best = 0, limit = old - old / 12;
 #pragma unroll
-  for (int c = 4; c >= 0; --c) {
-    const int v = __builtin_amdgcn_readlane(cost, c);
-    if (v < limit) { limit = v; best = c + G4_MIN_BLOCKS; }
+  for (int cap = G4_BM / 32; cap >= G4_MIN_BLOCKS; --cap) {
+    const int v = cost(cap);
+    if (v < limit) { limit = v; best = cap; }
   }
   return best;
+}
+
+// On the device lane i works out cap 4 + i.
+template <G4Type TY, int FEAT>
+__device__ __forceinline__ int g4_cap(const GemmArgs& args, const G4Segments& seg, const G4Tail& tail, int blocks, int lane) {
+  const int whole = g4_cap_rounds(tail);
+  if (TY == G4_F8 || whole == 0) return 0;
+  auto rows = [&](int g) {
+    int rb, re;
+    seg.get(args.g[g], rb, re);
+    return re - rb;
+  };
+  const int mine = g4_cap_cost(args, FEAT, rows, blocks, G4_MIN_BLOCKS + min(lane, 4));
+  return g4_best_cap(whole, args.g[0].kbytes / (2 * BK), [&](int cap) { return __builtin_amdgcn_readlane(mine, cap - G4_MIN_BLOCKS); });
+}
+
+// On the host, where the rows of a launch are known; -1: the device has to find it. On the device -> on the host, Linears in bf16, us: 700 rows
+// by 2560 x 10240 38.5 -> 37.5, 1500 57.8 -> 57.1; 6000 by 2560 x 2560 (whole tiles) 57.8 -> 57.0.
+inline int g4_host_cap(const GemmArgs& args, int feat, int min_pairs, int blocks) {
+  int total = 0, padding = 0;
+  for (int g = 0; g < args.G; ++g) {
+    if (args.g[g].row_begin < 0) return -1;
+    const int rows = args.g[g].row_end - args.g[g].row_begin, mt = (rows + G4_BM - 1) / G4_BM, nt = args.g[g].n_out / feat;
+    total += mt * nt;
+    padding += (mt * G4_BM - rows) * nt;
+  }
+  const int pairs = args.g[0].kbytes / (2 * BK);
+  const G4Tail tail = args.tail == nullptr || total == 0 ? G4Tail{total / blocks, total % blocks, 1} : g4_plan_tail(total, blocks, pairs, min_pairs, padding);
+  const int whole = g4_cap_rounds(tail);
+  if (whole == 0) return 0;
+  auto rows = [&](int g) { return args.g[g].row_end - args.g[g].row_begin; };
+  return g4_best_cap(whole, pairs, [&](int cap) { return g4_cap_cost(args, feat, rows, blocks, cap); });
 }
 
 template <G4Type TY, int EPI>
@@ -228,7 +269,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   const int xcd = blockIdx.x % HDMOE_NUM_XCD, slot = blockIdx.x / HDMOE_NUM_XCD;
   const int nslots = gridDim.x / HDMOE_NUM_XCD;
   const G4Tail tail = g4_tail_of<TY, FEAT>(args, segs, gridDim.x);
-  const int cap = EPI == G4_PARTIAL || SWIGLU || args.spread != 0 ? 0 : sgpr(g4_cap<TY, FEAT>(args, segs, tail, gridDim.x, lane));
+  const int cap = EPI == G4_PARTIAL || SWIGLU || args.spread != 0 ? 0 : args.cap >= 0 ? args.cap : sgpr(g4_cap<TY, FEAT>(args, segs, tail, gridDim.x, lane));
   // cap > 0: lane g looks up where group g comes in the order of heights: [first tile, tiles, height, m-tiles]
   v4i* const heights = reinterpret_cast<v4i*>(smem + G4_HEIGHTS);
   if (cap > 0) {

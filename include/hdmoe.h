@@ -103,6 +103,11 @@ const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E, int D, int
  * together. For tests and reports. No counterpart in the reference. */
 int hdmoe_tail_plan(int weight_dtype, int tiles, int K, int padding, int* rounds, int* left);
 
+/* Rows of a tile of the Linear on `rows` 16-bit activations (hdmoe_linear_groups with its working memory): 256, or 128 to 224 where
+ * no tile is cut along K and lower tiles fill the CUs' rounds better; 0 = sizes that its kernel does not take. weight_dtype
+ * HDMOE_W_BF16, HDMOE_W_F16 or HDMOE_W_E4M3FN_UPCAST. For tests and reports. No counterpart in the reference. */
+int hdmoe_linear_tile_rows(int weight_dtype, int rows, int K, int N);
+
 /* ---- stage entry points ------------------------------------------------------ */
 
 /* MoEGate.forward, comfy/ldm/hidream/model.py:263-283 (F.linear :268, softmax :270,
