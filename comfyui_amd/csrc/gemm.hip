@@ -1304,8 +1304,8 @@ FormChoice pick_form(const GemmShape& sh) {
   c.tall = (sh.fp8 || (sh.swiglu && !sh.g4_takes)) && !sh.split && !c.light && expected_tile_cost(sh, 5) < expected_tile_cost(sh, 4);
   // fp8 down projection on the 4-wave kernel, unless the 320-token tile saves more than a quarter of the rounds. Whole layer, 8- against
   // 4-wave, us: cut along K 260 tokens 110, 103; 600 177, 169; 1024 226, 207; 1536 254, 240; 2000 304, 284; whole tiles 4000
-  // 537, 503; 5000 649, 624 (320-token tiles would take 0.8 of the rounds); 8000 969, 917; 2300 (0.6 of the rounds) 341, 349. The forced forms
-  // are kernels of one family with the same bytes; this one sums 128 products at a time instead of 64 (an output of 1e7 differs).
+  // 537, 503; 5000 649, 624 (320-token tiles would take 0.8 of the rounds); 8000 969, 917; 2300 (0.6 of the rounds) 341, 349. Not with a
+  // forced form: the parts of a cut projection end elsewhere here (on pairs of K steps); uncut the bytes are the same.
   c.fp8_g4 = sh.fp8 && !sh.swiglu && sh.g4_takes && !c.light && f_light == HDMOE_FORM_AUTO && f_4w == HDMOE_FORM_AUTO &&
              !(c.tall && 4 * expected_tile_cost(sh, 5) < 3 * expected_tile_cost(sh, 4));
   if (c.fp8_g4) c.tall = false;

@@ -312,7 +312,7 @@ def step(dt, w8, gelu, stage, first, at):
 
 
 def frag8(kind, i):
-    """fp8: the 8 registers of a fragment (32 bytes per lane: its 16-byte chunks g and 4 + g, g = lane / 16)."""
+    """fp8: the 8 registers of a fragment (32 bytes per lane: the places g and 4 + g of its row in LDS, g = lane / 16; f8_chunk in gemm4w.h)."""
     return FRAG[(kind, i // 4)] + 8 * (i % 4)
 
 

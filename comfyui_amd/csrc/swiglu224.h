@@ -102,7 +102,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   // row (r >> 2) * 16 + t * 4 + (r & 3).
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
   int ld_row = wave * 8 + (lane >> 3);                 // row within a 32-row slab
-  int ld_chunk = (lane & 7) ^ swz(ld_row);
+  int ld_chunk = f8_chunk((lane & 7) ^ swz(ld_row));
   const int ldsw = sgpr((int)lds0 + wave * 1024);
   const int fr_row = lane & 15, fr_grp = lane >> 4, fr_swz = swz(fr_row);
   const int kb = args.g[0].kbytes;

@@ -69,8 +69,9 @@ const char* hdmoe_last_error(void);
 /* Kernel-form switches. No counterpart in the reference: both choose between kernels of this library whose results are
  * the same bit for bit, for tests that compare the forms and for measurements. Process-wide; a call in flight on
  * another thread sees the old or the new value. A HIP graph keeps the kernels that were captured. Where both are AUTO,
- * the fp8 contractions may run on kernels outside of that family, with sums of 128 products where these have 64: about
- * one output in 10^7 then differs from the forced forms' by a rounding.
+ * the fp8 contractions may run on kernels that no switch forces (swiglu224_kernel, the 4-wave form of the plain contractions): with
+ * the same bytes again, but for a down projection that is cut along K, whose parts those end on pairs of K steps, so that the
+ * fp32 sums of a row are added up in another order. Forcing either switch keeps both contractions off them.
  *   HDMOE_FORM_SWIGLU4W: the fp8 gate/up contraction has an 8-wave kernel (256- or 320-token tiles) and a 4-wave one
  *     (one wave per SIMD, 256-token tiles, a tile's SiLU*mul epilogue issued between the MFMAs of the next tile; needs
  *     K a multiple of 256 and at least 2048, and scale_in2). AUTO: the 4-wave kernel runs where neither the kernel on
