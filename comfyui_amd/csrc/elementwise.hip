@@ -415,11 +415,14 @@ int hdmoe_launch_quant_dispatch(const void* x_bf16, const int32_t* perm, const i
 
 int hdmoe_launch_quant_rows(const void* x_bf16, int64_t rows, int D, const float* scale_input_dev,
                             const float* scale_input_also_dev, void* out_fp8, hipStream_t s, const char* what) {
-  const long units = rows * (long)(D / 8);
-  const long blocks = (units + QUANT_UNITS * THREADS - 1) / (QUANT_UNITS * THREADS);
-  if (blocks > 0x7fffffff) return hdmoe_fail(HDMOE_E_SHAPE, "%s: %lld rows of %d are too many", what, (long long)rows, D);
-  hipLaunchKernelGGL(quant_rows_kernel, dim3((uint32_t)blocks), dim3(THREADS), 0, s, static_cast<const uint4*>(x_bf16), units,
-                     scale_input_dev, scale_input_also_dev, static_cast<uint2*>(out_fp8));
+  const long units = rows * (long)(D / 8), most = QUANT_UNITS * THREADS * (1l << 23);   // a launch has less than 2^32 threads
+  const uint4* const xp = static_cast<const uint4*>(x_bf16);
+  uint2* const op = static_cast<uint2*>(out_fp8);
+  for (long at = 0; at < units; at += most) {
+    const long n = units - at < most ? units - at : most;
+    const uint32_t blocks = (uint32_t)((n + QUANT_UNITS * THREADS - 1) / (QUANT_UNITS * THREADS));
+    hipLaunchKernelGGL(quant_rows_kernel, dim3(blocks), dim3(THREADS), 0, s, xp + at, n, scale_input_dev, scale_input_also_dev, op + at);
+  }
   return hdmoe_check_launch(what);
 }
 

@@ -236,3 +236,21 @@ def test_swiglu_epilogue_cast_overflows_to_nan_like_torch(dev, rows, next_scale)
     step = torch.maximum(want_f.abs(), torch.tensor(2.0 ** -6)) * 2.0 ** -3 * 1.001   # one e4m3 step at that magnitude
     assert bool(((got_f - want_f).abs()[ok] <= step[ok]).all())
     assert float((got_f[ok] == want_f[ok]).float().mean()) > 0.99
+
+
+def test_quant_fp8_of_more_blocks_than_a_launch_takes(dev):
+    """A launch has less than 2^32 threads; 8 values and two units a thread make that 6.9e10 values of a tensor."""
+    rows, D = (1 << 20) + 1, 1 << 16
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < rows * D * 3 + (4 << 30):
+        pytest.skip("needs 210 GB of device memory")
+    x = torch.empty((rows, D), dtype=BF16, device=dev)   # only what is looked at is filled
+    ends = [0, rows // 2 - 1, rows // 2, rows - 2, rows - 1]
+    for i in ends:
+        x[i] = torch.randn(D, device=dev).to(BF16)
+    s = torch.tensor(0.13, device=dev)
+    got = _hf().quant_fp8(x, s)
+    for i in ends:
+        assert torch.equal(got[i].view(torch.uint8), _hf().quant_fp8(x[i].clone(), s).view(torch.uint8)), i
+    del x, got
+    torch.cuda.empty_cache()
