@@ -95,6 +95,7 @@ SIGNATURES = {
     "hdmoe_set_kernel_form": (c_int, [c_int, c_int]),
     "hdmoe_get_kernel_form": (c_int, [c_int]),
     "hdmoe_gate_up_kernel_name": (ctypes.c_char_p, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
+    "hdmoe_plain_kernel_name": (ctypes.c_char_p, [c_int] * 8),
     "hdmoe_tail_plan": (c_int, [c_int, c_int, c_int, c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_int)]),
     "hdmoe_linear_tile_rows": (c_int, [c_int, c_int, c_int, c_int]),
     "hdmoe_gate_top2": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),

@@ -1603,6 +1603,16 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
                 : launch_grouped<BF16_PLAIN>(args, tile_bound, s, what);
 }
 
+// An fp8 Linear with a bias: the 192-token tile of the 8-wave kernel, where its rounds of tiles cost a tenth less than those of 256 tokens
+// (as expected_tile_cost counts them: rounds x (TT + 1)).
+// With the cast in front, 4-wave kernel on 256-token tiles against this, us, rows by K x N: 4480 by 2560 x 2560 39.4, 38.6 (180 and 240
+// tiles on 256 CUs); 193 by 4096 x 2560 41.2, 36.4 (fewer products of padding); 1000 by 2560 x 2560 34.4, 28.8; 300 by 2560 x 10240 32.0,
+// 27.4, 2000 63.8, 60.2; 9000 by 2048 x 2048 58.6, 54.1, by 4096 x 2560 103.6, 99.9; at the line 4480 by 4096 x 2560 53.5, 53.8.
+static bool fp8_linear_192(int rows, int N) {
+  auto cost = [&](int tt) { return (long)(((rows + 64 * tt - 1) / (64 * tt) * (N / BN) + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU) * (tt + 1); };
+  return 10 * cost(3) <= 9 * cost(4);
+}
+
 // Name of the kernel the gate/up contraction of a layer runs on (T tokens, E routed experts top-2 plus a shared expert
 // if Hs > 0), by the launcher's own rule and the current form switches: for reports that name the dominant kernel.
 extern "C" const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E, int D, int H, int Hs,
@@ -1630,6 +1640,31 @@ extern "C" const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E,
       if (!sh.fp8 && sh.g4_takes) return "gemm4w_kernel<SWIGLU>";
       return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 4>" : "grouped_gemm_kernel<BF16_SWIGLU, 4>";
   }
+}
+
+// The same for an fp8 contraction without activation: a down projection (E experts' segments of rows_dyn rows together, rows_static
+// of one more) in `parts` parts along K, or a Linear (E = 0) with a bias.
+extern "C" const char* hdmoe_plain_kernel_name(int rows_dyn, int E, int K_dyn, int rows_static, int K_static, int N, int parts,
+                                               int has_bias) {
+  if (rows_dyn < 0 || E < 0 || E > HDMOE_MAX_EXPERTS || rows_static < 0 || N <= 0 || N % BN != 0 || parts < 1) return "";
+  const int n_dyn = rows_dyn > 0 ? E : 0;
+  auto bad = [](int rows, int K) { return rows > 0 && (K <= 0 || K % BK != 0); };
+  if (bad(n_dyn, K_dyn) || bad(rows_static, K_static) || (n_dyn == 0 && rows_static == 0)) return "";
+  const bool takes = g4_takes_k(n_dyn > 0 ? rows_dyn : 0, K_dyn, rows_static, K_static);
+  if (has_bias != 0) {
+    if (fp8_linear_192(rows_static, N)) return "grouped_gemm_kernel<FP8_PLAIN_BIAS, 3>";
+    return takes ? "gemm4w_kernel<F8, BIAS>" : "grouped_gemm_kernel<FP8_PLAIN_BIAS, 4>";
+  }
+  GemmShape sh;
+  sh.swiglu = false; sh.fp8 = true; sh.split = parts > 1; sh.w8 = false; sh.w4_fits = sh.s224_fits = false;
+  sh.rows_dyn = n_dyn > 0 ? rows_dyn : 0; sh.n_dyn = n_dyn; sh.rows_static = rows_static;
+  sh.N_dyn = sh.N_static = N;
+  sh.g4_takes = takes;
+  const FormChoice c = pick_form(sh);
+  const int shortest = n_dyn > 0 && (rows_static == 0 || K_dyn < K_static) ? K_dyn : K_static;
+  if (c.fp8_g4 && shortest / (2 * BK) / parts >= 2) return parts > 1 ? "gemm4w_kernel<F8, PARTIAL>" : "gemm4w_kernel<F8, PLAIN>";
+  if (c.light) return parts > 1 ? "grouped_gemm_kernel<FP8_PLAIN, 2, LIGHT>" : "grouped_gemm_kernel<FP8_PLAIN, 4, LIGHT>";
+  return parts == 1 && c.tall ? "grouped_gemm_kernel<FP8_PLAIN, 5>" : "grouped_gemm_kernel<FP8_PLAIN, 4>";
 }
 
 // How the down projection of a layer is cut along K: a pure function of the sizes, so that the workspace layout and
@@ -1886,13 +1921,8 @@ int hdmoe_launch_linear_bias(int weight_dtype, const uint8_t* a, int rows, int K
   gg.bias = bias;
   gg.act = HDMOE_ACT_NONE;
   args.G = 1;
-  // The 192-token tile where its rounds of tiles cost a tenth less (as expected_tile_cost counts them: rounds x (TT + 1)).
-  // With the cast in front, 256- against 192-token tiles, us, rows by K x N: 4480 by 2560 x 2560 37.8, 35.4 (180 and 240 tiles on 256
-  // CUs); 193 by 4096 x 2560 44.5, 39.3 and 1 by 4096 x 2560 40.6, 33.8 (fewer products of padding); 1000 by 2560 x 2560 35.8, 32.0;
-  // 2000 by 2560 x 10240 67.6, 61.6; 9000 by 2048 x 2048 62.1, 55.4; below 30 us the host is the slower one.
   auto tiles = [&](int tt) { return (rows + 64 * tt - 1) / (64 * tt) * (N / BN); };
-  auto cost = [&](int tt) { return (long)((tiles(tt) + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU) * (tt + 1); };
-  if (10 * cost(3) <= 9 * cost(4)) return launch_grouped<FP8_PLAIN_BIAS, 3>(args, tiles(3), s, what);
+  if (fp8_linear_192(rows, N)) return launch_grouped<FP8_PLAIN_BIAS, 3>(args, tiles(3), s, what);
   // Else the 4-wave kernel. Without the cast, 8- against 4-wave on 256-token tiles: 8192 by 2560 x 10240 169.8, 157.7; 3000 67.8, 65.7;
   // 1300 36.2, 35.3; 5000 by 6912 x 2560 72.6, 68.5; 5000 by 2560 x 2560 33.8, 33.8.
   if (gemm4w_fits(args, false)) return launch_gemm4w<G4_F8, G4_BIAS>(args, rows, s, what);

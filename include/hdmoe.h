@@ -97,6 +97,9 @@ int hdmoe_get_kernel_form(int which);
  * if Hs > 0; has_scale_in2: the w2 Linears carry a scale_input) runs on under the current switches, for reports that
  * name the dominant kernel; "" for sizes the layer does not take. No counterpart in the reference. */
 const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E, int D, int H, int Hs, int has_scale_in2);
+/* The same for an fp8 contraction without activation: a down projection (rows_dyn rows of E experts, rows_static of one more) in
+ * `parts` parts along K, or a Linear on rows_static rows (E = 0), with has_bias or without. "" = sizes out of range. */
+const char* hdmoe_plain_kernel_name(int rows_dyn, int E, int K_dyn, int rows_static, int K_static, int N, int parts, int has_bias);
 
 /* How a contraction on 16-bit activations is dealt out when its `tiles` (256 rows x 256 features, gate/up 128) do not come out
  * even over the CUs: whole rounds of tiles, the tiles left over, and (returned) the parts along K that each of those is cut

@@ -49,9 +49,7 @@ def test_scales_that_one_cast_cannot_serve(dev):
     mods = [torch.zeros((1, 1, 512), dtype=BF16, device=dev) + 0.5 for _ in range(3)]
     assert bool(torch.isfinite(ff.forward_branch(x, *mods).float()).all())
     ff.w3.scale_input.data.fill_(0.25)
-    y = ff.forward_branch(x, *mods)
-    assert bool(torch.isnan(y.float()).all()) or torch.equal(y, HF.gated_residual(
-        ff(HF.ln_modulate(x.view(-1, 512), mods[1], mods[0], 40).view(1, 40, 512)).view(-1, 512), mods[2], x.view(-1, 512), 40).view_as(y))
+    assert bool(torch.isnan(ff.forward_branch(x, *mods).float()).all())   # (written through .data: the cached comparison still stands)
 
 
 def test_a_forward_of_ones_own_is_called(dev):

@@ -1,7 +1,8 @@
 """The fp8 Linear on its 192- and 256-token tiles (csrc/gemm.hip, hdmoe_launch_linear_bias): a row's bytes do not depend on the
 tile it falls into, and are the scaled product with the bias, rounded once.
 
-9000 rows by 10240 features take 256-token tiles, 1 to 1100 rows the 192-token ones."""
+9000 rows by 10240 features take 256-token tiles (of the 4-wave kernel; K = 384 of the 8-wave one), 1 to 1100 rows the 192-token ones.
+Operands on which the kernels' sums would differ if their products came in another order: test_gpu_fp8_same_sums.py."""
 import pytest
 import torch
 

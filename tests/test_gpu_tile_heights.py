@@ -3,10 +3,12 @@ tiles of different heights behind each other in a block, for each way a tile is 
 
 Bound: fp32 sums (K terms, each rounding at most 2^-24 of the running sum of magnitudes) rounded once to 16 bits; the activation is
 compared behind that rounding, with one more step for its own."""
+import ctypes
+
 import pytest
 import torch
 
-from comfyui_amd import synth
+from comfyui_amd import _lib, synth
 
 pytestmark = pytest.mark.gpu
 BF16, F16 = torch.bfloat16, torch.float16
@@ -23,12 +25,15 @@ def within(y, a, w, bias, scale, act, dt):
     assert bool((err <= lim).all()), float((err / lim).max())
 
 
-# rows of one Linear at 10 n-tiles: the caps come to 1 to 52 m-tiles of 4 to 8 blocks of 32 rows
-@pytest.mark.parametrize("rows", [129, 1690, 3100, 3333, 4161, 5249, 6500, 11111])
+# 10 n-tiles: 1 to 52 m-tiles
+@pytest.mark.parametrize("rows,K,height", [(129, 640, 128), (1690, 640, 128), (3100, 640, 128), (3333, 640, 160), (4161, 640, 192), (4801, 2560, 224),
+                                           (5249, 640, 256), (6500, 640, 128), (10209, 2560, 224), (11111, 640, 256)])
 @pytest.mark.parametrize("kind", ["bf16", "f16", "upcast"])
-def test_linear(dev, rows, kind):
+def test_linear(dev, rows, K, height, kind):
     from comfyui_amd import functional as HF
-    K, N = 640, 2560
+    N = 2560
+    code = {"bf16": _lib.W_BF16, "f16": _lib.W_F16, "upcast": _lib.W_E4M3FN_UPCAST}[kind]
+    assert _lib.lib.hdmoe_linear_tile_rows(code, rows, K, N) == height
     g = torch.Generator(device=dev).manual_seed(rows)
     dt = F16 if kind == "f16" else BF16
     a = torch.randn((rows, K), generator=g, device=dev).to(dt)
@@ -43,6 +48,38 @@ def test_linear(dev, rows, kind):
         for bias in (None, b):
             y = HF.linear(a, w, bias=bias)
             within(y, a, w, bias, 1.0, "none", dt)
+
+
+@pytest.mark.parametrize("code", [_lib.W_BF16, _lib.W_E4M3FN_UPCAST])
+def test_dense_down_projection(dev, code):
+    """The contraction without a bias: rows of a dense feed-forward on lower tiles are those of one on whole tiles (no working memory for
+    parts, and sizes at which the down projection is not cut)."""
+    D = H = 2560
+    g = torch.Generator(device=dev).manual_seed(code)
+    fw, keep = _lib.FfnWeights(), []
+    for i in (1, 2, 3):
+        w = torch.randn((D, H), generator=g, device=dev) * 0.02
+        if code == _lib.W_BF16:
+            keep.append(w.to(BF16))
+        else:
+            w8, s = synth.quantize_per_tensor(w)
+            keep += [s, w8]
+            setattr(fw, f"scale_w{i}", s.data_ptr())
+        setattr(fw, f"w{i}", keep[-1].data_ptr())
+    x = torch.randn((11999, D), generator=g, device=dev).to(BF16)
+
+    def run(rows):
+        ws = torch.empty(-(-rows * H * 2 // 256) * 256, dtype=torch.uint8, device=dev)
+        y = torch.full((rows + 1, D), 7.0, dtype=BF16, device=dev)
+        _lib.check(_lib.lib.hdmoe_ffn_swiglu(code, x.data_ptr(), rows, D, H, ctypes.byref(fw), y.data_ptr(), ws.data_ptr(), ws.numel(), None))
+        torch.cuda.synchronize()
+        assert bool((y[rows] == 7.0).all())
+        return y[:rows]
+    full = run(11999)
+    assert bool(torch.isfinite(full.float()).all()) and float(full.float().std()) > 0
+    for rows, height in ((11999, 256), (3073, 128), (3115, 128), (3627, 160), (8171, 192), (9803, 224)):
+        assert _lib.lib.hdmoe_linear_tile_rows(code, rows, H, D) == height
+        assert torch.equal(run(rows), full[:rows]), rows
 
 
 @pytest.mark.parametrize("sizes", [
