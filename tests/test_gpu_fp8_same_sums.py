@@ -41,13 +41,13 @@ def test_rows_of_a_linear(dev, K, N, sizes, with_bias):
         assert torch.equal(HF.linear(a[:rows].contiguous(), w, s, one, bias=bias), full[:rows]), rows
 
 
-def grouped(dev, sizes, K, N, swiglu, seed):
+def grouped(dev, sizes, K, N, swiglu, seed, scale=2.0 ** -17):
     g = torch.Generator(device=dev).manual_seed(seed)
     E, rows = len(sizes), sum(sizes)
     a = codes((rows, K), g, dev)
     offsets = torch.tensor([0] + list(torch.tensor(sizes).cumsum(0)), dtype=torch.int32, device=dev)
     ws = [[codes((N, K), g, dev) for _ in range(2)] for _ in range(E)]
-    scales = torch.tensor([2.0 ** -17, 2.0 ** -16, 0.75, 0.5], device=dev)
+    scales = torch.tensor([scale, 2 * scale, 0.75, 0.5], device=dev)
     arr = (_lib.FfnWeights * E)()
     for e in range(E):
         if swiglu:
@@ -65,6 +65,7 @@ def grouped(dev, sizes, K, N, swiglu, seed):
         torch.cuda.synchronize()
         return out
     run.keep = (a, offsets, ws, scales)
+    run.operands = a, ws
     return run
 
 
@@ -76,3 +77,17 @@ def test_forms(dev, forms, sizes, K, N, swiglu):
     got = run()
     set_form("HDMOE_SWIGLU4W", "0")
     assert torch.equal(run(), got) and got.float().std() > 0
+
+
+def test_forms_beyond_the_range(dev, forms):
+    """Outputs above 448, infinite sums' products and NaN operands: the same bytes as well."""
+    run = grouped(dev, (700, 900), 2048, 2560, True, 5, scale=2.0 ** -9)
+    a, ws = run.operands
+    a.view(torch.uint8)[::97, 5] = 0x7F
+    ws[1][0].view(torch.uint8)[3] = 0xFF
+    assert _lib.lib.hdmoe_gate_up_kernel_name(_lib.W_E4M3FN, 800, 2, 2048, 2560, 0, 1) == b"swiglu224_kernel"
+    got = run()
+    nan = (got & 0x7F) == 0x7F
+    assert 0.01 < float(nan.float().mean()) < 0.99
+    set_form("HDMOE_SWIGLU4W", "0")
+    assert torch.equal(run() & 0x7F, got & 0x7F) and torch.equal(run()[~nan], got[~nan])   # the sign of a NaN is nobody's
