@@ -8,7 +8,8 @@
 // in bf16). Through a scratch buffer in global memory (256-token tiles) that costs more than hiding the activation gains; 224 tokens leave
 // room for 22 of 28 pieces in registers (224 accumulators and 120 fragment registers are in use) and for 6 in LDS. 8192 tokens, 2560 x
 // (4 x 6912 + 3584), us: 8-wave kernel on 320-token tiles 652; 256-token tiles through a scratch buffer 660, of which the buffer 117 and
-// the hidden vector instructions 27; this kernel 577 (2.53 PFLOP/s). 4096 tokens: 365 (4-wave kernel of swiglu4w.h) -> 302.
+// the hidden vector instructions 27; this kernel 577 (2.53 PFLOP/s; back to back inside a layer, on other cards, 533 to 540: 2.7). 4096
+// tokens: 365 (4-wave kernel of swiglu4w.h) -> 302.
 //
 // Limits (the launcher takes another kernel otherwise): K the same for all groups, a multiple of 256 bytes and at least 2048, every
 // group with a scale_input for the consuming Linear (no clamp form of the cast), a gathered operand under 2 GiB.
