@@ -25,22 +25,25 @@ __device__ __forceinline__ float inv_scale(const float* s) { return hdmoe_q_unif
 
 // scale_in_also: scale_input of a second Linear that reads this cast (w3 beside w1). Where its cast factor differs the
 // one cast cannot serve both: the rows are written as NaN (products with a NaN factor).
-// One factor for all rows, so they are one array: a block takes QUANT_UNITS x 256 units of 16 bytes, a thread's loads all in flight
-// and as many blocks as that makes. Bound by memory (9000 rows of 4096: 5.3 TB/s) or, up to a thousand rows, by the launch. A wave per
-// row with a loop over its units -> this: 300 rows of 2560 3.0 -> 2.1 us, 4480 6.7 -> 6.8, 9000 rows of 4096 27.0 -> 20.9
-// (4 units: 2.3, 6.9 and 21.3; 8: 2.9, 7.0 and 22.4).
-constexpr int QUANT_UNITS = 2;
+// One factor for all rows, so they are one array: a block takes QUANT_UNITS x 256 units of 16 bytes at a time, a thread's loads all in flight.
+// Bound by memory (9000 rows of 4096: 5.3 TB/s) or, up to a thousand rows, by the launch. Up to QUANT_LOOP times the blocks that
+// are resident at once they loop, because the last round of blocks would be a short one; beyond, that matters less than their start.
+// A wave per row with a loop over its units -> this, us, rows of 2560: 300 3.6 -> 2.7, 4480 6.2 -> 5.6, 6000 8.1 -> 8.1, 7000 9.6 -> 9.8, 9000 of
+// 4096 18.8 -> 16.9 (without looping 6000 8.4, 7000 10.0; clamped 9.2 and 10.8; 4 units 3.0, 5.7, 7.4 and 16.9; one unit 2.5, 6.1, 8.0, 17.4).
+constexpr int QUANT_UNITS = 2, QUANT_RESIDENT = 8 * HDMOE_NUM_CU, QUANT_LOOP = 3;
 __global__ __launch_bounds__(THREADS) void quant_rows_kernel(const uint4* __restrict__ x, long units, const float* scale_in,
                                                              const float* scale_in_also, uint2* __restrict__ out) {
-  const long u0 = (long)blockIdx.x * (QUANT_UNITS * THREADS) + threadIdx.x;
-  uint4 v[QUANT_UNITS];
-#pragma unroll
-  for (int k = 0; k < QUANT_UNITS; ++k) v[k] = x[min(u0 + k * THREADS, units - 1)];
+  const long step = (long)gridDim.x * (QUANT_UNITS * THREADS);
   float inv = inv_scale(scale_in);
   if (scale_in_also != scale_in && inv_scale(scale_in_also) != inv) inv = __builtin_nanf("");
+  for (long u0 = (long)blockIdx.x * (QUANT_UNITS * THREADS) + threadIdx.x; u0 < units; u0 += step) {
+    uint4 v[QUANT_UNITS];
 #pragma unroll
-  for (int k = 0; k < QUANT_UNITS; ++k)
-    if (u0 + k * THREADS < units) out[u0 + k * THREADS] = quant8(v[k], inv);
+    for (int k = 0; k < QUANT_UNITS; ++k) v[k] = x[min(u0 + k * THREADS, units - 1)];
+#pragma unroll
+    for (int k = 0; k < QUANT_UNITS; ++k)
+      if (u0 + k * THREADS < units) out[u0 + k * THREADS] = quant8(v[k], inv);
+  }
 }
 
 // Quantise the rows the expert GEMMs read: sorted rows [0, rows_routed) gather token perm[r]/2 with the
@@ -420,7 +423,8 @@ int hdmoe_launch_quant_rows(const void* x_bf16, int64_t rows, int D, const float
   uint2* const op = static_cast<uint2*>(out_fp8);
   for (long at = 0; at < units; at += most) {
     const long n = units - at < most ? units - at : most;
-    const uint32_t blocks = (uint32_t)((n + QUANT_UNITS * THREADS - 1) / (QUANT_UNITS * THREADS));
+    uint32_t blocks = (uint32_t)((n + QUANT_UNITS * THREADS - 1) / (QUANT_UNITS * THREADS));
+    if (blocks > QUANT_RESIDENT && blocks <= QUANT_LOOP * QUANT_RESIDENT) blocks = QUANT_RESIDENT;
     hipLaunchKernelGGL(quant_rows_kernel, dim3(blocks), dim3(THREADS), 0, s, xp + at, n, scale_input_dev, scale_input_also_dev, op + at);
   }
   return hdmoe_check_launch(what);

@@ -99,7 +99,7 @@ def test_quant_fp8_scaled(dev, scale):
     assert torch.equal(got, want)
 
 
-@pytest.mark.parametrize("rows,D", [(1, 8), (3, 1368), (1, 4096), (1, 4104), (511, 8), (513, 8), (5000, 2560)])   # a block takes 512 units of 8
+@pytest.mark.parametrize("rows,D", [(1, 8), (3, 1368), (1, 4096), (1, 4104), (511, 8), (513, 8), (5000, 2560), (3072, 8192), (3073, 8192)])   # a block takes 512 units of 8, once or up to three times
 def test_quant_fp8_sizes(dev, rows, D):
     x = torch.randn((rows, D), generator=torch.Generator().manual_seed(rows)).to(BF16)
     s = torch.tensor(0.13, dtype=torch.float32)
