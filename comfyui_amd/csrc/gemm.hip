@@ -96,6 +96,9 @@ struct GemmGroup {
   float* pout;          // split K: row 0 of this group in part 0 of the fp32 partial sums, [parts][rows][n_out]
 };
 
+// What the lists of tiles are made of, group by group, packed for one load (Segments).
+struct GemmSegment { int row_begin, row_end, n_out, kbytes; };
+
 struct GemmArgs {
   GemmGroup g[MAX_GROUPS];
   const int32_t* offsets;  // segment bounds of the dynamic groups, n_offsets + 1 entries
@@ -116,7 +119,45 @@ struct GemmArgs {
   // gemm4w_kernel only
   uint8_t* scratch;       // with GELU: G4_SCRATCH bytes per block
   float* tail;            // room for the parts of tail tiles (G4_TAIL_BYTES), NULL = tiles are not cut
+  GemmSegment seg[MAX_GROUPS] __attribute__((aligned(16)));   // filled in by the launch functions (fill_segments)
   int cap;                // height of the tiles in blocks of 32 rows at most, 0 = whole tiles, -1 = by the segments' sizes
+};
+
+// a / b for 0 <= a, 0 < b; the approximate quotient of a below 2^22 is at most one off
+__device__ __forceinline__ int tile_div(int a, int b) {
+  if (a >> 22) return a / b;
+  const int q = (int)((float)a * __builtin_amdgcn_rcpf((float)b)), r = a - q * b;
+  return q + (r >= b ? 1 : 0) - (r < 0 ? 1 : 0);
+}
+
+// The groups' segments, lane g holding those of group g (none beyond the last one; dynamic groups come first). Read by one vector
+// load: a group at a time they arrive a line of the arguments at a time, each wait as long as memory's (0.5 us), and a launch of five groups
+// had looked its first tile up 4 to 6.5 us after its start. Whole pass, us: layer of 64 tokens 80.2 -> 75.5, 256 103.9 -> 98.6, 1024 in
+// bf16 313 -> 305, Hunyuan3D block of 1500 358 -> 347. (A word of every line of the arguments read at once by scalar loads: 64 tokens 78.0, and
+// 1 us more for every launch of one group.)
+struct Segments {
+  int rb, re, n_out, kbytes;
+  unsigned long long fixed;   // bit g: a static group (or none)
+  __device__ __forceinline__ Segments(const GemmArgs& args, int lane) {
+    typedef const __attribute__((address_space(4))) v4i* const_v4i_ptr;
+    v4i s = {0, 0, 0, 0};
+    if (lane < MAX_GROUPS) s = ((const_v4i_ptr)((const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(GemmArgs, seg)))[lane];
+    int from = 0, to = 0;
+    if (args.offsets != nullptr && lane < args.n_offsets) { from = args.offsets[lane]; to = args.offsets[lane + 1]; }
+    fixed = __ballot(s.x >= 0);
+    rb = s.x >= 0 ? s.x : from;
+    re = s.x >= 0 ? s.y : to;
+    n_out = s.z;
+    kbytes = s.w;
+  }
+  __device__ __forceinline__ void get(int g, int& begin, int& end) const {
+    begin = __builtin_amdgcn_readlane(rb, g);
+    end = __builtin_amdgcn_readlane(re, g);
+  }
+  __device__ __forceinline__ int rows(int g) const { return __builtin_amdgcn_readlane(re - rb, g); }
+  __device__ __forceinline__ int ntiles(int g, int feat) const { return __builtin_amdgcn_readlane((int)((unsigned)n_out / (unsigned)feat), g); }
+  __device__ __forceinline__ int bytes(int g) const { return __builtin_amdgcn_readlane(kbytes, g); }
+  __device__ __forceinline__ bool dynamic(int g) const { return !(fixed >> g & 1); }
 };
 
 __device__ __forceinline__ int swz(int row) { return ((row >> 1) & 7) ^ ((row & 1) << 2); }
@@ -280,12 +321,28 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_kernel(const GemmArgs a
   const int wq = wave & 3, wt = wave >> 2;
 
   // ---- tile enumeration (persistent blocks) ----------------------------------------------
-  // Segment bounds of the dynamic groups: one vector load, then lane reads.
-  int off_lane = 0;
-  if (args.offsets != nullptr && lane <= args.n_offsets) off_lane = args.offsets[lane];
-  auto seg = [&](const GemmGroup& gg, int& rb, int& re) {
-    if (gg.row_begin >= 0) { rb = gg.row_begin; re = gg.row_end; }
+  // (the 320-token tile has no registers for them: a group at a time out of the arguments there)
+  constexpr bool LANES = TT != 5;
+  [[maybe_unused]] auto segs = [&] {
+    if constexpr (LANES) return Segments(args, lane);
+    else return 0;
+  }();
+  [[maybe_unused]] int off_lane = 0;
+  if constexpr (!LANES) {
+    if (args.offsets != nullptr && lane <= args.n_offsets) off_lane = args.offsets[lane];
+  }
+  auto seg = [&](const GemmGroup& gg, [[maybe_unused]] int g, int& rb, int& re) {
+    if constexpr (LANES) segs.get(g, rb, re);
+    else if (gg.row_begin >= 0) { rb = gg.row_begin; re = gg.row_end; }
     else { rb = __builtin_amdgcn_readlane(off_lane, gg.dyn); re = __builtin_amdgcn_readlane(off_lane, gg.dyn + 1); }
+  };
+  auto dynamic = [&](int g) -> bool {
+    if constexpr (LANES) return segs.dynamic(g);
+    else return args.g[g].row_begin < 0;
+  };
+  auto ntiles_of = [&](int g) -> int {
+    if constexpr (LANES) return segs.ntiles(g, FEAT_PER_TILE);
+    else return args.g[g].n_out / FEAT_PER_TILE;
   };
   // the gathered token operand: as the groups describe it, or the alternative the flag selects
   const bool use_alt = args.alt.flag != nullptr && __builtin_amdgcn_readfirstlane(*args.alt.flag) == 0;
@@ -299,20 +356,20 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_kernel(const GemmArgs a
     int mt_dyn = 0, mt_static = 0;
     for (int g = 0; g < args.G; ++g) {
       int rb, re;
-      seg(args.g[g], rb, re);
+      seg(args.g[g], g, rb, re);
       const int mt = (re - rb + args.plan.bm - 1) / args.plan.bm;  // the plan's own tile height: the other kernel's count
-      if (args.g[g].row_begin < 0) mt_dyn += mt;
+      if (dynamic(g)) mt_dyn += mt;
       else mt_static += mt;
     }
-    plan_idx = hdmoe_plan_pick(args.plan, mt_dyn, mt_static, args.g[0].n_out / FEAT_PER_TILE);
+    plan_idx = hdmoe_plan_pick(args.plan, mt_dyn, mt_static, ntiles_of(0));
   }
   const int parts_dyn = args.nparts > 1 ? args.plan.pd[plan_idx] : 1, parts_static = args.nparts > 1 ? args.plan.ps[plan_idx] : 1;
-  auto parts_of = [&](int g) { return args.g[g].row_begin < 0 ? parts_dyn : parts_static; };
+  auto parts_of = [&](int g) { return dynamic(g) ? parts_dyn : parts_static; };
   int total = 0;
   for (int g = 0; g < args.G; ++g) {
     int rb, re;
-    seg(args.g[g], rb, re);
-    total += ((re - rb + BM - 1) / BM) * (args.g[g].n_out / FEAT_PER_TILE) * parts_of(g);
+    seg(args.g[g], g, rb, re);
+    total += ((re - rb + BM - 1) / BM) * ntiles_of(g) * parts_of(g);
   }
   // Each XCD (block ids congruent mod 8) walks one contiguous eighth of the tile list and its blocks take
   // consecutive tiles, so the CUs of an XCD share operand tiles in their L2.
@@ -320,6 +377,7 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_kernel(const GemmArgs a
   const int xcd = blockIdx.x % HDMOE_NUM_XCD, slot = blockIdx.x / HDMOE_NUM_XCD;
   const int nslots = gridDim.x / HDMOE_NUM_XCD;
 
+  auto div = [](int a, int b) { return LANES ? tile_div(a, b) : a / b; };
   struct Tile { int g, row0, rows_here, n0, kbytes, part, kt0, nkt; };
   auto decode = [&](int i) -> Tile {
     Tile d = {-1, 0, 0, 0, 0, 0, 0, 0};
@@ -332,9 +390,9 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_kernel(const GemmArgs a
       int k = 0;
       for (; k < args.G; ++k) {
         g = args.spread > 0 ? k : args.G - 1 - k;
-        seg(args.g[g], rb, re);
+        seg(args.g[g], g, rb, re);
         mtiles = (re - rb + BM - 1) / BM;
-        ntiles = args.g[g].n_out / FEAT_PER_TILE;
+        ntiles = ntiles_of(g);
         const long long tiles = (long long)mtiles * ntiles * parts_of(g);
         const int lo = (int)(xcd * tiles / HDMOE_NUM_XCD), hi = (int)((xcd + 1) * tiles / HDMOE_NUM_XCD);
         if (in_xcd < hi - lo) { L = lo + in_xcd; break; }
@@ -345,9 +403,9 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_kernel(const GemmArgs a
       L = xcd * per_xcd + in_xcd;
       if (in_xcd >= per_xcd || L >= total) return d;
       for (; g < args.G; ++g) {
-        seg(args.g[g], rb, re);
+        seg(args.g[g], g, rb, re);
         mtiles = (re - rb + BM - 1) / BM;
-        ntiles = args.g[g].n_out / FEAT_PER_TILE;
+        ntiles = ntiles_of(g);
         const int tiles = mtiles * ntiles * parts_of(g);
         if (L < tiles) break;
         L -= tiles;
@@ -355,24 +413,26 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_kernel(const GemmArgs a
       if (g >= args.G) return d;
     }
     // split K: the parts of a group one after the other (tiles of one part share operand slices, parts do not)
-    const int part = L / (mtiles * ntiles);
+    const int part = div(L, mtiles * ntiles);
     L -= part * (mtiles * ntiles);
     // bands of GROUP_M m-tiles; a short remainder joins the last band, so that the cheap partial m-tile at the
     // end of a segment is interleaved with full ones instead of forming a run of its own
     const int nbands = max(1, (mtiles + GROUP_M / 2) / GROUP_M);
-    const int band = min(L / (GROUP_M * ntiles), nbands - 1);
+    const int band = min(div(L, GROUP_M * ntiles), nbands - 1);
     const int first_m = band * GROUP_M;
     const int gm = band == nbands - 1 ? mtiles - first_m : GROUP_M;
     const int within = L - band * (GROUP_M * ntiles);
+    const int n = div(within, gm);
     d.g = g;
-    d.row0 = rb + (first_m + within % gm) * BM;
+    d.row0 = rb + (first_m + within - n * gm) * BM;
     d.rows_here = min(re - d.row0, BM);
-    d.n0 = (within / gm) * FEAT_PER_TILE;
-    d.kbytes = args.g[g].kbytes;
+    d.n0 = n * FEAT_PER_TILE;
+    if constexpr (LANES) d.kbytes = segs.bytes(g);
+    else d.kbytes = args.g[g].kbytes;
     const int ktf = d.kbytes / BK;
     d.part = part;
-    d.kt0 = ktf * part / parts_of(g);
-    d.nkt = ktf * (part + 1) / parts_of(g) - d.kt0;
+    d.kt0 = div(ktf * part, parts_of(g));
+    d.nkt = div(ktf * (part + 1), parts_of(g)) - d.kt0;
     return d;
   };
 
@@ -1084,8 +1144,12 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const SplitKReduceAr
   }
 }
 
+void fill_segments(GemmArgs& args) {
+  for (int g = 0; g < args.G; ++g) args.seg[g] = {args.g[g].row_begin, args.g[g].row_end, args.g[g].n_out, args.g[g].kbytes};
+}
+
 template <int MODE, int TT = 4, bool LIGHT = false>
-int launch_grouped(const GemmArgs& args, int tile_bound, hipStream_t s, const char* what) {
+int launch_grouped(GemmArgs& args, int tile_bound, hipStream_t s, const char* what) {
   // The opt-in for more than 64 KiB of dynamic LDS is a per-device function attribute: remembered per device
   // and instantiation (a race between two threads sets it twice, which is harmless).
   static bool attr_set[64] = {};
@@ -1098,6 +1162,7 @@ int launch_grouped(const GemmArgs& args, int tile_bound, hipStream_t s, const ch
     if (device >= 0) attr_set[device] = true;
   }
   if (tile_bound <= 0) return HDMOE_OK;
+  fill_segments(args);
   // persistent blocks: one per CU (128 KiB of LDS allow no second one), a multiple of the XCD count
   int grid = (tile_bound + HDMOE_NUM_XCD - 1) / HDMOE_NUM_XCD * HDMOE_NUM_XCD;
   if (grid > HDMOE_NUM_CU) grid = HDMOE_NUM_CU;
@@ -1147,6 +1212,7 @@ int launch_gemm4w(GemmArgs& args, int rows_mean, hipStream_t s, const char* what
     if (e != hipSuccess) return hdmoe_fail(HDMOE_E_LAUNCH, "%s: hipFuncSetAttribute: %s", what, hipGetErrorString(e));
     if (device >= 0) attr_set[device] = true;
   }
+  fill_segments(args);
   if (EPI == G4_PARTIAL || TY == G4_F8) args.tail = nullptr;
   if (args.tail != nullptr) {
     const GemmGroup& first = args.g[0];
@@ -1166,7 +1232,7 @@ int launch_gemm4w(GemmArgs& args, int rows_mean, hipStream_t s, const char* what
   return hdmoe_check_launch(what);
 }
 
-int launch_swiglu4w(const GemmArgs& args, int tile_bound, hipStream_t s, const char* what) {
+int launch_swiglu4w(GemmArgs& args, int tile_bound, hipStream_t s, const char* what) {
   static bool attr_set[64] = {};
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) device = -1;
@@ -1177,13 +1243,14 @@ int launch_swiglu4w(const GemmArgs& args, int tile_bound, hipStream_t s, const c
     if (device >= 0) attr_set[device] = true;
   }
   if (tile_bound <= 0) return HDMOE_OK;
+  fill_segments(args);
   int grid = (tile_bound + HDMOE_NUM_XCD - 1) / HDMOE_NUM_XCD * HDMOE_NUM_XCD;
   if (grid > HDMOE_NUM_CU) grid = HDMOE_NUM_CU;
   hipLaunchKernelGGL(swiglu4w_kernel, dim3(grid), dim3(W4_THREADS), W4_SMEM, s, args);
   return hdmoe_check_launch(what);
 }
 
-int launch_swiglu224(const GemmArgs& args, hipStream_t s, const char* what) {
+int launch_swiglu224(GemmArgs& args, hipStream_t s, const char* what) {
   static bool attr_set[64] = {};
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) device = -1;
@@ -1193,6 +1260,7 @@ int launch_swiglu224(const GemmArgs& args, hipStream_t s, const char* what) {
     if (e != hipSuccess) return hdmoe_fail(HDMOE_E_LAUNCH, "%s: hipFuncSetAttribute: %s", what, hipGetErrorString(e));
     if (device >= 0) attr_set[device] = true;
   }
+  fill_segments(args);
   // one block per CU whatever the number of tiles: a block without any ends at once
   hipLaunchKernelGGL(swiglu224_kernel, dim3(HDMOE_NUM_CU), dim3(G4_THREADS), S224_SMEM, s, args);
   return hdmoe_check_launch(what);

@@ -73,32 +73,15 @@ enum { G4_TOK_ADDR = 0, G4_W_ADDR = 2, G4_TOK_VOFF = 4, G4_W_VOFF = 12, G4_OUT_V
       G4_A10(11), G4_A10(12), G4_A10(13), G4_A10(14), G4_A10(15), G4_A10(16), G4_A10(17), G4_A10(18), G4_A10(19),     \
       G4_A10(20), G4_A10(21), G4_A10(22), G4_A10(23), G4_A10(24), "a250", "a251", "a252", "a253", "a254", "a255"
 
-// Segment bounds of the groups: lane g + 1 of off_lane holds the end of dynamic segment g.
-struct G4Segments {
-  const GemmArgs& args;
-  int off_lane;
-  __device__ __forceinline__ G4Segments(const GemmArgs& a, int lane) : args(a), off_lane(0) {
-    if (a.offsets != nullptr && lane <= a.n_offsets) off_lane = a.offsets[lane];
-  }
-  __device__ __forceinline__ void get(const GemmGroup& gg, int& rb, int& re) const {
-    if (gg.row_begin >= 0) { rb = gg.row_begin; re = gg.row_end; }
-    else {
-      const int dyn = __builtin_amdgcn_readfirstlane(gg.dyn);
-      rb = __builtin_amdgcn_readlane(off_lane, dyn);
-      re = __builtin_amdgcn_readlane(off_lane, dyn + 1);
-    }
-  }
-};
-
 // A tile by its index inside a group of mtiles x ntiles: bands of GROUP_M m-tiles, a short remainder joins the last one.
 __device__ __forceinline__ void g4_raster(int L, int mtiles, int ntiles, int& m, int& n) {
   const int nbands = max(1, (mtiles + GROUP_M / 2) / GROUP_M);
-  const int band = min(L / (GROUP_M * ntiles), nbands - 1);
+  const int band = min(tile_div(L, GROUP_M * ntiles), nbands - 1);
   const int first_m = band * GROUP_M;
   const int gm = band == nbands - 1 ? mtiles - first_m : GROUP_M;
   const int within = L - band * (GROUP_M * ntiles);
-  m = first_m + within % gm;
-  n = within / gm;
+  n = tile_div(within, gm);
+  m = first_m + within - n * gm;
 }
 
 // What is left when every block has had the same number of whole tiles (`rounds`): `tiles` of them, each cut along K into
@@ -127,17 +110,15 @@ __host__ __device__ inline G4Tail g4_plan_tail(int total, int blocks, int pairs,
 
 // The plan of a launch, from the segment sizes on the device; also its number of tiles.
 template <G4Type TY, int FEAT>
-__device__ __forceinline__ G4Tail g4_tail_of(const GemmArgs& args, const G4Segments& seg, int blocks) {
+__device__ __forceinline__ G4Tail g4_tail_of(const GemmArgs& args, const Segments& seg, int blocks) {
   int total = 0, padding = 0;
   for (int g = 0; g < args.G; ++g) {
-    int rb, re;
-    seg.get(args.g[g], rb, re);
-    const int nt = args.g[g].n_out / FEAT, mt = (re - rb + G4_BM - 1) / G4_BM;
+    const int rows = seg.rows(g), nt = seg.ntiles(g, FEAT), mt = (rows + G4_BM - 1) / G4_BM;
     total += mt * nt;
-    padding += (mt * G4_BM - (re - rb)) * nt;
+    padding += (mt * G4_BM - rows) * nt;
   }
   if (args.tail == nullptr || total == 0) return {total / blocks, total % blocks, 1};
-  return g4_plan_tail(total, blocks, args.g[0].kbytes / (2 * BK), TY == G4_W8 ? 3 : 2, padding);
+  return g4_plan_tail(total, blocks, seg.bytes(0) / (2 * BK), TY == G4_W8 ? 3 : 2, padding);
 }
 
 // Tiles of fewer rows, where the tiles left over are not cut. A segment of U blocks of 32 rows takes ceil(U / cap) m-tiles for a
@@ -157,20 +138,19 @@ __host__ __device__ __forceinline__ G4Heights g4_heights(int rows, int cap) {
   return {mt, max((units + mt - 1) / max(mt, 1), G4_MIN_BLOCKS)};
 }
 
-// What a cap comes to; rows(g): the rows of group g.
-template <class Rows>
-__host__ __device__ __forceinline__ int g4_cap_cost(const GemmArgs& args, int feat, const Rows& rows, int blocks, int cap) {
+// What a cap comes to; rows(g), ntiles(g): the rows of group g, its tiles along the features.
+template <class Rows, class Tiles>
+__host__ __device__ __forceinline__ int g4_cap_cost(int G, int pairs, const Rows& rows, const Tiles& ntiles, int blocks, int cap) {
   constexpr int PAIR[5] = {58, 70, 80, 90, 100};
   int n[5] = {0, 0, 0, 0, 0};                  // tiles of each height
-  for (int g = 0; g < args.G; ++g) {
+  for (int g = 0; g < G; ++g) {
     const int have = rows(g);
     if (have <= 0) continue;
     const G4Heights t = g4_heights(have, cap);
-    const int tiles = t.mt * (args.g[g].n_out / feat);
+    const int tiles = t.mt * ntiles(g);
 #pragma unroll
     for (int h = 0; h < 5; ++h) n[h] += t.height == h + G4_MIN_BLOCKS ? tiles : 0;
   }
-  const int pairs = args.g[0].kbytes / (2 * BK);
   int cost = 0, at = 0;
 #pragma unroll
   for (int h = 4; h >= 0; --h) {
@@ -202,16 +182,12 @@ __host__ __device__ __forceinline__ int g4_best_cap(int whole, int pairs, const 
 
 // On the device lane i works out cap 4 + i.
 template <G4Type TY, int FEAT>
-__device__ __forceinline__ int g4_cap(const GemmArgs& args, const G4Segments& seg, const G4Tail& tail, int blocks, int lane) {
+__device__ __forceinline__ int g4_cap(const GemmArgs& args, const Segments& seg, const G4Tail& tail, int blocks, int lane) {
   const int whole = g4_cap_rounds(tail);
   if (TY == G4_F8 || whole == 0) return 0;
-  auto rows = [&](int g) {
-    int rb, re;
-    seg.get(args.g[g], rb, re);
-    return re - rb;
-  };
-  const int mine = g4_cap_cost(args, FEAT, rows, blocks, G4_MIN_BLOCKS + min(lane, 4));
-  return g4_best_cap(whole, args.g[0].kbytes / (2 * BK), [&](int cap) { return __builtin_amdgcn_readlane(mine, cap - G4_MIN_BLOCKS); });
+  const int mine = g4_cap_cost(args.G, seg.bytes(0) / (2 * BK), [&](int g) { return seg.rows(g); }, [&](int g) { return seg.ntiles(g, FEAT); }, blocks,
+                               G4_MIN_BLOCKS + min(lane, 4));
+  return g4_best_cap(whole, seg.bytes(0) / (2 * BK), [&](int cap) { return __builtin_amdgcn_readlane(mine, cap - G4_MIN_BLOCKS); });
 }
 
 // On the host, where the rows of a launch are known; -1: the device has to find it. On the device -> on the host, Linears in bf16, us: 700 rows
@@ -229,7 +205,7 @@ inline int g4_host_cap(const GemmArgs& args, int feat, int min_pairs, int blocks
   const int whole = g4_cap_rounds(tail);
   if (whole == 0) return 0;
   auto rows = [&](int g) { return args.g[g].row_end - args.g[g].row_begin; };
-  return g4_best_cap(whole, pairs, [&](int cap) { return g4_cap_cost(args, feat, rows, blocks, cap); });
+  return g4_best_cap(whole, pairs, [&](int cap) { return g4_cap_cost(args.G, pairs, rows, [&](int g) { return args.g[g].n_out / feat; }, blocks, cap); });
 }
 
 template <G4Type TY, int EPI>
@@ -255,20 +231,19 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   // ---- work items: as grouped_gemm_kernel's tiles --------------------------------------------------------------
   // A wave's lanes look its block's next 64 items up at once and leave them in LDS (one by one, the decoding is a serial
   // chain of integer divisions that the matrix cores would wait for at every tile).
-  const G4Segments segs(args, lane);
-  auto seg = [&](const GemmGroup& gg, int& rb, int& re) { segs.get(gg, rb, re); };
+  const Segments segs(args, lane);
   int plan_idx = 0;
   if (EPI == G4_PARTIAL && args.plan.n > 1) {
     int mt_dyn = 0, mt_static = 0;
     for (int g = 0; g < args.G; ++g) {
       int rb, re;
-      seg(args.g[g], rb, re);
-      (args.g[g].row_begin < 0 ? mt_dyn : mt_static) += (re - rb + args.plan.bm - 1) / args.plan.bm;
+      segs.get(g, rb, re);
+      (segs.dynamic(g) ? mt_dyn : mt_static) += (re - rb + args.plan.bm - 1) / args.plan.bm;
     }
-    plan_idx = hdmoe_plan_pick(args.plan, mt_dyn, mt_static, args.g[0].n_out / FEAT);
+    plan_idx = hdmoe_plan_pick(args.plan, mt_dyn, mt_static, segs.ntiles(0, FEAT));
   }
-  auto parts_of = [&](const GemmGroup& gg) {
-    return EPI != G4_PARTIAL ? 1 : gg.row_begin < 0 ? args.plan.pd[plan_idx] : args.plan.ps[plan_idx];
+  auto parts_of = [&](int g) {
+    return EPI != G4_PARTIAL ? 1 : segs.dynamic(g) ? args.plan.pd[plan_idx] : args.plan.ps[plan_idx];
   };
   // Whole rounds of tiles: each XCD (block ids congruent mod 8) takes a contiguous eighth of the tile list and its blocks
   // take consecutive tiles, so the CUs of an XCD share operand tiles in their L2. The remainder (tail): the parts of
@@ -284,10 +259,10 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     v4i e = {0, 0, 0, 0};
     for (int g = 0; g < args.G; ++g) {
       int rb, re;
-      seg(args.g[g], rb, re);
+      segs.get(g, rb, re);
       if (re > rb && lane == g) {
         const G4Heights t = g4_heights(re - rb, cap);
-        e = v4i{0, t.mt * (args.g[g].n_out / FEAT), t.height, t.mt};
+        e = v4i{0, t.mt * segs.ntiles(g, FEAT), t.height, t.mt};
       }
     }
     for (int k = 0; k < args.G; ++k) {
@@ -306,11 +281,11 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
         const v4i t = heights[g];
         const int first = sgpr(t.x), tiles = sgpr(t.y), rows = sgpr(t.z) * 32, mtiles = sgpr(t.w);
         int rb, re, m, n;
-        seg(args.g[g], rb, re);
+        segs.get(g, rb, re);
         if (L < first || L >= first + tiles) continue;
-        g4_raster(L - first, mtiles, args.g[g].n_out / FEAT, m, n);
+        g4_raster(L - first, mtiles, segs.ntiles(g, FEAT), m, n);
         const int row0 = rb + m * rows;
-        e = v4i{g | min(re - row0, rows) << 16, row0, n, args.g[g].kbytes / BK << 16};
+        e = v4i{g | min(re - row0, rows) << 16, row0, n, segs.bytes(g) / BK << 16};
       }
       table[lane] = e;
       return;
@@ -334,26 +309,25 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     int g_at = -1, mtiles = 1, ntiles = 1, L = 0, rb_at = 0, re_at = 0, parts = 1, kt = 0;
     for (int k = 0; k < args.G; ++k) {
       const int g = args.spread < 0 ? args.G - 1 - k : k;
-      const GemmGroup& gg = args.g[g];
       int rb, re;
-      seg(gg, rb, re);
-      const int mt = (re - rb + G4_BM - 1) / G4_BM, nt = gg.n_out / FEAT, np = parts_of(gg);
+      segs.get(g, rb, re);
+      const int mt = (re - rb + G4_BM - 1) / G4_BM, nt = segs.ntiles(g, FEAT), np = parts_of(g);
       const long long tiles = (long long)mt * nt * np;
       const int lo = eighths ? (int)(xcd * tiles / HDMOE_NUM_XCD) : 0;
       const int hi = eighths ? (int)((xcd + 1) * tiles / HDMOE_NUM_XCD) : (int)tiles;
       if (some && g_at < 0) {
-        if (rem < hi - lo) { g_at = g; mtiles = mt; ntiles = nt; L = lo + rem; rb_at = rb; re_at = re; parts = np; kt = gg.kbytes / BK; }
+        if (rem < hi - lo) { g_at = g; mtiles = mt; ntiles = nt; L = lo + rem; rb_at = rb; re_at = re; parts = np; kt = segs.bytes(g) / BK; }
         else rem -= hi - lo;
       }
     }
     v4i e = {-1, 0, 0, 0};
     if (g_at >= 0) {
-      int part = L / (mtiles * ntiles), m, n;
+      int part = EPI == G4_PARTIAL ? tile_div(L, mtiles * ntiles) : 0, m, n;
       g4_raster(L - part * (mtiles * ntiles), mtiles, ntiles, m, n);
       const int row0 = rb_at + m * G4_BM;
       // parts start on a pair of K steps
       const int of = tail_slot > 0 ? tail.parts : parts, at = tail_slot > 0 ? tail_part : part;
-      const int kt0 = kt / 2 * at / of * 2, kt1 = kt / 2 * (at + 1) / of * 2;
+      const int kt0 = at == 0 ? 0 : tile_div(kt / 2 * at, of) * 2, kt1 = at + 1 == of ? kt : tile_div(kt / 2 * (at + 1), of) * 2;
       e = v4i{g_at | part << 8 | min(re_at - row0, G4_BM) << 16, row0, n | tail_slot << 16, kt0 | (kt1 - kt0) << 16};
     }
     table[lane] = e;
@@ -599,7 +573,7 @@ __global__ __launch_bounds__(256) void gemm4w_tail_kernel(const GemmArgs args, i
   constexpr int FEAT = SWIGLU ? 128 : 256;
   using Act = std::conditional_t<F16, HdmoeF16, HdmoeBf16>;
   const int lane = threadIdx.x & 63;
-  const G4Segments seg(args, lane);
+  const Segments seg(args, lane);
   const G4Tail tail = g4_tail_of<TY, FEAT>(args, seg, blocks);
   if (tail.parts <= 1) return;
   constexpr int PER_TILE = SWIGLU ? 16 : 32;   // blocks' worth of work of a tile
@@ -607,8 +581,8 @@ __global__ __launch_bounds__(256) void gemm4w_tail_kernel(const GemmArgs args, i
     const int t = item / PER_TILE;
     int L = __builtin_amdgcn_readfirstlane(tail.rounds * blocks + t), g = 0, m = 0, n = 0, rb = 0, re = 0;
     for (; g < args.G; ++g) {
-      seg.get(args.g[g], rb, re);
-      const int mt = (re - rb + G4_BM - 1) / G4_BM, nt = args.g[g].n_out / FEAT;
+      seg.get(g, rb, re);
+      const int mt = (re - rb + G4_BM - 1) / G4_BM, nt = seg.ntiles(g, FEAT);
       if (L < mt * nt) { g4_raster(L, mt, nt, m, n); break; }
       L -= mt * nt;
     }

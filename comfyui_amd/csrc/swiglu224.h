@@ -1,6 +1,6 @@
 // fp8 gate/up GEMM + SiLU*mul on 224-token tiles, the epilogue of a tile hidden behind the K loop of the next one.
 //
-// Included by gemm.hip inside its unnamed namespace, behind gemm4w.h (uses GemmArgs, GemmGroup, G4Segments, g4_raster, swz, make_rsrc).
+// Included by gemm.hip inside its unnamed namespace, behind gemm4w.h (uses GemmArgs, GemmGroup, Segments, g4_raster, swz, make_rsrc).
 //
 // Same contraction, rounding points and LDS tile format as grouped_gemm_kernel<FP8_SWIGLU, TT>
 // (/root/reference/comfy/ldm/hidream/model.py:238 behind /root/reference/comfy/ops.py:314-358) on the K loop of gemm4w.h's fp8 kernel.
@@ -45,12 +45,12 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   auto own = [](int v) { asm volatile("" : "+s"(v)); return v; };   // as in gemm4w_kernel
 
   // ---- tiles: as gemm4w_kernel's, whole rounds and what is left of them ---------------------------------------
-  const G4Segments segs(args, lane);
+  const Segments segs(args, lane);
   int total = 0;
   for (int g = 0; g < args.G; ++g) {
     int rb, re;
-    segs.get(args.g[g], rb, re);
-    total += (re - rb + S224_BM - 1) / S224_BM * (args.g[g].n_out / S224_FEAT);
+    segs.get(g, rb, re);
+    total += (re - rb + S224_BM - 1) / S224_BM * segs.ntiles(g, S224_FEAT);
   }
   const int xcd = blockIdx.x % HDMOE_NUM_XCD, slot = blockIdx.x / HDMOE_NUM_XCD;
   const int nslots = gridDim.x / HDMOE_NUM_XCD;
@@ -64,8 +64,8 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     int g_at = -1, mtiles = 1, ntiles = 1, L = 0, rb_at = 0, re_at = 0;
     for (int g = 0; g < args.G; ++g) {
       int rb, re;
-      segs.get(args.g[g], rb, re);
-      const int mt = (re - rb + S224_BM - 1) / S224_BM, nt = args.g[g].n_out / S224_FEAT;
+      segs.get(g, rb, re);
+      const int mt = (re - rb + S224_BM - 1) / S224_BM, nt = segs.ntiles(g, S224_FEAT);
       if (some && g_at < 0) {
         if (rem < mt * nt) { g_at = g; mtiles = mt; ntiles = nt; L = rem; rb_at = rb; re_at = re; }
         else rem -= mt * nt;
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   int ld_chunk = f8_chunk((lane & 7) ^ swz(ld_row));
   const int ldsw = sgpr((int)lds0 + wave * 1024);
   const int fr_row = lane & 15, fr_grp = lane >> 4, fr_swz = swz(fr_row);
-  const int kb = args.g[0].kbytes;
+  const int kb = segs.bytes(0);
   const int kb8 = sgpr(8 * kb), kb64 = sgpr(64 * kb), pairs = sgpr(kb / (2 * BK));
 
   v32i fa0, fb0, ctx, d0, d2;   // fragments of the tile about to start; addresses; deferred pieces

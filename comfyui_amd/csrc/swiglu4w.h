@@ -47,17 +47,12 @@ __global__ __launch_bounds__(W4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   auto sgpr = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
 
   // ---- tile enumeration: as grouped_gemm_kernel with one tile list cut in eighths ---------------------------
-  int off_lane = 0;
-  if (args.offsets != nullptr && lane <= args.n_offsets) off_lane = args.offsets[lane];
-  auto seg = [&](const GemmGroup& gg, int& rb, int& re) {
-    if (gg.row_begin >= 0) { rb = gg.row_begin; re = gg.row_end; }
-    else { rb = __builtin_amdgcn_readlane(off_lane, gg.dyn); re = __builtin_amdgcn_readlane(off_lane, gg.dyn + 1); }
-  };
+  const Segments segs(args, lane);
   int total = 0;
   for (int g = 0; g < args.G; ++g) {
     int rb, re;
-    seg(args.g[g], rb, re);
-    total += ((re - rb + W4_BM - 1) / W4_BM) * (args.g[g].n_out / W4_FEAT);
+    segs.get(g, rb, re);
+    total += ((re - rb + W4_BM - 1) / W4_BM) * segs.ntiles(g, W4_FEAT);
   }
   const int per_xcd = (total + HDMOE_NUM_XCD - 1) / HDMOE_NUM_XCD;
   const int xcd = blockIdx.x % HDMOE_NUM_XCD, slot = blockIdx.x / HDMOE_NUM_XCD;
@@ -70,22 +65,23 @@ __global__ __launch_bounds__(W4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     if (in_xcd >= per_xcd || L >= total) return d;
     int g = 0, rb = 0, re = 0, mtiles = 0, ntiles = 0;
     for (; g < args.G; ++g) {
-      seg(args.g[g], rb, re);
+      segs.get(g, rb, re);
       mtiles = (re - rb + W4_BM - 1) / W4_BM;
-      ntiles = args.g[g].n_out / W4_FEAT;
+      ntiles = segs.ntiles(g, W4_FEAT);
       if (L < mtiles * ntiles) break;
       L -= mtiles * ntiles;
     }
     if (g >= args.G) return d;
     const int nbands = max(1, (mtiles + GROUP_M / 2) / GROUP_M);
-    const int band = min(L / (GROUP_M * ntiles), nbands - 1);
+    const int band = min(tile_div(L, GROUP_M * ntiles), nbands - 1);
     const int first_m = band * GROUP_M;
     const int gm = band == nbands - 1 ? mtiles - first_m : GROUP_M;
     const int within = L - band * (GROUP_M * ntiles);
+    const int n = tile_div(within, gm);
     d.g = g;
-    d.row0 = rb + (first_m + within % gm) * W4_BM;
+    d.row0 = rb + (first_m + within - n * gm) * W4_BM;
     d.rows_here = min(re - d.row0, W4_BM);
-    d.n0 = (within / gm) * W4_FEAT;
+    d.n0 = n * W4_FEAT;
     return d;
   };
 
