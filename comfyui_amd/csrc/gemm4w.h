@@ -397,6 +397,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   // the operands of an item's loads: resources of tokens and weights, the lane's row offsets (gi: its row indices where the
   // group gathers its tokens); rows past the end of the tile get an offset beyond the buffer and read as zeros
   struct Source { Rsrc a, b0, b1; };
+  auto weight_voff = [&](int j, int wkb) { return ((SWIGLU ? (j >> 2) * 64 + (j & 1) * 32 : j * 32) + ld_wrow) * wkb + ld_chunk * 16; };
   auto set_source = [&](const Item& d, const v8i& rows, v16i& voff) -> Source {
     Source s = {{0, 0}, {0, 0}, {0, 0}};
     if (!d.some()) return s;   // no further item: the requests still go out, against empty buffers (zeros)
@@ -413,7 +414,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
       const int r = j * 32 + ld_row;
       const int row = by_list ? rows[j] >> shift : r;
       voff[j] = r < d.rows_here() ? row * kb + ld_chunk * 16 : (int)0x80000000u;
-      voff[8 + j] = ((SWIGLU ? (j >> 2) * 64 + (j & 1) * 32 : j * 32) + ld_wrow) * wkb + ld_chunk * 16;
+      voff[8 + j] = weight_voff(j, wkb);
     }
     return s;
   };
@@ -429,33 +430,42 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   };
   auto w_start = [](const Item& d) { return W8 ? d.kt0() * (BK / 2) : d.kt0() * BK; };
 
-  Source src = set_source(cur, load_rows(cur), voff_nxt);
-#pragma unroll
-  for (int j = 0; j < 16; ++j) ctx[G4_TOK_VOFF + j] = voff_nxt[j];
   // ---- the block's first two K steps (w8: weights of two pairs) as a burst --------------------------------------
+  // The first step's weights go out while the row indices are on their way, and the second step may still be when the first one starts (its
+  // wait is step 0's own; w8: that one lets the last 8 requests be out, which are weights there as everywhere).
+  Source src;
   {
     const GemmGroup& gg = args.g[cur.g()];
     const int kb = gg.kbytes, wkb = W8 ? kb >> 1 : kb;
+    const v8i rows = load_rows(cur);
+    gi = nxt.some() ? load_rows(nxt) : v8i{0, 0, 0, 0, 0, 0, 0, 0};
+    asm volatile("" : : : "memory");   // (the wait below counts the requests behind the first step's: none may change places with them)
+    const __amdgpu_buffer_rsrc_t pb0 = make_rsrc(gg.b0 + (size_t)cur.n0() * wkb, (uint32_t)FEAT * (uint32_t)wkb);
+    const __amdgpu_buffer_rsrc_t pb1 = SWIGLU ? make_rsrc(gg.b1 + (size_t)cur.n0() * wkb, (uint32_t)FEAT * (uint32_t)wkb) : pb0;
+    uint8_t* const base = smem + wave * 1024;
+    auto weights = [&](int st) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds((j >> 1) & 1 ? pb1 : pb0, (lds_ptr_t)(base + st * G4_STAGE + G4_W_TILE + j * 4096), 16,
+                                                 weight_voff(j, wkb), w_start(cur) + st * BK, 0, 0);
+    };
+    weights(0);
+    src = set_source(cur, rows, voff_nxt);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) ctx[G4_TOK_VOFF + j] = voff_nxt[j];
     const __amdgpu_buffer_rsrc_t pa = gg.gather != nullptr
         ? make_rsrc(gg.a, (uint32_t)gg.a_rows * (uint32_t)kb)
         : make_rsrc(gg.a + (size_t)cur.row0() * kb, (uint32_t)cur.rows_here() * (uint32_t)kb);
-    const __amdgpu_buffer_rsrc_t pb0 = make_rsrc(gg.b0 + (size_t)cur.n0() * wkb, (uint32_t)FEAT * (uint32_t)wkb);
-    const __amdgpu_buffer_rsrc_t pb1 = SWIGLU ? make_rsrc(gg.b1 + (size_t)cur.n0() * wkb, (uint32_t)FEAT * (uint32_t)wkb) : pb0;
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
-      uint8_t* const base = smem + st * G4_STAGE + wave * 1024;
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(pa, (lds_ptr_t)(base + j * 4096), 16, ctx[G4_TOK_VOFF + j], (cur.kt0() + st) * BK, 0, 0);
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds((j >> 1) & 1 ? pb1 : pb0, (lds_ptr_t)(base + G4_W_TILE + j * 4096), 16,
-                                                 ctx[G4_W_VOFF + j], w_start(cur) + st * BK, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(pa, (lds_ptr_t)(base + st * G4_STAGE + j * 4096), 16, ctx[G4_TOK_VOFF + j], (cur.kt0() + st) * BK, 0, 0);
+      asm volatile("" : : : "memory");
     }
+    weights(1);
   }
-  gi = nxt.some() ? load_rows(nxt) : v8i{0, 0, 0, 0, 0, 0, 0, 0};
-  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-  __syncthreads();
+  asm volatile("s_waitcnt vmcnt(16)\n\ts_barrier" : : : "memory");
   if constexpr (W8) asm volatile(HDMOE_G4_FILL_W8 : "={v[128:159]}"(fa0), "={v[160:191]}"(fb0), "+{v[96:127]}"(ctx) : : G4_CLOBBER_V);
   else if constexpr (F8) asm volatile(HDMOE_G4_FILL_F8 : "={v[128:159]}"(fa0), "={v[160:191]}"(fb0), "+{v[96:127]}"(ctx) : : "memory");
   else asm volatile(HDMOE_G4_FILL : "={v[128:159]}"(fa0), "={v[160:191]}"(fb0), "+{v[96:127]}"(ctx) : : "memory");

@@ -176,30 +176,39 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     return r;
   };
 
+  // ---- the block's first two K steps as a burst, as in gemm4w_kernel --------------------------------------------
   v8i voff;
-  Source src = set_source(cur, load_rows(cur), voff);
-#pragma unroll
-  for (int j = 0; j < S224_TT; ++j) ctx[S224_TOK_VOFF + j] = voff[j];
-  // ---- the block's first two K steps as a burst -----------------------------------------------------------------
+  Source src;
   {
     auto buffer = [](uint64_t lo, uint32_t bytes) { return make_rsrc(reinterpret_cast<const void*>(lo), bytes); };
-    const __amdgpu_buffer_rsrc_t pa = buffer(src.a, (uint32_t)src.ah);
-    const __amdgpu_buffer_rsrc_t pb0 = buffer(src.b, (uint32_t)S224_FEAT * (uint32_t)kb), pb1 = buffer(src.c, (uint32_t)S224_FEAT * (uint32_t)kb);
-#pragma unroll
-    for (int st = 0; st < 2; ++st) {
-      uint8_t* const base = smem + st * G4_STAGE + wave * 1024;
-#pragma unroll
-      for (int j = 0; j < S224_TT; ++j)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(pa, (lds_ptr_t)(base + j * 4096), 16, ctx[S224_TOK_VOFF + j], st * BK, 0, 0);
+    const GemmGroup& gg = args.g[cur.g()];
+    const v8i rows = load_rows(cur);
+    gi = nxt.some() ? load_rows(nxt) : v8i{0, 0, 0, 0, 0, 0, 0, 0};
+    asm volatile("" : : : "memory");   // (the wait below counts the requests behind the first step's: none may change places with them)
+    const __amdgpu_buffer_rsrc_t pb0 = make_rsrc(gg.b0 + (size_t)cur.n0() * kb, (uint32_t)S224_FEAT * (uint32_t)kb);
+    const __amdgpu_buffer_rsrc_t pb1 = make_rsrc(gg.b1 + (size_t)cur.n0() * kb, (uint32_t)S224_FEAT * (uint32_t)kb);
+    uint8_t* const base = smem + wave * 1024;
+    auto weights = [&](int st) {
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds((j >> 1) & 1 ? pb1 : pb0, (lds_ptr_t)(base + G4_W_TILE + j * 4096), 16, ctx[S224_W_VOFF],
+        __builtin_amdgcn_raw_ptr_buffer_load_lds((j >> 1) & 1 ? pb1 : pb0, (lds_ptr_t)(base + st * G4_STAGE + G4_W_TILE + j * 4096), 16, ctx[S224_W_VOFF],
                                                  st * BK + (j >> 2) * kb64 + (j & 1) * kb8, 0, 0);
+    };
+    weights(0);
+    src = set_source(cur, rows, voff);
+#pragma unroll
+    for (int j = 0; j < S224_TT; ++j) ctx[S224_TOK_VOFF + j] = voff[j];
+    const __amdgpu_buffer_rsrc_t pa = buffer(src.a, (uint32_t)src.ah);
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+#pragma unroll
+      for (int j = 0; j < S224_TT; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(pa, (lds_ptr_t)(base + st * G4_STAGE + j * 4096), 16, ctx[S224_TOK_VOFF + j], st * BK, 0, 0);
+      asm volatile("" : : : "memory");
     }
+    weights(1);
   }
-  gi = nxt.some() ? load_rows(nxt) : v8i{0, 0, 0, 0, 0, 0, 0, 0};
-  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-  __syncthreads();
+  asm volatile("s_waitcnt vmcnt(15)\n\ts_barrier" : : : "memory");
   asm volatile(HDMOE_S224_FILL : "={v[128:159]}"(fa0), "={a[224:255]}"(fb0), "+{v[96:127]}"(ctx) : : "memory");
 
   // per-tensor scales come through the scalar cache (gemm4w_kernel)
