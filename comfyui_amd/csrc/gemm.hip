@@ -1222,7 +1222,7 @@ int launch_gemm4w(GemmArgs& args, int rows_mean, hipStream_t s, const char* what
                      has_static ? last.row_end - last.row_begin : 0, last.n_out, last.kbytes, FEAT, TY == G4_W8) == 0)
       args.tail = nullptr;
   }
-  args.cap = TY == G4_F8 ? 0 : g4_host_cap(args, FEAT, TY == G4_W8 ? 3 : 2, HDMOE_NUM_CU);
+  args.cap = g4_host_cap(args, FEAT, TY == G4_W8 ? 3 : 2, HDMOE_NUM_CU);
   // one block per CU whatever the number of tiles: a block without any ends at once
   hipLaunchKernelGGL((gemm4w_kernel<TY, EPI>), dim3(HDMOE_NUM_CU), dim3(G4_THREADS), G4_SMEM, s, args);
   if constexpr (EPI != G4_PARTIAL && TY != G4_F8) {
@@ -1671,11 +1671,8 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
                 : launch_grouped<BF16_PLAIN>(args, tile_bound, s, what);
 }
 
-// An fp8 Linear with a bias: the 192-token tile of the 8-wave kernel, where its rounds of tiles cost a tenth less than those of 256 tokens
-// (as expected_tile_cost counts them: rounds x (TT + 1)).
-// With the cast in front, 4-wave kernel on 256-token tiles against this, us, rows by K x N: 4480 by 2560 x 2560 39.4, 38.6 (180 and 240
-// tiles on 256 CUs); 193 by 4096 x 2560 41.2, 36.4 (fewer products of padding); 1000 by 2560 x 2560 34.4, 28.8; 300 by 2560 x 10240 32.0,
-// 27.4, 2000 63.8, 60.2; 9000 by 2048 x 2048 58.6, 54.1, by 4096 x 2560 103.6, 99.9; at the line 4480 by 4096 x 2560 53.5, 53.8.
+// An fp8 Linear with a bias that the 4-wave kernel does not take (K no multiple of 256): the 192-token tile of the 8-wave kernel, where its
+// rounds of tiles cost a tenth less than those of 256 tokens (as expected_tile_cost counts them: rounds x (TT + 1)).
 static bool fp8_linear_192(int rows, int N) {
   auto cost = [&](int tt) { return (long)(((rows + 64 * tt - 1) / (64 * tt) * (N / BN) + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU) * (tt + 1); };
   return 10 * cost(3) <= 9 * cost(4);
@@ -1720,8 +1717,8 @@ extern "C" const char* hdmoe_plain_kernel_name(int rows_dyn, int E, int K_dyn, i
   if (bad(n_dyn, K_dyn) || bad(rows_static, K_static) || (n_dyn == 0 && rows_static == 0)) return "";
   const bool takes = g4_takes_k(n_dyn > 0 ? rows_dyn : 0, K_dyn, rows_static, K_static);
   if (has_bias != 0) {
-    if (fp8_linear_192(rows_static, N)) return "grouped_gemm_kernel<FP8_PLAIN_BIAS, 3>";
-    return takes ? "gemm4w_kernel<F8, BIAS>" : "grouped_gemm_kernel<FP8_PLAIN_BIAS, 4>";
+    if (takes) return "gemm4w_kernel<F8, BIAS>";
+    return fp8_linear_192(rows_static, N) ? "grouped_gemm_kernel<FP8_PLAIN_BIAS, 3>" : "grouped_gemm_kernel<FP8_PLAIN_BIAS, 4>";
   }
   GemmShape sh;
   sh.swiglu = false; sh.fp8 = true; sh.split = parts > 1; sh.w8 = false; sh.w4_fits = sh.s224_fits = false;
@@ -1990,10 +1987,8 @@ int hdmoe_launch_linear_bias(int weight_dtype, const uint8_t* a, int rows, int K
   gg.act = HDMOE_ACT_NONE;
   args.G = 1;
   auto tiles = [&](int tt) { return (rows + 64 * tt - 1) / (64 * tt) * (N / BN); };
-  if (fp8_linear_192(rows, N)) return launch_grouped<FP8_PLAIN_BIAS, 3>(args, tiles(3), s, what);
-  // Else the 4-wave kernel. Without the cast, 8- against 4-wave on 256-token tiles: 8192 by 2560 x 10240 169.8, 157.7; 3000 67.8, 65.7;
-  // 1300 36.2, 35.3; 5000 by 6912 x 2560 72.6, 68.5; 5000 by 2560 x 2560 33.8, 33.8.
   if (gemm4w_fits(args, false)) return launch_gemm4w<G4_F8, G4_BIAS>(args, rows, s, what);
+  if (fp8_linear_192(rows, N)) return launch_grouped<FP8_PLAIN_BIAS, 3>(args, tiles(3), s, what);
   return launch_grouped<FP8_PLAIN_BIAS>(args, tiles(4), s, what);
 }
 

@@ -129,7 +129,9 @@ __device__ __forceinline__ G4Tail g4_tail_of(const GemmArgs& args, const Segment
 // twelfth: the model takes a round with idle CUs for as long as a full one, but it has the higher clock. Whole tiles -> this: Linears in bf16,
 // 700 x 2560 x 10240 48.8 -> 38.8 us (240 tiles of 4 blocks for 120), 1700 x 2560 x 2560 48.1 -> 38.1, 3300 x 2560 x 2560 49.2 -> 43.0; with
 // e4m3fn weights 50.0 -> 37.4, 49.0 -> 36.8, 50.1 -> 42.3; Hunyuan3D block of 1250 tokens 367 -> 330, 1500 358 -> 348 (375 rows per expert:
-// 3 rounds of 8 or of 6 to 7 blocks). Not for SWIGLU, whose two halves of the weights every further m-tile reads again: 1300 tokens
+// 3 rounds of 8 or of 6 to 7 blocks); in fp8, 8-wave kernel on 192-token tiles -> this, without the cast: 4480 x 2560 x 2560 31.6 -> 28.7, 2000 25.8 ->
+// 21.8, 1000 22.0 -> 19.0, 2000 x 2560 x 10240 52.7 -> 46.9, 9000 x 2048 x 2048 44.0 -> 36.2, 193 x 4096 x 2560 28.4 -> 23.4; fp8 tiles are as
+// high as their rows need without a cap too. Not for SWIGLU, whose two halves of the weights every further m-tile reads again: 1300 tokens
 // in bf16 361 -> 367 us, 1024 tokens 294 -> 298. More than 24 rounds: one is not worth the search.
 constexpr int G4_TILE_COST = 150, G4_CAP_ROUNDS = 24;
 struct G4Heights { int mt, height; };
@@ -181,10 +183,10 @@ __host__ __device__ __forceinline__ int g4_best_cap(int whole, int pairs, const 
 }
 
 // On the device lane i works out cap 4 + i.
-template <G4Type TY, int FEAT>
+template <int FEAT>
 __device__ __forceinline__ int g4_cap(const GemmArgs& args, const Segments& seg, const G4Tail& tail, int blocks, int lane) {
   const int whole = g4_cap_rounds(tail);
-  if (TY == G4_F8 || whole == 0) return 0;
+  if (whole == 0) return 0;
   const int mine = g4_cap_cost(args.G, seg.bytes(0) / (2 * BK), [&](int g) { return seg.rows(g); }, [&](int g) { return seg.ntiles(g, FEAT); }, blocks,
                                G4_MIN_BLOCKS + min(lane, 4));
   return g4_best_cap(whole, seg.bytes(0) / (2 * BK), [&](int cap) { return __builtin_amdgcn_readlane(mine, cap - G4_MIN_BLOCKS); });
@@ -250,9 +252,9 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   // one K range before those of the next, again consecutive inside an XCD. Groups of different K (`spread`) or cut by the
   // caller's plan: every XCD takes its eighth of every group, longest tiles first.
   const int xcd = blockIdx.x % HDMOE_NUM_XCD, slot = blockIdx.x / HDMOE_NUM_XCD;
-  const int nslots = gridDim.x / HDMOE_NUM_XCD;
-  const G4Tail tail = g4_tail_of<TY, FEAT>(args, segs, gridDim.x);
-  const int cap = EPI == G4_PARTIAL || SWIGLU || args.spread != 0 ? 0 : args.cap >= 0 ? args.cap : sgpr(g4_cap<TY, FEAT>(args, segs, tail, gridDim.x, lane));
+  constexpr int nslots = HDMOE_NUM_CU / HDMOE_NUM_XCD;   // the grid is one block per CU
+  const G4Tail tail = g4_tail_of<TY, FEAT>(args, segs, HDMOE_NUM_CU);
+  const int cap = EPI == G4_PARTIAL || SWIGLU || args.spread != 0 ? 0 : args.cap >= 0 ? args.cap : sgpr(g4_cap<FEAT>(args, segs, tail, HDMOE_NUM_CU, lane));
   // cap > 0: lane g looks up where group g comes in the order of heights: [first tile, tiles, height, m-tiles]
   v4i* const heights = reinterpret_cast<v4i*>(smem + G4_HEIGHTS);
   if (cap > 0) {
@@ -275,7 +277,12 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   auto fill_table = [&](int base) {
     const int i = base + lane;
     if (cap > 0) {
-      const int L = i * (int)gridDim.x + xcd * nslots + slot;
+      // a last round of a few tiles is spread over the XCDs (consecutive blocks of it on the first ones: a Linear of 80 tiles 34.2 us, so 30.2)
+      int total = 0;
+      for (int g = 0; g < args.G; ++g) total += sgpr(heights[g].y);
+      const int full = total / HDMOE_NUM_CU, left = total % HDMOE_NUM_CU, share = (left + HDMOE_NUM_XCD - 1) / HDMOE_NUM_XCD;
+      const int L = i < full ? i * HDMOE_NUM_CU + xcd * nslots + slot
+                             : i == full && slot < share && xcd * share + slot < left ? full * HDMOE_NUM_CU + xcd * share + slot : -1;
       v4i e = {-1, 0, 0, 0};
       for (int g = 0; g < args.G; ++g) {
         const v4i t = heights[g];
@@ -300,9 +307,9 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
         const int units = tail.tiles * tail.parts, chunk = (units + HDMOE_NUM_XCD - 1) / HDMOE_NUM_XCD;
         const int w = xcd * chunk + slot;
         some = i == tail.rounds && slot < chunk && w < units;
-        const int t = some ? w % tail.tiles : 0;
-        tail_part = some ? w / tail.tiles : 0;
-        rem = tail.rounds * (int)gridDim.x + t;
+        tail_part = some ? tile_div(w, tail.tiles) : 0;
+        const int t = some ? w - tail_part * tail.tiles : 0;
+        rem = tail.rounds * HDMOE_NUM_CU + t;
         tail_slot = tail.parts > 1 ? 1 + t * tail.parts + tail_part : 0;
       }
     }
@@ -517,7 +524,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     ctx[G4_OUT_VOFF] = part ? wave * 8192 + lane * 16
                             : (wt * 16 + fr_row) * ldo + (cur.n0() + wq * (FEAT / 2) + fr_grp * 8) * OUT_BYTES;
     const int part_s = part ? sgpr(g4_part_blocks(cur.rows_here(), wave)) + 1 : 0;
-    const int nt = sgpr(cap > 0 ? max((cur.rows_here() + 31) >> 5, G4_MIN_BLOCKS) : G4_BM / 32);   // token blocks
+    const int nt = sgpr(F8 || cap > 0 ? max((cur.rows_here() + 31) >> 5, G4_MIN_BLOCKS) : G4_BM / 32);   // token blocks
     // row indices of nx2 and this tile's biases are loaded inside the statement
     const int32_t* const list = nx2.some() ? args.g[nx2.g()].gather : nullptr;
     const v4i gr = rsrc4(list != nullptr ? list + nx2.row0() : nullptr, list != nullptr ? (uint32_t)nx2.rows_here() * 4u : 0u);

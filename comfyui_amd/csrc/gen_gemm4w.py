@@ -69,7 +69,7 @@ class At:
     """Positions (MFMA index within a slice of `m`) of the events of a step of `nt` token blocks. last: of the pair that ends a
     tile, which fetches 8 token blocks whatever nt is."""
     def __init__(self, nt, last=False):
-        self.nt, self.m = nt, 8 * nt
+        self.nt, self.m, self.last = nt, 8 * nt, last
         self.loads = 8 if last else nt          # token loads of a step
         self.free = 16 + nt                     # slice 0: the stage has been read (8 + nt reads, one per MFMA); barrier
         self.load = self.free + 1               # first load of the step after the next, and MFMAs between two loads
@@ -79,11 +79,19 @@ class At:
         self.st, self.ld = self.m - 7, self.m - 4   # GELU, slice 0: piece stored, piece read back
 
 
-# the same for the fp8 step (64 MFMAs)
-FREE8_AT = 16
-LOAD8_AT = 18
-LOAD8_EVERY = 3
-LAND8_AT = 44
+class At8:
+    """The same for an fp8 step of `nt` token blocks, 8 nt MFMAs in quadrants: weights 0-3 / 4-7 by the token blocks `halves`."""
+    def __init__(self, nt, stage, last=False):
+        self.m = 8 * nt
+        h = (nt + 1) // 2
+        self.halves = (range(h), range(h, nt)) if stage == 0 else (range(h, nt), range(h))
+        first, second = (len(t) for t in self.halves)
+        self.loads = 8 if last else nt
+        self.free = 4 * first                       # the stage has been read; barrier
+        self.land = 4 * first + 8 * second - 4      # the next stage has landed; barrier, then the reads of the next step's first quadrant
+        n, lo = self.loads + 8, self.free + 2
+        self.load_at = [lo + 3 * j if nt == 8 else lo + j * (self.m - lo) // n for j in range(n)]
+        assert self.load_at[-1] < self.m and len(set(self.load_at)) == n
 
 
 def quad(b):
@@ -325,17 +333,16 @@ def reads8(stage, frags):
     return out
 
 
-def burst8(stage):
+def burst8(stage, nt=8):
     """The reads that a step out of `stage` starts from, and those it issues itself for its second half."""
-    t0, t1 = (range(4), range(4, 8)) if stage == 0 else (range(4, 8), range(4))
-    t0, t1 = [("a", t) for t in t0], [("a", t) for t in t1]
+    t0, t1 = ([("a", t) for t in h] for h in At8(nt, stage).halves)
     w0, w1 = [("b", f) for f in range(4)], [("b", f) for f in range(4, 8)]
-    return reads8(stage, [w0[0], t0[0]] + w0[1:] + t0[1:]), reads8(stage, [t1[0], w1[0], t1[1], t1[2], t1[3]] + w1[1:])
+    return reads8(stage, [w0[0], t0[0]] + w0[1:] + t0[1:]), reads8(stage, [t1[0], w1[0]] + t1[1:] + w1[1:])
 
 
-def mfma_order8(stage):
-    """Four quadrants of 4 x 4 MFMA tiles: (w0, t0), (w0, t1), (w1, t1), (w1, t0), t0 and t1 by step parity; token blocks outermost."""
-    t0, t1 = (range(4), range(4, 8)) if stage == 0 else (range(4, 8), range(4))
+def mfma_order8(nt, stage):
+    """Four quadrants of MFMA tiles: (w0, t0), (w0, t1), (w1, t1), (w1, t0), t0 and t1 by step parity; token blocks outermost."""
+    t0, t1 = At8(nt, stage).halves
     o = []
     for fts, tts in ((range(4), t0), (range(4), t1), (range(4, 8), t1), (range(4, 8), t0)):
         for k, tt in enumerate(tts):
@@ -343,22 +350,28 @@ def mfma_order8(stage):
     return o
 
 
-def young8(stage):
-    """As young(): the requests that may still be out when the next step's operands are there, those of this step."""
-    return sum(LOAD8_AT + j * LOAD8_EVERY < LAND8_AT for j in range(16))
-
-
-def step8(stage, first):
-    """One fp8 K step out of `stage`: 128 bytes are one MFMA deep, so a step has no second slice to read ahead; its 64 MFMAs go in
+def step8(stage, first, nt, last):
+    """One fp8 K step out of `stage`: 128 bytes are one MFMA deep, so a step has no second slice to read ahead; its 8 nt MFMAs go in
     quadrants instead, and the fragments of quadrants that are done are refilled from the next stage. Entry: the reads of
-    the first quadrant are in flight (burst8)."""
+    the first quadrant are in flight (burst8; of a tile's first step always those of 4 token blocks, whatever its height). last: of the pair
+    that ends a tile."""
     L = []
-    order = mfma_order8(stage)
-    own, nxt = burst8(stage)[1], burst8(stage ^ 1)[0]
-    ld = token_loads(stage) + weight_loads(stage, False)
-    events = {LOAD8_AT + j * LOAD8_EVERY: ld[j] for j in range(16)}
-    assert FREE8_AT <= LOAD8_AT and max(events) < 64
-    for q in range(64):
+    at = At8(nt, stage, last)
+    order = mfma_order8(nt, stage)
+    used = {}                                   # the last MFMA that reads a fragment
+    for q, (ft, tt) in enumerate(order):
+        used[("b", ft)] = used[("a", tt)] = q
+    own = burst8(stage, nt)[1]
+    nxt = burst8(stage ^ 1, nt)[0]
+    ends = last and stage == 1
+    if ends:                                    # token blocks 0-3, those that the last quadrant uses behind their last use
+        nxt = burst8(0)[0]
+    todo = [nxt[i:i + 2] for i in range(0, len(nxt), 2)]
+    reg = {quad(frag8(k, i)): (k, i) for k in "ab" for i in range(8)}
+    ld = token_loads(stage, at.loads) + weight_loads(stage, False)
+    events = dict(zip(at.load_at, ld))
+    assert len(own) // 2 <= at.free
+    for q in range(at.m):
         ft, tt = order[q]
         if q == 0:
             L.append("s_waitcnt lgkmcnt(0)")
@@ -372,19 +385,21 @@ def step8(stage, first):
             L.append(now[1])
         if q < 8:
             L += own[2 * q:2 * q + 2]
-        if q == FREE8_AT - 1:
+        if q == at.free - 1:
             L += ["s_waitcnt lgkmcnt(0)", "s_barrier"]
-        if q == LAND8_AT - 1:
-            L += [f"s_waitcnt vmcnt({young8(stage)})", "s_barrier"]
-        if 0 <= q - LAND8_AT < 8:   # they overwrite fragments of the quadrants behind; those of the third are freed four MFMAs apart
-            L += nxt[2 * (q - LAND8_AT):2 * (q - LAND8_AT) + 2]
+        if q == at.land - 1:   # the requests that may still be out are those of this step
+            L += [f"s_waitcnt vmcnt({sum(p < at.land for p in at.load_at)})", "s_barrier"]
+        # they overwrite fragments of the quadrants behind; those of the third are freed four MFMAs apart
+        if q >= at.land and todo and used.get(reg[todo[0][0].split(" ", 1)[1].split(",")[0]], -1) <= q:
+            L += todo.pop(0)
+    assert not todo
     L.append("s_add_u32 %[so], %[so], 128")
     return L
 
 
 def pair(dt, w8, gelu, first, at):
     if dt == "F8":
-        return step8(0, first) + step8(1, first)
+        return step8(0, first, at.nt, at.last) + step8(1, first, at.nt, at.last)
     L = []
     if gelu and not first:
         # pieces 2p, 2p + 1: the pair of K steps p (0..13) reads them back, pair p + 1 stores them (64 bytes per token each)
@@ -513,10 +528,10 @@ def swiglu_epilogue(w8):
     return L
 
 
-def partial_epilogue():
+def partial_epilogue(nt=8):
     """The raw fp32 sums, straight from the accumulators: 16 bytes (4 features) per lane and store."""
     L = []
-    for tt in range(8):
+    for tt in range(nt):
         L += out_row(tt)
         for ft in range(8):
             b = (8 * ft + tt) * 4
@@ -560,13 +575,15 @@ def gelu_drain(dt):
 
 
 def tile(dt, w8, gelu, bias, epi, heights=HEIGHTS):
-    """A tile of any height: the text of its number of token blocks, %[nt]. Raw sums where it is a part of a tile, which has 8 (%[part])."""
+    """A tile of any height: the text of its number of token blocks, %[nt]. 16 bits: raw sums where it is a part of a tile, which has 8
+    (%[part])."""
     texts = []
     for nt in heights:
+        parts = nt == 8 and dt != "F8"
         L = [f"{100 + nt}:"] + k_loop(dt, w8, gelu, bias, nt)
-        L += ["s_cmp_lg_u32 %[part], 0", "s_cbranch_scc1 41f"] if nt == 8 else []
+        L += ["s_cmp_lg_u32 %[part], 0", "s_cbranch_scc1 41f"] if parts else []
         L += epi(nt)
-        L += ["s_branch 199f", "41:"] + part_epilogue() if nt == 8 else []
+        L += ["s_branch 199f", "41:"] + part_epilogue() if parts else []
         texts += L + ["s_branch 199f"]
     jumps = []
     for nt in heights[1:]:
@@ -598,8 +615,8 @@ def generate():
     for dt in ("BF16", "F16"):
         texts.append((f"HDMOE_G4_DRAIN_{dt}", DRAIN_WAIT + gelu_drain(dt)))
     for bias in (False, True):
-        texts.append((f"HDMOE_G4_TILE_F8{'_BIAS' if bias else ''}", k_loop("F8", False, False, bias) + epilogue("F8", False, bias, False)))
-    texts.append(("HDMOE_G4_TILE_F8_PARTIAL", k_loop("F8", False, False, False) + partial_epilogue()))
+        texts.append((f"HDMOE_G4_TILE_F8{'_BIAS' if bias else ''}", tile("F8", False, False, bias, lambda nt: epilogue("F8", False, bias, False, nt))))
+    texts.append(("HDMOE_G4_TILE_F8_PARTIAL", tile("F8", False, False, False, partial_epilogue)))
     texts.append(("HDMOE_G4_FILL_F8", burst8(0)[0]))
     for name, lines in texts:
         check_trans(lines)

@@ -53,14 +53,14 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     total += (re - rb + S224_BM - 1) / S224_BM * segs.ntiles(g, S224_FEAT);
   }
   const int xcd = blockIdx.x % HDMOE_NUM_XCD, slot = blockIdx.x / HDMOE_NUM_XCD;
-  const int nslots = gridDim.x / HDMOE_NUM_XCD;
-  const int rounds = total / (int)gridDim.x, left = total % (int)gridDim.x, chunk = (left + HDMOE_NUM_XCD - 1) / HDMOE_NUM_XCD;
+  constexpr int nslots = HDMOE_NUM_CU / HDMOE_NUM_XCD;   // the grid is one block per CU
+  const int rounds = total / HDMOE_NUM_CU, left = total % HDMOE_NUM_CU, chunk = (left + HDMOE_NUM_XCD - 1) / HDMOE_NUM_XCD;
   v4i* const table = reinterpret_cast<v4i*>(smem + S224_TABLE) + wave * G4_TABLE_ITEMS;
   auto fill_table = [&](int base) {
     const int i = base + lane;
     const int w = xcd * chunk + slot;
     const bool some = i < rounds || (i == rounds && slot < chunk && w < left);
-    int rem = i < rounds ? xcd * (rounds * nslots) + slot + i * nslots : rounds * (int)gridDim.x + w;
+    int rem = i < rounds ? xcd * (rounds * nslots) + slot + i * nslots : rounds * HDMOE_NUM_CU + w;
     int g_at = -1, mtiles = 1, ntiles = 1, L = 0, rb_at = 0, re_at = 0;
     for (int g = 0; g < args.G; ++g) {
       int rb, re;

@@ -1,0 +1,47 @@
+"""fp8 contractions on tiles of fewer than 256 tokens (csrc/gen_gemm4w.py, step8): every height, behind each other in a block, few and many
+K steps, against 64-bit arithmetic on the same operands (the bound of test_gpu_gemm4w_fp8.py), and a row's bytes in tiles of other heights."""
+import pytest
+import torch
+
+from comfyui_amd import _lib
+from tests.test_gpu_gemm4w_fp8 import check, operands
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+# 10 or 40 n-tiles; the heights that the cost model picks (csrc/gemm4w.h, g4_best_cap) and the last tile's are 4 to 8 blocks of 32
+@pytest.mark.parametrize("with_bias", [False, True])
+@pytest.mark.parametrize("rows,k,n", [(1, 512, 2560), (128, 768, 2560), (129, 512, 2560), (257, 2560, 10240), (700, 768, 2560), (1185, 512, 10240),
+                                      (1300, 768, 10240), (2000, 2560, 2560), (3333, 512, 2560), (4161, 768, 2560), (4480, 2560, 2560),
+                                      (5000, 512, 2560), (6305, 768, 2560), (9001, 512, 2560)])
+def test_linear(dev, rows, k, n, with_bias):
+    from comfyui_amd import functional as HF
+    a, w = operands(rows, n, k, rows + k, dev)
+    bias = torch.randn(n, generator=torch.Generator().manual_seed(3)).to(BF16).to(dev) if with_bias else None
+    sw, si = torch.tensor(0.0007, device=dev), torch.tensor(0.6, device=dev)
+    y = HF.linear(a, w, sw, si, bias=bias)
+    check(y, a, w, float(sw * si), bias)
+    some = min(rows, 96)
+    assert torch.equal(HF.linear(a[-some:].contiguous(), w, sw, si, bias=bias), y[-some:])
+
+
+@pytest.mark.parametrize("sizes,k", [((129, 161, 193, 225, 256, 33, 0, 1), 512), ((400, 416, 450, 480, 511, 513, 300, 290), 768),
+                                     ((1000, 20, 2100, 257), 2560)])
+def test_segments(dev, sizes, k):
+    n, rows = 2560, sum(sizes)
+    off = torch.tensor([0] + list(torch.tensor(sizes).cumsum(0)), dtype=torch.int32)
+    a, _ = operands(rows, 256, k, rows, dev)
+    ws = [operands(1, n, k, 50 + e, dev)[1] for e in range(len(sizes))]
+    sw, si = torch.tensor(0.0005, device=dev), torch.tensor(0.5, device=dev)
+    arr = (_lib.FfnWeights * len(sizes))()
+    for e in range(len(sizes)):
+        arr[e].w2, arr[e].scale_w2, arr[e].scale_in2 = ws[e].data_ptr(), sw.data_ptr(), si.data_ptr()
+    y = torch.full((rows + 1, n), 7.0, dtype=BF16, device=dev)
+    offsets = off.to(dev)
+    _lib.check(_lib.lib.hdmoe_grouped_down(_lib.W_E4M3FN, a.data_ptr(), offsets.data_ptr(), rows, len(sizes), k, n, arr, y.data_ptr(), None))
+    torch.cuda.synchronize()
+    assert bool((y[rows] == 7.0).all())
+    for e in range(len(sizes)):
+        if sizes[e]:
+            check(y[off[e]:off[e + 1]], a[off[e]:off[e + 1]], ws[e], float(sw * si))
