@@ -1200,6 +1200,16 @@ size_t g4_tail_room(int n_dyn, int rows_mean, int n_out_dyn, int kb_dyn, int row
   return most;
 }
 
+// Whether tiles of two lengths are dealt out by g4_two_lengths: up to seven quarters of a round of the long ones (measured there).
+bool g4_two_pays(const GemmArgs& args, int rows_mean) {
+  long longs = 0;
+  for (int g = 0; g < args.G; ++g) {
+    const GemmGroup& gg = args.g[g];
+    if ((gg.row_begin < 0) == (args.spread > 0)) longs += (long)((gg.row_begin < 0 ? rows_mean : gg.row_end - gg.row_begin) + G4_BM - 1) / G4_BM * (gg.n_out / BN);
+  }
+  return 4 * longs <= 7 * HDMOE_NUM_CU;
+}
+
 template <G4Type TY, int EPI>
 int launch_gemm4w(GemmArgs& args, int rows_mean, hipStream_t s, const char* what) {
   constexpr int FEAT = EPI == G4_SWIGLU ? 128 : 256;
@@ -1222,7 +1232,7 @@ int launch_gemm4w(GemmArgs& args, int rows_mean, hipStream_t s, const char* what
                      has_static ? last.row_end - last.row_begin : 0, last.n_out, last.kbytes, FEAT, TY == G4_W8) == 0)
       args.tail = nullptr;
   }
-  args.cap = g4_host_cap(args, FEAT, TY == G4_W8 ? 3 : 2, HDMOE_NUM_CU);
+  args.cap = args.spread != 0 ? (g4_two_pays(args, rows_mean) ? -1 : 0) : g4_host_cap(args, FEAT, TY == G4_W8 ? 3 : 2, HDMOE_NUM_CU);
   // one block per CU whatever the number of tiles: a block without any ends at once
   hipLaunchKernelGGL((gemm4w_kernel<TY, EPI>), dim3(HDMOE_NUM_CU), dim3(G4_THREADS), G4_SMEM, s, args);
   if constexpr (EPI != G4_PARTIAL && TY != G4_F8) {

@@ -136,8 +136,13 @@ __device__ __forceinline__ G4Tail g4_tail_of(const GemmArgs& args, const Segment
 constexpr int G4_TILE_COST = 150, G4_CAP_ROUNDS = 24;
 struct G4Heights { int mt, height; };
 __host__ __device__ __forceinline__ G4Heights g4_heights(int rows, int cap) {
-  const int units = (rows + 31) >> 5, mt = (units + cap - 1) / cap;
-  return {mt, max((units + mt - 1) / max(mt, 1), G4_MIN_BLOCKS)};
+#if defined(__HIP_DEVICE_COMPILE__)
+  auto div = [](int a, int b) { return tile_div(a, b); };
+#else
+  auto div = [](int a, int b) { return a / b; };
+#endif
+  const int units = (rows + 31) >> 5, mt = div(units + cap - 1, cap);
+  return {mt, max(div(units + mt - 1, max(mt, 1)), G4_MIN_BLOCKS)};
 }
 
 // What a cap comes to; rows(g), ntiles(g): the rows of group g, its tiles along the features.
@@ -190,6 +195,45 @@ __device__ __forceinline__ int g4_cap(const GemmArgs& args, const Segments& seg,
   const int mine = g4_cap_cost(args.G, seg.bytes(0) / (2 * BK), [&](int g) { return seg.rows(g); }, [&](int g) { return seg.ntiles(g, FEAT); }, blocks,
                                G4_MIN_BLOCKS + min(lane, 4));
   return g4_best_cap(whole, seg.bytes(0) / (2 * BK), [&](int cap) { return __builtin_amdgcn_readlane(mine, cap - G4_MIN_BLOCKS); });
+}
+
+// Tiles of two lengths (a layer's down projection: the experts' K and the shared expert's, args.spread). The long ones go round by round
+// over the blocks; those without one in the last of these rounds (light blocks) take short ones first, as many rounds of them as fit beside a
+// long one, and what is left goes round by round over all, light blocks first (g4_place). Groups are long or short by args.spread.
+// The caps are those of the shortest longest block; others than whole tiles have to pay by a twelfth in fp8, an eighth in 16 bits (two rounds
+// of 7 blocks and more, 90 % of the cost, take as long: the clock falls with the CUs that are busy). Layers of 4 experts with K = 6912 and a
+// shared one with 3584, every XCD an eighth of every group -> this, us: fp8, 2600 tokens 319 -> 311, 3000 357 -> 344, 3500 405 -> 398, 4096 the
+// same, 4500 517 -> 499, 5000 549 -> 534; e4m3fn weights in bf16, 2100 491 -> 438, 3000 616 -> 588, 4080 the same; bf16, 2100 520 -> 468, 3000
+// 655 -> 637. With more than 448 long tiles the eighths are better or equal (fp8 8192 tokens 821 -> 826, 12000 1167 -> 1177).
+struct G4Two { int cost, light_rounds; };
+template <class Segs>
+__device__ __forceinline__ G4Two g4_two_lengths(const Segs& seg, int G, int spread, int feat, int cap_long, int cap_short) {
+  constexpr int PAIR[5] = {58, 70, 80, 90, 100}, BLOCKS = HDMOE_NUM_CU;
+  int n[5] = {0, 0, 0, 0, 0}, shorts = 0, top = 0, pairs_long = 0, pairs_short = 0;
+  for (int g = 0; g < G; ++g) {
+    const bool is_short = seg.dynamic(g) == (spread < 0);
+    (is_short ? pairs_short : pairs_long) = seg.bytes(g) / (2 * BK);
+    const G4Heights t = g4_heights(seg.rows(g), is_short ? cap_short : cap_long);
+    const int tiles = t.mt * seg.ntiles(g, feat);
+    if (is_short) { shorts += tiles; top = max(top, t.mt > 0 ? t.height : 0); }
+#pragma unroll
+    for (int h = 0; h < 5; ++h) n[h] += !is_short && t.height == h + G4_MIN_BLOCKS ? tiles : 0;
+  }
+  int heavy = 0, last = 0, at = 0, each = G4_TILE_COST;
+#pragma unroll
+  for (int h = 4; h >= 0; --h) {
+    const int to = at + n[h], started = (to + BLOCKS - 1) / BLOCKS - (at + BLOCKS - 1) / BLOCKS, tile = pairs_long * PAIR[h] + G4_TILE_COST;
+    heavy += started * tile;
+    last = started > 0 ? tile : last;
+    each += top == h + G4_MIN_BLOCKS ? pairs_short * PAIR[h] : 0;
+    at = to;
+  }
+  const int left = at % BLOCKS, lights = BLOCKS - left, light = left > 0 ? heavy - last : heavy;
+  const int light_rounds = left > 0 ? tile_div(last, each) : 0;
+  const int rest = shorts - light_rounds * lights;
+  if (rest <= 0) return {heavy, light_rounds};
+  const int q = rest / BLOCKS, r = rest % BLOCKS;
+  return {max(light + (light_rounds + q + (r > 0 ? 1 : 0)) * each, heavy + (q + (r > lights ? 1 : 0)) * each), light_rounds};
 }
 
 // On the host, where the rows of a launch are known; -1: the device has to find it. On the device -> on the host, Linears in bf16, us: 700 rows
@@ -254,8 +298,29 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   const int xcd = blockIdx.x % HDMOE_NUM_XCD, slot = blockIdx.x / HDMOE_NUM_XCD;
   constexpr int nslots = HDMOE_NUM_CU / HDMOE_NUM_XCD;   // the grid is one block per CU
   const G4Tail tail = g4_tail_of<TY, FEAT>(args, segs, HDMOE_NUM_CU);
-  const int cap = EPI == G4_PARTIAL || SWIGLU || args.spread != 0 ? 0 : args.cap >= 0 ? args.cap : sgpr(g4_cap<FEAT>(args, segs, tail, HDMOE_NUM_CU, lane));
-  // cap > 0: lane g looks up where group g comes in the order of heights: [first tile, tiles, height, m-tiles]
+  int cap = 0, cap_short = 0, light_rounds = 0;
+  if (EPI != G4_PARTIAL && !SWIGLU) {
+    if (args.cap >= 0) {
+      cap = args.cap;
+    } else if (args.spread == 0) {
+      cap = sgpr(g4_cap<FEAT>(args, segs, tail, HDMOE_NUM_CU, lane));
+    } else {   // lane i works out caps 4 + i / 5 and 4 + i % 5
+      const int c = min(lane, 24), c5 = c * 13 >> 6;
+      const G4Two mine = g4_two_lengths(segs, args.G, args.spread, FEAT, G4_MIN_BLOCKS + c5, G4_MIN_BLOCKS + c - 5 * c5);
+      int best = 24, limit = __builtin_amdgcn_readlane(mine.cost, 24);
+      limit -= limit / (F8 ? 12 : 8);
+#pragma unroll
+      for (int k = 0; k < 24; ++k) {
+        const int v = __builtin_amdgcn_readlane(mine.cost, k);
+        if (v < limit) { limit = v; best = k; }
+      }
+      cap = sgpr(G4_MIN_BLOCKS + best / 5);
+      cap_short = sgpr(G4_MIN_BLOCKS + best % 5);
+      light_rounds = __builtin_amdgcn_readlane(mine.light_rounds, best);
+    }
+  }
+  auto is_short = [&](int g) { return args.cap < 0 && args.spread != 0 && segs.dynamic(g) == (args.spread < 0); };
+  // cap > 0: lane g looks up where group g comes among those of its length in the order of heights: [first tile, tiles, height, m-tiles]
   v4i* const heights = reinterpret_cast<v4i*>(smem + G4_HEIGHTS);
   if (cap > 0) {
     v4i e = {0, 0, 0, 0};
@@ -263,13 +328,14 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
       int rb, re;
       segs.get(g, rb, re);
       if (re > rb && lane == g) {
-        const G4Heights t = g4_heights(re - rb, cap);
+        const G4Heights t = g4_heights(re - rb, is_short(g) ? cap_short : cap);
         e = v4i{0, t.mt * segs.ntiles(g, FEAT), t.height, t.mt};
       }
     }
     for (int k = 0; k < args.G; ++k) {
       const int h = __builtin_amdgcn_readlane(e.z, k), tiles = __builtin_amdgcn_readlane(e.y, k);
-      if (h > e.z || (h == e.z && k < lane)) e.x += tiles;
+      const bool other = args.cap < 0 && args.spread != 0 && segs.dynamic(k) != !(segs.fixed >> lane & 1);
+      if (!other && (h > e.z || (h == e.z && k < lane))) e.x += tiles;
     }
     if (lane < args.G) heights[lane] = e;   // every wave the same
   }
@@ -277,19 +343,17 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   auto fill_table = [&](int base) {
     const int i = base + lane;
     if (cap > 0) {
-      // a last round of a few tiles is spread over the XCDs (consecutive blocks of it on the first ones: a Linear of 80 tiles 34.2 us, so 30.2)
-      int total = 0;
-      for (int g = 0; g < args.G; ++g) total += sgpr(heights[g].y);
-      const int full = total / HDMOE_NUM_CU, left = total % HDMOE_NUM_CU, share = (left + HDMOE_NUM_XCD - 1) / HDMOE_NUM_XCD;
-      const int L = i < full ? i * HDMOE_NUM_CU + xcd * nslots + slot
-                             : i == full && slot < share && xcd * share + slot < left ? full * HDMOE_NUM_CU + xcd * share + slot : -1;
+      int longs = 0, shorts = 0;
+      for (int g = 0; g < args.G; ++g) (is_short(g) ? shorts : longs) += sgpr(heights[g].y);
+      const G4Place at = g4_place(longs, shorts, light_rounds, xcd, slot, i);
+      const int L = at.tile;
       v4i e = {-1, 0, 0, 0};
       for (int g = 0; g < args.G; ++g) {
         const v4i t = heights[g];
         const int first = sgpr(t.x), tiles = sgpr(t.y), rows = sgpr(t.z) * 32, mtiles = sgpr(t.w);
         int rb, re, m, n;
         segs.get(g, rb, re);
-        if (L < first || L >= first + tiles) continue;
+        if (L < first || L >= first + tiles || is_short(g) != at.is_short) continue;
         g4_raster(L - first, mtiles, segs.ntiles(g, FEAT), m, n);
         const int row0 = rb + m * rows;
         e = v4i{g | min(re - row0, rows) << 16, row0, n, segs.bytes(g) / BK << 16};

@@ -5,3 +5,7 @@ extern "C" void t_tail_unit(int swiglu, int item, int wave, int tile, int* out) 
   out[0] = u.q; out[1] = u.w; out[2] = u.tt;
 }
 extern "C" int t_part_blocks(int rows, int w) { return g4_part_blocks(rows, w); }
+extern "C" int t_place(int longs, int shorts, int light_rounds, int xcd, int slot, int i) {
+  const G4Place p = g4_place(longs, shorts, light_rounds, xcd, slot, i);
+  return p.tile < 0 ? -1 : p.tile * 2 + (p.is_short ? 1 : 0);
+}

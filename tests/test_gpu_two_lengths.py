@@ -1,0 +1,54 @@
+"""The down projection of a layer whose experts and shared expert have different K, on tiles of several heights dealt out by their length
+(csrc/gemm4w.h, g4_two_lengths; up to 448 tiles of the long kind): rows come out as they do among more tokens, where whole tiles are dealt out
+in eighths, and for fp8 as on the 8-wave kernels."""
+import pytest
+import torch
+
+from comfyui_amd import ops, synth
+from comfyui_amd.hidream import MOEFeedForwardSwiGLU
+from tests.helpers import saved_forms, set_form
+
+pytestmark = pytest.mark.gpu
+BF16, FP8 = torch.bfloat16, torch.float8_e4m3fn
+MOST = 6400   # 520 tiles of the longer kind
+
+
+@pytest.fixture
+def forms():
+    yield from saved_forms()
+
+
+def layer(dev, kind):
+    g = torch.Generator(device=dev).manual_seed(7)
+    o = {"fp8": lambda: ops.scaled_fp8_ops(fp8_matrix_mult=True, scale_input=True, override_dtype=FP8),
+         "upcast": lambda: ops.scaled_fp8_ops(fp8_matrix_mult=False, scale_input=False, override_dtype=FP8), "bf16": lambda: ops.disable_weight_init}[kind]()
+    m = MOEFeedForwardSwiGLU(synth.DIM, 4 * synth.DIM, 4, 2, dtype=BF16, device=dev, operations=o).eval()
+    for f in [*m.experts, m.shared_experts]:
+        for lin in (f.w1, f.w2, f.w3):
+            w = torch.randn(tuple(lin.weight.shape), generator=g, device=dev) * 0.02
+            if kind == "bf16":
+                lin.weight = torch.nn.Parameter(w.to(BF16), requires_grad=False)
+                continue
+            w8, s = synth.quantize_per_tensor(w)
+            lin.weight, lin.scale_weight = torch.nn.Parameter(w8, requires_grad=False), torch.nn.Parameter(s, requires_grad=False)
+            if kind == "fp8":
+                lin.scale_input = torch.nn.Parameter(torch.ones((), device=dev), requires_grad=False)
+    gate = torch.randn(tuple(m.gate.weight.shape), generator=g, device=dev) * 0.02
+    gate[0, :64] += 0.02   # uneven segments
+    m.gate.weight = torch.nn.Parameter(gate.to(BF16), requires_grad=False)
+    return m, torch.randn((1, MOST, synth.DIM), generator=g, device=dev).add_(0.2).to(BF16)
+
+
+@pytest.mark.parametrize("kind", ["fp8", "upcast", "bf16"])
+def test_rows_are_those_of_a_larger_call(dev, forms, kind):
+    m, x = layer(dev, kind)
+    m.batch_invariant = True   # no sums cut along K by the segments' sizes
+    with torch.no_grad():
+        full = m(x)
+        assert bool(torch.isfinite(full.float()).all()) and float(full.float().std()) > 0
+        for tokens in (2100, 2300, 2600, 3000, 4096, 4500, 5400):   # (in 16 bits 2049 are cut along K)
+            assert torch.equal(m(x[:, :tokens]), full[:, :tokens]), tokens
+        if kind == "fp8":
+            set_form("HDMOE_SWIGLU4W", "0")
+            assert torch.equal(m(x[:, :3000]), full[:, :3000])
+
