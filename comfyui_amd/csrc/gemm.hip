@@ -1792,6 +1792,48 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
     return fixed(parts < 1 ? 1 : (int)parts);
   }
 
+  // A dense feed-forward in fp8 on the 4-wave kernel, whose tiles can be lower (gemm4w.h): parts on 128-token tiles, which fill more CUs with
+  // fewer parts. In hundredths of a pair of K steps (24.6 ns) as in g4_cap_cost; a part's sums written and read again at about 5 TB/s, 100
+  // for the kernel that adds them up. Whole branch, D = 2560, H = 6912, us, on 256-token tiles (6 to 2 parts) -> this: 300 rows 61.0 -> 53.7 (6 parts),
+  // 512 63.4 -> 56.7 (4), 768 67.9 -> 61.2 (3), 1024 85.9 -> 79.5 (3), 1536 104.2 -> 97.1 (2), 2048 138.2 -> 129.4 (not cut).
+  if (weight_dtype == HDMOE_W_E4M3FN && !dyn && kts % 2 == 0 && kts >= 4) {
+    constexpr int PAIR[5] = {58, 70, 80, 90, 100};
+    const int pairs = kts / 2;
+    auto rounds = [&](int bm, int parts) { return ((long)(rows_static + bm - 1) / bm * nt * parts + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU; };
+    double best_cost = 1e30;
+    int best = 1;
+    for (int h = 4; h <= 8; ++h) best_cost = fmin(best_cost, (double)rounds(32 * h, 1) * (pairs * PAIR[h - 4] + G4_TILE_COST));
+    best_cost *= 0.95;   // a cut has to pay
+    for (int parts = 2; parts <= 6 && pairs / parts >= 3; ++parts) {
+      const double cost = (double)rounds(128, parts) * ((pairs + parts - 1) / parts * PAIR[0] + G4_TILE_COST) + (double)parts * rows_static * N * 8.0 / 123e3 + 100.0;
+      if (cost < best_cost) { best = parts; best_cost = cost; }
+    }
+    pl.bm = best > 1 ? 128 : TileCfg<4>::BM;
+    return fixed(best);
+  }
+  // A layer in fp8 on that kernel: the most parts whose tiles fit one round of blocks, on 128-token tiles with even segments, else on 256-token
+  // tiles with segments a standard deviation above the mean; beyond that none (g4_two_lengths deals the tiles out). The shared expert's
+  // tiles in as many parts as make them about as long. Whole layer, us, four to six candidates on 256-token tiles of which the device took the
+  // first that fitted -> this (three inputs each): 350 tokens 118 -> 113 ((2, 1) parts of 128), 400 123 -> 118, 450 150 -> 143, 500 147 -> 144, 640 145 ->
+  // 141 ((2, 1) of 256; of 128 in two rounds 164, whole tiles 157), 768 158 -> 156, 900 202 -> 199, 1024 209 -> 204 (whole), 1600 the same, 2000 266 ->
+  // 248. Not under 150 rows an expert: 300 tokens 106, 106, 260 103, 105.
+  if (weight_dtype == HDMOE_W_E4M3FN && dyn && rows_static > 0 && rows_dyn >= 150 * n_dyn && ktd % 2 == 0 && kts % 2 == 0 && ktd >= 4 && kts >= 4) {
+    const double mu = (double)rows_dyn / n_dyn;
+    for (int bm : {128, 256}) {
+      const int seg = bm == 128 ? (rows_dyn + n_dyn - 1) / n_dyn : (int)(mu + sqrt(mu));
+      const int mt_d = n_dyn * ((seg + bm - 1) / bm), mt_s = (rows_static + bm - 1) / bm;
+      for (int pd = 6; pd >= 2; --pd) {
+        const int ps = (int)fmin(fmax((double)pd * kts / ktd + 0.5, 1.0), (double)pd);
+        if (ktd / 2 / pd < 3 || kts / 2 / ps < 3 || (mt_d * pd + mt_s * ps) * nt > HDMOE_NUM_CU) continue;
+        pl.n = 1;
+        pl.pd[0] = pd;
+        pl.ps[0] = ps;
+        pl.bm = bm;
+        return pd;
+      }
+    }
+    return fixed(1);
+  }
   const int bm = TileCfg<4>::BM;
   const double red_unit = (double)N * 8.0 / 10e12 / 1.4e-6;  // K steps per row and part of partial sums
   if (!dyn || rows_static <= 0) {

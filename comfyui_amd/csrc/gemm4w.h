@@ -288,6 +288,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     }
     plan_idx = hdmoe_plan_pick(args.plan, mt_dyn, mt_static, segs.ntiles(0, FEAT));
   }
+  const int bm = EPI == G4_PARTIAL && F8 ? args.plan.bm : G4_BM;   // rows of a tile that is not capped
   auto parts_of = [&](int g) {
     return EPI != G4_PARTIAL ? 1 : segs.dynamic(g) ? args.plan.pd[plan_idx] : args.plan.ps[plan_idx];
   };
@@ -382,7 +383,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
       const int g = args.spread < 0 ? args.G - 1 - k : k;
       int rb, re;
       segs.get(g, rb, re);
-      const int mt = (re - rb + G4_BM - 1) / G4_BM, nt = segs.ntiles(g, FEAT), np = parts_of(g);
+      const int mt = EPI == G4_PARTIAL && F8 ? tile_div(re - rb + bm - 1, bm) : (re - rb + G4_BM - 1) / G4_BM, nt = segs.ntiles(g, FEAT), np = parts_of(g);
       const long long tiles = (long long)mt * nt * np;
       const int lo = eighths ? (int)(xcd * tiles / HDMOE_NUM_XCD) : 0;
       const int hi = eighths ? (int)((xcd + 1) * tiles / HDMOE_NUM_XCD) : (int)tiles;
@@ -395,11 +396,11 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     if (g_at >= 0) {
       int part = EPI == G4_PARTIAL ? tile_div(L, mtiles * ntiles) : 0, m, n;
       g4_raster(L - part * (mtiles * ntiles), mtiles, ntiles, m, n);
-      const int row0 = rb_at + m * G4_BM;
+      const int row0 = rb_at + m * bm;
       // parts start on a pair of K steps
       const int of = tail_slot > 0 ? tail.parts : parts, at = tail_slot > 0 ? tail_part : part;
       const int kt0 = at == 0 ? 0 : tile_div(kt / 2 * at, of) * 2, kt1 = at + 1 == of ? kt : tile_div(kt / 2 * (at + 1), of) * 2;
-      e = v4i{g_at | part << 8 | min(re_at - row0, G4_BM) << 16, row0, n | tail_slot << 16, kt0 | (kt1 - kt0) << 16};
+      e = v4i{g_at | part << 8 | min(re_at - row0, bm) << 16, row0, n | tail_slot << 16, kt0 | (kt1 - kt0) << 16};
     }
     table[lane] = e;
   };

@@ -379,14 +379,15 @@ int run_ffn(const char* what, int weight_dtype, const void* x_bf16, int rows, in
   if (int rc = hdmoe_launch_ffn_gemm(true, weight_dtype, nullptr, nullptr, 0, 0, nullptr, nullptr, a, rows, w, h, 0, 0, D, H,
                                      s, what, nullptr, 0, nullptr, 1, 0, true, nullptr, nullptr, tail))
     return rc;
-  const int parts = hdmoe_down_parts(0, 0, rows, D, 0, H, weight_dtype);
+  HdmoeSplitPlan plan;
+  const int parts = hdmoe_down_parts(0, 0, rows, D, 0, H, weight_dtype, &plan);
   float* partial = parts > 1 ? room : nullptr;
   HdmoeGatedResidual end = {nullptr, nullptr, 1};
   if (mod != nullptr) end = {static_cast<const uint16_t*>(mod->gate), static_cast<const uint16_t*>(x_bf16), mod->rows_per_batch};
   const bool end_here = mod != nullptr && parts > 1;   // the kernel that adds the parts up does the rest
   uint8_t* const y = mod != nullptr && !end_here ? rows_bf16 : static_cast<uint8_t*>(out_bf16);   // (the normalised rows are used up)
   if (int rc = hdmoe_launch_ffn_gemm(false, weight_dtype, nullptr, nullptr, 0, 0, nullptr, nullptr, h, rows, w, y, 0, 0, H, D, s, what,
-                                     nullptr, 0, partial, parts, 0, true, nullptr, nullptr, parts > 1 ? nullptr : tail,
+                                     nullptr, 0, partial, parts, 0, true, &plan, nullptr, parts > 1 ? nullptr : tail,
                                      end_here ? &end : nullptr))
     return rc;
   return mod == nullptr || end_here ? HDMOE_OK

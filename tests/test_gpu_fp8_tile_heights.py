@@ -45,3 +45,31 @@ def test_segments(dev, sizes, k):
     for e in range(len(sizes)):
         if sizes[e]:
             check(y[off[e]:off[e + 1]], a[off[e]:off[e + 1]], ws[e], float(sw * si))
+
+
+@pytest.mark.parametrize("rows,dim,hidden", [(257, 2560, 6912), (300, 512, 3584), (513, 2560, 6912), (768, 2560, 2560), (1300, 2560, 6912), (2048, 2560, 6912)])
+def test_dense_feed_forward(dev, rows, dim, hidden):
+    """Down projections in parts of 128-token tiles and whole, against the product of the h left in the workspace."""
+    import ctypes
+    L = _lib.lib
+    FP8 = torch.float8_e4m3fn
+    g = torch.Generator(device=dev).manual_seed(rows)
+    x = torch.randn((rows, dim), generator=g, device=dev).to(BF16)
+    w1, w3 = ((torch.randn((hidden, dim), generator=g, device=dev) * 40).to(FP8) for _ in range(2))
+    w2 = (torch.randn((dim, hidden), generator=g, device=dev) * 40).to(FP8)
+    scales = torch.tensor([0.0006, 0.0005, 0.0007, 0.5, 1.0], device=dev)
+    fw = _lib.FfnWeights()
+    fw.w1, fw.w2, fw.w3 = w1.data_ptr(), w2.data_ptr(), w3.data_ptr()
+    fw.scale_w1, fw.scale_w2, fw.scale_w3 = (scales[i:].data_ptr() for i in range(3))
+    fw.scale_in1 = fw.scale_in3 = scales[4:].data_ptr()
+    fw.scale_in2 = scales[3:].data_ptr()
+    nbytes = L.hdmoe_ffn_workspace_bytes(rows, dim, hidden, _lib.W_E4M3FN)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    y = torch.full((rows + 1, dim), 7.0, dtype=BF16, device=dev)
+    _lib.check(L.hdmoe_ffn_swiglu(_lib.W_E4M3FN, x.data_ptr(), rows, dim, hidden, ctypes.byref(fw), y.data_ptr(), ws.data_ptr(), nbytes, None))
+    torch.cuda.synchronize()
+    assert bool((y[rows] == 7.0).all())
+    at = -(-rows * dim // 256) * 256
+    h = ws[at:at + rows * hidden].view(FP8).view(rows, hidden)
+    assert float(h.float().std()) > 0.1
+    check(y[:rows], h, w2, float(scales[1]) * 0.5)
