@@ -99,6 +99,7 @@ struct HdmoeSplitPlan {
   int ps[HDMOE_PLAN_MAX];    // K parts of a tile of the static group (the shared expert)
   int bm;                    // tile height (tokens) the launch runs with
   int max_tiles;             // an entry before the last is taken only if its tiles number at most this
+  int fixed_pd, fixed_ps;    // the cut where the segments' sizes may not decide (fixed_k_cut of the arguments)
 };
 
 // mt_dyn / mt_static: m-tiles (tile height plan.bm) of all experts' segments / of the static group; ntiles_n: tiles

@@ -1759,7 +1759,7 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
   pl.max_tiles = HDMOE_NUM_CU;
   auto fixed = [&](int parts) {
     pl.n = 1;
-    pl.pd[0] = pl.ps[0] = parts;
+    pl.pd[0] = pl.ps[0] = pl.fixed_pd = pl.fixed_ps = parts;
     return parts;
   };
   const int eb = elem_bytes(weight_dtype);
@@ -1826,8 +1826,8 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
         const int ps = (int)fmin(fmax((double)pd * kts / ktd + 0.5, 1.0), (double)pd);
         if (ktd / 2 / pd < 3 || kts / 2 / ps < 3 || (mt_d * pd + mt_s * ps) * nt > HDMOE_NUM_CU) continue;
         pl.n = 1;
-        pl.pd[0] = pd;
-        pl.ps[0] = ps;
+        pl.pd[0] = pl.fixed_pd = pd;
+        pl.ps[0] = pl.fixed_ps = ps;
         pl.bm = bm;
         return pd;
       }
@@ -1889,9 +1889,16 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
     const int mt_d_hi = n_dyn * (int)(((long)(mu + sqrt(mu)) + bm - 1) / bm);
     if ((mt_d_hi * pl.pd[0] + mt_s * pl.ps[0]) * nt <= HDMOE_NUM_CU) {
       pl.n = 1;
+      pl.fixed_pd = pl.pd[0];
+      pl.fixed_ps = pl.ps[0];
       return pl.pd[0];
     }
   }
+  // 16-bit activations on the 4-wave kernel: where no candidate fits, whole tiles, dealt out by g4_two_lengths if that is so for even segments.
+  // The cost model's cut in more than a round -> this, layers, us: bf16, 1024 tokens with an expert above 512 rows 339 -> 306, 1800 469 -> 434, 2040 489 ->
+  // 459; e4m3fn weights, 1024 318 -> 265, 1800 441 -> 415, 2040 456 -> 433.
+  const bool whole16 = weight_dtype != HDMOE_W_E4M3FN && ktd % 2 == 0 && kts % 2 == 0 && ktd >= 6 && kts >= 6;
+  if (whole16 && pl.n == 0) return fixed(1);
   // Last entry, for when no candidate fits: the cheapest cut by the cost model. With candidates listed, their not
   // fitting means ragged segments, and the experts' m-tiles are counted one standard deviation above the mean
   // segment (counts are about binomial); with none, 12 % above the mean.
@@ -1911,10 +1918,12 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
         best_cost = cost;
       }
     }
-  pl.pd[pl.n] = best_d;
-  pl.ps[pl.n] = best_s;
+  pl.fixed_pd = best_d;
+  pl.fixed_ps = best_s;
+  pl.pd[pl.n] = whole16 ? 1 : best_d;
+  pl.ps[pl.n] = whole16 ? 1 : best_s;
   ++pl.n;
-  int most = 1;
+  int most = best_d;
   for (int i = 0; i < pl.n; ++i) most = pl.pd[i] > most ? pl.pd[i] : most;
   if (most == 1) return fixed(1);  // nothing is cut
   return most;
