@@ -83,6 +83,15 @@ struct HdmoeGatedResidual {
   int rows_per_batch;
 };
 
+// The dispatch of a few slots inside the gate/up GEMM (grouped_gemm_kernel): every block sorts them for itself, the first one leaves the
+// results of hdmoe_dispatch for the kernels behind it.
+struct HdmoeRoute {
+  const int32_t* idx;        // [n] expert of every flat slot; NULL = the dispatch has run before
+  int n, E;                  // n at most HDMOE_ROUTE_SLOTS
+  int32_t *counts, *offsets, *perm, *inv_perm;
+};
+constexpr int HDMOE_ROUTE_SLOTS = 512;   // one per thread of a block
+
 constexpr int HDMOE_NUM_CU = 256;   // MI355X
 constexpr int HDMOE_NUM_XCD = 8;
 

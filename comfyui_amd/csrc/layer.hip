@@ -11,7 +11,8 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
                           const int32_t* gather_dyn = nullptr, int gather_rows = 0, float* partial = nullptr,
                           int nparts = 1, int gather_shift = 0, bool reduce = true,
                           const HdmoeSplitPlan* plan = nullptr, const HdmoeAltOperand* alt = nullptr,
-                          float* tail = nullptr, const HdmoeGatedResidual* end = nullptr);
+                          float* tail = nullptr, const HdmoeGatedResidual* end = nullptr, const HdmoeRoute* route = nullptr);
+bool hdmoe_gate_up_routes(int weight_dtype, int rows_dyn, int n_dyn, int rows_static, int N_dyn, int N_static);
 int hdmoe_launch_ln_modulate(const void* x_bf16, const void* scale_bf16, const void* shift_bf16, int T, int D, int tokens_per_batch,
                              float eps, void* out_bf16, void* out_fp8, const float* scale_in, const float* scale_in_also, hipStream_t s,
                              const char* what);
@@ -253,9 +254,13 @@ extern "C" int hdmoe_moe_ffn(const hdmoe_layer_args* p, hdmoe_stream_t stream) {
     if (int rc = hdmoe_launch_gate(xin, p->gate_w, T, D, E, idx, tw, hist, s, "hdmoe_moe_ffn (gate)")) return rc;
   }
   mark();
-  if (int rc = hdmoe_launch_dispatch_scatter(idx, T, E, counts, offsets, perm, inv_perm, hist,
-                                             hdmoe_gate_tokens_per_block(T, D, E, fp8, ln_in_gate), s, "hdmoe_moe_ffn (dispatch)"))
-    return rc;
+  // a few slots: by the gate/up contraction itself
+  const HdmoeRoute route = {idx, (int)n, E, counts, offsets, perm, inv_perm};
+  const bool routes = hdmoe_gate_up_routes(wd, (int)n, E, Hs > 0 ? T : 0, H, Hs);
+  if (!routes)
+    if (int rc = hdmoe_launch_dispatch_scatter(idx, T, E, counts, offsets, perm, inv_perm, hist,
+                                               hdmoe_gate_tokens_per_block(T, D, E, fp8, ln_in_gate), s, "hdmoe_moe_ffn (dispatch)"))
+      return rc;
   mark();
 
   // bf16 weights: the GEMM reads the tokens themselves, the routed rows through the permutation (row perm[r] / 2
@@ -285,7 +290,7 @@ extern "C" int hdmoe_moe_ffn(const hdmoe_layer_args* p, hdmoe_stream_t stream) {
                                      a_static, Hs > 0 ? T : 0, p->shared, h_shared, D, H, D, Hs, s,
                                      "hdmoe_moe_ffn (gate/up)", perm, per_token ? T : (int)n, nullptr, 1,
                                      per_token ? 1 : 0, true, nullptr, decide ? &alt : nullptr,
-                                     tail))
+                                     tail, nullptr, routes ? &route : nullptr))
     return rc;
   mark();
   // down projections, both in one launch
