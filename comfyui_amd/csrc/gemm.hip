@@ -155,8 +155,9 @@ struct Segments {
     begin = __builtin_amdgcn_readlane(rb, g);
     end = __builtin_amdgcn_readlane(re, g);
   }
-  __device__ __forceinline__ int rows(int g) const { return __builtin_amdgcn_readlane(re - rb, g); }
-  __device__ __forceinline__ int ntiles(int g, int feat) const { return __builtin_amdgcn_readlane((int)((unsigned)n_out / (unsigned)feat), g); }
+  // (arithmetic behind the read: lane g may be switched off where these are called, and then forms nothing)
+  __device__ __forceinline__ int rows(int g) const { return __builtin_amdgcn_readlane(re, g) - __builtin_amdgcn_readlane(rb, g); }
+  __device__ __forceinline__ int ntiles(int g, int feat) const { return (int)((unsigned)__builtin_amdgcn_readlane(n_out, g) / (unsigned)feat); }
   __device__ __forceinline__ int bytes(int g) const { return __builtin_amdgcn_readlane(kbytes, g); }
   __device__ __forceinline__ bool dynamic(int g) const { return !(fixed >> g & 1); }
 };

@@ -352,12 +352,13 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
       for (int g = 0; g < args.G; ++g) {
         const v4i t = heights[g];
         const int first = sgpr(t.x), tiles = sgpr(t.y), rows = sgpr(t.z) * 32, mtiles = sgpr(t.w);
+        const int nt = segs.ntiles(g, FEAT), kt = segs.bytes(g) / BK;
         int rb, re, m, n;
         segs.get(g, rb, re);
         if (L < first || L >= first + tiles || is_short(g) != at.is_short) continue;
-        g4_raster(L - first, mtiles, segs.ntiles(g, FEAT), m, n);
+        g4_raster(L - first, mtiles, nt, m, n);
         const int row0 = rb + m * rows;
-        e = v4i{g | min(re - row0, rows) << 16, row0, n, segs.bytes(g) / BK << 16};
+        e = v4i{g | min(re - row0, rows) << 16, row0, n, kt << 16};
       }
       table[lane] = e;
       return;
