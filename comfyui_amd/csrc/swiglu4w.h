@@ -47,18 +47,34 @@ __global__ __launch_bounds__(W4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   auto sgpr = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
 
   // ---- tile enumeration: as grouped_gemm_kernel with one tile list cut in eighths ---------------------------
-  const Segments segs(args, lane);
+  // The block's first two tiles come from the packed segments; the later ones, looked up behind K loops, from the arguments and one register of
+  // bounds: four registers of segments across the statements, which leave the compiler 32, had 207 spilled, fragments on their way among them (layers of 512 tokens
+  // 149 us, so 135; 900 200 -> 178; 1024 209 -> 189), and with tile_div in the later ones still 9.
+  int off_lane = 0;
+  if (args.offsets != nullptr && lane <= args.n_offsets) off_lane = args.offsets[lane];
+  struct Late {
+    const GemmArgs& args;
+    int off_lane;
+    __device__ __forceinline__ void get(int g, int& rb, int& re) const {
+      const GemmGroup& gg = args.g[g];
+      if (gg.row_begin >= 0) { rb = gg.row_begin; re = gg.row_end; }
+      else { rb = __builtin_amdgcn_readlane(off_lane, gg.dyn); re = __builtin_amdgcn_readlane(off_lane, gg.dyn + 1); }
+    }
+    __device__ __forceinline__ int ntiles(int g, int feat) const { return args.g[g].n_out / feat; }
+  };
+  const Late late = {args, off_lane};
+  const Segments early(args, lane);
   int total = 0;
   for (int g = 0; g < args.G; ++g) {
     int rb, re;
-    segs.get(g, rb, re);
-    total += ((re - rb + W4_BM - 1) / W4_BM) * segs.ntiles(g, W4_FEAT);
+    early.get(g, rb, re);
+    total += ((re - rb + W4_BM - 1) / W4_BM) * early.ntiles(g, W4_FEAT);
   }
   const int per_xcd = (total + HDMOE_NUM_XCD - 1) / HDMOE_NUM_XCD;
   const int xcd = blockIdx.x % HDMOE_NUM_XCD, slot = blockIdx.x / HDMOE_NUM_XCD;
   const int nslots = gridDim.x / HDMOE_NUM_XCD;
   struct Tile4 { int g, row0, rows_here, n0; };
-  auto decode = [&](int i) -> Tile4 {
+  auto decode = [&](const auto& segs, int i) -> Tile4 {
     Tile4 d = {-1, 0, 0, 0};
     const int in_xcd = slot + i * nslots;
     int L = xcd * per_xcd + in_xcd;
@@ -73,11 +89,11 @@ __global__ __launch_bounds__(W4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     }
     if (g >= args.G) return d;
     const int nbands = max(1, (mtiles + GROUP_M / 2) / GROUP_M);
-    const int band = min(tile_div(L, GROUP_M * ntiles), nbands - 1);
+    const int band = min(L / (GROUP_M * ntiles), nbands - 1);
     const int first_m = band * GROUP_M;
     const int gm = band == nbands - 1 ? mtiles - first_m : GROUP_M;
     const int within = L - band * (GROUP_M * ntiles);
-    const int n = tile_div(within, gm);
+    const int n = within / gm;
     d.g = g;
     d.row0 = rb + (first_m + within - n * gm) * W4_BM;
     d.rows_here = min(re - d.row0, W4_BM);
@@ -90,9 +106,9 @@ __global__ __launch_bounds__(W4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   auto token_base = [&](const GemmGroup& gg) { return (use_alt && gg.gather != nullptr) ? args.alt.a : gg.a; };
   auto gather_shift = [&](const GemmGroup& gg) { return use_alt ? args.alt.shift : gg.gather_shift; };
 
-  Tile4 cur = decode(0);
+  Tile4 cur = decode(early, 0);
   if (cur.g < 0) return;   // block-uniform: every wave of the block leaves together
-  Tile4 nxt = decode(1);
+  Tile4 nxt = decode(early, 1);
 
   // ---- addressing ---------------------------------------------------------------------------------------------
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
@@ -233,7 +249,7 @@ __global__ __launch_bounds__(W4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     }
     if (nxt.g < 0) break;
     cur = nxt;
-    nxt = decode(i + 2);
+    nxt = decode(late, i + 2);
   }
   // ---- phase 2 of the last tile ------------------------------------------------------------------------------
   asm volatile(HDMOE4W_DRAIN_ASM

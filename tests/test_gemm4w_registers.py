@@ -1,4 +1,4 @@
-"""The built 4-wave kernels keep every value in registers (csrc/gemm4w.h, csrc/swiglu224.h).
+"""The built 4-wave kernels keep every value in registers (csrc/gemm4w.h, csrc/swiglu224.h, csrc/swiglu4w.h).
 
 Their statements use fixed registers that are free to the compiler in between. A spilled register tuple that is reloaded there
 and used in part is waited for in part: the rest arrives while a statement has the registers in use. So nothing may be
@@ -34,11 +34,11 @@ def test_no_kernel_of_the_4_wave_gemm_spills(tmp_path):
         notes = subprocess.run([READELF, "--notes", str(f)], capture_output=True, text=True, check=True).stdout
         for kernel in notes.split("- .agpr_count:")[1:]:
             name = re.search(r"\.name:\s+(\S+)", kernel).group(1)
-            if "gemm4w_kernel" in name or "swiglu224_kernel" in name:
+            if "gemm4w_kernel" in name or "swiglu224_kernel" in name or "swiglu4w_kernel" in name:
                 seen += 1
                 assert int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", kernel).group(1)) == 0, name
                 assert int(re.search(r"\.vgpr_spill_count:\s+(\d+)", kernel).group(1)) == 0, name
-    assert seen >= 15   # 14 forms of the one, the other
+    assert seen >= 16   # 14 forms of the first, the other two
 
 
 OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
