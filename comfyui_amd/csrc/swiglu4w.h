@@ -48,8 +48,9 @@ __global__ __launch_bounds__(W4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
 
   // ---- tile enumeration: as grouped_gemm_kernel with one tile list cut in eighths ---------------------------
   // The block's first two tiles come from the packed segments; the later ones, looked up behind K loops, from the arguments and one register of
-  // bounds: four registers of segments across the statements, which leave the compiler 32, had 207 spilled, fragments on their way among them (layers of 512 tokens
-  // 149 us, so 135; 900 200 -> 178; 1024 209 -> 189), and with tile_div in the later ones still 9.
+  // bounds. Four registers of segments across the statements, which leave the compiler 32, had row indices and offsets in memory, and their
+  // reloads wait for every request in flight: layers of 512 tokens 149 us, so 135, 900 200 -> 178, 1024 209 -> 189 (cold weights). With tile_div in
+  // the later look-ups still 9 registers.
   int off_lane = 0;
   if (args.offsets != nullptr && lane <= args.n_offsets) off_lane = args.offsets[lane];
   struct Late {
