@@ -1867,23 +1867,27 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
     return fixed(parts < 1 ? 1 : (int)parts);
   }
 
-  // A dense feed-forward in fp8 on the 4-wave kernel, whose tiles can be lower (gemm4w.h): parts on 128-token tiles, which fill more CUs with
-  // fewer parts. In hundredths of a pair of K steps (24.6 ns) as in g4_cap_cost; a part's sums written and read again at about 5 TB/s, 100
-  // for the kernel that adds them up. Whole branch, D = 2560, H = 6912, us, on 256-token tiles (6 to 2 parts) -> this: 300 rows 61.0 -> 53.7 (6 parts),
-  // 512 63.4 -> 56.7 (4), 768 67.9 -> 61.2 (3), 1024 85.9 -> 79.5 (3), 1536 104.2 -> 97.1 (2), 2048 138.2 -> 129.4 (not cut).
+  // A dense feed-forward in fp8 on the 4-wave kernel, whose tiles can be lower (gemm4w.h): parts on the lowest tiles that fill a round of CUs.
+  // In hundredths of a pair of K steps (24.6 ns) as in g4_cap_cost; a part's sums written and read again at about 5 TB/s, 100 for the kernel that
+  // adds them up. Whole tiles have 18 more per pair: each of their steps waits for the memory that cold weights come from (0.6 us a pair, nothing
+  // where the caches have them; parts share that wait). Whole branch, D = 2560, H = 6912, us, on 256-token tiles (6 to 3 parts) -> this, weights in the
+  // caches: 300 rows 61.0 -> 53.7 (6 parts), 512 63.4 -> 56.7 (4), 768 67.9 -> 61.2 (3), 1024 85.9 -> 79.5 (3), 1536 104.2 -> 97.1 (2). Beyond, cold and in
+  // the caches, on 256-token tiles, whole on lower ones, this: 1600 113.8 108.2, 120.2 103.5, 113.5 102.2; 1800 117.9 113.6, 121.1 106.2, 114.6 108.6;
+  // 2048 134.8 130.0, 138.7 120.7, 131.3 125.1 (192-token tiles); whole from 2176 rows on: 2300 142.4 135.3, 142.3 126.5.
   if (weight_dtype == HDMOE_W_E4M3FN && !dyn && kts % 2 == 0 && kts >= 4) {
-    constexpr int PAIR[5] = {58, 70, 80, 90, 100};
+    constexpr int PAIR[5] = {58, 70, 80, 90, 100}, COLD = 18;
     const int pairs = kts / 2;
     auto rounds = [&](int bm, int parts) { return ((long)(rows_static + bm - 1) / bm * nt * parts + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU; };
     double best_cost = 1e30;
-    int best = 1;
-    for (int h = 4; h <= 8; ++h) best_cost = fmin(best_cost, (double)rounds(32 * h, 1) * (pairs * PAIR[h - 4] + G4_TILE_COST));
+    int best = 1, height = 8;
+    for (int h = 4; h <= 8; ++h) best_cost = fmin(best_cost, (double)rounds(32 * h, 1) * (pairs * PAIR[h - 4] + G4_TILE_COST) + COLD * pairs);
     best_cost *= 0.95;   // a cut has to pay
-    for (int parts = 2; parts <= 6 && pairs / parts >= 3; ++parts) {
-      const double cost = (double)rounds(128, parts) * ((pairs + parts - 1) / parts * PAIR[0] + G4_TILE_COST) + (double)parts * rows_static * N * 8.0 / 123e3 + 100.0;
-      if (cost < best_cost) { best = parts; best_cost = cost; }
-    }
-    pl.bm = best > 1 ? 128 : TileCfg<4>::BM;
+    for (int parts = 2; parts <= 6 && pairs / parts >= 3; ++parts)
+      for (int h = 4; h <= 6; ++h) {
+        const double cost = (double)rounds(32 * h, parts) * ((pairs + parts - 1) / parts * PAIR[h - 4] + G4_TILE_COST) + (double)parts * rows_static * N * 8.0 / 123e3 + 100.0;
+        if (cost < best_cost) { best = parts; height = h; best_cost = cost; }
+      }
+    pl.bm = 32 * height;
     return fixed(best);
   }
   // A layer in fp8 on that kernel: the most parts whose tiles fit one round of blocks, on 128-token tiles with even segments, else on 256-token
