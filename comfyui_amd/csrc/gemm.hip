@@ -1873,7 +1873,7 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
   // where the caches have them; parts share that wait). Whole branch, D = 2560, H = 6912, us, on 256-token tiles (6 to 3 parts) -> this, weights in the
   // caches: 300 rows 61.0 -> 53.7 (6 parts), 512 63.4 -> 56.7 (4), 768 67.9 -> 61.2 (3), 1024 85.9 -> 79.5 (3), 1536 104.2 -> 97.1 (2). Beyond, cold and in
   // the caches, on 256-token tiles, whole on lower ones, this: 1600 113.8 108.2, 120.2 103.5, 113.5 102.2; 1800 117.9 113.6, 121.1 106.2, 114.6 108.6;
-  // 2048 134.8 130.0, 138.7 120.7, 131.3 125.1 (192-token tiles); whole from 2176 rows on: 2300 142.4 135.3, 142.3 126.5.
+  // 2048 134.8 130.0, 138.7 120.7, 131.3 125.1 (192-token tiles); whole from 2168 rows on: 2300 142.4 135.3, 142.3 126.5.
   if (weight_dtype == HDMOE_W_E4M3FN && !dyn && kts % 2 == 0 && kts >= 4) {
     constexpr int PAIR[5] = {58, 70, 80, 90, 100}, COLD = 18;
     const int pairs = kts / 2;
