@@ -151,8 +151,8 @@ def test_composed_path_matches_fused(dev):
     assert diff["rel_rms"] < 2e-3
 
 
-# cfg5-1024 is not a benchmark line: it is the size where the cut of the down projection is chosen on the device, with
-# a routing (one expert nearly empty, one heavy) under which no candidate cut fits one round of blocks
+# cfg5-1024 is not a benchmark line: its routing leaves one expert nearly empty and another heavy at a size where the down projection's
+# tiles are whole and the gate/up kernel is the 4-wave one on 256-token tiles
 @pytest.mark.parametrize("name", ["cfg1", "cfg2", "cfg3", "cfg5-256", "cfg5-1024", "cfg5-4096"])
 def test_benchmark_configs(dev, name):
     """The benchmark configurations at their full size: EVERY token of the output is compared with the oracle (an
@@ -548,17 +548,25 @@ def test_combine_over_the_partial_sums_of_a_cut_down_projection(dev, weights, to
     del keep
 
 
-def test_rows_do_not_depend_on_the_rest_of_the_batch_when_asked(dev):
-    """At 1024 tokens of HiDream's width the down projection is cut along K and the entry of the plan that runs is
-    picked on the device from the experts' segment sizes, so the fp32 summation order of a token's rows may follow the
+@pytest.mark.parametrize("weights", ["fp8", "bf16", "upcast"])
+def test_rows_do_not_depend_on_the_rest_of_the_batch_when_asked(dev, weights):
+    """At 1024 tokens of HiDream's width the down projection with 16-bit activations is cut along K where that fits one round of
+    blocks, which is decided on the device from the experts' segment sizes, so the fp32 summation order of a token's rows follows the
     routing of the other tokens. Two batches that share their first 256 tokens and route the other 768 differently
-    (evenly, with segments that do not fit the first candidate cut / all to the experts of one token, where it fits):
-    with `batch_invariant` set the cut is the same whatever the routing and the shared tokens come out byte for byte
-    the same. (Where both entries happen to hold the same cut they do so without the flag as well; the count printed
-    below says which.)"""
+    (evenly, with segments that do not fit the cut in (2, 1) parts, whose tiles are then left whole / all to the experts of one token,
+    where it fits): with `batch_invariant` set the cut is the same whatever the routing and the shared tokens come out byte for byte
+    the same; without it they do not, which says that both ran. In fp8 nothing is cut at this size and nothing depends on it. Either way
+    the ragged batch is as close to the oracle as other layers are."""
+    from comfyui_amd import _lib
+    from comfyui_amd import functional as HF
+    code = {"fp8": _lib.W_E4M3FN, "bf16": _lib.W_BF16, "upcast": _lib.W_E4M3FN_UPCAST}[weights]
+    lay = HF.layer_layout(1024, synth.DIM, synth.H_ROUTED, synth.H_SHARED, 4, code)
+    room = (lay.flags - lay.partials) // (3 * 1024 * synth.DIM * 4)
+    assert room == (0 if weights == "fp8" else 2)
     cfg = synth.make_config("cfg2")
-    sd = synth.to_state_dict(cfg["master"], "fp8")
-    m = synth.build_module({k: v.to(dev) for k, v in sd.items()}, "fp8", dev)
+    sd = synth.to_state_dict(cfg["master"], "bf16" if weights == "bf16" else "fp8", scale_input=weights == "fp8")
+    m = synth.build_module({k: v.to(dev) for k, v in sd.items()}, "bf16" if weights == "bf16" else "fp8", dev,
+                           fp8_matrix_mult=weights == "fp8", scale_input=weights == "fp8")
     xall = cfg["x"].reshape(-1, synth.DIM)
     tiles = lambda xs: int(sum(-(-int(c) // 256) for c in torch.bincount(
         O.gate_fixed_order(xs, sd["gate.weight"])[0].reshape(-1).long(), minlength=4)))
@@ -577,7 +585,10 @@ def test_rows_do_not_depend_on_the_rest_of_the_batch_when_asked(dev):
         outs[flag] = (ya, yb)
     differ = int((outs[False][0].view(torch.int16) != outs[False][1].view(torch.int16)).sum())
     print(f"\n{differ} of {256 * synth.DIM} outputs of the shared tokens differ between the batches without the flag")
+    assert (differ > 0) == (weights != "fp8")
     assert torch.equal(outs[True][0].view(torch.int16), outs[True][1].view(torch.int16))
-    ref = O.moe_forward(xa[:256].unsqueeze(0), oracle_params(sd, 4), "fp8mm")[0]
-    met = O.error_metrics(outs[True][0], ref)
-    assert met["rel_rms"] <= TOL_RMS_SAME_DATAFLOW["fp8"] and met["max_over_max"] <= TOL["fp8"], met
+    ref = O.moe_forward(xa[:256].unsqueeze(0), oracle_params(sd, 4), {"fp8": "fp8mm", "bf16": "plain", "upcast": "upcast"}[weights])[0]
+    kind = "bf16" if weights == "bf16" else "fp8"      # (upcast: a scaled operand is rounded by the oracle and not here)
+    for flag in (False, True):
+        met = O.error_metrics(outs[flag][0], ref)
+        assert met["rel_rms"] <= TOL_RMS_SAME_DATAFLOW[kind] and met["max_over_max"] <= TOL[kind], (flag, met)
