@@ -107,6 +107,7 @@ struct HdmoeSplitPlan {
   int pd[HDMOE_PLAN_MAX];    // K parts of a tile of the experts' groups
   int ps[HDMOE_PLAN_MAX];    // K parts of a tile of the static group (the shared expert)
   int bm;                    // tile height (tokens) the launch runs with
+  int bm_else;               // fp8: its height where the segments make more of those tiles than a round of blocks takes; 0 = the same
   int max_tiles;             // an entry before the last is taken only if its tiles number at most this
   int fixed_pd, fixed_ps;    // the cut where the segments' sizes may not decide (fixed_k_cut of the arguments)
 };

@@ -288,7 +288,14 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     }
     plan_idx = hdmoe_plan_pick(args.plan, mt_dyn, mt_static, segs.ntiles(0, FEAT));
   }
-  const int bm = EPI == G4_PARTIAL && F8 ? args.plan.bm : G4_BM;   // rows of a tile that is not capped
+  int bm = EPI == G4_PARTIAL && F8 ? args.plan.bm : G4_BM;   // rows of a tile that is not capped
+  if (EPI == G4_PARTIAL && F8 && args.plan.bm_else > 0) {    // (the plan has one entry)
+    const int parts = segs.fixed >> lane & 1 ? args.plan.ps[0] : args.plan.pd[0];
+    const int mine = tile_div(segs.re - segs.rb + bm - 1, bm) * (segs.n_out / FEAT) * parts;
+    int tiles = 0;
+    for (int g = 0; g < args.G; ++g) tiles += __builtin_amdgcn_readlane(mine, g);
+    if (tiles > HDMOE_NUM_CU) bm = args.plan.bm_else;
+  }
   auto parts_of = [&](int g) {
     return EPI != G4_PARTIAL ? 1 : segs.dynamic(g) ? args.plan.pd[plan_idx] : args.plan.ps[plan_idx];
   };

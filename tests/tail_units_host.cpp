@@ -1,4 +1,6 @@
 // Host-side export of comfyui_amd/csrc/tail_units.h for the CPU tests.
+#include <cmath>
+
 #include "../comfyui_amd/csrc/tail_units.h"
 extern "C" void t_tail_unit(int swiglu, int item, int wave, int tile, int* out) {
   const G4TailUnit u = g4_tail_unit(swiglu != 0, item, wave, tile);
@@ -9,3 +11,4 @@ extern "C" int t_place(int longs, int shorts, int light_rounds, int xcd, int slo
   const G4Place p = g4_place(longs, shorts, light_rounds, xcd, slot, i);
   return p.tile < 0 ? -1 : p.tile * 2 + (p.is_short ? 1 : 0);
 }
+extern "C" int t_cut_height(int bm, int rows, int n, int rows_static, int pd, int ps, int nt) { return g4_cut_height(bm, rows, n, rows_static, pd, ps, nt); }

@@ -48,3 +48,14 @@ def test_blocks_of_a_part_are_the_ones_with_rows(units):
     for rows in range(1, 257):
         for w in range(4):
             assert units.t_part_blocks(rows, w) == sum(tt * 32 + (w >> 1) * 16 < rows for tt in range(8))
+
+
+@pytest.mark.parametrize("tokens,want", [(300, 128), (450, 128), (475, 128), (482, 128), (484, 160), (500, 160), (512, 160)])
+def test_height_of_a_layers_cut_tiles(units, tokens, want):
+    """Four experts and a shared one in (2, 1) parts, 10 tiles along the features: three experts above 256 rows make 26 m-tiles of 128, one round
+    of blocks and four more."""
+    assert units.t_cut_height(128, 2 * tokens, 4, tokens, 2, 1, 10) == want
+    if want > 128:
+        over = [257, 257, 257, 2 * tokens - 771]
+        assert sum(-(-c // want) * 2 for c in over) + -(-tokens // want) <= 25
+    assert units.t_cut_height(256, 2 * tokens, 4, tokens, 2, 1, 10) == 256
