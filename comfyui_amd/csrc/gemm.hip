@@ -1435,12 +1435,12 @@ FormChoice pick_form(const GemmShape& sh) {
   // (16-bit weights: the gate/up contraction that stays with the 8-wave kernel, 2560 rows of 4 experts by 6912 features, K = 2624: 178
   // against 198 us; the down projection measured slower on the taller tile)
   c.tall = (sh.fp8 || (sh.swiglu && !sh.g4_takes)) && !sh.split && !c.light && expected_tile_cost(sh, 5) < expected_tile_cost(sh, 4);
-  // fp8 down projection on the 4-wave kernel, unless the 320-token tile saves more than a quarter of the rounds. Whole layer, 8- against
-  // 4-wave, us: cut along K 260 tokens 110, 103; 600 177, 169; 1024 226, 207; 1536 254, 240; 2000 304, 284; whole tiles 4000
-  // 537, 503; 5000 649, 624 (320-token tiles would take 0.8 of the rounds); 8000 969, 917; 2300 (0.6 of the rounds) 341, 349. Not with a
-  // forced form: the parts of a cut projection end elsewhere here (on pairs of K steps); uncut the bytes are the same.
-  c.fp8_g4 = sh.fp8 && !sh.swiglu && sh.g4_takes && !c.light && f_light == HDMOE_FORM_AUTO && f_4w == HDMOE_FORM_AUTO &&
-             !(c.tall && 4 * expected_tile_cost(sh, 5) < 3 * expected_tile_cost(sh, 4));
+  // fp8 down projection on the 4-wave kernel. Whole layer, 8- against 4-wave, us: cut along K 260 tokens 110, 103; 600 177, 169; 1024 226, 207; 1536
+  // 254, 240; 2000 304, 284; whole tiles 4000 537, 503; 5000 649, 624 (the 8-wave kernel's 320-token tiles would take 0.8 of the rounds of whole
+  // 256-token ones); 8000 969, 917. With 0.6 of their rounds too, now that tiles are as high as their rows need and of two lengths: 2100 tokens 279, 252;
+  // 2300 299, 279; 2560 346, 303, skewed 352, 306; dense branch of 6700 rows 300.1, 301.7, 8000 346.9, 344.3. Not with a forced form: the parts of a cut
+  // projection end elsewhere here (on pairs of K steps); uncut the bytes are the same.
+  c.fp8_g4 = sh.fp8 && !sh.swiglu && sh.g4_takes && !c.light && f_light == HDMOE_FORM_AUTO && f_4w == HDMOE_FORM_AUTO;
   if (c.fp8_g4) c.tall = false;
   c.short3 = !c.light && f_4w != HDMOE_FORM_ALWAYS && short_tile_pays(sh);
   if (f_light == HDMOE_FORM_AUTO && f_4w == HDMOE_FORM_AUTO && !c.light &&

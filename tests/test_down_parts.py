@@ -21,3 +21,9 @@ def test_parts(rows, want):
 
 def test_few_steps_are_not_cut():
     assert parts(1700, 512, 1280) == 1   # 5 pairs of K steps: no part has three
+
+
+@pytest.mark.parametrize("tokens", [1100, 2049, 2051, 2100, 2300, 2560, 2561, 4096, 8192])
+def test_whole_tiles_run_on_the_4_wave_kernel(tokens):
+    name = _lib.lib.hdmoe_plain_kernel_name(2 * tokens, 4, H, tokens, 3584, D, 1, 0)
+    assert name == b"gemm4w_kernel<F8, PLAIN>"

@@ -4,7 +4,7 @@ in eighths, and for fp8 as on the 8-wave kernels."""
 import pytest
 import torch
 
-from comfyui_amd import ops, synth
+from comfyui_amd import _lib, ops, synth
 from comfyui_amd.hidream import MOEFeedForwardSwiGLU
 from tests.helpers import saved_forms, set_form
 
@@ -46,9 +46,10 @@ def test_rows_are_those_of_a_larger_call(dev, forms, kind):
     with torch.no_grad():
         full = m(x)
         assert bool(torch.isfinite(full.float()).all()) and float(full.float().std()) > 0
-        for tokens in (1100, 1801, 2049, 2100, 2600, 3000, 4096, 4500, 5400):
+        for tokens in (1100, 1801, 2049, 2100, 2300, 2560, 2600, 3000, 4096, 4500, 5400):
+            if kind == "fp8":
+                assert _lib.lib.hdmoe_plain_kernel_name(2 * tokens, 4, synth.H_ROUTED, tokens, synth.H_SHARED, synth.DIM, 1, 0) == b"gemm4w_kernel<F8, PLAIN>"
             assert torch.equal(m(x[:, :tokens]), full[:, :tokens]), tokens
         if kind == "fp8":
             set_form("HDMOE_SWIGLU4W", "0")
             assert torch.equal(m(x[:, :3000]), full[:, :3000])
-
