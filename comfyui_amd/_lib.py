@@ -98,6 +98,8 @@ SIGNATURES = {
     "hdmoe_plain_kernel_name": (ctypes.c_char_p, [c_int] * 8),
     "hdmoe_tail_plan": (c_int, [c_int, c_int, c_int, c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_int)]),
     "hdmoe_linear_tile_rows": (c_int, [c_int, c_int, c_int, c_int]),
+    "hdmoe_fp8_linear_tile_rows": (c_int, [c_int, c_int, c_int]),
+    "hdmoe_two_lengths": (c_int, [c_int, ctypes.POINTER(c_int)] + [c_int] * 6 + [ctypes.POINTER(c_int)]),
     "hdmoe_gate_top2": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "hdmoe_gate_top2_f16": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "hdmoe_renorm_top2_bf16": (c_int, [c_void_p, c_int, c_void_p, c_void_p]),

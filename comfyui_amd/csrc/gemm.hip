@@ -2378,6 +2378,39 @@ extern "C" int hdmoe_linear_tile_rows(int weight_dtype, int rows, int K, int N) 
   return 32 * (cap > 0 ? g4_heights(rows, cap).height : G4_BM / 32);
 }
 
+// The same for a Linear on e4m3fn activations that the 4-wave kernel takes.
+extern "C" int hdmoe_fp8_linear_tile_rows(int rows, int K, int N) {
+  if (rows <= 0 || K <= 0 || N <= 0 || N % BN != 0 || K > 0x7fff * BK || K % BK != 0 || !g4_takes_k(0, 0, rows, K)) return 0;
+  GemmArgs args;
+  memset(&args, 0, sizeof(args));
+  args.G = 1;
+  args.g[0].row_end = rows;
+  args.g[0].n_out = N;
+  args.g[0].kbytes = K;
+  const int cap = g4_host_cap(args, BN, 2, HDMOE_NUM_CU);
+  return 32 * g4_heights(cap > 0 || rows < G4_BM ? rows : G4_BM, cap > 0 ? cap : G4_BM / 32).height;
+}
+
+// What g4_two_lengths makes of a layer's down projection (E segments of `rows` rows each and K elements of e4m3fn, one more of rows_static and
+// K_static): the longest block in hundredths of a pair of K steps, 0 for sizes it does not take. For tests and reports.
+extern "C" int hdmoe_two_lengths(int E, const int* rows, int K, int rows_static, int K_static, int N, int cap_long, int cap_short, int* light_rounds) {
+  auto cap_ok = [](int cap) { return cap >= G4_MIN_BLOCKS && cap <= G4_BM / 32; };
+  if (E <= 0 || E > HDMOE_MAX_EXPERTS || rows == nullptr || rows_static <= 0 || K <= 0 || K_static <= 0 || K % (2 * BK) != 0 || K_static % (2 * BK) != 0 ||
+      N <= 0 || N % BN != 0 || !cap_ok(cap_long) || !cap_ok(cap_short))
+    return 0;
+  struct Sizes {
+    int E, K, K_static, N, rows_static;
+    const int* of;
+    bool dynamic(int g) const { return g < E; }
+    int rows(int g) const { return g < E ? of[g] : rows_static; }
+    int bytes(int g) const { return g < E ? K : K_static; }
+    int ntiles(int, int feat) const { return N / feat; }
+  };
+  const G4Two t = g4_two_lengths(Sizes{E, K, K_static, N, rows_static, rows}, E + 1, K >= K_static ? 1 : -1, BN, cap_long, cap_short);
+  if (light_rounds != nullptr) *light_rounds = t.light_rounds;
+  return t.cost;
+}
+
 // Bytes a feed-forward's contractions on 16-bit activations can use for the parts of tail tiles: E experts of hidden width H on
 // rows_dyn rows together, one more of width Hs on rows_static. down_uncut: its down projection is not cut along K by itself.
 size_t hdmoe_tail_bytes(int weight_dtype, int rows_dyn, int E, int rows_static, int D, int H, int Hs, bool down_uncut) {

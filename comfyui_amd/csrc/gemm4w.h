@@ -32,7 +32,7 @@ constexpr int G4_TABLE = 131072;                  // LDS: [tok 0 | tok 1 | w 0 |
 constexpr int G4_TABLE_ITEMS = 64;                // items a wave's lanes look up at a time
 constexpr int G4_HEIGHTS = G4_TABLE + 4 * G4_TABLE_ITEMS * 16;   // 16 bytes per group
 constexpr int G4_SMEM = G4_HEIGHTS + MAX_GROUPS * 16;
-constexpr int G4_MIN_BLOCKS = 4;                  // least height of a tile of 16-bit activations, in token blocks of 32 rows
+constexpr int G4_MIN_BLOCKS = 4;                  // least height of a tile, in token blocks of 32 rows
 constexpr int G4_SCRATCH = 4 * 28 * 1024;         // GELU: bytes of scratch per block (28 pieces of 16 bytes per lane)
 constexpr int G4_GELU_PAIRS = 16;                 // pairs of K steps a deferred activation needs to hide behind
 
@@ -134,15 +134,17 @@ __device__ __forceinline__ G4Tail g4_tail_of(const GemmArgs& args, const Segment
 // high as their rows need without a cap too. Not for SWIGLU, whose two halves of the weights every further m-tile reads again: 1300 tokens
 // in bf16 361 -> 367 us, 1024 tokens 294 -> 298. More than 24 rounds: one is not worth the search.
 constexpr int G4_TILE_COST = 150, G4_CAP_ROUNDS = 24;
+__host__ __device__ __forceinline__ int g4_div(int a, int b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return tile_div(a, b);
+#else
+  return a / b;
+#endif
+}
 struct G4Heights { int mt, height; };
 __host__ __device__ __forceinline__ G4Heights g4_heights(int rows, int cap) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  auto div = [](int a, int b) { return tile_div(a, b); };
-#else
-  auto div = [](int a, int b) { return a / b; };
-#endif
-  const int units = (rows + 31) >> 5, mt = div(units + cap - 1, cap);
-  return {mt, max(div(units + mt - 1, max(mt, 1)), G4_MIN_BLOCKS)};
+  const int units = (rows + 31) >> 5, mt = g4_div(units + cap - 1, cap);
+  return {mt, max(g4_div(units + mt - 1, max(mt, 1)), G4_MIN_BLOCKS)};
 }
 
 // What a cap comes to; rows(g), ntiles(g): the rows of group g, its tiles along the features.
@@ -202,12 +204,12 @@ __device__ __forceinline__ int g4_cap(const GemmArgs& args, const Segments& seg,
 // long one, and what is left goes round by round over all, light blocks first (g4_place). Groups are long or short by args.spread.
 // The caps are those of the shortest longest block; others than whole tiles have to pay by a twelfth in fp8, an eighth in 16 bits (two rounds
 // of 7 blocks and more, 90 % of the cost, take as long: the clock falls with the CUs that are busy). Layers of 4 experts with K = 6912 and a
-// shared one with 3584, every XCD an eighth of every group -> this, us: fp8, 2600 tokens 319 -> 311, 3000 357 -> 344, 3500 405 -> 398, 4096 the
-// same, 4500 517 -> 499, 5000 549 -> 534; e4m3fn weights in bf16, 2100 491 -> 438, 3000 616 -> 588, 4080 the same; bf16, 2100 520 -> 468, 3000
+// shared one with 3584, every XCD an eighth of every group -> this, us: fp8, 2600 tokens 319 -> 311, 3000 357 -> 344, 3500 405 -> 398, 4096 460 ->
+// 450, 4500 517 -> 499, 5000 549 -> 534; e4m3fn weights in bf16, 2100 491 -> 438, 3000 616 -> 588, 4080 the same; bf16, 2100 520 -> 468, 3000
 // 655 -> 637. With more than 448 long tiles the eighths are better or equal (fp8 8192 tokens 821 -> 826, 12000 1167 -> 1177).
 struct G4Two { int cost, light_rounds; };
 template <class Segs>
-__device__ __forceinline__ G4Two g4_two_lengths(const Segs& seg, int G, int spread, int feat, int cap_long, int cap_short) {
+__host__ __device__ __forceinline__ G4Two g4_two_lengths(const Segs& seg, int G, int spread, int feat, int cap_long, int cap_short) {
   constexpr int PAIR[5] = {58, 70, 80, 90, 100}, BLOCKS = HDMOE_NUM_CU;
   int n[5] = {0, 0, 0, 0, 0}, shorts = 0, top = 0, pairs_long = 0, pairs_short = 0;
   for (int g = 0; g < G; ++g) {
@@ -229,7 +231,7 @@ __device__ __forceinline__ G4Two g4_two_lengths(const Segs& seg, int G, int spre
     at = to;
   }
   const int left = at % BLOCKS, lights = BLOCKS - left, light = left > 0 ? heavy - last : heavy;
-  const int light_rounds = left > 0 ? tile_div(last, each) : 0;
+  const int light_rounds = left > 0 ? g4_div(last, each) : 0;
   const int rest = shorts - light_rounds * lights;
   if (rest <= 0) return {heavy, light_rounds};
   const int q = rest / BLOCKS, r = rest % BLOCKS;

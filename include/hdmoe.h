@@ -111,6 +111,13 @@ int hdmoe_tail_plan(int weight_dtype, int tiles, int K, int padding, int* rounds
  * no tile is cut along K and lower tiles fill the CUs' rounds better; 0 = sizes that its kernel does not take. weight_dtype
  * HDMOE_W_BF16, HDMOE_W_F16 or HDMOE_W_E4M3FN_UPCAST. For tests and reports. No counterpart in the reference. */
 int hdmoe_linear_tile_rows(int weight_dtype, int rows, int K, int N);
+/* The same for a Linear on e4m3fn activations, whose tiles are as high as their rows need. */
+int hdmoe_fp8_linear_tile_rows(int rows, int K, int N);
+/* The longest block of a layer's fp8 down projection (E segments of rows[e] rows and K elements, rows_static and K_static of one more)
+ * on tiles of up to cap_long and cap_short blocks of 32 rows (4 to 8), dealt out by their length, in hundredths of a pair of K steps of a
+ * 256-row tile; and how many rounds of shorter tiles blocks take that have no longer one in the last round of those. 0 = sizes out of
+ * range. For tests and reports. No counterpart in the reference. */
+int hdmoe_two_lengths(int E, const int* rows, int K, int rows_static, int K_static, int N, int cap_long, int cap_short, int* light_rounds);
 
 /* ---- stage entry points ------------------------------------------------------ */
 

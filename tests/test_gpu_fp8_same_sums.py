@@ -24,7 +24,7 @@ def codes(shape, g, dev):
 
 @pytest.mark.parametrize("with_bias", [False, True])
 @pytest.mark.parametrize("K,N,sizes", [
-    (2560, 2560, (1, 300, 4800, 4801, 6400, 6401)),     # 128-, 192-, 256- and 320-token tiles of the 8-wave kernels, the 4-wave one
+    (2560, 2560, (1, 300, 4800, 4801, 6400, 6401)),     # tiles of 128 to 256 tokens of the 4-wave kernel; test_forms has the 8-wave ones
     (512, 10240, (100, 1100, 1281, 2300)),
     (4096, 2560, (200, 6400, 6401)),
 ])

@@ -10,13 +10,20 @@ pytestmark = pytest.mark.gpu
 BF16 = torch.bfloat16
 
 
-# 10 or 40 n-tiles; the heights that the cost model picks (csrc/gemm4w.h, g4_best_cap) and the last tile's are 4 to 8 blocks of 32
+HEIGHTS = {(3333, 512, 2560): 160, (4161, 768, 2560): 192, (4480, 2560, 2560): 192, (9001, 512, 2560): 192, (5600, 2560, 2560): 224, (1185, 512, 10240): 256,
+           (1300, 768, 10240): 256, (5000, 512, 2560): 256, (6305, 768, 2560): 256}   # the others 128
+
+
+# (up to 256 rows without a bias are the 8-wave kernel's) 10 or 40 n-tiles; the heights that the cost model picks (csrc/gemm4w.h, g4_best_cap), the last tile's may be lower
 @pytest.mark.parametrize("with_bias", [False, True])
-@pytest.mark.parametrize("rows,k,n", [(1, 512, 2560), (128, 768, 2560), (129, 512, 2560), (257, 2560, 10240), (700, 768, 2560), (1185, 512, 10240),
+@pytest.mark.parametrize("rows,k,n", [(5600, 2560, 2560), (1, 512, 2560), (128, 768, 2560), (129, 512, 2560), (257, 2560, 10240), (700, 768, 2560), (1185, 512, 10240),
                                       (1300, 768, 10240), (2000, 2560, 2560), (3333, 512, 2560), (4161, 768, 2560), (4480, 2560, 2560),
                                       (5000, 512, 2560), (6305, 768, 2560), (9001, 512, 2560)])
 def test_linear(dev, rows, k, n, with_bias):
     from comfyui_amd import functional as HF
+    assert _lib.lib.hdmoe_fp8_linear_tile_rows(rows, k, n) == HEIGHTS.get((rows, k, n), 128)
+    name = "gemm4w_kernel<F8, BIAS>" if with_bias else "gemm4w_kernel<F8, PLAIN>" if rows > 256 else "grouped_gemm_kernel<FP8_PLAIN, 4, LIGHT>"
+    assert _lib.lib.hdmoe_plain_kernel_name(0, 0, 0, rows, k, n, 1, int(with_bias)).decode() == name
     a, w = operands(rows, n, k, rows + k, dev)
     bias = torch.randn(n, generator=torch.Generator().manual_seed(3)).to(BF16).to(dev) if with_bias else None
     sw, si = torch.tensor(0.0007, device=dev), torch.tensor(0.6, device=dev)

@@ -42,3 +42,40 @@ def test_a_last_round_is_spread_over_the_xcds(place):
     for left in (8, 80, 129, 250):
         per_xcd = [sum(place(256 + left, 0, 0, xcd, slot, 1) >= 0 for slot in range(32)) for xcd in range(8)]
         assert sum(per_xcd) == left and max(per_xcd) == -(-left // 8)
+
+
+def heights(rows, cap):
+    blocks = -(-rows // 32)
+    mt = -(-blocks // cap)
+    return mt, max(4, -(-blocks // mt)) if mt else 4
+
+
+@pytest.mark.parametrize("seed", range(60))
+def test_the_longest_block_is_what_the_model_says(place, seed):
+    """csrc/gemm4w.h, g4_two_lengths, against the blocks that g4_place fills: long tiles from the highest to the lowest, short ones priced alike."""
+    from comfyui_amd import _lib
+    PAIR = {4: 58, 5: 70, 6: 80, 7: 90, 8: 100}
+    rng = random.Random(seed)
+    E, N = rng.choice([2, 4, 8, 16]), 256 * rng.choice([2, 8, 10])
+    K, Ks = rng.choice([(6912, 3584), (3584, 6912), (2560, 512), (512, 1024)])
+    T = rng.randint(300, 5000)
+    cuts = sorted(rng.randint(0, 2 * T) for _ in range(E - 1))
+    rows = [b - a for a, b in zip([0] + cuts, cuts + [2 * T])]
+    for cap_long, cap_short in ((8, 8), (4, 4), (5, 8), (7, 6)):
+        rounds = ctypes.c_int()
+        got = _lib.lib.hdmoe_two_lengths(E, (ctypes.c_int * E)(*rows), K, T, Ks, N, cap_long, cap_short, ctypes.byref(rounds))
+        groups = [(r, K) for r in rows] + [(T, Ks)]
+        kl, ks = max(K, Ks), min(K, Ks)
+        tiles = {k: sorted((h for r, kk in groups if kk == k for mt, h in [heights(r, cap_long if k == kl else cap_short)] for _ in range(mt * N // 256)),
+                           reverse=True) for k in (kl, ks)}
+        price = lambda k, h: k // 256 * PAIR[h] + 150
+        short = price(ks, tiles[ks][0])
+        longest = 0
+        for xcd in range(8):
+            for slot in range(32):
+                cost, i = 0, 0
+                while (v := place(len(tiles[kl]), len(tiles[ks]), rounds.value, xcd, slot, i)) >= 0:
+                    # a round of long tiles takes what its first one does
+                    cost, i = cost + (short if v & 1 else price(kl, tiles[kl][(v >> 1) // 256 * 256])), i + 1
+                longest = max(longest, cost)
+        assert got == longest, (rows, T, K, Ks, N, cap_long, cap_short)

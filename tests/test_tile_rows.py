@@ -1,4 +1,4 @@
-"""The height of the tiles of a 16-bit Linear (csrc/gemm4w.h, g4_best_cap) against its cost model written out: rounds over 256 CUs, the
+"""The height of the tiles of a Linear (csrc/gemm4w.h, g4_best_cap) against its cost model written out: rounds over 256 CUs, the
 highest tiles first, a pair of K steps priced by the height of the round's first tile."""
 import random
 
@@ -57,3 +57,29 @@ def test_sizes_out_of_range():
     assert tile_rows(_lib.W_BF16, 1000, 2624, 2560) == 0
     assert tile_rows(_lib.W_BF16, 1000, 2560, 2500) == 0
     assert tile_rows(_lib.W_BF16, 0, 2560, 2560) == 0
+
+
+def test_fp8_heights_are_the_cost_model():
+    """No tile is cut, and without a cap a tile is as high as its rows need."""
+    rng = random.Random(8)
+    seen = set()
+    for _ in range(20000):
+        rows = int(2 ** rng.uniform(0, 16))
+        K = 256 * rng.choice([rng.randint(2, 20), rng.randint(2, 60)])
+        N = 256 * rng.randint(1, 40)
+        pairs, nt, blocks = K // 256, N // 256, -(-rows // 32)
+        whole = -(-(-(-rows // 256) * nt) // CUS)
+        want, limit = max(4, min(8, blocks)), whole * (100 * pairs + 150)
+        limit -= limit // 12
+        for cap in (8, 7, 6, 5, 4):
+            mt = -(-blocks // cap)
+            height = max(4, -(-blocks // mt))
+            cost = -(-mt * nt // CUS) * (pairs * PAIR[height] + 150)
+            if whole <= 24 and cost < limit:
+                want, limit = height, cost
+        got = _lib.lib.hdmoe_fp8_linear_tile_rows(rows, K, N)
+        assert got == 32 * want, (rows, K, N)
+        seen.add(got)
+    assert seen == {128, 160, 192, 224, 256}
+    for bad in ((0, 2560, 2560), (1000, 384, 2560), (1000, 256, 2560), (1000, 2560, 2500)):
+        assert _lib.lib.hdmoe_fp8_linear_tile_rows(*bad) == 0
