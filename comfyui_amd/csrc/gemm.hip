@@ -1534,8 +1534,9 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
   const int eb = elem_bytes(weight_dtype);
   const bool fp8 = weight_dtype == HDMOE_W_E4M3FN;
   const int feat_per_tile = swiglu ? BN / 2 : BN;
-  // Split K (runs on the 256-token tile, or the 128-token one of the light form): nparts = the most parts any entry of
-  // the plan cuts a tile into (the partial-sum buffer holds that many); no plan = every tile in nparts parts
+  // Split K (on the 128-token tile of the light form; fp8 on the 4-wave kernel: tiles of plan->bm tokens, 128 to 256; else the
+  // 256-token tile): nparts = the most parts any entry of the plan cuts a tile into (the partial-sum buffer holds that many); no plan =
+  // every tile in nparts parts
   const bool split = !swiglu && partial != nullptr && nparts > 1;
   GemmShape shape;
   shape.swiglu = swiglu; shape.fp8 = fp8; shape.split = split; shape.w8 = w8;

@@ -291,11 +291,11 @@ class MOEFeedForwardSwiGLU(nn.Module):
         self.num_activated_experts = num_activated_experts
 
     # Not an attribute of the reference class. Set `module.batch_invariant = True` to have every token's output bytes
-    # independent of how the other tokens of the batch are routed: between a few hundred and about two thousand tokens
-    # the down projection is cut along K, and with 16-bit activations the tiles that either contraction has left over
-    # after whole rounds are, at any number of tokens; the cut that runs is otherwise picked from the experts' segment
-    # sizes, which changes the fp32 summation order (the last bit of an output) with the rest of the batch. Holds for the
-    # one-call path.
+    # independent of how the other tokens of the batch are routed: up to about a thousand tokens the down projection is
+    # cut along K, and with 16-bit activations the tiles that either contraction has left over after whole rounds are, at any
+    # number of tokens; with 16-bit activations (fp8: under 150 rows per expert) the cut that runs is otherwise picked from the
+    # experts' segment sizes, which changes the fp32 summation order (the last bit of an output) with the rest of the
+    # batch. Holds for the one-call path.
 
     # ---- fused path ----------------------------------------------------------------
 

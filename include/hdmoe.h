@@ -415,14 +415,14 @@ typedef struct hdmoe_layer_args {
    * two factors differ it writes NaN rows (the output of the call is then NaN, not a wrong number) and sets this
    * word to 1. A caller that caches its comparison of the values can poll the word and drop the cache. */
   int32_t* scale_check;
-  /* With a few hundred to about two thousand tokens the down projection is cut along K, and which of the candidate
-   * cuts runs is chosen on the device from the experts' segment sizes (the cut that fills one round of blocks). With
-   * 16-bit activations (HDMOE_W_BF16, HDMOE_W_E4M3FN_UPCAST) the same holds at any T for the tiles that both contractions
-   * have left over after whole rounds over the chip. The fp32 summation order of a row then depends on how the OTHER
+  /* Up to about 500 rows per expert (at the headline's widths 1000 tokens of 4 experts) the down projection is cut along K. With 16-bit activations (HDMOE_W_BF16, HDMOE_W_E4M3FN_UPCAST), and in fp8 under 150 rows per expert, which of the
+   * candidate cuts runs is chosen on the device from the experts' segment sizes (the cut that fills one round of blocks); elsewhere
+   * the sizes alone say. With 16-bit activations the tiles that both contractions have left over after whole rounds over the
+   * chip are cut by the segment sizes too, at any T. The fp32 summation order of a row then depends on how the OTHER
    * tokens of the batch were routed: the same token can differ in the last bit of its output between two batches. Nonzero
    * here fixes the cut from the sizes alone (the down projection's by the cost model, no tile of a last round), which
-   * makes every row's bytes a function of that row, its expert's weights and T only, at 2 to 10 % of the layer's time
-   * at those sizes (bf16 weights: 400 tokens 189 -> 211 us, 768 tokens 255 -> 280 us, from 1024 on no difference). */
+   * makes every row's bytes a function of that row, its expert's weights and T only, at 10 to 15 % of the layer's time where candidates
+   * are given up (bf16 weights: 400 tokens 177 -> 200 us, 768 tokens 241 -> 270 us; from 1000 on, and in fp8 at any T, no difference). */
   int fixed_k_cut;
 } hdmoe_layer_args;
 
