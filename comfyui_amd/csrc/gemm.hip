@@ -1892,17 +1892,16 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
     return fixed(best);
   }
   // A layer in fp8 on that kernel: the most parts whose tiles fit one round of blocks, on 128-token tiles with even segments (the device takes
-  // higher ones where its segments do not fit, g4_cut_height), else on 256-token tiles with segments a standard deviation above the
-  // mean; beyond that none (g4_two_lengths deals the tiles out). The shared expert's tiles in as many parts as make them about as long.
-  // Whole layer, us, candidates on 256-token tiles of which the device took the first that fitted (one at most sizes, seven around 500 tokens) -> this
-  // (three inputs each): 350 tokens 118 -> 113 ((2, 1) parts of 128), 400 123 -> 118, 450 150 -> 143, 500 147 -> 144, 640 145 -> 141 ((2, 1) of 256;
-  // of 128 in two rounds 164, whole tiles 157), 768 158 -> 156, 900 202 -> 199, 1024 209 -> 204 (whole), 1600 the same, 2000 266 -> 248. Not under 150
-  // rows an expert: 300 tokens 106, 106, 260 103, 105.
+  // higher ones where its segments do not fit, g4_cut_height), else on 256-token tiles with segments a standard deviation above the mean
+  // (g4_likely_tiles; width 4096, 500 tokens: (2, 1) parts 271 us, whole tiles 290); beyond that none (g4_two_lengths deals the tiles out).
+  // The shared expert's tiles in as many parts as make them about as long. Whole layer, us, candidates on 256-token tiles of which the device
+  // took the first that fitted (one at most sizes, seven around 500 tokens) -> this (three inputs each): 350 tokens 118 -> 113 ((2, 1) parts of
+  // 128), 400 123 -> 118, 450 150 -> 143, 500 147 -> 144, 640 145 -> 141 ((2, 1) of 256; of 128 in two rounds 164, whole tiles 157), 768 158 ->
+  // 156, 900 202 -> 199, 1024 209 -> 204 (whole), 1600 the same, 2000 266 -> 248. Not under 150 rows an expert: 300 tokens 106, 106, 260 103, 105.
   if (weight_dtype == HDMOE_W_E4M3FN && dyn && rows_static > 0 && rows_dyn >= 150 * n_dyn && ktd % 2 == 0 && kts % 2 == 0 && ktd >= 4 && kts >= 4) {
-    const double mu = (double)rows_dyn / n_dyn;
     for (int bm : {128, 256}) {
-      const int seg = bm == 128 ? (rows_dyn + n_dyn - 1) / n_dyn : (int)(mu + sqrt(mu));
-      const int mt_d = n_dyn * ((seg + bm - 1) / bm), mt_s = (rows_static + bm - 1) / bm;
+      const int mt_d = bm == 128 ? n_dyn * (((rows_dyn + n_dyn - 1) / n_dyn + bm - 1) / bm) : g4_likely_tiles(rows_dyn, n_dyn, bm);
+      const int mt_s = (rows_static + bm - 1) / bm;
       for (int pd = 6; pd >= 2; --pd) {
         const int ps = (int)fmin(fmax((double)pd * kts / ktd + 0.5, 1.0), (double)pd);
         if (ktd / 2 / pd < 3 || kts / 2 / ps < 3 || (mt_d * pd + mt_s * ps) * nt > HDMOE_NUM_CU) continue;

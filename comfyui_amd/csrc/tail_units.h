@@ -44,15 +44,21 @@ HDMOE_TAIL_HD G4Place g4_place(int longs, int shorts, int light_rounds, int xcd,
   return {true, tile < shorts ? tile : -1};
 }
 
+// The m-tiles of bm rows that n segments of `rows` rows together are counted as: each a standard deviation above the mean, and no more than
+// that many rows can make (four segments of 1024 rows: 7 of 256 rows, where each counted for itself would have two).
+inline int g4_likely_tiles(int rows, int n, int bm) {
+  const double mu = (double)rows / n;
+  const int each = n * (((int)(mu + std::sqrt(mu)) + bm - 1) / bm), most = rows > n ? (rows - n) / bm + n : rows;
+  return each < most ? each : most;
+}
+
 // The height of the tiles of a layer's down projection cut in pd / ps parts, `bm` or the next multiple of 32 with which n segments of `rows`
-// rows together, each a standard deviation above the mean, and the shared expert's `rows_static` fit one round of 256 blocks (nt tiles along
+// rows together (g4_likely_tiles) and the shared expert's `rows_static` fit one round of 256 blocks (nt tiles along
 // the features). Where it is not bm the device takes it if the segments' own tiles of bm rows are more than a round: the parts, and with them
 // the bytes, are the same. fp8 layers of 4 experts in (2, 1) parts, 128-token tiles -> this, us, three experts above 256 rows (one
 // input in seven at 512 tokens): 512 tokens 143 -> 135, 500 146 -> 133; fewer above 256 134.0 and 134.0, skewed 131.0 and 131.4. (Higher tiles whatever the
 // segments: skewed 134.)
 inline int g4_cut_height(int bm, int rows, int n, int rows_static, int pd, int ps, int nt) {
-  const double mu = (double)rows / n;
-  const int seg = (int)(mu + std::sqrt(mu));
-  while (bm < 256 && (n * ((seg + bm - 1) / bm) * pd + (rows_static + bm - 1) / bm * ps) * nt > 256) bm += 32;
+  while (bm < 256 && (g4_likely_tiles(rows, n, bm) * pd + (rows_static + bm - 1) / bm * ps) * nt > 256) bm += 32;
   return bm;
 }

@@ -27,3 +27,16 @@ def test_few_steps_are_not_cut():
 def test_whole_tiles_run_on_the_4_wave_kernel(tokens):
     name = _lib.lib.hdmoe_plain_kernel_name(2 * tokens, 4, H, tokens, 3584, D, 1, 0)
     assert name == b"gemm4w_kernel<F8, PLAIN>"
+
+
+def layer_parts(tokens, dim, h, hs, experts=4):
+    from comfyui_amd import functional as HF
+    lay = HF.layer_layout(tokens, dim, h, hs, experts, _lib.W_E4M3FN)
+    return (lay.flags - lay.partials) // (3 * tokens * dim * 4) or 1
+
+
+@pytest.mark.parametrize("dim,h,hs,tokens,want", [(2560, 6912, 3584, 512, 2), (2560, 6912, 3584, 960, 2), (2560, 6912, 3584, 1024, 1), (4096, 11008, 5632, 470, 3),
+                                                  (4096, 11008, 5632, 490, 2), (4096, 11008, 5632, 512, 2), (4096, 11008, 5632, 520, 1)])
+def test_parts_of_a_layer(dim, h, hs, tokens, want):
+    """Four experts of just under 256 rows make 7 tiles of 256 rows at most, not 8: two parts fit a round at width 4096."""
+    assert layer_parts(tokens, dim, h, hs) == want

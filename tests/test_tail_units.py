@@ -59,3 +59,14 @@ def test_height_of_a_layers_cut_tiles(units, tokens, want):
         over = [257, 257, 257, 2 * tokens - 771]
         assert sum(-(-c // want) * 2 for c in over) + -(-tokens // want) <= 25
     assert units.t_cut_height(256, 2 * tokens, 4, tokens, 2, 1, 10) == 256
+
+
+def test_likely_tiles_are_no_more_than_the_rows_make(units):
+    """Segments a standard deviation above the mean, against the most m-tiles of every division of the rows."""
+    assert [units.t_likely_tiles(2 * t, 4, 256) for t in (470, 490, 512, 600, 1000, 1024)] == [4, 7, 7, 8, 11, 11]
+    for rows, n, bm in ((9, 2, 4), (12, 3, 4), (13, 3, 4), (8, 4, 4), (2, 4, 4), (0, 3, 4), (17, 3, 8)):
+        def divisions(left, k):
+            return [(left,)] if k == 1 else [(a, *rest) for a in range(left + 1) for rest in divisions(left - a, k - 1)]
+        most = max(sum(-(-c // bm) for c in d) for d in divisions(rows, n))
+        mu = rows / n
+        assert units.t_likely_tiles(rows, n, bm) == min(most, n * -(-int(mu + mu ** 0.5) // bm))
