@@ -1875,6 +1875,7 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
   // caches: 300 rows 61.0 -> 53.7 (6 parts), 512 63.4 -> 56.7 (4), 768 67.9 -> 61.2 (3), 1024 85.9 -> 79.5 (3), 1536 104.2 -> 97.1 (2). Beyond, cold and in
   // the caches, on 256-token tiles, whole on lower ones, this: 1600 113.8 108.2, 120.2 103.5, 113.5 102.2; 1800 117.9 113.6, 121.1 106.2, 114.6 108.6;
   // 2048 134.8 130.0, 138.7 120.7, 131.3 125.1 (192-token tiles); whole from 2168 rows on: 2300 142.4 135.3, 142.3 126.5.
+  // Width 4096, 1700 rows: 207 202, 222 194, 207 202 (two parts on 224-token tiles); 1000 rows 147 141 on 256-token tiles in four parts, 153 137 here (two of 128).
   if (weight_dtype == HDMOE_W_E4M3FN && !dyn && kts % 2 == 0 && kts >= 4) {
     constexpr int PAIR[5] = {58, 70, 80, 90, 100}, COLD = 18;
     const int pairs = kts / 2;
@@ -1884,7 +1885,7 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
     for (int h = 4; h <= 8; ++h) best_cost = fmin(best_cost, (double)rounds(32 * h, 1) * (pairs * PAIR[h - 4] + G4_TILE_COST) + COLD * pairs);
     best_cost *= 0.95;   // a cut has to pay
     for (int parts = 2; parts <= 6 && pairs / parts >= 3; ++parts)
-      for (int h = 4; h <= 6; ++h) {
+      for (int h = 4; h <= 8; ++h) {
         const double cost = (double)rounds(32 * h, parts) * ((pairs + parts - 1) / parts * PAIR[h - 4] + G4_TILE_COST) + (double)parts * rows_static * N * 8.0 / 123e3 + 100.0;
         if (cost < best_cost) { best = parts; height = h; best_cost = cost; }
       }

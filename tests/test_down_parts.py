@@ -19,6 +19,12 @@ def test_parts(rows, want):
     assert parts(rows) == want
 
 
+@pytest.mark.parametrize("rows,want", [(1536, 2), (1537, 2), (1700, 2), (1793, 1)])
+def test_parts_on_tiles_of_any_height(rows, want):
+    """At width 4096 only 224- and 256-token tiles in two parts fit a round there; whole ones on 128-token tiles wait for cold weights."""
+    assert parts(rows, 4096, 11008) == want
+
+
 def test_few_steps_are_not_cut():
     assert parts(1700, 512, 1280) == 1   # 5 pairs of K steps: no part has three
 

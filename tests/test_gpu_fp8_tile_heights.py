@@ -55,9 +55,9 @@ def test_segments(dev, sizes, k):
 
 
 @pytest.mark.parametrize("rows,dim,hidden", [(257, 2560, 6912), (300, 512, 3584), (513, 2560, 6912), (768, 2560, 2560), (1300, 2560, 6912), (1700, 2560, 6912), (2048, 2560, 6912),
-                                             (2600, 2560, 6912)])
+                                             (2600, 2560, 6912), (1700, 4096, 11008)])
 def test_dense_feed_forward(dev, rows, dim, hidden):
-    """Down projections in parts of 128-, 160- and 192-token tiles and whole, against the product of the h left in the workspace."""
+    """Down projections in parts of 128-, 160-, 192- and 224-token tiles and whole, against the product of the h left in the workspace."""
     import ctypes
     L = _lib.lib
     FP8 = torch.float8_e4m3fn
