@@ -39,6 +39,7 @@
 
 #include "common.h"
 #include "numfmt.h"
+#include "tail_units.h"
 
 namespace {
 
@@ -434,14 +435,15 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_kernel(const GemmArgs a
       // Groups whose tiles differ in length (the K of the shared expert's down projection is about half the
       // routed experts'): every XCD takes its eighth of every group, longest tiles first, so each block gets
       // the same mix and the blocks end together.
-      int k = 0;
+      int k = 0, end = 0;
       for (; k < args.G; ++k) {
         g = args.spread > 0 ? k : args.G - 1 - k;
         seg(args.g[g], g, rb, re);
         mtiles = (re - rb + BM - 1) / BM;
         ntiles = ntiles_of(g);
-        const long long tiles = (long long)mtiles * ntiles * parts_of(g);
-        const int lo = (int)(xcd * tiles / HDMOE_NUM_XCD), hi = (int)((xcd + 1) * tiles / HDMOE_NUM_XCD);
+        const int from = end;
+        end += mtiles * ntiles * parts_of(g);
+        const int lo = g4_dealt(end, xcd) - g4_dealt(from, xcd), hi = g4_dealt(end, xcd + 1) - g4_dealt(from, xcd + 1);
         if (in_xcd < hi - lo) { L = lo + in_xcd; break; }
         in_xcd -= hi - lo;
       }
@@ -1845,11 +1847,14 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
   if ((!dyn && rows_static <= 0) || nt <= 0 || (ktd <= 0 && kts <= 0)) return fixed(1);
 
   // Few rows per segment (the rule of the light form in hdmoe_launch_ffn_gemm): the launch runs on 128-token
-  // tiles with K steps requested two ahead, and is bound by how fast the weights arrive, not by its K loops. About 150
-  // blocks keep enough loads in flight; more parts only add partial sums. The mean segment sits near the tile height,
-  // so segments are counted 1.5 times the mean: an expert that needs a second m-tile must not push the launch into a
-  // second round of blocks. (Whole layer, uniform / skewed routing, 256 tokens: 2 parts 99 / 102 us, 3 parts 95 / 110
-  // us; 128 tokens: 2 parts 88, 3 parts 81, 5 parts 96 us.)
+  // tiles with K steps requested two ahead, and is bound by how fast the weights arrive, not by its K loops. A layer: the most parts whose
+  // tiles fit one round of blocks however the rows fall to the experts (the sizes alone say, so that a row's sums do not depend on the
+  // others' routing), the shared expert's tiles in as many as make them about as long, rounded up first. Three parts of every tile up to 128
+  // tokens, two up to 256 -> this (weights from memory; two inputs each), us: fp8, 16 tokens 69.0 64.2 -> 66.7 61.3, 64 73.0 70.8 -> 70.2 67.1, 128
+  // 77.8 77.3 -> 75.0 74.4, 256 99.2 95.7 -> 94.0 91.4; bf16, 64 115.9 110.1 -> 110.3 102.4, 256 157.1 148.3 -> 146.2 139.9; e4m3fn weights in bf16,
+  // 64 109.4 108.6 -> 100.0 98.7, 256 134.6 135.3 -> 121.3 120.4. (Five parts of every tile, the shared expert's too: 64 tokens in fp8 72.3; the
+  // most parts that fit the real segments, picked on the device: 256 tokens 95.1, 200 89.0 where this has 90.8.)
+  // A dense feed-forward, and what fits no round: about 150 blocks keep enough loads in flight; segments counted 1.5 times the mean.
   if (hdmoe_few_rows(rows_dyn, n_dyn, rows_static)) {
     const int bm2 = TileCfg<2>::BM;
     pl.bm = bm2;
@@ -1865,6 +1870,19 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
     if (parts > HDMOE_NUM_CU / t2) parts = HDMOE_NUM_CU / t2;
     if (parts > 6) parts = 6;
     while (parts > 1 && kt2 / parts < 6) --parts;
+    if (dyn && rows_static > 0) {
+      const long mt_s = (rows_static + bm2 - 1) / bm2;
+      long mt_d = rows_dyn > n_dyn ? (rows_dyn - n_dyn) / bm2 + n_dyn : rows_dyn;   // the most that the rows make
+      if (mt_d > n_dyn * mt_s) mt_d = n_dyn * mt_s;                                 // (no expert has a token twice)
+      for (int pd = 6; pd > 1; --pd)
+        for (int ps = (int)fmin((pd * kts + ktd - 1) / ktd, pd); ps >= 1 && 2 * pd * kts <= (2 * ps + 1) * ktd; --ps) {
+          if (ktd / pd < 6 || kts / ps < 6 || (mt_d * pd + mt_s * ps) * nt > HDMOE_NUM_CU) continue;
+          pl.n = 1;
+          pl.pd[0] = pl.fixed_pd = pd;
+          pl.ps[0] = pl.fixed_ps = ps;
+          return pd;
+        }
+    }
     return fixed(parts < 1 ? 1 : (int)parts);
   }
 

@@ -388,15 +388,16 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
         tail_slot = tail.parts > 1 ? 1 + t * tail.parts + tail_part : 0;
       }
     }
-    int g_at = -1, mtiles = 1, ntiles = 1, L = 0, rb_at = 0, re_at = 0, parts = 1, kt = 0;
+    int g_at = -1, mtiles = 1, ntiles = 1, L = 0, rb_at = 0, re_at = 0, parts = 1, kt = 0, end = 0;
     for (int k = 0; k < args.G; ++k) {
       const int g = args.spread < 0 ? args.G - 1 - k : k;
       int rb, re;
       segs.get(g, rb, re);
       const int mt = EPI == G4_PARTIAL && F8 ? tile_div(re - rb + bm - 1, bm) : (re - rb + G4_BM - 1) / G4_BM, nt = segs.ntiles(g, FEAT), np = parts_of(g);
-      const long long tiles = (long long)mt * nt * np;
-      const int lo = eighths ? (int)(xcd * tiles / HDMOE_NUM_XCD) : 0;
-      const int hi = eighths ? (int)((xcd + 1) * tiles / HDMOE_NUM_XCD) : (int)tiles;
+      const int from = end;
+      end += mt * nt * np;
+      const int lo = eighths ? g4_dealt(end, xcd) - g4_dealt(from, xcd) : 0;
+      const int hi = eighths ? g4_dealt(end, xcd + 1) - g4_dealt(from, xcd + 1) : end - from;
       if (some && g_at < 0) {
         if (rem < hi - lo) { g_at = g; mtiles = mt; ntiles = nt; L = lo + rem; rb_at = rb; re_at = re; parts = np; kt = segs.bytes(g) / BK; }
         else rem -= hi - lo;

@@ -44,6 +44,12 @@ HDMOE_TAIL_HD G4Place g4_place(int longs, int shorts, int light_rounds, int xcd,
   return {true, tile < shorts ? tile : -1};
 }
 
+// Lists of tiles one behind the other, each dealt out to 8 XCDs in contiguous shares: the tiles in front of XCD `xcd`'s shares of all lists that
+// end at tile `end` of the whole. Its share of the list from tile a to tile b starts at tile g4_dealt(b, xcd) - g4_dealt(a, xcd) of it. The
+// shares of a list differ by at most one tile and so do the shares of all lists together; with each list cut in eighths by itself the odd tiles
+// fell to the same XCDs, and a round of 250 parts of five groups left 33 to one of 32 blocks.
+HDMOE_TAIL_HD int g4_dealt(int end, int xcd) { return (end >> 3) * xcd + ((end & 7) < xcd ? (end & 7) : xcd); }
+
 // The m-tiles of bm rows that n segments of `rows` rows together are counted as: each a standard deviation above the mean, and no more than
 // that many rows can make (four segments of 1024 rows: 7 of 256 rows, where each counted for itself would have two).
 inline int g4_likely_tiles(int rows, int n, int bm) {

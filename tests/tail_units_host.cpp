@@ -11,5 +11,6 @@ extern "C" int t_place(int longs, int shorts, int light_rounds, int xcd, int slo
   const G4Place p = g4_place(longs, shorts, light_rounds, xcd, slot, i);
   return p.tile < 0 ? -1 : p.tile * 2 + (p.is_short ? 1 : 0);
 }
+extern "C" int t_dealt(int end, int xcd) { return g4_dealt(end, xcd); }
 extern "C" int t_likely_tiles(int rows, int n, int bm) { return g4_likely_tiles(rows, n, bm); }
 extern "C" int t_cut_height(int bm, int rows, int n, int rows_static, int pd, int ps, int nt) { return g4_cut_height(bm, rows, n, rows_static, pd, ps, nt); }

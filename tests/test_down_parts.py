@@ -46,3 +46,28 @@ def layer_parts(tokens, dim, h, hs, experts=4):
 def test_parts_of_a_layer(dim, h, hs, tokens, want):
     """Four experts of just under 256 rows make 7 tiles of 256 rows at most, not 8: two parts fit a round at width 4096."""
     assert layer_parts(tokens, dim, h, hs) == want
+
+
+def few_rows_partials(tokens, code, dim=2560, h=6912, hs=3584, experts=4):
+    from comfyui_amd import functional as HF
+    lay = HF.layer_layout(tokens, dim, h, hs, experts, code)
+    return (lay.flags - lay.partials) // (3 * tokens * dim * 4) or 1
+
+
+@pytest.mark.parametrize("code", [_lib.W_E4M3FN, _lib.W_BF16, _lib.W_E4M3FN_UPCAST])
+@pytest.mark.parametrize("tokens,parts,shared", [(1, 6, 4), (16, 5, 3), (64, 5, 3), (128, 5, 3), (129, 4, 2), (130, 3, 2), (256, 3, 2)])
+def test_parts_of_few_rows_fit_a_round_however_they_are_routed(code, tokens, parts, shared):
+    """Every division of the slots that no token's two experts rule out, in 128-token tiles by 10 along the features."""
+    assert few_rows_partials(tokens, code) == parts
+    m = lambda rows: -(-rows // 128)
+    steps = sorted({1, 2, tokens // 2, tokens} | {v for v in (127, 128, 129) if v <= tokens})
+    for a in steps:
+        for b in steps:
+            for c in steps:
+                d = 2 * tokens - a - b - c
+                if 0 <= d <= tokens:
+                    assert ((m(a) + m(b) + m(c) + m(d)) * parts + m(tokens) * shared) * 10 <= 256
+
+
+def test_many_experts_keep_the_rule_by_the_mean_segment():
+    assert few_rows_partials(64, _lib.W_E4M3FN, experts=16) == 1   # 17 tiles by 10: two parts are no round

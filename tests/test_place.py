@@ -79,3 +79,21 @@ def test_the_longest_block_is_what_the_model_says(place, seed):
                     cost, i = cost + (short if v & 1 else price(kl, tiles[kl][(v >> 1) // 256 * 256])), i + 1
                 longest = max(longest, cost)
         assert got == longest, (rows, T, K, Ks, N, cap_long, cap_short)
+
+
+@pytest.mark.parametrize("lists", [[60, 60, 30, 60, 40], [30] * 5, [0, 1, 0, 7, 9], [250], [20] * 12, [40, 40, 40, 40, 20]] + [
+    [r.randrange(90) for _ in range(r.randrange(1, 17))] for r in [random.Random(9)] for _ in range(30)])
+def test_lists_are_dealt_out_evenly(tmp_path_factory, place, lists):
+    """csrc/tail_units.h, g4_dealt: each list in contiguous shares, no XCD more than one tile ahead in a list or in all of them, and a round of
+    256 blocks takes whatever has 256 tiles."""
+    so = next(tmp_path_factory.getbasetemp().glob("place*")) / "libplace.so"
+    dealt = ctypes.CDLL(str(so)).t_dealt
+    ends = [sum(lists[:k]) for k in range(len(lists) + 1)]
+    load = [0] * 8
+    for a, b in zip(ends, ends[1:]):
+        cuts = [dealt(b, x) - dealt(a, x) for x in range(9)]
+        assert cuts[0] == 0 and cuts[8] == b - a
+        shares = [cuts[x + 1] - cuts[x] for x in range(8)]
+        assert min(shares) >= (b - a) // 8 and max(shares) <= -(-(b - a) // 8)
+        load = [l + v for l, v in zip(load, shares)]
+    assert max(load) - min(load) <= 1 and max(load) == -(-ends[-1] // 8)
