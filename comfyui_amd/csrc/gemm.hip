@@ -1412,10 +1412,31 @@ bool short_tile_pays(const GemmShape& sh) {
 // The 224-token tile for fp8 gate/up: a round of it takes 3.85 units of expected_tile_cost (8192 tokens: 28.8 us, the 320-token
 // tile of 6 units 45), and half a unit goes for the last tile's activation, which nothing hides. Whole pass without and with it, us: layer of 260
 // tokens 105, 114; 350 129, 121; 512 145, 146; 600 167, 151; 1024 209, 208; 1300 229, 202; 1536 236, 226; 2300 338, 316; 4000 502, 449; 8000
-// 920, 823; 12000 1355, 1190; dense branch of 768 rows 78.5, 80.6; 1024 92, 105; 1500 115.2, 115.6; 1800 135, 123; 2048 138, 145.
+// 920, 823; 12000 1355, 1190; dense branch of 768 rows 78.5, 80.6; 1024 92, 105; 1500 115.2, 115.6; 1800 135, 123; 2048 138, 145. Those are
+// without low tiles; with them rounds are what s224_cost says of even segments: 450 tokens 135, 124; 900 177, 163 (256-token tiles before);
+// dense branch of 400 rows 55.3, 53.2; 450 64.9, 59.6; 512 62.0, 58.3 (192-token tiles before, which keep what is two of them high, the sizes
+// that their epilogue is tested at: 260 rows 52.7, 51.0; 300 61.6, 56.4).
 bool s224_pays(const GemmShape& sh, long other) {
-  const long rounds = (expected_tiles_of(sh, S224_BM) + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU;
-  return 77 * rounds + 10 <= 21 * other;
+  // the kernel's own choice of styles, for even segments
+  long whole = 0, best = 0;
+  for (int c = 0; c < S224_STYLES * S224_STYLES; ++c) {
+    long highs = 0, lows = 0;
+    auto add = [&](int groups, int rows, int N, int style) {
+      const S224Mix t = s224_mix(rows, style);
+      highs += (long)groups * t.highs * (N / S224_FEAT);
+      lows += (long)groups * t.lows * (N / S224_FEAT);
+    };
+    if (sh.n_dyn > 0) add(sh.n_dyn, (sh.rows_dyn + sh.n_dyn - 1) / sh.n_dyn, sh.N_dyn, c / S224_STYLES);
+    if (sh.rows_static > 0) add(1, sh.rows_static, sh.N_static, c % S224_STYLES);
+    if (c == 0) {
+      whole = best = (highs + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU * S224_HIGH;
+      if (highs > S224_TILES || (sh.n_dyn <= 0 && sh.rows_static <= 2 * TileCfg<3>::BM)) break;
+    } else {
+      const int cost = s224_cost((int)highs, (int)lows);
+      if (s224_low_pays(cost, (int)whole) && cost < best) best = cost;
+    }
+  }
+  return 77 * best + 10 * S224_HIGH <= 21 * S224_HIGH * other;
 }
 
 // light: the token blocks of a tile that hold no rows are skipped (fp8: the compiler-scheduled K loop instead of the

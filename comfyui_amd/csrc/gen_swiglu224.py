@@ -10,6 +10,9 @@ next stage. The epilogue of a tile packs w1 x and w3 x (scaled, rounded to bf16)
 them stay in registers, 6 go to LDS. SiLU, product, cast and stores are issued behind the MFMAs of the next tile's first 7
 pairs of K steps (a token block per pair; these pairs are written out, the others are a loop).
 
+A low tile has 128 tokens, 4 blocks per wave: the same loads (slabs without rows ask for nothing) and 32 MFMAs a step, in two texts, behind a
+tile of 7 and behind a low one.
+
 Register map (per wave):
   a[0:223]    accumulators acc[ft][tt] = a[(7*ft + tt)*4 : +3], ft: 16 weight rows (0-3 w1, 4-7 w3), tt: 16 tokens
   a[224:255]  weight fragments 0-3 (8 registers each)
@@ -31,6 +34,7 @@ from gen_gemm4w import DRAIN_WAIT, STAGE, W_TILE, Feeder, check_trans, quad  # n
 
 OUT = os.path.join(HERE, "swiglu224_asm.inc")
 NTT = 7
+LOW = 4                                           # 16-token blocks of a wave in a low tile
 CTX = 96
 TOK_ADDR = [CTX + 0, CTX + 1]                     # LDS address of the lane's token fragment, per 64-byte half of a step
 W_ADDR = [CTX + 2, CTX + 3]
@@ -38,20 +42,25 @@ TOK_VOFF = [CTX + 4 + j for j in range(NTT)]      # global byte offset of the la
 W_VOFF = CTX + 11                                 # same for weight slab 0; the others' distance goes in a scalar register
 NEXT = [CTX + 12 + j for j in range(NTT)]         # TOK_VOFF of the next tile
 DEF_ST = CTX + 19                                 # output byte offset of the lane in the deferred token block
-GATHER_VOFF = CTX + 20                            # byte offset of the lane's entry of slab 0 in the row index list
+GATHER_VOFF = CTX + 20                            # byte offset of the lane's entry of slabs 0-2 in the row index list, less 128 per slab
 STG = CTX + 21                                    # LDS address of the lane's deferred pieces
+GATHER_VOFF3, GATHER_VOFF4 = CTX + 22, CTX + 23   # of slab 3, which holds rows of both wave rows, and of slabs 4-6
 TMP = CTX + 24                                    # v[120:126]
 GATHER = 88
 RES = 34
 PIECES = [38 + 4 * i for i in range(12)] + [216 + 4 * i for i in range(10)]   # pieces 0-21 = token block * 4 + ft
 IN_LDS = list(range(len(PIECES), 4 * NTT))        # the others; read back into the registers of the first ones
 
-# positions (MFMA index within a step) of the events
-FREE_AT = 16        # the stage has been read; barrier
-LOAD_AT = [17 + round(2.55 * j) for j in range(15)]
-LAND_AT = 38        # the next stage has landed; barrier, then the reads of the next step's first quadrant
-STORE_AT = 55       # odd step: a finished token block
-STG_AT = 8          # reads of deferred pieces from LDS
+
+class At:
+    """Positions (MFMA index within a step) of the events, by the tile's token blocks per wave."""
+    def __init__(self, nt):
+        self.m = 8 * nt
+        self.free = 16              # the stage has been read; barrier
+        self.load = [17 + round((2.55 if nt == NTT else 1) * j) for j in range(15)]
+        self.land = {NTT: 38, LOW: 26}[nt]   # the next stage has landed; barrier, then the reads of the next step's first quadrant
+        self.store = self.m - 1     # odd step: a finished token block
+        self.stg = 8                # reads of deferred pieces from LDS
 
 
 def weight(f):
@@ -72,22 +81,23 @@ def reads(stage, frags):
             for k, i in frags for h in range(2)]
 
 
-def blocks(stage):
+def blocks(stage, nt):
     """Token blocks of the first and of the second quadrant."""
-    return (range(0, 4), range(4, NTT)) if stage == 0 else (range(4, NTT), range(0, 4))
+    cut = (nt + 1) // 2
+    return (range(0, cut), range(cut, nt)) if stage == 0 else (range(cut, nt), range(0, cut))
 
 
-def first_reads(stage):
-    t = list(blocks(stage)[0])
+def first_reads(stage, nt):
+    t = list(blocks(stage, nt)[0])
     return reads(stage, [("w", 0), ("t", t[0]), ("w", 1), ("w", 2), ("w", 3)] + [("t", x) for x in t[1:]])
 
 
-def own_reads(stage):
-    return reads(stage, [("t", x) for x in blocks(stage)[1]] + [("w", f) for f in range(4, 8)])
+def own_reads(stage, nt):
+    return reads(stage, [("t", x) for x in blocks(stage, nt)[1]] + [("w", f) for f in range(4, 8)])
 
 
-def mfma_order(stage):
-    t0, t1 = blocks(stage)
+def mfma_order(stage, nt):
+    t0, t1 = blocks(stage, nt)
     o = []
     for fts, tts in ((range(4), t0), (range(4), t1), (range(4, 8), t1), (range(4, 8), t0)):
         for k, tt in enumerate(tts):
@@ -135,24 +145,24 @@ def piece_at(i):
     return PIECES[i] if i < len(PIECES) else PIECES[i - len(PIECES)]
 
 
-def step(stage, first, block, stored):
+def step(stage, first, block, stored, nt):
     """One K step out of `stage`. Entry: the reads of its first quadrant are in flight. first: the accumulators start from zero.
     block: the deferred token block of this pair of steps (two of its pieces per step), None = none. stored: the step before ended with a
     store for certain."""
     L = []
-    order, own, nxt = mfma_order(stage), own_reads(stage), first_reads(stage ^ 1)
-    events = dict(zip(LOAD_AT, loads(stage)))
+    at = At(nt)
+    order, own, nxt = mfma_order(stage, nt), own_reads(stage, nt), first_reads(stage ^ 1, nt)
+    events = dict(zip(at.load, loads(stage)))
     pieces = [] if block is None else [4 * block + 2 * stage, 4 * block + 2 * stage + 1]
     from_lds = [i for i in pieces if i in IN_LDS]
-    start = FREE_AT if from_lds else 0
-    work = Feeder([op for i in pieces for op in silu_words(piece_at(i), RES + i % 4)], STORE_AT - 2 - start)
-    t1 = list(blocks(stage)[1])
-    n_first = 4 * len(blocks(stage)[0])
+    start = at.free if from_lds else 0
+    work = Feeder([op for i in pieces for op in silu_words(piece_at(i), RES + i % 4)], at.store - 2 - start)
+    n_first = 4 * len(blocks(stage, nt)[0])
     L += ["s_add_u32 s76, %[so], %[kb8]", "s_add_u32 s77, %[so], %[kb64]", "s_add_u32 s78, s76, %[kb64]"]
     for q, (ft, tt) in enumerate(order):
         if q == 0:
             L.append("s_waitcnt lgkmcnt(0)")
-        if q == n_first and q < FREE_AT:   # the second quadrant's tokens are there, its weights are the first's
+        if q == n_first and q < at.free:   # the second quadrant's tokens are there, its weights are the first's
             L.append("s_waitcnt lgkmcnt(8)")
         if q in events:
             L.append(events[q][0])
@@ -162,56 +172,59 @@ def step(stage, first, block, stored):
             L.append(events[q][1])
         if q < 8:
             L += own[2 * q:2 * q + 2]
-        if q == STG_AT:
+        if q == at.stg:
             L += [f"ds_read_b128 {quad(piece_at(i))}, v{STG} offset:{1024 * IN_LDS.index(i)}" for i in from_lds]
-        if q == FREE_AT - 1:
+        if q == at.free - 1:
             L += ["s_waitcnt lgkmcnt(0)", "s_barrier"]
-        if q == LAND_AT - 1:
+        if q == at.land - 1:
             # requests return in order: those of this step and the store are younger than the next step's operands
-            L += [f"s_waitcnt vmcnt({sum(p < LAND_AT for p in LOAD_AT) + stored})", "s_barrier"]
-        if q >= LAND_AT:
-            L += nxt[2 * (q - LAND_AT):2 * (q - LAND_AT) + 2]
-        if start <= q < STORE_AT - 2:
+            L += [f"s_waitcnt vmcnt({sum(p < at.land for p in at.load) + stored})", "s_barrier"]
+        if q >= at.land:
+            L += nxt[2 * (q - at.land):2 * (q - at.land) + 2]
+        if start <= q < at.store - 2:
             L += work.take()
-        if q == STORE_AT and block is not None and stage == 1:
+        if q == at.store and block is not None and stage == 1:
             L += [f"buffer_store_dwordx4 {quad(RES)}, v{DEF_ST}, %[dro], 0 offen", f"v_add_u32 v{DEF_ST}, %[dldo], v{DEF_ST}"]
-    assert work.done() and len(own) <= 16 and len(nxt) <= 2 * (len(order) - LAND_AT)
+    assert work.done() and len(own) <= 16 and len(nxt) <= 2 * (len(order) - at.land)
     # a fragment is overwritten behind the last MFMA that reads it
     last = {}
     for q, (ft, tt) in enumerate(order):
         last[("w", ft)] = last[("t", tt)] = q
     for k, r in enumerate(nxt):
-        for key, reg in [(("w", f), weight(f)) for f in range(8)] + [(("t", t), token(t)) for t in range(NTT)]:
+        for key, reg in [(("w", f), weight(f)) for f in range(8)] + [(("t", t), token(t)) for t in range(nt)]:
             if any(half(reg, h) in r for h in range(2)):
-                assert last[key] <= LAND_AT + k // 2, (stage, key)
+                assert last[key] <= at.land + k // 2, (stage, key)
     L.append("s_add_u32 %[so], %[so], 128")
     return L
 
 
-def pair(first, block):
-    return step(0, first, block, block not in (None, 0)) + step(1, False, block, False)
+def pair(first, block, nt):
+    return step(0, first, block, block not in (None, 0), nt) + step(1, False, block, False, nt)
 
 
-def k_loop():
-    """All K steps of a tile in pairs, %[n] of them (at least 8). Before the last pair the loads turn to the first two steps of the
-    next tile and the row indices of the tile after it are requested."""
+def k_loop(nt, before):
+    """All K steps of a tile of nt blocks in pairs, %[n] of them (at least 8), behind a tile of `before`. Before the last pair the loads turn
+    to the first two steps of the next tile and the row indices of the tile after it are requested. The last step reads the first quadrant of
+    the next tile's first one: a lower tile's is part of it."""
     L = ["s_mov_b64 s[64:65], %[ra]", "s_mov_b64 s[66:67], %[rah]", "s_mov_b64 s[68:69], %[rb]", "s_mov_b64 s[70:71], %[rbh]",
-         "s_mov_b64 s[72:73], %[rc]", "s_mov_b64 s[74:75], %[rbh]", f"s_sub_u32 %[n], %[n], {NTT}"]
-    for b in range(NTT):
-        L += pair(b == 0, b)
-    L += ["11:", "s_cmp_eq_u32 %[n], 1", "s_cbranch_scc1 13f", "14:"] + pair(False, None)
+         "s_mov_b64 s[72:73], %[rc]", "s_mov_b64 s[74:75], %[rbh]", f"s_sub_u32 %[n], %[n], {before}"]
+    for b in range(before):
+        L += pair(b == 0, b, nt)
+    L += ["11:", "s_cmp_eq_u32 %[n], 1", "s_cbranch_scc1 13f", "14:"] + pair(False, None, nt)
     L += ["s_sub_u32 %[n], %[n], 1", "s_cmp_lg_u32 %[n], 0", "s_cbranch_scc1 11b", "s_branch 12f"]
     L += ["13:", "s_mov_b64 s[64:65], %[na]", "s_mov_b64 s[66:67], %[nah]", "s_mov_b64 s[68:69], %[nb]", "s_mov_b64 s[72:73], %[nc]",
           "s_mov_b32 s70, %[nbn]", "s_mov_b32 s74, %[nbn]", "s_mov_b32 %[so], 0"]
     L += [f"v_mov_b32 v{TOK_VOFF[j]}, v{NEXT[j]}" for j in range(NTT)]
-    L += [f"buffer_load_dword v{GATHER + j}, v{GATHER_VOFF}, %[gr], 0 offen offset:{128 * j}" for j in range(NTT)]
+    for j in range(NTT):
+        v, off = (GATHER_VOFF, 128 * j) if j < 3 else (GATHER_VOFF3, 0) if j == 3 else (GATHER_VOFF4, 128 * (j - 4))
+        L.append(f"buffer_load_dword v{GATHER + j}, v{v}, %[gr], 0 offen offset:{off}")
     return L + ["s_branch 14b", "12:", "s_nop 15"]
 
 
-def epilogue():
+def epilogue(nt):
     """acc * scale rounded to bf16, w1 x and w3 x packed into a word; work registers v[160:215]."""
     L = []
-    for i in range(4 * NTT):
+    for i in range(4 * nt):
         tt, ft = divmod(i, 4)
         w = 160 + 12 * (i % 4)
         for e in range(4):
@@ -227,22 +240,32 @@ def epilogue():
     return L
 
 
+def tile():
+    """A tile by its text, %[text]: 0 = 7 blocks behind a tile of 7, 1 = a low one behind a tile of 7, 2 = a low one behind a low one. (The
+    blocks' tiles go from high to low.)"""
+    L = ["s_cmp_eq_u32 %[text], 1", "s_cbranch_scc1 101f", "s_cmp_eq_u32 %[text], 2", "s_cbranch_scc1 102f"]
+    L += k_loop(NTT, NTT) + epilogue(NTT) + ["s_branch 109f", "101:"] + k_loop(LOW, NTT) + epilogue(LOW)
+    return L + ["s_branch 109f", "102:"] + k_loop(LOW, LOW) + epilogue(LOW) + ["109:"]
+
+
 def drain():
-    """The deferred pieces of a block's last tile, with nothing to hide behind."""
+    """The deferred pieces of a block's last tile, with nothing to hide behind; %[text] other than 0: a low one."""
     L = []
     for tt in range(NTT):
+        if tt == LOW:
+            L += ["s_cmp_lg_u32 %[text], 0", "s_cbranch_scc1 21f"]
         for g in range(4):
             i = 4 * tt + g
             if i in IN_LDS:
                 L += [f"ds_read_b128 {quad(piece_at(i))}, v{STG} offset:{1024 * IN_LDS.index(i)}", "s_waitcnt lgkmcnt(0)"]
             L += [op for op, _ in silu_words(piece_at(i), RES + g)]
         L += [f"buffer_store_dwordx4 {quad(RES)}, v{DEF_ST}, %[dro], 0 offen", f"v_add_u32 v{DEF_ST}, %[dldo], v{DEF_ST}"]
-    return L + ["s_nop 7"]
+    return L + ["21:", "s_nop 7"]
 
 
 def generate():
     out = ["// Generated by gen_swiglu224.py; do not edit. See that script for the register map and the schedule.", ""]
-    for name, lines in (("HDMOE_S224_TILE", k_loop() + epilogue()), ("HDMOE_S224_FILL", first_reads(0)), ("HDMOE_S224_DRAIN", DRAIN_WAIT + drain())):
+    for name, lines in (("HDMOE_S224_TILE", tile()), ("HDMOE_S224_FILL", first_reads(0, NTT)), ("HDMOE_S224_DRAIN", DRAIN_WAIT + drain())):
         check_trans(lines)
         out.append(f"#define {name} \\")
         out.append(" \\\n".join('  "' + ln + '\\n"' for ln in lines))

@@ -68,3 +68,29 @@ inline int g4_cut_height(int bm, int rows, int n, int rows_static, int pd, int p
   while (bm < 256 && (g4_likely_tiles(rows, n, bm) * pd + (rows_static + bm - 1) / bm * ps) * nt > 256) bm += 32;
   return bm;
 }
+
+// The tiles of a segment on swiglu224_kernel (swiglu224.h): high ones of 224 rows, then low ones of 128. Styles: 0 high ones alone; 1 the last
+// one low if its rows fit; 2 what is left after full ones in low ones; 3 the last full one's rows too; 4 low ones alone.
+struct S224Mix { int highs, lows; };
+HDMOE_TAIL_HD S224Mix s224_mix(int rows, int style) {
+  const int full = (int)((unsigned)rows / 224u), rest = rows - full * 224, all = full + (rest > 0 ? 1 : 0);
+  const int keep = style == 0 || (style == 1 && rest > 128) ? all : style <= 2 ? full : style == 3 ? (full > 0 ? full - 1 : 0) : 0;
+  const int left = rows - keep * 224;
+  return {keep, left > 0 ? (left + 127) >> 7 : 0};
+}
+
+// How the list of a launch is dealt out: highs in whole rounds of 256 blocks, what is left of them to as many blocks, lows to the other ones first
+// (g4_place). What the longest block comes to, a high tile being S224_HIGH. A low one is 64 by its matrix instructions; 75 because all lows of an
+// expert read its weights once more (priced at 66 layers of 1000 and 1500 tokens took 4 and 3 % longer than without; 83 and 92 lose 450 and
+// 800 tokens). Others than high tiles alone have to pay by a 24th: the clock falls with the CUs that are busy (a 13th loses 2 % at 1200, 1300 and
+// 2300 tokens and 1 % at 4096, a 30th gains nothing more). Beyond 16 rounds there is nothing to gain.
+constexpr int S224_HIGH = 100, S224_LOW = 75, S224_STYLES = 5, S224_TILES = 4096;
+HDMOE_TAIL_HD bool s224_low_pays(int cost, int whole) { return cost < whole - whole / 24; }
+HDMOE_TAIL_HD int s224_cost(int highs, int lows) {
+  const int full = highs >> 8, left = highs & 255, lights = 256 - left, light = full * S224_HIGH, heavy = light + (left > 0 ? S224_HIGH : 0);
+  const int first = left > 0 ? 1 : 0, rest = lows - first * lights;
+  if (rest <= 0) return heavy;
+  const int q = rest >> 8, r = rest & 255;
+  const int a = light + (first + q + (r > 0 ? 1 : 0)) * S224_LOW, b = heavy + (left > 0 ? q + (r > lights ? 1 : 0) : 0) * S224_LOW;
+  return a > b ? a : b;
+}

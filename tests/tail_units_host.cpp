@@ -14,3 +14,5 @@ extern "C" int t_place(int longs, int shorts, int light_rounds, int xcd, int slo
 extern "C" int t_dealt(int end, int xcd) { return g4_dealt(end, xcd); }
 extern "C" int t_likely_tiles(int rows, int n, int bm) { return g4_likely_tiles(rows, n, bm); }
 extern "C" int t_cut_height(int bm, int rows, int n, int rows_static, int pd, int ps, int nt) { return g4_cut_height(bm, rows, n, rows_static, pd, ps, nt); }
+extern "C" int t_mix(int rows, int style) { const S224Mix t = s224_mix(rows, style); return t.highs | t.lows << 16; }
+extern "C" int t_s224_cost(int highs, int lows) { return s224_cost(highs, lows); }

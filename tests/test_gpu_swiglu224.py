@@ -27,6 +27,13 @@ def codes(h):
     ((447, 449), 2560, 384, 0.37),           # one row less than two tiles, one more
     ((1, 0, 700, 2299), 2560, 1024, 1.0),    # empty and nearly empty segments
     ((1500, 1500), 6912, 256, 0.25),         # 27 pairs of K steps
+    # low tiles of 128 tokens too (csrc/tail_units.h, s224_mix):
+    ((330,), 2048, 23040, 1.0),              # one behind a high tile
+    ((225,), 2304, 32000, 0.5),              # alone, two for some blocks, one row in the last
+    ((384, 380, 390, 382), 2560, 4608, 1.0), # three and four alone
+    ((390, 392), 2560, 8960, 0.7),           # two behind one high tile, rows of one in the first of its halves alone
+    ((455, 450), 2048, 16384, 1.0),          # 224 + 7 rows in two
+    ((270, 262), 2048, 23040, 1.0),
     ((8192,), 2048, 57600, 2.0),             # 65 tiles for some blocks: the tables of work are filled a second time
 ])
 def test_grouped_swiglu(dev, forms, sizes, D, H, s_next):
