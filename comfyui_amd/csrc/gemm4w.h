@@ -28,14 +28,21 @@ constexpr int G4_THREADS = 256;
 constexpr int G4_BM = 256;                        // tokens per block tile
 constexpr int G4_STAGE = 32768;
 constexpr int G4_W_TILE = 65536;
-constexpr int G4_TABLE = 131072;                  // LDS: [tok 0 | tok 1 | w 0 | w 1 | work item tables of the 4 waves]
+constexpr int G4_TABLE = 131072;                  // LDS: [tok 0 | tok 1 | w 0 | w 1 | work item tables of the 4 waves | groups]
 constexpr int G4_TABLE_ITEMS = 64;                // items a wave's lanes look up at a time
-constexpr int G4_HEIGHTS = G4_TABLE + 4 * G4_TABLE_ITEMS * 16;   // 16 bytes per group
-constexpr int G4_SMEM = G4_HEIGHTS + MAX_GROUPS * 16;
+constexpr int G4_HEIGHTS = G4_TABLE + 4 * G4_TABLE_ITEMS * 16;   // 16 bytes per group, and 16 more (tile_mix)
+constexpr int G4_SMEM = G4_HEIGHTS + (MAX_GROUPS + 1) * 16;
 constexpr int G4_MIN_BLOCKS = 4;                  // least height of a tile, in token blocks of 32 rows
 constexpr int G4_SCRATCH = 4 * 28 * 1024;         // GELU: bytes of scratch per block (28 pieces of 16 bytes per lane)
 constexpr int G4_GELU_PAIRS = 16;                 // pairs of K steps a deferred activation needs to hide behind
 
+// Gate/up on 16-bit activations ends its blocks' lists on low tiles of 128 rows as swiglu224.h does (tile_mix). A low one costs 78 of a whole one's
+// 100, and with 16-bit weights 27 more where it is the only one of its segment: weights of more than the memory-side cache come from memory
+// again for it alone (layer of 500 tokens, three experts a little over 256 rows: 202 -> 210 us without that). Up to 6 rounds of tiles; 3000
+// tokens 593 -> 600 us. Tiles are as high as their rows need in any case. Before -> this, us: layers in bf16, 500 tokens 205 -> 197, 800 251 -> 244,
+// 1000 285 -> 272, 1024 289 -> 283, 1500 370 -> 365; e4m3fn weights, 500 176 -> 166, 1000 264 -> 252, 1024 266 -> 255, 1800 404 -> 379; dense branch in bf16,
+// 256 rows 98.7 -> 90.0, 400 101.9 -> 92.2, 1500 179 -> 170; e4m3fn weights 91.0 -> 77.9, 93.7 -> 78.6, 170 -> 157.
+constexpr int G4_LOW_COST = 78, G4_LOW_ALONE = 27, G4_MIX_TILES = 6 * HDMOE_NUM_CU;
 constexpr int G4_TAIL_MAX_PARTS = 12;
 constexpr size_t G4_TAIL_BYTES = (size_t)HDMOE_NUM_CU * G4_BM * 256 * 4;  // fp32 sums of one tile per block
 
@@ -131,8 +138,8 @@ __device__ __forceinline__ G4Tail g4_tail_of(const GemmArgs& args, const Segment
 // e4m3fn weights 50.0 -> 37.4, 49.0 -> 36.8, 50.1 -> 42.3; Hunyuan3D block of 1250 tokens 367 -> 330, 1500 358 -> 348 (375 rows per expert:
 // 3 rounds of 8 or of 6 to 7 blocks); in fp8, 8-wave kernel on 192-token tiles -> this, without the cast: 4480 x 2560 x 2560 31.6 -> 28.7, 2000 25.8 ->
 // 21.8, 1000 22.0 -> 19.0, 2000 x 2560 x 10240 52.7 -> 46.9, 9000 x 2048 x 2048 44.0 -> 36.2, 193 x 4096 x 2560 28.4 -> 23.4; fp8 tiles are as
-// high as their rows need without a cap too. Not for SWIGLU, whose two halves of the weights every further m-tile reads again: 1300 tokens
-// in bf16 361 -> 367 us, 1024 tokens 294 -> 298. More than 24 rounds: one is not worth the search.
+// high as their rows need without a cap too. Not for SWIGLU, whose two halves of the weights every further m-tile reads again (1300 tokens
+// in bf16 361 -> 367 us, 1024 tokens 294 -> 298): it has whole tiles and low ones behind them (tile_mix). More than 24 rounds: one is not worth the search.
 constexpr int G4_TILE_COST = 150, G4_CAP_ROUNDS = 24;
 __host__ __device__ __forceinline__ int g4_div(int a, int b) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -256,6 +263,74 @@ inline int g4_host_cap(const GemmArgs& args, int feat, int min_pairs, int blocks
   return g4_best_cap(whole, pairs, [&](int cap) { return g4_cap_cost(args.G, pairs, rows, [&](int g) { return args.g[g].n_out / feat; }, blocks, cap); });
 }
 
+// High and low tiles of the segments (tail_units.h), lane g looking after group g: leaves [segment begin, end, high m-tiles | low ones << 16, tiles
+// along the features] of each group and [rounds of high tiles, high tiles beyond, low tiles] behind them in `groups` (LDS, every wave the
+// same) and says whether there are low ones. low_cost: of a low tile in hundredths of a high one's; alone: more where it is the only one of its
+// segment; most: high tiles at which low ones are looked for.
+__device__ __forceinline__ bool tile_mix(const Segments& segs, int G, int lane, int high, int feat, int low_cost, int alone, int most, v4i* groups) {
+  const int rows = segs.re - segs.rb, nt = (int)((unsigned)segs.n_out / (unsigned)feat), whole = s224_mix(rows, 0, high).highs * nt;
+  int highs = 0, lows = 0, style = 0;
+  for (int g = 0; g < G; ++g) highs += __builtin_amdgcn_readlane(whole, g);
+  if (highs <= most) {   // lane i: style i / 5 of the experts and i % 5 of the static group
+    const int c = min(lane, S224_STYLES * S224_STYLES - 1), of_dyn = c * 13 >> 6, of_fix = c - 5 * of_dyn;
+    int tiles = 0, single = 0;   // high ones | low ones << 16; low ones that share their weights with none
+    for (int g = 0; g < G; ++g) {
+      const S224Mix t = s224_mix(__builtin_amdgcn_readlane(rows, g), segs.dynamic(g) ? of_dyn : of_fix, high);
+      const int n = __builtin_amdgcn_readlane(nt, g);
+      tiles += (t.highs | t.lows << 16) * n;
+      single += t.lows == 1 ? n : 0;
+    }
+    if (alone > 0) low_cost += tile_div(alone * single, max(tiles >> 16, 1));
+    const int mine = s224_cost(tiles & 0xffff, tiles >> 16, low_cost) << 5 | c;
+    const int first = __builtin_amdgcn_readlane(mine, 0);
+    int best = first;
+#pragma unroll
+    for (int k = 1; k < S224_STYLES * S224_STYLES; ++k) best = min(best, __builtin_amdgcn_readlane(mine, k));
+    if (s224_low_pays(best >> 5, first >> 5)) {
+      const int pick = best & 31, pick_dyn = pick * 13 >> 6;
+      style = segs.fixed >> lane & 1 ? pick - 5 * pick_dyn : pick_dyn;
+      tiles = __builtin_amdgcn_readlane(tiles, pick);
+      highs = tiles & 0xffff;
+      lows = tiles >> 16;
+    }
+  }
+  const S224Mix t = s224_mix(rows, style, high);
+  v4i e = {segs.rb, segs.re, t.highs | t.lows << 16, nt};
+  if (lane == MAX_GROUPS) e = v4i{highs / HDMOE_NUM_CU, highs % HDMOE_NUM_CU, lows, 0};
+  if (lane <= MAX_GROUPS) groups[lane] = e;
+  return lows > 0;
+}
+// Item i of a block's list: g < 0: none.
+struct MixedTile { int g, row0, rows, n; bool low; };
+__device__ __forceinline__ MixedTile mixed_tile(const v4i* groups, int G, int lane, int xcd, int slot, int i, int high) {
+  constexpr int nslots = HDMOE_NUM_CU / HDMOE_NUM_XCD;
+  const v4i mine = groups[min(lane, MAX_GROUPS)];
+  const int rounds = __builtin_amdgcn_readlane(mine.x, MAX_GROUPS), left = __builtin_amdgcn_readlane(mine.y, MAX_GROUPS),
+            lows = __builtin_amdgcn_readlane(mine.z, MAX_GROUPS);
+  // whole rounds: an XCD's blocks take a contiguous eighth of the list
+  const G4Place at = g4_place(left, lows, left > 0 ? 1 : 0, xcd, slot, i - rounds);
+  const bool low = i >= rounds && at.is_short;
+  int rem = i < rounds ? xcd * (rounds * nslots) + slot + i * nslots : low ? at.tile : rounds * HDMOE_NUM_CU + at.tile;
+  int g_at = -1, mtiles = 1, ntiles = 1, L = 0, rb_at = 0, re_at = 0;
+  for (int g = 0; g < G; ++g) {
+    const int rb = __builtin_amdgcn_readlane(mine.x, g), re = __builtin_amdgcn_readlane(mine.y, g), mts = __builtin_amdgcn_readlane(mine.z, g),
+              nt = __builtin_amdgcn_readlane(mine.w, g), mt = low ? mts >> 16 : mts & 0xffff;
+    if (rem >= 0 && g_at < 0) {
+      if (rem < mt * nt) { g_at = g; mtiles = mt; ntiles = nt; L = rem; rb_at = rb + (low ? (mts & 0xffff) * high : 0); re_at = re; }
+      else rem -= mt * nt;
+    }
+  }
+  MixedTile t = {g_at, 0, 0, 0, low};
+  if (g_at >= 0) {
+    int m;
+    g4_raster(L, mtiles, ntiles, m, t.n);
+    const int height = low ? 128 : high;
+    t.row0 = rb_at + m * height;
+    t.rows = min(re_at - t.row0, height);
+  }
+  return t;
+}
+
 template <G4Type TY, int EPI>
 __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm4w_kernel(const GemmArgs args) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass drops the stub of a kernel whose register operands it cannot parse
@@ -349,9 +424,20 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     }
     if (lane < args.G) heights[lane] = e;   // every wave the same
   }
+  bool mixed = false;
+  if constexpr (SWIGLU) {
+    if (tail.parts == 1) mixed = tile_mix(segs, args.G, lane, G4_BM, FEAT, G4_LOW_COST, W8 ? 0 : G4_LOW_ALONE, G4_MIX_TILES, heights);
+  }
   v4i* const table = reinterpret_cast<v4i*>(smem + G4_TABLE) + wave * G4_TABLE_ITEMS;
   auto fill_table = [&](int base) {
     const int i = base + lane;
+    if (SWIGLU && mixed) {
+      const MixedTile t = mixed_tile(heights, args.G, lane, xcd, slot, i, G4_BM);
+      v4i e = {-1, 0, 0, 0};
+      if (t.g >= 0) e = v4i{t.g | t.rows << 16, t.row0, t.n, segs.bytes(0) / BK << 16};
+      table[lane] = e;
+      return;
+    }
     if (cap > 0) {
       int longs = 0, shorts = 0;
       for (int g = 0; g < args.G; ++g) (is_short(g) ? shorts : longs) += sgpr(heights[g].y);
@@ -600,7 +686,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     ctx[G4_OUT_VOFF] = part ? wave * 8192 + lane * 16
                             : (wt * 16 + fr_row) * ldo + (cur.n0() + wq * (FEAT / 2) + fr_grp * 8) * OUT_BYTES;
     const int part_s = part ? sgpr(g4_part_blocks(cur.rows_here(), wave)) + 1 : 0;
-    const int nt = sgpr(F8 || cap > 0 ? max((cur.rows_here() + 31) >> 5, G4_MIN_BLOCKS) : G4_BM / 32);   // token blocks
+    const int nt = sgpr(F8 || cap > 0 || (SWIGLU && !part) ? max((cur.rows_here() + 31) >> 5, G4_MIN_BLOCKS) : G4_BM / 32);   // token blocks
     // row indices of nx2 and this tile's biases are loaded inside the statement
     const int32_t* const list = nx2.some() ? args.g[nx2.g()].gather : nullptr;
     const v4i gr = rsrc4(list != nullptr ? list + nx2.row0() : nullptr, list != nullptr ? (uint32_t)nx2.rows_here() * 4u : 0u);

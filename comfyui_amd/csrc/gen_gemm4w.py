@@ -492,12 +492,12 @@ def epilogue(dt, w8, bias, gelu, nt=8):
     return L
 
 
-def swiglu_epilogue(w8):
+def swiglu_epilogue(w8, nt=8):
     """bf16(bf16(silu(w1 x)) * (w3 x)): the wave's ft 0-3 are w1 rows, ft 4-7 the same features of w3. Two values at a
     time; registers v[192:255]."""
     L = []
     n = 0
-    for tt in range(8):
+    for tt in range(nt):
         L += out_row(tt)
         for g in range(2):
             o = 192 + 4 * (n % 2)
@@ -608,7 +608,7 @@ def generate():
         name = f"HDMOE_G4_TILE_{dt}{'_W8' if w8 else ''}{'_GELU' if gelu else '_BIAS' if bias else ''}"
         texts.append((name, tile(dt, w8, gelu, bias, lambda nt: epilogue(dt, w8, bias, gelu, nt))))
     for w8 in (False, True):
-        texts.append((f"HDMOE_G4_TILE_BF16{'_W8' if w8 else ''}_SWIGLU", tile("BF16", w8, False, False, lambda nt: swiglu_epilogue(w8), HEIGHTS[:1])))
+        texts.append((f"HDMOE_G4_TILE_BF16{'_W8' if w8 else ''}_SWIGLU", tile("BF16", w8, False, False, lambda nt: swiglu_epilogue(w8, nt))))
         texts.append((f"HDMOE_G4_TILE_BF16{'_W8' if w8 else ''}_PARTIAL", k_loop("BF16", w8, False, False) + partial_epilogue()))
     texts.append(("HDMOE_G4_FILL", reads(0, 0, False, 0)))
     texts.append(("HDMOE_G4_FILL_W8", reads(0, 0, True, 0) + ["s_waitcnt lgkmcnt(0)"] + [i for i, _ in conversions(0)]))

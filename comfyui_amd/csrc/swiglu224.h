@@ -85,63 +85,14 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   const bool use_alt = args.alt.flag != nullptr && sgpr(*args.alt.flag) == 0;   // the alternative token operand (GemmArgs::alt)
   v4i* const records = reinterpret_cast<v4i*>(smem + S224_RECORDS);
   v4i* const groups = reinterpret_cast<v4i*>(smem + S224_GROUPS);
-  {
-    const int rows = segs.re - segs.rb, nt = (int)((unsigned)segs.n_out / S224_FEAT), whole = s224_mix(rows, 0).highs * nt;
-    int highs = 0, lows = 0, style = 0;
-    for (int g = 0; g < args.G; ++g) highs += __builtin_amdgcn_readlane(whole, g);
-    if (highs <= S224_TILES) {   // lane i: style i / 5 of the experts and i % 5 of the static group
-      const int c = min(lane, S224_STYLES * S224_STYLES - 1), of_dyn = c * 13 >> 6, of_fix = c - 5 * of_dyn;
-      int tiles = 0;   // high ones | low ones << 16
-      for (int g = 0; g < args.G; ++g) {
-        const S224Mix t = s224_mix(__builtin_amdgcn_readlane(rows, g), segs.dynamic(g) ? of_dyn : of_fix);
-        tiles += (t.highs | t.lows << 16) * __builtin_amdgcn_readlane(nt, g);
-      }
-      const int mine = s224_cost(tiles & 0xffff, tiles >> 16) << 5 | c;
-      const int first = __builtin_amdgcn_readlane(mine, 0);
-      int best = first;
-#pragma unroll
-      for (int k = 1; k < S224_STYLES * S224_STYLES; ++k) best = min(best, __builtin_amdgcn_readlane(mine, k));
-      if (s224_low_pays(best >> 5, first >> 5)) {
-        const int pick = best & 31, pick_dyn = pick * 13 >> 6;
-        style = segs.fixed >> lane & 1 ? pick - 5 * pick_dyn : pick_dyn;
-        tiles = __builtin_amdgcn_readlane(tiles, pick);
-        highs = tiles & 0xffff;
-        lows = tiles >> 16;
-      }
-    }
-    const S224Mix t = s224_mix(rows, style);
-    v4i e = {segs.rb, segs.re, t.highs | t.lows << 16, nt};
-    if (lane == MAX_GROUPS) e = v4i{highs / HDMOE_NUM_CU, highs % HDMOE_NUM_CU, lows, 0};
-    if (lane <= MAX_GROUPS) groups[lane] = e;   // every wave the same
-  }
+  tile_mix(segs, args.G, lane, S224_BM, S224_FEAT, S224_LOW, 0, S224_TILES, groups);
   const int xcd = blockIdx.x % HDMOE_NUM_XCD, slot = blockIdx.x / HDMOE_NUM_XCD;
-  constexpr int nslots = HDMOE_NUM_CU / HDMOE_NUM_XCD;   // the grid is one block per CU
   v4i* const table = reinterpret_cast<v4i*>(smem + S224_TABLE) + wave * G4_TABLE_ITEMS;
   auto fill_table = [&](int base) {
     const int l = lane_now(), i = base + l;
-    const v4i mine = groups[min(l, MAX_GROUPS)];
-    const int rounds = __builtin_amdgcn_readlane(mine.x, MAX_GROUPS), left = __builtin_amdgcn_readlane(mine.y, MAX_GROUPS),
-              lows = __builtin_amdgcn_readlane(mine.z, MAX_GROUPS);
-    // whole rounds: an XCD's blocks take a contiguous eighth of the list
-    const G4Place at = g4_place(left, lows, left > 0 ? 1 : 0, xcd, slot, i - rounds);
-    const bool low = i >= rounds && at.is_short;
-    int rem = i < rounds ? xcd * (rounds * nslots) + slot + i * nslots : low ? at.tile : rounds * HDMOE_NUM_CU + at.tile;
-    int g_at = -1, mtiles = 1, ntiles = 1, L = 0, rb_at = 0, re_at = 0;
-    for (int g = 0; g < args.G; ++g) {
-      const int rb = __builtin_amdgcn_readlane(mine.x, g), re = __builtin_amdgcn_readlane(mine.y, g), mts = __builtin_amdgcn_readlane(mine.z, g),
-                nt = __builtin_amdgcn_readlane(mine.w, g), mt = low ? mts >> 16 : mts & 0xffff;
-      if (rem >= 0 && g_at < 0) {
-        if (rem < mt * nt) { g_at = g; mtiles = mt; ntiles = nt; L = rem; rb_at = rb + (low ? (mts & 0xffff) * S224_BM : 0); re_at = re; }
-        else rem -= mt * nt;
-      }
-    }
+    const MixedTile t = mixed_tile(groups, args.G, l, xcd, slot, i, S224_BM);
     v4i e = {-1, 0, 0, 0};
-    if (g_at >= 0) {
-      int m, n;
-      g4_raster(L, mtiles, ntiles, m, n);
-      const int height = low ? 32 * S224_LOW_TT : S224_BM, row0 = rb_at + m * height;
-      e = v4i{g_at | (low ? 256 : 0) | min(re_at - row0, height) << 16, row0, n, 0};
-    }
+    if (t.g >= 0) e = v4i{t.g | (t.low ? 256 : 0) | t.rows << 16, t.row0, t.n, 0};
     table[l] = e;
   };
   struct Item {

@@ -72,10 +72,10 @@ inline int g4_cut_height(int bm, int rows, int n, int rows_static, int pd, int p
 // The tiles of a segment on swiglu224_kernel (swiglu224.h): high ones of 224 rows, then low ones of 128. Styles: 0 high ones alone; 1 the last
 // one low if its rows fit; 2 what is left after full ones in low ones; 3 the last full one's rows too; 4 low ones alone.
 struct S224Mix { int highs, lows; };
-HDMOE_TAIL_HD S224Mix s224_mix(int rows, int style) {
-  const int full = (int)((unsigned)rows / 224u), rest = rows - full * 224, all = full + (rest > 0 ? 1 : 0);
+HDMOE_TAIL_HD S224Mix s224_mix(int rows, int style, int high = 224) {
+  const int full = (int)((unsigned)rows / (unsigned)high), rest = rows - full * high, all = full + (rest > 0 ? 1 : 0);
   const int keep = style == 0 || (style == 1 && rest > 128) ? all : style <= 2 ? full : style == 3 ? (full > 0 ? full - 1 : 0) : 0;
-  const int left = rows - keep * 224;
+  const int left = rows - keep * high;
   return {keep, left > 0 ? (left + 127) >> 7 : 0};
 }
 
@@ -86,11 +86,11 @@ HDMOE_TAIL_HD S224Mix s224_mix(int rows, int style) {
 // 2300 tokens and 1 % at 4096, a 30th gains nothing more). Beyond 16 rounds there is nothing to gain.
 constexpr int S224_HIGH = 100, S224_LOW = 75, S224_STYLES = 5, S224_TILES = 4096;
 HDMOE_TAIL_HD bool s224_low_pays(int cost, int whole) { return cost < whole - whole / 24; }
-HDMOE_TAIL_HD int s224_cost(int highs, int lows) {
+HDMOE_TAIL_HD int s224_cost(int highs, int lows, int low = S224_LOW) {
   const int full = highs >> 8, left = highs & 255, lights = 256 - left, light = full * S224_HIGH, heavy = light + (left > 0 ? S224_HIGH : 0);
   const int first = left > 0 ? 1 : 0, rest = lows - first * lights;
   if (rest <= 0) return heavy;
   const int q = rest >> 8, r = rest & 255;
-  const int a = light + (first + q + (r > 0 ? 1 : 0)) * S224_LOW, b = heavy + (left > 0 ? q + (r > lights ? 1 : 0) : 0) * S224_LOW;
+  const int a = light + (first + q + (r > 0 ? 1 : 0)) * low, b = heavy + (left > 0 ? q + (r > lights ? 1 : 0) : 0) * low;
   return a > b ? a : b;
 }
