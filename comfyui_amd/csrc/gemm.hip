@@ -1317,19 +1317,20 @@ int launch_swiglu4w(GemmArgs& args, int tile_bound, hipStream_t s, const char* w
   return hdmoe_check_launch(what);
 }
 
+template <bool CLAMP>
 int launch_swiglu224(GemmArgs& args, hipStream_t s, const char* what) {
   static bool attr_set[64] = {};
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) device = -1;
   if (device < 0 || !attr_set[device]) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&swiglu224_kernel),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&swiglu224_kernel<CLAMP>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, S224_SMEM);
     if (e != hipSuccess) return hdmoe_fail(HDMOE_E_LAUNCH, "%s: hipFuncSetAttribute: %s", what, hipGetErrorString(e));
     if (device >= 0) attr_set[device] = true;
   }
   fill_segments(args);
   // one block per CU whatever the number of tiles: a block without any ends at once
-  hipLaunchKernelGGL(swiglu224_kernel, dim3(HDMOE_NUM_CU), dim3(G4_THREADS), S224_SMEM, s, args);
+  hipLaunchKernelGGL(swiglu224_kernel<CLAMP>, dim3(HDMOE_NUM_CU), dim3(G4_THREADS), S224_SMEM, s, args);
   return hdmoe_check_launch(what);
 }
 
@@ -1567,8 +1568,10 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
   shape.N_dyn = N_dyn; shape.N_static = N_static;
   shape.w4_fits = true;  // settled below, once the groups are filled in
   const int K_any = n_dyn > 0 ? K_dyn : K_static;
-  shape.s224_fits = fp8 && swiglu && K_any % (2 * BK) == 0 && K_any >= 16 * BK && (shape.rows_static == 0 || (K_static == K_any && shared->scale_in2 != nullptr));
-  for (int e = 0; e < n_dyn; ++e) shape.s224_fits = shape.s224_fits && experts[e].scale_in2 != nullptr;
+  shape.s224_fits = fp8 && swiglu && K_any % (2 * BK) == 0 && K_any >= 16 * BK && (shape.rows_static == 0 || K_static == K_any);
+  const bool has_next = n_dyn > 0 ? experts[0].scale_in2 != nullptr : shared != nullptr && shared->scale_in2 != nullptr;
+  for (int e = 0; e < n_dyn; ++e) shape.s224_fits = shape.s224_fits && (experts[e].scale_in2 != nullptr) == has_next;
+  if (shape.rows_static > 0) shape.s224_fits = shape.s224_fits && (shared->scale_in2 != nullptr) == has_next;
   shape.g4_takes = g4_takes_k(n_dyn > 0 ? rows_dyn : 0, K_dyn * eb, shape.rows_static, K_static * eb);
   FormChoice choice = pick_form(shape);
   if (route != nullptr) choice = routing_form(shape);
@@ -1745,7 +1748,7 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
     shape.w4_fits = swiglu4w_fits(args, op_bytes);
     shape.s224_fits = shape.s224_fits && swiglu224_fits(args);
     choice = pick_form(shape);
-    if (choice.form == FORM_S224) return launch_swiglu224(args, s, what);
+    if (choice.form == FORM_S224) return args.g[0].s_next == nullptr ? launch_swiglu224<true>(args, s, what) : launch_swiglu224<false>(args, s, what);
   }
   switch (choice.form) {
     case FORM_RING3: {
@@ -1799,7 +1802,7 @@ extern "C" const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E,
   sh.N_dyn = H; sh.N_static = Hs;
   const int kb = D * elem_bytes(weight_dtype);
   sh.g4_takes = kb % (2 * BK) == 0 && kb >= 4 * BK;
-  sh.s224_fits = sh.fp8 && has_scale_in2 != 0 && kb % (2 * BK) == 0 && kb >= 16 * BK && H % S224_FEAT == 0 && (Hs <= 0 || Hs % S224_FEAT == 0);
+  sh.s224_fits = sh.fp8 && kb % (2 * BK) == 0 && kb >= 16 * BK && H % S224_FEAT == 0 && (Hs <= 0 || Hs % S224_FEAT == 0);
   sh.w4_fits = sh.fp8 && has_scale_in2 != 0 && kb % (2 * BK) == 0 && kb >= 16 * BK && H % W4_FEAT == 0 &&
                (Hs <= 0 || Hs % W4_FEAT == 0) && (long long)T * kb < (1ll << 31);
   switch (pick_form(sh).form) {

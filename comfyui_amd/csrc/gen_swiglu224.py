@@ -116,9 +116,9 @@ def loads(stage):
     return out
 
 
-def silu_words(src, dst):
+def silu_words(src, dst, clamp):
     """Four words (low half bf16(w1 x), high half bf16(w3 x)) src.. -> four e4m3fn bytes in dst: s = bf16(silu(g)), m = bf16(s u),
-    e4m3fn(bf16(m %[inv])), two values at a time: list of (instruction, cycles)."""
+    e4m3fn(bf16(m %[inv])), or clamp: e4m3fn(m within +-%[inv]), NaN as it is; two values at a time: list of (instruction, cycles)."""
     ga, ua, gb, ub, ta, tb, pk = range(TMP, TMP + 7)
     o = []
     for p in range(2):
@@ -135,7 +135,8 @@ def silu_words(src, dst):
               (f"v_mul_f32 v{ta}, v{ta}, v{ua}", 4), (f"v_mul_f32 v{tb}, v{tb}, v{ub}", 4),
               (f"v_cvt_pk_bf16_f32 v{pk}, v{ta}, v{tb}", 4),
               (f"v_lshlrev_b32 v{ta}, 16, v{pk}", 4), (f"v_and_b32 v{tb}, 0xffff0000, v{pk}", 4),
-              (f"v_mul_f32 v{ta}, %[inv], v{ta}", 4), (f"v_mul_f32 v{tb}, %[inv], v{tb}", 4),
+              *([(f"v_minimum3_f32 v{t}, v{t}, %[inv], %[inv]", 4) for t in (ta, tb)] + [(f"v_maximum3_f32 v{t}, v{t}, -%[inv], -%[inv]", 4) for t in (ta, tb)]
+                if clamp else [(f"v_mul_f32 v{t}, %[inv], v{t}", 4) for t in (ta, tb)]),
               (f"v_cvt_pk_bf16_f32 v{pk}, v{ta}, v{tb}", 4),
               (f"v_cvt_scalef32_pk_fp8_bf16 v{dst}, v{pk}, 1.0" + (" op_sel:[0,0,1]" if p else ""), 4)]
     return o
@@ -145,7 +146,7 @@ def piece_at(i):
     return PIECES[i] if i < len(PIECES) else PIECES[i - len(PIECES)]
 
 
-def step(stage, first, block, stored, nt):
+def step(stage, first, block, stored, nt, clamp):
     """One K step out of `stage`. Entry: the reads of its first quadrant are in flight. first: the accumulators start from zero.
     block: the deferred token block of this pair of steps (two of its pieces per step), None = none. stored: the step before ended with a
     store for certain."""
@@ -156,7 +157,7 @@ def step(stage, first, block, stored, nt):
     pieces = [] if block is None else [4 * block + 2 * stage, 4 * block + 2 * stage + 1]
     from_lds = [i for i in pieces if i in IN_LDS]
     start = at.free if from_lds else 0
-    work = Feeder([op for i in pieces for op in silu_words(piece_at(i), RES + i % 4)], at.store - 2 - start)
+    work = Feeder([op for i in pieces for op in silu_words(piece_at(i), RES + i % 4, clamp)], at.store - 2 - start)
     n_first = 4 * len(blocks(stage, nt)[0])
     L += ["s_add_u32 s76, %[so], %[kb8]", "s_add_u32 s77, %[so], %[kb64]", "s_add_u32 s78, s76, %[kb64]"]
     for q, (ft, tt) in enumerate(order):
@@ -198,19 +199,19 @@ def step(stage, first, block, stored, nt):
     return L
 
 
-def pair(first, block, nt):
-    return step(0, first, block, block not in (None, 0), nt) + step(1, False, block, False, nt)
+def pair(first, block, nt, clamp):
+    return step(0, first, block, block not in (None, 0), nt, clamp) + step(1, False, block, False, nt, clamp)
 
 
-def k_loop(nt, before):
+def k_loop(nt, before, clamp):
     """All K steps of a tile of nt blocks in pairs, %[n] of them (at least 8), behind a tile of `before`. Before the last pair the loads turn
     to the first two steps of the next tile and the row indices of the tile after it are requested. The last step reads the first quadrant of
     the next tile's first one: a lower tile's is part of it."""
     L = ["s_mov_b64 s[64:65], %[ra]", "s_mov_b64 s[66:67], %[rah]", "s_mov_b64 s[68:69], %[rb]", "s_mov_b64 s[70:71], %[rbh]",
          "s_mov_b64 s[72:73], %[rc]", "s_mov_b64 s[74:75], %[rbh]", f"s_sub_u32 %[n], %[n], {before}"]
     for b in range(before):
-        L += pair(b == 0, b, nt)
-    L += ["11:", "s_cmp_eq_u32 %[n], 1", "s_cbranch_scc1 13f", "14:"] + pair(False, None, nt)
+        L += pair(b == 0, b, nt, clamp)
+    L += ["11:", "s_cmp_eq_u32 %[n], 1", "s_cbranch_scc1 13f", "14:"] + pair(False, None, nt, clamp)
     L += ["s_sub_u32 %[n], %[n], 1", "s_cmp_lg_u32 %[n], 0", "s_cbranch_scc1 11b", "s_branch 12f"]
     L += ["13:", "s_mov_b64 s[64:65], %[na]", "s_mov_b64 s[66:67], %[nah]", "s_mov_b64 s[68:69], %[nb]", "s_mov_b64 s[72:73], %[nc]",
           "s_mov_b32 s70, %[nbn]", "s_mov_b32 s74, %[nbn]", "s_mov_b32 %[so], 0"]
@@ -240,15 +241,15 @@ def epilogue(nt):
     return L
 
 
-def tile():
+def tile(clamp):
     """A tile by its text, %[text]: 0 = 7 blocks behind a tile of 7, 1 = a low one behind a tile of 7, 2 = a low one behind a low one. (The
     blocks' tiles go from high to low.)"""
     L = ["s_cmp_eq_u32 %[text], 1", "s_cbranch_scc1 101f", "s_cmp_eq_u32 %[text], 2", "s_cbranch_scc1 102f"]
-    L += k_loop(NTT, NTT) + epilogue(NTT) + ["s_branch 109f", "101:"] + k_loop(LOW, NTT) + epilogue(LOW)
-    return L + ["s_branch 109f", "102:"] + k_loop(LOW, LOW) + epilogue(LOW) + ["109:"]
+    L += k_loop(NTT, NTT, clamp) + epilogue(NTT) + ["s_branch 109f", "101:"] + k_loop(LOW, NTT, clamp) + epilogue(LOW)
+    return L + ["s_branch 109f", "102:"] + k_loop(LOW, LOW, clamp) + epilogue(LOW) + ["109:"]
 
 
-def drain():
+def drain(clamp):
     """The deferred pieces of a block's last tile, with nothing to hide behind; %[text] other than 0: a low one."""
     L = []
     for tt in range(NTT):
@@ -258,14 +259,15 @@ def drain():
             i = 4 * tt + g
             if i in IN_LDS:
                 L += [f"ds_read_b128 {quad(piece_at(i))}, v{STG} offset:{1024 * IN_LDS.index(i)}", "s_waitcnt lgkmcnt(0)"]
-            L += [op for op, _ in silu_words(piece_at(i), RES + g)]
+            L += [op for op, _ in silu_words(piece_at(i), RES + g, clamp)]
         L += [f"buffer_store_dwordx4 {quad(RES)}, v{DEF_ST}, %[dro], 0 offen", f"v_add_u32 v{DEF_ST}, %[dldo], v{DEF_ST}"]
     return L + ["21:", "s_nop 7"]
 
 
 def generate():
     out = ["// Generated by gen_swiglu224.py; do not edit. See that script for the register map and the schedule.", ""]
-    for name, lines in (("HDMOE_S224_TILE", tile()), ("HDMOE_S224_FILL", first_reads(0, NTT)), ("HDMOE_S224_DRAIN", DRAIN_WAIT + drain())):
+    for name, lines in (("HDMOE_S224_TILE", tile(False)), ("HDMOE_S224_FILL", first_reads(0, NTT)), ("HDMOE_S224_DRAIN", DRAIN_WAIT + drain(False)),
+                        ("HDMOE_S224_TILE_CLAMP", tile(True)), ("HDMOE_S224_DRAIN_CLAMP", DRAIN_WAIT + drain(True))):
         check_trans(lines)
         out.append(f"#define {name} \\")
         out.append(" \\\n".join('  "' + ln + '\\n"' for ln in lines))

@@ -19,8 +19,8 @@
 // What a tile needs of its group sits in LDS and the first requests go out without a wait behind one another: with both read out of
 // the arguments field by field the launch of a layer of 1200 tokens took 3 us longer, and a pass of 8192 tokens 5 us.
 //
-// Limits (the launcher takes another kernel otherwise): K the same for all groups, a multiple of 256 bytes and at least 2048, every
-// group with a scale_input for the consuming Linear (no clamp form of the cast), a gathered operand under 2 GiB.
+// Limits (the launcher takes another kernel otherwise): K the same for all groups, a multiple of 256 bytes and at least 2048, the
+// consuming Linears all with a scale_input or all without, a gathered operand under 2 GiB.
 #include "swiglu224_asm.inc"
 
 constexpr int S224_BM = 224;                      // tokens per block tile
@@ -47,6 +47,10 @@ enum { S224_TOK_ADDR = 0, S224_W_ADDR = 2, S224_TOK_VOFF = 4, S224_W_VOFF = 11, 
       G4_A10(11), G4_A10(12), G4_A10(13), G4_A10(14), G4_A10(15), G4_A10(16), G4_A10(17), G4_A10(18), G4_A10(19),     \
       G4_A10(20), G4_A10(21), "a220", "a221", "a222", "a223"
 
+// CLAMP: the consuming Linears have no scale_input, their cast clamps to the fp8 range (two more vector instructions behind the MFMAs for
+// two values). Whole pass of such a layer on the 8-wave kernel -> here, us: 400 tokens 139.5 -> 115.1, 700 171 -> 144, 1300 237 -> 193, 3000 385 -> 337,
+// 4096 508 -> 444, 8192 918 -> 825.
+template <bool CLAMP>
 __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void swiglu224_kernel(const GemmArgs args) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass drops the stub of a kernel whose register operands it cannot parse
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -81,7 +85,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   const int kb = segs.bytes(0);
   auto value = [](unsigned long long p, unsigned long long or_p) { return *(const __attribute__((address_space(1))) float*)(p != 0 ? p : or_p); };
   const float v_sb0 = value(field[2].y, 0), v_sb1 = value(field[3].x, 0), v_in = value(field[3].y, field[2].y),
-              v_in_b = value(field[4].x != 0 ? field[4].x : field[3].y, field[2].y), v_next = value(field[4].y, 0);
+              v_in_b = value(field[4].x != 0 ? field[4].x : field[3].y, field[2].y), v_next = CLAMP ? 0.0f : value(field[4].y, 0);
   const bool use_alt = args.alt.flag != nullptr && sgpr(*args.alt.flag) == 0;   // the alternative token operand (GemmArgs::alt)
   v4i* const records = reinterpret_cast<v4i*>(smem + S224_RECORDS);
   v4i* const groups = reinterpret_cast<v4i*>(smem + S224_GROUPS);
@@ -249,7 +253,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   if (lane < args.G) {
     const float s_in = field[3].y != 0 ? v_in : 1.0f, s_in_b = field[4].x != 0 || field[3].y != 0 ? v_in_b : 1.0f;
     records[4 * lane + 3] = v4i{segs.n_out, __float_as_int(s_in * v_sb0), __float_as_int(s_in_b * v_sb1),
-                                __float_as_int(hdmoe_dev_round_bf16(__fdiv_rn(1.0f, v_next)))};
+                                __float_as_int(CLAMP ? 448.0f : hdmoe_dev_round_bf16(__fdiv_rn(1.0f, v_next)))};
   }
   // the tile whose activation is still to be applied (none: an empty buffer), its output pitch times 16 and its cast factor
   v4i dro = rsrc4(0, 0);
@@ -279,13 +283,16 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     const int nbn = sgpr(nxt.some() ? S224_FEAT * kb : 0);
     int n = sgpr(pairs), so = sgpr(2 * BK);
     text = sgpr(!cur.low() ? 0 : i > 0 && text == 0 ? 1 : 2);
-    asm volatile(HDMOE_S224_TILE
-                 : "+{v[128:159]}"(fa0), "+{a[224:255]}"(fb0), "+{v[96:127]}"(ctx), "+{v[38:69]}"(d0), "+{v[70:85]}"(d1),
-                   "+{v[216:247]}"(d2), "+{v[248:255]}"(d3), "={v[88:95]}"(gi), [n] "+s"(n), [so] "+s"(so)
-                 : [ra] "s"(src.a), [rah] "s"(src.ah), [rb] "s"(src.b), [rc] "s"(src.c), [rbh] "s"(bh), [na] "s"(nsrc.a), [nah] "s"(nsrc.ah),
-                   [nb] "s"(nsrc.b), [nc] "s"(nsrc.c), [nbn] "s"(nbn), [gr] "s"(gr), [dro] "s"(dro), [dldo] "s"(sgpr(dldo)), [inv] "s"(sgpr(inv)),
-                   [sc] "s"(sc), [su] "s"(su), [kb8] "s"(kb8), [kb64] "s"(kb64), [ldsw] "s"(ldsw), [text] "s"(text)
-                 : S224_CLOBBER);
+#define S224_TILE(TEXT) \
+    asm volatile(TEXT \
+                 : "+{v[128:159]}"(fa0), "+{a[224:255]}"(fb0), "+{v[96:127]}"(ctx), "+{v[38:69]}"(d0), "+{v[70:85]}"(d1), \
+                   "+{v[216:247]}"(d2), "+{v[248:255]}"(d3), "={v[88:95]}"(gi), [n] "+s"(n), [so] "+s"(so) \
+                 : [ra] "s"(src.a), [rah] "s"(src.ah), [rb] "s"(src.b), [rc] "s"(src.c), [rbh] "s"(bh), [na] "s"(nsrc.a), [nah] "s"(nsrc.ah), \
+                   [nb] "s"(nsrc.b), [nc] "s"(nsrc.c), [nbn] "s"(nbn), [gr] "s"(gr), [dro] "s"(dro), [dldo] "s"(sgpr(dldo)), [inv] "s"(sgpr(inv)), \
+                   [sc] "s"(sc), [su] "s"(su), [kb8] "s"(kb8), [kb64] "s"(kb64), [ldsw] "s"(ldsw), [text] "s"(text) \
+                 : S224_CLOBBER)
+    if constexpr (CLAMP) S224_TILE(HDMOE_S224_TILE_CLAMP);
+    else S224_TILE(HDMOE_S224_TILE);
     const v4i r2 = records[4 * cur.g() + 2], r3 = records[4 * cur.g() + 3];
     const int ldo = sgpr(r3.x);   // one byte per feature
     dro = rsrc4(pair64(r2.z, r2.w) + (uint64_t)(uint32_t)cur.row0 * (uint32_t)ldo, (uint32_t)cur.rows_here() * (uint32_t)ldo);
@@ -299,9 +306,12 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     nxt = nx2;
     nx2 = nx3;
   }
-  asm volatile(HDMOE_S224_DRAIN
-               : "+{v[128:159]}"(fa0), "+{a[224:255]}"(fb0), "+{v[96:127]}"(ctx), "+{v[38:69]}"(d0), "+{v[70:85]}"(d1), "+{v[216:247]}"(d2), "+{v[248:255]}"(d3)
-               : [dro] "s"(dro), [dldo] "s"(sgpr(dldo)), [inv] "s"(sgpr(inv)), [text] "s"(sgpr(text)) : S224_CLOBBER_V);
+#define S224_DRAIN(TEXT) \
+  asm volatile(TEXT \
+               : "+{v[128:159]}"(fa0), "+{a[224:255]}"(fb0), "+{v[96:127]}"(ctx), "+{v[38:69]}"(d0), "+{v[70:85]}"(d1), "+{v[216:247]}"(d2), "+{v[248:255]}"(d3) \
+               : [dro] "s"(dro), [dldo] "s"(sgpr(dldo)), [inv] "s"(sgpr(inv)), [text] "s"(sgpr(text)) : S224_CLOBBER_V)
+  if constexpr (CLAMP) S224_DRAIN(HDMOE_S224_DRAIN_CLAMP);
+  else S224_DRAIN(HDMOE_S224_DRAIN);
   __builtin_amdgcn_s_waitcnt(0x0f70);  // the empty requests of the last pair have come back before the LDS is given up
 #endif
 }
@@ -312,6 +322,6 @@ inline bool swiglu224_fits(const GemmArgs& args) {
   const int kb = args.g[0].kbytes;
   if (kb % (2 * BK) != 0 || kb < 16 * BK) return false;
   for (int g = 0; g < args.G; ++g)
-    if (args.g[g].kbytes != kb || args.g[g].s_next == nullptr || args.g[g].n_out % S224_FEAT != 0) return false;
+    if (args.g[g].kbytes != kb || (args.g[g].s_next == nullptr) != (args.g[0].s_next == nullptr) || args.g[g].n_out % S224_FEAT != 0) return false;
   return true;
 }

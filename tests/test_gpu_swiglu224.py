@@ -123,3 +123,32 @@ def test_graph_replays(dev, forms):
             torch.cuda.synchronize()
             assert torch.equal(static_y, want)
             assert torch.equal(m(v), want)
+
+
+@pytest.mark.parametrize("sizes,D,H", [((447, 449), 2560, 384), ((1, 0, 700, 2299), 2048, 1024), ((330,), 2048, 23040), ((225,), 2304, 32000)])
+def test_clamped(dev, forms, sizes, D, H):
+    """Consuming Linears without a scale_input: values beyond the fp8 range end at its limits, NaN stays NaN."""
+    g = torch.Generator(device=dev).manual_seed(sum(sizes) + H)
+    E, rows = len(sizes), sum(sizes)
+    assert _lib.lib.hdmoe_gate_up_kernel_name(_lib.W_E4M3FN, rows // 2, E, D, H, 0, 0) == b"swiglu224_kernel"
+    a = torch.randn((rows, D), generator=g, device=dev).to(FP8)
+    a.view(torch.uint8)[rows // 2, 5] = 0x7F   # NaN
+    offsets = torch.tensor([0] + list(torch.tensor(sizes).cumsum(0)), dtype=torch.int32, device=dev)
+    ws = [[(torch.randn((H, D), generator=g, device=dev) * 40).to(FP8) for _ in range(2)] for _ in range(E)]
+    scales = torch.tensor([[0.006, 0.02 + 0.005 * e] for e in range(E)], device=dev)
+    arr = (_lib.FfnWeights * E)()
+    for e in range(E):
+        arr[e].w1, arr[e].w3 = ws[e][0].data_ptr(), ws[e][1].data_ptr()
+        arr[e].scale_w1, arr[e].scale_w3 = scales[e, 0:].data_ptr(), scales[e, 1:].data_ptr()
+    out = []
+    for form in ("0", None):
+        set_form("HDMOE_SWIGLU4W", form)
+        h = torch.full((rows + 1, H), 0x55, dtype=torch.uint8, device=dev)
+        _lib.check(_lib.lib.hdmoe_grouped_swiglu(_lib.W_E4M3FN, a.data_ptr(), offsets.data_ptr(), rows, E, D, H, arr, h.data_ptr(), None))
+        torch.cuda.synchronize()
+        assert bool((h[rows] == 0x55).all())
+        out.append(h[:rows])
+    nan = [(h & 0x7F) == 0x7F for h in out]
+    assert bool(nan[1][rows // 2].all()) and int(nan[1].sum()) == H and torch.equal(*nan)
+    assert torch.equal(out[0][~nan[0]], out[1][~nan[1]])
+    assert bool((out[1] == 0x7E).any()) and bool((out[1] == 0xFE).any())   # both limits
