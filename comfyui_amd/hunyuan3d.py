@@ -70,16 +70,21 @@ def _need(x):
                            f"{x.device}; there is no CPU path")
 
 
-def _plain_bf16(lin, x):
-    """True when `lin` can join a grouped launch as it stands: weight (and bias) of x's dtype (bf16 or fp16) on x's
-    device, nothing to apply to them first."""
+def _plain_pair(lin, x):
+    """(weight, bias) of a Linear that can join a grouped launch as it stands: weight (and bias) of x's dtype (bf16 or fp16) on x's
+    device, nothing to apply to them first. None otherwise. (Looking a parameter up in its module takes the host as long as the rest.)"""
     if getattr(lin, "weight_function", None) or getattr(lin, "bias_function", None):
-        return False
+        return None
     if getattr(lin, "scale_weight", None) is not None:
-        return False
-    if lin.weight.dtype != x.dtype or lin.weight.device != x.device:
-        return False
-    return lin.bias is None or (lin.bias.dtype == x.dtype and lin.bias.device == x.device)
+        return None
+    weight, bias = lin.weight, lin.bias
+    if weight.dtype != x.dtype or weight.device != x.device:
+        return None
+    return (weight, bias) if bias is None or (bias.dtype == x.dtype and bias.device == x.device) else None
+
+
+def _plain_bf16(lin, x):
+    return _plain_pair(lin, x) is not None
 
 
 class FeedForward(nn.Module):
@@ -95,20 +100,24 @@ class FeedForward(nn.Module):
         self.net.append(nn.Dropout(dropout))
         self.net.append(operations.Linear(inner_dim, dim_out, device=device, dtype=dtype))
 
-    def stage_weights(self):
-        """((proj weight, bias), (out weight, bias))"""
-        return (self.net[0].proj.weight, self.net[0].proj.bias), (self.net[2].weight, self.net[2].bias)
+    def stages(self, x):
+        """((proj weight, bias), (out weight, bias)) if both Linears can join a grouped launch, else None."""
+        act, _, out = self.net
+        first = _plain_pair(act.proj, x)
+        second = _plain_pair(out, x) if first is not None else None
+        return (first, second) if second is not None else None
 
     def fusable(self, x):
-        return _plain_bf16(self.net[0].proj, x) and _plain_bf16(self.net[2], x)
+        return self.stages(x) is not None
 
     def forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
         x2 = hidden_states.reshape(-1, hidden_states.shape[-1]).contiguous()
         _need(x2)
-        if not self.fusable(x2):
+        stages = self.stages(x2)
+        if stages is None:
             y = self.net[2](self.net[0](x2))     # net[1] is Dropout, the identity at inference
             return y.view(*hidden_states.shape[:-1], y.shape[-1])
-        w_in, w_out = self.stage_weights()
+        w_in, w_out = stages
         _, h = HF.grouped_linear(x2[:0], None, [], a_static=x2, shared=w_in, act="gelu",
                                  fixed_k_cut=amd_ops._batch_invariant(self.net[0].proj))
         _, y = HF.grouped_linear(h[:0], None, [], a_static=h, shared=w_out, act="none",
@@ -164,7 +173,8 @@ class MoEBlock(nn.Module):
         gate_w = amd_ops.cast_to(self.gate.weight, dtype=x2.dtype, device=x2.device).contiguous()
         idx, w = HF.gate_top2(x2, gate_w)
         _, offsets, perm, inv_perm = HF.dispatch(idx, self.num_experts)
-        if not (all(e.fusable(x2) for e in self.experts) and self.shared_experts.fusable(x2)):
+        stages = [f.stages(x2) for f in (*self.experts, self.shared_experts)]
+        if any(v is None for v in stages):
             xs = HF.permute_bf16(x2, perm)
             y = torch.empty_like(xs)
             bounds = offsets.tolist()  # host sync: segment sizes steer the per-expert calls
@@ -173,9 +183,7 @@ class MoEBlock(nn.Module):
                 if hi > lo:
                     y[lo:hi] = expert(xs[lo:hi])
             return HF.combine(y, inv_perm, w, self.shared_experts(x2)).view(*orig_shape)
-        stage1 = [e.stage_weights()[0] for e in self.experts]
-        stage2 = [e.stage_weights()[1] for e in self.experts]
-        sh1, sh2 = self.shared_experts.stage_weights()
+        (*stage1, sh1), (*stage2, sh2) = zip(*stages)
         fixed = amd_ops._batch_invariant(self)
         # the experts' first Linear reads the routed rows through the permutation: no copy in expert order
         h, h_sh = HF.grouped_linear_tokens(x2, perm, offsets, stage1, shared=sh1, act="gelu", fixed_k_cut=fixed)
