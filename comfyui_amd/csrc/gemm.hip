@@ -1500,13 +1500,15 @@ FormChoice routing_form(const GemmShape& sh) {
   return c;
 }
 
-// Whether gate/up on 16-bit activations runs on the 4-wave kernel: what fits it, but for the three-stage ring (every segment
-// inside a 128-token tile) and the case one_round5 (hdmoe_launch_ffn_gemm).
+// Whether gate/up on 16-bit activations runs on the 4-wave kernel: what fits it, but for the three-stage ring (experts with every segment
+// inside a 128-token tile, whose tiles fill the CUs) and the case one_round5 (hdmoe_launch_ffn_gemm). A dense feed-forward of so few rows makes 54
+// tiles of 6912 features, which the ring leaves at that and the 4-wave kernel cuts along K: whole branch in bf16, us: 8 rows 68.0 -> 55.8, 64
+// 76.9 -> 62.0, 128 87.6 -> 71.0.
 bool swiglu_on_g4(const GemmShape& sh) {
   if (sh.fp8 || !sh.g4_takes) return false;
   if (sh.w8) return true;
-  if (hdmoe_few_rows(sh.rows_dyn, sh.n_dyn, sh.rows_static) && sh.rows_static <= TileCfg<2>::BM &&
-      (sh.n_dyn <= 0 || sh.rows_dyn <= TileCfg<2>::BM / 2 * sh.n_dyn))
+  if (sh.n_dyn > 0 && hdmoe_few_rows(sh.rows_dyn, sh.n_dyn, sh.rows_static) && sh.rows_static <= TileCfg<2>::BM &&
+      sh.rows_dyn <= TileCfg<2>::BM / 2 * sh.n_dyn)
     return false;
   return !pick_form(sh).one_round5;
 }
@@ -1727,7 +1729,7 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
   if (!fp8) {
     // The 4-wave kernel (gemm4w.h) takes whatever fits it: a K step of a 256 x 256 tile takes 1.36 to 1.45 us there and
     // 1.7 to 1.8 us in the 8-wave kernel (16384 x 13824 x 2560: 0.81 against 0.96 ms). Left to the 8-wave kernels: the
-    // three-stage ring for gate/up with every segment inside a 128-token tile (16-bit weights), the case one_round5, K that is
+    // three-stage ring for gate/up with every expert's segment inside a 128-token tile (16-bit weights), the case one_round5, K that is
     // not a multiple of 128, and, where tiles cannot be cut (no room for the parts), one Linear on up to 128 rows (2560 x 2560: 37
     // against 43 us: the 8-wave kernel leaves out the token blocks without rows).
     const bool g4 = gemm4w_fits(args, w8);
@@ -1806,7 +1808,9 @@ extern "C" const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E,
   sh.w4_fits = sh.fp8 && has_scale_in2 != 0 && kb % (2 * BK) == 0 && kb >= 16 * BK && H % W4_FEAT == 0 &&
                (Hs <= 0 || Hs % W4_FEAT == 0) && (long long)T * kb < (1ll << 31);
   switch (pick_form(sh).form) {
-    case FORM_RING3: return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 2, LIGHT>" : "grouped_gemm_kernel<BF16_SWIGLU, 2, LIGHT>";
+    case FORM_RING3:
+      if (swiglu_on_g4(sh)) return "gemm4w_kernel<SWIGLU>";
+      return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 2, LIGHT>" : "grouped_gemm_kernel<BF16_SWIGLU, 2, LIGHT>";
     case FORM_LIGHT4: return "grouped_gemm_kernel<FP8_SWIGLU, 4, LIGHT>";
     case FORM_W4: return "swiglu4w_kernel";
     case FORM_S224: return "swiglu224_kernel";
