@@ -686,7 +686,8 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     ctx[G4_OUT_VOFF] = part ? wave * 8192 + lane * 16
                             : (wt * 16 + fr_row) * ldo + (cur.n0() + wq * (FEAT / 2) + fr_grp * 8) * OUT_BYTES;
     const int part_s = part ? sgpr(g4_part_blocks(cur.rows_here(), wave)) + 1 : 0;
-    const int nt = sgpr(F8 || cap > 0 || (SWIGLU && !part) ? max((cur.rows_here() + 31) >> 5, G4_MIN_BLOCKS) : G4_BM / 32);   // token blocks
+    // token blocks: as its rows need (whole 256-row texts for what is not cut: Hunyuan3D block of 128 tokens 215.7 us, so 202.5; 300 230.8, 218.3)
+    const int nt = sgpr(F8 || cap > 0 || (EPI != G4_PARTIAL && !part) ? max((cur.rows_here() + 31) >> 5, G4_MIN_BLOCKS) : G4_BM / 32);
     // row indices of nx2 and this tile's biases are loaded inside the statement
     const int32_t* const list = nx2.some() ? args.g[nx2.g()].gather : nullptr;
     const v4i gr = rsrc4(list != nullptr ? list + nx2.row0() : nullptr, list != nullptr ? (uint32_t)nx2.rows_here() * 4u : 0u);
