@@ -1898,7 +1898,7 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
     if (parts > HDMOE_NUM_CU / t2) parts = HDMOE_NUM_CU / t2;
     if (parts > 6) parts = 6;
     while (parts > 1 && kt2 / parts < 6) --parts;
-    if (dyn && rows_static > 0) {
+    if (ktd > 0 && kts > 0) {   // (a width under one K step: no cut, and the call is refused)
       const long mt_s = (rows_static + bm2 - 1) / bm2;
       long mt_d = rows_dyn > n_dyn ? (rows_dyn - n_dyn) / bm2 + n_dyn : rows_dyn;   // the most that the rows make
       if (mt_d > n_dyn * mt_s) mt_d = n_dyn * mt_s;                                 // (no expert has a token twice)
