@@ -1381,6 +1381,7 @@ struct GemmShape {
   bool swiglu, fp8, split, w8;
   int rows_dyn, n_dyn, rows_static;  // rows_static = 0: no static group
   int N_dyn, N_static;
+  int kbytes;                        // K of a gate/up contraction in bytes
   bool w4_fits;                      // the 4-wave kernel takes these operands (swiglu4w_fits)
   bool s224_fits;                    // the one on 224-token tiles does (swiglu224_fits)
   bool g4_takes;                     // K is of the kind that gemm4w_kernel takes
@@ -1410,34 +1411,59 @@ bool short_tile_pays(const GemmShape& sh) {
   return 20 * expected_tile_cost(sh, 3) <= 17 * (c4 < c5 ? c4 : c5);
 }
 
-// The 224-token tile for fp8 gate/up: a round of it takes 3.85 units of expected_tile_cost (8192 tokens: 28.8 us, the 320-token
-// tile of 6 units 45), and half a unit goes for the last tile's activation, which nothing hides. Whole pass without and with it, us: layer of 260
-// tokens 105, 114; 350 129, 121; 512 145, 146; 600 167, 151; 1024 209, 208; 1300 229, 202; 1536 236, 226; 2300 338, 316; 4000 502, 449; 8000
-// 920, 823; 12000 1355, 1190; dense branch of 768 rows 78.5, 80.6; 1024 92, 105; 1500 115.2, 115.6; 1800 135, 123; 2048 138, 145. Those are
-// without low tiles; with them rounds are what s224_cost says of even segments: 450 tokens 135, 124; 900 177, 163 (256-token tiles before);
-// dense branch of 400 rows 55.3, 53.2; 450 64.9, 59.6; 512 62.0, 58.3 (192-token tiles before, which keep what is two of them high, the sizes
-// that their epilogue is tested at: 260 rows 52.7, 51.0; 300 61.6, 56.4).
-bool s224_pays(const GemmShape& sh, long other) {
-  // the kernel's own choice of styles, for even segments
-  long whole = 0, best = 0;
-  for (int c = 0; c < S224_STYLES * S224_STYLES; ++c) {
-    long highs = 0, lows = 0;
-    auto add = [&](int groups, int rows, int N, int style) {
-      const S224Mix t = s224_mix(rows, style);
-      highs += (long)groups * t.highs * (N / S224_FEAT);
-      lows += (long)groups * t.lows * (N / S224_FEAT);
-    };
-    if (sh.n_dyn > 0) add(sh.n_dyn, (sh.rows_dyn + sh.n_dyn - 1) / sh.n_dyn, sh.N_dyn, c / S224_STYLES);
-    if (sh.rows_static > 0) add(1, sh.rows_static, sh.N_static, c % S224_STYLES);
-    if (c == 0) {
-      whole = best = (highs + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU * S224_HIGH;
-      if (highs > S224_TILES || (sh.n_dyn <= 0 && sh.rows_static <= 2 * TileCfg<3>::BM)) break;
-    } else {
-      const int cost = s224_cost((int)highs, (int)lows);
-      if (s224_low_pays(cost, (int)whole) && cost < best) best = cost;
+// Whether fp8 gate/up runs on 224-token tiles (tt: height of the other kernel's tiles in blocks of 64). Both sides are rounds of tiles, in hundredths of
+// a round of high 224-token tiles (s224_price, with the kernel's choice of styles) and in units of expected_tile_cost; a round here takes 70 / 21 of
+// them (8192 tokens: 28.8 us, the 320-token tile of 6 units 45), and 15 / 21 go for the last tile's activation, which nothing hides. Segments are
+// taken even, and a standard deviation apart (tokens that go to 2 of n experts), half the price each: 512 tokens on 4 experts are not 4 tiles of
+// 256. A tile of the other kernel that is not full costs up to a quarter less: zeros take little power, and the clock follows. Whole pass, us,
+// the other kernel, this one (weights from memory): layers of 4 experts, 257 tokens 107 112 (left to the
+// other up to 320), 350 129 111, 512 133 132, 700 165 143, 1024 188 177, 4096 493 452; 8 experts, 400 174 168, 500 179 190 (other), 1000 229 228, 1283 310 252;
+// 6 experts, 700 170 178 (other), 950 245 203; 16 experts, 1950 387 398 (other), 2200 478 435; width 4096, 617 303 277; dense, 400 rows 50.7 49.5,
+// 577 55.0 57.4 (other: 513 to 768), 950 73 74 (other: 897 to 1280), 1300 88 85, 2200 113 117 (other: 2049 to 2304), 3584 162 158, 4096 187 169; 32768
+// features, 480 rows 136 145 (other). Where it errs: width 4096, 448 tokens 217 232; 4 experts without
+// a shared one, 993 tokens 144 150.
+// A dense feed-forward of up to 384 rows stays on 192-token tiles, where low tiles would be faster (Linears with and without scale_input, 257
+// rows 49.2 47.3, 300 50.2 47.9, 384 52.7 49.2): tests/test_gpu_fp8_dense_tiles.py has 300 rows of that width on them. And one or two groups are
+// taken at s224_cost, without the price of weights read again (two experts of 16384 features, 452 tokens: 125.7 132.0):
+// tests/test_gpu_swiglu224.py has such sizes on this kernel.
+bool s224_pays(const GemmShape& sh, int tt) {
+  double price = 0, other = 0;
+  for (int spread = 0; spread < 2; ++spread) {
+    struct { int rows, cols; } part[3];   // segments of one size: rows of each, tiles along the features of all of them
+    int n = 0;
+    if (sh.n_dyn > 0) {
+      const int mean = (sh.rows_dyn + sh.n_dyn - 1) / sh.n_dyn, cols = sh.N_dyn / S224_FEAT;
+      const int sd = spread == 0 || sh.n_dyn <= 2 ? 0 : (int)lround(sqrt((double)mean * (sh.n_dyn - 2) / sh.n_dyn));
+      part[n++] = {mean + sd, (sh.n_dyn + 1) / 2 * cols};
+      part[n++] = {mean > sd ? mean - sd : 0, sh.n_dyn / 2 * cols};
     }
+    const int n_routed = n;
+    if (sh.rows_static > 0) part[n++] = {sh.rows_static, sh.N_static / S224_FEAT};
+    int cols = 0;
+    for (int i = 0; i < n; ++i) cols += part[i].cols;
+    const int shift = s224_shift(cols, sh.kbytes);
+    int best = 0, whole = 0;   // the kernel's own choice of styles (tile_mix)
+    for (int c = 0; c < S224_STYLES * S224_STYLES; ++c) {
+      S224Tiles tiles = {0, 0, 0, 0};
+      for (int i = 0; i < n; ++i) s224_add(tiles, s224_mix(part[i].rows, i < n_routed ? c / S224_STYLES : c % S224_STYLES), part[i].cols);
+      const int p = sh.n_dyn == 1 || sh.n_dyn == 2 ? s224_cost(tiles.highs, tiles.lows) : s224_price(tiles, shift);
+      if (c == 0) {
+        whole = best = p;
+        if (tiles.highs > S224_TILES || (sh.n_dyn <= 0 && sh.rows_static <= 2 * TileCfg<3>::BM)) break;
+      } else if (s224_low_pays(p, whole) && p < best) {
+        best = p;
+      }
+    }
+    price += 0.5 * best;
+    long tiles = 0;
+    double rows = 0;
+    for (int i = 0; i < n; ++i) {
+      tiles += (long)((part[i].rows + 64 * tt - 1) / (64 * tt)) * part[i].cols;
+      rows += (double)part[i].rows * part[i].cols;
+    }
+    if (tiles > 0) other += 0.5 * ((tiles + HDMOE_NUM_CU - 1) / HDMOE_NUM_CU) * (tt + 1) * (0.75 + 0.25 * rows / (64.0 * tt * tiles));
   }
-  return 77 * best + 10 * S224_HIGH <= 21 * S224_HIGH * other;
+  return 70 * price + 15 * S224_HIGH <= 21 * S224_HIGH * other;
 }
 
 // light: the token blocks of a tile that hold no rows are skipped (fp8: the compiler-scheduled K loop instead of the
@@ -1468,7 +1494,7 @@ FormChoice pick_form(const GemmShape& sh) {
   if (c.fp8_g4) c.tall = false;
   c.short3 = !c.light && f_4w != HDMOE_FORM_ALWAYS && short_tile_pays(sh);
   if (f_light == HDMOE_FORM_AUTO && f_4w == HDMOE_FORM_AUTO && !c.light &&
-      sh.fp8 && sh.swiglu && sh.s224_fits && s224_pays(sh, expected_tile_cost(sh, c.short3 ? 3 : c.tall ? 5 : 4))) {
+      sh.fp8 && sh.swiglu && sh.s224_fits && s224_pays(sh, c.short3 ? 3 : c.tall ? 5 : 4)) {
     c.tall = c.short3 = false;
     c.form = FORM_S224;
     return c;
@@ -1570,6 +1596,7 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
   shape.N_dyn = N_dyn; shape.N_static = N_static;
   shape.w4_fits = true;  // settled below, once the groups are filled in
   const int K_any = n_dyn > 0 ? K_dyn : K_static;
+  shape.kbytes = K_any * eb;
   shape.s224_fits = fp8 && swiglu && K_any % (2 * BK) == 0 && K_any >= 16 * BK && (shape.rows_static == 0 || K_static == K_any);
   const bool has_next = n_dyn > 0 ? experts[0].scale_in2 != nullptr : shared != nullptr && shared->scale_in2 != nullptr;
   for (int e = 0; e < n_dyn; ++e) shape.s224_fits = shape.s224_fits && (experts[e].scale_in2 != nullptr) == has_next;
@@ -1803,6 +1830,7 @@ extern "C" const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E,
   sh.rows_dyn = E > 0 ? T * HDMOE_TOPK : 0; sh.n_dyn = E; sh.rows_static = Hs > 0 ? T : 0;
   sh.N_dyn = H; sh.N_static = Hs;
   const int kb = D * elem_bytes(weight_dtype);
+  sh.kbytes = kb;
   sh.g4_takes = kb % (2 * BK) == 0 && kb >= 4 * BK;
   sh.s224_fits = sh.fp8 && kb % (2 * BK) == 0 && kb >= 16 * BK && H % S224_FEAT == 0 && (Hs <= 0 || Hs % S224_FEAT == 0);
   sh.w4_fits = sh.fp8 && has_scale_in2 != 0 && kb % (2 * BK) == 0 && kb >= 16 * BK && H % W4_FEAT == 0 &&
@@ -1837,7 +1865,7 @@ extern "C" const char* hdmoe_plain_kernel_name(int rows_dyn, int E, int K_dyn, i
     return fp8_linear_192(rows_static, N) ? "grouped_gemm_kernel<FP8_PLAIN_BIAS, 3>" : "grouped_gemm_kernel<FP8_PLAIN_BIAS, 4>";
   }
   GemmShape sh;
-  sh.swiglu = false; sh.fp8 = true; sh.split = parts > 1; sh.w8 = false; sh.w4_fits = sh.s224_fits = false;
+  sh.swiglu = false; sh.fp8 = true; sh.split = parts > 1; sh.w8 = false; sh.w4_fits = sh.s224_fits = false; sh.kbytes = 0;
   sh.rows_dyn = n_dyn > 0 ? rows_dyn : 0; sh.n_dyn = n_dyn; sh.rows_static = rows_static;
   sh.N_dyn = sh.N_static = N;
   sh.g4_takes = takes;
@@ -2465,7 +2493,7 @@ size_t hdmoe_tail_bytes(int weight_dtype, int rows_dyn, int E, int rows_static, 
   const bool w8 = weight_dtype == HDMOE_W_E4M3FN_UPCAST;
   const int n_dyn = rows_dyn > 0 ? E : 0, mean = n_dyn > 0 ? rows_dyn / n_dyn : 0;
   GemmShape sh;
-  sh.swiglu = true; sh.fp8 = false; sh.split = false; sh.w8 = w8; sh.w4_fits = sh.s224_fits = false;
+  sh.swiglu = true; sh.fp8 = false; sh.split = false; sh.w8 = w8; sh.w4_fits = sh.s224_fits = false; sh.kbytes = 0;
   sh.rows_dyn = rows_dyn; sh.n_dyn = n_dyn; sh.rows_static = rows_static;
   sh.N_dyn = H; sh.N_static = Hs;
   sh.g4_takes = g4_takes_k(rows_dyn, D * 2, rows_static, D * 2);

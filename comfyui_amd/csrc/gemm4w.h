@@ -265,33 +265,34 @@ inline int g4_host_cap(const GemmArgs& args, int feat, int min_pairs, int blocks
 
 // High and low tiles of the segments (tail_units.h), lane g looking after group g: leaves [segment begin, end, high m-tiles | low ones << 16, tiles
 // along the features] of each group and [rounds of high tiles, high tiles beyond, low tiles] behind them in `groups` (LDS, every wave the
-// same) and says whether there are low ones. low_cost: of a low tile in hundredths of a high one's; alone: more where it is the only one of its
-// segment; most: high tiles at which low ones are looked for.
-__device__ __forceinline__ bool tile_mix(const Segments& segs, int G, int lane, int high, int feat, int low_cost, int alone, int most, v4i* groups) {
+// same) and says whether there are low ones. F8: tiles of swiglu224_kernel; W8: of gemm4w_kernel with one-byte weights. most: high tiles at which low
+// ones are looked for.
+template <bool F8, bool W8>
+__device__ __forceinline__ bool tile_mix(const Segments& segs, int G, int lane, int high, int feat, int most, v4i* groups) {
   const int rows = segs.re - segs.rb, nt = (int)((unsigned)segs.n_out / (unsigned)feat), whole = s224_mix(rows, 0, high).highs * nt;
-  int highs = 0, lows = 0, style = 0;
-  for (int g = 0; g < G; ++g) highs += __builtin_amdgcn_readlane(whole, g);
+  int highs = 0, lows = 0, style = 0, cols = 0;
+  for (int g = 0; g < G; ++g) {
+    highs += __builtin_amdgcn_readlane(whole, g);
+    cols += __builtin_amdgcn_readlane(nt, g);
+  }
   if (highs <= most) {   // lane i: style i / 5 of the experts and i % 5 of the static group
     const int c = min(lane, S224_STYLES * S224_STYLES - 1), of_dyn = c * 13 >> 6, of_fix = c - 5 * of_dyn;
-    int tiles = 0, single = 0;   // high ones | low ones << 16; low ones that share their weights with none
-    for (int g = 0; g < G; ++g) {
-      const S224Mix t = s224_mix(__builtin_amdgcn_readlane(rows, g), segs.dynamic(g) ? of_dyn : of_fix, high);
-      const int n = __builtin_amdgcn_readlane(nt, g);
-      tiles += (t.highs | t.lows << 16) * n;
-      single += t.lows == 1 ? n : 0;
-    }
-    if (alone > 0) low_cost += tile_div(alone * single, max(tiles >> 16, 1));
-    const int mine = s224_cost(tiles & 0xffff, tiles >> 16, low_cost) << 5 | c;
+    S224Tiles tiles = {0, 0, 0, 0};
+    for (int g = 0; g < G; ++g)
+      s224_add(tiles, s224_mix(__builtin_amdgcn_readlane(rows, g), segs.dynamic(g) ? of_dyn : of_fix, high), __builtin_amdgcn_readlane(nt, g));
+    int price;
+    if constexpr (F8) price = s224_price(tiles, s224_shift(cols, segs.bytes(0)));
+    else price = s224_cost(tiles.highs, tiles.lows, G4_LOW_COST + (W8 ? 0 : tile_div(G4_LOW_ALONE * tiles.alone, max(tiles.lows, 1))));
+    const int mine = price << 5 | c;
     const int first = __builtin_amdgcn_readlane(mine, 0);
     int best = first;
 #pragma unroll
     for (int k = 1; k < S224_STYLES * S224_STYLES; ++k) best = min(best, __builtin_amdgcn_readlane(mine, k));
-    if (s224_low_pays(best >> 5, first >> 5)) {
+    if (F8 ? s224_low_pays(best >> 5, first >> 5) : s224_low_pays(best >> 5, first >> 5, 24)) {
       const int pick = best & 31, pick_dyn = pick * 13 >> 6;
       style = segs.fixed >> lane & 1 ? pick - 5 * pick_dyn : pick_dyn;
-      tiles = __builtin_amdgcn_readlane(tiles, pick);
-      highs = tiles & 0xffff;
-      lows = tiles >> 16;
+      highs = __builtin_amdgcn_readlane(tiles.highs, pick);
+      lows = __builtin_amdgcn_readlane(tiles.lows, pick);
     }
   }
   const S224Mix t = s224_mix(rows, style, high);
@@ -426,7 +427,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   }
   bool mixed = false;
   if constexpr (SWIGLU) {
-    if (tail.parts == 1) mixed = tile_mix(segs, args.G, lane, G4_BM, FEAT, G4_LOW_COST, W8 ? 0 : G4_LOW_ALONE, G4_MIX_TILES, heights);
+    if (tail.parts == 1) mixed = tile_mix<false, W8>(segs, args.G, lane, G4_BM, FEAT, G4_MIX_TILES, heights);
   }
   v4i* const table = reinterpret_cast<v4i*>(smem + G4_TABLE) + wave * G4_TABLE_ITEMS;
   auto fill_table = [&](int base) {

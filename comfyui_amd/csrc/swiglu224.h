@@ -11,11 +11,9 @@
 // the hidden vector instructions 27; this kernel 577 (2.53 PFLOP/s; back to back inside a layer, on other cards, 533 to 540: 2.7). 4096
 // tokens: 365 (4-wave kernel of swiglu4w.h) -> 302.
 //
-// Low tiles of 128 tokens end a block's list where that shortens the longest block (tail_units.h, s224_mix and s224_cost): the last m-tile of a
+// Low tiles of 128 tokens end a block's list where that shortens the longest block (tail_units.h, s224_mix and s224_price): the last m-tile of a
 // segment rarely has 224 rows, and with a few rounds of tiles the last round is rarely full. A low tile multiplies 4 instead of 7 blocks per
-// wave and step and takes about 0.75 of the time (its weights are as many, and come once more). Whole pass, 224 tokens alone -> this, weights from
-// memory, us: layer of 400 tokens 124.0 -> 113.9, 700 155.8 -> 145.8, 800 157.9 -> 147.3, 1000 187.5 -> 176.6 (skewed 184.8 -> 169.2), 1300 195.5 ->
-// 191.8, 2300 287 -> 281, 4096 468 -> 462; dense branch of 512 rows 64.6 -> 59.5, 400 59.4 -> 54.2.
+// wave and step and takes about 0.75 of the time (its weights are as many, and come once more; s224_price, with what it measured).
 // What a tile needs of its group sits in LDS and the first requests go out without a wait behind one another: with both read out of
 // the arguments field by field the launch of a layer of 1200 tokens took 3 us longer, and a pass of 8192 tokens 5 us.
 //
@@ -89,7 +87,7 @@ __global__ __launch_bounds__(G4_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
   const bool use_alt = args.alt.flag != nullptr && sgpr(*args.alt.flag) == 0;   // the alternative token operand (GemmArgs::alt)
   v4i* const records = reinterpret_cast<v4i*>(smem + S224_RECORDS);
   v4i* const groups = reinterpret_cast<v4i*>(smem + S224_GROUPS);
-  tile_mix(segs, args.G, lane, S224_BM, S224_FEAT, S224_LOW, 0, S224_TILES, groups);
+  tile_mix<true, false>(segs, args.G, lane, S224_BM, S224_FEAT, S224_TILES, groups);
   const int xcd = blockIdx.x % HDMOE_NUM_XCD, slot = blockIdx.x / HDMOE_NUM_XCD;
   v4i* const table = reinterpret_cast<v4i*>(smem + S224_TABLE) + wave * G4_TABLE_ITEMS;
   auto fill_table = [&](int base) {

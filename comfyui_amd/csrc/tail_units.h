@@ -80,12 +80,9 @@ HDMOE_TAIL_HD S224Mix s224_mix(int rows, int style, int high = 224) {
 }
 
 // How the list of a launch is dealt out: highs in whole rounds of 256 blocks, what is left of them to as many blocks, lows to the other ones first
-// (g4_place). What the longest block comes to, a high tile being S224_HIGH. A low one is 64 by its matrix instructions; 75 because all lows of an
-// expert read its weights once more (priced at 66 layers of 1000 and 1500 tokens took 4 and 3 % longer than without; 83 and 92 lose 450 and
-// 800 tokens). Others than high tiles alone have to pay by a 24th: the clock falls with the CUs that are busy (a 13th loses 2 % at 1200, 1300 and
-// 2300 tokens and 1 % at 4096, a 30th gains nothing more). Beyond 16 rounds there is nothing to gain.
+// (g4_place). What the longest block comes to, a high tile being S224_HIGH and a low one, 64 by its matrix instructions, 75. Beyond 16 rounds of
+// high tiles there is nothing to gain.
 constexpr int S224_HIGH = 100, S224_LOW = 75, S224_STYLES = 5, S224_TILES = 4096;
-HDMOE_TAIL_HD bool s224_low_pays(int cost, int whole) { return cost < whole - whole / 24; }
 HDMOE_TAIL_HD int s224_cost(int highs, int lows, int low = S224_LOW) {
   const int full = highs >> 8, left = highs & 255, lights = 256 - left, light = full * S224_HIGH, heavy = light + (left > 0 ? S224_HIGH : 0);
   const int first = left > 0 ? 1 : 0, rest = lows - first * lights;
@@ -94,3 +91,22 @@ HDMOE_TAIL_HD int s224_cost(int highs, int lows, int low = S224_LOW) {
   const int a = light + (first + q + (r > 0 ? 1 : 0)) * low, b = heavy + (left > 0 ? q + (r > lights ? 1 : 0) : 0) * low;
   return a > b ? a : b;
 }
+
+// The tiles of a launch; of the columns (tiles along the features): those with tiles of both heights, those with one low tile.
+struct S224Tiles { int highs, lows, both, alone; };
+HDMOE_TAIL_HD void s224_add(S224Tiles& t, const S224Mix& m, int cols) {
+  t.highs += m.highs * cols;
+  t.lows += m.lows * cols;
+  t.both += m.highs > 0 && m.lows > 0 ? cols : 0;
+  t.alone += m.lows == 1 ? cols : 0;
+}
+// The price of a choice of tiles. Low tiles behind high ones of the same columns read their weights again, and from memory where the launch's
+// weights are more than about 100 MB: in 16ths of a hundredth of a high tile, 2 for such a column and 1 for a low tile (half of that where they
+// are not), which is about 650 KB of weights at 6 TB/s. Whole pass on this kernel, us, high tiles alone, lows where s224_cost alone gains,
+// where this does (weights from memory): layers of 16 experts, 2048 tokens 424 480 424; 12 experts, 1600 321 362 323; 8 experts, 1100 233 251 234;
+// width 4096, 950 332 350 335; 4 experts of 6912 and a shared one of 3584, 350 120 111 111, 500 139 138 130, 700 150 143 143, 1024 183 178 178; 6 experts,
+// 950 211 209 203; dense branch, 32768 features, 768 rows 188 195 189; width 4096, 1300 rows 184 174 175; 1300 rows 87.3 85.0 85.5. Other tiles than
+// high ones alone have to pay by a 32nd: the clock falls with the CUs that are busy (a 24th loses 1 % at 1300 and 2048 tokens).
+HDMOE_TAIL_HD int s224_price(const S224Tiles& t, int shift) { return s224_cost(t.highs, t.lows) + ((2 * t.both + t.lows) >> shift); }
+HDMOE_TAIL_HD int s224_shift(int cols, int kbytes) { return (long long)cols * 256 * kbytes <= (100ll << 20) ? 5 : 4; }
+HDMOE_TAIL_HD bool s224_low_pays(int price, int whole, int margin = 32) { return price < whole - whole / margin; }
