@@ -1526,16 +1526,22 @@ FormChoice routing_form(const GemmShape& sh) {
   return c;
 }
 
-// Whether gate/up on 16-bit activations runs on the 4-wave kernel: what fits it, but for the three-stage ring (experts with every segment
-// inside a 128-token tile, whose tiles fill the CUs) and the case one_round5 (hdmoe_launch_ffn_gemm). A dense feed-forward of so few rows makes 54
-// tiles of 6912 features, which the ring leaves at that and the 4-wave kernel cuts along K: whole branch in bf16, us: 8 rows 68.0 -> 55.8, 64
-// 76.9 -> 62.0, 128 87.6 -> 71.0.
-bool swiglu_on_g4(const GemmShape& sh) {
+// Whether gate/up on 16-bit activations runs on the 4-wave kernel: what fits it, but for the three-stage ring (every segment inside a 128-token
+// tile) and the case one_round5 (hdmoe_launch_ffn_gemm). Of the ring's sizes a dense feed-forward goes to the 4-wave kernel where that cuts its
+// tiles along K (has_room: the working memory holds the parts), so that more of the CUs fetch weights. Whole branch in bf16, us, ring -> cut: 2560 x
+// 6912 (54 tiles in 4 parts), 1 row 59.3 -> 47.9, 64 67.0 -> 54.1, 128 79.4 -> 61.4; 2560 x 1024, 64 38.7 -> 32.8; 4096 x 11008 (2 parts) 96.0 -> 89.4; 5120 x
+// 13824 (2 parts) 134.4 -> 116.6. Not cut, ring and 4-wave kernel: 2560 x 6912 without the room, 64 rows 66.9 72.9; 512 x 6912 28.3 30.8; 2560 x 16384,
+// 64 rows 91.2 96.2; 2560 x 32768 138.7 141.8. (512 x 256, which are two tiles, 18.3 20.8: under a tile for each XCD it is the launch that counts, and
+// tests/test_gpu_dense_few_rows.py has these on the 4-wave kernel.)
+bool swiglu_on_g4(const GemmShape& sh, bool has_room) {
   if (sh.fp8 || !sh.g4_takes) return false;
   if (sh.w8) return true;
-  if (sh.n_dyn > 0 && hdmoe_few_rows(sh.rows_dyn, sh.n_dyn, sh.rows_static) && sh.rows_static <= TileCfg<2>::BM &&
-      sh.rows_dyn <= TileCfg<2>::BM / 2 * sh.n_dyn)
-    return false;
+  if (hdmoe_few_rows(sh.rows_dyn, sh.n_dyn, sh.rows_static) && sh.rows_static <= TileCfg<2>::BM &&
+      (sh.n_dyn <= 0 || sh.rows_dyn <= TileCfg<2>::BM / 2 * sh.n_dyn)) {
+    if (sh.n_dyn > 0) return false;
+    return sh.N_static / (BN / 2) < HDMOE_NUM_XCD ||
+           (has_room && g4_tail_room(0, 0, 0, 0, sh.rows_static, sh.N_static, sh.kbytes, BN / 2, false) > 0);
+  }
   return !pick_form(sh).one_round5;
 }
 
@@ -1756,7 +1762,7 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
   if (!fp8) {
     // The 4-wave kernel (gemm4w.h) takes whatever fits it: a K step of a 256 x 256 tile takes 1.36 to 1.45 us there and
     // 1.7 to 1.8 us in the 8-wave kernel (16384 x 13824 x 2560: 0.81 against 0.96 ms). Left to the 8-wave kernels: the
-    // three-stage ring for gate/up with every expert's segment inside a 128-token tile (16-bit weights), the case one_round5, K that is
+    // three-stage ring for gate/up with every segment inside a 128-token tile (16-bit weights, unless cut: swiglu_on_g4), the case one_round5, K that is
     // not a multiple of 128, and, where tiles cannot be cut (no room for the parts), one Linear on up to 128 rows (2560 x 2560: 37
     // against 43 us: the 8-wave kernel leaves out the token blocks without rows).
     const bool g4 = gemm4w_fits(args, w8);
@@ -1766,7 +1772,7 @@ int hdmoe_launch_ffn_gemm(bool swiglu, int weight_dtype, const uint8_t* a_dyn, c
                     : launch_gemm4w<G4_W8, G4_PLAIN>(args, rows_mean, s, what);
     }
     if (choice.one_round5) return launch_grouped<BF16_SWIGLU, 5>(args, tile_bound, s, what);
-    if (swiglu && g4 && swiglu_on_g4(shape)) return launch_gemm4w<G4_BF16, G4_SWIGLU>(args, rows_mean, s, what);
+    if (swiglu && g4 && swiglu_on_g4(shape, tail != nullptr)) return launch_gemm4w<G4_BF16, G4_SWIGLU>(args, rows_mean, s, what);
     if (!swiglu && g4 && (tail != nullptr || rows_mean > 128 || rows_static > 128))
       return launch_gemm4w<G4_BF16, G4_PLAIN>(args, rows_mean, s, what);
   }
@@ -1837,7 +1843,7 @@ extern "C" const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E,
                (Hs <= 0 || Hs % W4_FEAT == 0) && (long long)T * kb < (1ll << 31);
   switch (pick_form(sh).form) {
     case FORM_RING3:
-      if (swiglu_on_g4(sh)) return "gemm4w_kernel<SWIGLU>";
+      if (swiglu_on_g4(sh, true)) return "gemm4w_kernel<SWIGLU>";
       return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 2, LIGHT>" : "grouped_gemm_kernel<BF16_SWIGLU, 2, LIGHT>";
     case FORM_LIGHT4: return "grouped_gemm_kernel<FP8_SWIGLU, 4, LIGHT>";
     case FORM_W4: return "swiglu4w_kernel";
@@ -1846,7 +1852,7 @@ extern "C" const char* hdmoe_gate_up_kernel_name(int weight_dtype, int T, int E,
     case FORM_TALL5: return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 5>" : "grouped_gemm_kernel<BF16_SWIGLU, 5>";
     default:
       if (pick_form(sh).one_round5) return "grouped_gemm_kernel<BF16_SWIGLU, 5>";
-      if (!sh.fp8 && sh.g4_takes) return "gemm4w_kernel<SWIGLU>";
+      if (swiglu_on_g4(sh, true)) return "gemm4w_kernel<SWIGLU>";
       return sh.fp8 ? "grouped_gemm_kernel<FP8_SWIGLU, 4>" : "grouped_gemm_kernel<BF16_SWIGLU, 4>";
   }
 }
@@ -2493,11 +2499,11 @@ size_t hdmoe_tail_bytes(int weight_dtype, int rows_dyn, int E, int rows_static, 
   const bool w8 = weight_dtype == HDMOE_W_E4M3FN_UPCAST;
   const int n_dyn = rows_dyn > 0 ? E : 0, mean = n_dyn > 0 ? rows_dyn / n_dyn : 0;
   GemmShape sh;
-  sh.swiglu = true; sh.fp8 = false; sh.split = false; sh.w8 = w8; sh.w4_fits = sh.s224_fits = false; sh.kbytes = 0;
+  sh.swiglu = true; sh.fp8 = false; sh.split = false; sh.w8 = w8; sh.w4_fits = sh.s224_fits = false; sh.kbytes = D * 2;
   sh.rows_dyn = rows_dyn; sh.n_dyn = n_dyn; sh.rows_static = rows_static;
   sh.N_dyn = H; sh.N_static = Hs;
   sh.g4_takes = g4_takes_k(rows_dyn, D * 2, rows_static, D * 2);
-  const size_t up = swiglu_on_g4(sh) ? g4_tail_room(n_dyn, mean, H, D * 2, rows_static, Hs, D * 2, BN / 2, w8) : 0;
+  const size_t up = swiglu_on_g4(sh, true) ? g4_tail_room(n_dyn, mean, H, D * 2, rows_static, Hs, D * 2, BN / 2, w8) : 0;
   const size_t down = down_uncut ? g4_tail_room(n_dyn, mean, D, H * 2, rows_static, D, Hs * 2, BN, w8) : 0;
   return up > down ? up : down;
 }
