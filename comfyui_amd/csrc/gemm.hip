@@ -1890,8 +1890,9 @@ extern "C" const char* hdmoe_plain_kernel_name(int rows_dyn, int E, int K_dyn, i
 // blocks lasts as long as its longest tile; more tiles than CUs last about the total divided by the CUs plus half a
 // tile of slack; a cut adds the fp32 partial sums written and read again (8 bytes per output and part; they stay in
 // the memory-side cache at these sizes, about 10 TB/s; one step is about 1.4 us).
+// less_room: the cut of few rows that takes less room, for a workspace that holds no more (hdmoe_moe_ffn).
 int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn, int K_static, int weight_dtype,
-                     HdmoeSplitPlan* plan) {
+                     HdmoeSplitPlan* plan, bool less_room) {
   HdmoeSplitPlan local;
   HdmoeSplitPlan& pl = plan != nullptr ? *plan : local;
   memset(&pl, 0, sizeof(pl));
@@ -1916,7 +1917,7 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
   // 77.8 77.3 -> 75.0 74.4, 256 99.2 95.7 -> 94.0 91.4; bf16, 64 115.9 110.1 -> 110.3 102.4, 256 157.1 148.3 -> 146.2 139.9; e4m3fn weights in bf16,
   // 64 109.4 108.6 -> 100.0 98.7, 256 134.6 135.3 -> 121.3 120.4. (Five parts of every tile, the shared expert's too: 64 tokens in fp8 72.3; the
   // most parts that fit the real segments, picked on the device: 256 tokens 95.1, 200 89.0 where this has 90.8.)
-  // A dense feed-forward, and what fits no round: about 150 blocks keep enough loads in flight; segments counted 1.5 times the mean.
+  // A dense feed-forward, what fits no round, and less_room: about 150 blocks keep enough loads in flight; segments counted 1.5 times the mean.
   if (hdmoe_few_rows(rows_dyn, n_dyn, rows_static)) {
     const int bm2 = TileCfg<2>::BM;
     pl.bm = bm2;
@@ -1932,7 +1933,7 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
     if (parts > HDMOE_NUM_CU / t2) parts = HDMOE_NUM_CU / t2;
     if (parts > 6) parts = 6;
     while (parts > 1 && kt2 / parts < 6) --parts;
-    if (ktd > 0 && kts > 0) {   // (a width under one K step: no cut, and the call is refused)
+    if (ktd > 0 && kts > 0 && !less_room) {   // (a width under one K step: no cut, and the call is refused)
       const long mt_s = (rows_static + bm2 - 1) / bm2;
       long mt_d = rows_dyn > n_dyn ? (rows_dyn - n_dyn) / bm2 + n_dyn : rows_dyn;   // the most that the rows make
       if (mt_d > n_dyn * mt_s) mt_d = n_dyn * mt_s;                                 // (no expert has a token twice)

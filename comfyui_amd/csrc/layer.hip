@@ -24,7 +24,7 @@ int hdmoe_launch_combine_partials(const float* partial, long long part_stride, c
                                   const void* gate_bf16, const void* residual_bf16, int tokens_per_batch, int T, int D,
                                   void* out_bf16, hipStream_t s, const char* what);
 int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn, int K_static, int weight_dtype,
-                     HdmoeSplitPlan* plan = nullptr);
+                     HdmoeSplitPlan* plan = nullptr, bool less_room = false);
 int hdmoe_check_gemm_shape(const char* what, int weight_dtype, long rows, int K, int N, int feat_per_tile);
 int hdmoe_launch_quant_dispatch(const void* x_bf16, const int32_t* perm, const int32_t* offsets, int T, int D, int E,
                                 const float* const* scale_input, const float* shared_scale, bool with_shared,
@@ -56,9 +56,9 @@ extern "C" int hdmoe_version(void) { return HDMOE_VERSION; }
 extern "C" const char* hdmoe_last_error(void) { return hdmoe_error_buffer(); }
 
 namespace {
-size_t layer_down_bytes(int T, int D, int H, int Hs, int E, int weight_dtype) {
+size_t layer_down_bytes(int T, int D, int H, int Hs, int E, int weight_dtype, bool less_room) {
   const size_t n = (size_t)T * HDMOE_TOPK;
-  const int parts = hdmoe_down_parts((int)n, E, Hs > 0 ? T : 0, D, H, Hs, weight_dtype);
+  const int parts = hdmoe_down_parts((int)n, E, Hs > 0 ? T : 0, D, H, Hs, weight_dtype, nullptr, less_room);
   return parts > 1 ? (size_t)parts * (n + (Hs > 0 ? (size_t)T : 0)) * D * 4 : 0;
 }
 size_t ffn_down_bytes(int rows, int D, int H, int weight_dtype) {
@@ -67,13 +67,8 @@ size_t ffn_down_bytes(int rows, int D, int H, int weight_dtype) {
 }
 }  // namespace
 
-extern "C" int hdmoe_layer_layout_get(int T, int D, int H, int Hs, int E, int weight_dtype,
-                                      hdmoe_layer_layout* out) {
-  HDMOE_REQUIRE_PTR(out);
-  if (T < 0 || D <= 0 || H <= 0 || Hs < 0 || E < 1 || E > HDMOE_MAX_EXPERTS ||
-      (weight_dtype != HDMOE_W_BF16 && weight_dtype != HDMOE_W_E4M3FN && weight_dtype != HDMOE_W_E4M3FN_UPCAST))
-    return hdmoe_fail(HDMOE_E_SHAPE, "hdmoe_layer_layout_get: T=%d D=%d H=%d Hs=%d E=%d dtype=%d", T, D, H, Hs, E,
-                      weight_dtype);
+// T, D and the others as hdmoe_layer_layout_get has checked them; less_room as in hdmoe_down_parts
+static void layer_layout(int T, int D, int H, int Hs, int E, int weight_dtype, bool less_room, hdmoe_layer_layout* out) {
   const size_t eb = weight_dtype == HDMOE_W_E4M3FN ? 1 : 2;
   const size_t n = (size_t)T * HDMOE_TOPK;
   const bool fp8 = weight_dtype == HDMOE_W_E4M3FN;
@@ -101,7 +96,7 @@ extern "C" int hdmoe_layer_layout_get(int T, int D, int H, int Hs, int E, int we
   // normalised + modulated tokens of the optional block fusion, [T,D] bf16
   out->normed = take((size_t)T * D * 2);
   // fp32 partial sums of a down projection cut along K (small token counts), [parts][2T + T][D]
-  const size_t down_bytes = layer_down_bytes(T, D, H, Hs, E, weight_dtype);
+  const size_t down_bytes = layer_down_bytes(T, D, H, Hs, E, weight_dtype, less_room);
   out->partials = take(down_bytes);
   // one word the gate + cast kernel leaves for the gate/up GEMM: which layout of the fp8 tokens it wrote
   out->flags = take(256);
@@ -110,6 +105,16 @@ extern "C" int hdmoe_layer_layout_get(int T, int D, int H, int Hs, int E, int we
   const size_t tail_bytes = T > 0 ? hdmoe_tail_bytes(weight_dtype, (int)n, E, Hs > 0 ? T : 0, D, H, Hs, down_bytes == 0) : 0;
   if (tail_bytes > down_bytes) take(tail_bytes);
   out->total = off;
+}
+
+extern "C" int hdmoe_layer_layout_get(int T, int D, int H, int Hs, int E, int weight_dtype,
+                                      hdmoe_layer_layout* out) {
+  HDMOE_REQUIRE_PTR(out);
+  if (T < 0 || D <= 0 || H <= 0 || Hs < 0 || E < 1 || E > HDMOE_MAX_EXPERTS ||
+      (weight_dtype != HDMOE_W_BF16 && weight_dtype != HDMOE_W_E4M3FN && weight_dtype != HDMOE_W_E4M3FN_UPCAST))
+    return hdmoe_fail(HDMOE_E_SHAPE, "hdmoe_layer_layout_get: T=%d D=%d H=%d Hs=%d E=%d dtype=%d", T, D, H, Hs, E,
+                      weight_dtype);
+  layer_layout(T, D, H, Hs, E, weight_dtype, false, out);
   return HDMOE_OK;
 }
 
@@ -130,6 +135,14 @@ extern "C" int hdmoe_moe_ffn(const hdmoe_layer_args* p, hdmoe_stream_t stream) {
   hdmoe_layer_layout l;
   if (int rc = hdmoe_layer_layout_get(T, D, H, Hs, E, wd, &l)) return rc;
   if (Hs > 0) HDMOE_REQUIRE_PTR(p->shared);
+  // a workspace that does not hold it all: fewer parts of a down projection of few rows
+  bool less_room = false;
+  if (p->workspace_bytes < l.total) {
+    hdmoe_layer_layout less;
+    layer_layout(T, D, H, Hs, E, wd, true, &less);
+    less_room = less.total < l.total;
+    if (less_room) l = less;
+  }
   const size_t need = l.flags + 256;   // the parts of tail tiles may do without theirs
   if (p->workspace_bytes < need || (reinterpret_cast<uintptr_t>(p->workspace) & 255))
     return hdmoe_fail(HDMOE_E_WORKSPACE, "hdmoe_moe_ffn: workspace %zu bytes, need %zu (256-byte aligned)",
@@ -295,7 +308,7 @@ extern "C" int hdmoe_moe_ffn(const hdmoe_layer_args* p, hdmoe_stream_t stream) {
   mark();
   // down projections, both in one launch
   HdmoeSplitPlan plan;  // candidate cuts; the kernels pick one by the real segment sizes
-  const int parts = hdmoe_down_parts((int)n, E, Hs > 0 ? T : 0, D, H, Hs, wd, &plan);
+  const int parts = hdmoe_down_parts((int)n, E, Hs > 0 ? T : 0, D, H, Hs, wd, &plan, less_room);
   if (p->fixed_k_cut != 0 && plan.n > 1) {  // the cost model's entry, whatever the routing
     plan.pd[0] = plan.fixed_pd;
     plan.ps[0] = plan.fixed_ps;

@@ -432,7 +432,9 @@ typedef struct hdmoe_layer_args {
 /* The workspace size already includes room for the normalised tokens of the block fusion and, with 16-bit activations and
  * sizes whose last round of tiles is cut along K, up to 64 MiB for the parts (at the end, behind hdmoe_layer_layout.flags, unless
  * the partial sums' room serves). A call with a smaller workspace that holds everything else is taken too: no such tile is
- * cut then. */
+ * cut then, and the down projection of a few tokens is cut in fewer parts along K where the room is for those (a row's sums are added
+ * up in another order). The size can fall as T grows, with the parts that a tile is cut into: one buffer for calls of up to T tokens takes the
+ * largest of their sizes. */
 size_t hdmoe_layer_workspace_bytes(int T, int D, int H, int Hs, int E, int weight_dtype);
 int hdmoe_moe_ffn(const hdmoe_layer_args* args, hdmoe_stream_t stream);
 
