@@ -100,9 +100,13 @@ class FeedForward(nn.Module):
         self.net.append(nn.Dropout(dropout))
         self.net.append(operations.Linear(inner_dim, dim_out, device=device, dtype=dtype))
 
+    def stage_weights(self):
+        """((proj weight, bias), (out weight, bias))"""
+        return (self.net[0].proj.weight, self.net[0].proj.bias), (self.net[2].weight, self.net[2].bias)
+
     def stages(self, x):
-        """((proj weight, bias), (out weight, bias)) if both Linears can join a grouped launch, else None."""
-        act, _, out = self.net
+        """stage_weights() if both Linears can join a grouped launch, else None; each module and parameter is looked up once."""
+        act, _, out, *_ = self.net
         first = _plain_pair(act.proj, x)
         second = _plain_pair(out, x) if first is not None else None
         return (first, second) if second is not None else None
@@ -113,7 +117,7 @@ class FeedForward(nn.Module):
     def forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
         x2 = hidden_states.reshape(-1, hidden_states.shape[-1]).contiguous()
         _need(x2)
-        stages = self.stages(x2)
+        stages = _stages(self, x2)
         if stages is None:
             y = self.net[2](self.net[0](x2))     # net[1] is Dropout, the identity at inference
             return y.view(*hidden_states.shape[:-1], y.shape[-1])
@@ -123,6 +127,13 @@ class FeedForward(nn.Module):
         _, y = HF.grouped_linear(h[:0], None, [], a_static=h, shared=w_out, act="none",
                                  fixed_k_cut=amd_ops._batch_invariant(self.net[2]))
         return y.view(*hidden_states.shape[:-1], y.shape[-1])
+
+
+def _stages(ff, x):
+    """FeedForward.stages, by way of fusable and stage_weights where a module has its own."""
+    if type(ff) is FeedForward and "fusable" not in ff.__dict__ and "stage_weights" not in ff.__dict__:
+        return ff.stages(x)
+    return ff.stage_weights() if ff.fusable(x) else None
 
 
 class MoEGate(nn.Module):
@@ -173,7 +184,7 @@ class MoEBlock(nn.Module):
         gate_w = amd_ops.cast_to(self.gate.weight, dtype=x2.dtype, device=x2.device).contiguous()
         idx, w = HF.gate_top2(x2, gate_w)
         _, offsets, perm, inv_perm = HF.dispatch(idx, self.num_experts)
-        stages = [f.stages(x2) for f in (*self.experts, self.shared_experts)]
+        stages = [_stages(f, x2) for f in (*self.experts, self.shared_experts)]
         if any(v is None for v in stages):
             xs = HF.permute_bf16(x2, perm)
             y = torch.empty_like(xs)
