@@ -1913,7 +1913,8 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
   // tiles with K steps requested two ahead, and is bound by how fast the weights arrive, not by its K loops. A layer: the most parts whose
   // tiles fit one round of blocks however the rows fall to the experts (the sizes alone say, so that a row's sums do not depend on the
   // others' routing), the shared expert's tiles in as many as make them about as long, rounded up first. Three parts of every tile up to 128
-  // tokens, two up to 256 -> this (weights from memory; two inputs each), us: fp8, 16 tokens 69.0 64.2 -> 66.7 61.3, 64 73.0 70.8 -> 70.2 67.1, 128
+  // tokens, two up to 256 -> this (weights from memory; two inputs each; rounded down only where the experts' tiles gain a part by it: 8
+  // experts, 256 tokens in fp8 (2, 2) parts 166.9, (2, 1) 170.2), us: fp8, 16 tokens 69.0 64.2 -> 66.7 61.3, 64 73.0 70.8 -> 70.2 67.1, 128
   // 77.8 77.3 -> 75.0 74.4, 256 99.2 95.7 -> 94.0 91.4; bf16, 64 115.9 110.1 -> 110.3 102.4, 256 157.1 148.3 -> 146.2 139.9; e4m3fn weights in bf16,
   // 64 109.4 108.6 -> 100.0 98.7, 256 134.6 135.3 -> 121.3 120.4. (Five parts of every tile, the shared expert's too: 64 tokens in fp8 72.3; the
   // most parts that fit the real segments, picked on the device: 256 tokens 95.1, 200 89.0 where this has 90.8.)
@@ -1939,6 +1940,7 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
       if (mt_d > n_dyn * mt_s) mt_d = n_dyn * mt_s;                                 // (no expert has a token twice)
       for (int pd = 6; pd > 1; --pd)
         for (int ps = (int)fmin((pd * kts + ktd - 1) / ktd, pd); ps >= 1 && 2 * pd * kts <= (2 * ps + 1) * ktd; --ps) {
+          if (pd <= parts && ps * ktd < pd * kts) continue;
           if (ktd / pd < 6 || kts / ps < 6 || (mt_d * pd + mt_s * ps) * nt > HDMOE_NUM_CU) continue;
           pl.n = 1;
           pl.pd[0] = pl.fixed_pd = pd;
