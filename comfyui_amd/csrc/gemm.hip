@@ -1439,13 +1439,13 @@ bool s224_pays(const GemmShape& sh, int tt) {
     }
     const int n_routed = n;
     if (sh.rows_static > 0) part[n++] = {sh.rows_static, sh.N_static / S224_FEAT};
-    int cols = 0;
+    int cols = 0, shift = 4;
     for (int i = 0; i < n; ++i) cols += part[i].cols;
-    const int shift = s224_shift(cols, sh.kbytes);
     int best = 0, whole = 0;   // the kernel's own choice of styles (tile_mix)
     for (int c = 0; c < S224_STYLES * S224_STYLES; ++c) {
       S224Tiles tiles = {0, 0, 0, 0};
       for (int i = 0; i < n; ++i) s224_add(tiles, s224_mix(part[i].rows, i < n_routed ? c / S224_STYLES : c % S224_STYLES), part[i].cols);
+      if (c == 0) shift = s224_shift(cols, sh.kbytes, tiles.highs);
       const int p = sh.n_dyn == 1 || sh.n_dyn == 2 ? s224_cost(tiles.highs, tiles.lows) : s224_price(tiles, shift);
       if (c == 0) {
         whole = best = p;

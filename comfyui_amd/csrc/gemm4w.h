@@ -281,7 +281,7 @@ __device__ __forceinline__ bool tile_mix(const Segments& segs, int G, int lane, 
     for (int g = 0; g < G; ++g)
       s224_add(tiles, s224_mix(__builtin_amdgcn_readlane(rows, g), segs.dynamic(g) ? of_dyn : of_fix, high), __builtin_amdgcn_readlane(nt, g));
     int price;
-    if constexpr (F8) price = s224_price(tiles, s224_shift(cols, segs.bytes(0)));
+    if constexpr (F8) price = s224_price(tiles, s224_shift(cols, segs.bytes(0), highs));
     else price = s224_cost(tiles.highs, tiles.lows, G4_LOW_COST + (W8 ? 0 : tile_div(G4_LOW_ALONE * tiles.alone, max(tiles.lows, 1))));
     const int mine = price << 5 | c;
     const int first = __builtin_amdgcn_readlane(mine, 0);

@@ -102,11 +102,16 @@ HDMOE_TAIL_HD void s224_add(S224Tiles& t, const S224Mix& m, int cols) {
 }
 // The price of a choice of tiles. Low tiles behind high ones of the same columns read their weights again, and from memory where the launch's
 // weights are more than about 100 MB: in 16ths of a hundredth of a high tile, 2 for such a column and 1 for a low tile (half of that where they
-// are not), which is about 650 KB of weights at 6 TB/s. Whole pass on this kernel, us, high tiles alone, lows where s224_cost alone gains,
+// are not), which is about 650 KB of weights at 6 TB/s; nothing from 8 rounds on where they stay in the memory-side cache (4 experts and a shared one,
+// 4096 tokens, high tiles alone 475.5 and 475.4, this 469.8 and 471.4). Whole pass on this kernel, us, high tiles alone, lows where s224_cost alone gains,
 // where this does (weights from memory): layers of 16 experts, 2048 tokens 424 480 424; 12 experts, 1600 321 362 323; 8 experts, 1100 233 251 234;
 // width 4096, 950 332 350 335; 4 experts of 6912 and a shared one of 3584, 350 120 111 111, 500 139 138 130, 700 150 143 143, 1024 183 178 178; 6 experts,
 // 950 211 209 203; dense branch, 32768 features, 768 rows 188 195 189; width 4096, 1300 rows 184 174 175; 1300 rows 87.3 85.0 85.5. Other tiles than
 // high ones alone have to pay by a 32nd: the clock falls with the CUs that are busy (a 24th loses 1 % at 1300 and 2048 tokens).
 HDMOE_TAIL_HD int s224_price(const S224Tiles& t, int shift) { return s224_cost(t.highs, t.lows) + ((2 * t.both + t.lows) >> shift); }
-HDMOE_TAIL_HD int s224_shift(int cols, int kbytes) { return (long long)cols * 256 * kbytes <= (100ll << 20) ? 5 : 4; }
+// whole: high tiles alone
+HDMOE_TAIL_HD int s224_shift(int cols, int kbytes, int whole) {
+  const long long bytes = (long long)cols * 256 * kbytes;
+  return bytes <= (100ll << 20) ? 5 : bytes <= (200ll << 20) && whole >= 8 * 256 ? 8 : 4;
+}
 HDMOE_TAIL_HD bool s224_low_pays(int price, int whole, int margin = 32) { return price < whole - whole / margin; }

@@ -40,10 +40,16 @@ def test_low_tiles_that_end_a_round(lib, tokens):
     assert styles(lib, [tokens // 2 + d for d in (-8, 8, -8, 8)], tokens) != (0, 0)
 
 
+@pytest.mark.parametrize("rows,low", [(128, False), (256, True), (257, True), (400, True), (513, False), (1024, False), (1300, True), (1500, True), (2000, False)])
+def test_low_tiles_on_16_bit_activations(lib, rows, low):
+    """A dense feed-forward of 6912 features on 256-row tiles."""
+    assert (lib.t_style16(rows, H, 27) != 0) == low
+
+
 def test_price(lib):
     assert lib.t_price(432, 0, 0, 4) == 200 and lib.t_price(432, 32, 0, 4) == 202   # beside the last round's high tiles
     assert lib.t_price(1144, 864, 864, 4) > lib.t_price(2008, 0, 0, 4)
-    assert lib.t_shift(86, 4096) == 5 and lib.t_shift(244, 2560) == 4 and lib.t_shift(1 << 20, 1 << 20) == 4
+    assert lib.t_shift(86, 4096, 1) == 5 and lib.t_shift(244, 2560, 2047) == 4 and lib.t_shift(244, 2560, 2048) == 8 and lib.t_shift(1 << 20, 1 << 20, 4096) == 4
 
 
 def name(tokens, experts, d=2560, h=6912, hs=3584, scaled=1):
