@@ -1910,10 +1910,11 @@ int hdmoe_down_parts(int rows_dyn, int n_dyn, int rows_static, int N, int K_dyn,
   if ((!dyn && rows_static <= 0) || nt <= 0 || (ktd <= 0 && kts <= 0)) return fixed(1);
 
   // Few rows per segment (the rule of the light form in hdmoe_launch_ffn_gemm): the launch runs on 128-token
-  // tiles with K steps requested two ahead, and is bound by how fast the weights arrive, not by its K loops. A layer: the most parts whose
+  // tiles with K steps requested two ahead, and is bound by how fast the weights arrive, not by its K loops. (e4m3fn weights in bf16 run on 256-row
+  // tiles, of which the rows can make fewer: for them the count below is the most, and from 129 tokens on five and three parts would fit.) A layer: the most parts whose
   // tiles fit one round of blocks however the rows fall to the experts (the sizes alone say, so that a row's sums do not depend on the
   // others' routing), the shared expert's tiles in as many as make them about as long, rounded up first. Three parts of every tile up to 128
-  // tokens, two up to 256 -> this (weights from memory; two inputs each; rounded down only where the experts' tiles gain a part by it: 8
+  // tokens, two up to 256 -> this (weights from memory, two inputs each; rounded down only where the experts' tiles gain a part by it: 8
   // experts, 256 tokens in fp8 (2, 2) parts 166.9, (2, 1) 170.2), us: fp8, 16 tokens 69.0 64.2 -> 66.7 61.3, 64 73.0 70.8 -> 70.2 67.1, 128
   // 77.8 77.3 -> 75.0 74.4, 256 99.2 95.7 -> 94.0 91.4; bf16, 64 115.9 110.1 -> 110.3 102.4, 256 157.1 148.3 -> 146.2 139.9; e4m3fn weights in bf16,
   // 64 109.4 108.6 -> 100.0 98.7, 256 134.6 135.3 -> 121.3 120.4. (Five parts of every tile, the shared expert's too: 64 tokens in fp8 72.3; the
