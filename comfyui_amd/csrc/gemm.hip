@@ -1411,21 +1411,20 @@ bool short_tile_pays(const GemmShape& sh) {
   return 20 * expected_tile_cost(sh, 3) <= 17 * (c4 < c5 ? c4 : c5);
 }
 
-// Whether fp8 gate/up runs on 224-token tiles (tt: height of the other kernel's tiles in blocks of 64). Both sides are rounds of tiles, in hundredths of
-// a round of high 224-token tiles (s224_price, with the kernel's choice of styles) and in units of expected_tile_cost; a round here takes 70 / 21 of
-// them (8192 tokens: 28.8 us, the 320-token tile of 6 units 45), and 15 / 21 go for the last tile's activation, which nothing hides. Segments are
-// taken even, and a standard deviation apart (tokens that go to 2 of n experts), half the price each: 512 tokens on 4 experts are not 4 tiles of
-// 256. A tile of the other kernel that is not full costs up to a quarter less: zeros take little power, and the clock follows. Whole pass, us,
-// the other kernel, this one (weights from memory): layers of 4 experts, 257 tokens 107 112 (left to the
-// other up to 320), 350 129 111, 512 133 132, 700 165 143, 1024 188 177, 4096 493 452; 8 experts, 400 174 168, 500 179 190 (other), 1000 229 228, 1283 310 252;
-// 6 experts, 700 170 178 (other), 950 245 203; 16 experts, 1950 387 398 (other), 2200 478 435; width 4096, 617 303 277; dense, 400 rows 50.7 49.5,
-// 577 55.0 57.4 (other: 513 to 768), 950 73 74 (other: 897 to 1280), 1300 88 85, 2200 113 117 (other: 2049 to 2304), 3584 162 158, 4096 187 169; 32768
-// features, 480 rows 136 145 (other). Where it errs: width 4096, 448 tokens 217 232; 4 experts without
-// a shared one, 993 tokens 144 150.
-// A dense feed-forward of up to 384 rows stays on 192-token tiles, where low tiles would be faster (Linears with and without scale_input, 257
-// rows 49.2 47.3, 300 50.2 47.9, 384 52.7 49.2): tests/test_gpu_fp8_dense_tiles.py has 300 rows of that width on them. And one or two groups are
-// taken at s224_cost, without the price of weights read again (two experts of 16384 features, 452 tokens: 125.7 132.0):
-// tests/test_gpu_swiglu224.py has such sizes on this kernel.
+// Whether fp8 gate/up runs on 224-token tiles (tt: height of the other kernel's tiles in blocks of 64). Both sides are rounds of tiles, in
+// hundredths of a round of high 224-token tiles (s224_price, with the kernel's choice of styles) and in units of expected_tile_cost; a round here
+// takes 70 / 21 of them (8192 tokens: 28.8 us, the 320-token tile of 6 units 45), and 15 / 21 go for the last tile's activation, which nothing
+// hides. Segments are taken even, and a standard deviation apart (tokens that go to 2 of n experts), half the price each: 512 tokens on 4 experts
+// are not 4 tiles of 256. A tile of the other kernel that is not full costs up to a quarter less: zeros take little power, and the clock follows.
+// Whole pass, us, the other kernel, this one (weights from memory): layers of 4 experts, 257 tokens 107 112 (left to the other up to 320), 350 129
+// 111, 512 133 132, 700 165 143, 1024 188 177, 4096 493 452; 8 experts, 400 174 168, 500 179 190 (other), 1000 229 228, 1283 310 252; 6 experts,
+// 700 170 178 (other), 950 245 203; 16 experts, 1950 387 398 (other), 2200 478 435; width 4096, 617 303 277; dense, 400 rows 50.7 49.5, 577 55.0
+// 57.4 (other: 513 to 768), 950 73 74 (other: 897 to 1280), 1300 88 85, 2200 113 117 (other: 2049 to 2304), 3584 162 158, 4096 187 169; 32768
+// features, 480 rows 136 145 (other). Where it errs: width 4096, 448 tokens 217 232; 4 experts without a shared one, 993 tokens 144 150.
+// A dense feed-forward of up to 384 rows stays on 192-token tiles, where low tiles would be faster (Linears with and without scale_input, 257 rows
+// 49.2 47.3, 300 50.2 47.9, 384 52.7 49.2): tests/test_gpu_fp8_dense_tiles.py has 300 rows of that width on them. And one or two groups are taken
+// at s224_cost, without the price of weights read again (two experts of 16384 features, 452 tokens: 125.7 132.0): tests/test_gpu_swiglu224.py has
+// such sizes on this kernel.
 bool s224_pays(const GemmShape& sh, int tt) {
   double price = 0, other = 0;
   for (int spread = 0; spread < 2; ++spread) {
