@@ -1417,7 +1417,7 @@ bool short_tile_pays(const GemmShape& sh) {
 // hides. Segments are taken even, and a standard deviation apart (tokens that go to 2 of n experts), half the price each: 512 tokens on 4 experts
 // are not 4 tiles of 256. A tile of the other kernel that is not full costs up to a quarter less: zeros take little power, and the clock follows.
 // Whole pass, us, the other kernel, this one (weights from memory): layers of 4 experts, 257 tokens 107 112 (left to the other up to 320), 350 129
-// 111, 512 133 132, 700 165 143, 1024 188 177, 4096 493 452; 8 experts, 400 174 168, 500 179 190 (other), 1000 229 228, 1283 310 252; 6 experts,
+// 111, 512 133 132, 700 165 143, 1024 188 177, 4096 493 452; 8 experts, 400 174 168, 500 179 190 (other), 1000 229 228, 1300 310 252; 6 experts,
 // 700 170 178 (other), 950 245 203; 16 experts, 1950 387 398 (other), 2200 478 435; width 4096, 617 303 277; dense, 400 rows 50.7 49.5, 577 55.0
 // 57.4 (other: 513 to 768), 950 73 74 (other: 897 to 1280), 1300 88 85, 2200 113 117 (other: 2049 to 2304), 3584 162 158, 4096 187 169; 32768
 // features, 480 rows 136 145 (other). Where it errs: width 4096, 448 tokens 217 232; 4 experts without a shared one, 993 tokens 144 150.
